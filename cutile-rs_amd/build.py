@@ -34,8 +34,9 @@ IMAGES = {
     "mxgemm": "mxfp8_gemm.hip",
     "nvfp4": "nvfp4_gemm.hip",
     "rng": "rng.hip",
+    "gemmsmall": "gemm_small.hip",
 }
-HOST_SOURCES = ["hip_api.cpp", "driver.cpp", "kernel_table.cpp", "launch.cpp", "runtime.cpp", "tuning.cpp"]
+HOST_SOURCES = ["hip_api.cpp", "driver.cpp", "kernel_table.cpp", "launch.cpp", "runtime.cpp", "tuning.cpp", "workspace.cpp"]
 # The recording stand-in for the HIP runtime (include/cutile_hip_testing.h) is not part of the product library: the CPU
 # tests load a second library, the same objects plus this source.
 TESTING_SOURCES = ["fake_hip.cpp"]

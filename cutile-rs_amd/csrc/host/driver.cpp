@@ -165,6 +165,7 @@ cutile_status_t cutile_stream_create(cutile_device_t device, cutile_stream_t* st
 
 cutile_status_t cutile_stream_release(cutile_device_t device, cutile_stream_t stream) {
   CUTILE_REQUIRE(device && stream, CUTILE_ERR_INVALID_ARGUMENT, "null argument");
+  release_split_workspace(device, (hipStream_t)stream);
   std::lock_guard<std::mutex> lock(device->mutex);
   device->idle_streams.push_back((hipStream_t)stream);
   return CUTILE_SUCCESS;

@@ -155,6 +155,11 @@ hipError_t f_hipLaunchHostFunc(hipStream_t s, hipHostFn_t fn, void* user) {
   fn(user);
   return hipSuccess;
 }
+hipError_t f_hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status) {
+  FAKE_FAIL("hipStreamIsCapturing");
+  *status = s && fs(s)->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
 hipError_t f_hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
   FAKE_FAIL("hipStreamBeginCapture");
   if (!s || fs(s)->capturing) return hipErrorInvalidValue;
@@ -392,6 +397,7 @@ HipApi make_fake_table() {
   t.hipStreamQuery = f_hipStreamQuery;
   t.hipLaunchHostFunc = f_hipLaunchHostFunc;
   t.hipStreamBeginCapture = f_hipStreamBeginCapture;
+  t.hipStreamIsCapturing = f_hipStreamIsCapturing;
   t.hipStreamEndCapture = f_hipStreamEndCapture;
   t.hipStreamWriteValue32 = f_hipStreamWriteValue32;
   t.hipEventCreateWithFlags = f_hipEventCreateWithFlags;

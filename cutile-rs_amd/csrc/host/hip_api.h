@@ -28,6 +28,7 @@ namespace cutile {
   X(hipStreamQuery, hipError_t, (hipStream_t))                                                         \
   X(hipLaunchHostFunc, hipError_t, (hipStream_t, hipHostFn_t, void*))                                  \
   X(hipStreamBeginCapture, hipError_t, (hipStream_t, hipStreamCaptureMode))                            \
+  X(hipStreamIsCapturing, hipError_t, (hipStream_t, hipStreamCaptureStatus*))                          \
   X(hipStreamEndCapture, hipError_t, (hipStream_t, hipGraph_t*))                                       \
   X(hipStreamWriteValue32, hipError_t, (hipStream_t, void*, uint32_t, unsigned int))                   \
   X(hipEventCreateWithFlags, hipError_t, (hipEvent_t*, unsigned int))                                  \

@@ -20,6 +20,7 @@ extern const unsigned char cutile_img_fmha_start[], cutile_img_fmha_end[];
 extern const unsigned char cutile_img_mxgemm_start[], cutile_img_mxgemm_end[];
 extern const unsigned char cutile_img_nvfp4_start[], cutile_img_nvfp4_end[];
 extern const unsigned char cutile_img_rng_start[], cutile_img_rng_end[];
+extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_end[];
 }
 
 namespace cutile {
@@ -44,6 +45,7 @@ ImageRef image_ref(Image img) {
     case IMG_MXGEMM: return {cutile_img_mxgemm_start, cutile_img_mxgemm_end};
     case IMG_NVFP4: return {cutile_img_nvfp4_start, cutile_img_nvfp4_end};
     case IMG_RNG: return {cutile_img_rng_start, cutile_img_rng_end};
+    case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
     default: return {nullptr, nullptr};
   }
 }
@@ -206,6 +208,13 @@ std::vector<KernelEntry> build_table() {
   for (const char* dt : {"bf16", "bf16f32", "f16", "f32"})
     add("gemm", keep(std::string(dt) + "_generic"), keep(std::string("gemm_entry__") + dt + "_generic"), IMG_GEMM, 256,
         (uint32_t)((64 * 17 + 16 * 65) * 4), 0, 0, 0, 0, dt, 0, 2);
+
+  // few rows of x: workgroups per strip of columns and K split (any alignment, any partition shape)
+  for (const char* dt : {"bf16", "f16", "bf16f32"})
+    for (auto t : {std::array<int, 2>{16, 64}, std::array<int, 2>{16, 128}, std::array<int, 2>{32, 64}, std::array<int, 2>{64, 64}}) {
+      std::string v = std::string(dt) + "_thin" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
+      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, (uint32_t)(8 * t[0] * (t[1] + 4) * 4), 0, t[1], 0, t[0], dt, 0, 2);
+    }
 
   // batched GEMM (cutile-examples/examples/batch_matmul.rs): the pipelined bodies with the batch on a grid axis
   for (const char* kind : {"q", "r"})          // rings of three a stages and two b stages (q: on v_mfma_f32_16x16x32, any K; r: whole K tiles only)

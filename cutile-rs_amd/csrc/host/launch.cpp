@@ -140,7 +140,7 @@ struct ArgPacker {
 thread_local int g_launch_mode = 0;
 // Shape class of the launch being resolved (set by the launchers that tuning records cover) and where the last
 // resolved variant came from: "caller" (opts.variant), "record:<bucket>" (a verified tuning record), "pinned"
-// (cutile_kernel_set_preferred_variant) or "table" (the table's order).
+// (cutile_kernel_set_preferred_variant), "size" (the launcher's rule on extents) or "table" (the table's order).
 thread_local std::string g_bucket;
 thread_local std::string g_last_source;
 thread_local std::string g_last_bucket;
@@ -255,11 +255,12 @@ cutile_status_t resolve_grid(const cutile_partition_arg_t* out, const cutile_lau
 }
 
 // Picks the variant.  Precedence: the caller's variant, the function-wide pin set at run time
-// (cutile_kernel_set_preferred_variant), the shape class's winner (a verified tuning record or
+// (cutile_kernel_set_preferred_variant), `sized` (the launcher's own rule for extents that the shape classes of the tuning
+// records do not tell apart), the shape class's winner (a verified tuning record or
 // cutile_kernel_set_preferred_variant_for), then `fallback` (the table's order).  A pin or a winner that does not fit
 // these arguments is passed over, not an error.
 cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* opts, const std::string& fallback,
-                              const std::vector<std::string>& acceptable, Resolved* r) {
+                              const std::vector<std::string>& acceptable, Resolved* r, const std::string& sized = std::string()) {
   std::string want;
   g_last_source = "caller";
   g_last_bucket = g_bucket;
@@ -271,6 +272,10 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
       want = pref;
       g_last_source = "pinned";
     }
+  }
+  if (want.empty() && fits(sized)) {
+    want = sized;
+    g_last_source = "size";
   }
   if (want.empty() && !g_bucket.empty()) {
     ensure_tuning_records_loaded();
@@ -306,6 +311,28 @@ uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 // The streaming GEMM variants ("..._s2x4"): a family of kernels behind one variant name.
 bool is_stream_variant(const char* variant) { return strstr(variant, "_s2x4") != nullptr; }
+// How many workgroups may share an output block of `floats` f32 values when a launch has `blocks` of them (1: none may).
+uint32_t split_limit(uint64_t blocks, uint64_t floats) {
+  return blocks > kSplitCounters ? 1u : (uint32_t)std::max<uint64_t>(1, kSplitPartialBytes / (blocks * floats * sizeof(float)));
+}
+// The thin GEMM kernels: no output tile of their own, tile[1] columns a strip, tile[3] rows in a pass.
+bool is_thin(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
+// The one for `rows` rows of x and an n-column y, or "" where the tiled kernels are the better ones.  Measured at M = 1 to 64,
+// f16 and bf16 (us, thin against the 128 x 128 tiles): 4096 x 4096 10 - 21 against 53, K = 14336 25 - 41 against 175,
+// 14336 x 4096 24 - 35 against 54, 1024 x 1024 5 - 9 against 11.  128-column strips where there are enough of them to keep
+// three quarters of the compute units busy (28672 x 8192, one row: 83 us against 92 with 64-column strips); with more
+// than 32 rows x costs as many bytes as y and that many columns are better off with tiles (129 against 113 us).
+std::string thin_variant(const std::string& dt, int64_t rows, int64_t n, int32_t k) {
+  if (rows > 64 || n < 64 || k <= 64) return "";   // one 64-row step: nothing for the other seven wavefronts to share
+  const bool many = n >= 192 * 128;
+  if (many && rows > 32) return "";
+  return dt + (rows > 32 ? "_thin64x64" : rows > 16 ? "_thin32x64" : many ? "_thin16x128" : "_thin16x64");
+}
+// K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8
+// wavefronts (N = K = 4096, one row: 19.1, 12.6, 10.4, 11.3, 15.4 us with 1, 2, 4, 8, 16 splits; K = 1024: 5.0, 5.3, 5.8, 7.2).
+uint32_t thin_splits(uint64_t blocks, int32_t k, int cus) {
+  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8 * 2)));
+}
 // An output of this size or more is read and stored past the caches (it cannot still be cached when its consumer runs,
 // and the caches are left to the operand panels): the rule of the staged epilogue, decided on the host for this family.
 constexpr int64_t kStreamedOutputBytes = 64ll << 20;
@@ -1930,11 +1957,23 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
           (k_valid % 64 == 0 || strstr(e.variant, "_r") == nullptr) && strchr(e.variant, '+') == nullptr &&
           (whole_tiles || !is_stream_variant(e.variant)))
         acceptable.push_back(e.variant);
+  // Few rows: the thin kernels take any partition shape and any row alignment, need rows of unit stride and a strip of
+  // y's columns, and cover 64 rows in a pass (more rows are further passes over y).
+  const bool row_layout = x->strides[1] == 1 && y->strides[1] == 1 && zt.strides[1] == 1 && dt != "f32" && extent_bytes_2d(*x) < kDescriptorLimit &&
+                          extent_bytes_2d(*y) < kDescriptorLimit && extent_bytes_2d(zt) < kDescriptorLimit;
+  const int64_t cover_m = std::min<int64_t>((int64_t)tg[0] * bm, zt.shape[0]), cover_n = std::min<int64_t>((int64_t)tg[1] * bn, zt.shape[1]);
+  const std::string fallback = acceptable.empty() ? dt + "_generic" : acceptable[0];
+  std::string sized;
+  if (row_layout && x->shape[0] > 0 && k_valid > 0) {
+    for (const auto& e : kernel_table())
+      if (is_thin(&e) && strcmp(e.function, "gemm") == 0 && dt == e.dtype && y->shape[1] >= e.tile[1]) acceptable.push_back(e.variant);
+    sized = thin_variant(dt, cover_m, y->shape[1], k_valid);
+  }
   acceptable.push_back(dt + "_generic");
   Resolved res;
   // shape class for tuning records: the tile, and whether the tiles fit one wave of workgroups over the 256 CUs
   BucketScope bucket(dt + "_" + std::to_string(bm) + "x" + std::to_string(bn) + ((uint64_t)tg[0] * tg[1] <= 256 ? "|tiles<=256" : "|tiles>256"));
-  if (cutile_status_t s = resolve_entry("gemm", opts, acceptable[0], acceptable, &res)) return s;
+  if (cutile_status_t s = resolve_entry("gemm", opts, fallback, acceptable, &res, sized)) return s;
   uint32_t stream_grid = 0;
   if (is_stream_variant(res.entry->variant)) {
     if (cutile_status_t s = stream_member(&res, "gemm", accumulate != 0, zt, (uint64_t)tg[0] * tg[1], &stream_grid)) return s;
@@ -1949,12 +1988,29 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   args.push_tensor(*x);
   args.push_tensor(*y);
   args.push_val<int32_t>(k_total);
+  if (is_thin(res.entry)) {
+    args.push_val<int32_t>((int32_t)cover_m);
+    args.push_val<int32_t>((int32_t)cover_n);
+    args.push_val<int32_t>(accumulate ? 1 : 0);
+    uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
+    SplitWorkspace ws;
+    int cus = 256;
+    if (g_launch_mode != 2)
+      if (cutile_status_t s = compute_units(res.device, &cus)) return s;
+    const uint64_t blocks = (uint64_t)grid[0] * grid[1];
+    const uint32_t splits = std::min(thin_splits(blocks, k_valid, cus), split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
+    if (splits > 1 && g_launch_mode == 0) {
+      if (cutile_status_t s = split_workspace(res.device, (hipStream_t)stream, &ws)) return s;
+      if (ws.partials) grid[2] = splits;
+    }
+    args.push_val<void*>(ws.partials);
+    args.push_val<void*>(ws.counters);
+    return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
+  }
   args.push_tile_grid(tg);
   args.push_val<int32_t>(accumulate ? 1 : 0);
   uint32_t grid[3] = {stream_grid ? stream_grid : tg[0] * tg[1], 1, 1};
   if (res.entry->tile[0] == 0) {   // any-layout kernel: 64x64 outputs per workgroup over the covered region
-    const uint64_t cover_m = std::min<uint64_t>((uint64_t)tg[0] * bm, zt.shape[0]);
-    const uint64_t cover_n = std::min<uint64_t>((uint64_t)tg[1] * bn, zt.shape[1]);
     grid[0] = std::max<uint32_t>(1, div_up(cover_m, 64));
     grid[1] = std::max<uint32_t>(1, div_up(cover_n, 64));
   }

@@ -22,6 +22,7 @@ struct cutile_device {
   std::vector<hipStream_t> idle_streams;  // released streams, reused before creating new ones
   uint64_t streams_created = 0;
   int compute_units = 0;  // filled on first use by compute_units()
+  std::map<hipStream_t, void*> split_workspaces;   // workspace.cpp
   // Code objects of the kernel table loaded on this device: image id -> module.
   std::map<int, cutile_module*> table_modules;
   // Resolved functions: symbol -> hipFunction_t.
@@ -36,6 +37,15 @@ void reset_runtime_for_testing();
 void reset_async_runtime_for_testing();
 // Device the calling thread is bound to (hipGetDevice), as a handle.
 cutile_status_t current_device(cutile_device_t* device);
+// Where the workgroups of a launch that splits the K axis of one output block leave their partial sums (workspace.cpp).
+constexpr size_t kSplitCounters = 4096;                  // output blocks of one launch
+constexpr size_t kSplitPartialBytes = 16u << 20;
+struct SplitWorkspace {
+  float* partials = nullptr;      // nullptr: none to be had, the launch must not split
+  uint32_t* counters = nullptr;   // kSplitCounters words, all 0 between launches
+};
+cutile_status_t split_workspace(cutile_device_t device, hipStream_t stream, SplitWorkspace* out);
+void release_split_workspace(cutile_device_t device, hipStream_t stream);
 // Compute units of the device (cached).
 cutile_status_t compute_units(cutile_device_t device, int* count);
 

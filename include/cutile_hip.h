@@ -241,7 +241,7 @@ cutile_status_t cutile_kernel_set_preferred_variant_for(const char* function, co
 cutile_status_t cutile_tuning_reload(const char* directory);
 const char* cutile_tuning_report(void);           /* one line per file: applied / refused / warning; valid until the thread's next call */
 int32_t cutile_tuning_applied_count(void);        /* buckets with a winner from a record */
-/* Where the calling thread's last launcher call took its variant from: "caller", "record:<bucket>", "pinned" or "table";
+/* Where the calling thread's last launcher call took its variant from: "caller", "record:<bucket>", "pinned", "size" (a launcher's rule on extents) or "table";
  * and the shape class that call was filed under ("" for launchers without classes). */
 const char* cutile_last_resolved_source(void);
 const char* cutile_last_resolved_bucket(void);

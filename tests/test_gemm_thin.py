@@ -1,0 +1,84 @@
+"""The GEMM kernels for few rows of x (gemm_small.hip): strips of columns, K split over wavefronts and workgroups."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from util import normal_bf16_bits, normal_f16_bits, rel_l2, to_dev_bf16
+
+SIZES = [
+    # rows, n, k: edges of the 16-row blocks, of the 64-column strip and of the 64-row K step; odd rows start on 2-byte boundaries
+    (1, 64, 64), (1, 64, 8), (16, 65, 63), (17, 127, 65), (32, 129, 1), (33, 200, 130), (48, 64, 4096), (64, 1000, 257), (5, 4096, 2048),
+    (1, 1024, 8200), (64, 192, 6144),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("dtype,accumulate", [("bf16", True), ("f16", False), ("bf16f32", True)])
+def test_gpu_thin_gemm(ct, dev, m, n, k, dtype, accumulate):
+    f16 = dtype == "f16"
+    bits = normal_f16_bits if f16 else normal_bf16_bits
+    to_dev = (lambda b: torch.from_numpy(b.view(np.float16)).to(dev)) if f16 else (lambda b: to_dev_bf16(b, dev))
+    widen = oracle.f16_bits_to_f32 if f16 else oracle.bf16_bits_to_f32
+    a, b = bits((m, k), 901), bits((k, n), 902)
+    out = {"bf16": torch.bfloat16, "f16": torch.float16, "bf16f32": torch.float32}[dtype]
+    x, y = to_dev(a), to_dev(b)
+    z0 = torch.from_numpy(oracle.normal_f32((m, n), 903)).to(dev).to(out)
+    z = torch.full((m + 1, n), 7.0, dtype=out, device=dev)      # a row behind z that nothing may touch
+    for _ in range(2):                                           # the second launch finds the first one's counters at 0
+        z[:m] = z0
+        forced = None if k > 64 else f"{dtype}_thin{16 if m <= 16 else 32 if m <= 32 else 64}x64"    # one step: not chosen by itself
+        ct.gemm(ct.partition(z[:m], [128, 128]), x, y, k, accumulate=accumulate, generics=[dtype, 128, 128, 1], variant=forced)
+        assert "_thin" in ct.last_resolved()["variant"] and ct.last_resolved()["source"] == ("caller" if forced else "size")
+        torch.cuda.synchronize()
+        ref = widen(a).astype(np.float64) @ widen(b).astype(np.float64) + (z0.double().cpu().numpy() if accumulate else 0)
+        # one rounding to the output type (2^-9 bf16, 2^-12 f16 relative) over f32 sums of k products
+        assert rel_l2(z[:m].double().cpu().numpy(), ref) <= {"bf16": 2.0 ** -9, "f16": 2.0 ** -12, "bf16f32": 2e-6}[dtype]
+        assert torch.all(z[m] == 7.0)
+
+
+@pytest.mark.gpu
+def test_gpu_thin_gemm_streams_and_prefix(ct, dev):
+    """split launches on two streams at once (each stream has partial sums of its own), and a launch over the first tile row only"""
+    k, n = 8192, 1024
+    x = torch.from_numpy(normal_f16_bits((40, k), 911).view(np.float16)).to(dev)
+    ys = [torch.from_numpy(normal_f16_bits((k, n), 912 + i).view(np.float16)).to(dev) for i in range(2)]
+    want = [(x.double() @ y.double()) for y in ys]
+    streams = [torch.cuda.Stream() for _ in ys]
+    zs = [torch.zeros(40, n, dtype=torch.float16, device=dev) for _ in range(8)]
+    torch.cuda.synchronize()
+    for i, z in enumerate(zs):
+        ct.gemm(ct.partition(z, [128, 128]), x, ys[i % 2], k, accumulate=False, stream=streams[i % 2].cuda_stream)
+    torch.cuda.synchronize()
+    for i, z in enumerate(zs):
+        assert rel_l2(z.double().cpu().numpy(), want[i % 2].cpu().numpy()) <= 2.0 ** -12 and torch.equal(z, zs[i % 2])
+    z = torch.full((40, n), 3.0, dtype=torch.float16, device=dev)
+    ct.gemm(ct.partition(z, [16, 64], prefix=True), x, ys[0], k, accumulate=False, grid=(1, 2, 1))
+    torch.cuda.synchronize()
+    assert torch.equal(z[:16, :128], zs[0][:16, :128]) and torch.all(z[16:] == 3.0) and torch.all(z[:, 128:] == 3.0)
+
+
+@pytest.mark.gpu
+def test_gpu_thin_gemm_captured_and_replayed(ct, dev):
+    """a captured launch does not split K (its workspace would belong to a stream); every replay equals float64 to f16 rounding"""
+    k, n = 4096, 256
+    x = torch.from_numpy(normal_f16_bits((3, k), 921).view(np.float16)).to(dev)
+    y = torch.from_numpy(normal_f16_bits((k, n), 922).view(np.float16)).to(dev)
+    z = torch.zeros(3, n, dtype=torch.float16, device=dev)
+    launch = lambda stream=None: ct.gemm(ct.partition(z, [128, 128]), x, y, k, accumulate=False, stream=stream)
+    launch()
+    torch.cuda.synchronize()
+    graph = ct.CapturedGraph().capture(launch)
+    want = (x.double() @ y.double()).cpu().numpy()
+    try:
+        for _ in range(3):
+            z.zero_()
+            torch.cuda.synchronize()
+            graph.launch()
+            graph.synchronize()
+            assert rel_l2(z.double().cpu().numpy(), want) <= 2.0 ** -12
+            launch()
+            torch.cuda.synchronize()
+    finally:
+        graph.close()
