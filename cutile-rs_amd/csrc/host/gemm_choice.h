@@ -1,0 +1,90 @@
+// Which GEMM kernel a launch takes from its extents, where the shape classes of the tuning records are too coarse:
+// few rows, outputs of fewer 256 x 256 tiles than compute units (or of a few more), and rows off 16-byte boundaries.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+#include <cstdio>
+#include <cstring>
+
+namespace cutile {
+
+struct GemmShape {
+  const char* dtype;       // the table's name of the operand / output types: bf16, f16, bf16f32
+  int64_t m, n;            // outputs the launch covers
+  int64_t y_cols;          // columns of y (a strip or a tile of the gemm_small.hip kernels must lie inside them)
+  int32_t k;
+  bool aligned;            // rows on 16-byte boundaries, whole output covered: the ring kernels can take it
+  bool own_tile;           // the partition's tile has kernels of its own
+};
+
+struct GemmChoice {
+  char variant[48] = "";   // "": the partition's own tile (tuning record, then the table's order)
+};
+
+// K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8
+// wavefronts (N = K = 4096, one row: 19.1, 12.6, 10.4, 11.3, 15.4 us with 1, 2, 4, 8, 16 splits; K = 1024: 5.0, 5.3, 5.8, 7.2).
+inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus) {
+  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8 * 2)));
+}
+// K splits of a staged launch: up to two workgroups per compute unit, at least 8 K tiles each (1262 x 128 x 16128, 40 tiles of
+// 64 x 64: 99, 54, 40, 32, 30 us with 1, 2, 3, 4, 8 splits; 128 x 4096 x 4096, 128 tiles: 40, 28.5, 28.0, 28.2, 47).
+inline uint32_t staged_splits(uint64_t blocks, int32_t k, int cus) {
+  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(int64_t)(2 * (uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8), 8}));
+}
+
+inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
+  GemmChoice c;
+  if (s.k <= 64) return c;   // one K tile: nothing to stage, split or overlap
+  auto pick = [&](const char* kernel) { snprintf(c.variant, sizeof(c.variant), "%s_%s", s.dtype, kernel); };
+  // Few rows.  Measured at 1 to 64 rows, f16 and bf16 (us, thin against 128 x 128 tiles): 4096 x 4096 10 - 21 against 53,
+  // K = 14336 25 - 41 against 175, 14336 x 4096 24 - 35 against 54, 1024 x 1024 5 - 9 against 11.  128-column strips where
+  // there are enough of them to keep three quarters of the compute units busy (28672 x 8192, one row: 83 us against 92);
+  // with more than 32 rows x costs as many bytes as y and that many columns are better off with tiles (129 against 113 us).
+  // Up to 128 rows (two passes over y, the second from L2) while the strips of both passes fit the chip once
+  // (4096 x 4096 23 us against 27 with staged tiles; 14336 x 4096 60 against 46).
+  const bool many = s.n >= 192 * 128;
+  if (s.y_cols >= 64 && ((s.m <= 64 && !(many && s.m > 32)) || (s.m <= 128 && 2 * ((s.n + 63) / 64) <= cus))) {
+    pick(s.m > 32 ? "thin64x64" : s.m > 16 ? "thin32x64" : many && s.y_cols >= 128 ? "thin16x128" : "thin16x64");
+    return c;
+  }
+  auto tiles = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
+  const double kt = s.k / 64.0;
+  double best = 1e30;
+  // The ring kernels.  One K tile of a launch that fills few compute units costs `few` us, of one that fills all of them `all`
+  // us (operands through the same L2s, and the clock): from 4096-deep products with 64 to 256 tiles of each shape.  1500 x 14336 x
+  // 4096 predicted 152, 172, 169 us for 192 x 256, 256 x 256, 128 x 256 tiles, measured 152, 172, 168.
+  struct RingTile { const char* kernel; int bm, bn; double few, all; };
+  static const RingTile kRing[] = {{"256x256x64_q2x4", 256, 256, 1.08, 1.42}, {"192x256x64_q2x4", 192, 256, 0.88, 1.12}, {"256x128x64_q4x2", 256, 128, 0.67, 0.82},
+                                   {"128x256x64_q2x4", 128, 256, 0.68, 0.82}, {"192x128x64_q2x2", 192, 128, 0.66, 0.74}};
+  // (up to K = 512 the start and the output of a tile are most of a launch: the partition's own tile, if it has kernels)
+  const bool ring = s.aligned && (s.k > 512 || !s.own_tile) && strcmp(s.dtype, "bf16f32") != 0;
+  if (ring) {
+    for (const RingTile& r : kRing) {
+      const uint64_t t = tiles(r.bm, r.bn), rest = t % cus;
+      const double us = kt * ((double)(t / cus) * r.all + (rest ? r.few + (r.all - r.few) * (double)rest / cus : 0.0)) + 4.0 * (double)((t + cus - 1) / cus);
+      if (us < best * 0.98) best = us, pick(r.kernel);
+    }
+    // 128 x 128: two workgroups to a compute unit
+    const uint64_t t = tiles(128, 128), slots = 2 * (uint64_t)cus, rest = t % slots;
+    const double part = rest == 0 ? 0.0 : rest <= (uint64_t)cus ? 0.50 + 0.12 * (double)rest / cus : 0.62 + 0.38 * (double)(rest - cus) / cus;
+    const double us = kt * ((double)(t / slots) * 1.0 + part) + 4.0 * (double)((t + slots - 1) / slots);
+    if (us < best * 0.98) best = us, pick("128x128x64_q2x2");
+  }
+  // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
+  // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
+  if (!s.own_tile || (ring && tiles(128, 128) < (uint64_t)cus / 2)) {
+    struct StagedTile { const char* kernel; int bm, bn, per_cu; double one, more; };   // us per K tile: alone on a compute unit, and each of several
+    static const StagedTile kStaged[] = {{"staged128x128", 128, 128, 2, 0.75, 0.62}, {"staged64x128", 64, 128, 3, 0.63, 0.38}, {"staged64x64", 64, 64, 4, 0.52, 0.235}};
+    for (const StagedTile& r : kStaged) {
+      if (s.y_cols < r.bn) continue;
+      const uint64_t t = tiles(r.bm, r.bn), sk = r.bm * r.bn == 64 * 64 ? staged_splits(t, s.k, cus) : 1;
+      const double w = (double)((t * sk + cus - 1) / cus);
+      const double us = kt / (double)sk * std::max(r.one * std::max(1.0, w / r.per_cu), r.more * w) + 5.0 +
+                        (sk > 1 ? 6.0 + 8e-6 / 5.0 * (double)(s.m * s.n * (int64_t)sk) : 0.0);
+      if (us < best * 0.98) best = us, pick(r.kernel);
+    }
+  }
+  return c;
+}
+
+}  // namespace cutile

@@ -216,6 +216,20 @@ std::vector<KernelEntry> build_table() {
       add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, (uint32_t)(8 * t[0] * (t[1] + 4) * 4), 0, t[1], 0, t[0], dt, 0, 2);
     }
 
+  // the ring on tiles between 128 x 128 and 256 x 256
+  for (const char* dt : {"bf16", "f16"})
+    for (auto t : {std::array<int, 4>{192, 256, 2, 4}, std::array<int, 4>{128, 256, 2, 4}, std::array<int, 4>{256, 128, 4, 2}, std::array<int, 4>{192, 128, 2, 2}}) {
+      std::string v = std::string(dt) + "_" + std::to_string(t[0]) + "x" + std::to_string(t[1]) + "x64_q" + std::to_string(t[2]) + "x" + std::to_string(t[3]);
+      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * t[3] * 64), (uint32_t)((3 * t[0] * 64 + 2 * 64 * t[1]) * 2), t[0], t[1], 64, 0, dt, 0, 2);
+    }
+  // medium sizes: register-staged tiles, K split over workgroups (any alignment, any partition shape); two LDS stages
+  for (const char* dt : {"bf16", "f16", "bf16f32"})
+    for (auto t : {std::array<int, 3>{64, 64, 4}, std::array<int, 3>{64, 128, 4}, std::array<int, 3>{128, 64, 4}, std::array<int, 3>{128, 128, 4},
+                   std::array<int, 3>{256, 128, 8}}) {
+      std::string v = std::string(dt) + "_staged" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
+      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * 64), (uint32_t)(2 * 64 * 2 * (t[0] + t[1])), 0, t[1], 64, t[0], dt, 0, 2);
+    }
+
   // batched GEMM (cutile-examples/examples/batch_matmul.rs): the pipelined bodies with the batch on a grid axis
   for (const char* kind : {"q", "r"})          // rings of three a stages and two b stages (q: on v_mfma_f32_16x16x32, any K; r: whole K tiles only)
     for (const char* dt : {"bf16", "f16"}) {

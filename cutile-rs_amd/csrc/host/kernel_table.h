@@ -20,7 +20,7 @@ struct KernelEntry {
   Image image;
   uint32_t block[3];
   uint32_t lds_bytes;
-  int32_t tile[4];       // (BM, BN, BK, extra); 0 = not tile-specific; thin GEMM kernels: (0, strip columns, 0, rows)
+  int32_t tile[4];       // (BM, BN, BK, extra); 0 = not tile-specific; gemm_small.hip: (0, columns, K tile or 0, rows)
   const char* dtype;     // element type the variant is written for, or ""
   int64_t capacity;      // row-wise kernels: longest segment held in registers; 0 = n/a
   int32_t rank;          // elementwise kernels: tensor rank; 0 = n/a

@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "common.h"
+#include "gemm_choice.h"
 #include "kernel_table.h"
 #include "runtime_state.h"
 #include "scratch.h"
@@ -254,6 +255,19 @@ cutile_status_t resolve_grid(const cutile_partition_arg_t* out, const cutile_lau
   return cutile_infer_launch_grid(explicit_grid, parts, 1, grid);
 }
 
+cutile_status_t load_resolved(const char* function, const std::string& variant, Resolved* r) {
+  r->entry = find_entry(function, variant);
+  CUTILE_REQUIRE(r->entry, CUTILE_ERR_KERNEL_NOT_FOUND, "no variant '%s' of kernel '%s'; available: %s",
+                 variant.c_str(), function, list_variants(function).c_str());
+  g_last_entry = r->entry;
+  g_last_fn = nullptr;
+  if (g_launch_mode == 2) return CUTILE_SUCCESS;   // specialize-only: the identity is known, nothing is loaded
+  if (cutile_status_t s = current_device(&r->device)) return s;
+  if (cutile_status_t s = load_entry(r->device, r->entry, &r->fn)) return s;
+  g_last_fn = r->fn;
+  return CUTILE_SUCCESS;
+}
+
 // Picks the variant.  Precedence: the caller's variant, the function-wide pin set at run time
 // (cutile_kernel_set_preferred_variant), `sized` (the launcher's own rule for extents that the shape classes of the tuning
 // records do not tell apart), the shape class's winner (a verified tuning record or
@@ -295,16 +309,30 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
     return fail(CUTILE_ERR_KERNEL_NOT_FOUND, "variant '%s' of kernel '%s' does not fit these arguments; fitting: %s",
                 want.c_str(), function, list.c_str());
   }
-  r->entry = find_entry(function, want);
-  CUTILE_REQUIRE(r->entry, CUTILE_ERR_KERNEL_NOT_FOUND, "no variant '%s' of kernel '%s'; available: %s",
-                 want.c_str(), function, list_variants(function).c_str());
-  g_last_entry = r->entry;
-  g_last_fn = nullptr;
-  if (g_launch_mode == 2) return CUTILE_SUCCESS;   // specialize-only: the identity is known, nothing is loaded
-  if (cutile_status_t s = current_device(&r->device)) return s;
-  if (cutile_status_t s = load_entry(r->device, r->entry, &r->fn)) return s;
-  g_last_fn = r->fn;
-  return CUTILE_SUCCESS;
+  return load_resolved(function, want, r);
+}
+
+// Nobody but the launcher has a say (no caller's variant, pin or record) and its choice is known to fit.
+cutile_status_t resolve_own(const char* function, const char* variant, const char* source, Resolved* r) {
+  g_last_source = source;
+  g_last_bucket = g_bucket;
+  return load_resolved(function, variant, r);
+}
+
+// The table's first kernel for a partition's tile shape, or nullptr.
+const KernelEntry* first_of_tile(const char* function, const std::string& dtype, int bm, int bn) {
+  for (const auto& e : kernel_table())
+    if (e.tile[0] == bm && e.tile[1] == bn && strcmp(e.function, function) == 0 && dtype == e.dtype) return &e;
+  return nullptr;
+}
+
+// Compute units of the calling thread's device; 256 (an MI355X) where a specialize-only launch asks without a device.
+cutile_status_t current_device_units(int* cus) {
+  *cus = 256;
+  if (g_launch_mode == 2) return CUTILE_SUCCESS;
+  cutile_device_t device = nullptr;
+  if (cutile_status_t s = current_device(&device)) return s;
+  return compute_units(device, cus);
 }
 
 uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
@@ -315,24 +343,10 @@ bool is_stream_variant(const char* variant) { return strstr(variant, "_s2x4") !=
 uint32_t split_limit(uint64_t blocks, uint64_t floats) {
   return blocks > kSplitCounters ? 1u : (uint32_t)std::max<uint64_t>(1, kSplitPartialBytes / (blocks * floats * sizeof(float)));
 }
-// The thin GEMM kernels: no output tile of their own, tile[1] columns a strip, tile[3] rows in a pass.
-bool is_thin(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
-// The one for `rows` rows of x and an n-column y, or "" where the tiled kernels are the better ones.  Measured at M = 1 to 64,
-// f16 and bf16 (us, thin against the 128 x 128 tiles): 4096 x 4096 10 - 21 against 53, K = 14336 25 - 41 against 175,
-// 14336 x 4096 24 - 35 against 54, 1024 x 1024 5 - 9 against 11.  128-column strips where there are enough of them to keep
-// three quarters of the compute units busy (28672 x 8192, one row: 83 us against 92 with 64-column strips); with more
-// than 32 rows x costs as many bytes as y and that many columns are better off with tiles (129 against 113 us).
-std::string thin_variant(const std::string& dt, int64_t rows, int64_t n, int32_t k) {
-  if (rows > 64 || n < 64 || k <= 64) return "";   // one 64-row step: nothing for the other seven wavefronts to share
-  const bool many = n >= 192 * 128;
-  if (many && rows > 32) return "";
-  return dt + (rows > 32 ? "_thin64x64" : rows > 16 ? "_thin32x64" : many ? "_thin16x128" : "_thin16x64");
-}
-// K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8
-// wavefronts (N = K = 4096, one row: 19.1, 12.6, 10.4, 11.3, 15.4 us with 1, 2, 4, 8, 16 splits; K = 1024: 5.0, 5.3, 5.8, 7.2).
-uint32_t thin_splits(uint64_t blocks, int32_t k, int cus) {
-  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8 * 2)));
-}
+// The GEMM kernels that take any partition shape and any row alignment: tile[3] x tile[1] outputs a workgroup, thin ones
+// (strips of columns) and staged ones (tiles).
+bool is_gemm_small(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
+bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0; }
 // An output of this size or more is read and stored past the caches (it cannot still be cached when its consumer runs,
 // and the caches are left to the operand panels): the rule of the staged epilogue, decided on the host for this family.
 constexpr int64_t kStreamedOutputBytes = 64ll << 20;
@@ -1950,30 +1964,58 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   // running on from tile to tile) take whole tiles in M, N and K only, and at least three K tiles.
   const bool whole_tiles = (int64_t)tg[0] * bm == zt.shape[0] && (int64_t)tg[1] * bn == zt.shape[1] && x->shape[0] >= zt.shape[0] &&
                            y->shape[1] >= zt.shape[1] && k_valid == k_total && k_total % 64 == 0 && k_total >= 192;
-  std::vector<std::string> acceptable;
-  if (fast_layout)
-    for (const auto& e : kernel_table())
-      if (strcmp(e.function, "gemm") == 0 && dt == e.dtype && e.tile[0] == bm && e.tile[1] == bn &&
-          (k_valid % 64 == 0 || strstr(e.variant, "_r") == nullptr) && strchr(e.variant, '+') == nullptr &&
-          (whole_tiles || !is_stream_variant(e.variant)))
-        acceptable.push_back(e.variant);
-  // Few rows: the thin kernels take any partition shape and any row alignment, need rows of unit stride and a strip of
-  // y's columns, and cover 64 rows in a pass (more rows are further passes over y).
-  const bool row_layout = x->strides[1] == 1 && y->strides[1] == 1 && zt.strides[1] == 1 && dt != "f32" && extent_bytes_2d(*x) < kDescriptorLimit &&
-                          extent_bytes_2d(*y) < kDescriptorLimit && extent_bytes_2d(zt) < kDescriptorLimit;
+  uint32_t full[3];
+  cutile_partition_grid(z, full);
+  const bool full_cover = tg[0] == full[0] && tg[1] == full[1];
   const int64_t cover_m = std::min<int64_t>((int64_t)tg[0] * bm, zt.shape[0]), cover_n = std::min<int64_t>((int64_t)tg[1] * bn, zt.shape[1]);
-  const std::string fallback = acceptable.empty() ? dt + "_generic" : acceptable[0];
-  std::string sized;
-  if (row_layout && x->shape[0] > 0 && k_valid > 0) {
-    for (const auto& e : kernel_table())
-      if (is_thin(&e) && strcmp(e.function, "gemm") == 0 && dt == e.dtype && y->shape[1] >= e.tile[1]) acceptable.push_back(e.variant);
-    sized = thin_variant(dt, cover_m, y->shape[1], k_valid);
+  // The kernels of gemm_small.hip take any partition shape and any row alignment; they need rows of unit stride and operands
+  // that reach as far as the output.
+  const bool row_layout = x->strides[1] == 1 && y->strides[1] == 1 && zt.strides[1] == 1 && !in_f32 && x->shape[0] >= cover_m &&
+                          y->shape[1] >= cover_n && k_valid > 0 && extent_bytes_2d(*x) < kDescriptorLimit &&
+                          extent_bytes_2d(*y) < kDescriptorLimit && extent_bytes_2d(zt) < kDescriptorLimit;
+  const KernelEntry* own_tile = fast_layout ? first_of_tile("gemm", dt, bm, bn) : nullptr;   // fits any K: the table's first are not the "_r" and "_s" ones
+  GemmChoice sized;
+  int cus = 256;
+  if (row_layout) {
+    if (cutile_status_t s = current_device_units(&cus)) return s;
+    sized = choose_gemm({dt.c_str(), cover_m, cover_n, y->shape[1], k_valid, fast_layout && full_cover, own_tile != nullptr}, cus);
   }
-  acceptable.push_back(dt + "_generic");
+  // 256 x 256 partitions: the tuning records tell the kernels of that tile apart
+  const bool record_first = bm == 256 && bn == 256 && strstr(sized.variant, "_256x256x64_q2x4") != nullptr;
+  // every kernel that fits these arguments: those of the partition's tile first, then those of other tiles, which compute the
+  // same output when the launch covers all of z
+  auto fitting = [&] {
+    std::vector<std::string> acceptable, others;
+    for (const auto& e : kernel_table()) {
+      if (strcmp(e.function, "gemm") != 0 || dt != e.dtype || strchr(e.variant, '+') != nullptr) continue;
+      if (is_gemm_small(&e)) {
+        if (row_layout && y->shape[1] >= e.tile[1]) others.push_back(e.variant);
+      } else if (e.tile[0] > 0 && fast_layout && (k_valid % 64 == 0 || strstr(e.variant, "_r") == nullptr) && (whole_tiles || !is_stream_variant(e.variant))) {
+        if (e.tile[0] == bm && e.tile[1] == bn)
+          acceptable.push_back(e.variant);
+        else if (full_cover && strstr(e.variant, "x64_q") != nullptr)
+          others.push_back(e.variant);
+      }
+    }
+    acceptable.insert(acceptable.end(), others.begin(), others.end());
+    acceptable.push_back(dt + "_generic");
+    return acceptable;
+  };
   Resolved res;
   // shape class for tuning records: the tile, and whether the tiles fit one wave of workgroups over the 256 CUs
   BucketScope bucket(dt + "_" + std::to_string(bm) + "x" + std::to_string(bn) + ((uint64_t)tg[0] * tg[1] <= 256 ? "|tiles<=256" : "|tiles>256"));
-  if (cutile_status_t s = resolve_entry("gemm", opts, fallback, acceptable, &res, sized)) return s;
+  const std::string fallback = record_first ? sized.variant : own_tile ? own_tile->variant : dt + "_generic";
+  if (record_first) sized.variant[0] = 0;
+  ensure_tuning_records_loaded();
+  if ((opts && opts->variant) || !preferred_variant("gemm").empty() || (!sized.variant[0] && !preferred_variant_for("gemm", g_bucket).empty())) {
+    if (cutile_status_t s = resolve_entry("gemm", opts, fallback, fitting(), &res, sized.variant)) return s;
+  } else if (cutile_status_t s = resolve_own("gemm", sized.variant[0] ? sized.variant : fallback.c_str(), sized.variant[0] ? "size" : "table", &res)) {
+    return s;
+  }
+  if (res.entry->tile[0] > 0 && (res.entry->tile[0] != bm || res.entry->tile[1] != bn)) {   // the kernel's own tiles over the same z
+    tg[0] = div_up(zt.shape[0], res.entry->tile[0]);
+    tg[1] = div_up(zt.shape[1], res.entry->tile[1]);
+  }
   uint32_t stream_grid = 0;
   if (is_stream_variant(res.entry->variant)) {
     if (cutile_status_t s = stream_member(&res, "gemm", accumulate != 0, zt, (uint64_t)tg[0] * tg[1], &stream_grid)) return s;
@@ -1988,23 +2030,31 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   args.push_tensor(*x);
   args.push_tensor(*y);
   args.push_val<int32_t>(k_total);
-  if (is_thin(res.entry)) {
+  if (is_gemm_small(res.entry)) {
     args.push_val<int32_t>((int32_t)cover_m);
     args.push_val<int32_t>((int32_t)cover_n);
     args.push_val<int32_t>(accumulate ? 1 : 0);
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
     SplitWorkspace ws;
-    int cus = 256;
-    if (g_launch_mode != 2)
-      if (cutile_status_t s = compute_units(res.device, &cus)) return s;
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
-    const uint32_t splits = std::min(thin_splits(blocks, k_valid, cus), split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
+    uint32_t splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(blocks, k_valid, cus);
+    splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
       if (cutile_status_t s = split_workspace(res.device, (hipStream_t)stream, &ws)) return s;
-      if (ws.partials) grid[2] = splits;
+      if (!ws.partials) splits = 1;
     }
     args.push_val<void*>(ws.partials);
     args.push_val<void*>(ws.counters);
+    if (is_thin(res.entry)) {
+      grid[2] = splits;
+    } else {
+      args.push_val<uint32_t>(grid[1]);
+      args.push_val<uint32_t>(grid[0]);
+      args.push_val<uint32_t>(splits);
+      CUTILE_REQUIRE(blocks * splits <= 0x7fffffffull, CUTILE_ERR_KERNEL_LAUNCH, "gemm: %llu output tiles do not fit a launch grid axis", (unsigned long long)blocks);
+      grid[0] = (uint32_t)(blocks * splits);
+      grid[1] = 1;
+    }
     return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
   }
   args.push_tile_grid(tg);

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "gemm_common.h"
+#include "gemm_ring16.h"
 #include "kernel_args.h"
 
 using namespace cutile;
@@ -24,6 +25,22 @@ __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t total) 
 // order, whatever order they arrived in, so the sum does not depend on timing.
 __device__ __forceinline__ void store_partial(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float load_partial(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// eight neighbours at once (8-byte aligned)
+__device__ __forceinline__ void store_partials(float* p, const float* f) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p) + i,
+                       (uint64_t)__builtin_bit_cast(uint32_t, f[2 * i]) | (uint64_t)__builtin_bit_cast(uint32_t, f[2 * i + 1]) << 32, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_partials(const float* p, float* f) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    f[2 * i] = __builtin_bit_cast(float, (uint32_t)v);
+    f[2 * i + 1] = __builtin_bit_cast(float, (uint32_t)(v >> 32));
+  }
+}
 // Called by the whole workgroup after its partials are stored: true in the workgroup that arrives last of `splits`.
 __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t splits, uint32_t* shared_flag) {
   __builtin_amdgcn_s_waitcnt(0);   // this wavefront's partials have reached memory
@@ -209,6 +226,227 @@ struct GemmThin {
   }
 };
 
+// ---- medium sizes: register-staged tiles, K split over workgroups -------------------------------------------------------
+// For the outputs that are too few 256 x 256 tiles to fill the chip, and for rows that do not start on 16-byte boundaries
+// (the direct global -> LDS fetches of gemm_bf16.hip cannot take those).  K tiles of 64 go global -> registers -> LDS: two
+// tiles are in flight in registers while a third is multiplied out of one of two LDS stages, so a load has two K tiles to
+// land and one barrier per K tile is enough.  gridDim.z workgroups share the K tiles of an output tile.
+template <int BM, int BN, int WAVES_M, int WAVES_N, typename OutT, typename InT>
+struct GemmStaged {
+  static constexpr int BK = 64, kWaves = WAVES_M * WAVES_N, kThreads = kWaves * 64;
+  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 16, TN = WN / 16;
+  static constexpr int UB = BN / 8;                                    // 16-byte units of a y-tile row
+  static constexpr int kALoads = BM * 8 / kThreads, kBLoads = BK * UB / kThreads;
+  static constexpr int kABytes = BM * BK * 2, kBBytes = BK * BN * 2, kStageBytes = kABytes + kBBytes;
+  static constexpr int kOutRows = 2 * kStageBytes / (BN * 4) < BM ? 2 * kStageBytes / (BN * 4) : BM;   // output rows the stages hold in f32
+  static constexpr int kOutPasses = (BM + kOutRows - 1) / kOutRows;
+  static constexpr int RPW = kOutRows < WM ? kOutRows : WM;
+  static_assert(kALoads * kThreads == BM * 8 && kBLoads * kThreads == BK * UB && UB >= 8, "tile must split evenly");
+  static_assert(kOutRows % WM == 0 || WM % kOutRows == 0, "an output pass takes whole wavefront sub-tiles");
+
+  __device__ static __forceinline__ int a_lds_off(int r, int u) { return r * (BK * 2) + ((u ^ ((r >> 1) & 7)) << 4); }
+  __device__ static __forceinline__ int b_swizzle(int r) { return (((r & 3) << 2) | (((r >> 3) & 1) << 1)) & (UB - 1); }
+  __device__ static __forceinline__ int b_lds_off(int r, int u) { return r * (BN * 2) + ((u ^ b_swizzle(r)) << 4); }
+  __device__ static __forceinline__ u32x4 load16(const unsigned char* p) {   // any 2-byte boundary
+    u32x4 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
+    return v;
+  }
+
+  __device__ static void run(const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y, int32_t k_total, int32_t cover_m,
+                             int32_t cover_n, int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n,
+                             uint32_t splits) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
+    __shared__ uint32_t last;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WAVES_N, wn = wave % WAVES_N, l16 = lane & 15, grp = lane >> 4;
+    // split-major order: an XCD's contiguous share is neighbouring tiles on one range of K
+    const uint32_t tiles = tiles_m * tiles_n, pos = xcd_contiguous(blockIdx.x, tiles * splits), split = pos / tiles, tile = pos % tiles;
+    const uint32_t per_group = kGroupM * tiles_n, first_m = tile / per_group * kGroupM, group_rows = min(tiles_m - first_m, (uint32_t)kGroupM);
+    const uint32_t pm = first_m + tile % per_group % group_rows, pn = tile % per_group / group_rows;
+    const int32_t M = x.shape[0], N = y.shape[1];
+    const int64_t lda = (int64_t)x.strides[0] * 2, ldb = (int64_t)y.strides[0] * 2;   // bytes
+    const int32_t k_valid = min(min(x.shape[1], y.shape[0]), k_total);
+    const int32_t row0 = pm * BM, col_first = pn * BN, col0 = max(0, min(col_first, N - BN));   // the last column of tiles is moved back into y
+    const int32_t full = k_valid / BK, kt0 = (int32_t)((int64_t)full * split / splits), kt1 = (int32_t)((int64_t)full * (split + 1) / splits);
+
+    // per-lane byte offsets of the loads (operands end below 2 GiB; the K advance is scalar) and of the LDS writes
+    static_assert(kThreads % 16 == 0 && kThreads / 8 % 16 == 0 && kThreads / UB % 16 == 0, "the swizzle terms repeat from load to load");
+    const int a_r = tid / 8, b_r = tid / UB, a_k = tid % 8 * 8;
+    uint32_t a_off[kALoads];
+#pragma unroll
+    for (int i = 0; i < kALoads; ++i)   // rows past the end repeat the last one and are not stored
+      a_off[i] = (uint32_t)(min(row0 + a_r + i * (kThreads / 8), M - 1) * lda) + a_k * 2;
+    const uint32_t b_off = (uint32_t)(b_r * ldb) + (uint32_t)(col0 + tid % UB * 8) * 2;
+    const int64_t b_next = kThreads / UB * ldb;
+    const int a_st = a_lds_off(a_r, tid % 8), b_st = kABytes + b_lds_off(b_r, tid % UB);
+    const unsigned char* const xp = (const unsigned char*)x.ptr;
+    const unsigned char* const yp = (const unsigned char*)y.ptr;
+    struct Tile {
+      u32x4 a[kALoads], b[kBLoads];
+    };
+    auto fetch = [&](Tile& t, int32_t kt) {
+      const int32_t k0 = kt * BK;
+#pragma unroll
+      for (int i = 0; i < kALoads; ++i) t.a[i] = load16(xp + (int64_t)k0 * 2 + a_off[i]);
+#pragma unroll
+      for (int i = 0; i < kBLoads; ++i) t.b[i] = load16(yp + k0 * ldb + i * b_next + b_off);
+    };
+    auto stage = [&](const Tile& t, unsigned char* s) {
+#pragma unroll
+      for (int i = 0; i < kALoads; ++i) *reinterpret_cast<u32x4*>(s + a_st + i * (kThreads * 16)) = t.a[i];
+#pragma unroll
+      for (int i = 0; i < kBLoads; ++i) *reinterpret_cast<u32x4*>(s + b_st + i * (kThreads * 16)) = t.b[i];
+    };
+
+    const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4;
+    int a_addr[2], b_addr[TN];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) a_addr[ks] = a_lds_off(wm * WM + l16, ks * 4 + grp);
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      const int n = wn * WN + tn * 16 + tr_col;
+      b_addr[tn] = kABytes + b_lds_off(grp * 8 + tr_row, n >> 3) + (n & 7) * 2;   // rows r, r + 4, r + 32 share their swizzle term
+    }
+    f32x4 acc[TN][TM];
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](const unsigned char* s) {
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        bf16x8 a[TM], b[TN];
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) a[tm] = *reinterpret_cast<const bf16x8*>(s + a_addr[ks] + tm * (16 * BK * 2));
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) {
+          const unsigned char* p = s + b_addr[tn] + ks * 32 * (BN * 2);
+          s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))p);
+          s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(p + 4 * (BN * 2)));
+          b[tn] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = mfma_16x16x32<InT>(b[tn], a[tm], acc[tn][tm]);
+        __builtin_amdgcn_sched_barrier(0);   // one K step's fragments at a time
+      }
+    };
+
+    unsigned char* const s0 = lds;
+    unsigned char* const s1 = lds + kStageBytes;
+    Tile t0, t1;
+    if (kt0 < kt1) {
+      fetch(t0, kt0);
+      if (kt0 + 1 < kt1) fetch(t1, kt0 + 1);
+      stage(t0, s0);
+      if (kt0 + 2 < kt1) fetch(t0, kt0 + 2);
+      __syncthreads();
+    }
+    for (int32_t kt = kt0; kt < kt1; kt += 2) {
+      multiply(s0);
+      if (kt + 1 >= kt1) break;
+      stage(t1, s1);
+      if (kt + 3 < kt1) fetch(t1, kt + 3);
+      __syncthreads();
+      multiply(s1);
+      if (kt + 2 >= kt1) break;
+      stage(t0, s0);
+      if (kt + 4 < kt1) fetch(t0, kt + 4);
+      __syncthreads();
+    }
+
+    // The ragged last K tile, straight into a stage: K positions past the end are 0 on both sides.
+    if (k_valid % BK != 0 && split == splits - 1) {
+      const int32_t k0 = full * BK;
+      __syncthreads();
+#pragma unroll 1
+      for (int c = tid; c < BM * 8; c += kThreads) {
+        const uint16_t* row = reinterpret_cast<const uint16_t*>(xp + (int64_t)min(row0 + c / 8, M - 1) * lda);
+        uint32_t h[4];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int32_t k = k0 + c % 8 * 8 + e;
+          const uint32_t v = k < k_valid ? row[k] : 0u;
+          h[e / 2] = e % 2 ? h[e / 2] | v << 16 : v;
+        }
+        *reinterpret_cast<u32x4*>(s0 + a_lds_off(c / 8, c % 8)) = u32x4{h[0], h[1], h[2], h[3]};
+      }
+#pragma unroll 1
+      for (int c = tid; c < BK * UB; c += kThreads) {
+        const int32_t k = k0 + c / UB;
+        u32x4 v = {0, 0, 0, 0};
+        if (k < k_valid) v = load16(yp + k * ldb + (int64_t)(col0 + c % UB * 8) * 2);
+        *reinterpret_cast<u32x4*>(s0 + kABytes + b_lds_off(c / UB, c % UB)) = v;
+      }
+      __syncthreads();
+      multiply(s0);
+    }
+
+    // Output: a pass puts kOutRows rows of the tile into the stages as f32 (16-byte chunk c of row r at chunk c ^ (r & 15)),
+    // then a thread takes 8 neighbouring columns of a row at a time: 16-byte accesses of z and of the partial sums.
+    OutT* zp = (OutT*)z.ptr;
+    const int32_t ldz = z.strides[0];
+    auto store = [&](int r, int u, const float* v) {
+      const int32_t gr = row0 + r, gc = col0 + u * 8;
+      if (gr >= cover_m || gc >= cover_n) return;
+      OutT* dst = zp + (int64_t)gr * ldz + gc;
+      if (gc >= col_first && gc + 8 <= cover_n) {
+        OutT o[8];
+        if (accumulate) __builtin_memcpy(o, __builtin_assume_aligned(dst, sizeof(OutT)), sizeof(o));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (OutT)(accumulate ? v[e] + (float)o[e] : v[e]);
+        __builtin_memcpy(__builtin_assume_aligned(dst, sizeof(OutT)), o, sizeof(o));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (gc + e >= col_first && gc + e < cover_n) dst[e] = (OutT)(accumulate ? v[e] + (float)dst[e] : v[e]);
+      }
+    };
+    float* mine = partials + (int64_t)tile * splits * (BM * BN);
+    for (int pass = 0; pass < kOutPasses; ++pass) {
+      __syncthreads();   // the stages (or the previous pass) have been read
+      const int first = pass * kOutRows;
+      if (wm * WM < first + kOutRows && first < wm * WM + WM) {
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          const int r = wm * WM + tm * 16 + l16 - first;
+          if (kOutPasses > 1 && (wm * WM + tm * 16 < first || wm * WM + tm * 16 >= first + kOutRows)) continue;
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn)
+            *reinterpret_cast<f32x4*>(lds + r * (BN * 4) + (((wn * (WN / 4) + tn * 4 + grp) ^ (r & 15)) << 4)) = acc[tn][tm];
+        }
+      }
+      __syncthreads();
+      for (int o = tid; o < kOutRows * UB; o += kThreads) {
+        const int r = o / UB, u = o % UB;
+        if (first + r >= BM || row0 + first + r >= cover_m) break;   // rows only grow with o
+        f32x4 v[2] = {*reinterpret_cast<const f32x4*>(lds + r * (BN * 4) + (((2 * u) ^ (r & 15)) << 4)),
+                      *reinterpret_cast<const f32x4*>(lds + r * (BN * 4) + (((2 * u + 1) ^ (r & 15)) << 4))};
+        const float f[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
+        if (splits == 1)
+          store(first + r, u, f);
+        else
+          store_partials(mine + (int64_t)split * (BM * BN) + (first + r) * BN + u * 8, f);
+      }
+    }
+    if (splits == 1 || !last_to_arrive(counters + tile, splits, &last)) return;
+    for (int o = tid; o < BM * UB; o += kThreads) {
+      const int r = o / UB, u = o % UB;
+      if (row0 + r >= cover_m) break;
+      float sum[8] = {};
+      for (uint32_t k = 0; k < splits; ++k) {
+        float f[8];
+        load_partials(mine + (int64_t)k * (BM * BN) + r * BN + u * 8, f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] += f[e];
+      }
+      store(r, u, sum);
+    }
+  }
+};
+
 }  // namespace
 
 #define GEMM_THIN_KERNEL(NAME, IN_T, OUT_T, MB, CPL)                                                                                \
@@ -225,3 +463,34 @@ struct GemmThin {
 GEMM_THIN_FAMILY(bf16, __bf16, __bf16)
 GEMM_THIN_FAMILY(f16, _Float16, _Float16)
 GEMM_THIN_FAMILY(bf16f32, __bf16, float)
+
+#define GEMM_STAGED_KERNEL(NAME, IN_T, OUT_T, BM, BN, WVM, WVN)                                                                     \
+  extern "C" __global__ void __launch_bounds__(WVM * WVN * 64, 2)                                                                   \
+      gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k_total, int32_t cover_m, int32_t cover_n,       \
+                         int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits) { \
+    GemmStaged<BM, BN, WVM, WVN, OUT_T, IN_T>::run(z, x, y, k_total, cover_m, cover_n, accumulate, partials, counters, tiles_m,       \
+                                                   tiles_n, splits);                                                                \
+  }
+#define GEMM_STAGED_FAMILY(T, IN_T, OUT_T)                     \
+  GEMM_STAGED_KERNEL(T##_staged64x64, IN_T, OUT_T, 64, 64, 2, 2)    \
+  GEMM_STAGED_KERNEL(T##_staged64x128, IN_T, OUT_T, 64, 128, 2, 2)  \
+  GEMM_STAGED_KERNEL(T##_staged128x64, IN_T, OUT_T, 128, 64, 2, 2)  \
+  GEMM_STAGED_KERNEL(T##_staged128x128, IN_T, OUT_T, 128, 128, 2, 2) \
+  GEMM_STAGED_KERNEL(T##_staged256x128, IN_T, OUT_T, 256, 128, 4, 2)
+GEMM_STAGED_FAMILY(bf16, __bf16, __bf16)
+GEMM_STAGED_FAMILY(f16, _Float16, _Float16)
+GEMM_STAGED_FAMILY(bf16f32, __bf16, float)
+
+// ---- ring tiles between 128 x 128 and 256 x 256 ---------------------------------------------------------------------------
+#define GEMM_RING_TILE_KERNEL(NAME, BM, BN, WVM, WVN, T)                                                                            \
+  extern "C" __global__ void __launch_bounds__(WVM * WVN * 64)                                                                      \
+      gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k, TileGrid g, int32_t accumulate) {             \
+    GemmRing16<BM, BN, WVM, WVN, T, T>::run(z, x, y, k, g, accumulate);                                                             \
+  }
+#define GEMM_RING_TILE_FAMILY(N, T)                             \
+  GEMM_RING_TILE_KERNEL(N##_192x256x64_q2x4, 192, 256, 2, 4, T) \
+  GEMM_RING_TILE_KERNEL(N##_128x256x64_q2x4, 128, 256, 2, 4, T) \
+  GEMM_RING_TILE_KERNEL(N##_256x128x64_q4x2, 256, 128, 4, 2, T) \
+  GEMM_RING_TILE_KERNEL(N##_192x128x64_q2x2, 192, 128, 2, 2, T)
+GEMM_RING_TILE_FAMILY(bf16, __bf16)
+GEMM_RING_TILE_FAMILY(f16, _Float16)

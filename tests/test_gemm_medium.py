@@ -1,0 +1,64 @@
+"""The GEMM kernels between few rows and 256 x 256 tiles: register-staged tiles (any row alignment, K split over
+workgroups) and the ring on 192 x 256, 128 x 256, 256 x 128 and 192 x 128 tiles."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from util import normal_bf16_bits, normal_f16_bits, rel_l2, to_dev_bf16, to_dev_f16
+
+BOUND = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "bf16f32": 2e-6}      # unit roundoff of the output type (a few outputs can all sit near it); f32 sums
+
+
+def _run(ct, dev, m, n, k, dtype, variant, accumulate, tile=(128, 128)):
+    bits, to_dev = (normal_f16_bits, to_dev_f16) if dtype == "f16" else (normal_bf16_bits, to_dev_bf16)
+    widen = oracle.f16_bits_to_f32 if dtype == "f16" else oracle.bf16_bits_to_f32
+    a, b = bits((m, k), 931), bits((k, n), 932)
+    out = {"bf16": torch.bfloat16, "f16": torch.float16, "bf16f32": torch.float32}[dtype]
+    x, y = to_dev(a, dev), to_dev(b, dev)
+    z0 = torch.from_numpy(oracle.normal_f32((m, n), 933)).to(dev).to(out)
+    z = torch.full((m + 1, n), 7.0, dtype=out, device=dev)           # a row behind z that nothing may touch
+    ref = widen(a).astype(np.float64) @ widen(b).astype(np.float64) + (z0.double().cpu().numpy() if accumulate else 0)
+    for _ in range(2):                                                # the second launch finds the first one's counters at 0
+        z[:m] = z0
+        ct.gemm(ct.partition(z[:m], list(tile)), x, y, k, accumulate=accumulate, generics=[dtype, *tile, 1], variant=variant)
+        torch.cuda.synchronize()
+        assert rel_l2(z[:m].double().cpu().numpy(), ref) <= BOUND[dtype]
+        assert torch.all(z[m] == 7.0)
+    return ct.last_resolved()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", ["64x64", "64x128", "128x128"])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 65), (65, 129, 64), (129, 255, 127), (128, 128, 200), (200, 131, 8), (67, 640, 4100), (130, 1001, 1030)])
+@pytest.mark.parametrize("dtype,accumulate", [("bf16", True), ("f16", False), ("bf16f32", True)])
+def test_gpu_staged_gemm(ct, dev, tile, m, n, k, dtype, accumulate):
+    _run(ct, dev, m, n, k, dtype, f"{dtype}_staged{tile}", accumulate)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", ["192x256x64_q2x4", "128x256x64_q2x4", "256x128x64_q4x2", "192x128x64_q2x2"])
+@pytest.mark.parametrize("m,n,k", [(192, 256, 64), (257, 264, 72), (500, 520, 640), (1, 8, 1032)])
+@pytest.mark.parametrize("dtype,accumulate", [("bf16", True), ("f16", False)])
+def test_gpu_ring_tiles(ct, dev, tile, m, n, k, dtype, accumulate):
+    _run(ct, dev, m, n, k, dtype, f"{dtype}_{tile}", accumulate, tile=(256, 256))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,aligned", [(300, 512, 2048, True), (1500, 1024, 1024, True), (300, 515, 1000, False), (2100, 129, 700, False)])
+def test_gpu_medium_gemm_by_size(ct, dev, m, n, k, aligned):
+    got = _run(ct, dev, m, n, k, "f16", None, True)
+    assert got["source"] == "size" and ("_staged" in got["variant"] or (aligned and "_q" in got["variant"]))
+
+
+def test_rows_of_x_or_columns_of_y_missing_leave_the_size_rule(fake_hip):
+    """x with fewer rows, or y with fewer columns, than the output reads zeros there: the kernels of the size rule do not"""
+    ct = fake_hip
+    h = torch.half
+    z = torch.empty(300, 512, dtype=h)
+    ct.gemm(ct.partition(z, [128, 128]), torch.empty(300, 1001, dtype=h), torch.empty(1001, 512, dtype=h), 1001)
+    assert "_staged" in ct.last_resolved()["variant"]
+    ct.gemm(ct.partition(z, [128, 128]), torch.empty(299, 1001, dtype=h), torch.empty(1001, 512, dtype=h), 1001)
+    assert ct.last_resolved()["variant"] == "f16_generic"
+    ct.gemm(ct.partition(z, [128, 128]), torch.empty(300, 1001, dtype=h), torch.empty(1001, 511, dtype=h), 1001)
+    assert ct.last_resolved()["variant"] == "f16_generic"
