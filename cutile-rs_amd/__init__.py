@@ -345,34 +345,64 @@ def _opts(grid=None, generics=None, variant=None):
     return o, keep
 
 
+_raw_stream = None      # (device) -> handle of torch's current stream there, once torch runs on a GPU
+
+
 def _stream(stream) -> int:
+    global _raw_stream
     if stream is not None:
         return int(stream)
     import torch
 
-    return torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else 0
+    if _raw_stream is None:
+        if not torch.cuda.is_available():
+            return 0
+        torch.cuda.current_stream()      # initialises torch's GPU state; the handle alone is twenty times cheaper to ask for
+        _raw_stream = torch._C._cuda_getCurrentRawStream
+    return _raw_stream(torch._C._cuda_getDevice())
+
+
+_launchers: dict = {}    # entry launchers of the loaded library behind the marshalling extension
+
+
+def _launcher(name: str):
+    if not _launchers:
+        import importlib.util
+
+        path = os.path.join(_HERE, "lib", "cutile_marshal.so")
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: run `python cutile-rs_amd/build.py` (or __graft_entry__.build()) first")
+        import torch  # noqa: F401  (the extension reads its tensors)
+
+        spec = importlib.util.spec_from_file_location("cutile_marshal", path)
+        marshal = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(marshal)
+        _launchers.update({n: marshal.launcher(n, C.cast(getattr(lib(), "cutile_launch_" + n), C.c_void_p).value) for n in marshal.names()})
+    return _launchers[name]
+
+
+def _launch(name: str, *args) -> None:
+    """cutile_launch_<name>: tensors, (tensor, element type), partitions, numbers and (grid, generics, variant) in the order of
+    the C signature"""
+    status = (_launchers.get(name) or _launcher(name))(*args)
+    if status:
+        check(status)
 
 
 # ---- entry launchers (reference argument order) ---------------------------------------------
 def saxpy(y: Partition, a: float, x, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """y <- a*x + y.  cutile-examples/examples/saxpy.rs:12-17."""
-    o, _k = _opts(grid, generics, variant)
-    xa = tensor_arg(x)
-    check(lib().cutile_launch_saxpy(_stream(stream), C.byref(y.arg()), float(a), C.byref(xa), C.byref(o)))
+    _launch("saxpy", _stream(stream), y, float(a), x, (grid, generics, variant))
 
 
 def axpy(z: Partition, a: float, x, y, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """z <- a*x + y (rank 1)."""
-    o, _k = _opts(grid, generics, variant)
-    xa, ya = tensor_arg(x), tensor_arg(y)
-    check(lib().cutile_launch_axpy(_stream(stream), C.byref(z.arg()), float(a), C.byref(xa), C.byref(ya), C.byref(o)))
+    _launch("axpy", _stream(stream), z, float(a), x, y, (grid, generics, variant))
 
 
 def add(z: Partition, x, y, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """z <- x + y.  README.md:29-38 of the reference."""
-    o, _k = _opts(grid, generics, variant)
-    xa, ya = tensor_arg(x), tensor_arg(y)
-    check(lib().cutile_launch_add(_stream(stream), C.byref(z.arg()), C.byref(xa), C.byref(ya), C.byref(o)))
+    _launch("add", _stream(stream), z, x, y, (grid, generics, variant))
 
 
 def full(value, t: Partition, *, stream=None, grid=None, variant=None) -> None:
@@ -393,37 +423,28 @@ def eye(t: Partition, *, stream=None, grid=None, generics=None) -> None:
 
 def relu(input_output: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-examples/examples/async_mlp.rs:56-61: max(0, x) in place over [D] tiles of an f32 vector"""
-    o, _k = _opts(grid, generics, None)
-    check(lib().cutile_launch_relu(_stream(stream), C.byref(input_output.arg()), C.byref(o)))
+    _launch("relu", _stream(stream), input_output, (grid, generics, None))
 
 
 def dropout(p: float, x, x_keep, out: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-examples/examples/dropout.rs:17-32: out = select(x_keep > p, x_keep, 0) / (1 - p); x is never read"""
-    o, _k = _opts(grid, generics, None)
-    xa, ka = tensor_arg(x), tensor_arg(x_keep)
-    check(lib().cutile_launch_dropout(_stream(stream), float(p), C.byref(xa), C.byref(ka), C.byref(out.arg()), C.byref(o)))
+    _launch("dropout", _stream(stream), float(p), x, x_keep, out, (grid, generics, None))
 
 
 def scale_ptr(out_ptr: int, in_ptr: int, scale: float, length: int, *, stream=None, grid=None) -> None:
     """cutile-examples/examples/scale_ptr.rs:26-80: out[i] = in[i] * scale for i < length on raw device pointers (f32);
     the launch grid is required, as for every launcher without a partition argument"""
-    o, _k = _opts(grid, None, None)
-    check(lib().cutile_launch_scale_ptr(_stream(stream), C.c_void_p(out_ptr), C.c_void_p(in_ptr), float(scale), int(length),
-                                        C.byref(o)))
+    _launch("scale_ptr", _stream(stream), int(out_ptr), int(in_ptr), float(scale), int(length), (grid, None, None))
 
 
 def matvec(z: Partition, x, y, k: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-examples/examples/async_mlp.rs:38-54: z[r] += sum_k x[r, k] * y[k] over [BM] tiles of z (f32)"""
-    o, _k = _opts(grid, generics, None)
-    xa, ya = tensor_arg(x), tensor_arg(y)
-    check(lib().cutile_launch_matvec(_stream(stream), C.byref(z.arg()), C.byref(xa), C.byref(ya), int(k), C.byref(o)))
+    _launch("matvec", _stream(stream), z, x, y, int(k), (grid, generics, None))
 
 
 def batch_matmul(c: Partition, a, b, k: int, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-examples/examples/batch_matmul.rs:16-44: c[p] = a[p] . b[p] over [1, BM, BN] tiles of c"""
-    o, _k = _opts(grid, generics, variant)
-    aa, ba = tensor_arg(a), tensor_arg(b)
-    check(lib().cutile_launch_batch_matmul(_stream(stream), C.byref(c.arg()), C.byref(aa), C.byref(ba), int(k), C.byref(o)))
+    _launch("batch_matmul", _stream(stream), c, a, b, int(k), (grid, generics, variant))
 
 
 def linspace(t: Partition, start: float, step: float, *, stream=None, grid=None) -> None:
@@ -432,117 +453,76 @@ def linspace(t: Partition, start: float, step: float, *, stream=None, grid=None)
 
 
 def convert(src, dst: Partition, *, stream=None, grid=None) -> None:
-    o, _k = _opts(grid, None, None)
-    sa = tensor_arg(src)
-    check(lib().cutile_launch_convert(_stream(stream), C.byref(sa), C.byref(dst.arg()), C.byref(o)))
+    _launch("convert", _stream(stream), src, dst, (grid, None, None))
 
 
 def rms_norm_f16(x, w, out: Partition, eps: float, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-kernels/src/norms.rs:16-60."""
-    o, _k = _opts(grid, generics, variant)
-    xa, wa = tensor_arg(x), tensor_arg(w)
-    check(lib().cutile_launch_rms_norm_f16(_stream(stream), C.byref(xa), C.byref(wa), C.byref(out.arg()), float(eps),
-                                           C.byref(o)))
+    _launch("rms_norm_f16", _stream(stream), x, w, out, float(eps), (grid, generics, variant))
 
 
 def rms_norm_f32(x, w, out: Partition, eps: float, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """the f32 example form, cutile-examples/examples/rms_norm.rs:17-61 (square root rounded toward minus infinity)"""
-    o, _k = _opts(grid, generics, variant)
-    xa, wa = tensor_arg(x), tensor_arg(w)
-    check(lib().cutile_launch_rms_norm_f32(_stream(stream), C.byref(xa), C.byref(wa), C.byref(out.arg()), float(eps),
-                                           C.byref(o)))
+    _launch("rms_norm_f32", _stream(stream), x, w, out, float(eps), (grid, generics, variant))
 
 
 def rms_norm_all_f16(x, w, out: Partition, eps: float, *, generics, stream=None, grid=None) -> None:
     """cutile-benchmarks/benches/rmsnorm.rs:20-66: every operation in f16; generics = [N, BLOCK_SIZE]."""
-    o, _k = _opts(grid, generics, None)
-    xa, wa = tensor_arg(x), tensor_arg(w)
-    check(lib().cutile_launch_rms_norm_all_f16(_stream(stream), C.byref(xa), C.byref(wa), C.byref(out.arg()), float(eps),
-                                               C.byref(o)))
+    _launch("rms_norm_all_f16", _stream(stream), x, w, out, float(eps), (grid, generics, None))
 
 
 def softmax_all_f16(x, y: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-benchmarks/benches/softmax.rs:19-35 with its own arithmetic: every operation in f16."""
-    o, _k = _opts(grid, generics, None)
-    xa = tensor_arg(x)
-    check(lib().cutile_launch_softmax_all_f16(_stream(stream), C.byref(xa), C.byref(y.arg()), C.byref(o)))
+    _launch("softmax_all_f16", _stream(stream), x, y, (grid, generics, None))
 
 
 def softmax(x, y: Partition, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-benchmarks/benches/softmax.rs:19-35."""
-    o, _k = _opts(grid, generics, variant)
-    xa = tensor_arg(x)
-    check(lib().cutile_launch_softmax(_stream(stream), C.byref(xa), C.byref(y.arg()), C.byref(o)))
+    _launch("softmax", _stream(stream), x, y, (grid, generics, variant))
 
 
 def add_rms_norm_f16(residual, x, w, out: Partition, residual_out: Partition, eps: float, *, stream=None, grid=None,
                      generics=None, variant=None) -> None:
     """combined = residual + x; out = RMSNorm(combined) * w; residual_out = combined (cutile-kernels norms.rs:68-136)"""
-    ra, xa, wa = tensor_arg(residual), tensor_arg(x), tensor_arg(w)
-    o, keep = _opts(grid, generics, variant)
-    check(lib().cutile_launch_add_rms_norm_f16(_stream(stream), C.byref(ra), C.byref(xa), C.byref(wa), C.byref(out.arg()),
-                                               C.byref(residual_out.arg()), C.c_float(eps), C.byref(o)))
+    _launch("add_rms_norm_f16", _stream(stream), residual, x, w, out, residual_out, float(eps), (grid, generics, variant))
 
 
 def qk_norm_f16(q, k, q_weight, k_weight, out: Partition, eps: float, num_q_rows: int, *, stream=None, grid=None,
                 generics=None, variant=None) -> None:
     """rows < num_q_rows of out: RMSNorm(q) * q_weight; the rest: RMSNorm(k) * k_weight (norms.rs:143-216)"""
-    qa, ka, qw, kw = tensor_arg(q), tensor_arg(k), tensor_arg(q_weight), tensor_arg(k_weight)
-    o, keep = _opts(grid, generics, variant)
-    check(lib().cutile_launch_qk_norm_f16(_stream(stream), C.byref(qa), C.byref(ka), C.byref(qw), C.byref(kw),
-                                          C.byref(out.arg()), C.c_float(eps), int(num_q_rows), C.byref(o)))
+    _launch("qk_norm_f16", _stream(stream), q, k, q_weight, k_weight, out, float(eps), int(num_q_rows), (grid, generics, variant))
 
 
 def add_2d_f16(out: Partition, lhs, rhs, *, stream=None, grid=None, generics=None, variant=None) -> None:
-    la, ra = tensor_arg(lhs), tensor_arg(rhs)
-    o, keep = _opts(grid, generics, variant)
-    check(lib().cutile_launch_add_2d_f16(_stream(stream), C.byref(out.arg()), C.byref(la), C.byref(ra), C.byref(o)))
+    _launch("add_2d_f16", _stream(stream), out, lhs, rhs, (grid, generics, variant))
 
 
 def silu_mul_2d_f16(out: Partition, gate, up, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """out = sigmoid(gate) * gate * up (pointwise.rs:46-78)"""
-    ga, ua = tensor_arg(gate), tensor_arg(up)
-    o, keep = _opts(grid, generics, variant)
-    check(lib().cutile_launch_silu_mul_2d_f16(_stream(stream), C.byref(out.arg()), C.byref(ga), C.byref(ua), C.byref(o)))
+    _launch("silu_mul_2d_f16", _stream(stream), out, gate, up, (grid, generics, variant))
 
 
 def rope_f16(out: Partition, x, inv_freq, position_start=0, *, k=None, num_q_heads: int = 0, stream=None, grid=None,
              generics=None) -> None:
     """Rotary embedding (positional.rs).  `position_start` is an int (rope_seq_f16) or a one-element
     uint32/int32 device tensor (the dynpos forms); with `k`, heads >= num_q_heads of out come from k."""
-    xa, fa = tensor_arg(x), tensor_arg(inv_freq)
-    ka = tensor_arg(k) if k is not None else None
-    pos_dev = None
-    pos = 0
-    if isinstance(position_start, int):
-        pos = position_start
-    else:
-        pos_dev = tensor_arg(position_start, dtype=U32)
-    o, keep = _opts(grid, generics, None)
-    check(lib().cutile_launch_rope_f16(_stream(stream), C.byref(xa), C.byref(ka) if ka is not None else None, C.byref(fa),
-                                       C.byref(pos_dev) if pos_dev is not None else None, int(pos), C.byref(out.arg()),
-                                       int(num_q_heads), C.byref(o)))
+    by_value = isinstance(position_start, int)
+    _launch("rope_f16", _stream(stream), x, k, inv_freq, None if by_value else (position_start, U32), position_start if by_value else 0, out,
+            int(num_q_heads), (grid, generics, None))
 
 
 def kv_cache_update_f16(new_k, new_v, k_cache: Partition, v_cache: Partition, position_start, seq_len: int, *, stream=None,
                         grid=None, generics=None) -> None:
     """cache[h, position_start + s] = new[s, h] (kv_cache.rs); position_start: int or one-element device tensor"""
-    ka, va = tensor_arg(new_k), tensor_arg(new_v)
-    pos_dev, pos = (None, int(position_start)) if isinstance(position_start, int) else (tensor_arg(position_start, dtype=U32), 0)
-    o, keep = _opts(grid, generics, None)
-    check(lib().cutile_launch_kv_cache_update_f16(_stream(stream), C.byref(ka), C.byref(va), C.byref(k_cache.arg()),
-                                                  C.byref(v_cache.arg()), C.byref(pos_dev) if pos_dev is not None else None,
-                                                  pos, int(seq_len), C.byref(o)))
+    by_value = isinstance(position_start, int)
+    _launch("kv_cache_update_f16", _stream(stream), new_k, new_v, k_cache, v_cache, None if by_value else (position_start, U32),
+            position_start if by_value else 0, int(seq_len), (grid, generics, None))
 
 
 def fmha_decode_gqa_split(q, k, v, att_out: Partition, lse_out: Partition, qk_scale: float, position_start, *, stream=None,
                           grid=None, generics=None, variant=None) -> None:
     """split-KV decode attention (attention.rs:737-902); position_start: one-element device tensor"""
-    qa, ka, va, pa = tensor_arg(q), tensor_arg(k), tensor_arg(v), tensor_arg(position_start, dtype=U32)
-    o, keep = _opts(grid, generics, variant)
-    check(lib().cutile_launch_fmha_decode_gqa_split(_stream(stream), C.byref(qa), C.byref(ka), C.byref(va),
-                                                    C.byref(att_out.arg()), C.byref(lse_out.arg()), C.c_float(qk_scale),
-                                                    C.byref(pa), C.byref(o)))
+    _launch("fmha_decode_gqa_split", _stream(stream), q, k, v, att_out, lse_out, float(qk_scale), (position_start, U32), (grid, generics, variant))
 
 
 def attention_decode_kernel_grouped_f16(q, k, v, att, lse, softmax_scale: float, s_kv, *, tile_n: int = 64,
@@ -553,28 +533,21 @@ def attention_decode_kernel_grouped_f16(q, k, v, att, lse, softmax_scale: float,
     def group(t, rank):
         if t.dim() != rank or t.stride(-1) != 1:
             raise ValueError(f"attention_decode_kernel_grouped: expected rank {rank} with unit innermost stride")
-        return (C.c_void_p(t.data_ptr()), (C.c_int32 * rank)(*t.shape), (C.c_int32 * (rank - 1))(*t.stride()[:-1]))
-    o, keep = _opts(grid, generics, None)
+        return t.data_ptr(), tuple(t.shape), t.stride()[:-1]
     qgts = int(query_group_tile_size) if query_group_tile_size is not None else max(int(q.shape[2]), 1)
-    check(lib().cutile_launch_attention_decode_kernel_grouped_f16(
-        _stream(stream), *group(q, 4), *group(k, 4), *group(v, 4), *group(att, 5), *group(lse, 4), C.c_float(softmax_scale),
-        C.c_void_p(s_kv.data_ptr()), int(tile_n), int(kv_len_per_split), qgts, C.byref(o)))
+    _launch("attention_decode_kernel_grouped_f16", _stream(stream), *group(q, 4), *group(k, 4), *group(v, 4), *group(att, 5), *group(lse, 4),
+            float(softmax_scale), s_kv.data_ptr(), int(tile_n), int(kv_len_per_split), qgts, (grid, generics, None))
 
 
 def splitk_reduce_merge(att_partial, lse_partial, out: Partition, *, stream=None, grid=None, generics=None) -> None:
-    aa, la = tensor_arg(att_partial), tensor_arg(lse_partial)
-    o, keep = _opts(grid, generics, None)
-    check(lib().cutile_launch_splitk_reduce_merge(_stream(stream), C.byref(aa), C.byref(la), C.byref(out.arg()), C.byref(o)))
+    _launch("splitk_reduce_merge", _stream(stream), att_partial, lse_partial, out, (grid, generics, None))
 
 
 def fmha_decode_gqa_noalloc(q, k, v, out: Partition, qk_scale: float, position_start, num_kv_splits: int, bn: int = 64, *,
                             stream=None) -> None:
     """split-KV decode attention and merge in one call that allocates nothing: the partial results live in the
     library's device-resident scratch array (8 MiB per GPU); position_start: one-element device tensor"""
-    qa, ka, va, pa = tensor_arg(q), tensor_arg(k), tensor_arg(v), tensor_arg(position_start, dtype=U32)
-    check(lib().cutile_launch_fmha_decode_gqa_noalloc(_stream(stream), C.byref(qa), C.byref(ka), C.byref(va),
-                                                      C.byref(out.arg()), C.c_float(qk_scale), C.byref(pa),
-                                                      int(num_kv_splits), int(bn)))
+    _launch("fmha_decode_gqa_noalloc", _stream(stream), q, k, v, out, float(qk_scale), (position_start, U32), int(num_kv_splits), int(bn))
 
 
 def fmha_decode_gqa_noalloc_prepare(q, k, v, out: Partition, position_start, num_kv_splits: int, bn: int = 64) -> None:
@@ -594,10 +567,7 @@ def scratch_capacity() -> int:
 def gemm(z: Partition, x, y, k: int, *, accumulate: bool = True, stream=None, grid=None, generics=None,
          variant=None) -> None:
     """cutile-benchmarks/benches/gemm.rs:20-41 (z is read as the initial accumulator)."""
-    o, _k = _opts(grid, generics, variant)
-    xa, ya = tensor_arg(x), tensor_arg(y)
-    check(lib().cutile_launch_gemm(_stream(stream), C.byref(z.arg()), C.byref(xa), C.byref(ya), int(k),
-                                   int(accumulate), C.byref(o)))
+    _launch("gemm", _stream(stream), z, x, y, int(k), int(accumulate), (grid, generics, variant))
 
 
 def gemm_persistent(z: MappedPartition, x, y, *, stream=None, grid=None, generics=None, variant=None) -> None:
@@ -658,10 +628,7 @@ def mapped_tile_index(z: MappedPartition, *, stream=None, grid=None) -> None:
 def fmha(out: Partition, q, k, v, qk_scale: float, input_pos: int = 0, query_group_size: int = 1, *,
          causal: bool = False, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-examples/examples/flash_attention_causal.rs:19-134."""
-    o, _k = _opts(grid, generics, variant)
-    qa, ka, va = tensor_arg(q), tensor_arg(k), tensor_arg(v)
-    check(lib().cutile_launch_fmha(_stream(stream), C.byref(out.arg()), C.byref(qa), C.byref(ka), C.byref(va),
-                                   float(qk_scale), int(input_pos), int(query_group_size), int(causal), C.byref(o)))
+    _launch("fmha", _stream(stream), out, q, k, v, float(qk_scale), int(input_pos), int(query_group_size), int(causal), (grid, generics, variant))
 
 
 KVBM_STACKED_NHD, KVBM_STACKED_HND = 0, 1
@@ -681,87 +648,65 @@ def kvbm_copy_f16(to_stacked: bool, stacked_layout: int, contiguous_layout: int,
 
 def add_rms_norm_decode_raw_f16(residual, x, w, out, residual_out, eps: float, *, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/norms.rs:22-153: one row of N halves, the tensors' addresses passed as raw pointers"""
-    o, _k = _opts(None, generics, None)
-    check(lib().cutile_launch_add_rms_norm_decode_raw_f16(_stream(stream), *[C.c_void_p(t.data_ptr()) for t in (residual, x, w, out, residual_out)],
-                                                          C.c_float(eps), int(w.numel()), C.byref(o)))
+    _launch("add_rms_norm_decode_raw_f16", _stream(stream), *[t.data_ptr() for t in (residual, x, w, out, residual_out)], float(eps), int(w.numel()),
+            (None, generics, None))
 
 
 def qk_norm_rope_kv_prefill_raw_f16(q, k, v, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache, eps: float, position_start: int,
                                     seq_len: int, *, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/fused_transformer.rs:22-345; the reference takes raw pointers, this wrapper takes the
     contiguous tensors q [seq, q_heads, D], k / v [seq, kv_heads, D], caches [kv_heads, MAX_SEQ, D] and passes their addresses"""
-    o, _k = _opts(None, generics, None)
-    for t in (q, k, v, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache):
+    tensors = (q, k, v, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache)
+    for t in tensors:
         if not t.is_contiguous():
             raise CutileError(-5, "qk_norm_rope_kv_prefill_raw_f16: raw-pointer kernel, every tensor must be contiguous")
-    check(lib().cutile_launch_qk_norm_rope_kv_prefill_raw_f16(
-        _stream(stream), *[C.c_void_p(t.data_ptr()) for t in (q, k, v, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache)],
-        C.c_float(eps), int(position_start), int(seq_len), int(q.shape[1]), int(k.shape[1]), int(q.shape[2]), int(k_cache.shape[1]),
-        C.byref(o)))
+    _launch("qk_norm_rope_kv_prefill_raw_f16", _stream(stream), *[t.data_ptr() for t in tensors], float(eps), int(position_start), int(seq_len),
+            int(q.shape[1]), int(k.shape[1]), int(q.shape[2]), int(k_cache.shape[1]), (None, generics, None))
 
 
 def qk_norm_rope_kv_decode_raw_f16(qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache, position_start, eps: float,
                                    num_q_heads: int, num_kv_heads: int, *, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/fused_transformer.rs:356-625; qkv: one token's q, k and v heads back to back"""
-    o, _k = _opts(None, generics, None)
-    pa = tensor_arg(position_start, dtype=U32)
-    d = int(k_cache.shape[2])
-    check(lib().cutile_launch_qk_norm_rope_kv_decode_raw_f16(
-        _stream(stream), *[C.c_void_p(t.data_ptr()) for t in (qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache)],
-        C.byref(pa), C.c_float(eps), int(num_q_heads), int(num_kv_heads), d, int(k_cache.shape[1]), C.byref(o)))
+    _launch("qk_norm_rope_kv_decode_raw_f16", _stream(stream), *[t.data_ptr() for t in (qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache)],
+            (position_start, U32), float(eps), int(num_q_heads), int(num_kv_heads), int(k_cache.shape[2]), int(k_cache.shape[1]), (None, generics, None))
 
 
 def group_gemm_f16_nt_desc(a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, num_groups: int, *, stream=None, grid=None,
                            generics=None, variant=None) -> None:
     """cutile-kernels/src/experimental/moe.rs:67-128: pointer tables (int64) and descriptor tables (int32 [groups, 8]:
     rows, cols, row stride) in device memory; generics [BM, BN, BK, NUM_SM]"""
-    o, _k = _opts(grid, generics, variant)
-    t = [tensor_arg(x) for x in (a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas)]
-    check(lib().cutile_launch_group_gemm_f16_nt_desc(_stream(stream), *[C.byref(x) for x in t], int(num_groups), C.byref(o)))
+    _launch("group_gemm_f16_nt_desc", _stream(stream), a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, int(num_groups), (grid, generics, variant))
 
 
-def _u32_partition(p: Partition) -> PartitionArg:
-    """the argument record of a partition of u32 values held in an int32 / uint32 tensor"""
-    return (p if p.dtype is not None else Partition(p.tensor, p.shape, p.prefix, U32)).arg()
+def _u32_partition(p: Partition) -> Partition:
+    """a partition of u32 values held in an int32 / uint32 tensor"""
+    return p if p.dtype is not None else Partition(p.tensor, p.shape, p.prefix, U32)
 
 
 def argmax_blocks_f16(logits, block_max: Partition, block_idx: Partition, length: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/argmax.rs:21-71; block_idx: an int32 / uint32 tensor of u32 indices"""
-    o, _k = _opts(grid, generics, None)
-    la = tensor_arg(logits)
-    check(lib().cutile_launch_argmax_blocks_f16(_stream(stream), C.byref(la), C.byref(block_max.arg()), C.byref(_u32_partition(block_idx)),
-                                                int(length), C.byref(o)))
+    _launch("argmax_blocks_f16", _stream(stream), logits, block_max, _u32_partition(block_idx), int(length), (grid, generics, None))
 
 
 def lm_head_argmax_blocks_f16(weights, hidden, block_max: Partition, block_idx: Partition, vocab_size: int, *, stream=None,
                               grid=None, generics=None) -> None:
     """cutile-kernels/src/argmax.rs:88-158"""
-    o, _k = _opts(grid, generics, None)
-    wa, ha = tensor_arg(weights), tensor_arg(hidden)
-    check(lib().cutile_launch_lm_head_argmax_blocks_f16(_stream(stream), C.byref(wa), C.byref(ha), C.byref(block_max.arg()),
-                                                        C.byref(_u32_partition(block_idx)), int(vocab_size), C.byref(o)))
+    _launch("lm_head_argmax_blocks_f16", _stream(stream), weights, hidden, block_max, _u32_partition(block_idx), int(vocab_size), (grid, generics, None))
 
 
 def argmax_reduce_blocks_to_u32(block_max, block_idx, out: Partition, num_blocks: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/argmax.rs:173-213"""
-    o, _k = _opts(grid, generics, None)
-    ma, ia = tensor_arg(block_max), tensor_arg(block_idx, dtype=U32)
-    check(lib().cutile_launch_argmax_reduce_blocks_to_u32(_stream(stream), C.byref(ma), C.byref(ia), C.byref(_u32_partition(out)),
-                                                          int(num_blocks), C.byref(o)))
+    _launch("argmax_reduce_blocks_to_u32", _stream(stream), block_max, (block_idx, U32), _u32_partition(out), int(num_blocks), (grid, generics, None))
 
 
 def embedding_batch_f16(token_ids, table, out: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/embeddings.rs:21-41; token_ids: an int32 / uint32 tensor of u32 ids"""
-    o, _k = _opts(grid, generics, None)
-    ia, ta = tensor_arg(token_ids, dtype=U32), tensor_arg(table)
-    check(lib().cutile_launch_embedding_batch_f16(_stream(stream), C.byref(ia), C.byref(ta), C.byref(out.arg()), C.byref(o)))
+    _launch("embedding_batch_f16", _stream(stream), (token_ids, U32), table, out, (grid, generics, None))
 
 
 def gather_row_f16(src, out: Partition, row_idx: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/pointwise.rs:86-99"""
-    o, _k = _opts(grid, generics, None)
-    sa = tensor_arg(src)
-    check(lib().cutile_launch_gather_row_f16(_stream(stream), C.byref(sa), C.byref(out.arg()), int(row_idx), C.byref(o)))
+    _launch("gather_row_f16", _stream(stream), src, out, int(row_idx), (grid, generics, None))
 
 
 def fmha_seq_f16(q, k, v, out: Partition, qk_scale: float, query_group_size: int, *, kv_len: int = 0, query_start: int = 0,
@@ -773,45 +718,32 @@ def fmha_seq_f16(q, k, v, out: Partition, qk_scale: float, query_group_size: int
       flash_attn_causal_seq_dynpos_f16 (:128-231) position_start (one u32 on the device), kv_len_from_position
       fmha_prefill_causal (:242-391), fmha_prefill_gqa (:408-587)   kv_len, query_start by value, causal or not
       fmha_causal (:598-726)                      position_start, every key of k"""
-    o, _k = _opts(grid, generics, variant)
-    qa, ka, va = tensor_arg(q), tensor_arg(k), tensor_arg(v)
-    pa = tensor_arg(position_start, dtype=U32) if position_start is not None else None
-    check(lib().cutile_launch_fmha_seq_f16(_stream(stream), C.byref(qa), C.byref(ka), C.byref(va), C.byref(out.arg()),
-                                           C.c_float(qk_scale), int(query_group_size), int(kv_len), int(query_start),
-                                           C.byref(pa) if pa is not None else None, int(kv_len_from_position), int(causal),
-                                           C.byref(o)))
+    _launch("fmha_seq_f16", _stream(stream), q, k, v, out, float(qk_scale), int(query_group_size), int(kv_len), int(query_start),
+            (position_start, U32) if position_start is not None else None, int(kv_len_from_position), int(causal), (grid, generics, variant))
 
 
 def fmha_prefill_gqa_lpt_raw_f16(q, k, v, out, qk_scale: float, query_group_size: int, kv_len: int, query_start: int, group: int, *,
                                  causal: bool = True, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/attention.rs:22-377; contiguous q / out [q_len, q_heads, D] and k / v [kv_heads, kv_len, D]
     passed as raw addresses"""
-    o, _k = _opts(None, generics, None)
-    check(lib().cutile_launch_fmha_prefill_gqa_lpt_raw_f16(
-        _stream(stream), *[C.c_void_p(t.data_ptr()) for t in (q, k, v, out)], C.c_float(qk_scale), int(query_group_size), int(q.shape[0]),
-        int(kv_len), int(query_start), int(q.shape[1]) // int(group), int(group), int(q.shape[2]), int(causal), C.byref(o)))
+    _launch("fmha_prefill_gqa_lpt_raw_f16", _stream(stream), *[t.data_ptr() for t in (q, k, v, out)], float(qk_scale), int(query_group_size),
+            int(q.shape[0]), int(kv_len), int(query_start), int(q.shape[1]) // int(group), int(group), int(q.shape[2]), int(causal), (None, generics, None))
 
 
 def linear_tile_mxfp8(z: Partition, x, y, x_scales, y_scales, alpha: float = 1.0, *, stream=None, grid=None,
                       generics=None, variant=None) -> None:
     """cutile-examples/examples/mxfp8.rs:34-64.  x, y: uint8 (or float8_e4m3fn) tensors of
     e4m3fn bytes; scales: uint8 (or float8_e8m0fnu) tensors of e8m0 bytes."""
-    o, _k = _opts(grid, generics, variant)
-    xa, ya = tensor_arg(x, F8E4M3FN), tensor_arg(y, F8E4M3FN)
-    xsa, ysa = tensor_arg(x_scales, F8E8M0FNU), tensor_arg(y_scales, F8E8M0FNU)
-    check(lib().cutile_launch_linear_tile_mxfp8(_stream(stream), C.byref(z.arg()), C.byref(xa), C.byref(ya),
-                                                C.byref(xsa), C.byref(ysa), float(alpha), C.byref(o)))
+    _launch("linear_tile_mxfp8", _stream(stream), z, (x, F8E4M3FN), (y, F8E4M3FN), (x_scales, F8E8M0FNU), (y_scales, F8E8M0FNU), float(alpha),
+            (grid, generics, variant))
 
 
 def linear_tile_nvfp4(z: Partition, x, y, x_scales, y_scales, alpha: float = 1.0, *, stream=None, grid=None,
                       generics=None, variant=None) -> None:
     """cutile-examples/examples/nvfp4.rs:24-78.  x [M, K/2], y [N, K/2]: uint8 tensors of packed e2m1 pairs (low
     nibble first); scales [M, K/16], [N, K/16]: uint8 (or float8_e4m3fn) tensors of e4m3fn bytes; z f32 or bf16."""
-    o, _k = _opts(grid, generics, variant)
-    xa, ya = tensor_arg(x, F4E2M1FNX2), tensor_arg(y, F4E2M1FNX2)
-    xsa, ysa = tensor_arg(x_scales, F8E4M3FN), tensor_arg(y_scales, F8E4M3FN)
-    check(lib().cutile_launch_linear_tile_nvfp4(_stream(stream), C.byref(z.arg()), C.byref(xa), C.byref(ya),
-                                                C.byref(xsa), C.byref(ysa), float(alpha), C.byref(o)))
+    _launch("linear_tile_nvfp4", _stream(stream), z, (x, F4E2M1FNX2), (y, F4E2M1FNX2), (x_scales, F8E4M3FN), (y_scales, F8E4M3FN), float(alpha),
+            (grid, generics, variant))
 
 
 # ---- table / device helpers -------------------------------------------------------------------

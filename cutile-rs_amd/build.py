@@ -153,6 +153,24 @@ def build_scratch_library(force: bool = False) -> str:
     return SCRATCH_LIB_PATH
 
 
+MARSHAL_PATH = os.path.join(LIB_DIR, "cutile_marshal.so")
+
+
+def build_marshal(force: bool = False) -> str:
+    """The CPython extension that reads torch tensors into the ABI's records for the Python binding (host code only)."""
+    src = os.path.join(ROOT, "csrc", "bind", "marshal.cpp")
+    header = os.path.join(ROOT, "..", "include", "cutile_hip.h")
+    if force or not _newer(MARSHAL_PATH, [src, header]):
+        import sysconfig
+
+        import torch
+        inc, libs = (os.path.join(os.path.dirname(torch.__file__), d) for d in ("include", "lib"))
+        _run([CXX, "-std=c++17", "-O2", "-g0", "-fPIC", "-shared", "-w", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+              "-I" + sysconfig.get_paths()["include"], "-I" + inc, "-I" + os.path.join(inc, "torch", "csrc", "api", "include"), src, "-o", MARSHAL_PATH,
+              "-L" + libs, "-ltorch_python", "-ltorch_cpu", "-lc10"])   # found by name: torch has loaded them
+    return MARSHAL_PATH
+
+
 CPP_TEST_DIR = os.path.join(ROOT, "..", "tests", "cpp")
 CPP_TESTS = {
     # binary -> (source, library it links: True = the product library, "testing" = the one with the recording runtime, extra flags)
@@ -218,6 +236,7 @@ def build(force: bool = False) -> str:
     build_tuner(force)
     build_scratch_library(force)
     build_probes(force)
+    build_marshal(force)
     build_cpp_tests(force)
     return lib
 

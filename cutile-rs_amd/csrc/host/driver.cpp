@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "common.h"
+#include "kernel_table.h"
 #include "runtime_state.h"
 
 using namespace cutile;
@@ -23,6 +24,9 @@ namespace cutile {
 namespace {
 std::mutex g_devices_mutex;
 std::map<int, std::unique_ptr<cutile_device>> g_devices;
+// Devices handed out before, by ordinal, readable without the mutex: a launch asks for the current one every time.
+constexpr int kKnownDevices = 64;
+std::atomic<cutile_device*> g_known_devices[kKnownDevices];
 std::once_flag g_init_once;
 cutile_status_t g_init_status = CUTILE_SUCCESS;
 std::string g_init_error;
@@ -40,7 +44,12 @@ cutile_status_t ensure_init() {
 void reset_runtime_for_testing() {
   reset_async_runtime_for_testing();
   std::lock_guard<std::mutex> lock(g_devices_mutex);
+  for (auto& d : g_known_devices) d = nullptr;
   g_devices.clear();
+}
+
+cutile_device_t known_device(int ordinal) {
+  return ordinal >= 0 && ordinal < kKnownDevices ? g_known_devices[ordinal].load(std::memory_order_acquire) : nullptr;
 }
 
 }  // namespace cutile
@@ -71,9 +80,11 @@ cutile_status_t cutile_device_get(int32_t ordinal, cutile_device_t* device) {
   if (it == g_devices.end()) {
     auto d = std::make_unique<cutile_device>();
     d->ordinal = ordinal;
+    d->function_slots.reset(new std::atomic<hipFunction_t>[kernel_table().size()]());
     it = g_devices.emplace(ordinal, std::move(d)).first;
   }
   *device = it->second.get();
+  if (ordinal < kKnownDevices) g_known_devices[ordinal].store(*device, std::memory_order_release);
   return CUTILE_SUCCESS;
 }
 

@@ -9,6 +9,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <string_view>
 #include <unordered_map>
 
 // Code objects, embedded by embed.S (one ELF image per kernel source file).
@@ -29,6 +30,7 @@ namespace {
 std::atomic<uint64_t> g_module_loads{0};
 std::mutex g_pref_mutex;
 std::map<std::string, std::string> g_preferred;
+std::atomic<size_t> g_preferred_count{0};
 // winners of tuning records: "function|bucket" -> variant
 std::map<std::string, std::string> g_bucket_preferred;
 
@@ -384,6 +386,17 @@ const std::vector<KernelEntry>& kernel_table() {
   return table;
 }
 
+const std::vector<const KernelEntry*>& kernels_of(const char* function) {
+  static const auto& index = *[] {
+    auto* m = new std::unordered_map<std::string_view, std::vector<const KernelEntry*>>();
+    for (const auto& e : kernel_table()) (*m)[e.function].push_back(&e);
+    return m;
+  }();
+  static const std::vector<const KernelEntry*> none;
+  auto it = index.find(function);
+  return it == index.end() ? none : it->second;
+}
+
 // (function, variant) -> entry.  Every launch looks its kernel up at least once, so the table is indexed once
 // (the first entry of a key wins, as a scan in table order would find it).
 const KernelEntry* find_entry(const char* function, const std::string& variant) {
@@ -411,6 +424,7 @@ std::string list_variants(const char* function) {
 }
 
 std::string preferred_variant(const char* function) {
+  if (g_preferred_count.load(std::memory_order_acquire) == 0) return std::string();   // the usual case: nothing is pinned
   std::lock_guard<std::mutex> lock(g_pref_mutex);
   auto it = g_preferred.find(function);
   return it == g_preferred.end() ? std::string() : it->second;
@@ -432,12 +446,21 @@ void count_module_load() { g_module_loads.fetch_add(1, std::memory_order_relaxed
 
 cutile_status_t load_entry(cutile_device_t device, const KernelEntry* entry, hipFunction_t* fn) {
   CUTILE_REQUIRE(device && entry && fn, CUTILE_ERR_INVALID_ARGUMENT, "null argument");
+  // Functions resolved before are read without the lock.
+  const size_t slot = (size_t)(entry - kernel_table().data());
+  if (device->function_slots) {
+    if (hipFunction_t known = device->function_slots[slot].load(std::memory_order_acquire)) {
+      *fn = known;
+      return CUTILE_SUCCESS;
+    }
+  }
   // The device mutex makes the load single-flight: concurrent first launches of
   // one kernel load its code object once (tile_kernel.rs:371-399,705-733).
   std::lock_guard<std::mutex> lock(device->mutex);
   auto fit = device->functions.find(entry->symbol);
   if (fit != device->functions.end()) {
     *fn = fit->second;
+    device->function_slots[slot].store(*fn, std::memory_order_release);
     return CUTILE_SUCCESS;
   }
   CUTILE_API_OR_RETURN(api);
@@ -461,6 +484,7 @@ cutile_status_t load_entry(cutile_device_t device, const KernelEntry* entry, hip
   hipFunction_t f = nullptr;
   CUTILE_HIP_OR_RETURN(api, hipModuleGetFunction(&f, mod->handle, entry->symbol));
   device->functions[entry->symbol] = f;
+  device->function_slots[slot].store(f, std::memory_order_release);
   *fn = f;
   return CUTILE_SUCCESS;
 }
@@ -488,12 +512,14 @@ cutile_status_t cutile_kernel_set_preferred_variant(const char* function, const 
   std::lock_guard<std::mutex> lock(g_pref_mutex);
   if (!variant) {
     g_preferred.erase(function);
+    g_preferred_count = g_preferred.size();
     return CUTILE_SUCCESS;
   }
   CUTILE_REQUIRE(find_entry(function, variant) != nullptr, CUTILE_ERR_KERNEL_NOT_FOUND,
                  "no variant '%s' of kernel '%s'; available: %s", variant, function,
                  list_variants(function).c_str());
   g_preferred[function] = variant;
+  g_preferred_count = g_preferred.size();
   return CUTILE_SUCCESS;
 }
 

@@ -28,6 +28,8 @@ struct KernelEntry {
 
 const std::vector<KernelEntry>& kernel_table();
 
+// The entries of one function, in table order; empty if there are none.
+const std::vector<const KernelEntry*>& kernels_of(const char* function);
 // Finds the entry (function, variant); nullptr if absent.
 const KernelEntry* find_entry(const char* function, const std::string& variant);
 // Resolves the entry's hipFunction_t on `device`, loading its code object on

@@ -34,17 +34,17 @@ using namespace cutile;
 namespace cutile {
 
 cutile_status_t current_device(cutile_device_t* device) {
-  if (cutile_status_t s = ensure_init()) return s;
   CUTILE_API_OR_RETURN(api);
   int ord = 0;
+  if (api->hipGetDevice(&ord) == hipSuccess && (*device = known_device(ord))) return CUTILE_SUCCESS;
+  if (cutile_status_t s = ensure_init()) return s;
   CUTILE_HIP_OR_RETURN(api, hipGetDevice(&ord));
   return cutile_device_get(ord, device);
 }
 
 cutile_status_t compute_units(cutile_device_t device, int* count) {
   CUTILE_REQUIRE(device && count, CUTILE_ERR_INVALID_ARGUMENT, "null argument");
-  std::lock_guard<std::mutex> lock(device->mutex);
-  if (device->compute_units <= 0) {
+  if (device->compute_units.load(std::memory_order_relaxed) <= 0) {
     CUTILE_API_OR_RETURN(api);
     int v = 0;
     CUTILE_HIP_OR_RETURN(api, hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device->ordinal));
@@ -112,11 +112,19 @@ size_t scalar_bits(cutile_dtype_t dt, double v, int64_t iv, unsigned char out[8]
 // Kernel-argument buffer laid out like the kernarg segment: every value at its
 // natural alignment, in push order.
 struct ArgPacker {
-  std::vector<unsigned char> buf;
+  unsigned char small[512];             // every entry launcher's list (two partitions, four tensors and scalars take less than 400 bytes)
+  std::vector<unsigned char> large;     // a longer list of a user's own kernel
+  size_t used = 0;
+  unsigned char* data() { return large.empty() ? small : large.data(); }
   void push(const void* v, size_t size, size_t align) {
-    size_t off = (buf.size() + align - 1) / align * align;
-    buf.resize(off + size);
-    memcpy(buf.data() + off, v, size);
+    const size_t off = (used + align - 1) / align * align;
+    if (off + size > sizeof(small)) {
+      if (large.empty()) large.assign(small, small + used);
+      large.resize(off + size);
+    }
+    memset(data() + used, 0, off - used);
+    memcpy(data() + off, v, size);
+    used = off + size;
   }
   template <typename T>
   void push_val(T v) { push(&v, sizeof(T), alignof(T)); }
@@ -166,8 +174,8 @@ cutile_status_t launch_packed(hipFunction_t fn, const uint32_t grid[3], const ui
   CUTILE_REQUIRE(grid[0] <= 0x7fffffffu && grid[1] <= 65535u && grid[2] <= 65535u &&
                      (uint64_t)grid[0] * block[0] <= 0xffffffffull,
                  CUTILE_ERR_KERNEL_LAUNCH, "launch grid (%u, %u, %u) exceeds what one dispatch can hold", grid[0], grid[1], grid[2]);
-  size_t size = args.buf.size();
-  void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, args.buf.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
+  size_t size = args.used;
+  void* extra[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, args.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &size,
                    HIP_LAUNCH_PARAM_END};
   CUTILE_HIP_OR_RETURN(api, hipModuleLaunchKernel(fn, grid[0], grid[1], grid[2], block[0], block[1], block[2],
                                                   dyn_lds, (hipStream_t)stream, nullptr, extra));
@@ -321,8 +329,8 @@ cutile_status_t resolve_own(const char* function, const char* variant, const cha
 
 // The table's first kernel for a partition's tile shape, or nullptr.
 const KernelEntry* first_of_tile(const char* function, const std::string& dtype, int bm, int bn) {
-  for (const auto& e : kernel_table())
-    if (e.tile[0] == bm && e.tile[1] == bn && strcmp(e.function, function) == 0 && dtype == e.dtype) return &e;
+  for (const KernelEntry* e : kernels_of(function))
+    if (e->tile[0] == bm && e->tile[1] == bn && dtype == e->dtype) return e;
   return nullptr;
 }
 
@@ -843,8 +851,8 @@ cutile_status_t cutile_launch_convert(cutile_stream_t stream, const cutile_tenso
 // wavefronts; only segments too long for that take more vectors per lane.
 static std::vector<std::string> fitting_row_variants(const char* fn_name, const std::string& prefix, int64_t seg_len) {
   std::vector<const KernelEntry*> fit;
-  for (const auto& e : kernel_table())
-    if (strcmp(e.function, fn_name) == 0 && e.capacity >= seg_len &&
+  for (const KernelEntry* entry : kernels_of(fn_name))
+    if (const KernelEntry& e = *entry; e.capacity >= seg_len &&
         strncmp(e.variant, prefix.c_str(), prefix.size()) == 0)
       fit.push_back(&e);
   std::stable_sort(fit.begin(), fit.end(), [](const KernelEntry* a, const KernelEntry* b) {
@@ -1986,8 +1994,9 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   // same output when the launch covers all of z
   auto fitting = [&] {
     std::vector<std::string> acceptable, others;
-    for (const auto& e : kernel_table()) {
-      if (strcmp(e.function, "gemm") != 0 || dt != e.dtype || strchr(e.variant, '+') != nullptr) continue;
+    for (const KernelEntry* entry : kernels_of("gemm")) {
+      const KernelEntry& e = *entry;
+      if (dt != e.dtype || strchr(e.variant, '+') != nullptr) continue;
       if (is_gemm_small(&e)) {
         if (row_layout && y->shape[1] >= e.tile[1]) others.push_back(e.variant);
       } else if (e.tile[0] > 0 && fast_layout && (k_valid % 64 == 0 || strstr(e.variant, "_r") == nullptr) && (whole_tiles || !is_stream_variant(e.variant))) {
@@ -2104,8 +2113,8 @@ cutile_status_t cutile_launch_batch_matmul(cutile_stream_t stream, const cutile_
   const int32_t k_valid = std::min(std::min(a->shape[2], b->shape[1]), k_total);
   std::vector<std::string> acceptable;
   if (fast_layout)
-    for (const auto& e : kernel_table())
-      if (strcmp(e.function, "batch_matmul") == 0 && dt == e.dtype && e.tile[0] == bm && e.tile[1] == bn &&
+    for (const KernelEntry* entry : kernels_of("batch_matmul"))
+      if (const KernelEntry& e = *entry; dt == e.dtype && e.tile[0] == bm && e.tile[1] == bn &&
           (k_valid % 64 == 0 || strstr(e.variant, "_r") == nullptr))
         acceptable.push_back(e.variant);
   acceptable.push_back(dt + "_generic");
@@ -2303,8 +2312,8 @@ cutile_status_t cutile_launch_gemm_persistent(cutile_stream_t stream, const cuti
                            y->shape[0] >= kx && kx % 64 == 0 && kx >= 192 && m.rank == 2;
   std::vector<std::string> acceptable;
   if (fast_layout)
-    for (const auto& e : kernel_table())
-      if (strcmp(e.function, "gemm_persistent") == 0 && strcmp(e.dtype, dt) == 0 && e.tile[0] == bm && e.tile[1] == bn &&
+    for (const KernelEntry* entry : kernels_of("gemm_persistent"))
+      if (const KernelEntry& e = *entry; strcmp(e.dtype, dt) == 0 && e.tile[0] == bm && e.tile[1] == bn &&
           strchr(e.variant, '+') == nullptr && (whole_tiles || !is_stream_variant(e.variant)))
         acceptable.push_back(e.variant);
   acceptable.push_back(std::string(dt) + "_generic");
@@ -2360,8 +2369,8 @@ cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, con
                  "group_gemm_f16_nt_desc: the launch grid (%u) must equal NUM_SM = %d", grid[0], num_sm_generic);
   if (!grid[0]) grid[0] = (uint32_t)num_sm_generic;
   std::vector<std::string> acceptable;
-  for (const auto& e : kernel_table())
-    if (strcmp(e.function, "group_gemm_nt_desc") == 0 && e.tile[0] == bm && e.tile[1] == bn) acceptable.push_back(e.variant);
+  for (const KernelEntry* entry : kernels_of("group_gemm_nt_desc"))
+    if (const KernelEntry& e = *entry; e.tile[0] == bm && e.tile[1] == bn) acceptable.push_back(e.variant);
   CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND,
                  "no precompiled variant of group_gemm_f16_nt_desc<BM=%d, BN=%d>; available: %s", bm, bn,
                  list_variants("group_gemm_nt_desc").c_str());
@@ -2520,8 +2529,8 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
                  CUTILE_ERR_KERNEL_NOT_FOUND, "fmha: the rows of one (batch, head) of q, k, v and out must each end below 2 GiB from the first");
   const std::string dt = cutile_dtype_name(q->dtype);
   std::vector<std::string> acceptable, same_bn;
-  for (const auto& e : kernel_table())
-    if (strcmp(e.function, "fmha") == 0 && dt == e.dtype && e.tile[0] == bm && e.tile[2] == d) {
+  for (const KernelEntry* entry : kernels_of("fmha"))
+    if (const KernelEntry& e = *entry; dt == e.dtype && e.tile[0] == bm && e.tile[2] == d) {
       acceptable.push_back(e.variant);
       if (e.tile[1] == bn_user) same_bn.push_back(e.variant);
     }
@@ -2619,8 +2628,8 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   // kernel tile: the ping-pong kernel for long D = 128 prefills, else the largest tile of that D
   const char* function = position_start ? "fmha_seq" : "fmha";
   std::vector<const KernelEntry*> fit;
-  for (const auto& e : kernel_table())
-    if (strcmp(e.function, function) == 0 && strcmp(e.dtype, "f16") == 0 && e.tile[2] == d) fit.push_back(&e);
+  for (const KernelEntry* entry : kernels_of(function))
+    if (const KernelEntry& e = *entry; strcmp(e.dtype, "f16") == 0 && e.tile[2] == d) fit.push_back(&e);
   CUTILE_REQUIRE(!fit.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "no precompiled sequence attention for f16, D = %d; available: %s", d,
                  list_variants(function).c_str());
   const bool long_prefill = rows_cov >= 256 && kv_len > 0;
@@ -2748,8 +2757,8 @@ cutile_status_t cutile_launch_linear_tile_mxfp8(cutile_stream_t stream, const cu
   // A kernel tile that is a whole multiple of the partition tile computes the
   // same output when the launch covers the whole tensor.
   std::vector<const KernelEntry*> fit;
-  for (const auto& e : kernel_table())
-    if (strcmp(e.function, "linear_tile") == 0 && dt == e.dtype &&
+  for (const KernelEntry* entry : kernels_of("linear_tile"))
+    if (const KernelEntry& e = *entry; dt == e.dtype &&
         ((e.tile[0] == bm && e.tile[1] == bn) || (full_cover && e.tile[0] % bm == 0 && e.tile[1] % bn == 0)))
       fit.push_back(&e);
   std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
@@ -2837,8 +2846,8 @@ cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cu
   // A kernel tile that is a whole multiple of the partition tile computes the same output when the
   // launch covers the whole tensor (the reference example's 16x16 tiles run on the 32x32 kernel).
   std::vector<const KernelEntry*> fit;
-  for (const auto& e : kernel_table())
-    if (strcmp(e.function, "linear_tile_nvfp4") == 0 && dt == e.dtype &&
+  for (const KernelEntry* entry : kernels_of("linear_tile_nvfp4"))
+    if (const KernelEntry& e = *entry; dt == e.dtype &&
         ((e.tile[0] == bm && e.tile[1] == bn) || (full_cover && e.tile[0] % bm == 0 && e.tile[1] % bn == 0)))
       fit.push_back(&e);
   std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {

@@ -1,5 +1,6 @@
 // Process-global runtime objects behind the opaque C handles.
 #pragma once
+#include <atomic>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -21,12 +22,14 @@ struct cutile_device {
   std::mutex mutex;
   std::vector<hipStream_t> idle_streams;  // released streams, reused before creating new ones
   uint64_t streams_created = 0;
-  int compute_units = 0;  // filled on first use by compute_units()
+  std::atomic<int> compute_units{0};  // filled on first use by compute_units()
   std::map<hipStream_t, void*> split_workspaces;   // workspace.cpp
   // Code objects of the kernel table loaded on this device: image id -> module.
   std::map<int, cutile_module*> table_modules;
   // Resolved functions: symbol -> hipFunction_t.
   std::map<std::string, hipFunction_t> functions;
+  // The same by position in the kernel table, readable without the mutex (one slot per table entry, made with the device).
+  std::unique_ptr<std::atomic<hipFunction_t>[]> function_slots;
 };
 
 namespace cutile {
@@ -46,6 +49,8 @@ struct SplitWorkspace {
 };
 cutile_status_t split_workspace(cutile_device_t device, hipStream_t stream, SplitWorkspace* out);
 void release_split_workspace(cutile_device_t device, hipStream_t stream);
+// The device of that ordinal if cutile_device_get has handed it out before, else nullptr.
+cutile_device_t known_device(int ordinal);
 // Compute units of the device (cached).
 cutile_status_t compute_units(cutile_device_t device, int* count);
 
