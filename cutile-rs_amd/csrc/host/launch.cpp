@@ -869,10 +869,12 @@ static std::vector<std::string> fitting_row_variants(const char* fn_name, const 
 // Launch grid of a row-wise kernel over `segments` tile rows: register-resident
 // variants take 4 / WPR segments per workgroup, the any-layout ones walk the
 // segments with a grid stride.
-static void row_launch_grid(const KernelEntry* e, uint64_t segments, uint32_t grid[3]) {
+// `row_bytes`: length of a segment whose elements are adjacent (0: they are not); the any-layout kernels put four rows
+// of up to 4 KiB or two of up to 8 KiB into a workgroup (kAnyRowPerWave, rowwise.hip).
+static void row_launch_grid(const KernelEntry* e, uint64_t segments, uint32_t grid[3], int64_t row_bytes = 0) {
   grid[0] = grid[1] = grid[2] = 1;
   if (e->capacity <= 0)
-    grid[0] = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(segments, 1), 1u << 20);
+    grid[0] = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(row_bytes <= 0 || row_bytes > 8192 ? segments : div_up(segments, row_bytes > 4096 ? 2 : 4), 1), 1u << 20);
   else if (e->tile[1] > 0)   // short-row variants: tile[1] rows per workgroup
     grid[0] = std::max<uint32_t>(1, div_up(segments, e->tile[1]));
   else
@@ -933,7 +935,7 @@ cutile_status_t cutile_launch_rms_norm_f16(cutile_stream_t stream, const cutile_
   args.push_tile_grid(tg);
   const uint64_t rows = std::min<uint64_t>(tg[0], ot.shape[0]);
   uint32_t grid[3];
-  row_launch_grid(res.entry, rows, grid);
+  row_launch_grid(res.entry, rows, grid, x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1 ? 2 * (int64_t)n : 0);
   return launch_packed(res.fn, grid, res.entry->block, rms_norm_residency_lds(res.entry, n), stream, args);
 }
 
@@ -1124,8 +1126,9 @@ static cutile_status_t launch_fused_norm(const char* fn, cutile_stream_t stream,
   if (qk) args.push_val<int32_t>(*num_q_rows);
   args.push_tile_grid(tg);
   const uint64_t rows = std::min<uint64_t>(tg[0], ot.shape[0]);
+  auto unit = [](const cutile_tensor_arg_t& t) { return t.strides[t.rank - 1] == 1; };
   uint32_t grid[3];
-  row_launch_grid(res.entry, rows, grid);
+  row_launch_grid(res.entry, rows, grid, unit(*a) && unit(*b) && unit(*w) && (!w2 || unit(*w2)) && unit(ot) && (!out2 || unit(out2->tensor)) ? 2 * (int64_t)n : 0);
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 
@@ -1929,7 +1932,7 @@ cutile_status_t cutile_launch_softmax(cutile_stream_t stream, const cutile_tenso
   args.push_tile_grid(tg);
   const uint64_t segments = rows * tg[1];
   uint32_t grid[3];
-  row_launch_grid(res.entry, segments, grid);
+  row_launch_grid(res.entry, segments, grid, x->strides[1] == 1 && yt.strides[1] == 1 ? (int64_t)bn * (int64_t)cutile_dtype_size(x->dtype) : 0);
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 

@@ -265,6 +265,110 @@ __device__ __forceinline__ void add_rms_norm_rows(const _Float16* __restrict__ r
   }
 }
 
+// ---- rows of unit stride that are not whole 16-byte vectors -----------------------------------------------------------
+// A row of an odd number of halves starts on any 2-byte boundary.  The element walks below read it two (softmax: three) times,
+// 2 bytes a lane: softmax of 4000 x 5001, 52 us, 1.5 TB/s.  Here the row is read once and stays in registers: whole 16-byte
+// vectors from its first 16-byte boundary on (aligned accesses: vectors counted from an odd half cost a third more), and the up to
+// 7 elements before and after them as one value in a lane of the row's first wavefront.  WPR wavefronts share a row of
+// up to WPR * 64 * VPL vectors; a workgroup walks rows with a grid stride.  4000 x 5001: softmax 52 -> 16 us, RMSNorm 17 us, the
+// fused residual form 27 us (5 - 6 TB/s, the rate of the aligned kernels).
+constexpr int64_t kAnyRowMost = 4 * 64 * 8 * 16;      // bytes of the longest row held in registers (WPR 4, VPL 8)
+constexpr int64_t kAnyRowPerWave = 64 * 4 * 16;       // rows of up to this many bytes take one wavefront each (the launcher sizes the grid by it)
+typedef u32x4 Unaligned __attribute__((aligned(2)));
+template <typename T, int WPR>
+struct RowShape {
+  static constexpr int E = 16 / sizeof(T);
+  int32_t head, vectors, extra;   // elements before the first boundary, whole vectors, this lane's single element (-1: none)
+  __device__ RowShape(const T* row, int32_t n, int sub, int lane) {
+    head = min(n, (int32_t)((0 - (uintptr_t)row) & 15) / (int32_t)sizeof(T));
+    vectors = (n - head) / E;
+    const int32_t tail = head + vectors * E;
+    extra = sub != 0 ? -1 : lane < head ? lane : lane >= 16 && lane - 16 < n - tail ? tail + lane - 16 : -1;
+  }
+  // first element of vector i of this lane, or -1
+  __device__ __forceinline__ int32_t at(int sub, int lane, int i) const {
+    const int32_t v = sub * 64 + lane + i * (64 * WPR);
+    return v < vectors ? head + v * E : -1;
+  }
+};
+template <typename T>
+__device__ __forceinline__ u32x4 load_any(const T* p) { return *reinterpret_cast<const Unaligned*>(p); }
+template <typename T>
+__device__ __forceinline__ void store_any(T* p, u32x4 v) { *reinterpret_cast<Unaligned*>(p) = v; }
+
+// RMSNorm of one source or (ADD) of the sum of two; `sum_out` receives the sum.
+struct AnyRow {
+  const _Float16 *x, *add, *w;
+  _Float16 *out, *sum_out;
+};
+template <int WPR, int VPL, bool ADD, typename RowOf>
+__device__ __forceinline__ void norm_rows_any(RowOf row_of, int32_t n, int64_t rows, float eps) {
+  using V = Vec16<_Float16>;
+  constexpr int ROWS_PER_WG = kWaves / WPR;
+  __shared__ float lds[2][kWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = wave / WPR, sub = wave % WPR;
+  int turn = 0;
+  for (int64_t first = (int64_t)blockIdx.x * ROWS_PER_WG; first < rows; first += (int64_t)gridDim.x * ROWS_PER_WG, turn ^= 1) {
+    const int64_t row = first + slot;
+    const bool live = row < rows;
+    const AnyRow r = row_of(live ? row : first);
+    const RowShape<_Float16, WPR> shape(r.x, live ? n : 0, sub, lane);
+    V xv[VPL], av[ADD ? VPL : 1];
+    float extra = 0.0f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i)
+      if (const int32_t j = shape.at(sub, lane, i); j >= 0) {
+        xv[i].raw = load_any(r.x + j);
+        if (ADD) av[i].raw = load_any(r.add + j);
+      }
+    if (shape.extra >= 0) extra = (float)r.x[shape.extra] + (ADD ? (float)r.add[shape.extra] : 0.0f);
+    float ss = extra * extra;   // vectors outside the row are 0
+#pragma unroll
+    for (int i = 0; i < VPL; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float f = ADD ? (float)xv[i].v[e] + (float)av[i].v[e] : (float)xv[i].v[e];
+        ss = __builtin_fmaf(f, f, ss);
+      }
+    ss = group_reduce<WPR, false>(ss, lds[turn], slot, sub);
+    const float inv = __builtin_amdgcn_rsqf(ss / (float)n + eps);
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int32_t j = shape.at(sub, lane, i);
+      if (j < 0) continue;
+      asm volatile("" : "+v"(xv[i].raw));   // widened again here: held as f32, the row would take twice the registers
+      V wv, ov, sv;
+      wv.raw = load_any(r.w + j);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float f = ADD ? (float)xv[i].v[e] + (float)av[i].v[e] : (float)xv[i].v[e];
+        ov.v[e] = (_Float16)((f * inv) * (float)wv.v[e]);
+        if (ADD) sv.v[e] = (_Float16)f;
+      }
+      store_any(r.out + j, ov.raw);
+      if (ADD) store_any(r.sum_out + j, sv.raw);
+    }
+    if (shape.extra >= 0) {
+      r.out[shape.extra] = (_Float16)((extra * inv) * (float)r.w[shape.extra]);
+      if (ADD) r.sum_out[shape.extra] = (_Float16)extra;
+    }
+  }
+}
+template <bool ADD, typename RowOf>
+__device__ __forceinline__ void norm_rows_any_length(RowOf row_of, int32_t n, int64_t rows, float eps) {
+  const int64_t bytes = (int64_t)n * 2;
+  if (bytes <= 64 * 16)
+    norm_rows_any<1, 1, ADD>(row_of, n, rows, eps);
+  else if (bytes <= kAnyRowPerWave)
+    norm_rows_any<1, 4, ADD>(row_of, n, rows, eps);
+  else if (bytes <= 2 * kAnyRowPerWave)
+    norm_rows_any<2, 4, ADD>(row_of, n, rows, eps);
+  else if (bytes <= 4 * kAnyRowPerWave)
+    norm_rows_any<4, 4, ADD>(row_of, n, rows, eps);
+  else
+    norm_rows_any<4, 8, ADD>(row_of, n, rows, eps);
+}
+
 // Any N / any strides for the two fused forms: one workgroup per row, inputs re-read (L2).
 __device__ __forceinline__ void fused_norm_row_generic(const TensorArg<2>& a, const TensorArg<2>* b_add,
                                                        const TensorArg<2>* b_alt, const TensorArg<1>& w,
@@ -272,6 +376,22 @@ __device__ __forceinline__ void fused_norm_row_generic(const TensorArg<2>& a, co
                                                        const PartitionArg<2>* out2, float eps, int64_t rows,
                                                        int64_t split) {
   // b_add: second addend (add_rms_norm); b_alt / w_alt: source and weight for rows >= split (qk_norm)
+  const int32_t cols = a.shape[1];
+  if (a.strides[1] == 1 && (!b_add || (b_add->strides[1] == 1 && b_add->shape[1] >= cols)) && (!b_alt || (b_alt->strides[1] == 1 && b_alt->shape[1] == cols)) &&
+      w.strides[0] == 1 && w.shape[0] >= cols && (!w_alt || (w_alt->strides[0] == 1 && w_alt->shape[0] >= cols)) && out.strides[1] == 1 &&
+      out.shape[1] >= cols && (!out2 || (out2->strides[1] == 1 && out2->shape[1] >= cols)) && (int64_t)cols * 2 <= kAnyRowMost) {
+    const auto row_of = [&](int64_t row) {
+      const bool second = b_alt && row >= split;
+      return AnyRow{second ? (const _Float16*)b_alt->ptr + (row - split) * b_alt->strides[0] : (const _Float16*)a.ptr + row * a.strides[0],
+                    b_add ? (const _Float16*)b_add->ptr + row * b_add->strides[0] : nullptr, (const _Float16*)(second ? w_alt : &w)->ptr,
+                    (_Float16*)out.ptr + row * out.strides[0], out2 ? (_Float16*)out2->ptr + row * out2->strides[0] : nullptr};
+    };
+    if (b_add)
+      norm_rows_any_length<true>(row_of, cols, rows, eps);
+    else
+      norm_rows_any_length<false>(row_of, cols, rows, eps);
+    return;
+  }
   __shared__ float lds[kWaves];
   const int wave = threadIdx.x >> 6;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
@@ -311,6 +431,15 @@ __device__ __forceinline__ void fused_norm_row_generic(const TensorArg<2>& a, co
 __device__ __forceinline__ void rms_norm_row_generic(const TensorArg<2>& x, const TensorArg<1>& w,
                                                      const PartitionArg<2>& out, float eps,
                                                      int64_t rows) {
+  if (x.strides[1] == 1 && w.strides[0] == 1 && w.shape[0] >= x.shape[1] && out.strides[1] == 1 && out.shape[1] >= x.shape[1] &&
+      (int64_t)x.shape[1] * 2 <= kAnyRowMost) {
+    norm_rows_any_length<false>(
+        [&](int64_t row) {
+          return AnyRow{(const _Float16*)x.ptr + row * x.strides[0], nullptr, (const _Float16*)w.ptr, (_Float16*)out.ptr + row * out.strides[0], nullptr};
+        },
+        x.shape[1], rows, eps);
+    return;
+  }
   __shared__ float lds[kWaves];
   const int wave = threadIdx.x >> 6;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
@@ -415,15 +544,101 @@ __device__ __forceinline__ void softmax_segments(const T* __restrict__ x, int64_
   }
 }
 
+// Rows of unit stride, tiles of any width: the segment in registers, read once (norm_rows_any above says why).
+template <typename T, int WPR, int VPL>
+__device__ __forceinline__ void softmax_segments_any(const TensorArg<2>& x, const PartitionArg<2>& y, int32_t segs_per_row, int64_t n_segments) {
+  using V = Vec16<T>;
+  constexpr int E = V::N, SEGS_PER_WG = kWaves / WPR;
+  __shared__ float lds[2][kWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = wave / WPR, sub = wave % WPR;
+  const int32_t bn = y.pshape[1];
+  for (int64_t first = (int64_t)blockIdx.x * SEGS_PER_WG; first < n_segments; first += (int64_t)gridDim.x * SEGS_PER_WG) {
+    const int64_t seg = first + slot;
+    const bool live = seg < n_segments;
+    const int64_t row = !live ? 0 : segs_per_row == 1 ? seg : seg / segs_per_row;
+    const int32_t col0 = !live || segs_per_row == 1 ? 0 : (int32_t)(seg % segs_per_row) * bn;
+    const int32_t len = live ? bn : 0;                                                          // takes part (0 beyond x: padding)
+    const int32_t x_valid = live && row < x.shape[0] ? min(bn, x.shape[1] - col0) : 0;          // readable
+    const int32_t y_valid = live && row < y.shape[0] ? min(bn, y.shape[1] - col0) : 0;          // storable
+    const T* xr = (const T*)x.ptr + row * x.strides[0] + col0;
+    const RowShape<T, WPR> shape(xr, max(x_valid, 0), sub, lane);
+    V xv[VPL];
+    float extra = -INFINITY;             // outside the segment: its exponential is 0
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int32_t j = shape.at(sub, lane, i);
+      if (j >= 0) {
+        xv[i].raw = load_any(xr + j);
+      } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) xv[i].v[e] = (T)-INFINITY;
+      }
+    }
+    if (shape.extra >= 0) extra = to_f32(xr[shape.extra]);
+    const int32_t padding = len - max(x_valid, 0);   // zeros beyond x inside the segment
+    float m = padding > 0 ? fmaxf(extra, 0.0f) : extra;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i)
+#pragma unroll
+      for (int e = 0; e < E; ++e) m = fmaxf(m, to_f32(xv[i].v[e]));
+    m = group_reduce<WPR, true>(m, lds[0], slot, sub);
+    const float mb = m * kLog2e;
+    auto exponential = [&](float v) { return __builtin_amdgcn_exp2f(__builtin_fmaf(v, kLog2e, -mb)); };
+    float s = exponential(extra);
+    if (padding > 0 && sub == 0 && lane == 0) s += (float)padding * exponential(0.0f);
+    // the exponentials are formed again for the store: held, they would take twice the registers of the row itself
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      asm volatile("" : "+v"(xv[i].raw));   // nor the widened values
+#pragma unroll
+      for (int e = 0; e < E; ++e) s += exponential(to_f32(xv[i].v[e]));
+    }
+    s = group_reduce<WPR, false>(s, lds[1], slot, sub);
+    const float inv = 1.0f / s;
+    auto quotient = [&](float v) { return sizeof(T) == 4 ? (T)(exponential(v) / s) : (T)(exponential(v) * inv); };
+    T* yr = (T*)y.ptr + row * y.strides[0] + col0;
+    if (y_valid >= x_valid) {            // the usual case: y holds what x holds, vector for vector
+#pragma unroll
+      for (int i = 0; i < VPL; ++i) {
+        const int32_t j = shape.at(sub, lane, i);
+        if (j < 0) continue;
+        asm volatile("" : "+v"(xv[i].raw));
+        V ov;
+#pragma unroll
+        for (int e = 0; e < E; ++e) ov.v[e] = quotient(to_f32(xv[i].v[e]));
+        store_any(yr + j, ov.raw);
+      }
+      if (shape.extra >= 0) yr[shape.extra] = quotient(extra);
+      for (int32_t j = max(x_valid, 0) + sub * 64 + lane; j < y_valid; j += 64 * WPR) yr[j] = quotient(0.0f);
+    } else {                             // y is narrower than x
+      for (int32_t j = sub * 64 + lane; j < y_valid; j += 64 * WPR) yr[j] = quotient(to_f32(xr[j]));
+    }
+  }
+}
+
 // Any tile width / any strides: one workgroup per segment, three passes (the
 // segment stays in L2 between them).
 template <typename T>
 __device__ __forceinline__ void softmax_segment_generic(const TensorArg<2>& x,
                                                         const PartitionArg<2>& y,
                                                         int32_t segs_per_row, int64_t n_segments) {
+  const int32_t bn = y.pshape[1];
+  const int64_t bytes = (int64_t)bn * (int64_t)sizeof(T);
+  if (x.strides[1] == 1 && y.strides[1] == 1 && bytes <= kAnyRowMost) {
+    if (bytes <= 64 * 16)
+      softmax_segments_any<T, 1, 1>(x, y, segs_per_row, n_segments);
+    else if (bytes <= kAnyRowPerWave)
+      softmax_segments_any<T, 1, 4>(x, y, segs_per_row, n_segments);
+    else if (bytes <= 2 * kAnyRowPerWave)
+      softmax_segments_any<T, 2, 4>(x, y, segs_per_row, n_segments);
+    else if (bytes <= 4 * kAnyRowPerWave)
+      softmax_segments_any<T, 4, 4>(x, y, segs_per_row, n_segments);
+    else
+      softmax_segments_any<T, 4, 8>(x, y, segs_per_row, n_segments);
+    return;
+  }
   __shared__ float lds[2][kWaves];
   const int wave = threadIdx.x >> 6;
-  const int32_t bn = y.pshape[1];
   for (int64_t seg = blockIdx.x; seg < n_segments; seg += gridDim.x) {
     const int64_t row = seg / segs_per_row;
     const int32_t col0 = (int32_t)(seg % segs_per_row) * bn;
@@ -530,20 +745,20 @@ RMS_NORM_SHORT_KERNEL(32)
 FUSED_NORM_VARIANTS(ADD_RMS_NORM_KERNEL)
 FUSED_NORM_VARIANTS(QK_NORM_KERNEL)
 
-extern "C" __global__ void __launch_bounds__(kThreads)
+extern "C" __global__ void __launch_bounds__(kThreads, 4)
     add_rms_norm_f16_entry__generic(TensorArg<2> residual, TensorArg<2> x, TensorArg<1> w, PartitionArg<2> out,
                                     PartitionArg<2> residual_out, float eps, TileGrid g) {
   int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
   fused_norm_row_generic(x, &residual, nullptr, w, nullptr, out, &residual_out, eps, rows, INT64_MAX);
 }
-extern "C" __global__ void __launch_bounds__(kThreads)
+extern "C" __global__ void __launch_bounds__(kThreads, 4)
     qk_norm_f16_entry__generic(TensorArg<2> q, TensorArg<2> k, TensorArg<1> qw, TensorArg<1> kw, PartitionArg<2> out,
                                float eps, int32_t num_q_rows, TileGrid g) {
   int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
   fused_norm_row_generic(q, nullptr, &k, qw, &kw, out, nullptr, eps, rows, (int64_t)num_q_rows);
 }
 
-extern "C" __global__ void __launch_bounds__(kThreads)
+extern "C" __global__ void __launch_bounds__(kThreads, 4)
     rms_norm_f16_entry__generic(TensorArg<2> x, TensorArg<1> w, PartitionArg<2> out, float eps,
                                 TileGrid g) {
   int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
@@ -914,7 +1129,7 @@ SOFTMAX_VARIANTS(_Float16, f16)
 SOFTMAX_VARIANTS(float, f32)
 
 #define SOFTMAX_GENERIC(T, NAME)                                                                    \
-  extern "C" __global__ void __launch_bounds__(kThreads)                                           \
+  extern "C" __global__ void __launch_bounds__(kThreads, 6)                                           \
       softmax_entry__##NAME##_generic(TensorArg<2> x, PartitionArg<2> y, TileGrid g) {              \
     int64_t rows = min((int64_t)g.x * y.pshape[0], (int64_t)y.shape[0]);                           \
     softmax_segment_generic<T>(x, y, (int32_t)g.y, rows * (int64_t)g.y);                           \
