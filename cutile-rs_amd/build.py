@@ -35,6 +35,7 @@ IMAGES = {
     "nvfp4": "nvfp4_gemm.hip",
     "rng": "rng.hip",
     "gemmsmall": "gemm_small.hip",
+    "scaledflat": "scaled_flat.hip",
 }
 HOST_SOURCES = ["hip_api.cpp", "driver.cpp", "kernel_table.cpp", "launch.cpp", "runtime.cpp", "tuning.cpp", "workspace.cpp"]
 # The recording stand-in for the HIP runtime (include/cutile_hip_testing.h) is not part of the product library: the CPU

@@ -87,4 +87,46 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
   return c;
 }
 
+// ---- block-scaled products ----
+struct ScaledShape {
+  int64_t m, n;
+  int32_t pieces;          // 64-byte pieces of a row: 64 (fp8) or 128 (fp4) values of K
+  bool fp4;
+};
+// K splits of a scaled_flat.hip launch: up to half the compute units busy, at least two 128-byte steps for each of the 8
+// wavefronts (mxfp8, 64 x 1024 x 8192, 32 strips: 16.7, 13.2, 12.5 us with 1, 2, 4 splits; 16 x 4096 x 4096, 64 strips: 9.4,
+// 9.4, 10.5; nvfp4 of that size 9.9, 11.7, 13.1; 16 x 1024 x 1024 6.6, 8.0, 8.5).
+inline uint32_t scaled_splits(uint64_t blocks, int32_t pieces, int cus) {
+  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / 2 / std::max<uint64_t>(blocks, 1)), pieces / (2 * 8 * 2)));
+}
+// The kernel by name, or nullptr: the partition's own (tuning record, then the table's order).  us per 64-byte piece of K for
+// one block on each compute unit, measured at K = 4096 (mxfp8: 16 x 4096 9.4 us, 64 x 4096 13.4, 512 x 4096 21 on 64 x 128 blocks, 24 with
+// 128 x 128 tiles; nvfp4: 9.9, 14.7, 24).  The 256 x 256 kernels are the better ones where their tiles come near to filling the chip.
+inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus) {
+  if (s.pieces <= 4) return nullptr;   // two steps: nothing to share out
+  auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
+  if (s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
+  struct Kernel { const char* name; int bm, bn; double fp8, fp4; };
+  static const Kernel kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20}, {"flat32x64", 32, 64, 0.12, 0.28}, {"flat64x64", 64, 64, 0.155, 0.36},
+                                 {"flat64x128", 64, 128, 0.27, 0.62}, {"flat128x128", 128, 128, 0.52, 1.12}};
+  const char* name = nullptr;
+  double best = 1e30;
+  for (const Kernel& k : kFlat) {
+    const uint64_t b = blocks(k.bm, k.bn), waves = (b + cus - 1) / cus;
+    const double us = (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + 3.5);
+    if (us < best) best = us, name = k.name;
+  }
+  if (!s.fp4) {   // two workgroups to a compute unit
+    const uint64_t b = blocks(128, 128), rest = b % (2 * (uint64_t)cus);
+    const double us = (double)(b / (2 * (uint64_t)cus)) * (0.58 * s.pieces + 4) + (rest == 0 ? 0.0 : (rest <= (uint64_t)cus ? 0.31 : 0.58) * s.pieces + 4);
+    if (us < best) best = us, name = "128x128x128_e2x2";
+  } else if (own_m == 256 && own_n == 256) {
+    const uint64_t b = blocks(256, 256), waves = (b + cus - 1) / cus;
+    const double part = (double)std::min<uint64_t>(b, cus) / cus;
+    const double us = (double)waves * (s.pieces * (1.85 + 2.1 * std::max(0.0, part - 0.25) / 0.75) + 4);
+    if (us < best) return nullptr;
+  }
+  return name;
+}
+
 }  // namespace cutile

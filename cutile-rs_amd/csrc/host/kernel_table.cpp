@@ -22,6 +22,7 @@ extern const unsigned char cutile_img_mxgemm_start[], cutile_img_mxgemm_end[];
 extern const unsigned char cutile_img_nvfp4_start[], cutile_img_nvfp4_end[];
 extern const unsigned char cutile_img_rng_start[], cutile_img_rng_end[];
 extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_end[];
+extern const unsigned char cutile_img_scaledflat_start[], cutile_img_scaledflat_end[];
 }
 
 namespace cutile {
@@ -48,6 +49,7 @@ ImageRef image_ref(Image img) {
     case IMG_NVFP4: return {cutile_img_nvfp4_start, cutile_img_nvfp4_end};
     case IMG_RNG: return {cutile_img_rng_start, cutile_img_rng_end};
     case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
+    case IMG_SCALED_FLAT: return {cutile_img_scaledflat_start, cutile_img_scaledflat_end};
     default: return {nullptr, nullptr};
   }
 }
@@ -371,11 +373,22 @@ std::vector<KernelEntry> build_table() {
   mx("f32", 256, 256, 4, 2, "e");
   mx("bf16", 256, 256, 2, 2);
   mx("bf16", 256, 256, 2, 4);
-  mx("bf16", 128, 128, 2, 2);
+  mx("bf16", 128, 128, 2, 2, "e");
+  mx("f32", 128, 128, 2, 2, "e");
   mx("f32", 256, 256, 2, 2);
-  mx("f32", 128, 128, 2, 2);
   mx("f32", 32, 32, 1, 1);
   mx("f32", 64, 64, 1, 1);
+
+  // ---- block-scaled products without LDS stages (scaled_flat.hip): any partition shape; LDS = one f32 copy of the block per share of K ----
+  for (const char* dt : {"bf16", "f32"})
+    for (auto t : {std::array<int, 3>{16, 64, 8}, std::array<int, 3>{32, 64, 8}, std::array<int, 3>{64, 64, 8}, std::array<int, 3>{64, 128, 4},
+                   std::array<int, 3>{128, 128, 2}})
+      for (const char* kind : {"mxfp8", "nvfp4"}) {
+        const bool mx8 = kind[0] == 'm';
+        std::string v = std::string(mx8 ? "mxfp8_" : "") + dt + "_flat" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
+        add(mx8 ? "linear_tile" : "linear_tile_nvfp4", keep(v), keep((mx8 ? "linear_tile_entry__" : "linear_tile_nvfp4_entry__") + v), IMG_SCALED_FLAT, 512,
+            (uint32_t)(t[2] * t[0] * (t[1] + 4) * 4), 0, t[1], 0, t[0], dt, 0, 2);
+      }
   return t;
 }
 

@@ -355,6 +355,83 @@ uint32_t split_limit(uint64_t blocks, uint64_t floats) {
 // (strips of columns) and staged ones (tiles).
 bool is_gemm_small(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
 bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0; }
+// The block-scaled kernels without LDS stages (scaled_flat.hip): tile[3] x tile[1] outputs a workgroup, any partition shape.
+bool is_scaled_flat(const KernelEntry* e) { return e->image == IMG_SCALED_FLAT; }
+
+// Picks the kernel of a block-scaled product.  A kernel tile that is a whole multiple of the partition tile computes the
+// same output when the launch covers the whole tensor (a 16 x 16 example partition runs on the 32 x 32 kernel), and so do
+// the kernels without LDS stages, which take `flat` launches: whole outputs, scale rows on 4-byte boundaries.
+cutile_status_t resolve_scaled(const char* function, const char* prefix, const std::string& dt, int bm, int bn, bool full_cover, bool flat,
+                               const ScaledShape& shape, const cutile_launch_opts_t* opts, const std::string& missing, int* cus, Resolved* res) {
+  std::vector<const KernelEntry*> fit, others;
+  for (const KernelEntry* e : kernels_of(function)) {
+    if (dt != e->dtype) continue;
+    if (is_scaled_flat(e)) {
+      if (flat) others.push_back(e);
+    } else if ((e->tile[0] == bm && e->tile[1] == bn) || (full_cover && e->tile[0] % bm == 0 && e->tile[1] % bn == 0)) {
+      fit.push_back(e);
+    }
+  }
+  CUTILE_REQUIRE(!fit.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "%s; available: %s", missing.c_str(), list_variants(function).c_str());
+  std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
+    bool ea = a->tile[0] == bm && a->tile[1] == bn, eb = b->tile[0] == bm && b->tile[1] == bn;
+    if (ea != eb) return ea;
+    return a->tile[0] * a->tile[1] < b->tile[0] * b->tile[1];
+  });
+  *cus = 256;
+  std::string sized;
+  if (flat) {
+    if (cutile_status_t s = current_device_units(cus)) return s;
+    if (const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus)) sized = prefix + dt + "_" + kernel;
+  }
+  if (!sized.empty() && !(opts && opts->variant) && preferred_variant(function).empty()) return resolve_own(function, sized.c_str(), "size", res);
+  std::vector<std::string> acceptable;
+  for (const KernelEntry* e : fit) acceptable.push_back(e->variant);
+  for (const KernelEntry* e : others) acceptable.push_back(e->variant);
+  return resolve_entry(function, opts, acceptable[0], acceptable, res, sized);
+}
+
+// Launches it; `pieces` = 64-byte pieces of a row.
+cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutile_partition_arg_t* z, const cutile_tensor_arg_t* x,
+                              const cutile_tensor_arg_t* y, const cutile_tensor_arg_t* xs, const cutile_tensor_arg_t* ys, float alpha,
+                              const uint32_t tg[3], int32_t pieces, int cus) {
+  const cutile_tensor_arg_t& zt = z->tensor;
+  ArgPacker args;
+  args.push_partition(*z);
+  args.push_tensor(*x);
+  args.push_tensor(*y);
+  args.push_tensor(*xs);
+  args.push_tensor(*ys);
+  args.push_val<float>(alpha);
+  if (is_scaled_flat(res.entry)) {
+    const uint32_t tiles_m = div_up(zt.shape[0], res.entry->tile[3]), tiles_n = div_up(zt.shape[1], res.entry->tile[1]);
+    const uint64_t blocks = (uint64_t)tiles_m * tiles_n;
+    SplitWorkspace ws;
+    uint32_t splits = std::min(scaled_splits(blocks, pieces, cus),
+                               split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
+    if (splits > 1 && g_launch_mode == 0) {
+      if (cutile_status_t s = split_workspace(res.device, (hipStream_t)stream, &ws)) return s;
+      if (!ws.partials) splits = 1;
+    }
+    args.push_val<void*>(ws.partials);
+    args.push_val<void*>(ws.counters);
+    args.push_val<uint32_t>(tiles_m);
+    args.push_val<uint32_t>(tiles_n);
+    args.push_val<uint32_t>(splits);
+    CUTILE_REQUIRE(blocks * splits <= 0x7fffffffull, CUTILE_ERR_KERNEL_LAUNCH, "linear_tile: %llu output tiles do not fit a launch grid axis",
+                   (unsigned long long)blocks);
+    const uint32_t grid[3] = {(uint32_t)(blocks * splits), 1, 1};
+    return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
+  }
+  uint32_t kg[3] = {tg[0], tg[1], 1};
+  if (res.entry->tile[0] != z->partition_shape[0] || res.entry->tile[1] != z->partition_shape[1]) {
+    kg[0] = div_up(zt.shape[0], res.entry->tile[0]);
+    kg[1] = div_up(zt.shape[1], res.entry->tile[1]);
+  }
+  args.push_tile_grid(kg);
+  const uint32_t grid[3] = {kg[0] * kg[1], 1, 1};
+  return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
+}
 // An output of this size or more is read and stored past the caches (it cannot still be cached when its consumer runs,
 // and the caches are left to the operand panels): the rule of the staged epilogue, decided on the host for this family.
 constexpr int64_t kStreamedOutputBytes = 64ll << 20;
@@ -2757,41 +2834,13 @@ cutile_status_t cutile_launch_linear_tile_mxfp8(cutile_stream_t stream, const cu
                  "below 2 GiB from their first element (x spans %lld bytes, y %lld, z %lld)",
                  (long long)extent_bytes_2d(*x), (long long)extent_bytes_2d(*y), (long long)extent_bytes_2d(zt));
   const std::string dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
-  // A kernel tile that is a whole multiple of the partition tile computes the
-  // same output when the launch covers the whole tensor.
-  std::vector<const KernelEntry*> fit;
-  for (const KernelEntry* entry : kernels_of("linear_tile"))
-    if (const KernelEntry& e = *entry; dt == e.dtype &&
-        ((e.tile[0] == bm && e.tile[1] == bn) || (full_cover && e.tile[0] % bm == 0 && e.tile[1] % bn == 0)))
-      fit.push_back(&e);
-  std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
-    bool ea = a->tile[0] == bm && a->tile[1] == bn, eb = b->tile[0] == bm && b->tile[1] == bn;
-    if (ea != eb) return ea;
-    return a->tile[0] * a->tile[1] < b->tile[0] * b->tile[1];
-  });
-  std::vector<std::string> acceptable;
-  for (auto* e : fit) acceptable.push_back(e->variant);
-  CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND,
-                 "no precompiled variant of linear_tile<%d, %d, %d, %d> -> %s; available: %s", bm, bn, bk_user,
-                 bk_user / 32, dt.c_str(), list_variants("linear_tile").c_str());
-  Resolved res;
+  const std::string missing = "no precompiled variant of linear_tile<" + std::to_string(bm) + ", " + std::to_string(bn) + ", " + std::to_string(bk_user) +
+                              ", " + std::to_string(bk_user / 32) + "> -> " + dt;
   BucketScope bucket("mxfp8_" + dt + "_" + std::to_string(bm) + "x" + std::to_string(bn));
-  if (cutile_status_t s = resolve_entry("linear_tile", opts, acceptable[0], acceptable, &res)) return s;
-  uint32_t kg[3] = {tg[0], tg[1], 1};
-  if (res.entry->tile[0] != bm || res.entry->tile[1] != bn) {
-    kg[0] = div_up(M, res.entry->tile[0]);
-    kg[1] = div_up(N, res.entry->tile[1]);
-  }
-  ArgPacker args;
-  args.push_partition(*z);
-  args.push_tensor(*x);
-  args.push_tensor(*y);
-  args.push_tensor(*xs);
-  args.push_tensor(*ys);
-  args.push_val<float>(alpha);
-  args.push_tile_grid(kg);
-  uint32_t grid[3] = {kg[0] * kg[1], 1, 1};
-  return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
+  Resolved res;
+  int cus = 256;
+  if (cutile_status_t s = resolve_scaled("linear_tile", "mxfp8_", dt, bm, bn, full_cover, full_cover, {M, N, K / 64, false}, opts, missing, &cus, &res)) return s;
+  return launch_scaled(res, stream, z, x, y, xs, ys, alpha, tg, K / 64, cus);
 }
 
 cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cutile_partition_arg_t* z,
@@ -2846,40 +2895,13 @@ cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cu
                  "end below 2 GiB from their first element (x spans %lld bytes, y %lld, z %lld)",
                  (long long)extent_bytes_2d(*x), (long long)extent_bytes_2d(*y), (long long)extent_bytes_2d(zt));
   const std::string dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
-  // A kernel tile that is a whole multiple of the partition tile computes the same output when the
-  // launch covers the whole tensor (the reference example's 16x16 tiles run on the 32x32 kernel).
-  std::vector<const KernelEntry*> fit;
-  for (const KernelEntry* entry : kernels_of("linear_tile_nvfp4"))
-    if (const KernelEntry& e = *entry; dt == e.dtype &&
-        ((e.tile[0] == bm && e.tile[1] == bn) || (full_cover && e.tile[0] % bm == 0 && e.tile[1] % bn == 0)))
-      fit.push_back(&e);
-  std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
-    bool ea = a->tile[0] == bm && a->tile[1] == bn, eb = b->tile[0] == bm && b->tile[1] == bn;
-    if (ea != eb) return ea;
-    return a->tile[0] * a->tile[1] < b->tile[0] * b->tile[1];
-  });
-  std::vector<std::string> acceptable;
-  for (auto* e : fit) acceptable.push_back(e->variant);
-  CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND,
-                 "no precompiled variant of nvfp4 linear_tile<%d, %d, %d, %d, %d> -> %s; available: %s", bm, bn, bk_user, bk_user / 2,
-                 bk_user / 16, dt.c_str(), list_variants("linear_tile_nvfp4").c_str());
+  const std::string missing = "no precompiled variant of nvfp4 linear_tile<" + std::to_string(bm) + ", " + std::to_string(bn) + ", " + std::to_string(bk_user) +
+                              ", " + std::to_string(bk_user / 2) + ", " + std::to_string(bk_user / 16) + "> -> " + dt;
+  const bool flat = full_cover && KP >= 128 && xs->strides[0] % 4 == 0 && ys->strides[0] % 4 == 0 && ((uintptr_t)xs->ptr & 3) == 0 && ((uintptr_t)ys->ptr & 3) == 0;
   Resolved res;
-  if (cutile_status_t s = resolve_entry("linear_tile_nvfp4", opts, acceptable[0], acceptable, &res)) return s;
-  uint32_t kg[3] = {tg[0], tg[1], 1};
-  if (res.entry->tile[0] != bm || res.entry->tile[1] != bn) {
-    kg[0] = div_up(M, res.entry->tile[0]);
-    kg[1] = div_up(N, res.entry->tile[1]);
-  }
-  ArgPacker args;
-  args.push_partition(*z);
-  args.push_tensor(*x);
-  args.push_tensor(*y);
-  args.push_tensor(*xs);
-  args.push_tensor(*ys);
-  args.push_val<float>(alpha);
-  args.push_tile_grid(kg);
-  uint32_t grid[3] = {kg[0] * kg[1], 1, 1};
-  return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
+  int cus = 256;
+  if (cutile_status_t s = resolve_scaled("linear_tile_nvfp4", "", dt, bm, bn, full_cover, flat, {M, N, (KP + 63) / 64, true}, opts, missing, &cus, &res)) return s;
+  return launch_scaled(res, stream, z, x, y, xs, ys, alpha, tg, (KP + 63) / 64, cus);
 }
 
 }  // extern "C"
