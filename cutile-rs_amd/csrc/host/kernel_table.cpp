@@ -291,9 +291,10 @@ std::vector<KernelEntry> build_table() {
     add("gemm_persistent", keep(v), keep("gemm_persistent_entry__" + v), IMG_GEMM, (uint32_t)(t[2] * t[3] * 64),
         (uint32_t)(2 * (t[0] * 64 + 64 * t[1]) * 2), t[0], t[1], 64, 0, "f16", 0, 2);
     // the grouped form keeps the group descriptors live across the tile loop: 2 x 4 wavefronts at 256 x 256 (no spills)
+    // (at 128 x 128 the name stands for the ring of three x and two y stages)
     std::string gv = t[0] == 256 ? std::string("f16_256x256x64_d2x4") : v;
     add("group_gemm_nt_desc", keep(gv), keep("group_gemm_nt_desc_entry__" + gv), IMG_GEMM, (uint32_t)(t[2] * t[3] * 64),
-        (uint32_t)(2 * (t[0] * 64 + 64 * t[1]) * 2), t[0], t[1], 64, 0, "f16", 0, 2);
+        (uint32_t)(((t[0] == 256 ? 2 : 3) * t[0] * 64 + 2 * 64 * t[1]) * 2), t[0], t[1], 64, 0, "f16", 0, 2);
   }
   for (const char* dt : {"bf16", "f16", "f32"})
     add("gemm_persistent", keep(std::string(dt) + "_generic"), keep(std::string("gemm_persistent_entry__") + dt + "_generic"),

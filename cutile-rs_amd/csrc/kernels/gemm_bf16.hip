@@ -1300,7 +1300,6 @@ __device__ __forceinline__ void group_gemm_desc(const TensorArg<1>& a_ptrs, cons
     group_gemm_desc<GemmDirect<BM, BN, WVM, WVN, _Float16, _Float16>, BM, BN>(a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, num_groups); \
   }
 GROUP_GEMM_KERNEL(f16_256x256x64_d2x4, 256, 256, 2, 4)
-GROUP_GEMM_KERNEL(f16_128x128x64_d2x2, 128, 128, 2, 2)
 
 #define GEMM_RING_KERNEL(NAME, BM, BN, WVM, WVN, OUT_T)                                          \
   extern "C" __global__ void __launch_bounds__(WVM* WVN * 64)                                  \
@@ -1343,6 +1342,14 @@ extern "C" __global__ void __launch_bounds__(512)
     group_gemm_nt_desc_entry__f16_256x256x64_q2x4(TensorArg<1> a_ptrs, TensorArg<1> b_ptrs, TensorArg<1> c_ptrs, TensorArg<2> a_metas,
                                                   TensorArg<2> b_metas, TensorArg<2> c_metas, int32_t num_groups) {
   group_gemm_desc<GemmRing16<256, 256, 2, 4, _Float16, _Float16>, 256, 256>(a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, num_groups);
+}
+// Groups of few rows read their B once: what counts is how much of it is on its way.  A workgroup a compute unit with two
+// stages waits for one K tile after another (32 groups of 32 x 4096 x 4096: 263 us, 4.1 TB/s); the ring, with its fetches issued
+// between the products, takes 194 us (5.6 TB/s); 16 groups of 9 x 1024 x 4608 69 -> 48 us, 8 of 47 x 3328 x 512 22 -> 12 us.
+extern "C" __global__ void __launch_bounds__(256)
+    group_gemm_nt_desc_entry__f16_128x128x64_d2x2(TensorArg<1> a_ptrs, TensorArg<1> b_ptrs, TensorArg<1> c_ptrs, TensorArg<2> a_metas,
+                                                  TensorArg<2> b_metas, TensorArg<2> c_metas, int32_t num_groups) {
+  group_gemm_desc<GemmRing16<128, 128, 2, 2, _Float16, _Float16>, 128, 128>(a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, num_groups);
 }
 #define GEMM_RING16_WALK_KERNEL(NAME, BM, BN, WVM, WVN, T)                                        \
   extern "C" __global__ void __launch_bounds__(WVM* WVN * 64)                                  \

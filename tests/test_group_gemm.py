@@ -137,3 +137,24 @@ def test_gpu_group_gemm_desc(ct, dev, tile, num_sm):
     ct.group_gemm_f16_nt_desc(ap, bp, cp, am, bmeta, cm, 2, generics=[tile, tile, 64, num_sm])
     torch.cuda.synchronize()
     assert rel_l2(c_t[1].float().cpu().numpy(), refs[1]) <= 1e-2 and torch.all(c_t[3] == 5.0) and torch.all(c_t[5] == 5.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("num_sm", [5, 256])
+def test_gpu_group_gemm_few_rows(ct, dev, num_sm):
+    """128 x 128 tiles: inner sizes around the depth of the ring, rows off every block, tiles of different groups in turn on one workgroup"""
+    shapes = [(1, 128, 16), (7, 144, 64), (33, 256, 80), (129, 16, 128), (2, 128, 144), (64, 400, 192), (130, 272, 208), (5, 128, 1040)]   # (m, n, k)
+    a_t, b_t, c_t, refs = [], [], [], []
+    for i, (m, n, k) in enumerate(shapes):
+        ab, bb = f16b(oracle.normal_f32((m, k), 891 + i)), f16b(oracle.normal_f32((k, n), 901 + i, 0, k ** -0.5))
+        a_t.append(_dev16(ab, dev))
+        b_t.append(_dev16(bb, dev))
+        c_t.append(torch.full((m + 1, n), 7.0, dtype=torch.half, device=dev))    # a row behind C that nothing may touch
+        refs.append(f16v(ab).astype(np.float64) @ f16v(bb).astype(np.float64))
+    (ap, am), (bp, bm), (cp, cm) = [_tables(t, dev) for t in (a_t, b_t, [c[:-1] for c in c_t])]
+    for _ in range(2):
+        ct.group_gemm_f16_nt_desc(ap, bp, cp, am, bm, cm, len(shapes), generics=[128, 128, 64, num_sm])
+    torch.cuda.synchronize()
+    for c, ref in zip(c_t, refs):
+        assert rel_l2(c[:-1].double().cpu().numpy(), ref) <= 2.0 ** -11      # one rounding to f16 over f32 sums
+        assert torch.all(c[-1] == 7.0)
