@@ -73,13 +73,19 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
   if (!s.own_tile || (ring && tiles(128, 128) < (uint64_t)cus / 2)) {
-    struct StagedTile { const char* kernel; int bm, bn, per_cu; double one, more; };   // us per K tile: alone on a compute unit, and each of several
-    static const StagedTile kStaged[] = {{"staged128x128", 128, 128, 2, 0.75, 0.62}, {"staged64x128", 64, 128, 3, 0.63, 0.38}, {"staged64x64", 64, 64, 4, 0.52, 0.235}};
+    // us per K tile: alone on a compute unit, and each of several; us of start and output.  256 x 128 fills a compute unit by itself:
+    // the fewest bytes per product, but nothing runs beside its start and its output, so it is the better one where K is long
+    // against them, and up to two rounds of workgroups (bf16, us with it, and with the best other tile: 2749 x 2583 x 8862 154, 182;
+    // 256 x 32003 x 4096 79, 91; 200 x 50021 x 1024, two rounds, 45, 47; 1000 x 20001 x 1024, three, 68, 59; 2746 x 2163 x 338 15.3, 13.6).
+    struct StagedTile { const char* kernel; int bm, bn, per_cu; double one, more, ends; };
+    static const StagedTile kStaged[] = {{"staged256x128", 256, 128, 1, 1.13, 1.13, 6.5}, {"staged128x128", 128, 128, 2, 0.75, 0.62, 5.0},
+                                         {"staged64x128", 64, 128, 3, 0.63, 0.38, 5.0}, {"staged64x64", 64, 64, 4, 0.52, 0.235, 5.0}};
     for (const StagedTile& r : kStaged) {
       if (s.y_cols < r.bn) continue;
       const uint64_t t = tiles(r.bm, r.bn), sk = r.bm * r.bn == 64 * 64 ? staged_splits(t, s.k, cus) : 1;
       const double w = (double)((t * sk + cus - 1) / cus);
-      const double us = kt / (double)sk * std::max(r.one * std::max(1.0, w / r.per_cu), r.more * w) + 5.0 +
+      if (r.per_cu == 1 && w > 2) continue;
+      const double us = kt / (double)sk * std::max(r.one * std::max(1.0, w / r.per_cu), r.more * w) + r.ends +
                         (sk > 1 ? 6.0 + 8e-6 / 5.0 * (double)(s.m * s.n * (int64_t)sk) : 0.0);
       if (us < best * 0.98) best = us, pick(r.kernel);
     }

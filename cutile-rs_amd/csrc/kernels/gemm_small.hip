@@ -433,7 +433,6 @@ GEMM_THIN_FAMILY(bf16f32, __bf16, float)
 #define GEMM_STAGED_FAMILY(T, IN_T, OUT_T)                     \
   GEMM_STAGED_KERNEL(T##_staged64x64, IN_T, OUT_T, 64, 64, 2, 2)    \
   GEMM_STAGED_KERNEL(T##_staged64x128, IN_T, OUT_T, 64, 128, 2, 2)  \
-  GEMM_STAGED_KERNEL(T##_staged128x64, IN_T, OUT_T, 128, 64, 2, 2)  \
   GEMM_STAGED_KERNEL(T##_staged128x128, IN_T, OUT_T, 128, 128, 2, 2) \
   GEMM_STAGED_KERNEL(T##_staged256x128, IN_T, OUT_T, 256, 128, 4, 2)
 GEMM_STAGED_FAMILY(bf16, __bf16, __bf16)

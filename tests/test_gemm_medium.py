@@ -29,8 +29,8 @@ def _run(ct, dev, m, n, k, dtype, variant, accumulate, tile=(128, 128)):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("tile", ["64x64", "64x128", "128x128"])
-@pytest.mark.parametrize("m,n,k", [(1, 128, 65), (65, 129, 64), (129, 255, 127), (128, 128, 200), (200, 131, 8), (67, 640, 4100), (130, 1001, 1030)])
+@pytest.mark.parametrize("tile", ["64x64", "64x128", "128x128", "256x128"])
+@pytest.mark.parametrize("m,n,k", [(1, 128, 65), (65, 129, 64), (129, 255, 127), (128, 128, 200), (200, 131, 8), (67, 640, 4100), (130, 1001, 1030), (257, 260, 192)])
 @pytest.mark.parametrize("dtype,accumulate", [("bf16", True), ("f16", False), ("bf16f32", True)])
 def test_gpu_staged_gemm(ct, dev, tile, m, n, k, dtype, accumulate):
     _run(ct, dev, m, n, k, dtype, f"{dtype}_staged{tile}", accumulate)
