@@ -347,9 +347,10 @@ uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 // The streaming GEMM variants ("..._s2x4"): a family of kernels behind one variant name.
 bool is_stream_variant(const char* variant) { return strstr(variant, "_s2x4") != nullptr; }
-// How many workgroups may share an output block of `floats` f32 values when a launch has `blocks` of them (1: none may).
+// How many workgroups may share an output block of `floats` f32 values when a launch has `blocks` of them (1: none may;
+// a launch over no block, from an explicit grid with a zero axis, is refused where it would be enqueued).
 uint32_t split_limit(uint64_t blocks, uint64_t floats) {
-  return blocks > kSplitCounters ? 1u : (uint32_t)std::max<uint64_t>(1, kSplitPartialBytes / (blocks * floats * sizeof(float)));
+  return blocks == 0 || blocks > kSplitCounters ? 1u : (uint32_t)std::max<uint64_t>(1, kSplitPartialBytes / (blocks * floats * sizeof(float)));
 }
 // The GEMM kernels that take any partition shape and any row alignment: tile[3] x tile[1] outputs a workgroup, thin ones
 // (strips of columns) and staged ones (tiles).

@@ -579,3 +579,18 @@ def test_tuning_records_choose_variants_per_shape_class_and_stale_ones_are_refus
         assert "refused" in report and "1 bucket(s) of kernel rms_norm_f16" in report
     finally:
         ct.tuning_reload(None)
+
+
+def test_gemm_over_no_tile_is_an_error_on_every_route(fake_hip):
+    """an explicit grid with a zero axis over a prefix partition: refused with a status, whichever kernel the sizes choose"""
+    ct = fake_hip
+    h = torch.half
+    for m, n, k, kernel in ((4, 4096, 4096, "_thin"), (300, 515, 1000, "_staged"), (2000, 4096, 1024, "_q"), (4, 64, 64, "_d")):
+        z = torch.zeros(m, n, dtype=h)
+        for grid in ((0, 1, 1), (1, 0, 1)):
+            n0 = ct.lib().cutile_testing_launch_count()
+            with pytest.raises(ct.CutileError, match="has a zero axis"):
+                ct.gemm(ct.partition(z, [128, 128], prefix=True), torch.zeros(m, k, dtype=h), torch.zeros(k, n, dtype=h), k, grid=grid)
+            assert ct.lib().cutile_testing_launch_count() == n0
+        ct.gemm(ct.partition(z, [128, 128]), torch.zeros(m, k, dtype=h), torch.zeros(k, n, dtype=h), k)
+        assert kernel in ct.last_resolved()["variant"]
