@@ -126,6 +126,7 @@ const char* f_hipGetErrorString(hipError_t e) {
     default: return "fake runtime error";
   }
 }
+hipError_t f_hipGetLastError(void) { return hipSuccess; }
 hipError_t f_hipStreamCreateWithFlags(hipStream_t* s, unsigned int) {
   FAKE_FAIL("hipStreamCreateWithFlags");
   *s = reinterpret_cast<hipStream_t>(new FakeStream());
@@ -392,6 +393,7 @@ HipApi make_fake_table() {
   t.hipDeviceTotalMem = f_hipDeviceTotalMem;
   t.hipGetDevicePropertiesR0600 = f_hipGetDeviceProperties;
   t.hipGetErrorString = f_hipGetErrorString;
+  t.hipGetLastError = f_hipGetLastError;
   t.hipStreamCreateWithFlags = f_hipStreamCreateWithFlags;
   t.hipStreamSynchronize = f_hipStreamSynchronize;
   t.hipStreamQuery = f_hipStreamQuery;

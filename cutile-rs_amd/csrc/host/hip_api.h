@@ -23,6 +23,7 @@ namespace cutile {
   X(hipDeviceTotalMem, hipError_t, (size_t*, hipDevice_t))                                             \
   X(hipGetDevicePropertiesR0600, hipError_t, (hipDeviceProp_tR0600*, int))                             \
   X(hipGetErrorString, const char*, (hipError_t))                                                      \
+  X(hipGetLastError, hipError_t, (void))                                                               \
   X(hipStreamCreateWithFlags, hipError_t, (hipStream_t*, unsigned int))                                \
   X(hipStreamSynchronize, hipError_t, (hipStream_t))                                                   \
   X(hipStreamQuery, hipError_t, (hipStream_t))                                                         \

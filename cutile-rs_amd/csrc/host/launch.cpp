@@ -411,7 +411,7 @@ cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutil
     uint32_t splits = std::min(scaled_splits(blocks, pieces, cus),
                                split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
-      if (cutile_status_t s = split_workspace(res.device, (hipStream_t)stream, &ws)) return s;
+      ws = split_workspace(res.device, (hipStream_t)stream);
       if (!ws.partials) splits = 1;
     }
     args.push_val<void*>(ws.partials);
@@ -2130,7 +2130,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     uint32_t splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
-      if (cutile_status_t s = split_workspace(res.device, (hipStream_t)stream, &ws)) return s;
+      ws = split_workspace(res.device, (hipStream_t)stream);
       if (!ws.partials) splits = 1;
     }
     args.push_val<void*>(ws.partials);

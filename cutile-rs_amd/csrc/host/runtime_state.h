@@ -24,6 +24,7 @@ struct cutile_device {
   uint64_t streams_created = 0;
   std::atomic<int> compute_units{0};  // filled on first use by compute_units()
   std::map<hipStream_t, void*> split_workspaces;   // workspace.cpp
+  uint32_t split_retry_after = 0;                  // launches to go before a refused workspace is asked for again
   // Code objects of the kernel table loaded on this device: image id -> module.
   std::map<int, cutile_module*> table_modules;
   // Resolved functions: symbol -> hipFunction_t.
@@ -47,7 +48,7 @@ struct SplitWorkspace {
   float* partials = nullptr;      // nullptr: none to be had, the launch must not split
   uint32_t* counters = nullptr;   // kSplitCounters words, all 0 between launches
 };
-cutile_status_t split_workspace(cutile_device_t device, hipStream_t stream, SplitWorkspace* out);
+SplitWorkspace split_workspace(cutile_device_t device, hipStream_t stream);
 void release_split_workspace(cutile_device_t device, hipStream_t stream);
 // The device of that ordinal if cutile_device_get has handed it out before, else nullptr.
 cutile_device_t known_device(int ordinal);

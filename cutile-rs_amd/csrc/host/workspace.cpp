@@ -5,37 +5,54 @@
 // streams never share one.  A stream handle names another stream only after the runtime has drained and freed the first.
 // At most kMaxWorkspaces per device (16 MiB each); cutile_stream_release gives back the one of its stream.  Where there is
 // none to be had, the caller launches its unsplit form: beyond the limit, while the stream is being captured (a graph may
-// be replayed on another stream beside eager work on this one), and on the per-thread default stream (one handle, many streams).
+// be replayed on another stream beside eager work on this one), on the per-thread default stream (one handle, many streams),
+// and where the runtime refuses the memory (another allocator may hold the card): a product needs none to be computed.
 #include "runtime_state.h"
 
 namespace cutile {
 namespace {
 constexpr size_t kMaxWorkspaces = 16;
-}
+// After a refused allocation this many launches of streams without a workspace go ahead unsplit before it is asked for again:
+// a request that fails costs more than the launch.
+constexpr uint32_t kRetryAfter = 256;
 
-cutile_status_t split_workspace(cutile_device_t device, hipStream_t stream, SplitWorkspace* out) {
-  *out = {};
-  CUTILE_API_OR_RETURN(api);
-  if (stream == hipStreamPerThread) return CUTILE_SUCCESS;
+// The runtime's own record of a refusal that is dealt with here: the next call of somebody else would report it.
+SplitWorkspace none_to_be_had(const HipApi* api) {
+  api->hipGetLastError();
+  return {};
+}
+}  // namespace
+
+SplitWorkspace split_workspace(cutile_device_t device, hipStream_t stream) {
+  const HipApi* api = hip();
+  if (!api || stream == hipStreamPerThread) return {};
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  CUTILE_HIP_OR_RETURN(api, hipStreamIsCapturing(stream, &capture));
-  if (capture != hipStreamCaptureStatusNone) return CUTILE_SUCCESS;
+  if (api->hipStreamIsCapturing(stream, &capture) != hipSuccess) return none_to_be_had(api);   // the launch itself will say why
+  if (capture != hipStreamCaptureStatusNone) return {};
   std::lock_guard<std::mutex> lock(device->mutex);
   auto it = device->split_workspaces.find(stream);
   if (it == device->split_workspaces.end()) {
-    if (device->split_workspaces.size() >= kMaxWorkspaces) return CUTILE_SUCCESS;
+    if (device->split_workspaces.size() >= kMaxWorkspaces) return {};
+    if (device->split_retry_after > 0) {
+      --device->split_retry_after;
+      return {};
+    }
     void* p = nullptr;
-    CUTILE_HIP_OR_RETURN(api, hipMallocAsync(&p, kSplitCounters * sizeof(uint32_t) + kSplitPartialBytes, stream));
-    const hipError_t e = api->hipMemsetD8Async((hipDeviceptr_t)p, 0, kSplitCounters * sizeof(uint32_t), stream);
-    if (e != hipSuccess) {
+    if (api->hipMallocAsync(&p, kSplitCounters * sizeof(uint32_t) + kSplitPartialBytes, stream) != hipSuccess) {
+      device->split_retry_after = kRetryAfter;
+      return none_to_be_had(api);
+    }
+    if (api->hipMemsetD8Async((hipDeviceptr_t)p, 0, kSplitCounters * sizeof(uint32_t), stream) != hipSuccess) {
       api->hipFreeAsync(p, stream);
-      return from_hip(e, "hipMemsetD8Async");
+      device->split_retry_after = kRetryAfter;
+      return none_to_be_had(api);
     }
     it = device->split_workspaces.emplace(stream, p).first;
   }
-  out->counters = (uint32_t*)it->second;
-  out->partials = (float*)((unsigned char*)it->second + kSplitCounters * sizeof(uint32_t));
-  return CUTILE_SUCCESS;
+  SplitWorkspace ws;
+  ws.counters = (uint32_t*)it->second;
+  ws.partials = (float*)((unsigned char*)it->second + kSplitCounters * sizeof(uint32_t));
+  return ws;
 }
 
 void release_split_workspace(cutile_device_t device, hipStream_t stream) {

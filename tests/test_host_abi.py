@@ -594,3 +594,48 @@ def test_gemm_over_no_tile_is_an_error_on_every_route(fake_hip):
             assert ct.lib().cutile_testing_launch_count() == n0
         ct.gemm(ct.partition(z, [128, 128]), torch.zeros(m, k, dtype=h), torch.zeros(k, n, dtype=h), k)
         assert kernel in ct.last_resolved()["variant"]
+
+
+def _split_products(ct):
+    """one launch of each family that shares K between workgroups: (launch, workgroups of the split grid, of the unsplit one)"""
+    h, u8 = torch.half, torch.uint8
+    x, y, z = torch.zeros(1, 4096, dtype=h), torch.zeros(4096, 4096, dtype=h), torch.zeros(1, 4096, dtype=h)
+    xo, yo, zo = torch.zeros(200, 4099, dtype=h), torch.zeros(4099, 515, dtype=h), torch.zeros(200, 515, dtype=h)
+    q, w, zq = torch.zeros(64, 8192, dtype=u8), torch.zeros(1024, 8192, dtype=u8), torch.zeros(64, 1024, dtype=torch.bfloat16)
+    qs, ws = torch.zeros(64, 256, dtype=u8), torch.zeros(1024, 256, dtype=u8)
+    return [("_thin", lambda s=None: ct.gemm(ct.partition(z, [128, 128]), x, y, 4096, stream=s)),
+            ("_staged", lambda s=None: ct.gemm(ct.partition(zo, [128, 128]), xo, yo, 4099, stream=s)),
+            ("_flat", lambda s=None: ct.linear_tile_mxfp8(ct.partition(zq, [128, 128]), q, w, qs, ws, stream=s))]
+
+
+def _workgroups(ct):
+    rec, _ = _last(ct)
+    return rec.grid[0] * rec.grid[1] * rec.grid[2]
+
+
+def _new_stream(ct):
+    dev, stream = C.c_void_p(), C.c_void_p()
+    ct.check(ct.lib().cutile_device_get(0, C.byref(dev)))
+    ct.check(ct.lib().cutile_stream_create(dev, C.byref(stream)))
+    return dev, stream
+
+
+@pytest.mark.parametrize("refused", ["hipMallocAsync", "hipMemsetD8Async", "hipStreamIsCapturing"])
+def test_split_products_run_unsplit_where_the_runtime_refuses_their_workspace(fake_hip, refused):
+    """out of memory (or any other refusal) on a stream's first split launch is not the launch's error: it runs unsplit, the
+    next launches do not ask again at once, and the workspace is had once the memory is there"""
+    ct = fake_hip
+    for kernel, launch in _split_products(ct):
+        dev, stream = _new_stream(ct)
+        ct.check(ct.lib().cutile_testing_inject_failure(refused.encode(), 2, 1))
+        launch(stream.value)
+        assert kernel in ct.last_resolved()["variant"]
+        unsplit = _workgroups(ct)
+        counts = []
+        for _ in range(300):
+            launch(stream.value)
+            counts.append(_workgroups(ct))
+        assert counts[-1] > unsplit and counts == sorted(counts) and set(counts) == {unsplit, counts[-1]} - ({unsplit} if counts[0] > unsplit else set())
+        if refused != "hipStreamIsCapturing":
+            assert counts.count(unsplit) == 256
+        ct.check(ct.lib().cutile_stream_release(dev, stream))
