@@ -11,7 +11,9 @@
 
 namespace cutile {
 namespace {
-constexpr size_t kMaxWorkspaces = 16;
+// More than the 32 streams that torch's pool deals out on a device, its default stream and as many of a program's own: a
+// stream made elsewhere keeps its workspace until the process ends (nothing tells this library that it is gone).  1 GiB at most.
+constexpr size_t kMaxWorkspaces = 64;
 // After a refused allocation this many launches of streams without a workspace go ahead unsplit before it is asked for again:
 // a request that fails costs more than the launch.
 constexpr uint32_t kRetryAfter = 256;

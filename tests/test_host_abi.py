@@ -639,3 +639,22 @@ def test_split_products_run_unsplit_where_the_runtime_refuses_their_workspace(fa
         if refused != "hipStreamIsCapturing":
             assert counts.count(unsplit) == 256
         ct.check(ct.lib().cutile_stream_release(dev, stream))
+
+
+def test_split_products_on_more_streams_than_a_pool_deals_out(fake_hip):
+    """48 streams of a process split K (a stream pool holds 32); beyond the limit a stream runs unsplit until another is released"""
+    ct = fake_hip
+    _, launch = _split_products(ct)[0]
+    launch()
+    split = _workgroups(ct)
+    streams, counts = [], []
+    for _ in range(70):
+        streams.append(_new_stream(ct))
+        launch(streams[-1][1].value)
+        counts.append(_workgroups(ct))
+    assert counts[:48] == [split] * 48 and counts[-1] < split and counts == sorted(counts, reverse=True)
+    ct.check(ct.lib().cutile_stream_release(*streams[0]))
+    launch(streams[-1][1].value)
+    assert _workgroups(ct) == split
+    for pair in streams[1:]:
+        ct.check(ct.lib().cutile_stream_release(*pair))
