@@ -26,9 +26,11 @@ struct GemmChoice {
 inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus) {
   return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8 * 2)));
 }
-// K splits of a staged launch: up to two workgroups per compute unit, at least 8 K tiles each (1262 x 128 x 16128, 40 tiles of
-// 64 x 64: 99, 54, 40, 32, 30 us with 1, 2, 3, 4, 8 splits; 128 x 4096 x 4096, 128 tiles: 40, 28.5, 28.0, 28.2, 47).
-inline uint32_t staged_splits(uint64_t blocks, int32_t k, int cus) {
+// K splits of a staged launch, as priced below and as launched: 64 x 64 tiles only (64 x 128 with two splits and with none: 336 x
+// 2575 x 1350 21.9, 17.8 us; 586 x 1537 x 1527 25.8, 20.4; 193 x 867 x 1070 17.0, 15.5; 130 x 1001 x 1030 15.8, 14.4), up to two workgroups per compute unit, at least 8 K tiles each (1262 x 128 x 16128, 40 tiles: 99, 54, 40, 32,
+// 30 us with 1, 2, 3, 4, 8 splits; 128 x 4096 x 4096, 128 tiles: 40, 28.5, 28.0, 28.2, 47).
+inline uint32_t staged_splits(int bm, int bn, uint64_t blocks, int32_t k, int cus) {
+  if (bm != 64 || bn != 64) return 1;
   return (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(int64_t)(2 * (uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8), 8}));
 }
 
@@ -82,7 +84,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
                                          {"staged64x128", 64, 128, 3, 0.63, 0.38, 5.0}, {"staged64x64", 64, 64, 4, 0.52, 0.235, 5.0}};
     for (const StagedTile& r : kStaged) {
       if (s.y_cols < r.bn) continue;
-      const uint64_t t = tiles(r.bm, r.bn), sk = r.bm * r.bn == 64 * 64 ? staged_splits(t, s.k, cus) : 1;
+      const uint64_t t = tiles(r.bm, r.bn), sk = staged_splits(r.bm, r.bn, t, s.k, cus);
       const double w = (double)((t * sk + cus - 1) / cus);
       if (r.per_cu == 1 && w > 2) continue;
       const double us = kt / (double)sk * std::max(r.one * std::max(1.0, w / r.per_cu), r.more * w) + r.ends +

@@ -2127,7 +2127,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
     SplitWorkspace ws;
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
-    uint32_t splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(blocks, k_valid, cus);
+    uint32_t splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
       ws = split_workspace(res.device, (hipStream_t)stream);

@@ -189,9 +189,10 @@ struct GemmThin {
 // For the outputs that are too few 256 x 256 tiles to fill the chip, and for rows that do not start on 16-byte boundaries
 // (the direct global -> LDS fetches of gemm_bf16.hip cannot take those).  K tiles of 64 go global -> registers -> LDS: two
 // tiles are in flight in registers while a third is multiplied out of one of two LDS stages, so a load has two K tiles to
-// land and one barrier per K tile is enough.  gridDim.z workgroups share the K tiles of an output tile.
+// land and one barrier per K tile is enough.  Several workgroups may share the K tiles of a 64 x 64 output tile (SPLIT).
 template <int BM, int BN, int WAVES_M, int WAVES_N, typename OutT, typename InT>
 struct GemmStaged {
+  static constexpr bool SPLIT = BM == 64 && BN == 64;   // the tile that the launcher splits (staged_splits)
   static constexpr int BK = 64, kWaves = WAVES_M * WAVES_N, kThreads = kWaves * 64;
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 16, TN = WN / 16;
   static constexpr int UB = BN / 8;                                    // 16-byte units of a y-tile row
@@ -214,7 +215,8 @@ struct GemmStaged {
 
   __device__ static void run(const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y, int32_t k_total, int32_t cover_m,
                              int32_t cover_n, int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n,
-                             uint32_t splits) {
+                             uint32_t launch_splits) {
+    const uint32_t splits = SPLIT ? launch_splits : 1;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
     __shared__ uint32_t last;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

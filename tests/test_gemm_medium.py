@@ -62,3 +62,17 @@ def test_rows_of_x_or_columns_of_y_missing_leave_the_size_rule(fake_hip):
     assert ct.last_resolved()["variant"] == "f16_generic"
     ct.gemm(ct.partition(z, [128, 128]), torch.empty(300, 1001, dtype=h), torch.empty(1001, 511, dtype=h), 1001)
     assert ct.last_resolved()["variant"] == "f16_generic"
+
+
+def test_staged_launches_split_what_the_size_rule_prices(fake_hip):
+    """64 x 64 tiles share K between workgroups, the larger staged tiles never do: chosen by size or named by the caller"""
+    ct = fake_hip
+    from test_host_abi import _workgroups
+    h = torch.half
+    for m, n, k, variant, tiles, split in ((336, 2575, 1350, None, 6 * 21, False), (300, 515, 4000, None, 5 * 9, True),
+                                           (336, 2575, 1350, "f16_staged64x64", 6 * 41, True), (300, 515, 4000, "f16_staged128x128", 3 * 5, False),
+                                           (300, 515, 4000, "f16_staged64x128", 5 * 5, False), (300, 515, 4000, "f16_staged256x128", 2 * 5, False)):
+        ct.gemm(ct.partition(torch.empty(m, n, dtype=h), [128, 128]), torch.empty(m, k, dtype=h), torch.empty(k, n, dtype=h), k, variant=variant)
+        got = ct.last_resolved()["variant"]
+        assert got == (variant or ("f16_staged64x64" if split else "f16_staged64x128"))
+        assert _workgroups(ct) % tiles == 0 and (_workgroups(ct) > tiles) == split
