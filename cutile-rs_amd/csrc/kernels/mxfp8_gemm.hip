@@ -734,7 +734,9 @@ struct MxGemmDirect16 {
 
 MX_KERNEL(mxfp8_bf16_256x256x128_w2x2, 256, 256, 2, 2, __bf16)
 MX_KERNEL(mxfp8_bf16_256x256x128_w2x4, 256, 256, 2, 4, __bf16)
+MX_KERNEL(mxfp8_bf16_128x128x128_w2x2, 128, 128, 2, 2, __bf16)
 MX_KERNEL(mxfp8_f32_256x256x128_w2x2, 256, 256, 2, 2, float)
+MX_KERNEL(mxfp8_f32_128x128x128_w2x2, 128, 128, 2, 2, float)
 MX_KERNEL(mxfp8_f32_32x32x128_w1x1, 32, 32, 1, 1, float)
 MX_KERNEL(mxfp8_f32_64x64x128_w1x1, 64, 64, 1, 1, float)
 
@@ -758,7 +760,7 @@ MX_DIRECT_KERNEL(mxfp8_f32_256x256x128_d2x4, 256, 256, 2, 4, float)
 
 MX_DIRECT16_KERNEL(mxfp8_bf16_256x256x128_e4x2, 256, 256, 4, 2, __bf16)
 MX_DIRECT16_KERNEL(mxfp8_f32_256x256x128_e4x2, 256, 256, 4, 2, float)
-// 128 x 128 tiles, two workgroups to a compute unit: against the register-staged form, which it replaced, 1000 x 4096 x 4096 38.5 -> 26.3 us,
+// 128 x 128 tiles, two workgroups to a compute unit: against the register-staged form (only for callers that name it), 1000 x 4096 x 4096 38.5 -> 26.3 us,
 // 2000 x 4096 x 4096 65 -> 41 us, with the same error (1.60e-5 against 64 bits, both).  Alone on a compute unit it waits for memory.
 MX_DIRECT16_KERNEL(mxfp8_bf16_128x128x128_e2x2, 128, 128, 2, 2, __bf16)
 MX_DIRECT16_KERNEL(mxfp8_f32_128x128x128_e2x2, 128, 128, 2, 2, float)

@@ -72,3 +72,34 @@ def test_gpu_scaled_rule(ct, dev):
     assert "flat" not in chosen(16, 4096, 4096, scales=lambda r, c: torch.zeros(r, c + 2, dtype=torch.uint8, device=dev)[:, :c])
     assert "flat" not in chosen(512, 512, 4096, tile=(256, 256), grid=(1, 1, 1))
     torch.cuda.synchronize()
+
+
+def test_register_staged_mxfp8_tiles_of_128_by_name(fake_hip):
+    """a caller's or a tuner's name for the register-staged 128 x 128 kernel holds; left to itself a launch takes the direct one"""
+    ct = fake_hip
+    u8 = lambda *shape: torch.zeros(*shape, dtype=torch.uint8)
+    for out, dt in (("bf16", torch.bfloat16), ("f32", torch.float32)):
+        launch = lambda **kw: ct.linear_tile_mxfp8(ct.partition(torch.zeros(128, 128, dtype=dt), [128, 128]), u8(128, 128), u8(128, 128), u8(128, 4),
+                                                   u8(128, 4), **kw)
+        launch()
+        assert ct.last_resolved()["variant"] == f"mxfp8_{out}_128x128x128_e2x2"
+        launch(variant=f"mxfp8_{out}_128x128x128_w2x2")
+        assert ct.last_resolved()["variant"] == f"mxfp8_{out}_128x128x128_w2x2" and ct.last_resolved()["source"] == "caller"
+        ct.set_preferred_variant("linear_tile", f"mxfp8_{out}_128x128x128_w2x2")
+        try:
+            launch()
+            assert ct.last_resolved()["variant"] == f"mxfp8_{out}_128x128x128_w2x2" and ct.last_resolved()["source"] == "pinned"
+        finally:
+            ct.set_preferred_variant("linear_tile", None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+def test_gpu_register_staged_mxfp8_tiles_of_128(ct, dev, out):
+    m, n, k = 130, 260, 640
+    (xq, xs), (yq, ys) = [oracle.mx_quantize_e4m3(oracle.normal_f32(s, 971)) for s in ((m, k), (n, k))]
+    ref = oracle.mx_gemm_f32(xq, yq, xs, ys, 1.0)
+    z = torch.full((m + 1, n), 7.0, dtype=torch.float32 if out == "f32" else torch.bfloat16, device=dev)
+    ct.linear_tile_mxfp8(ct.partition(z[:m], [128, 128]), *[_dev(v, dev) for v in (xq, yq, xs, ys)], 1.0, variant=f"mxfp8_{out}_128x128x128_w2x2")
+    torch.cuda.synchronize()
+    assert rel_l2(z[:m].float().cpu().numpy(), ref) <= (1e-4 if out == "f32" else 4e-3) and torch.all(z[m] == 7.0)
