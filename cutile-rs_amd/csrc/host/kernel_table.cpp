@@ -32,8 +32,18 @@ std::atomic<uint64_t> g_module_loads{0};
 std::mutex g_pref_mutex;
 std::map<std::string, std::string> g_preferred;
 std::atomic<size_t> g_preferred_count{0};
-// winners of tuning records: "function|bucket" -> variant
-std::map<std::string, std::string> g_bucket_preferred;
+// winners of shape classes: "function|bucket" -> variant, and whether a tuning record named it (otherwise the program, at run time)
+struct ClassWinner {
+  std::string variant;
+  bool from_record;
+};
+std::map<std::string, ClassWinner> g_bucket_preferred;
+std::atomic<size_t> g_run_time_winners{0};   // how many of them the program named
+void count_run_time_winners() {   // under g_pref_mutex
+  size_t n = 0;
+  for (const auto& kv : g_bucket_preferred) n += !kv.second.from_record;
+  g_run_time_winners.store(n, std::memory_order_release);
+}
 
 struct ImageRef {
   const unsigned char* start;
@@ -445,16 +455,32 @@ std::string preferred_variant(const char* function) {
   return it == g_preferred.end() ? std::string() : it->second;
 }
 
-std::string preferred_variant_for(const char* function, const std::string& bucket) {
-  if (bucket.empty()) return std::string();
+std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time) {
+  if (bucket.empty() || (at_run_time && g_run_time_winners.load(std::memory_order_acquire) == 0)) return std::string();
   std::lock_guard<std::mutex> lock(g_pref_mutex);
   auto it = g_bucket_preferred.find(std::string(function) + "|" + bucket);
-  return it == g_bucket_preferred.end() ? std::string() : it->second;
+  return it == g_bucket_preferred.end() || it->second.from_record == at_run_time ? std::string() : it->second.variant;
+}
+
+cutile_status_t set_class_winner(const char* function, const char* bucket, const char* variant, bool from_record) {
+  std::lock_guard<std::mutex> lock(g_pref_mutex);
+  const std::string key = std::string(function) + "|" + bucket;
+  if (!variant) {
+    g_bucket_preferred.erase(key);
+    count_run_time_winners();
+    return CUTILE_SUCCESS;
+  }
+  CUTILE_REQUIRE(find_entry(function, variant) != nullptr, CUTILE_ERR_KERNEL_NOT_FOUND,
+                 "no variant '%s' of kernel '%s'; available: %s", variant, function, list_variants(function).c_str());
+  g_bucket_preferred[key] = {variant, from_record};
+  count_run_time_winners();
+  return CUTILE_SUCCESS;
 }
 
 void clear_bucket_preferences() {
   std::lock_guard<std::mutex> lock(g_pref_mutex);
   g_bucket_preferred.clear();
+  count_run_time_winners();
 }
 
 void count_module_load() { g_module_loads.fetch_add(1, std::memory_order_relaxed); }
@@ -540,16 +566,8 @@ cutile_status_t cutile_kernel_set_preferred_variant(const char* function, const 
 
 cutile_status_t cutile_kernel_set_preferred_variant_for(const char* function, const char* bucket, const char* variant) {
   CUTILE_REQUIRE(function && bucket && *bucket, CUTILE_ERR_INVALID_ARGUMENT, "function or bucket is null");
-  std::lock_guard<std::mutex> lock(g_pref_mutex);
-  const std::string key = std::string(function) + "|" + bucket;
-  if (!variant) {
-    g_bucket_preferred.erase(key);
-    return CUTILE_SUCCESS;
-  }
-  CUTILE_REQUIRE(find_entry(function, variant) != nullptr, CUTILE_ERR_KERNEL_NOT_FOUND,
-                 "no variant '%s' of kernel '%s'; available: %s", variant, function, list_variants(function).c_str());
-  g_bucket_preferred[key] = variant;
-  return CUTILE_SUCCESS;
+  ensure_tuning_records_loaded();   // so that their loading at the first launch does not undo this call
+  return set_class_winner(function, bucket, variant, false);
 }
 
 const char* cutile_library_version(void) { return "0.1.0"; }

@@ -37,8 +37,9 @@ const KernelEntry* find_entry(const char* function, const std::string& variant);
 cutile_status_t load_entry(cutile_device_t device, const KernelEntry* entry, hipFunction_t* fn);
 // Preferred variant set through cutile_kernel_set_preferred_variant, or "".
 std::string preferred_variant(const char* function);
-// Winner a tuning record names for (function, shape-class bucket), or "".
-std::string preferred_variant_for(const char* function, const std::string& bucket);
+// Winner of (function, shape-class bucket) that the program set at run time, or (at_run_time false) that a tuning record names; or "".
+std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time);
+cutile_status_t set_class_winner(const char* function, const char* bucket, const char* variant, bool from_record);
 void clear_bucket_preferences();
 // Loads the tuning records once per process (tuning.cpp); cheap afterwards.
 void ensure_tuning_records_loaded();

@@ -277,9 +277,9 @@ cutile_status_t load_resolved(const char* function, const std::string& variant, 
 }
 
 // Picks the variant.  Precedence: the caller's variant, the function-wide pin set at run time
-// (cutile_kernel_set_preferred_variant), `sized` (the launcher's own rule for extents that the shape classes of the tuning
-// records do not tell apart), the shape class's winner (a verified tuning record or
-// cutile_kernel_set_preferred_variant_for), then `fallback` (the table's order).  A pin or a winner that does not fit
+// (cutile_kernel_set_preferred_variant), the shape class's winner set at run time (cutile_kernel_set_preferred_variant_for),
+// `sized` (the launcher's own rule for extents that the shape classes of the tuning records do not tell apart), the shape
+// class's winner of a verified tuning record, then `fallback` (the table's order).  A pin or a winner that does not fit
 // these arguments is passed over, not an error.
 cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* opts, const std::string& fallback,
                               const std::vector<std::string>& acceptable, Resolved* r, const std::string& sized = std::string()) {
@@ -295,18 +295,20 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
       g_last_source = "pinned";
     }
   }
-  if (want.empty() && fits(sized)) {
-    want = sized;
-    g_last_source = "size";
-  }
-  if (want.empty() && !g_bucket.empty()) {
+  auto class_winner = [&](bool at_run_time) {
     ensure_tuning_records_loaded();
-    std::string pref = preferred_variant_for(function, g_bucket);
+    std::string pref = preferred_variant_for(function, g_bucket, at_run_time);
     if (fits(pref)) {
       want = pref;
       g_last_source = "record:" + g_bucket;
     }
+  };
+  if (want.empty() && !g_bucket.empty()) class_winner(true);
+  if (want.empty() && fits(sized)) {
+    want = sized;
+    g_last_source = "size";
   }
+  if (want.empty() && !g_bucket.empty()) class_winner(false);
   if (want.empty()) {
     want = fallback;
     g_last_source = "table";
@@ -385,7 +387,8 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
     if (cutile_status_t s = current_device_units(cus)) return s;
     if (const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus)) sized = prefix + dt + "_" + kernel;
   }
-  if (!sized.empty() && !(opts && opts->variant) && preferred_variant(function).empty()) return resolve_own(function, sized.c_str(), "size", res);
+  if (!sized.empty() && !(opts && opts->variant) && preferred_variant(function).empty() && preferred_variant_for(function, g_bucket, true).empty())
+    return resolve_own(function, sized.c_str(), "size", res);
   std::vector<std::string> acceptable;
   for (const KernelEntry* e : fit) acceptable.push_back(e->variant);
   for (const KernelEntry* e : others) acceptable.push_back(e->variant);
@@ -2097,7 +2100,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   const std::string fallback = record_first ? sized.variant : own_tile ? own_tile->variant : dt + "_generic";
   if (record_first) sized.variant[0] = 0;
   ensure_tuning_records_loaded();
-  if ((opts && opts->variant) || !preferred_variant("gemm").empty() || (!sized.variant[0] && !preferred_variant_for("gemm", g_bucket).empty())) {
+  if ((opts && opts->variant) || !preferred_variant("gemm").empty() || !preferred_variant_for("gemm", g_bucket, true).empty() ||
+      (!sized.variant[0] && !preferred_variant_for("gemm", g_bucket, false).empty())) {
     if (cutile_status_t s = resolve_entry("gemm", opts, fallback, fitting(), &res, sized.variant)) return s;
   } else if (cutile_status_t s = resolve_own("gemm", sized.variant[0] ? sized.variant : fallback.c_str(), sized.variant[0] ? "size" : "table", &res)) {
     return s;

@@ -76,7 +76,7 @@ void load_directory(const std::string& dir) {
     for (auto& e : verified.value().first.entries) {
       auto v = e.config.str("variant");
       if (!v) continue;
-      if (cutile_kernel_set_preferred_variant_for(kernel.c_str(), e.bucket.c_str(), v->c_str()) == CUTILE_SUCCESS) ++n;
+      if (set_class_winner(kernel.c_str(), e.bucket.c_str(), v->c_str(), true) == CUTILE_SUCCESS) ++n;
       else g_report += "warning " + path + ": bucket " + e.bucket + " names an unknown variant " + *v + "\n";
     }
     g_applied += n;

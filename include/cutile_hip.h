@@ -231,7 +231,8 @@ cutile_status_t cutile_kernel_set_preferred_variant(const char* function, const 
 /* The same per shape class: `bucket` names the class a launcher derives from its arguments (what
  * cutile_last_resolved_bucket reports after a launch, e.g. "bf16_256x256|tiles>256" for gemm).  This is how the winners of
  * verified tuning records reach the launchers; order of precedence at a launch: the caller's variant, the function-wide
- * pin (an explicit run-time choice beats a file on disk), the bucket's winner, the table's order. */
+ * pin, the bucket's winner set by this call (explicit run-time choices beat rules and files), the launcher's own rule on
+ * extents (gemm and linear_tile*: finer than their buckets), the bucket's winner in a tuning record, the table's order. */
 cutile_status_t cutile_kernel_set_preferred_variant_for(const char* function, const char* bucket, const char* variant);
 /* Tuning records (cutile/src/tune.rs:762-1016): JSON records of autotuner winners, one file per kernel, in the directory
  * `tuned` beside the library (or $CUTILE_TUNING_RECORDS; empty = none), loaded on the first launcher call.  A record is

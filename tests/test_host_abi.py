@@ -658,3 +658,41 @@ def test_split_products_on_more_streams_than_a_pool_deals_out(fake_hip):
     assert _workgroups(ct) == split
     for pair in streams[1:]:
         ct.check(ct.lib().cutile_stream_release(*pair))
+
+
+def test_class_winner_set_at_run_time_beats_the_size_rule(fake_hip):
+    """set_preferred_variant_for decides where its variant fits, also where a launcher has a rule of its own; a winner that does
+    not fit is passed over, and taking it away gives the rule back"""
+    ct = fake_hip
+    h, u8 = torch.half, torch.uint8
+    gemm = lambda m, n, k: ct.gemm(ct.partition(torch.empty(m, n, dtype=h), [128, 128]), torch.empty(m, k, dtype=h), torch.empty(k, n, dtype=h), k)
+    linear = lambda m, n, k: ct.linear_tile_mxfp8(ct.partition(torch.empty(m, n, dtype=torch.bfloat16), [128, 128]), torch.empty(m, k, dtype=u8),
+                                                  torch.empty(n, k, dtype=u8), torch.empty(m, k // 32, dtype=u8), torch.empty(n, k // 32, dtype=u8))
+    for function, launch, pinned, unfit in (("gemm", lambda: gemm(2048, 2048, 2048), "f16_128x128x64_d2x2", "f16_256x256x64_d4x2"),
+                                            ("gemm", lambda: gemm(4, 4096, 4096), "f16_128x128x64_d2x2", "bf16_thin16x64"),
+                                            ("linear_tile", lambda: linear(16, 4096, 4096), "mxfp8_bf16_128x128x128_e2x2", "mxfp8_f32_64x64x128_w1x1")):
+        launch()
+        rule = ct.last_resolved()
+        assert rule["source"] == "size" and rule["variant"] != pinned
+        try:
+            ct.set_preferred_variant_for(function, rule["bucket"], pinned)
+            launch()
+            assert ct.last_resolved()["variant"] == pinned and ct.last_resolved()["source"] == "record:" + rule["bucket"]
+            ct.set_preferred_variant_for(function, rule["bucket"], unfit)
+            launch()
+            assert ct.last_resolved()["variant"] == rule["variant"] and ct.last_resolved()["source"] == "size"
+        finally:
+            ct.set_preferred_variant_for(function, rule["bucket"], None)
+        launch()
+        assert ct.last_resolved()["variant"] == rule["variant"]
+
+
+def test_class_winner_set_before_the_first_launch_holds():
+    """the tuning records are loaded at the first launch; a choice that the program made before it stays"""
+    import subprocess, sys
+
+    code = ("import torch, __graft_entry__ as e; ct = e.load_package(testing=True); ct.check(ct.lib().cutile_testing_use_fake_hip(1));"
+            "ct.set_preferred_variant_for('gemm', 'f16_128x128|tiles<=256', 'f16_128x128x64_d2x2'); h = torch.half;"
+            "ct.gemm(ct.partition(torch.empty(2048, 2048, dtype=h), [128, 128]), torch.empty(2048, 2048, dtype=h), torch.empty(2048, 2048, dtype=h), 2048);"
+            "assert ct.last_resolved()['variant'] == 'f16_128x128x64_d2x2', ct.last_resolved()")
+    subprocess.check_call([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
