@@ -96,7 +96,8 @@ struct GemmRing16 {
     const int32_t row0 = pm * BM, col0 = pn * BN;
     const int32_t k_valid = min(min(x.shape[1], y.shape[0]), k_total);
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(x.ptr, (uint32_t)(((int64_t)(M - 1) * lda + x.shape[1]) * 2));
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(y.ptr, (uint32_t)(((int64_t)(y.shape[0] - 1) * ldb + N) * 2));
+    // (a group of inner size 0 has no row of y: the prologue's masked fetches must still find themselves out of range)
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(y.ptr, y.shape[0] > 0 ? (uint32_t)(((int64_t)(y.shape[0] - 1) * ldb + N) * 2) : 0u);
     constexpr uint32_t kOob = 0x80000000u;
 
     // Global side of the fetches (per lane, K tile 0; the K advance is scalar).

@@ -158,3 +158,17 @@ def test_gpu_group_gemm_few_rows(ct, dev, num_sm):
     for c, ref in zip(c_t, refs):
         assert rel_l2(c[:-1].double().cpu().numpy(), ref) <= 2.0 ** -11      # one rounding to f16 over f32 sums
         assert torch.all(c[-1] == 7.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [128, 256])
+def test_gpu_group_gemm_without_inner_size(ct, dev, tile):
+    """an inner size of 0 beside ordinary groups: the empty sum is 0 and nothing of B is read, whatever its row stride"""
+    wide = torch.full((8, 640), float("nan"), dtype=torch.half, device=dev)
+    a_t = [torch.ones(130, 64, dtype=torch.half, device=dev)[:, :0], torch.ones(16, 32, dtype=torch.half, device=dev)]
+    b_t = [wide[:0, :272], torch.ones(32, 272, dtype=torch.half, device=dev)]
+    c_t = [torch.full((131, 272), 7.0, dtype=torch.half, device=dev)[:130], torch.full((16, 272), 7.0, dtype=torch.half, device=dev)]
+    (ap, am), (bp, bm), (cp, cm) = [_tables(t, dev) for t in (a_t, b_t, c_t)]
+    ct.group_gemm_f16_nt_desc(ap, bp, cp, am, bm, cm, 2, generics=[tile, tile, 64, 8])
+    torch.cuda.synchronize()
+    assert not c_t[0].any() and torch.all(c_t[1] == 32.0)
