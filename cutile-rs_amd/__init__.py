@@ -377,7 +377,8 @@ def _launcher(name: str):
         spec = importlib.util.spec_from_file_location("cutile_marshal", path)
         marshal = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(marshal)
-        _launchers.update({n: marshal.launcher(n, C.cast(getattr(lib(), "cutile_launch_" + n), C.c_void_p).value) for n in marshal.names()})
+        _launchers.update({n: marshal.launcher(n, C.cast(getattr(lib(), "cutile_launch_" + n), C.c_void_p).value, tensor_arg, Partition)
+                           for n in marshal.names()})
     return _launchers[name]
 
 

@@ -10,6 +10,7 @@
 #include <c10/core/ScalarType.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstring>
 #include <string>
 #include <tuple>
 #include <utility>
@@ -19,6 +20,30 @@
 namespace {
 
 PyObject *s_tensor, *s_shape, *s_prefix, *s_dtype, *s_arg;   // attribute names of the binding's Partition
+
+// What the binding does in Python for the objects that are not read here: anything that offers a tensor's or a partition's methods.
+struct Binding {
+  PyObject* tensor_arg;        // tensor_arg(object, element type or None) -> the ABI's record as a ctypes structure
+  PyObject* partition_type;    // the class Partition; objects of any other class are asked for their record: o.arg()
+};
+
+// Copies a ctypes structure; takes the reference.
+template <typename T>
+bool take_record(PyObject* record, T* out) {
+  if (!record) return false;
+  Py_buffer view;
+  bool ok = PyObject_GetBuffer(record, &view, PyBUF_SIMPLE) == 0;
+  if (ok) {
+    ok = view.len == (Py_ssize_t)sizeof(T);
+    if (ok)
+      memcpy(out, view.buf, sizeof(T));
+    else
+      PyErr_Format(PyExc_TypeError, "expected a record of %zd bytes, got one of %zd (%s)", (Py_ssize_t)sizeof(T), view.len, Py_TYPE(record)->tp_name);
+    PyBuffer_Release(&view);
+  }
+  Py_DECREF(record);
+  return ok;
+}
 
 int dtype_of(const at::Tensor& t) {
   switch (t.scalar_type()) {
@@ -42,11 +67,9 @@ int dtype_of(const at::Tensor& t) {
   }
 }
 
-bool fill_tensor(PyObject* o, int dtype, cutile_tensor_arg_t* a) try {
-  if (!THPVariable_Check(o)) {
-    PyErr_Format(PyExc_TypeError, "expected a torch tensor, got %s", Py_TYPE(o)->tp_name);
-    return false;
-  }
+bool fill_tensor(PyObject* o, int dtype, const Binding& b, cutile_tensor_arg_t* a) try {
+  if (!THPVariable_Check(o))
+    return take_record(dtype < 0 ? PyObject_CallFunctionObjArgs(b.tensor_arg, o, nullptr) : PyObject_CallFunction(b.tensor_arg, "Oi", o, dtype), a);
   const at::Tensor& t = THPVariable_Unpack(o);
   const int64_t rank = t.dim();
   if (rank > CUTILE_MAX_RANK) {
@@ -80,12 +103,13 @@ bool to_int(PyObject* o, long long* v) {
   return !(*v == -1 && PyErr_Occurred());
 }
 
-bool fill_partition(PyObject* o, cutile_partition_arg_t* p) {
+bool fill_partition(PyObject* o, const Binding& b, cutile_partition_arg_t* p) {
+  if ((PyObject*)Py_TYPE(o) != b.partition_type) return take_record(PyObject_CallMethodNoArgs(o, s_arg), p);
   PyObject *tensor = PyObject_GetAttr(o, s_tensor), *shape = nullptr, *prefix = nullptr, *dtype = nullptr;
   bool ok = tensor && (shape = PyObject_GetAttr(o, s_shape)) && (prefix = PyObject_GetAttr(o, s_prefix)) && (dtype = PyObject_GetAttr(o, s_dtype));
   long long code = -1;
   if (ok && dtype != Py_None) ok = to_int(dtype, &code);
-  ok = ok && fill_tensor(tensor, (int)code, &p->tensor);
+  ok = ok && fill_tensor(tensor, (int)code, b, &p->tensor);
   PyObject* seq = ok ? PySequence_Fast(shape, "a partition's shape is a sequence of integers") : nullptr;
   if ((ok = seq != nullptr)) {
     if (PySequence_Fast_GET_SIZE(seq) != p->tensor.rank) {
@@ -115,7 +139,7 @@ struct From;
 template <>
 struct From<void*> {   // a stream or a device address
   void* v;
-  bool read(PyObject* o) {
+  bool read(PyObject* o, const Binding&) {
     v = o == Py_None ? nullptr : PyLong_AsVoidPtr(o);
     return !PyErr_Occurred();
   }
@@ -126,7 +150,7 @@ struct From<const void*> : From<void*> {};
 template <>
 struct From<int32_t> {
   long long v;
-  bool read(PyObject* o) { return to_int(o, &v); }
+  bool read(PyObject* o, const Binding&) { return to_int(o, &v); }
   int32_t get() { return (int32_t)v; }
 };
 template <>
@@ -136,7 +160,7 @@ struct From<int64_t> : From<int32_t> {
 template <>
 struct From<double> {
   double v;
-  bool read(PyObject* o) {
+  bool read(PyObject* o, const Binding&) {
     v = PyFloat_AsDouble(o);
     return !(v == -1.0 && PyErr_Occurred());
   }
@@ -149,7 +173,7 @@ struct From<float> : From<double> {
 template <>
 struct From<const int32_t*> {   // a sequence of at most 8 integers
   int32_t v[8];
-  bool read(PyObject* o) {
+  bool read(PyObject* o, const Binding&) {
     PyObject* seq = PySequence_Fast(o, "expected a sequence of integers");
     bool ok = seq != nullptr;
     if (ok && PySequence_Fast_GET_SIZE(seq) > 8) {
@@ -170,18 +194,22 @@ template <>
 struct From<const cutile_tensor_arg_t*> {   // a tensor, (tensor, element type) or None
   cutile_tensor_arg_t a;
   bool present;
-  bool read(PyObject* o) {
+  bool read(PyObject* o, const Binding& b) {
     if (!(present = o != Py_None)) return true;
-    if (!PyTuple_Check(o)) return fill_tensor(o, -1, &a);
+    if (!PyTuple_Check(o)) return fill_tensor(o, -1, b, &a);
+    if (PyTuple_GET_SIZE(o) != 2) {
+      PyErr_SetString(PyExc_TypeError, "expected a tensor, got a tuple");
+      return false;
+    }
     long long code;
-    return to_int(PyTuple_GET_ITEM(o, 1), &code) && fill_tensor(PyTuple_GET_ITEM(o, 0), (int)code, &a);
+    return to_int(PyTuple_GET_ITEM(o, 1), &code) && fill_tensor(PyTuple_GET_ITEM(o, 0), (int)code, b, &a);
   }
   const cutile_tensor_arg_t* get() { return present ? &a : nullptr; }
 };
 template <>
 struct From<const cutile_partition_arg_t*> {
   cutile_partition_arg_t a;
-  bool read(PyObject* o) { return fill_partition(o, &a); }
+  bool read(PyObject* o, const Binding& b) { return fill_partition(o, b, &a); }
   const cutile_partition_arg_t* get() { return &a; }
 };
 template <>
@@ -190,7 +218,7 @@ struct From<const cutile_launch_opts_t*> {   // (grid or None, generics or None,
   cutile_launch_opts_t o{};
   std::string text[kMost];
   const char* items[kMost];
-  bool read(PyObject* t) {
+  bool read(PyObject* t, const Binding&) {
     if (t == Py_None) return true;
     PyObject *grid = PyTuple_GET_ITEM(t, 0), *generics = PyTuple_GET_ITEM(t, 1), *variant = PyTuple_GET_ITEM(t, 2);
     if (grid != Py_None) {
@@ -232,9 +260,9 @@ struct From<const cutile_launch_opts_t*> {   // (grid or None, generics or None,
 };
 
 template <typename... A, size_t... I>
-PyObject* call_with(cutile_status_t (*fn)(A...), PyObject* const* args, std::index_sequence<I...>) {
+PyObject* call_with(cutile_status_t (*fn)(A...), const Binding& b, PyObject* const* args, std::index_sequence<I...>) {
   std::tuple<From<A>...> from;
-  if (!(std::get<I>(from).read(args[I]) && ...)) return nullptr;
+  if (!(std::get<I>(from).read(args[I], b) && ...)) return nullptr;
   cutile_status_t status;
   Py_BEGIN_ALLOW_THREADS   // a launch may wait for room in a full queue
   status = fn(std::get<I>(from).get()...);
@@ -242,9 +270,9 @@ PyObject* call_with(cutile_status_t (*fn)(A...), PyObject* const* args, std::ind
   return PyLong_FromLong(status);
 }
 template <typename... A>
-PyObject* call(cutile_status_t (*fn)(A...), PyObject* const* args, Py_ssize_t n) {
+PyObject* call(cutile_status_t (*fn)(A...), const Binding& b, PyObject* const* args, Py_ssize_t n) {
   if (n != (Py_ssize_t)sizeof...(A)) return PyErr_Format(PyExc_TypeError, "the launcher takes %zd arguments, got %zd", (Py_ssize_t)sizeof...(A), n);
-  return call_with(fn, args, std::make_index_sequence<sizeof...(A)>());
+  return call_with(fn, b, args, std::make_index_sequence<sizeof...(A)>());
 }
 
 // A launcher of one loaded library: name -> signature from the header, address from the binding.
@@ -261,22 +289,29 @@ struct Launcher {
   PyObject_HEAD
   vectorcallfunc vectorcall;
   void* address;
-  PyObject* (*invoke)(void* address, PyObject* const* args, Py_ssize_t n);
+  Binding binding;             // owned references
+  PyObject* (*invoke)(const Launcher& l, PyObject* const* args, Py_ssize_t n);
 };
 PyObject* launcher_call(PyObject* self, PyObject* const* args, size_t nargsf, PyObject* kwnames) {
   if (kwnames && PyTuple_GET_SIZE(kwnames)) return PyErr_Format(PyExc_TypeError, "a launcher takes positional arguments only");
   Launcher* l = (Launcher*)self;
-  return l->invoke(l->address, args, PyVectorcall_NARGS(nargsf));
+  return l->invoke(*l, args, PyVectorcall_NARGS(nargsf));
+}
+void launcher_dealloc(PyObject* self) {
+  Binding& b = ((Launcher*)self)->binding;
+  Py_XDECREF(b.tensor_arg);
+  Py_XDECREF(b.partition_type);
+  PyObject_Free(self);
 }
 PyTypeObject launcher_type = {PyVarObject_HEAD_INIT(nullptr, 0) "cutile_marshal.Launcher", sizeof(Launcher)};
 
 #define INVOKE(NAME)                                                                      \
-  PyObject* invoke_##NAME(void* address, PyObject* const* args, Py_ssize_t n) {           \
-    return call(reinterpret_cast<decltype(&cutile_launch_##NAME)>(address), args, n);     \
+  PyObject* invoke_##NAME(const Launcher& l, PyObject* const* args, Py_ssize_t n) {       \
+    return call(reinterpret_cast<decltype(&cutile_launch_##NAME)>(l.address), l.binding, args, n); \
   }
 LAUNCHERS(INVOKE)
 
-const struct { const char* name; PyObject* (*invoke)(void*, PyObject* const*, Py_ssize_t); } kLaunchers[] = {
+const struct { const char* name; PyObject* (*invoke)(const Launcher&, PyObject* const*, Py_ssize_t); } kLaunchers[] = {
 #define ROW(NAME) {#NAME, invoke_##NAME},
     LAUNCHERS(ROW)};
 
@@ -297,13 +332,17 @@ PyObject* names(PyObject*, PyObject*) {
 PyObject* launcher(PyObject*, PyObject* args) {
   const char* name;
   unsigned long long address;
-  if (!PyArg_ParseTuple(args, "sK", &name, &address)) return nullptr;
+  PyObject *tensor_arg, *partition_type;
+  if (!PyArg_ParseTuple(args, "sKOO", &name, &address, &tensor_arg, &partition_type)) return nullptr;
   for (auto& k : kLaunchers)
     if (strcmp(k.name, name) == 0) {
       Launcher* l = PyObject_New(Launcher, &launcher_type);
       if (!l) return nullptr;
       l->vectorcall = launcher_call;
       l->address = (void*)(uintptr_t)address;
+      Py_INCREF(tensor_arg);
+      Py_INCREF(partition_type);
+      l->binding = {tensor_arg, partition_type};
       l->invoke = k.invoke;
       return (PyObject*)l;
     }
@@ -311,7 +350,7 @@ PyObject* launcher(PyObject*, PyObject* args) {
 }
 
 PyMethodDef methods[] = {{"names", names, METH_NOARGS, "names of the launchers this module can call"},
-                         {"launcher", launcher, METH_VARARGS, "launcher(name, address): the callable for cutile_launch_<name> at that address"},
+                         {"launcher", launcher, METH_VARARGS, "launcher(name, address, tensor_arg, Partition): the callable for cutile_launch_<name> at that address"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "cutile_marshal", nullptr, -1, methods};
 
@@ -326,7 +365,7 @@ PyMODINIT_FUNC PyInit_cutile_marshal() {
   launcher_type.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_VECTORCALL;
   launcher_type.tp_vectorcall_offset = offsetof(Launcher, vectorcall);
   launcher_type.tp_call = PyVectorcall_Call;
-  launcher_type.tp_dealloc = (destructor)PyObject_Free;
+  launcher_type.tp_dealloc = launcher_dealloc;
   if (PyType_Ready(&launcher_type) < 0) return nullptr;
   return PyModule_Create(&module);
 }

@@ -696,3 +696,50 @@ def test_class_winner_set_before_the_first_launch_holds():
             "ct.gemm(ct.partition(torch.empty(2048, 2048, dtype=h), [128, 128]), torch.empty(2048, 2048, dtype=h), torch.empty(2048, 2048, dtype=h), 2048);"
             "assert ct.last_resolved()['variant'] == 'f16_128x128x64_d2x2', ct.last_resolved()")
     subprocess.check_call([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
+def test_objects_that_only_offer_a_tensors_or_a_partitions_methods(fake_hip):
+    """a launcher takes what `tensor_arg` and `Partition.arg` read: the same launch as from the tensors themselves; everything
+    else is refused with an exception"""
+    ct = fake_hip
+
+    class Buffer:                # no torch tensor: what tensor_arg asks for
+        def __init__(self, t):
+            self.t, self.dtype, self.shape = t, t.dtype, t.shape
+        data_ptr = lambda self: self.t.data_ptr()
+        dim = lambda self: self.t.dim()
+        stride = lambda self, i: self.t.stride(i)
+
+    class Tiles:                 # no Partition: what a launcher asks for
+        def __init__(self, p):
+            self.p = p
+        arg = lambda self: self.p.arg()
+
+    class Halved(ct.Partition):  # a Partition that says itself what it is
+        def arg(self):
+            return ct.Partition(self.tensor[:2], self.shape).arg()
+
+    y, x = torch.zeros(4, 8), torch.ones(4, 8)
+    ct.saxpy(ct.partition(y, [2, 2]), 2.0, x)
+    rec, want = _last(ct)
+    grid = tuple(rec.grid)
+    for tiles in (ct.partition(Buffer(y), [2, 2]), Tiles(ct.partition(y, [2, 2])), Tiles(ct.partition(Buffer(y), [2, 2]))):
+        ct.saxpy(tiles, 2.0, Buffer(x))
+        rec, args = _last(ct)
+        assert args == want and tuple(rec.grid) == grid
+    ct.saxpy(ct.partition(y[:2], [2, 2]), 2.0, x[:2])
+    _, half = _last(ct)
+    ct.saxpy(Halved(y, [2, 2]), 2.0, x[:2])
+    assert _last(ct)[1] == half
+    # an element type stated by the launcher
+    ids, table, out = torch.zeros(4, dtype=torch.int32), torch.zeros(16, 8, dtype=torch.half), torch.zeros(4, 8, dtype=torch.half)
+    ct.embedding_batch_f16(ids, table, ct.partition(out, [1, 8]))
+    want = _last(ct)[1]
+    ct.embedding_batch_f16(Buffer(ids), Buffer(table), ct.partition(out, [1, 8]))
+    assert _last(ct)[1] == want
+    n0 = ct.lib().cutile_testing_launch_count()
+    for tiles, operand in ((ct.partition(y, [2, 2]), (x,)), (ct.partition(y, [2, 2]), ()), (ct.partition(y, [2, 2]), 3.0), (y, x), (None, x),
+                           (ct.mapped(ct.partition(y, [2, 2]), [1, 1], 1), x), (ct.partition(Buffer(y), [2]), x)):
+        with pytest.raises((AttributeError, TypeError, ct.CutileError)):
+            ct.saxpy(tiles, 2.0, operand)
+    assert ct.lib().cutile_testing_launch_count() == n0
