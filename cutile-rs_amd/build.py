@@ -161,14 +161,20 @@ def build_marshal(force: bool = False) -> str:
     """The CPython extension that reads torch tensors into the ABI's records for the Python binding (host code only)."""
     src = os.path.join(ROOT, "csrc", "bind", "marshal.cpp")
     header = os.path.join(ROOT, "..", "include", "cutile_hip.h")
-    if force or not _newer(MARSHAL_PATH, [src, header]):
-        import sysconfig
+    import sysconfig
 
-        import torch
+    import torch
+    # it reads torch's own tensor objects: another torch or interpreter than it was built with cannot load it, or worse, can
+    built_with = os.path.join(BUILD_DIR, "marshal_built_with.txt")
+    host = f"torch {torch.__version__}, python {sys.version}"
+    if force or not _newer(MARSHAL_PATH, [src, header]) or not os.path.exists(built_with) or open(built_with).read() != host:
         inc, libs = (os.path.join(os.path.dirname(torch.__file__), d) for d in ("include", "lib"))
         _run([CXX, "-std=c++17", "-O2", "-g0", "-fPIC", "-shared", "-w", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
               "-I" + sysconfig.get_paths()["include"], "-I" + inc, "-I" + os.path.join(inc, "torch", "csrc", "api", "include"), src, "-o", MARSHAL_PATH,
               "-L" + libs, "-ltorch_python", "-ltorch_cpu", "-lc10"])   # found by name: torch has loaded them
+        os.makedirs(BUILD_DIR, exist_ok=True)
+        with open(built_with, "w") as f:
+            f.write(host)
     return MARSHAL_PATH
 
 

@@ -743,3 +743,24 @@ def test_objects_that_only_offer_a_tensors_or_a_partitions_methods(fake_hip):
         with pytest.raises((AttributeError, TypeError, ct.CutileError)):
             ct.saxpy(tiles, 2.0, operand)
     assert ct.lib().cutile_testing_launch_count() == n0
+
+
+def test_marshalling_extension_is_rebuilt_for_another_torch(monkeypatch, tmp_path):
+    """it is compiled against torch's headers and reads torch's objects: a newer file is not enough to keep it"""
+    import __graft_entry__ as entry
+
+    build, compiled = entry._load_build_script(), []
+    monkeypatch.setattr(build, "BUILD_DIR", str(tmp_path))
+    monkeypatch.setattr(build, "MARSHAL_PATH", str(tmp_path / "cutile_marshal.so"))
+
+    def compile(command):
+        compiled.append(command)
+        (tmp_path / "cutile_marshal.so").write_bytes(b"")
+    monkeypatch.setattr(build, "_run", compile)
+    for _ in range(2):
+        build.build_marshal()
+    assert len(compiled) == 1
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    for _ in range(2):
+        build.build_marshal()
+    assert len(compiled) == 2
