@@ -53,23 +53,25 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
   const double kt = s.k / 64.0;
   double best = 1e30;
   // The ring kernels.  One K tile of a launch that fills few compute units costs `few` us, of one that fills all of them `all`
-  // us (operands through the same L2s, and the clock): from 4096-deep products with 64 to 256 tiles of each shape.  1500 x 14336 x
-  // 4096 predicted 152, 172, 169 us for 192 x 256, 256 x 256, 128 x 256 tiles, measured 152, 172, 168.
-  struct RingTile { const char* kernel; int bm, bn; double few, all; };
-  static const RingTile kRing[] = {{"256x256x64_q2x4", 256, 256, 1.08, 1.42}, {"192x256x64_q2x4", 192, 256, 0.88, 1.12}, {"256x128x64_q4x2", 256, 128, 0.67, 0.82},
-                                   {"128x256x64_q2x4", 128, 256, 0.68, 0.82}, {"192x128x64_q2x2", 192, 128, 0.66, 0.74}};
+  // us (operands through the same L2s, and the clock), and a round of workgroups `ends` us besides: least squares over 744 products of 65 to
+  // 6000 rows, f16 and bf16, every kernel timed on operands that stay in the caches and on operands from memory, and the mean of the
+  // two taken (each within 10 % for nine products in ten).  1500 x 14336 x 4096: 160, 186, 190 us for 192 x 256, 256 x 256, 128 x 256 tiles.
+  struct RingTile { const char* kernel; int bm, bn; double few, all, ends; };
+  static const RingTile kRing[] = {{"256x256x64_q2x4", 256, 256, 1.04, 1.50, 7.3}, {"192x256x64_q2x4", 192, 256, 0.83, 1.20, 6.3}, {"256x128x64_q4x2", 256, 128, 0.65, 0.88, 5.3},
+                                   {"128x256x64_q2x4", 128, 256, 0.63, 0.95, 5.1}, {"192x128x64_q2x2", 192, 128, 0.615, 0.75, 5.5}};
   // (up to K = 512 the start and the output of a tile are most of a launch: the partition's own tile, if it has kernels)
   const bool ring = s.aligned && (s.k > 512 || !s.own_tile) && strcmp(s.dtype, "bf16f32") != 0;
   if (ring) {
     for (const RingTile& r : kRing) {
       const uint64_t t = tiles(r.bm, r.bn), rest = t % cus;
-      const double us = kt * ((double)(t / cus) * r.all + (rest ? r.few + (r.all - r.few) * (double)rest / cus : 0.0)) + 4.0 * (double)((t + cus - 1) / cus);
+      const double us = kt * ((double)(t / cus) * r.all + (rest ? r.few + (r.all - r.few) * (double)rest / cus : 0.0)) + r.ends * (double)((t + cus - 1) / cus);
       if (us < best * 0.98) best = us, pick(r.kernel);
     }
-    // 128 x 128: two workgroups to a compute unit
+    // 128 x 128: two workgroups to a compute unit, each at half its pace as soon as there are more than compute units (1623 x 2944 x
+    // 14016 f16, 299 tiles: 214 us, 192 x 128 tiles 151; 619 x 8832 x 7552 bf16, 345 tiles: 137, 256 x 128 tiles 90)
     const uint64_t t = tiles(128, 128), slots = 2 * (uint64_t)cus, rest = t % slots;
-    const double part = rest == 0 ? 0.0 : rest <= (uint64_t)cus ? 0.50 + 0.12 * (double)rest / cus : 0.62 + 0.38 * (double)(rest - cus) / cus;
-    const double us = kt * ((double)(t / slots) * 1.0 + part) + 4.0 * (double)((t + slots - 1) / slots);
+    const double part = rest == 0 ? 0.0 : rest <= (uint64_t)cus ? 0.475 + 0.125 * (double)rest / cus : 1.05 + 0.02 * (double)(rest - cus) / cus;
+    const double us = kt * ((double)(t / slots) * 1.07 + part) + 4.5 * (double)((t + slots - 1) / slots);
     if (us < best * 0.98) best = us, pick("128x128x64_q2x2");
   }
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
@@ -79,16 +81,24 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
     // the fewest bytes per product, but nothing runs beside its start and its output, so it is the better one where K is long
     // against them, and up to two rounds of workgroups (bf16, us with it, and with the best other tile: 2749 x 2583 x 8862 154, 182;
     // 256 x 32003 x 4096 79, 91; 200 x 50021 x 1024, two rounds, 45, 47; 1000 x 20001 x 1024, three, 68, 59; 2746 x 2163 x 338 15.3, 13.6).
-    struct StagedTile { const char* kernel; int bm, bn, per_cu; double one, more, ends; };
-    static const StagedTile kStaged[] = {{"staged256x128", 256, 128, 1, 1.13, 1.13, 6.5}, {"staged128x128", 128, 128, 2, 0.75, 0.62, 5.0},
-                                         {"staged64x128", 64, 128, 3, 0.63, 0.38, 5.0}, {"staged64x64", 64, 64, 4, 0.52, 0.235, 5.0}};
+    // Rows on 16-byte boundaries cost less (the second set, fitted like the ring's; the splits' share too): with the first set, ring tiles
+    // were taken for small outputs of middling K (us with ring, 64 x 64 and two-stage tiles: 220 x 64 x 1408 14.4, 9.3, 11.5; 665 x 320 x 704 9.5,
+    // 6.7, 8.2; from memory 14.6, 10.1, 14.9 and 10.2, 7.7, 10.5).  The two-stage tiles are the better ones where operands are in the
+    // caches and K is about 1500 (936 x 640 x 1536 12.7 us, ring 16.0), and the worse ones where they are not (21.6, 17.5).
+    struct Cost { double one, more, ends, split, sum; };
+    struct StagedTile { const char* kernel; int bm, bn, per_cu; Cost any, aligned; };
+    static const StagedTile kStaged[] = {{"staged256x128", 256, 128, 1, {1.13, 1.13, 6.5, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
+                                         {"staged128x128", 128, 128, 2, {0.75, 0.62, 5.0, 0, 0}, {0.715, 0.625, 5.05, 0, 0}},
+                                         {"staged64x128", 64, 128, 3, {0.63, 0.38, 5.0, 0, 0}, {0.55, 0.43, 3.9, 0, 0}},
+                                         {"staged64x64", 64, 64, 4, {0.52, 0.235, 5.0, 6.0, 1.6e-6}, {0.32, 0.257, 3.6, 4.1, 4.4e-6}}};
     for (const StagedTile& r : kStaged) {
       if (s.y_cols < r.bn) continue;
       const uint64_t t = tiles(r.bm, r.bn), sk = staged_splits(r.bm, r.bn, t, s.k, cus);
       const double w = (double)((t * sk + cus - 1) / cus);
       if (r.per_cu == 1 && w > 2) continue;
-      const double us = kt / (double)sk * std::max(r.one * std::max(1.0, w / r.per_cu), r.more * w) + r.ends +
-                        (sk > 1 ? 6.0 + 8e-6 / 5.0 * (double)(s.m * s.n * (int64_t)sk) : 0.0);
+      const Cost& c1 = ring ? r.aligned : r.any;
+      const double us = kt / (double)sk * std::max(c1.one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
+                        (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
       if (us < best * 0.98) best = us, pick(r.kernel);
     }
   }

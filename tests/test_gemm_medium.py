@@ -76,3 +76,16 @@ def test_staged_launches_split_what_the_size_rule_prices(fake_hip):
         got = ct.last_resolved()["variant"]
         assert got == (variant or ("f16_staged64x64" if split else "f16_staged64x128"))
         assert _workgroups(ct) % tiles == 0 and (_workgroups(ct) > tiles) == split
+
+
+def test_small_outputs_of_middling_inner_size_take_staged_tiles(fake_hip):
+    """the size rule where the 128 x 128 ring was taken and is the slowest: few tiles of K between 512 and 1500, and somewhat more
+    tiles than compute units"""
+    ct = fake_hip
+    buf = torch.empty(48 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+    for m, n, k, want in ((220, 64, 1408, "staged64x64"), (665, 320, 704, "staged64x64"), (221, 256, 1088, "staged64x64"), (562, 384, 640, "staged64x64"),
+                          (1623, 2944, 14016, "192x128x64_q2x2"), (619, 8832, 4096, "256x128x64_q4x2"), (2048, 2048, 2048, "128x128x64_q2x2"),
+                          (1500, 14336, 2048, "192x256x64_q2x4"), (4096, 4096, 4096, "256x256x64_q2x4")):
+        ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k)
+        assert ct.last_resolved()["variant"] == "f16_" + want, (m, n, k)
