@@ -2,6 +2,7 @@
 #include "kernel_table.h"
 #include "toolchain.h"   // written by the build: CUTILE_TOOLCHAIN_FINGERPRINT
 
+#include <algorithm>
 #include <array>
 #include <atomic>
 #include <cstring>
@@ -227,7 +228,7 @@ std::vector<KernelEntry> build_table() {
   for (const char* dt : {"bf16", "f16", "bf16f32"})
     for (auto t : {std::array<int, 2>{16, 64}, std::array<int, 2>{16, 128}, std::array<int, 2>{32, 64}, std::array<int, 2>{64, 64}}) {
       std::string v = std::string(dt) + "_thin" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
-      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, (uint32_t)(8 * t[0] * (t[1] + 4) * 4), 0, t[1], 0, t[0], dt, 0, 2);
+      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, (uint32_t)(8 * t[0] * (t[1] + 4) * 4 + 4), 0, t[1], 0, t[0], dt, 0, 2);
     }
 
   // the ring on tiles between 128 x 128 and 256 x 256
@@ -240,7 +241,8 @@ std::vector<KernelEntry> build_table() {
   for (const char* dt : {"bf16", "f16", "bf16f32"})
     for (auto t : {std::array<int, 3>{64, 64, 4}, std::array<int, 3>{64, 128, 4}, std::array<int, 3>{128, 128, 4}, std::array<int, 3>{256, 128, 8}}) {
       std::string v = std::string(dt) + "_staged" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
-      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * 64), (uint32_t)(2 * 64 * 2 * (t[0] + t[1])), 0, t[1], 64, t[0], dt, 0, 2);
+      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * 64), (uint32_t)(2 * 64 * 2 * (t[0] + t[1]) + (t[0] * t[1] == 64 * 64 ? 4 : 0)), 0, t[1],
+          64, t[0], dt, 0, 2);
     }
 
   // batched GEMM (cutile-examples/examples/batch_matmul.rs): the pipelined bodies with the batch on a grid axis
@@ -391,15 +393,17 @@ std::vector<KernelEntry> build_table() {
   mx("f32", 32, 32, 1, 1);
   mx("f32", 64, 64, 1, 1);
 
-  // ---- block-scaled products without LDS stages (scaled_flat.hip): any partition shape; LDS = one f32 copy of the block per share of K ----
+  // ---- block-scaled products through wave-private stages (scaled_flat.hip): any partition shape; LDS = the eight wavefronts' stages, which
+  // become one f32 copy of the block per share of K, whichever is larger (t[2] shares; a stage holds t[3] rows of x and 64 of y) ----
   for (const char* dt : {"bf16", "f32"})
-    for (auto t : {std::array<int, 3>{16, 64, 8}, std::array<int, 3>{32, 64, 8}, std::array<int, 3>{64, 64, 8}, std::array<int, 3>{64, 128, 4},
-                   std::array<int, 3>{128, 128, 2}})
+    for (auto t : {std::array<int, 4>{16, 64, 8, 16}, std::array<int, 4>{32, 64, 8, 32}, std::array<int, 4>{64, 64, 8, 64}, std::array<int, 4>{64, 128, 4, 64},
+                   std::array<int, 4>{128, 128, 2, 64}})
       for (const char* kind : {"mxfp8", "nvfp4"}) {
         const bool mx8 = kind[0] == 'm';
         std::string v = std::string(mx8 ? "mxfp8_" : "") + dt + "_flat" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
+        const int stages = 8 * ((64 + t[3]) * (128 + (mx8 ? 4 : 16)) + 32), sums = t[2] * t[0] * (t[1] + 4) * 4;
         add(mx8 ? "linear_tile" : "linear_tile_nvfp4", keep(v), keep((mx8 ? "linear_tile_entry__" : "linear_tile_nvfp4_entry__") + v), IMG_SCALED_FLAT, 512,
-            (uint32_t)(t[2] * t[0] * (t[1] + 4) * 4), 0, t[1], 0, t[0], dt, 0, 2);
+            (uint32_t)(std::max(stages, sums) + 4), 0, t[1], 0, t[0], dt, 0, 2);
       }
   return t;
 }

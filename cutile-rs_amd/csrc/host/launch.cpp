@@ -358,12 +358,12 @@ uint32_t split_limit(uint64_t blocks, uint64_t floats) {
 // (strips of columns) and staged ones (tiles).
 bool is_gemm_small(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
 bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0; }
-// The block-scaled kernels without LDS stages (scaled_flat.hip): tile[3] x tile[1] outputs a workgroup, any partition shape.
+// The block-scaled kernels on wave-private stages (scaled_flat.hip): tile[3] x tile[1] outputs a workgroup, any partition shape.
 bool is_scaled_flat(const KernelEntry* e) { return e->image == IMG_SCALED_FLAT; }
 
 // Picks the kernel of a block-scaled product.  A kernel tile that is a whole multiple of the partition tile computes the
 // same output when the launch covers the whole tensor (a 16 x 16 example partition runs on the 32 x 32 kernel), and so do
-// the kernels without LDS stages, which take `flat` launches: whole outputs, scale rows on 4-byte boundaries.
+// the kernels on wave-private stages, which take `flat` launches: whole outputs, scale rows on 4-byte boundaries.
 cutile_status_t resolve_scaled(const char* function, const char* prefix, const std::string& dt, int bm, int bn, bool full_cover, bool flat,
                                const ScaledShape& shape, const cutile_launch_opts_t* opts, const std::string& missing, int* cus, Resolved* res) {
   std::vector<const KernelEntry*> fit, others;

@@ -764,3 +764,21 @@ def test_marshalling_extension_is_rebuilt_for_another_torch(monkeypatch, tmp_pat
     for _ in range(2):
         build.build_marshal()
     assert len(compiled) == 2
+
+
+@pytest.mark.parametrize("image,entries", [("gemmsmall", 32), ("scaledflat", 20)])
+def test_lds_bytes_of_the_table_are_those_of_the_code_objects(fake_hip, image, entries):
+    """cutile_kernel_info_t.lds_bytes against the metadata of the code objects, for the images whose kernels share arrays between
+    stages and sums"""
+    import re, subprocess
+
+    ct = fake_hip
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", os.path.join(root, "cutile-rs_amd", "lib", image + ".hsaco")],
+                           stdout=subprocess.PIPE, text=True, check=True).stdout
+    kernels = notes.split("- .agpr_count")[1:]
+    assert len(kernels) == entries
+    for kernel in kernels:
+        symbol = re.search(r"\n    \.name: +(\S+)", kernel)[1]
+        function, variant = symbol.split("_entry__")
+        assert ct.kernel_lookup(function, variant=variant).lds_bytes == int(re.search(r"\.group_segment_fixed_size: (\d+)", kernel)[1]), symbol
