@@ -208,8 +208,13 @@ class SoftmaxAllF16(Softmax):
 
 def tuned_tile(kernel, problem, default):
     """The tile shape the tuner's (tile, variant) sweep chose for this problem (cutile-rs_amd/tune/tune_baseline.cpp files
-    it in the kernel's tuning record under the bucket "problem|<problem>"), or `default` where no record says."""
+    it in the kernel's tuning record under the bucket "problem|<problem>"), or `default` where no record says or the
+    library refuses the record (another build than it was measured with)."""
     path = os.path.join(ROOT, "cutile-rs_amd", "tuned", kernel + ".json")
+    import __graft_entry__ as entry
+
+    if not any(line.startswith("applied ") and f"/{kernel}.json:" in line for line in entry.load_package().tuning_report().splitlines()):
+        return default, "default"
     try:
         with open(path) as f:
             for e in json.load(f).get("entries", []):

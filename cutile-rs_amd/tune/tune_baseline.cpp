@@ -7,7 +7,9 @@
 // the arguments is recorded as invalid by the tuner; the rest are timed with the do_bench protocol (cache flushed
 // before every repetition, median); the winner is filed under the shape class the launcher reports for the launch
 // (cutile_last_resolved_bucket) with the variant's fingerprint as its key.  The library applies the records it can
-// verify on start-up (csrc/host/tuning.cpp).
+// verify on start-up (csrc/host/tuning.cpp).  The table's own choice stays the winner unless another one beats it by more than
+// kMargin: below that the order of two medians changes from run to run (GEMM bf16 8192^3, _p2x4 / _q2x4: 0.8065 / 0.8088 ms, 0.8121 /
+// 0.8126 ms in one run), and launched one after another on changing operands _q2x4, the table's, is 5 % ahead (802 us against 848).
 #include <cutile/cutile.hpp>
 
 #include <cmath>
@@ -20,6 +22,34 @@ namespace {
 
 std::shared_ptr<Stream> g_stream;
 std::map<std::string, tune::Record> g_records;
+constexpr float kMargin = 0.01f;
+const char* const kGate = "do_bench median, 512 MiB flush, N(0,1) operands; the table's own choice stays unless beaten by 1 %";
+
+// Kernels that no shape class is decided for: the any-layout fallbacks (never the answer for a shape a tiled variant fits), and those for
+// few rows and small outputs, which the launchers choose by a rule on extents.
+bool is_class_candidate(const std::string& variant) {
+  for (const char* kind : {"generic", "_thin", "_staged"})
+    if (variant.find(kind) != std::string::npos) return false;
+  const size_t flat = variant.find("_flat");   // "_flat64x128"; axpy's "_flat" is the contiguous form
+  return flat == std::string::npos || flat + 5 == variant.size();
+}
+
+std::string last_variant() {
+  const char* function = nullptr;
+  cutile_kernel_info_t info{};
+  return cutile_last_resolved_kernel(&function, &info) == CUTILE_SUCCESS ? info.variant : "";
+}
+
+// The winner among the measured trials, given the id of the table's own choice ("" if it is none of them).
+const tune::Trial* winner(const tune::Output& out, const std::string& own) {
+  const tune::Trial *best = nullptr, *mine = nullptr;
+  for (auto& t : out.trials) {
+    if (!t.measured) continue;
+    if (t.config_id == out.best->id && (!best || t.median_ms < best->median_ms)) best = &t;
+    if (t.config_id == own && (!mine || t.median_ms < mine->median_ms)) mine = &t;   // (the two best are timed again, interleaved)
+  }
+  return mine && best && mine->median_ms <= best->median_ms * (1.0f + kMargin) ? mine : best;
+}
 
 template <class T>
 std::shared_ptr<Tensor<T>> converted(Tensor<float> t, std::vector<int32_t> shape) {
@@ -29,10 +59,9 @@ std::shared_ptr<Tensor<T>> converted(Tensor<float> t, std::vector<int32_t> shape
 
 // `launch(variant, stream)` enqueues one launch with the named variant ("" = the library's own choice).
 bool tune_one(const std::string& kernel, const std::string& what, const std::function<Result<Unit>(const std::string&, const std::shared_ptr<Stream>&)>& launch) {
-  // every precompiled variant except the any-layout fallbacks (never the answer for a shape a tiled variant fits)
   std::vector<tune::Config> configs;
   for (auto& c : tune::variant_configs(kernel))
-    if (c.str("variant")->find("generic") == std::string::npos) configs.push_back(c);
+    if (is_class_candidate(*c.str("variant"))) configs.push_back(c);
   printf("tuning %s  %s: %zu candidates\n", kernel.c_str(), what.c_str(), configs.size());
   bench::BenchOptions bo;
   bo.warmup = std::chrono::milliseconds(20);
@@ -52,27 +81,29 @@ bool tune_one(const std::string& kernel, const std::string& what, const std::fun
     return false;
   }
   const tune::Output& out = tuned.value();
-  const std::string best = *out.best->str("variant");
-  // the class this launch belongs to, as the launcher files it
+  // the class this launch belongs to, as the launcher files it, and the table's own choice
   if (launch("", g_stream).is_err() || g_stream->synchronize().is_err()) return false;
-  const std::string bucket = cutile_last_resolved_bucket();
+  const std::string bucket = cutile_last_resolved_bucket(), own = last_variant();
   if (bucket.empty()) { fprintf(stderr, "tune %s: launcher reports no shape class\n", kernel.c_str()); return false; }
-  float best_ms = INFINITY;
-  size_t reps = 0;
   printf("%s  %s  [%s]\n", kernel.c_str(), what.c_str(), bucket.c_str());
-  for (auto& t : out.trials) {
-    std::string name;
-    for (auto& c : configs) if (c.id == t.config_id) name = *c.str("variant");
-    if (t.measured) printf("    %-40s median %8.4f ms  min %8.4f ms  (%zu reps)%s\n", name.c_str(), t.median_ms, t.min_ms, t.reps, name == best ? "   <- winner" : "");
-    if (t.measured && t.config_id == out.best->id && t.median_ms < best_ms) { best_ms = t.median_ms; reps = t.reps; }
-  }
+  auto named = [&](const std::string& id) -> const tune::Config* { for (auto& c : configs) if (c.id == id) return &c; return nullptr; };
+  std::string own_id;
+  for (auto& c : configs) if (*c.str("variant") == own) own_id = c.id;
+  const tune::Trial* won = winner(out, own_id);
+  const tune::Config& config = *named(won->config_id);
+  const std::string best = *config.str("variant");
+  const float best_ms = won->median_ms;
+  const size_t reps = won->reps;
+  for (auto& t : out.trials)
+    if (t.measured) printf("    %-40s median %8.4f ms  min %8.4f ms  (%zu reps)%s%s\n", named(t.config_id)->str("variant")->c_str(), t.median_ms, t.min_ms, t.reps,
+                           t.config_id == own_id ? "   <- table" : "", &t == won ? "   <- winner" : "");
   auto it = g_records.find(kernel);
   if (it == g_records.end()) {
     auto ws = tune::Workspace::of_kernel(kernel, tune::space_hash(configs)).unwrap();
     it = g_records.emplace(kernel, tune::Record(ws)).first;
-    it->second.gate = "do_bench median, 512 MiB flush, N(0,1) operands";
+    it->second.gate = kGate;
   }
-  it->second.insert({bucket, *out.best, best_ms, reps, tune::variant_key(kernel, best).unwrap()});
+  it->second.insert({bucket, config, best_ms, reps, tune::variant_key(kernel, best).unwrap()});
   return true;
 }
 
@@ -110,22 +141,26 @@ bool tune_tiles(const std::string& kernel, const std::string& what, const std::s
     return false;
   }
   const tune::Output& out = tuned.value();
-  const std::string best = *out.best->str("variant");
-  float best_ms = INFINITY;
-  size_t reps = 0;
-  for (auto& t : out.trials) {
-    std::string name;
-    for (auto& c : configs) if (c.id == t.config_id) name = *c.str("variant");
-    if (t.measured) printf("    %-40s median %8.4f ms  min %8.4f ms  (%zu reps)%s\n", name.c_str(), t.median_ms, t.min_ms, t.reps, name == best ? "   <- winner" : "");
-    if (t.measured && t.config_id == out.best->id && t.median_ms < best_ms) { best_ms = t.median_ms; reps = t.reps; }
-  }
+  auto named = [&](const std::string& id) -> const tune::Config* { for (auto& c : configs) if (c.id == id) return &c; return nullptr; };
+  std::string own_id;   // what the table launches on the largest tiles
+  if (launch(256, 256, "", g_stream).is_err() || g_stream->synchronize().is_err()) return false;
+  const std::string own = last_variant();
+  for (auto& c : configs) if (*c.str("variant") == own) own_id = c.id;
+  const tune::Trial* won = winner(out, own_id);
+  const tune::Config& config = *named(won->config_id);
+  const std::string best = *config.str("variant");
+  const float best_ms = won->median_ms;
+  const size_t reps = won->reps;
+  for (auto& t : out.trials)
+    if (t.measured) printf("    %-40s median %8.4f ms  min %8.4f ms  (%zu reps)%s%s\n", named(t.config_id)->str("variant")->c_str(), t.median_ms, t.min_ms, t.reps,
+                           t.config_id == own_id ? "   <- table" : "", &t == won ? "   <- winner" : "");
   auto it = g_records.find(kernel);
   if (it == g_records.end()) {
     auto ws = tune::Workspace::of_kernel(kernel, tune::space_hash(configs)).unwrap();
     it = g_records.emplace(kernel, tune::Record(ws)).first;
-    it->second.gate = "do_bench median, 512 MiB flush, N(0,1) operands";
+    it->second.gate = kGate;
   }
-  it->second.insert({"problem|" + what, *out.best, best_ms, reps, tune::variant_key(kernel, best).unwrap()});
+  it->second.insert({"problem|" + what, config, best_ms, reps, tune::variant_key(kernel, best).unwrap()});
   return true;
 }
 

@@ -86,3 +86,19 @@ def test_default_run_leaves_out_the_example_programs():
     assert set(bench.BASELINE_CONFIGS) <= names
     extra = {w.name for w in bench.make_extra_workloads()}
     assert extra and not (extra & names)
+
+
+def test_the_tile_is_the_tuning_records_only_where_the_library_applies_it(monkeypatch):
+    import __graft_entry__ as entry
+
+    class Package:
+        tuning_report = staticmethod(lambda: "")
+    monkeypatch.setattr(entry, "load_package", lambda: Package)
+    path = os.path.join(bench.ROOT, "cutile-rs_amd", "lib", "..", "tuned", "gemm.json")
+    problem = "bf16|8192x8192x8192"
+    Package.tuning_report = staticmethod(lambda: f"applied {path}: 5 bucket(s) of kernel gemm\n")
+    assert bench.tuned_tile("gemm", problem, (128, 128)) == ((256, 256), "tuning record")
+    for report in (f"refused {path}: stale tuning record at {path}: source_hash mismatch\n", "tuning records: switched off\n",
+                   f"applied {path.replace('gemm', 'batch_gemm')}: 1 bucket(s) of kernel batch_gemm\n"):
+        Package.tuning_report = staticmethod(lambda: report)
+        assert bench.tuned_tile("gemm", problem, (128, 128)) == ((128, 128), "default")

@@ -782,3 +782,16 @@ def test_lds_bytes_of_the_table_are_those_of_the_code_objects(fake_hip, image, e
         symbol = re.search(r"\n    \.name: +(\S+)", kernel)[1]
         function, variant = symbol.split("_entry__")
         assert ct.kernel_lookup(function, variant=variant).lds_bytes == int(re.search(r"\.group_segment_fixed_size: (\d+)", kernel)[1]), symbol
+
+
+def test_shipped_tuning_records_are_those_of_this_build():
+    """a change to a kernel's code object makes the library refuse its record, and with it the measured winners: re-tune
+    (cutile-rs_amd/bin/tune_baseline) or delete it"""
+    import subprocess, sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = {k: v for k, v in os.environ.items() if k != "CUTILE_TUNING_RECORDS"}
+    report = subprocess.check_output([sys.executable, "-c", "import __graft_entry__ as e; print(e.load_package().tuning_report())"], cwd=root, env=env, text=True)
+    files = sorted(f for f in os.listdir(os.path.join(root, "cutile-rs_amd", "tuned")) if f.endswith(".json"))
+    lines = report.strip().splitlines()
+    assert len(lines) == len(files) and all(l.startswith("applied ") and f"/{f}:" in l for l, f in zip(lines, files)), report
