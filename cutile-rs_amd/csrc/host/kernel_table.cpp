@@ -164,12 +164,14 @@ std::vector<KernelEntry> build_table() {
       add(fn, keep(v), keep(std::string(fn) + "_entry__" + v), IMG_ROWWISE, 256, 0, 0, 0, rv.vpl, rv.wpr, "f16",
           (int64_t)rv.wpr * 64 * rv.vpl * 8, 2);
     }
-    add(fn, "generic", keep(std::string(fn) + "_entry__generic"), IMG_ROWWISE, 256, 0, 0, 0, 0, 0, "f16", 0, 2);
   }
-  add("rms_norm_f16", "generic", "rms_norm_f16_entry__generic", IMG_ROWWISE, 256, 0, 0, 0, 0, 0, "f16", 0, 2);
+  // any layout: rows in registers where they can be, and the element walk alone
+  for (const char* fn : {"add_rms_norm_f16", "qk_norm_f16", "rms_norm_f16"})
+    for (const char* kind : {"generic", "walk"})
+      add(fn, kind, keep(std::string(fn) + "_entry__" + kind), IMG_ROWWISE, 256, 0, 0, 0, 0, 0, "f16", 0, 2);
   add("rms_norm", "f32", "rms_norm_entry__f32", IMG_ROWWISE, 256, 0, 0, 0, 0, 0, "f32", 0, 2);   // the f32 example form
-  add("softmax", "f16_generic", "softmax_entry__f16_generic", IMG_ROWWISE, 256, 0, 0, 0, 0, 0, "f16", 0, 2);
-  add("softmax", "f32_generic", "softmax_entry__f32_generic", IMG_ROWWISE, 256, 0, 0, 0, 0, 0, "f32", 0, 2);
+  for (const char* kind : {"f16_generic", "f32_generic", "f16_walk", "f32_walk"})
+    add("softmax", kind, keep(std::string("softmax_entry__") + kind), IMG_ROWWISE, 256, 0, 0, 0, 0, 0, kind[1] == '1' ? "f16" : "f32", 0, 2);
 
   // ---- bf16 GEMM: LDS = 2 stages x (BM*BK + BK*BN) x 2 bytes ----
   auto gemm = [&](const char* dtype, int bm, int bn, int bk, int wvm, int wvn, const char* kind = "w") {

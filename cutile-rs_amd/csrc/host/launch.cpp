@@ -947,15 +947,23 @@ static std::vector<std::string> fitting_row_variants(const char* fn_name, const 
   return names;
 }
 
+// The any-layout kernels of a row-wise function, behind the ones that fit: `held` rows of `bytes` (adjacent elements) are at most what
+// the "generic" kernels hold in registers (kAnyRowMost, rowwise.hip), everything else is walked.  Both take every call.
+static bool row_held(bool adjacent, int64_t bytes) { return adjacent && bytes <= 32768; }
+static void add_any_layout(bool held, const std::string& prefix, std::vector<std::string>* acceptable) {
+  acceptable->push_back(prefix + (held ? "generic" : "walk"));
+  acceptable->push_back(prefix + (held ? "walk" : "generic"));
+}
+
 // Launch grid of a row-wise kernel over `segments` tile rows: register-resident
 // variants take 4 / WPR segments per workgroup, the any-layout ones walk the
 // segments with a grid stride.
-// `row_bytes`: length of a segment whose elements are adjacent (0: they are not); the any-layout kernels put four rows
+// `row_bytes`: length of a segment that is held in registers (0: it is walked); the any-layout kernels put four rows
 // of up to 4 KiB or two of up to 8 KiB into a workgroup (kAnyRowPerWave, rowwise.hip).
 static void row_launch_grid(const KernelEntry* e, uint64_t segments, uint32_t grid[3], int64_t row_bytes = 0) {
   grid[0] = grid[1] = grid[2] = 1;
   if (e->capacity <= 0)
-    grid[0] = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(row_bytes <= 0 || row_bytes > 8192 ? segments : div_up(segments, row_bytes > 4096 ? 2 : 4), 1), 1u << 20);
+    grid[0] = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(row_bytes <= 0 || row_bytes > 8192 || strstr(e->variant, "walk") ? segments : div_up(segments, row_bytes > 4096 ? 2 : 4), 1), 1u << 20);
   else if (e->tile[1] > 0)   // short-row variants: tile[1] rows per workgroup
     grid[0] = std::max<uint32_t>(1, div_up(segments, e->tile[1]));
   else
@@ -1003,7 +1011,8 @@ cutile_status_t cutile_launch_rms_norm_f16(cutile_stream_t stream, const cutile_
                       aligned16(w->ptr);
   std::vector<std::string> acceptable;
   if (vec_ok) acceptable = fitting_row_variants("rms_norm_f16", "", n);
-  acceptable.push_back("generic");
+  const bool held = row_held(x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1, 2 * (int64_t)n);
+  add_any_layout(held, "", &acceptable);
   Resolved res;
   BucketScope bucket("n" + pow2_class(n));
   if (cutile_status_t s = resolve_entry("rms_norm_f16", opts, acceptable[0], acceptable, &res)) return s;
@@ -1016,7 +1025,7 @@ cutile_status_t cutile_launch_rms_norm_f16(cutile_stream_t stream, const cutile_
   args.push_tile_grid(tg);
   const uint64_t rows = std::min<uint64_t>(tg[0], ot.shape[0]);
   uint32_t grid[3];
-  row_launch_grid(res.entry, rows, grid, x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1 ? 2 * (int64_t)n : 0);
+  row_launch_grid(res.entry, rows, grid, held ? 2 * (int64_t)n : 0);
   return launch_packed(res.fn, grid, res.entry->block, rms_norm_residency_lds(res.entry, n), stream, args);
 }
 
@@ -1193,7 +1202,9 @@ static cutile_status_t launch_fused_norm(const char* fn, cutile_stream_t stream,
                       w->strides[0] == 1 && aligned16(w->ptr) && (!w2 || (w2->strides[0] == 1 && aligned16(w2->ptr)));
   std::vector<std::string> acceptable;
   if (vec_ok) acceptable = fitting_row_variants(fn, "", n);
-  acceptable.push_back("generic");
+  auto unit = [](const cutile_tensor_arg_t& t) { return t.strides[t.rank - 1] == 1; };
+  const bool held = row_held(unit(*a) && unit(*b) && unit(*w) && (!w2 || unit(*w2)) && unit(ot) && (!out2 || unit(out2->tensor)), 2 * (int64_t)n);
+  add_any_layout(held, "", &acceptable);
   Resolved res;
   if (cutile_status_t s = resolve_entry(fn, opts, acceptable[0], acceptable, &res)) return s;
   ArgPacker args;
@@ -1207,9 +1218,8 @@ static cutile_status_t launch_fused_norm(const char* fn, cutile_stream_t stream,
   if (qk) args.push_val<int32_t>(*num_q_rows);
   args.push_tile_grid(tg);
   const uint64_t rows = std::min<uint64_t>(tg[0], ot.shape[0]);
-  auto unit = [](const cutile_tensor_arg_t& t) { return t.strides[t.rank - 1] == 1; };
   uint32_t grid[3];
-  row_launch_grid(res.entry, rows, grid, unit(*a) && unit(*b) && unit(*w) && (!w2 || unit(*w2)) && unit(ot) && (!out2 || unit(out2->tensor)) ? 2 * (int64_t)n : 0);
+  row_launch_grid(res.entry, rows, grid, held ? 2 * (int64_t)n : 0);
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 
@@ -2003,7 +2013,9 @@ cutile_status_t cutile_launch_softmax(cutile_stream_t stream, const cutile_tenso
                       aligned16(yt.ptr) && (uint64_t)x->shape[0] >= rows;
   std::vector<std::string> acceptable;
   if (vec_ok) acceptable = fitting_row_variants("softmax", dt + "_w", bn);
-  acceptable.push_back(dt + "_generic");
+  const int64_t row_bytes = (int64_t)bn * (int64_t)cutile_dtype_size(x->dtype);
+  const bool held = row_held(x->strides[1] == 1 && yt.strides[1] == 1, row_bytes);
+  add_any_layout(held, dt + "_", &acceptable);
   Resolved res;
   BucketScope bucket(dt + "|bn" + pow2_class(bn));
   if (cutile_status_t s = resolve_entry("softmax", opts, acceptable[0], acceptable, &res)) return s;
@@ -2013,7 +2025,7 @@ cutile_status_t cutile_launch_softmax(cutile_stream_t stream, const cutile_tenso
   args.push_tile_grid(tg);
   const uint64_t segments = rows * tg[1];
   uint32_t grid[3];
-  row_launch_grid(res.entry, segments, grid, x->strides[1] == 1 && yt.strides[1] == 1 ? (int64_t)bn * (int64_t)cutile_dtype_size(x->dtype) : 0);
+  row_launch_grid(res.entry, segments, grid, held ? row_bytes : 0);
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 

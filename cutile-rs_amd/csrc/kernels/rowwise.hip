@@ -272,7 +272,7 @@ __device__ __forceinline__ void add_rms_norm_rows(const _Float16* __restrict__ r
 // 7 elements before and after them as one value in a lane of the row's first wavefront.  WPR wavefronts share a row of
 // up to WPR * 64 * VPL vectors; a workgroup walks rows with a grid stride.  4000 x 5001: softmax 52 -> 16 us, RMSNorm 17 us, the
 // fused residual form 27 us (5 - 6 TB/s, the rate of the aligned kernels).
-constexpr int64_t kAnyRowMost = 4 * 64 * 8 * 16;      // bytes of the longest row held in registers (WPR 4, VPL 8)
+constexpr int64_t kAnyRowMost = 4 * 64 * 8 * 16;      // bytes of the longest row held in registers (WPR 4, VPL 8); the launchers know it too
 constexpr int64_t kAnyRowPerWave = 64 * 4 * 16;       // rows of up to this many bytes take one wavefront each (the launcher sizes the grid by it)
 typedef u32x4 Unaligned __attribute__((aligned(2)));
 template <typename T, int WPR>
@@ -369,29 +369,16 @@ __device__ __forceinline__ void norm_rows_any_length(RowOf row_of, int32_t n, in
     norm_rows_any<4, 8, ADD>(row_of, n, rows, eps);
 }
 
-// Any N / any strides for the two fused forms: one workgroup per row, inputs re-read (L2).
-__device__ __forceinline__ void fused_norm_row_generic(const TensorArg<2>& a, const TensorArg<2>* b_add,
-                                                       const TensorArg<2>* b_alt, const TensorArg<1>& w,
-                                                       const TensorArg<1>* w_alt, const PartitionArg<2>& out,
-                                                       const PartitionArg<2>* out2, float eps, int64_t rows,
-                                                       int64_t split) {
+// Any N / any strides for the two fused forms: one workgroup per row, inputs re-read (L2).  The element walks have kernels of their
+// own ("walk") beside the any-layout ones ("generic"), which hold a row in registers where they can: with those registers a compute
+// unit keeps five or six wavefronts a SIMD instead of eight, and a walk lives on what is in flight (us in the one and in the other kernel: q / k
+// rows 808 x 25727 149, 95; RMSNorm of strided rows 334134 x 101 310, 252; f32 softmax 2275 x 9349 105, 94).
+__device__ __forceinline__ void fused_norm_row_walk(const TensorArg<2>& a, const TensorArg<2>* b_add,
+                                                    const TensorArg<2>* b_alt, const TensorArg<1>& w,
+                                                    const TensorArg<1>* w_alt, const PartitionArg<2>& out,
+                                                    const PartitionArg<2>* out2, float eps, int64_t rows,
+                                                    int64_t split) {
   // b_add: second addend (add_rms_norm); b_alt / w_alt: source and weight for rows >= split (qk_norm)
-  const int32_t cols = a.shape[1];
-  if (a.strides[1] == 1 && (!b_add || (b_add->strides[1] == 1 && b_add->shape[1] >= cols)) && (!b_alt || (b_alt->strides[1] == 1 && b_alt->shape[1] == cols)) &&
-      w.strides[0] == 1 && w.shape[0] >= cols && (!w_alt || (w_alt->strides[0] == 1 && w_alt->shape[0] >= cols)) && out.strides[1] == 1 &&
-      out.shape[1] >= cols && (!out2 || (out2->strides[1] == 1 && out2->shape[1] >= cols)) && (int64_t)cols * 2 <= kAnyRowMost) {
-    const auto row_of = [&](int64_t row) {
-      const bool second = b_alt && row >= split;
-      return AnyRow{second ? (const _Float16*)b_alt->ptr + (row - split) * b_alt->strides[0] : (const _Float16*)a.ptr + row * a.strides[0],
-                    b_add ? (const _Float16*)b_add->ptr + row * b_add->strides[0] : nullptr, (const _Float16*)(second ? w_alt : &w)->ptr,
-                    (_Float16*)out.ptr + row * out.strides[0], out2 ? (_Float16*)out2->ptr + row * out2->strides[0] : nullptr};
-    };
-    if (b_add)
-      norm_rows_any_length<true>(row_of, cols, rows, eps);
-    else
-      norm_rows_any_length<false>(row_of, cols, rows, eps);
-    return;
-  }
   __shared__ float lds[kWaves];
   const int wave = threadIdx.x >> 6;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
@@ -425,21 +412,35 @@ __device__ __forceinline__ void fused_norm_row_generic(const TensorArg<2>& a, co
     __syncthreads();
   }
 }
+__device__ __forceinline__ void fused_norm_row_generic(const TensorArg<2>& a, const TensorArg<2>* b_add,
+                                                       const TensorArg<2>* b_alt, const TensorArg<1>& w,
+                                                       const TensorArg<1>* w_alt, const PartitionArg<2>& out,
+                                                       const PartitionArg<2>* out2, float eps, int64_t rows,
+                                                       int64_t split) {
+  const int32_t cols = a.shape[1];
+  if (a.strides[1] == 1 && (!b_add || (b_add->strides[1] == 1 && b_add->shape[1] >= cols)) && (!b_alt || (b_alt->strides[1] == 1 && b_alt->shape[1] == cols)) &&
+      w.strides[0] == 1 && w.shape[0] >= cols && (!w_alt || (w_alt->strides[0] == 1 && w_alt->shape[0] >= cols)) && out.strides[1] == 1 &&
+      out.shape[1] >= cols && (!out2 || (out2->strides[1] == 1 && out2->shape[1] >= cols)) && (int64_t)cols * 2 <= kAnyRowMost) {
+    const auto row_of = [&](int64_t row) {
+      const bool second = b_alt && row >= split;
+      return AnyRow{second ? (const _Float16*)b_alt->ptr + (row - split) * b_alt->strides[0] : (const _Float16*)a.ptr + row * a.strides[0],
+                    b_add ? (const _Float16*)b_add->ptr + row * b_add->strides[0] : nullptr, (const _Float16*)(second ? w_alt : &w)->ptr,
+                    (_Float16*)out.ptr + row * out.strides[0], out2 ? (_Float16*)out2->ptr + row * out2->strides[0] : nullptr};
+    };
+    if (b_add)
+      norm_rows_any_length<true>(row_of, cols, rows, eps);
+    else
+      norm_rows_any_length<false>(row_of, cols, rows, eps);
+    return;
+  }
+  fused_norm_row_walk(a, b_add, b_alt, w, w_alt, out, out2, eps, rows, split);
+}
 
 // Any N / any strides: one workgroup per row, the row is re-read for the second
 // pass (it is still in L2).
-__device__ __forceinline__ void rms_norm_row_generic(const TensorArg<2>& x, const TensorArg<1>& w,
-                                                     const PartitionArg<2>& out, float eps,
-                                                     int64_t rows) {
-  if (x.strides[1] == 1 && w.strides[0] == 1 && w.shape[0] >= x.shape[1] && out.strides[1] == 1 && out.shape[1] >= x.shape[1] &&
-      (int64_t)x.shape[1] * 2 <= kAnyRowMost) {
-    norm_rows_any_length<false>(
-        [&](int64_t row) {
-          return AnyRow{(const _Float16*)x.ptr + row * x.strides[0], nullptr, (const _Float16*)w.ptr, (_Float16*)out.ptr + row * out.strides[0], nullptr};
-        },
-        x.shape[1], rows, eps);
-    return;
-  }
+__device__ __forceinline__ void rms_norm_row_walk(const TensorArg<2>& x, const TensorArg<1>& w,
+                                                  const PartitionArg<2>& out, float eps,
+                                                  int64_t rows) {
   __shared__ float lds[kWaves];
   const int wave = threadIdx.x >> 6;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
@@ -461,6 +462,20 @@ __device__ __forceinline__ void rms_norm_row_generic(const TensorArg<2>& x, cons
     }
     __syncthreads();  // lds is reused by the next row
   }
+}
+__device__ __forceinline__ void rms_norm_row_generic(const TensorArg<2>& x, const TensorArg<1>& w,
+                                                     const PartitionArg<2>& out, float eps,
+                                                     int64_t rows) {
+  if (x.strides[1] == 1 && w.strides[0] == 1 && w.shape[0] >= x.shape[1] && out.strides[1] == 1 && out.shape[1] >= x.shape[1] &&
+      (int64_t)x.shape[1] * 2 <= kAnyRowMost) {
+    norm_rows_any_length<false>(
+        [&](int64_t row) {
+          return AnyRow{(const _Float16*)x.ptr + row * x.strides[0], nullptr, (const _Float16*)w.ptr, (_Float16*)out.ptr + row * out.strides[0], nullptr};
+        },
+        x.shape[1], rows, eps);
+    return;
+  }
+  rms_norm_row_walk(x, w, out, eps, rows);
 }
 
 // ---- softmax -----------------------------------------------------------------------------
@@ -619,24 +634,10 @@ __device__ __forceinline__ void softmax_segments_any(const TensorArg<2>& x, cons
 // Any tile width / any strides: one workgroup per segment, three passes (the
 // segment stays in L2 between them).
 template <typename T>
-__device__ __forceinline__ void softmax_segment_generic(const TensorArg<2>& x,
-                                                        const PartitionArg<2>& y,
-                                                        int32_t segs_per_row, int64_t n_segments) {
+__device__ __forceinline__ void softmax_segment_walk(const TensorArg<2>& x,
+                                                     const PartitionArg<2>& y,
+                                                     int32_t segs_per_row, int64_t n_segments) {
   const int32_t bn = y.pshape[1];
-  const int64_t bytes = (int64_t)bn * (int64_t)sizeof(T);
-  if (x.strides[1] == 1 && y.strides[1] == 1 && bytes <= kAnyRowMost) {
-    if (bytes <= 64 * 16)
-      softmax_segments_any<T, 1, 1>(x, y, segs_per_row, n_segments);
-    else if (bytes <= kAnyRowPerWave)
-      softmax_segments_any<T, 1, 4>(x, y, segs_per_row, n_segments);
-    else if (bytes <= 2 * kAnyRowPerWave)
-      softmax_segments_any<T, 2, 4>(x, y, segs_per_row, n_segments);
-    else if (bytes <= 4 * kAnyRowPerWave)
-      softmax_segments_any<T, 4, 4>(x, y, segs_per_row, n_segments);
-    else
-      softmax_segments_any<T, 4, 8>(x, y, segs_per_row, n_segments);
-    return;
-  }
   __shared__ float lds[2][kWaves];
   const int wave = threadIdx.x >> 6;
   for (int64_t seg = blockIdx.x; seg < n_segments; seg += gridDim.x) {
@@ -667,6 +668,27 @@ __device__ __forceinline__ void softmax_segment_generic(const TensorArg<2>& x,
     }
     __syncthreads();
   }
+}
+template <typename T>
+__device__ __forceinline__ void softmax_segment_generic(const TensorArg<2>& x,
+                                                        const PartitionArg<2>& y,
+                                                        int32_t segs_per_row, int64_t n_segments) {
+  const int32_t bn = y.pshape[1];
+  const int64_t bytes = (int64_t)bn * (int64_t)sizeof(T);
+  if (x.strides[1] == 1 && y.strides[1] == 1 && bytes <= kAnyRowMost) {
+    if (bytes <= 64 * 16)
+      softmax_segments_any<T, 1, 1>(x, y, segs_per_row, n_segments);
+    else if (bytes <= kAnyRowPerWave)
+      softmax_segments_any<T, 1, 4>(x, y, segs_per_row, n_segments);
+    else if (bytes <= 2 * kAnyRowPerWave)
+      softmax_segments_any<T, 2, 4>(x, y, segs_per_row, n_segments);
+    else if (bytes <= 4 * kAnyRowPerWave)
+      softmax_segments_any<T, 4, 4>(x, y, segs_per_row, n_segments);
+    else
+      softmax_segments_any<T, 4, 8>(x, y, segs_per_row, n_segments);
+    return;
+  }
+  softmax_segment_walk<T>(x, y, segs_per_row, n_segments);
 }
 
 }  // namespace
@@ -751,11 +773,23 @@ extern "C" __global__ void __launch_bounds__(kThreads, 4)
   int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
   fused_norm_row_generic(x, &residual, nullptr, w, nullptr, out, &residual_out, eps, rows, INT64_MAX);
 }
+extern "C" __global__ void __launch_bounds__(kThreads)
+    add_rms_norm_f16_entry__walk(TensorArg<2> residual, TensorArg<2> x, TensorArg<1> w, PartitionArg<2> out,
+                                    PartitionArg<2> residual_out, float eps, TileGrid g) {
+  int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
+  fused_norm_row_walk(x, &residual, nullptr, w, nullptr, out, &residual_out, eps, rows, INT64_MAX);
+}
 extern "C" __global__ void __launch_bounds__(kThreads, 4)
     qk_norm_f16_entry__generic(TensorArg<2> q, TensorArg<2> k, TensorArg<1> qw, TensorArg<1> kw, PartitionArg<2> out,
                                float eps, int32_t num_q_rows, TileGrid g) {
   int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
   fused_norm_row_generic(q, nullptr, &k, qw, &kw, out, nullptr, eps, rows, (int64_t)num_q_rows);
+}
+extern "C" __global__ void __launch_bounds__(kThreads)
+    qk_norm_f16_entry__walk(TensorArg<2> q, TensorArg<2> k, TensorArg<1> qw, TensorArg<1> kw, PartitionArg<2> out,
+                               float eps, int32_t num_q_rows, TileGrid g) {
+  int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
+  fused_norm_row_walk(q, nullptr, &k, qw, &kw, out, nullptr, eps, rows, (int64_t)num_q_rows);
 }
 
 extern "C" __global__ void __launch_bounds__(kThreads, 4)
@@ -763,6 +797,12 @@ extern "C" __global__ void __launch_bounds__(kThreads, 4)
                                 TileGrid g) {
   int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
   rms_norm_row_generic(x, w, out, eps, rows);
+}
+extern "C" __global__ void __launch_bounds__(kThreads)
+    rms_norm_f16_entry__walk(TensorArg<2> x, TensorArg<1> w, PartitionArg<2> out, float eps,
+                                TileGrid g) {
+  int64_t rows = min((int64_t)g.x, (int64_t)out.shape[0]);
+  rms_norm_row_walk(x, w, out, eps, rows);
 }
 
 // rms_norm<N, BLOCK_SIZE>(x: [-1, N] f32, w: [N] f32, out: [1, N] tiles f32, eps) — the f32 example form
@@ -1128,11 +1168,13 @@ SOFTMAX_ALL_F16_KERNEL(32, 8)
 SOFTMAX_VARIANTS(_Float16, f16)
 SOFTMAX_VARIANTS(float, f32)
 
-#define SOFTMAX_GENERIC(T, NAME)                                                                    \
-  extern "C" __global__ void __launch_bounds__(kThreads, 6)                                           \
-      softmax_entry__##NAME##_generic(TensorArg<2> x, PartitionArg<2> y, TileGrid g) {              \
+#define SOFTMAX_GENERIC(T, NAME, KIND, BODY, ...)                                                   \
+  extern "C" __global__ void __launch_bounds__(__VA_ARGS__)                                        \
+      softmax_entry__##NAME##_##KIND(TensorArg<2> x, PartitionArg<2> y, TileGrid g) {               \
     int64_t rows = min((int64_t)g.x * y.pshape[0], (int64_t)y.shape[0]);                           \
-    softmax_segment_generic<T>(x, y, (int32_t)g.y, rows * (int64_t)g.y);                           \
+    BODY<T>(x, y, (int32_t)g.y, rows * (int64_t)g.y);                                              \
   }
-SOFTMAX_GENERIC(_Float16, f16)
-SOFTMAX_GENERIC(float, f32)
+SOFTMAX_GENERIC(_Float16, f16, generic, softmax_segment_generic, kThreads, 6)
+SOFTMAX_GENERIC(float, f32, generic, softmax_segment_generic, kThreads, 6)
+SOFTMAX_GENERIC(_Float16, f16, walk, softmax_segment_walk, kThreads)
+SOFTMAX_GENERIC(float, f32, walk, softmax_segment_walk, kThreads)

@@ -1,7 +1,7 @@
 // Tunes the variant choice of the benchmark configurations on the GPU this runs on and writes one provenance-checked
 // record per kernel (cutile/src/tune.rs:293-420 Autotuner, :762-906 Record):
 //
-//     cutile-rs_amd/bin/tune_baseline <output directory>      (normally cutile-rs_amd/tuned)
+//     cutile-rs_amd/bin/tune_baseline <output directory> [kernel ...]      (normally cutile-rs_amd/tuned; all kernels)
 //
 // For every configuration: the candidates are all precompiled variants of the kernel; a candidate that does not fit
 // the arguments is recorded as invalid by the tuner; the rest are timed with the do_bench protocol (cache flushed
@@ -12,6 +12,7 @@
 // 0.8126 ms in one run), and launched one after another on changing operands _q2x4, the table's, is 5 % ahead (802 us against 848).
 #include <cutile/cutile.hpp>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <map>
@@ -22,13 +23,15 @@ namespace {
 
 std::shared_ptr<Stream> g_stream;
 std::map<std::string, tune::Record> g_records;
+std::vector<std::string> g_kernels;   // the kernels asked for; none: all
+bool wanted(const std::string& kernel) { return g_kernels.empty() || std::find(g_kernels.begin(), g_kernels.end(), kernel) != g_kernels.end(); }
 constexpr float kMargin = 0.01f;
 const char* const kGate = "do_bench median, 512 MiB flush, N(0,1) operands; the table's own choice stays unless beaten by 1 %";
 
 // Kernels that no shape class is decided for: the any-layout fallbacks (never the answer for a shape a tiled variant fits), and those for
 // few rows and small outputs, which the launchers choose by a rule on extents.
 bool is_class_candidate(const std::string& variant) {
-  for (const char* kind : {"generic", "_thin", "_staged"})
+  for (const char* kind : {"generic", "walk", "_thin", "_staged"})
     if (variant.find(kind) != std::string::npos) return false;
   const size_t flat = variant.find("_flat");   // "_flat64x128"; axpy's "_flat" is the contiguous form
   return flat == std::string::npos || flat + 5 == variant.size();
@@ -59,6 +62,7 @@ std::shared_ptr<Tensor<T>> converted(Tensor<float> t, std::vector<int32_t> shape
 
 // `launch(variant, stream)` enqueues one launch with the named variant ("" = the library's own choice).
 bool tune_one(const std::string& kernel, const std::string& what, const std::function<Result<Unit>(const std::string&, const std::shared_ptr<Stream>&)>& launch) {
+  if (!wanted(kernel)) return true;
   std::vector<tune::Config> configs;
   for (auto& c : tune::variant_configs(kernel))
     if (is_class_candidate(*c.str("variant"))) configs.push_back(c);
@@ -113,6 +117,7 @@ bool tune_one(const std::string& kernel, const std::string& what, const std::fun
 // record under the bucket "problem|<what>" with the parameters (variant, bm, bn); bench.py partitions z accordingly.
 bool tune_tiles(const std::string& kernel, const std::string& what, const std::string& dtype,
                 const std::function<Result<Unit>(int, int, const std::string&, const std::shared_ptr<Stream>&)>& launch) {
+  if (!wanted(kernel)) return true;
   std::vector<tune::Config> configs;
   for (auto& c : tune::variant_configs(kernel)) {
     const std::string v = *c.str("variant");
@@ -173,9 +178,10 @@ Result<Unit> enqueue(L launcher, const std::string& variant, const std::shared_p
 }  // namespace
 
 int main(int argc, char** argv) {
-  if (argc < 2) { fprintf(stderr, "usage: %s <output directory>\n", argv[0]); return 2; }
+  if (argc < 2) { fprintf(stderr, "usage: %s <output directory> [kernel ...]\n", argv[0]); return 2; }
   setvbuf(stdout, nullptr, _IOLBF, 0);
   const std::string out_dir = argv[1];
+  g_kernels.assign(argv + 2, argv + argc);
   cutile_tuning_reload("");                              // tune against the table's own order, not against older records
   g_stream = Device::create(0).unwrap()->new_stream().unwrap();
   bool all = true;
