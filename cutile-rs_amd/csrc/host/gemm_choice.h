@@ -40,12 +40,15 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
   auto pick = [&](const char* kernel) { snprintf(c.variant, sizeof(c.variant), "%s_%s", s.dtype, kernel); };
   // Few rows.  Measured at 1 to 64 rows, f16 and bf16 (us, thin against 128 x 128 tiles): 4096 x 4096 10 - 21 against 53,
   // K = 14336 25 - 41 against 175, 14336 x 4096 24 - 35 against 54, 1024 x 1024 5 - 9 against 11.  128-column strips where
-  // there are enough of them to keep three quarters of the compute units busy (28672 x 8192, one row: 83 us against 92);
-  // with more than 32 rows x costs as many bytes as y and that many columns are better off with tiles (129 against 113 us).
+  // there are enough of them to keep three quarters of the compute units busy (28672 x 8192, one row: 83 us against 92).
+  // With more than 32 rows a workgroup fills a compute unit by itself (139 KB of partial sums), so strips are the better ones only while
+  // they fit the chip once: over 459 products of 33 to 64 rows the tiles chosen below take 0.55 to 0.98 times the strips' time beyond 16384
+  // columns, 0.76 in the mean (us: 60 x 19072 x 448 12.5 against 9.0 and 7.5 from memory and from the caches), and the best of them 1.10 up to there.
   // Up to 128 rows (two passes over y, the second from L2) while the strips of both passes fit the chip once
   // (4096 x 4096 23 us against 27 with staged tiles; 14336 x 4096 60 against 46).
   const bool many = s.n >= 192 * 128;
-  if (s.y_cols >= 64 && ((s.m <= 64 && !(many && s.m > 32)) || (s.m <= 128 && 2 * ((s.n + 63) / 64) <= cus))) {
+  const int64_t strips = (s.n + 63) / 64;
+  if (s.y_cols >= 64 && (s.m <= 32 || (s.m <= 64 && strips <= cus) || (s.m <= 128 && 2 * strips <= cus))) {
     pick(s.m > 32 ? "thin64x64" : s.m > 16 ? "thin32x64" : many && s.y_cols >= 128 ? "thin16x128" : "thin16x64");
     return c;
   }

@@ -82,3 +82,15 @@ def test_gpu_thin_gemm_captured_and_replayed(ct, dev):
             torch.cuda.synchronize()
     finally:
         graph.close()
+
+
+def test_more_than_32_rows_take_strips_while_they_fit_the_chip_once(fake_hip):
+    """a workgroup of the 64-row strips fills a compute unit: beyond 256 strips the launch would run twice as long"""
+    ct = fake_hip
+    buf = torch.empty(32 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+    for m, n, k, want in ((33, 16384, 448, "thin64x64"), (64, 16321, 448, "thin64x64"), (33, 16385, 448, "staged"), (60, 19072, 448, "128x128x64_d2x2"),
+                          (46, 16960, 1024, "128x128x64_q2x2"), (49, 22001, 1001, "staged"), (32, 19072, 448, "thin32x64"), (1, 32000, 448, "thin16x128"),
+                          (128, 8192, 448, "thin64x64"), (128, 8256, 448, "128x128x64_d2x2")):
+        ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k, generics=["f16", 128, 128, 1, k])
+        assert ct.last_resolved()["variant"].startswith("f16_" + want), (m, n, k, ct.last_resolved()["variant"])
