@@ -38,7 +38,7 @@ struct ClassWinner {
   std::string variant;
   bool from_record;
 };
-std::map<std::string, ClassWinner> g_bucket_preferred;
+std::unordered_map<std::string, ClassWinner> g_bucket_preferred;   // every launch of a function with shape classes looks here
 std::atomic<size_t> g_run_time_winners{0};   // how many of them the program named
 void count_run_time_winners() {   // under g_pref_mutex
   size_t n = 0;
@@ -461,11 +461,24 @@ std::string preferred_variant(const char* function) {
   return it == g_preferred.end() ? std::string() : it->second;
 }
 
-std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time) {
-  if (bucket.empty() || (at_run_time && g_run_time_winners.load(std::memory_order_acquire) == 0)) return std::string();
+std::string class_winner(const char* function, const std::string& bucket, bool* from_record) {
+  *from_record = false;
+  if (bucket.empty()) return std::string();
+  std::string key;
+  key.reserve(96);
+  key.append(function).append("|").append(bucket);
   std::lock_guard<std::mutex> lock(g_pref_mutex);
-  auto it = g_bucket_preferred.find(std::string(function) + "|" + bucket);
-  return it == g_bucket_preferred.end() || it->second.from_record == at_run_time ? std::string() : it->second.variant;
+  auto it = g_bucket_preferred.find(key);
+  if (it == g_bucket_preferred.end()) return std::string();
+  *from_record = it->second.from_record;
+  return it->second.variant;
+}
+
+std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time) {
+  if (at_run_time && g_run_time_winners.load(std::memory_order_acquire) == 0) return std::string();
+  bool from_record = false;
+  std::string variant = class_winner(function, bucket, &from_record);
+  return from_record == at_run_time ? std::string() : variant;
 }
 
 cutile_status_t set_class_winner(const char* function, const char* bucket, const char* variant, bool from_record) {

@@ -37,7 +37,9 @@ const KernelEntry* find_entry(const char* function, const std::string& variant);
 cutile_status_t load_entry(cutile_device_t device, const KernelEntry* entry, hipFunction_t* fn);
 // Preferred variant set through cutile_kernel_set_preferred_variant, or "".
 std::string preferred_variant(const char* function);
-// Winner of (function, shape-class bucket) that the program set at run time, or (at_run_time false) that a tuning record names; or "".
+// Winner of (function, shape-class bucket), or "", and whether a tuning record names it (otherwise the program did, at run time).
+std::string class_winner(const char* function, const std::string& bucket, bool* from_record);
+// The winner of (function, shape-class bucket) that the program set at run time, or (at_run_time false) that a tuning record names; or "".
 std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time);
 cutile_status_t set_class_winner(const char* function, const char* bucket, const char* variant, bool from_record);
 void clear_bucket_preferences();

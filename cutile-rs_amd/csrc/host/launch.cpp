@@ -295,20 +295,23 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
       g_last_source = "pinned";
     }
   }
-  auto class_winner = [&](bool at_run_time) {
+  std::string winner;
+  bool from_record = false;
+  if (want.empty() && !g_bucket.empty()) {
     ensure_tuning_records_loaded();
-    std::string pref = preferred_variant_for(function, g_bucket, at_run_time);
-    if (fits(pref)) {
-      want = pref;
-      g_last_source = "record:" + g_bucket;
-    }
-  };
-  if (want.empty() && !g_bucket.empty()) class_winner(true);
-  if (want.empty() && fits(sized)) {
+    winner = class_winner(function, g_bucket, &from_record);
+    if (!fits(winner)) winner.clear();
+  }
+  if (!winner.empty() && from_record && fits(sized)) {
+    want = sized;
+    g_last_source = "size";
+  } else if (!winner.empty()) {
+    want = winner;
+    g_last_source = "record:" + g_bucket;
+  } else if (want.empty() && fits(sized)) {
     want = sized;
     g_last_source = "size";
   }
-  if (want.empty() && !g_bucket.empty()) class_winner(false);
   if (want.empty()) {
     want = fallback;
     g_last_source = "table";
