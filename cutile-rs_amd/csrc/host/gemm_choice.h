@@ -88,7 +88,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
     // were taken for small outputs of middling K (us with ring, 64 x 64 and two-stage tiles: 220 x 64 x 1408 14.4, 9.3, 11.5; 665 x 320 x 704 9.5,
     // 6.7, 8.2; from memory 14.6, 10.1, 14.9 and 10.2, 7.7, 10.5).  The two-stage tiles are the better ones where operands are in the
     // caches and K is about 1500 (936 x 640 x 1536 12.7 us, ring 16.0), and the worse ones where they are not (21.6, 17.5).
-    // (0.265: with the fitted 0.257 the two K / V projections of 1500 x 1024 x 4096, 384 tiles of 64 x 64, took 42 us each against 38 on the ring)
+    // (0.265: with the fitted 0.257 the two K / V projections of 1500 x 1024 x 4096, 384 tiles of 64 x 64, took 42 us each, on the ring 40)
     struct Cost { double one, more, ends, split, sum; };
     struct StagedTile { const char* kernel; int bm, bn, per_cu; Cost any, aligned; };
     static const StagedTile kStaged[] = {{"staged256x128", 256, 128, 1, {1.13, 1.13, 6.5, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
