@@ -128,6 +128,7 @@ inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int
   if (s.pieces <= 4) return nullptr;   // two steps: nothing to share out
   auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   if (s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
+  // (fp8 on 128 x 128: the direct pipeline below is always the cheaper one; only a name reaches flat128x128 there)
   struct Kernel { const char* name; int bm, bn; double fp8, fp4; };
   static const Kernel kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20}, {"flat32x64", 32, 64, 0.12, 0.28}, {"flat64x64", 64, 64, 0.155, 0.36},
                                  {"flat64x128", 64, 128, 0.27, 0.62}, {"flat128x128", 128, 128, 0.52, 1.12}};
