@@ -49,6 +49,9 @@ DEVICE_FLAGS = [
     "--offload-arch=gfx950", "--cuda-device-only", "--no-gpu-bundle-output", "-c", "-O3", "-std=c++17",
     # packed FP32 instructions are kept off on purpose
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # no compilation-unit id: it hashes the source's path, and with it a code object and its fingerprint (which the tuning records name)
+    # would differ from directory to directory
+    "-fuse-cuid=none",
 ]
 # extra device-compiler flags for one-off builds (e.g. -DNAME=1), space separated
 DEVICE_FLAGS += os.environ.get("CUTILE_EXTRA_DEVICE_FLAGS", "").split()

@@ -45,13 +45,15 @@ std::string last_variant() {
 
 // The winner among the measured trials, given the id of the table's own choice ("" if it is none of them).
 const tune::Trial* winner(const tune::Output& out, const std::string& own) {
-  const tune::Trial *best = nullptr, *mine = nullptr;
+  std::vector<const tune::Trial*> best, mine;
   for (auto& t : out.trials) {
     if (!t.measured) continue;
-    if (t.config_id == out.best->id && (!best || t.median_ms < best->median_ms)) best = &t;
-    if (t.config_id == own && (!mine || t.median_ms < mine->median_ms)) mine = &t;   // (the two best are timed again, interleaved)
+    if (t.config_id == out.best->id) best.push_back(&t);
+    if (t.config_id == own) mine.push_back(&t);
   }
-  return mine && best && mine->median_ms <= best->median_ms * (1.0f + kMargin) ? mine : best;
+  // the two best met again, interleaved; where the table's own choice was not among them, the first round has to do
+  if (mine.empty() || best.size() > mine.size()) return mine.empty() || mine[0]->median_ms > best[0]->median_ms * (1.0f + kMargin) ? best.back() : mine[0];
+  return mine.back()->median_ms <= best.back()->median_ms * (1.0f + kMargin) ? mine.back() : best.back();
 }
 
 template <class T>

@@ -795,3 +795,16 @@ def test_shipped_tuning_records_are_those_of_this_build():
     files = sorted(f for f in os.listdir(os.path.join(root, "cutile-rs_amd", "tuned")) if f.endswith(".json"))
     lines = report.strip().splitlines()
     assert len(lines) == len(files) and all(l.startswith("applied ") and f"/{f}:" in l for l, f in zip(lines, files)), report
+
+
+def test_code_objects_do_not_depend_on_the_directory(tmp_path):
+    """the tuning records name a code object's fingerprint: a build in another directory has to give the same one"""
+    import __graft_entry__ as entry
+
+    build = entry._load_build_script()
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    for f in os.listdir(build.KERNEL_DIR):
+        if f.endswith(".h") or f == "rng.hip":
+            (tmp_path / f).write_bytes(open(os.path.join(build.KERNEL_DIR, f), "rb").read())
+    build._run([build.HIPCC] + build.DEVICE_FLAGS + ["-o", str(tmp_path / "rng.hsaco"), str(tmp_path / "rng.hip")])
+    assert (tmp_path / "rng.hsaco").read_bytes() == open(os.path.join(root, "cutile-rs_amd", "lib", "rng.hsaco"), "rb").read()
