@@ -1,4 +1,4 @@
-// One output block computed by several workgroups that share K, and the order in which workgroups take blocks.
+// One output block computed by several workgroups that share K.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -6,12 +6,6 @@
 
 namespace cutile {
 namespace gemm {
-
-// position of this workgroup in an XCD-contiguous order of `total` items (workgroups are dealt round-robin to the XCDs)
-__device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t total) {
-  const uint32_t xcd = id % kNumXcd, q = total / kNumXcd, r = total % kNumXcd;
-  return xcd * q + min(xcd, r) + id / kNumXcd;
-}
 
 // ---- partial sums of one output block computed by several workgroups (split K) -----------------------------------------
 // The launch's workspace holds, per output block, one f32 copy of the block per K split and a counter that is 0 between
