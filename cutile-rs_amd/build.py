@@ -36,6 +36,7 @@ IMAGES = {
     "rng": "rng.hip",
     "gemmsmall": "gemm_small.hip",
     "scaledflat": "scaled_flat.hip",
+    "gemmtiles": "gemm_tiles.hip",
 }
 HOST_SOURCES = ["hip_api.cpp", "driver.cpp", "kernel_table.cpp", "launch.cpp", "runtime.cpp", "tuning.cpp", "workspace.cpp"]
 # The recording stand-in for the HIP runtime (include/cutile_hip_testing.h) is not part of the product library: the CPU

@@ -19,7 +19,59 @@ struct GemmShape {
 
 struct GemmChoice {
   char variant[48] = "";   // "": the partition's own tile (tuning record, then the table's order)
+  bool shares_k = false;   // one of kRingTiles, with its K tiles shared
 };
+
+// Output tiles of bm x bn of a launch.
+inline uint64_t tiles_of(int64_t m, int64_t n, int bm, int bn) { return (uint64_t)((m + bm - 1) / bm) * (uint64_t)((n + bn - 1) / bn); }
+
+// The ring kernels and those of four or five whole stages (gemm_tiles.hip).  One K tile of a launch that fills few compute units costs
+// `few` us, of one that fills all of them `all` us (operands through the same L2s, and the clock), and a round of workgroups `ends` us besides.
+struct RingTile {
+  const char* kernel;
+  int bm, bn;
+  double few, all, ends;
+};
+// Least squares over 170 products of 65 to 5000 rows, f16 and bf16, operands from memory, every kernel with K unshared and shared by
+// 2 to 8 workgroups (3800 times; 5 to 8 % rms).  Over those sizes the kernel that this prices lowest takes 1.02 times the best one's time.
+constexpr RingTile kRingTiles[] = {{"256x256x64_q2x4", 256, 256, 1.03, 1.36, 8.05}, {"192x256x64_q2x4", 192, 256, 0.82, 1.08, 7.2}, {"256x128x64_q4x2", 256, 128, 0.62, 0.865, 5.95},
+                                   {"128x256x64_q2x4", 128, 256, 0.62, 0.845, 5.7}, {"192x128x64_q2x2", 192, 128, 0.44, 0.72, 4.5}, {"128x128x64_q2x2", 128, 128, 0.325, 0.55, 4.2}};
+// Workgroups that share a tile: each stores its partial tile, and the last one reads them all.  us a value of one output tile, and of all of them.
+constexpr double kShareEach = 4.2e-5, kShareAll = 1.0e-6, kShareOnce = 0.7;
+// The one that a kernel of that tile is, by the tile shape and by the marker of these kernels in its name.
+inline const RingTile* ring_tile(const char* variant, int bm, int bn) {
+  if (bm == 0 || strstr(variant, "x64_q") == nullptr) return nullptr;
+  for (const RingTile& r : kRingTiles)
+    if (r.bm == bm && r.bn == bn) return &r;
+  return nullptr;
+}
+struct RingPlan {
+  uint32_t splits;   // workgroups that share the K tiles of an output tile
+  bool two;          // 128 x 128: two workgroups to a compute unit, on the ring (K unshared)
+  double us;
+};
+// What the launch costs with the best number of workgroups to an output tile; as priced and as launched.  `partial_bytes` = room for partial tiles, 0: K is not shared.
+inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, int cus, uint64_t partial_bytes) {
+  const uint64_t t = tiles_of(m, n, r.bm, r.bn);
+  const int64_t kt = (k + 63) / 64;
+  RingPlan best{1, false, 1e30};
+  for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
+    if (s > 1 && (t * s > (uint64_t)cus || kt < 4 * s || t * s * (uint64_t)(r.bm * r.bn * 4) > partial_bytes)) break;
+    const uint64_t g = t * s, rest = g % cus;
+    const double us = (double)((kt + s - 1) / s) * ((double)(g / cus) * r.all + (rest ? r.few + (r.all - r.few) * (double)rest / cus : 0.0)) +
+                      r.ends * (double)((g + cus - 1) / cus) + (s > 1 ? kShareOnce + (kShareEach * s + kShareAll * (double)g) * (r.bm * r.bn) : 0.0);
+    if (us < best.us * 0.98) best = {s, false, us};
+  }
+  if (r.bm == 128 && r.bn == 128) {
+    // two workgroups to a compute unit, each at half its pace as soon as there are more than compute units (1623 x 2944 x
+    // 14016 f16, 299 tiles: 214 us, 192 x 128 tiles 151; 619 x 8832 x 7552 bf16, 345 tiles: 137, 256 x 128 tiles 90)
+    const uint64_t slots = 2 * (uint64_t)cus, rest = t % slots;
+    const double part = rest == 0 ? 0.0 : rest <= (uint64_t)cus ? 0.475 + 0.125 * (double)rest / cus : 1.05 + 0.02 * (double)(rest - cus) / cus;
+    const double us = (double)kt * ((double)(t / slots) * 1.07 + part) + 4.5 * (double)((t + slots - 1) / slots);
+    if (us < best.us * 1.04) best = {1, true, us};
+  }
+  return best;
+}
 
 // K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8
 // wavefronts (N = K = 4096, one row: 19.1, 12.6, 10.4, 11.3, 15.4 us with 1, 2, 4, 8, 16 splits; K = 1024: 5.0, 5.3, 5.8, 7.2).
@@ -34,7 +86,7 @@ inline uint32_t staged_splits(int bm, int bn, uint64_t blocks, int32_t k, int cu
   return (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(int64_t)(2 * (uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8), 8}));
 }
 
-inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
+inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_bytes) {
   GemmChoice c;
   if (s.k <= 64) return c;   // one K tile: nothing to stage, split or overlap
   auto pick = [&](const char* kernel) { snprintf(c.variant, sizeof(c.variant), "%s_%s", s.dtype, kernel); };
@@ -55,28 +107,18 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
   auto tiles = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   const double kt = s.k / 64.0;
   double best = 1e30;
-  // The ring kernels.  One K tile of a launch that fills few compute units costs `few` us, of one that fills all of them `all`
-  // us (operands through the same L2s, and the clock), and a round of workgroups `ends` us besides: least squares over 744 products of 65 to
-  // 6000 rows, f16 and bf16, every kernel timed on operands that stay in the caches and on operands from memory, and the mean of the
-  // two taken (each within 10 % for nine products in ten).  1500 x 14336 x 4096: 160, 186, 190 us for 192 x 256, 256 x 256, 128 x 256 tiles.
-  struct RingTile { const char* kernel; int bm, bn; double few, all, ends; };
-  static const RingTile kRing[] = {{"256x256x64_q2x4", 256, 256, 1.04, 1.50, 7.3}, {"192x256x64_q2x4", 192, 256, 0.83, 1.20, 6.3}, {"256x128x64_q4x2", 256, 128, 0.65, 0.88, 5.3},
-                                   {"128x256x64_q2x4", 128, 256, 0.63, 0.95, 5.1}, {"192x128x64_q2x2", 192, 128, 0.615, 0.75, 5.5}};
   // (up to K = 512 the start and the output of a tile are most of a launch: the partition's own tile, if it has kernels)
   const bool ring = s.aligned && (s.k > 512 || !s.own_tile) && strcmp(s.dtype, "bf16f32") != 0;
-  if (ring) {
-    for (const RingTile& r : kRing) {
-      const uint64_t t = tiles(r.bm, r.bn), rest = t % cus;
-      const double us = kt * ((double)(t / cus) * r.all + (rest ? r.few + (r.all - r.few) * (double)rest / cus : 0.0)) + r.ends * (double)((t + cus - 1) / cus);
-      if (us < best * 0.98) best = us, pick(r.kernel);
+  if (ring)
+    for (const RingTile& r : kRingTiles) {
+      // a handful of tiles of a short K: 64 x 64 staged ones, priced below (us there and on 128 x 128: 263 x 64 x 1728 9.4, 10.8; 141 x
+      // 320 x 2496 11.3, 12.3; beyond, 250 x 384 x 4352 16.3, 14.4)
+      if (s.k <= 2560 && tiles_of(s.m, s.n, 128, 128) < 16) break;
+      const RingPlan p = ring_plan(r, s.m, s.n, s.k, cus, partial_bytes);
+      // (128 x 256 against 256 x 128, f16: 619 x 8832 x 4096 56.7 us, 59.0; 620 x 5000 x 4096 40.8, 39.6; 600 x 8192 x 4096 54.1, 55.8; equal for
+      // bf16: the prices are good to 5 %, so only where it is the cheaper one by more)
+      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, pick(r.kernel), c.shares_k = p.splits > 1;
     }
-    // 128 x 128: two workgroups to a compute unit, each at half its pace as soon as there are more than compute units (1623 x 2944 x
-    // 14016 f16, 299 tiles: 214 us, 192 x 128 tiles 151; 619 x 8832 x 7552 bf16, 345 tiles: 137, 256 x 128 tiles 90)
-    const uint64_t t = tiles(128, 128), slots = 2 * (uint64_t)cus, rest = t % slots;
-    const double part = rest == 0 ? 0.0 : rest <= (uint64_t)cus ? 0.475 + 0.125 * (double)rest / cus : 1.05 + 0.02 * (double)(rest - cus) / cus;
-    const double us = kt * ((double)(t / slots) * 1.07 + part) + 4.5 * (double)((t + slots - 1) / slots);
-    if (us < best * 0.98) best = us, pick("128x128x64_q2x2");
-  }
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
   if (!s.own_tile || (ring && tiles(128, 128) < (uint64_t)cus / 2)) {
@@ -103,7 +145,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus) {
       const Cost& c1 = ring ? r.aligned : r.any;
       const double us = kt / (double)sk * std::max(c1.one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
                         (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      if (us < best * 0.98) best = us, pick(r.kernel);
+      if (us < best * 0.98) best = us, pick(r.kernel), c.shares_k = false;
     }
   }
   return c;

@@ -23,6 +23,7 @@ extern const unsigned char cutile_img_mxgemm_start[], cutile_img_mxgemm_end[];
 extern const unsigned char cutile_img_nvfp4_start[], cutile_img_nvfp4_end[];
 extern const unsigned char cutile_img_rng_start[], cutile_img_rng_end[];
 extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_end[];
+extern const unsigned char cutile_img_gemmtiles_start[], cutile_img_gemmtiles_end[];
 extern const unsigned char cutile_img_scaledflat_start[], cutile_img_scaledflat_end[];
 }
 
@@ -59,6 +60,7 @@ ImageRef image_ref(Image img) {
     case IMG_MXGEMM: return {cutile_img_mxgemm_start, cutile_img_mxgemm_end};
     case IMG_NVFP4: return {cutile_img_nvfp4_start, cutile_img_nvfp4_end};
     case IMG_RNG: return {cutile_img_rng_start, cutile_img_rng_end};
+    case IMG_GEMM_TILES: return {cutile_img_gemmtiles_start, cutile_img_gemmtiles_end};
     case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
     case IMG_SCALED_FLAT: return {cutile_img_scaledflat_start, cutile_img_scaledflat_end};
     default: return {nullptr, nullptr};
@@ -233,11 +235,17 @@ std::vector<KernelEntry> build_table() {
       add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, (uint32_t)(8 * t[0] * (t[1] + 4) * 4 + 4), 0, t[1], 0, t[0], dt, 0, 2);
     }
 
-  // the ring on tiles between 128 x 128 and 256 x 256
+  // tiles between 128 x 128 and 256 x 256, K shared by workgroups where the launcher says so: the ring, and four or five whole stages
+  // on eight wavefronts at 192 x 128 (under the name of the ring of four that it replaces) and for a 128 x 128 tile that has a compute
+  // unit to itself.  "+": members of a variant that only the launcher names ("+split" = the ring of that name with its K shared).
+  struct Tile { const char* name; int bm, bn, stages_m, stages_n; };
   for (const char* dt : {"bf16", "f16"})
-    for (auto t : {std::array<int, 4>{192, 256, 2, 4}, std::array<int, 4>{128, 256, 2, 4}, std::array<int, 4>{256, 128, 4, 2}, std::array<int, 4>{192, 128, 2, 2}}) {
-      std::string v = std::string(dt) + "_" + std::to_string(t[0]) + "x" + std::to_string(t[1]) + "x64_q" + std::to_string(t[2]) + "x" + std::to_string(t[3]);
-      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * t[3] * 64), (uint32_t)((3 * t[0] * 64 + 2 * 64 * t[1]) * 2), t[0], t[1], 64, 0, dt, 0, 2);
+    for (const Tile& t : {Tile{"192x256x64_q2x4", 192, 256, 3, 2}, Tile{"128x256x64_q2x4", 128, 256, 3, 2}, Tile{"256x128x64_q4x2", 256, 128, 3, 2},
+                          Tile{"192x128x64_q2x2", 192, 128, 4, 4}, Tile{"256x256x64_q2x4+split", 256, 256, 3, 2}, Tile{"128x128x64_q2x2+lone", 128, 128, 5, 5}}) {
+      const std::string v = std::string(dt) + "_" + t.name;
+      std::string sym = "gemm_entry__" + v;
+      std::replace(sym.begin(), sym.end(), '+', '_');
+      add("gemm", keep(v), keep(sym), strchr(t.name, '+') ? IMG_GEMM_TILES : IMG_GEMM_SMALL, 512, (uint32_t)((t.stages_m * t.bm + t.stages_n * t.bn) * 64 * 2), t.bm, t.bn, 64, 0, dt, 0, 2);
     }
   // medium sizes: register-staged tiles, K split over workgroups (any alignment, any partition shape); two LDS stages
   for (const char* dt : {"bf16", "f16", "bf16f32"})

@@ -158,6 +158,7 @@ struct BucketScope {
   ~BucketScope() { g_bucket.clear(); }
 };
 thread_local const KernelEntry* g_last_entry = nullptr;
+thread_local const KernelEntry* g_last_member = nullptr;   // the same, or the member of its family that the launch took
 thread_local hipFunction_t g_last_fn = nullptr;
 
 cutile_status_t launch_packed(hipFunction_t fn, const uint32_t grid[3], const uint32_t block[3],
@@ -267,7 +268,7 @@ cutile_status_t load_resolved(const char* function, const std::string& variant, 
   r->entry = find_entry(function, variant);
   CUTILE_REQUIRE(r->entry, CUTILE_ERR_KERNEL_NOT_FOUND, "no variant '%s' of kernel '%s'; available: %s",
                  variant.c_str(), function, list_variants(function).c_str());
-  g_last_entry = r->entry;
+  g_last_entry = g_last_member = r->entry;
   g_last_fn = nullptr;
   if (g_launch_mode == 2) return CUTILE_SUCCESS;   // specialize-only: the identity is known, nothing is loaded
   if (cutile_status_t s = current_device(&r->device)) return s;
@@ -360,6 +361,8 @@ uint32_t split_limit(uint64_t blocks, uint64_t floats) {
 // The GEMM kernels that take any partition shape and any row alignment: tile[3] x tile[1] outputs a workgroup, thin ones
 // (strips of columns) and staged ones (tiles).
 bool is_gemm_small(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
+// The GEMM kernels whose workgroups may share the K tiles of an output tile (gemm_tiles.h).
+bool is_gemm_tile(const KernelEntry* e) { return e->image == IMG_GEMM_TILES || (e->image == IMG_GEMM_SMALL && e->tile[0] != 0); }
 bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0; }
 // The block-scaled kernels on wave-private stages (scaled_flat.hip): tile[3] x tile[1] outputs a workgroup, any partition shape.
 bool is_scaled_flat(const KernelEntry* e) { return e->image == IMG_SCALED_FLAT; }
@@ -442,6 +445,28 @@ cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutil
 // An output of this size or more is read and stored past the caches (it cannot still be cached when its consumer runs,
 // and the caches are left to the operand panels): the rule of the staged epilogue, decided on the host for this family.
 constexpr int64_t kStreamedOutputBytes = 64ll << 20;
+// Replaces the resolved entry by a member of its family ("+" behind the variant's name), which only the launcher names.
+cutile_status_t use_member(Resolved* r, const char* function, const std::string& member) {
+  const KernelEntry* e = find_entry(function, member);
+  CUTILE_REQUIRE(e, CUTILE_ERR_KERNEL_NOT_FOUND, "kernel '%s' has no member '%s'", function, member.c_str());
+  if (g_launch_mode != 2) {
+    if (e != r->entry)
+      if (cutile_status_t s = load_entry(r->device, e, &r->fn)) return s;
+    g_last_fn = r->fn;
+  }
+  r->entry = g_last_member = e;
+  return CUTILE_SUCCESS;
+}
+
+// The code objects of every kernel that the size rule of the GEMM picks from.
+cutile_status_t load_gemm_images(cutile_device_t device) {
+  for (const char* v : {"f16_128x128x64_q2x2", "f16_192x256x64_q2x4", "f16_128x128x64_q2x2+lone"}) {
+    hipFunction_t fn;
+    if (cutile_status_t s = load_entry(device, find_entry("gemm", v), &fn)) return s;
+  }
+  return CUTILE_SUCCESS;
+}
+
 // Replaces the resolved family entry by the member for (z read as the initial accumulator?, z past the caches?) and
 // gives the launch grid: one workgroup per compute unit, or per tile if there are fewer tiles.
 cutile_status_t stream_member(Resolved* r, const char* function, bool accumulate, const cutile_tensor_arg_t& zt, uint64_t tiles,
@@ -450,15 +475,12 @@ cutile_status_t stream_member(Resolved* r, const char* function, bool accumulate
   std::string member = r->entry->variant;
   if (!accumulate) member += "+new";
   if (!past_caches) member += "+cached";
-  const KernelEntry* e = find_entry(function, member);
-  CUTILE_REQUIRE(e, CUTILE_ERR_KERNEL_NOT_FOUND, "kernel '%s' has no member '%s'", function, member.c_str());
+  const char* family = r->entry->variant;
+  if (cutile_status_t s = use_member(r, function, member)) return s;
+  r->entry = find_entry(function, family);   // the launcher goes on by the family's name
   int cus = 256;
-  if (g_launch_mode != 2) {
+  if (g_launch_mode != 2)
     if (cutile_status_t s = compute_units(r->device, &cus)) return s;
-    if (e != r->entry)
-      if (cutile_status_t s = load_entry(r->device, e, &r->fn)) return s;
-    g_last_fn = r->fn;
-  }
   *grid = (uint32_t)std::min<uint64_t>(tiles, (uint64_t)std::max(cus, 1));
   return CUTILE_SUCCESS;
 }
@@ -2083,9 +2105,20 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   const KernelEntry* own_tile = fast_layout ? first_of_tile("gemm", dt, bm, bn) : nullptr;   // fits any K: the table's first are not the "_r" and "_s" ones
   GemmChoice sized;
   int cus = 256;
+  SplitWorkspace ws;
+  uint64_t partial_bytes = kSplitPartialBytes;
   if (row_layout) {
     if (cutile_status_t s = current_device_units(&cus)) return s;
-    sized = choose_gemm({dt.c_str(), cover_m, cover_n, y->shape[1], k_valid, fast_layout && full_cover, own_tile != nullptr}, cus);
+    const GemmShape shape{dt.c_str(), cover_m, cover_n, y->shape[1], k_valid, fast_layout && full_cover, own_tile != nullptr};
+    sized = choose_gemm(shape, cus, partial_bytes);
+    if (sized.shares_k && g_launch_mode != 2) {
+      cutile_device_t device = nullptr;
+      if (cutile_status_t s = current_device(&device)) return s;
+      // a captured launch has no workspace and takes the best kernel of those that need none: their code objects are loaded here
+      if (cutile_status_t s = load_gemm_images(device)) return s;
+      if (g_launch_mode == 0) ws = split_workspace(device, (hipStream_t)stream);
+      if (g_launch_mode == 0 && !ws.partials) sized = choose_gemm(shape, cus, partial_bytes = 0);
+    }
   }
   // 256 x 256 partitions: the tuning records tell the kernels of that tile apart
   const bool record_first = bm == 256 && bn == 256 && strstr(sized.variant, "_256x256x64_q2x4") != nullptr;
@@ -2134,6 +2167,18 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
       if (cutile_status_t s = compute_units(res.device, &cus)) return s;
     stream_grid = (uint32_t)std::min<uint64_t>((uint64_t)tg[0] * tg[1], (uint64_t)std::max(cus, 1));
   }
+  uint32_t splits = 1;
+  if (const RingTile* ring = row_layout && fast_layout && full_cover ? ring_tile(res.entry->variant, res.entry->tile[0], res.entry->tile[1]) : nullptr) {
+    RingPlan plan = ring_plan(*ring, cover_m, cover_n, k_valid, cus, partial_bytes);
+    if (plan.splits > 1 && !ws.partials && g_launch_mode == 0) {   // a kernel that the caller or a record names
+      ws = split_workspace(res.device, (hipStream_t)stream);
+      if (!ws.partials) plan = ring_plan(*ring, cover_m, cover_n, k_valid, cus, 0);
+    }
+    splits = plan.splits;
+    const char* member = ring->bm == 256 && ring->bn == 256 && splits > 1 ? "+split" : ring->bm == 128 && ring->bn == 128 && !plan.two ? "+lone" : nullptr;
+    if (member)
+      if (cutile_status_t s = use_member(&res, "gemm", std::string(res.entry->variant) + member)) return s;
+  }
   ArgPacker args;
   args.push_partition(*z);
   args.push_tensor(*x);
@@ -2144,9 +2189,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     args.push_val<int32_t>((int32_t)cover_n);
     args.push_val<int32_t>(accumulate ? 1 : 0);
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
-    SplitWorkspace ws;
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
-    uint32_t splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
+    splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
       ws = split_workspace(res.device, (hipStream_t)stream);
@@ -2169,6 +2213,12 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   args.push_tile_grid(tg);
   args.push_val<int32_t>(accumulate ? 1 : 0);
   uint32_t grid[3] = {stream_grid ? stream_grid : tg[0] * tg[1], 1, 1};
+  if (is_gemm_tile(res.entry)) {
+    args.push_val<void*>(ws.partials);
+    args.push_val<void*>(ws.counters);
+    args.push_val<uint32_t>(splits);
+    grid[0] *= splits;
+  }
   if (res.entry->tile[0] == 0) {   // any-layout kernel: 64x64 outputs per workgroup over the covered region
     grid[0] = std::max<uint32_t>(1, div_up(cover_m, 64));
     grid[1] = std::max<uint32_t>(1, div_up(cover_n, 64));
@@ -3024,10 +3074,10 @@ cutile_status_t cutile_last_resolved_kernel(const char** function, cutile_kernel
   CUTILE_REQUIRE(g_last_entry, CUTILE_ERR_STATE, "no launcher call has resolved a kernel on this thread yet");
   *function = g_last_entry->function;
   info->function = (cutile_function_t)g_last_fn;
-  info->symbol = g_last_entry->symbol;
+  info->symbol = g_last_member->symbol;
   info->variant = g_last_entry->variant;
-  memcpy(info->block, g_last_entry->block, sizeof(info->block));
-  info->lds_bytes = g_last_entry->lds_bytes;
+  memcpy(info->block, g_last_member->block, sizeof(info->block));
+  info->lds_bytes = g_last_member->lds_bytes;
   memcpy(info->tile, g_last_entry->tile, sizeof(info->tile));
   return CUTILE_SUCCESS;
 }

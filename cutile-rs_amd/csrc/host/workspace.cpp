@@ -3,7 +3,7 @@
 // One workspace per (device, stream), allocated at the first launch that wants one and kept: launches on a stream run one
 // after another, so its workspace has one user at a time, from whatever host thread they were enqueued, and different
 // streams never share one.  A stream handle names another stream only after the runtime has drained and freed the first.
-// At most kMaxWorkspaces per device (16 MiB each); cutile_stream_release gives back the one of its stream.  Where there is
+// At most kMaxWorkspaces per device (40 MiB each); cutile_stream_release gives back the one of its stream.  Where there is
 // none to be had, the caller launches its unsplit form: beyond the limit, while the stream is being captured (a graph may
 // be replayed on another stream beside eager work on this one), on the per-thread default stream (one handle, many streams),
 // and where the runtime refuses the memory (another allocator may hold the card): a product needs none to be computed.
@@ -12,7 +12,7 @@
 namespace cutile {
 namespace {
 // More than the 32 streams that torch's pool deals out on a device, its default stream and as many of a program's own: a
-// stream made elsewhere keeps its workspace until the process ends (nothing tells this library that it is gone).  1 GiB at most.
+// stream made elsewhere keeps its workspace until the process ends (nothing tells this library that it is gone).  2.5 GiB at most.
 constexpr size_t kMaxWorkspaces = 64;
 // After a refused allocation this many launches of streams without a workspace go ahead unsplit before it is asked for again:
 // a request that fails costs more than the launch.

@@ -90,8 +90,8 @@ __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t total) 
 }
 
 // Tile index for this workgroup: XCD-contiguous, then grouped along M.  Any number of tiles: with the plain order where it is no
-// multiple of 8, each XCD fetched every panel of both operands (f16, us before and after: 600 x 7000 x 2048 on 192 x 128 tiles, 220 of
-// them, 33.8 and 29.3; 1305 x 8512 x 8640 on 192 x 256 tiles, 238, 183.9 and 170.9; 902 x 9472 x 3584, 185, 72.6 and 68.6).
+// multiple of 8, each XCD fetched every panel of both operands (f16, us before and after: 1844 x 11264 x 3584 on 128 x 256 tiles, 660 of them,
+// 193 and 154; 902 x 9472 x 3584 on 192 x 256 tiles, 185, 72 and 65).
 __device__ __forceinline__ void tile_coords(uint32_t tiles_m, uint32_t tiles_n, uint32_t* pm,
                                             uint32_t* pn) {
   const uint32_t id = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
@@ -133,6 +133,10 @@ __device__ __forceinline__ void tile_of_id(uint32_t id, uint32_t tiles_m, uint32
 // rows of one write pass fall on distinct banks.
 template <int WN>
 constexpr int kEpilogueBytesPerWave = 32 * WN * 4;
+
+// (a band of 32 columns has 8 chunks a row)
+template <int WN>
+constexpr int kBandSwizzle = WN / 4 < 16 ? WN / 4 - 1 : 15;
 
 // An output too large to still be cached when its consumer runs is read and stored past the caches
 // (nontemporal), which leaves them to the operand panels: measured +1.8 % at 8192^3 (128 MiB of bf16),
@@ -208,10 +212,10 @@ __device__ __forceinline__ void store_bands_staged(BandWriter write_band, unsign
       const int r = pass * ROWS_PER_PASS + rd_row;
       const int32_t gr = wave_row0 + tm * 32 + r;
       const unsigned char* src = stage + r * PITCH;
-      f32x4 lo = *reinterpret_cast<const f32x4*>(src + (((rd_col >> 2) ^ (r & 15)) << 4));
+      f32x4 lo = *reinterpret_cast<const f32x4*>(src + (((rd_col >> 2) ^ (r & kBandSwizzle<WN>)) << 4));
       const u32x4 o = old[tm][pass];
       if constexpr (sizeof(OutT) == 2) {
-        f32x4 hi = *reinterpret_cast<const f32x4*>(src + ((((rd_col >> 2) + 1) ^ (r & 15)) << 4));
+        f32x4 hi = *reinterpret_cast<const f32x4*>(src + ((((rd_col >> 2) + 1) ^ (r & kBandSwizzle<WN>)) << 4));
         if (accumulate) {
           lo[0] += stored_lo<OutT>(o.x);
           lo[1] += stored_hi<OutT>(o.x);
@@ -278,7 +282,7 @@ __device__ __forceinline__ void store_tile_staged16(f32x4_acc (&acc)[TN][TM], un
           for (int tn = 0; tn < TN; ++tn) {
             const int r = h * 16 + l16;
             const f32x4 v = {acc[tn][band * 2 + h][0], acc[tn][band * 2 + h][1], acc[tn][band * 2 + h][2], acc[tn][band * 2 + h][3]};
-            *reinterpret_cast<f32x4*>(stage + r * PITCH + (((tn * 4 + grp) ^ (r & 15)) << 4)) = v;
+            *reinterpret_cast<f32x4*>(stage + r * PITCH + (((tn * 4 + grp) ^ (r & kBandSwizzle<TN * 16>)) << 4)) = v;
           }
       },
       stage, zp, ldz, zM, zN, wave_row0, wave_col0, lane, accumulate);

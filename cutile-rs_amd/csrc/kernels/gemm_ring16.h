@@ -77,8 +77,14 @@ struct GemmRing16 {
     }
   }
 
+  struct AllOfK {
+    template <typename Acc>
+    __device__ __forceinline__ bool operator()(Acc&, uint32_t*) const { return true; }
+  };
+  // `combine(acc, flag)`: adds what other workgroups have summed of this tile; false where another one stores it
+  template <typename Combine = AllOfK>
   __device__ static __forceinline__ void run_tile(const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y,
-                                                  int32_t k_total, uint32_t pm, uint32_t pn, int32_t accumulate) {
+                                                  int32_t k_total, uint32_t pm, uint32_t pn, int32_t accumulate, Combine combine = Combine{}) {
     // Separately named stages: the compiler can then tell a refill of one from
     // operand reads of another and adds no waits of its own.
     __shared__ __attribute__((aligned(1024))) unsigned char xs0[kABytes];
@@ -274,6 +280,8 @@ struct GemmRing16 {
     // stages are free to carry the output (two wavefronts share an x stage, the
     // last two take the y stages).
     __syncthreads();
+    static_assert(kWaves <= 8, "no output band lies in the last y half");
+    if (!combine(acc, reinterpret_cast<uint32_t*>(ys1b))) return;
     static_assert(2 * kEpilogueBytesPerWave<WN> <= kABytes && kEpilogueBytesPerWave<WN> <= kBBytes / 2 && kWaves <= 10,
                   "the output bands must fit the stages");
     unsigned char* band = wave < 2 ? xs0 : wave < 4 ? xs1 : wave < 6 ? xs2 : wave == 6 ? ys0a : wave == 7 ? ys0b : wave == 8 ? ys1a : ys1b;

@@ -4,7 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "gemm_common.h"
-#include "gemm_ring16.h"
+#include "gemm_tiles.h"
 #include "kernel_args.h"
 #include "split_k.h"
 
@@ -441,16 +441,11 @@ GEMM_STAGED_FAMILY(bf16, __bf16, __bf16)
 GEMM_STAGED_FAMILY(f16, _Float16, _Float16)
 GEMM_STAGED_FAMILY(bf16f32, __bf16, float)
 
-// ---- ring tiles between 128 x 128 and 256 x 256 ---------------------------------------------------------------------------
-#define GEMM_RING_TILE_KERNEL(NAME, BM, BN, WVM, WVN, T)                                                                            \
-  extern "C" __global__ void __launch_bounds__(WVM * WVN * 64)                                                                      \
-      gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k, TileGrid g, int32_t accumulate) {             \
-    GemmRing16<BM, BN, WVM, WVN, T, T>::run(z, x, y, k, g, accumulate);                                                             \
-  }
-#define GEMM_RING_TILE_FAMILY(N, T)                             \
-  GEMM_RING_TILE_KERNEL(N##_192x256x64_q2x4, 192, 256, 2, 4, T) \
-  GEMM_RING_TILE_KERNEL(N##_128x256x64_q2x4, 128, 256, 2, 4, T) \
-  GEMM_RING_TILE_KERNEL(N##_256x128x64_q4x2, 256, 128, 4, 2, T) \
-  GEMM_RING_TILE_KERNEL(N##_192x128x64_q2x2, 192, 128, 2, 2, T)
-GEMM_RING_TILE_FAMILY(bf16, __bf16)
-GEMM_RING_TILE_FAMILY(f16, _Float16)
+// ---- tiles between 128 x 128 and 256 x 256 (gemm_tiles.h) ----------------------------------------------------------------------
+#define GEMM_TILES_FAMILY(N, T)                                  \
+  GEMM_RING_KERNEL(N##_192x256x64_q2x4, 192, 256, 2, 4, T)       \
+  GEMM_RING_KERNEL(N##_128x256x64_q2x4, 128, 256, 2, 4, T)       \
+  GEMM_RING_KERNEL(N##_256x128x64_q4x2, 256, 128, 4, 2, T)       \
+  GEMM_STAGES_KERNEL(N##_192x128x64_q2x2, 192, 128, 2, 4, 4, T)
+GEMM_TILES_FAMILY(bf16, __bf16)
+GEMM_TILES_FAMILY(f16, _Float16)

@@ -43,5 +43,54 @@ __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t split
   return *shared_flag != 0;
 }
 
+// A tile held in a workgroup's accumulators, computed by `splits` workgroups: false in all but the one that arrives last, whose
+// accumulators then hold the sum (in split order).  `mine` = the tile's share of the workspace; a partial tile lies there register
+// by register, thread by thread: 16 bytes a lane, whole lines, and a thread reads only what its namesakes wrote.
+constexpr int kAgentScope = 16;   // buffer accesses with sc1: past the L2, which the XCDs do not share
+template <int TM, int TN, int THREADS>
+__device__ __forceinline__ bool combine_tile(f32x4 (&acc)[TN][TM], float* mine, uint32_t* counter, uint32_t split, uint32_t splits, uint32_t* shared_flag) {
+  constexpr uint32_t kTile = TM * TN * THREADS * 16;   // bytes
+  const __amdgpu_buffer_rsrc_t part = make_rsrc(mine, kTile * splits);
+#pragma unroll
+  for (int r = 0; r < TM * TN; ++r)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[r % TN][r / TN]), part, threadIdx.x * 16, split * kTile + r * (THREADS * 16), kAgentScope);
+  if (!last_to_arrive(counter, splits, shared_flag)) return false;
+  auto add = [&](uint32_t k) {
+#pragma unroll
+    for (int r = 0; r < TM * TN; ++r)
+      acc[r % TN][r / TN] += __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(part, threadIdx.x * 16, k * kTile + r * (THREADS * 16), kAgentScope));
+  };
+  if (splits == 2) {   // a sum of two: either order
+    add(1 - split);
+    return true;
+  }
+#pragma unroll
+  for (int r = 0; r < TM * TN; ++r) acc[r % TN][r / TN] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t k = 0; k < splits; ++k) add(k);
+  return true;
+}
+
+// Tile, split and the operands of a launch of tiles_m x tiles_n x splits workgroups (split-major: an XCD's contiguous share is neighbouring
+// tiles of one range of K): x, y and k are cut to the K tiles of the split.
+struct SplitTile {
+  uint32_t pm, pn, tile, split;
+};
+template <int BK, int BYTES>
+__device__ __forceinline__ SplitTile split_tile(uint32_t tiles_m, uint32_t tiles_n, uint32_t splits, TensorArg<2>& x, TensorArg<2>& y, int32_t& k) {
+  const uint32_t tiles = tiles_m * tiles_n, pos = xcd_contiguous(blockIdx.x, tiles * splits);
+  SplitTile t;
+  t.split = pos / tiles, t.tile = pos % tiles;
+  const uint32_t per_group = kGroupM * tiles_n, first_m = t.tile / per_group * kGroupM, rows = min(tiles_m - first_m, (uint32_t)kGroupM);
+  t.pm = first_m + t.tile % per_group % rows, t.pn = t.tile % per_group / rows;
+  const int32_t k_tiles = (min(min(x.shape[1], y.shape[0]), k) + BK - 1) / BK;
+  const int32_t k0 = (int32_t)((int64_t)k_tiles * t.split / splits) * BK, k1 = (int32_t)((int64_t)k_tiles * (t.split + 1) / splits) * BK;
+  x.ptr = (unsigned char*)x.ptr + (int64_t)k0 * BYTES;
+  y.ptr = (unsigned char*)y.ptr + (int64_t)k0 * y.strides[0] * BYTES;
+  x.shape[1] = max(0, min(x.shape[1], min(k, k1)) - k0);
+  y.shape[0] = max(0, min(y.shape[0], min(k, k1)) - k0);
+  k = min(x.shape[1], y.shape[0]);
+  return t;
+}
+
 }  // namespace gemm
 }  // namespace cutile
