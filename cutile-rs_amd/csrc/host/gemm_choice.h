@@ -86,8 +86,50 @@ inline uint32_t staged_splits(int bm, int bn, uint64_t blocks, int32_t k, int cu
   return (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(int64_t)(2 * (uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8), 8}));
 }
 
+// f32: strips of 64 columns by 16, 32 or 64 rows (gemm_f32.hip).  ns a K position of a strip with the compute unit to itself (the chip then
+// does 83, 88 and 94 TFLOP/s on the matrix cores, of 157 nominal), us of start and output; least squares over 119 products of 1 to 4096
+// rows, K shared by 1 to 16 workgroups (10 to 12 % rms; the strip and split priced lowest take 1.02 times the best ones' time).  The any-layout kernel
+// that ran before: 3 x 2160 x 2208 338 us, strips 9.9; 567 x 64 x 378 49, 6.2; 403 x 1232 x 5728 1055, 119; 107 x 364 x 6461 1345, 19.
+struct F32Strip {
+  const char* kernel;
+  int rows;
+  double k, each;   // `each`: ns a value of an output strip for each of the workgroups that share its K
+};
+constexpr F32Strip kF32Strips[] = {{"strip16x64", 16, 6.35, 0.23}, {"strip32x64", 32, 11.8, 0.11}, {"strip64x64", 64, 22.3, 0.055}};
+inline const F32Strip* f32_strip(int rows) {
+  for (const F32Strip& r : kF32Strips)
+    if (r.rows == rows) return &r;
+  return nullptr;
+}
+struct F32Plan {
+  uint32_t splits;
+  double us;
+};
+inline F32Plan f32_plan(const F32Strip& r, int64_t m, int64_t n, int32_t k, int cus, uint64_t partial_bytes) {
+  const uint64_t t = tiles_of(m, n, r.rows, 64);
+  F32Plan best{1, 1e30};
+  for (uint32_t s : {1u, 2u, 4u, 8u, 16u}) {
+    if (s > 1 && (t * s > 2 * (uint64_t)cus || k < 128 * (int64_t)s || t * s * (uint64_t)(r.rows * 64 * 4) > partial_bytes)) break;
+    const uint64_t g = t * s;
+    const double rounds = (double)std::max<uint64_t>(1, (g + cus - 1) / cus), values = r.rows * 64;
+    const double us = (double)k / s * r.k * 1e-3 * rounds + 2.1 * (rounds + 1) + (s > 1 ? 0.8 + (r.each * s * 1e-3 + 4e-6 * (double)g / cus) * values : 0.0);
+    if (us < best.us * 0.98) best = {s, us};
+  }
+  return best;
+}
+
 inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_bytes) {
   GemmChoice c;
+  if (strcmp(s.dtype, "f32") == 0) {
+    const F32Strip* best = nullptr;
+    double us = 1e30;
+    for (const F32Strip& r : kF32Strips) {
+      const F32Plan p = f32_plan(r, s.m, s.n, s.k, cus, partial_bytes);
+      if (s.y_cols >= 64 && p.us < us * 0.98) us = p.us, best = &r;
+    }
+    if (best) snprintf(c.variant, sizeof(c.variant), "f32_%s", best->kernel);
+    return c;
+  }
   if (s.k <= 64) return c;   // one K tile: nothing to stage, split or overlap
   auto pick = [&](const char* kernel) { snprintf(c.variant, sizeof(c.variant), "%s_%s", s.dtype, kernel); };
   // Few rows.  Measured at 1 to 64 rows, f16 and bf16 (us, thin against 128 x 128 tiles): 4096 x 4096 10 - 21 against 53,

@@ -23,6 +23,7 @@ extern const unsigned char cutile_img_mxgemm_start[], cutile_img_mxgemm_end[];
 extern const unsigned char cutile_img_nvfp4_start[], cutile_img_nvfp4_end[];
 extern const unsigned char cutile_img_rng_start[], cutile_img_rng_end[];
 extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_end[];
+extern const unsigned char cutile_img_gemmf32_start[], cutile_img_gemmf32_end[];
 extern const unsigned char cutile_img_gemmtiles_start[], cutile_img_gemmtiles_end[];
 extern const unsigned char cutile_img_scaledflat_start[], cutile_img_scaledflat_end[];
 }
@@ -60,6 +61,7 @@ ImageRef image_ref(Image img) {
     case IMG_MXGEMM: return {cutile_img_mxgemm_start, cutile_img_mxgemm_end};
     case IMG_NVFP4: return {cutile_img_nvfp4_start, cutile_img_nvfp4_end};
     case IMG_RNG: return {cutile_img_rng_start, cutile_img_rng_end};
+    case IMG_GEMM_F32: return {cutile_img_gemmf32_start, cutile_img_gemmf32_end};
     case IMG_GEMM_TILES: return {cutile_img_gemmtiles_start, cutile_img_gemmtiles_end};
     case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
     case IMG_SCALED_FLAT: return {cutile_img_scaledflat_start, cutile_img_scaledflat_end};
@@ -254,6 +256,12 @@ std::vector<KernelEntry> build_table() {
       add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * 64), (uint32_t)(2 * 64 * 2 * (t[0] + t[1]) + (t[0] * t[1] == 64 * 64 ? 4 : 0)), 0, t[1],
           64, t[0], dt, 0, 2);
     }
+
+  // f32 on the matrix cores: strips of 64 columns, K dealt to 8 wavefronts and to the workgroups of a strip
+  for (int rows : {16, 32, 64}) {
+    const std::string v = "f32_strip" + std::to_string(rows) + "x64";
+    add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_F32, 512, (uint32_t)(8 * rows * 68 * 4 + 4), 0, 64, 0, rows, "f32", 0, 2);
+  }
 
   // batched GEMM (cutile-examples/examples/batch_matmul.rs): the pipelined bodies with the batch on a grid axis
   for (const char* kind : {"q", "r"})          // rings of three a stages and two b stages (q: on v_mfma_f32_16x16x32, any K; r: whole K tiles only)

@@ -11,7 +11,7 @@
 
 namespace cutile {
 
-enum Image : int { IMG_ELEMENTWISE = 0, IMG_ROWWISE, IMG_GEMM, IMG_FMHA, IMG_MXGEMM, IMG_NVFP4, IMG_RNG, IMG_GEMM_SMALL, IMG_SCALED_FLAT, IMG_GEMM_TILES, IMG_COUNT };
+enum Image : int { IMG_ELEMENTWISE = 0, IMG_ROWWISE, IMG_GEMM, IMG_FMHA, IMG_MXGEMM, IMG_NVFP4, IMG_RNG, IMG_GEMM_SMALL, IMG_SCALED_FLAT, IMG_GEMM_TILES, IMG_GEMM_F32, IMG_COUNT };
 
 struct KernelEntry {
   const char* function;  // entry name in the reference, e.g. "gemm"
@@ -20,7 +20,7 @@ struct KernelEntry {
   Image image;
   uint32_t block[3];
   uint32_t lds_bytes;
-  int32_t tile[4];       // (BM, BN, BK, extra); 0 = not tile-specific; gemm_small.hip: (0, columns, K tile or 0, rows)
+  int32_t tile[4];       // (BM, BN, BK, extra); 0 = not tile-specific; gemm_small.hip, gemm_f32.hip: (0, columns, K tile or 0, rows)
   const char* dtype;     // element type the variant is written for, or ""
   int64_t capacity;      // row-wise kernels: longest segment held in registers; 0 = n/a
   int32_t rank;          // elementwise kernels: tensor rank; 0 = n/a

@@ -360,7 +360,7 @@ uint32_t split_limit(uint64_t blocks, uint64_t floats) {
 }
 // The GEMM kernels that take any partition shape and any row alignment: tile[3] x tile[1] outputs a workgroup, thin ones
 // (strips of columns) and staged ones (tiles).
-bool is_gemm_small(const KernelEntry* e) { return e->image == IMG_GEMM_SMALL && e->tile[0] == 0; }
+bool is_gemm_small(const KernelEntry* e) { return (e->image == IMG_GEMM_SMALL && e->tile[0] == 0) || e->image == IMG_GEMM_F32; }
 // The GEMM kernels whose workgroups may share the K tiles of an output tile (gemm_tiles.h).
 bool is_gemm_tile(const KernelEntry* e) { return e->image == IMG_GEMM_TILES || (e->image == IMG_GEMM_SMALL && e->tile[0] != 0); }
 bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0; }
@@ -2099,7 +2099,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   const int64_t cover_m = std::min<int64_t>((int64_t)tg[0] * bm, zt.shape[0]), cover_n = std::min<int64_t>((int64_t)tg[1] * bn, zt.shape[1]);
   // The kernels of gemm_small.hip take any partition shape and any row alignment; they need rows of unit stride and operands
   // that reach as far as the output.
-  const bool row_layout = x->strides[1] == 1 && y->strides[1] == 1 && zt.strides[1] == 1 && !in_f32 && x->shape[0] >= cover_m &&
+  const bool row_layout = x->strides[1] == 1 && y->strides[1] == 1 && zt.strides[1] == 1 && x->shape[0] >= cover_m &&
                           y->shape[1] >= cover_n && k_valid > 0 && extent_bytes_2d(*x) < kDescriptorLimit &&
                           extent_bytes_2d(*y) < kDescriptorLimit && extent_bytes_2d(zt) < kDescriptorLimit;
   const KernelEntry* own_tile = fast_layout ? first_of_tile("gemm", dt, bm, bn) : nullptr;   // fits any K: the table's first are not the "_r" and "_s" ones
@@ -2190,7 +2190,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     args.push_val<int32_t>(accumulate ? 1 : 0);
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
-    splits = is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
+    const F32Strip* strip = in_f32 ? f32_strip(res.entry->tile[3]) : nullptr;
+    splits = strip ? f32_plan(*strip, cover_m, cover_n, k_valid, cus, kSplitPartialBytes).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
       ws = split_workspace(res.device, (hipStream_t)stream);

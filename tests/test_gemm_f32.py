@@ -1,0 +1,50 @@
+"""f32 GEMM on the matrix cores: strips of 16, 32 and 64 rows by 64 columns against float64, and the calls that stay on the any-layout kernel."""
+import numpy as np
+import pytest
+import torch
+
+from util import rel_l2
+
+
+# one strip exactly, its edges, a ragged last step of K, fewer K positions than a step, K dealt to several workgroups, odd row pitches
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", ["f32_strip16x64", "f32_strip32x64", "f32_strip64x64", None])
+@pytest.mark.parametrize("m,n,k", [(16, 64, 256), (1, 64, 1), (64, 128, 16), (65, 65, 17), (3, 127, 4099), (33, 641, 511), (200, 333, 1300)])
+@pytest.mark.parametrize("accumulate", [True, False])
+def test_gpu_f32_strips(ct, dev, variant, m, n, k, accumulate):
+    g = np.random.default_rng(7 * m + n + k)
+    a, b, c = (g.standard_normal(s).astype(np.float32) for s in ((m, k), (k, n), (m, n)))
+    want = a.astype(np.float64) @ b.astype(np.float64) + (c if accumulate else 0)
+    z = torch.full((m + 1, n), 7.0, device=dev)                         # a row behind z that nothing may touch
+    x, y = torch.from_numpy(a).to(dev), torch.from_numpy(b).to(dev)
+    for _ in range(2):                                                  # the second launch finds the first one's counters at 0
+        z[:m] = torch.from_numpy(c).to(dev)
+        ct.gemm(ct.partition(z[:m], [64, 64]), x, y, k, accumulate=accumulate, generics=["f32", 64, 64, 1], variant=variant)
+        torch.cuda.synchronize()
+        assert ct.last_resolved()["variant"].startswith("f32_strip")
+        # a sum of k products in f32 is off by sqrt(k) roundings of 2^-24 of its own size at most, whatever their order
+        assert rel_l2(z[:m].double().cpu().numpy(), want) <= 2.0 ** -24 * (2 + np.sqrt(k))
+        assert torch.all(z[m] == 7.0)
+
+
+@pytest.mark.gpu
+def test_gpu_f32_partial_cover(ct, dev):
+    """a grid over part of z stores that part alone"""
+    x, y, z = torch.ones(100, 40, device=dev), torch.ones(40, 200, device=dev), torch.zeros(100, 200, device=dev)
+    ct.gemm(ct.partition(z, [16, 48], prefix=True), x, y, 40, grid=(3, 2, 1), accumulate=False, generics=["f32", 16, 48, 8])
+    torch.cuda.synchronize()
+    want = torch.zeros(100, 200, device=dev)
+    want[:48, :96] = 40
+    assert torch.equal(z, want)
+
+
+def test_f32_calls_that_the_strips_do_not_take(fake_hip):
+    """strided columns, operands shorter than the output, fewer than 64 columns of y: the any-layout kernel, as before"""
+    ct = fake_hip
+    e = torch.empty
+    for z, x, y in ((e(64, 128), e(64, 64), e(128, 64).T), (e(64, 128), e(63, 64), e(64, 128)), (e(64, 128), e(64, 64), e(64, 127)),
+                    (e(64, 63), e(64, 64), e(64, 63)), (e(64, 256)[:, ::2], e(64, 64), e(64, 128))):
+        ct.gemm(ct.partition(z, [16, 16]), x, y, 64, generics=["f32", 16, 16, 8])
+        assert ct.last_resolved()["variant"] == "f32_generic"
+    ct.gemm(ct.partition(e(64, 128), [16, 16]), e(64, 64), e(64, 128), 64, generics=["f32", 16, 16, 8])
+    assert ct.last_resolved()["variant"].startswith("f32_strip") and ct.last_resolved()["source"] == "size"
