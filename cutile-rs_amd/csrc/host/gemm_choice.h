@@ -205,10 +205,31 @@ struct ScaledShape {
 inline uint32_t scaled_splits(uint64_t blocks, int32_t pieces, int cus) {
   return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / 2 / std::max<uint64_t>(blocks, 1)), pieces / (2 * 8 * 2)));
 }
+// fp8 on 128 x 128 tiles that have a compute unit each (mxfp8_tiles.hip), K shared by up to 8 workgroups in whole blocks of 512 positions: us a K tile
+// of 128 where few compute units are busy and where all are, us of start and output, and of partial tiles (113 times of 54 products, 9.5 % rms).
+// Against the two-stage kernel: 1000 x 4096 x 4096 26.5 -> 22.3 us, 1943 x 1472 x 7296 50 -> 37, 459 x 4416 x 512 7.6 -> 6.6; against strips, with K
+// shared by two: 859 x 1600 x 5888 28.4 -> 19.6, 360 x 4352 x 6912 35 -> 28.
+struct MxPlan {
+  uint32_t splits;   // 0: more tiles than compute units
+  double us;
+};
+inline MxPlan mx_plan(int64_t m, int64_t n, int32_t pieces, int cus, uint64_t partial_bytes) {
+  const uint64_t t = tiles_of(m, n, 128, 128);
+  const int64_t kt = pieces / 2;
+  MxPlan best{0, 1e30};
+  for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
+    const uint64_t g = t * s;
+    if (g > (uint64_t)cus || (s > 1 && (kt < 8 * s || g * 128 * 128 * 4 > partial_bytes))) break;
+    const double tiles = s > 1 ? (double)((kt + 4 * s - 1) / (4 * s) * 4) : (double)kt;
+    const double us = tiles * (0.405 + 0.255 * (double)g / cus) + 4.3 + (s > 1 ? (4.4e-5 * s + 1e-6 * (double)g) * 128 * 128 : 0.0);
+    if (us < best.us * 0.98) best = {s, us};
+  }
+  return best;
+}
 // The kernel by name, or nullptr: the partition's own (tuning record, then the table's order).  us per 64-byte piece of K for
 // one block on each compute unit, measured at K = 4096 (mxfp8: 16 x 4096 9.4 us, 64 x 4096 13.4, 512 x 4096 21 on 64 x 128 blocks, 24 with
 // 128 x 128 tiles; nvfp4: 9.9, 14.7, 24).  The 256 x 256 kernels are the better ones where their tiles come near to filling the chip.
-inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus) {
+inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus, uint64_t partial_bytes) {
   if (s.pieces <= 4) return nullptr;   // two steps: nothing to share out
   auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   if (s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
@@ -223,7 +244,11 @@ inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int
     const double us = (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + 3.5);
     if (us < best) best = us, name = k.name;
   }
-  if (!s.fp4) {   // two workgroups to a compute unit
+  if (!s.fp4) {
+    const MxPlan lone = mx_plan(s.m, s.n, s.pieces, cus, partial_bytes);
+    if (lone.splits && lone.us < best) best = lone.us, name = "128x128x128_e2x2";
+  }
+  if (!s.fp4 && blocks(128, 128) > (uint64_t)cus) {   // two workgroups to a compute unit
     const uint64_t b = blocks(128, 128), rest = b % (2 * (uint64_t)cus);
     const double us = (double)(b / (2 * (uint64_t)cus)) * (0.58 * s.pieces + 4) + (rest == 0 ? 0.0 : (rest <= (uint64_t)cus ? 0.31 : 0.58) * s.pieces + 4);
     if (us < best) best = us, name = "128x128x128_e2x2";

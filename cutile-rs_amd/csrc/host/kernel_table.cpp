@@ -24,6 +24,7 @@ extern const unsigned char cutile_img_nvfp4_start[], cutile_img_nvfp4_end[];
 extern const unsigned char cutile_img_rng_start[], cutile_img_rng_end[];
 extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_end[];
 extern const unsigned char cutile_img_gemmf32_start[], cutile_img_gemmf32_end[];
+extern const unsigned char cutile_img_mxtiles_start[], cutile_img_mxtiles_end[];
 extern const unsigned char cutile_img_gemmtiles_start[], cutile_img_gemmtiles_end[];
 extern const unsigned char cutile_img_scaledflat_start[], cutile_img_scaledflat_end[];
 }
@@ -62,6 +63,7 @@ ImageRef image_ref(Image img) {
     case IMG_NVFP4: return {cutile_img_nvfp4_start, cutile_img_nvfp4_end};
     case IMG_RNG: return {cutile_img_rng_start, cutile_img_rng_end};
     case IMG_GEMM_F32: return {cutile_img_gemmf32_start, cutile_img_gemmf32_end};
+    case IMG_MX_TILES: return {cutile_img_mxtiles_start, cutile_img_mxtiles_end};
     case IMG_GEMM_TILES: return {cutile_img_gemmtiles_start, cutile_img_gemmtiles_end};
     case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
     case IMG_SCALED_FLAT: return {cutile_img_scaledflat_start, cutile_img_scaledflat_end};
@@ -413,6 +415,11 @@ std::vector<KernelEntry> build_table() {
 
   // ---- block-scaled products through wave-private stages (scaled_flat.hip): any partition shape; LDS = the eight wavefronts' stages, which
   // become one f32 copy of the block per share of K, whichever is larger (t[2] shares; a stage holds t[3] rows of x and 64 of y) ----
+  // the member of "e2x2" for tiles that have a compute unit each: four stages and two scale blocks, eight wavefronts, K shared by workgroups
+  for (const char* out : {"bf16", "f32"}) {
+    const std::string v = std::string("mxfp8_") + out + "_128x128x128_e2x2";
+    add("linear_tile", keep(v + "+lone"), keep("linear_tile_entry__" + v + "_lone"), IMG_MX_TILES, 512, 4 * 256 * 128 + 2 * 256 * 16, 128, 128, 128, 0, out, 0, 2);
+  }
   for (const char* dt : {"bf16", "f32"})
     for (auto t : {std::array<int, 4>{16, 64, 8, 16}, std::array<int, 4>{32, 64, 8, 32}, std::array<int, 4>{64, 64, 8, 64}, std::array<int, 4>{64, 128, 4, 64},
                    std::array<int, 4>{128, 128, 2, 64}})

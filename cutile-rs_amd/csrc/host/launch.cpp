@@ -367,14 +367,21 @@ bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0;
 // The block-scaled kernels on wave-private stages (scaled_flat.hip): tile[3] x tile[1] outputs a workgroup, any partition shape.
 bool is_scaled_flat(const KernelEntry* e) { return e->image == IMG_SCALED_FLAT; }
 
+// Room for the partial tiles of a block-scaled product, and the workspace once somebody has asked for it.
+struct ScaledRoom {
+  uint64_t bytes = kSplitPartialBytes;
+  SplitWorkspace ws;
+};
+
 // Picks the kernel of a block-scaled product.  A kernel tile that is a whole multiple of the partition tile computes the
 // same output when the launch covers the whole tensor (a 16 x 16 example partition runs on the 32 x 32 kernel), and so do
 // the kernels on wave-private stages, which take `flat` launches: whole outputs, scale rows on 4-byte boundaries.
 cutile_status_t resolve_scaled(const char* function, const char* prefix, const std::string& dt, int bm, int bn, bool full_cover, bool flat,
-                               const ScaledShape& shape, const cutile_launch_opts_t* opts, const std::string& missing, int* cus, Resolved* res) {
+                               const ScaledShape& shape, const cutile_launch_opts_t* opts, const std::string& missing, cutile_stream_t stream, int* cus,
+                               ScaledRoom* room, Resolved* res) {
   std::vector<const KernelEntry*> fit, others;
   for (const KernelEntry* e : kernels_of(function)) {
-    if (dt != e->dtype) continue;
+    if (e->image == IMG_MX_TILES || dt != e->dtype) continue;   // (members, which only launch_scaled names)
     if (is_scaled_flat(e)) {
       if (flat) others.push_back(e);
     } else if ((e->tile[0] == bm && e->tile[1] == bn) || (full_cover && e->tile[0] % bm == 0 && e->tile[1] % bn == 0)) {
@@ -391,7 +398,19 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
   std::string sized;
   if (flat) {
     if (cutile_status_t s = current_device_units(cus)) return s;
-    if (const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus)) sized = prefix + dt + "_" + kernel;
+    const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes);
+    if (kernel && strcmp(kernel, "128x128x128_e2x2") == 0 && mx_plan(shape.m, shape.n, shape.pieces, *cus, room->bytes).splits > 1 && g_launch_mode != 2) {
+      // a captured launch has no workspace and takes the best kernel of those that need none: their code object is loaded here
+      cutile_device_t device = nullptr;
+      hipFunction_t fn;
+      if (cutile_status_t s = current_device(&device)) return s;
+      if (cutile_status_t s = load_entry(device, find_entry(function, "mxfp8_bf16_flat64x64"), &fn)) return s;
+      if (g_launch_mode == 0) {
+        room->ws = split_workspace(device, (hipStream_t)stream);
+        if (!room->ws.partials) kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes = 0);
+      }
+    }
+    if (kernel) sized = prefix + dt + "_" + kernel;
   }
   if (!sized.empty() && !(opts && opts->variant) && preferred_variant(function).empty() && preferred_variant_for(function, g_bucket, true).empty())
     return resolve_own(function, sized.c_str(), "size", res);
@@ -401,10 +420,23 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
   return resolve_entry(function, opts, acceptable[0], acceptable, res, sized);
 }
 
+// Replaces the resolved entry by a member of its family ("+" behind the variant's name), which only the launcher names.
+cutile_status_t use_member(Resolved* r, const char* function, const std::string& member) {
+  const KernelEntry* e = find_entry(function, member);
+  CUTILE_REQUIRE(e, CUTILE_ERR_KERNEL_NOT_FOUND, "kernel '%s' has no member '%s'", function, member.c_str());
+  if (g_launch_mode != 2) {
+    if (e != r->entry)
+      if (cutile_status_t s = load_entry(r->device, e, &r->fn)) return s;
+    g_last_fn = r->fn;
+  }
+  r->entry = g_last_member = e;
+  return CUTILE_SUCCESS;
+}
+
 // Launches it; `pieces` = 64-byte pieces of a row.
 cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutile_partition_arg_t* z, const cutile_tensor_arg_t* x,
                               const cutile_tensor_arg_t* y, const cutile_tensor_arg_t* xs, const cutile_tensor_arg_t* ys, float alpha,
-                              const uint32_t tg[3], int32_t pieces, int cus) {
+                              const uint32_t tg[3], int32_t pieces, int cus, ScaledRoom room) {
   const cutile_tensor_arg_t& zt = z->tensor;
   ArgPacker args;
   args.push_partition(*z);
@@ -439,25 +471,25 @@ cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutil
     kg[1] = div_up(zt.shape[1], res.entry->tile[1]);
   }
   args.push_tile_grid(kg);
-  const uint32_t grid[3] = {kg[0] * kg[1], 1, 1};
+  uint32_t grid[3] = {kg[0] * kg[1], 1, 1};
+  if (strstr(res.entry->variant, "_128x128x128_e2x2") != nullptr && grid[0] <= (uint32_t)cus && pieces >= 4) {   // a compute unit to each tile
+    uint32_t splits = mx_plan(zt.shape[0], zt.shape[1], pieces, cus, kg[0] == div_up(zt.shape[0], 128) && kg[1] == div_up(zt.shape[1], 128) ? room.bytes : 0).splits;
+    if (splits > 1 && g_launch_mode == 0 && !room.ws.partials) {   // a kernel that the caller or a record names
+      room.ws = split_workspace(res.device, (hipStream_t)stream);
+      if (!room.ws.partials) splits = 1;
+    }
+    splits = std::max(splits, 1u);   // (a partial launch may cover fewer tiles than z has)
+    if (cutile_status_t s = use_member(&res, res.entry->function, std::string(res.entry->variant) + "+lone")) return s;
+    args.push_val<void*>(room.ws.partials);
+    args.push_val<void*>(room.ws.counters);
+    args.push_val<uint32_t>(splits);
+    grid[0] *= splits;
+  }
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 // An output of this size or more is read and stored past the caches (it cannot still be cached when its consumer runs,
 // and the caches are left to the operand panels): the rule of the staged epilogue, decided on the host for this family.
 constexpr int64_t kStreamedOutputBytes = 64ll << 20;
-// Replaces the resolved entry by a member of its family ("+" behind the variant's name), which only the launcher names.
-cutile_status_t use_member(Resolved* r, const char* function, const std::string& member) {
-  const KernelEntry* e = find_entry(function, member);
-  CUTILE_REQUIRE(e, CUTILE_ERR_KERNEL_NOT_FOUND, "kernel '%s' has no member '%s'", function, member.c_str());
-  if (g_launch_mode != 2) {
-    if (e != r->entry)
-      if (cutile_status_t s = load_entry(r->device, e, &r->fn)) return s;
-    g_last_fn = r->fn;
-  }
-  r->entry = g_last_member = e;
-  return CUTILE_SUCCESS;
-}
-
 // The code objects of every kernel that the size rule of the GEMM picks from.
 cutile_status_t load_gemm_images(cutile_device_t device) {
   for (const char* v : {"f16_128x128x64_q2x2", "f16_192x256x64_q2x4", "f16_128x128x64_q2x2+lone"}) {
@@ -2910,8 +2942,9 @@ cutile_status_t cutile_launch_linear_tile_mxfp8(cutile_stream_t stream, const cu
   BucketScope bucket("mxfp8_" + dt + "_" + std::to_string(bm) + "x" + std::to_string(bn));
   Resolved res;
   int cus = 256;
-  if (cutile_status_t s = resolve_scaled("linear_tile", "mxfp8_", dt, bm, bn, full_cover, full_cover, {M, N, K / 64, false}, opts, missing, &cus, &res)) return s;
-  return launch_scaled(res, stream, z, x, y, xs, ys, alpha, tg, K / 64, cus);
+  ScaledRoom room;
+  if (cutile_status_t s = resolve_scaled("linear_tile", "mxfp8_", dt, bm, bn, full_cover, full_cover, {M, N, K / 64, false}, opts, missing, stream, &cus, &room, &res)) return s;
+  return launch_scaled(res, stream, z, x, y, xs, ys, alpha, tg, K / 64, cus, room);
 }
 
 cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cutile_partition_arg_t* z,
@@ -2971,8 +3004,9 @@ cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cu
   const bool flat = full_cover && KP >= 128 && xs->strides[0] % 4 == 0 && ys->strides[0] % 4 == 0 && ((uintptr_t)xs->ptr & 3) == 0 && ((uintptr_t)ys->ptr & 3) == 0;
   Resolved res;
   int cus = 256;
-  if (cutile_status_t s = resolve_scaled("linear_tile_nvfp4", "", dt, bm, bn, full_cover, flat, {M, N, (KP + 63) / 64, true}, opts, missing, &cus, &res)) return s;
-  return launch_scaled(res, stream, z, x, y, xs, ys, alpha, tg, (KP + 63) / 64, cus);
+  ScaledRoom room;
+  if (cutile_status_t s = resolve_scaled("linear_tile_nvfp4", "", dt, bm, bn, full_cover, flat, {M, N, (KP + 63) / 64, true}, opts, missing, stream, &cus, &room, &res)) return s;
+  return launch_scaled(res, stream, z, x, y, xs, ys, alpha, tg, (KP + 63) / 64, cus, room);
 }
 
 }  // extern "C"
