@@ -73,6 +73,8 @@ inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, in
   return best;
 }
 
+// 16-bit weights of this size are not found in the caches by the launch that reads them next (gemm_thin.h).
+inline bool streamed_past_caches(int64_t n, int32_t k) { return n * k * 2 >= (96ll << 20); }
 // K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8
 // wavefronts (N = K = 4096, one row: 19.1, 12.6, 10.4, 11.3, 15.4 us with 1, 2, 4, 8, 16 splits; K = 1024: 5.0, 5.3, 5.8, 7.2).
 inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus) {
@@ -140,7 +142,8 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
   // columns, 0.76 in the mean (us: 60 x 19072 x 448 12.5 against 9.0 and 7.5 from memory and from the caches), and the best of them 1.10 up to there.
   // Up to 128 rows (two passes over y, the second from L2) while the strips of both passes fit the chip once
   // (4096 x 4096 23 us against 27 with staged tiles; 14336 x 4096 60 against 46).
-  const bool many = s.n >= 192 * 128;
+  // From 96 strips of 128 columns on where y is streamed past the caches (4096 x 14336, 112 strips and two workgroups to each: 22.1 us, 64-column strips 23.0).
+  const bool many = s.n >= 192 * 128 || (s.m <= 16 && s.n >= 96 * 128 && streamed_past_caches(s.n, s.k));
   const int64_t strips = (s.n + 63) / 64;
   if (s.y_cols >= 64 && (s.m <= 32 || (s.m <= 64 && strips <= cus) || (s.m <= 128 && 2 * strips <= cus))) {
     pick(s.m > 32 ? "thin64x64" : s.m > 16 ? "thin32x64" : many && s.y_cols >= 128 ? "thin16x128" : "thin16x64");

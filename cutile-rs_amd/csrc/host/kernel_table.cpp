@@ -236,7 +236,10 @@ std::vector<KernelEntry> build_table() {
   for (const char* dt : {"bf16", "f16", "bf16f32"})
     for (auto t : {std::array<int, 2>{16, 64}, std::array<int, 2>{16, 128}, std::array<int, 2>{32, 64}, std::array<int, 2>{64, 64}}) {
       std::string v = std::string(dt) + "_thin" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
-      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, (uint32_t)(8 * t[0] * (t[1] + 4) * 4 + 4), 0, t[1], 0, t[0], dt, 0, 2);
+      const uint32_t sums = (uint32_t)(8 * t[0] * (t[1] + 4) * 4 + 4);
+      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, 512, sums, 0, t[1], 0, t[0], dt, 0, 2);
+      if (t[0] == 16)   // the member that reads y past the caches
+        add("gemm", keep(v + "+nt"), keep("gemm_entry__" + v + "_nt"), IMG_GEMM_TILES, 512, sums, 0, t[1], 0, t[0], dt, 0, 2);
     }
 
   // tiles between 128 x 128 and 256 x 256, K shared by workgroups where the launcher says so: the ring, and four or five whole stages

@@ -360,9 +360,9 @@ uint32_t split_limit(uint64_t blocks, uint64_t floats) {
 }
 // The GEMM kernels that take any partition shape and any row alignment: tile[3] x tile[1] outputs a workgroup, thin ones
 // (strips of columns) and staged ones (tiles).
-bool is_gemm_small(const KernelEntry* e) { return (e->image == IMG_GEMM_SMALL && e->tile[0] == 0) || e->image == IMG_GEMM_F32; }
+bool is_gemm_small(const KernelEntry* e) { return ((e->image == IMG_GEMM_SMALL || e->image == IMG_GEMM_TILES) && e->tile[0] == 0) || e->image == IMG_GEMM_F32; }
 // The GEMM kernels whose workgroups may share the K tiles of an output tile (gemm_tiles.h).
-bool is_gemm_tile(const KernelEntry* e) { return e->image == IMG_GEMM_TILES || (e->image == IMG_GEMM_SMALL && e->tile[0] != 0); }
+bool is_gemm_tile(const KernelEntry* e) { return (e->image == IMG_GEMM_TILES || e->image == IMG_GEMM_SMALL) && e->tile[0] != 0; }
 bool is_thin(const KernelEntry* e) { return is_gemm_small(e) && e->tile[2] == 0; }
 // The block-scaled kernels on wave-private stages (scaled_flat.hip): tile[3] x tile[1] outputs a workgroup, any partition shape.
 bool is_scaled_flat(const KernelEntry* e) { return e->image == IMG_SCALED_FLAT; }
@@ -2211,6 +2211,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     if (member)
       if (cutile_status_t s = use_member(&res, "gemm", std::string(res.entry->variant) + member)) return s;
   }
+  if (is_thin(res.entry) && !in_f32 && cover_m <= 16 && res.entry->tile[3] == 16 && streamed_past_caches(cover_n, k_valid))   // y is read once
+    if (cutile_status_t s = use_member(&res, "gemm", std::string(res.entry->variant) + "+nt")) return s;
   ArgPacker args;
   args.push_partition(*z);
   args.push_tensor(*x);

@@ -1,5 +1,6 @@
-// Members of the GEMM tile families that only the launcher names (gemm_tiles.h): the 256 x 256 ring with its K shared, and the 128 x 128
-// tile that has a compute unit to itself.
+// Members of GEMM families that only the launcher names: the 256 x 256 ring with its K shared, the 128 x 128 tile that has a compute unit
+// to itself (gemm_tiles.h), and strips that read y past the caches (gemm_thin.h).
+#include "gemm_thin.h"
 #include "gemm_tiles.h"
 
 using namespace cutile;
@@ -10,3 +11,10 @@ using namespace cutile::gemm;
   GEMM_RING_KERNEL(N##_256x256x64_q2x4_split, 256, 256, 2, 4, T)
 GEMM_TILES_FAMILY(bf16, __bf16)
 GEMM_TILES_FAMILY(f16, _Float16)
+
+#define GEMM_THIN_NT_FAMILY(T, IN_T, OUT_T)                    \
+  GEMM_THIN_KERNEL(T##_thin16x64_nt, IN_T, OUT_T, 1, 4, true)  \
+  GEMM_THIN_KERNEL(T##_thin16x128_nt, IN_T, OUT_T, 1, 8, true)
+GEMM_THIN_NT_FAMILY(bf16, __bf16, __bf16)
+GEMM_THIN_NT_FAMILY(f16, _Float16, _Float16)
+GEMM_THIN_NT_FAMILY(bf16f32, __bf16, float)

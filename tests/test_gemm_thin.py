@@ -94,3 +94,35 @@ def test_more_than_32_rows_take_strips_while_they_fit_the_chip_once(fake_hip):
                           (128, 8192, 448, "thin64x64"), (128, 8256, 448, "128x128x64_d2x2")):
         ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k, generics=["f16", 128, 128, 1, k])
         assert ct.last_resolved()["variant"].startswith("f16_" + want), (m, n, k, ct.last_resolved()["variant"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,member", [(1, 12290, 4100, "thin16x128_nt"), (16, 8201, 6150, "thin16x64_nt"), (3, 24601, 2049, "thin16x128_nt")])
+def test_gpu_large_weights_past_the_caches(ct, dev, m, n, k, member, dtype):
+    """96 MiB of y and more: strips that read it past the caches, odd rows and ragged K included"""
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x = torch.randn(m, k, device=dev, generator=g).to(dtype)
+    y = (torch.randn(k, n, device=dev, generator=g) / k ** 0.5).to(dtype)
+    z = torch.full((m + 1, n), 7.0, dtype=dtype, device=dev)             # a row behind z that nothing may touch
+    want = (x.double() @ y.double()).cpu().numpy()
+    for _ in range(2):                                                    # the second launch finds the first one's counters at 0
+        ct.gemm(ct.partition(z[:m], [128, 128]), x, y, k, accumulate=False, generics=["f16" if dtype == torch.float16 else "bf16", 128, 128, 1])
+        torch.cuda.synchronize()
+        assert ct.last_resolved()["symbol"].endswith(member)
+        assert rel_l2(z[:m].double().cpu().numpy(), want) <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)
+        assert torch.all(z[m] == 7.0)
+
+
+def test_weights_that_may_be_cached_keep_plain_loads(fake_hip):
+    """below 96 MiB of y, and with more than 16 rows, the strips read through the caches"""
+    ct = fake_hip
+    buf = torch.empty(80 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+    for m, n, k, want in ((1, 4096, 4096, "thin16x64"), (1, 8192, 6143, "thin16x64"), (1, 8192, 6144, "thin16x64_nt"), (1, 14336, 4096, "thin16x128_nt"),
+                          (17, 4096, 14336, "thin32x64"), (33, 4096, 14336, "thin64x64")):
+        ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k)
+        got = ct.last_resolved()
+        assert got["symbol"] == "gemm_entry__f16_" + want and got["variant"] == "f16_" + want.replace("_nt", ""), (m, n, k, got)
+    ct.gemm(ct.partition(view(20, 8192), [128, 128]), view(20, 6144), view(6144, 8192), 6144, variant="f16_thin16x64")
+    assert ct.last_resolved()["symbol"] == "gemm_entry__f16_thin16x64"
