@@ -799,8 +799,8 @@ extern "C" __global__ void __launch_bounds__(kThreads)
 
 // logits[r] = sum_k f32(weights[r, k]) * f32(hidden[0, k]) for the 64 rows of block b, then the block's winner.
 // The weights are read once, 16 bytes per lane and nontemporally (a [vocab, K] matrix streams through once per
-// token); the hidden vector sits in LDS.  The launch holds two workgroups per compute unit, each taking a
-// contiguous run of blocks (a stream of this kind reads fastest from few resident wavefronts); a wavefront takes
+// token); the hidden vector sits in LDS.  A workgroup takes a contiguous run of blocks, as many as the launch gives it (a
+// stream of this kind reads fastest from few resident wavefronts); a wavefront takes
 // 16 of a block's 64 rows, two at a time, 1024 columns per step, and requests the next step's weights before it
 // multiplies the current ones.
 namespace {

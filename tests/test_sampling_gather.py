@@ -182,3 +182,30 @@ def test_gpu_embedding_and_gather_row(ct, dev):
     ct.gather_row_f16(td, ct.partition(wide, [1000]), 999)
     torch.cuda.synchronize()
     assert np.array_equal(wide.cpu().numpy().view(np.uint16), oracle.gather_row_f16(table, 999, 5000))
+
+
+def test_lm_head_workgroups(fake_hip):
+    """runs of blocks on two workgroups per compute unit while these come out even, else a workgroup to a block"""
+    ct = fake_hip
+    from test_host_abi import _workgroups
+    for blocks, want in ((1, 1), (512, 512), (513, 513), (602, 602), (853, 853), (854, 512), (1024, 512), (1025, 1025), (2004, 512)):
+        ct.lm_head_argmax_blocks_f16(torch.empty(blocks * 64, 32, dtype=torch.half), torch.empty(1, 32, dtype=torch.half),
+                                     ct.partition(torch.empty(blocks), [1]), ct.partition(torch.empty(blocks, dtype=torch.int32), [1]), blocks * 64)
+        assert _workgroups(ct) == want, blocks
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vocab,k", [(513 * 64, 64), (602 * 64 - 5, 96), (911 * 64, 32)])
+def test_gpu_lm_head_runs_and_single_blocks(ct, dev, vocab, k):
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    w, h = torch.randn(vocab, k, device=dev, generator=g).half(), torch.randn(1, k, device=dev, generator=g).half()
+    blocks = -(-vocab // 64)
+    top, idx = torch.zeros(blocks, device=dev), torch.zeros(blocks, dtype=torch.int32, device=dev)
+    ct.lm_head_argmax_blocks_f16(w, h, ct.partition(top, [1]), ct.partition(idx, [1]), vocab)
+    torch.cuda.synchronize()
+    logits = torch.full((blocks * 64,), -1e30, dtype=torch.float64, device=dev)
+    logits[:vocab] = (w.double() @ h.double().T).flatten()
+    want = logits.view(blocks, 64).max(1).values
+    # k products in f32 sums: sqrt(k) roundings of 2^-24 of sums of about sqrt(k)
+    assert torch.all((top.double() - want).abs() <= 2.0 ** -22 * k + 1e-6)
+    assert torch.all((logits[idx.long()] - want).abs() <= 2.0 ** -22 * k + 1e-6)
