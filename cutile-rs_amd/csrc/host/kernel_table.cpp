@@ -25,6 +25,7 @@ extern const unsigned char cutile_img_rng_start[], cutile_img_rng_end[];
 extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_end[];
 extern const unsigned char cutile_img_gemmf32_start[], cutile_img_gemmf32_end[];
 extern const unsigned char cutile_img_mxtiles_start[], cutile_img_mxtiles_end[];
+extern const unsigned char cutile_img_gemmgroup_start[], cutile_img_gemmgroup_end[];
 extern const unsigned char cutile_img_gemmtiles_start[], cutile_img_gemmtiles_end[];
 extern const unsigned char cutile_img_scaledflat_start[], cutile_img_scaledflat_end[];
 }
@@ -64,6 +65,7 @@ ImageRef image_ref(Image img) {
     case IMG_RNG: return {cutile_img_rng_start, cutile_img_rng_end};
     case IMG_GEMM_F32: return {cutile_img_gemmf32_start, cutile_img_gemmf32_end};
     case IMG_MX_TILES: return {cutile_img_mxtiles_start, cutile_img_mxtiles_end};
+    case IMG_GEMM_GROUP: return {cutile_img_gemmgroup_start, cutile_img_gemmgroup_end};
     case IMG_GEMM_TILES: return {cutile_img_gemmtiles_start, cutile_img_gemmtiles_end};
     case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
     case IMG_SCALED_FLAT: return {cutile_img_scaledflat_start, cutile_img_scaledflat_end};
@@ -330,6 +332,8 @@ std::vector<KernelEntry> build_table() {
     add("group_gemm_nt_desc", keep(gv), keep("group_gemm_nt_desc_entry__" + gv), IMG_GEMM, (uint32_t)(t[2] * t[3] * 64),
         (uint32_t)(((t[0] == 256 ? 2 : 3) * t[0] * 64 + 2 * 64 * t[1]) * 2), t[0], t[1], 64, 0, "f16", 0, 2);
   }
+  add("group_gemm_nt_desc", "f16_128x128x64_d2x2+ahead", "group_gemm_nt_desc_entry__f16_128x128x64_d2x2_ahead", IMG_GEMM_GROUP, 512,
+      4 * (128 * 64 + 64 * 128) * 2 + 256 * 64 + 48, 128, 128, 64, 0, "f16", 0, 2);
   for (const char* dt : {"bf16", "f16", "f32"})
     add("gemm_persistent", keep(std::string(dt) + "_generic"), keep(std::string("gemm_persistent_entry__") + dt + "_generic"),
         IMG_GEMM, 256, (uint32_t)((64 * 17 + 16 * 65) * 4), 0, 0, 0, 0, dt, 0, 2);

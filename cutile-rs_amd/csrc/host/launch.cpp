@@ -2521,6 +2521,7 @@ cutile_status_t cutile_launch_gemm_persistent(cutile_stream_t stream, const cuti
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 
+constexpr int kMostGroupsAhead = 256;   // groups whose descriptors the kernel of gemm_group.hip holds
 // group_gemm_f16_nt_desc (cutile-kernels/src/experimental/moe.rs:67-128): no partition argument, so the launch grid
 // (NUM_SM workgroups) comes from .grid() or the NUM_SM generic, and the tile shape from the BM / BN generics.
 cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, const cutile_tensor_arg_t* a_ptrs,
@@ -2559,7 +2560,7 @@ cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, con
   if (!grid[0]) grid[0] = (uint32_t)num_sm_generic;
   std::vector<std::string> acceptable;
   for (const KernelEntry* entry : kernels_of("group_gemm_nt_desc"))
-    if (const KernelEntry& e = *entry; e.tile[0] == bm && e.tile[1] == bn) acceptable.push_back(e.variant);
+    if (const KernelEntry& e = *entry; e.tile[0] == bm && e.tile[1] == bn && strchr(e.variant, '+') == nullptr) acceptable.push_back(e.variant);
   CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND,
                  "no precompiled variant of group_gemm_f16_nt_desc<BM=%d, BN=%d>; available: %s", bm, bn,
                  list_variants("group_gemm_nt_desc").c_str());
@@ -2568,10 +2569,27 @@ cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, con
   o.n_generics = 0;
   Resolved res;
   if (cutile_status_t s = resolve_entry("group_gemm_nt_desc", &o, acceptable[0], acceptable, &res)) return s;
+  bool ahead = false;
+  if (bm == 128 && bn == 128 && num_groups <= kMostGroupsAhead && !(opts && opts->variant)) {
+    int cus = 256;
+    if (g_launch_mode != 2)
+      if (cutile_status_t s = compute_units(res.device, &cus)) return s;
+    // It takes a compute unit's LDS for itself: of more workgroups than compute units some would only start when others end, where the
+    // ring's 80 KiB let two run side by side (512 workgroups, 32 groups of 32 x 4096 x 4096: 198 us on the ring; 256 here: 183).  A launch of
+    // no more than half of the compute units leaves room beside itself on purpose.
+    ahead = (int)grid[0] <= cus && 2 * (int)grid[0] > cus;
+  }
+  if (ahead)
+    if (cutile_status_t s = use_member(&res, "group_gemm_nt_desc", "f16_128x128x64_d2x2+ahead")) return s;
   ArgPacker args;
   for (int i = 0; i < 3; ++i) args.push_tensor(*ptrs[i]);
   for (int i = 0; i < 3; ++i) args.push_tensor(*metas[i]);
   args.push_val<int32_t>(num_groups);
+  if (ahead) {   // (it finds out itself whether it shares K: what the tables hold is not known here)
+    const SplitWorkspace ws = g_launch_mode == 0 ? split_workspace(res.device, (hipStream_t)stream) : SplitWorkspace{};
+    args.push_val<void*>(ws.partials);
+    args.push_val<void*>(ws.counters);
+  }
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 

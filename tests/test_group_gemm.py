@@ -63,6 +63,21 @@ def test_group_gemm_launcher_takes_its_grid_from_num_sm(fake_hip):
     assert _last(ct)[0].symbol == b"gemm_persistent_entry__f16_128x128x64_d2x2"
 
 
+def test_group_gemm_with_a_workgroup_to_each_compute_unit(fake_hip):
+    """128 x 128 tiles on 256 compute units: the kernel that fetches ahead, on more than half of them and with descriptors that fit its LDS"""
+    ct = fake_hip
+    from test_host_abi import _last
+    ptrs, metas = torch.zeros(300, dtype=torch.int64), torch.zeros(300, 8, dtype=torch.int32)
+    old = b"group_gemm_nt_desc_entry__f16_128x128x64_d2x2"
+    for groups, num_sm, variant, ahead in [(4, 256, None, True), (256, 129, None, True), (257, 256, None, False), (4, 128, None, False), (4, 257, None, False),
+                                           (4, 256, "f16_128x128x64_d2x2", False)]:
+        ct.group_gemm_f16_nt_desc(ptrs, ptrs, ptrs, metas, metas, metas, groups, generics=[128, 128, 64, num_sm], variant=variant)
+        rec, _ = _last(ct)
+        assert rec.symbol == (old + b"_ahead" if ahead else old) and tuple(rec.block) == ((512 if ahead else 256), 1, 1) and rec.grid[0] == num_sm
+    with pytest.raises(ct.CutileError, match="variant"):
+        ct.group_gemm_f16_nt_desc(ptrs, ptrs, ptrs, metas, metas, metas, 4, generics=[128, 128, 64, 256], variant="f16_128x128x64_d2x2+ahead")
+
+
 # ---- HIP kernels (GPU) --------------------------------------------------------------------------
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,tile,accumulate", [(512, 768, 1024, 256, False), (300, 264, 192, 256, True), (128, 128, 64, 128, False),
@@ -172,3 +187,39 @@ def test_gpu_group_gemm_without_inner_size(ct, dev, tile):
     ct.group_gemm_f16_nt_desc(ap, bp, cp, am, bm, cm, 2, generics=[tile, tile, 64, 8])
     torch.cuda.synchronize()
     assert not c_t[0].any() and torch.all(c_t[1] == 32.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes,num_sm", [
+    ([(3, 272, 512), (0, 128, 64), (40, 128, 1032), (16, 144, 1600)], 256),         # K shared, by groups of different inner sizes; a ragged last K tile
+    ([(70, 128, 8 * 64)], 256), ([(70, 128, 16 * 64)], 256), ([(128, 128, 17 * 64 + 16)], 131),     # around the least K that is shared
+    ([(129, 128, 2048), (16, 128, 0)], 256),                                        # two rows of tiles, beside a group without an inner size
+    ([(1 + i % 5, 16, 16 + 16 * (i % 9)) for i in range(255)] + [(130, 400, 336)], 256),   # as many groups as there may be; several tiles to a workgroup
+])
+def test_gpu_group_gemm_ahead(ct, dev, shapes, num_sm):
+    """the kernel with the chip to itself against 64 bits and, bit for bit where K is not shared, against the ring it stands in for; also from
+    inside a captured graph, where K is never shared"""
+    a_t, b_t, c_t, r_t, g_t, refs = [], [], [], [], [], []
+    for i, (m, n, k) in enumerate(shapes):
+        ab, bb = f16b(oracle.normal_f32((max(m, 1), max(k, 1)), 911 + i)), f16b(oracle.normal_f32((max(k, 1), n), 921 + i, 0, max(k, 1) ** -0.5))
+        a_t.append(_dev16(ab, dev)[:m, :k])
+        b_t.append(_dev16(bb, dev)[:k])
+        for t in (c_t, r_t, g_t):
+            t.append(torch.full((m + 1, n), 7.0, dtype=torch.half, device=dev))
+        refs.append(f16v(ab)[:m, :k].astype(np.float64) @ f16v(bb)[:k].astype(np.float64))
+    (ap, am), (bp, bm), (cp, cm), (rp, rm), (gp, gm) = [_tables(t, dev) for t in (a_t, b_t, *[[c[:-1] for c in t] for t in (c_t, r_t, g_t)])]
+    ct.group_gemm_f16_nt_desc(ap, bp, rp, am, bm, rm, len(shapes), generics=[128, 128, 64, num_sm], variant="f16_128x128x64_d2x2")
+    for _ in range(3):
+        ct.group_gemm_f16_nt_desc(ap, bp, cp, am, bm, cm, len(shapes), generics=[128, 128, 64, num_sm])
+    torch.cuda.synchronize()
+    launch = lambda stream: ct.group_gemm_f16_nt_desc(ap, bp, gp, am, bm, gm, len(shapes), generics=[128, 128, 64, num_sm], stream=stream)
+    graph = ct.CapturedGraph().capture(launch)
+    try:
+        for _ in range(2):
+            graph.launch()
+            graph.synchronize()
+    finally:
+        graph.close()
+    for c, r, g, ref in zip(c_t, r_t, g_t, refs):
+        assert torch.equal(g, r) and torch.all(c[-1] == 7.0)
+        assert not ref.any() and not c[:-1].any() or rel_l2(c[:-1].double().cpu().numpy(), ref) <= 2.0 ** -11      # one rounding to f16 over f32 sums
