@@ -74,6 +74,12 @@ def test_group_gemm_with_a_workgroup_to_each_compute_unit(fake_hip):
         ct.group_gemm_f16_nt_desc(ptrs, ptrs, ptrs, metas, metas, metas, groups, generics=[128, 128, 64, num_sm], variant=variant)
         rec, _ = _last(ct)
         assert rec.symbol == (old + b"_ahead" if ahead else old) and tuple(rec.block) == ((512 if ahead else 256), 1, 1) and rec.grid[0] == num_sm
+    ct.set_preferred_variant("group_gemm_nt_desc", old.decode().split("__")[1])
+    try:
+        ct.group_gemm_f16_nt_desc(ptrs, ptrs, ptrs, metas, metas, metas, 4, generics=[128, 128, 64, 256])
+        assert _last(ct)[0].symbol == old                                              # the pinned kernel stays
+    finally:
+        ct.set_preferred_variant("group_gemm_nt_desc", None)
     with pytest.raises(ct.CutileError, match="variant"):
         ct.group_gemm_f16_nt_desc(ptrs, ptrs, ptrs, metas, metas, metas, 4, generics=[128, 128, 64, 256], variant="f16_128x128x64_d2x2+ahead")
 
