@@ -40,6 +40,7 @@ IMAGES = {
     "gemmf32": "gemm_f32.hip",
     "mxtiles": "mxfp8_tiles.hip",
     "gemmgroup": "gemm_group.hip",
+    "fmhakeys": "fmha_keys.hip",
 }
 HOST_SOURCES = ["hip_api.cpp", "driver.cpp", "kernel_table.cpp", "launch.cpp", "runtime.cpp", "tuning.cpp", "workspace.cpp"]
 # The recording stand-in for the HIP runtime (include/cutile_hip_testing.h) is not part of the product library: the CPU

@@ -26,6 +26,7 @@ extern const unsigned char cutile_img_gemmsmall_start[], cutile_img_gemmsmall_en
 extern const unsigned char cutile_img_gemmf32_start[], cutile_img_gemmf32_end[];
 extern const unsigned char cutile_img_mxtiles_start[], cutile_img_mxtiles_end[];
 extern const unsigned char cutile_img_gemmgroup_start[], cutile_img_gemmgroup_end[];
+extern const unsigned char cutile_img_fmhakeys_start[], cutile_img_fmhakeys_end[];
 extern const unsigned char cutile_img_gemmtiles_start[], cutile_img_gemmtiles_end[];
 extern const unsigned char cutile_img_scaledflat_start[], cutile_img_scaledflat_end[];
 }
@@ -66,6 +67,7 @@ ImageRef image_ref(Image img) {
     case IMG_GEMM_F32: return {cutile_img_gemmf32_start, cutile_img_gemmf32_end};
     case IMG_MX_TILES: return {cutile_img_mxtiles_start, cutile_img_mxtiles_end};
     case IMG_GEMM_GROUP: return {cutile_img_gemmgroup_start, cutile_img_gemmgroup_end};
+    case IMG_FMHA_KEYS: return {cutile_img_fmhakeys_start, cutile_img_fmhakeys_end};
     case IMG_GEMM_TILES: return {cutile_img_gemmtiles_start, cutile_img_gemmtiles_end};
     case IMG_GEMM_SMALL: return {cutile_img_gemmsmall_start, cutile_img_gemmsmall_end};
     case IMG_SCALED_FLAT: return {cutile_img_scaledflat_start, cutile_img_scaledflat_end};
@@ -373,6 +375,16 @@ std::vector<KernelEntry> build_table() {
     add("fmha_seq", keep(v), keep("fmha_seq_entry__" + v), IMG_FMHA, (uint32_t)(t[0] / 32 * 64),
         (uint32_t)(2 * 2 * t[1] * t[2] * 2), t[0], t[1], t[2], 0, "f16", 0, 3);
   }
+  // wavefronts that share the keys of 32 or 64 query rows: for the launcher's own rule alone, whatever rows the caller's partition has
+  for (const char* function : {"fmha", "fmha_seq"})
+    for (const char* dt : {"bf16", "f16"})
+      for (int d : {64, 128})
+        for (int rows : {32, 64}) {
+          if (function[4] == '_' && dt[0] == 'b') continue;
+          std::string v = std::string(dt) + "_" + std::to_string(rows) + "x" + (rows == 32 ? "256x" : "128x") + std::to_string(d);
+          add(function, keep(v + "+keys"), keep(std::string(function) + "_entry__" + v + "_keys"), IMG_FMHA_KEYS, 512,
+              (uint32_t)(512 * d * 2 + 2 * 8 * 32 * 4), rows, rows == 32 ? 256 : 128, d, 0, dt, 0, 3);
+        }
 
   // ---- decode attention: one workgroup per (KV head, split); tile = (GROUP, 0, D) ----
   for (int d : {64, 128, 256})

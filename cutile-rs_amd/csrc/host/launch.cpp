@@ -2692,6 +2692,29 @@ cutile_status_t cutile_launch_mapped_shared_cache_update_f32(cutile_stream_t str
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 
+namespace {
+// Attention whose longest chain of keys decides its time, not its work (fmha_keys.hip): the query rows of a workgroup whose wavefronts share
+// the keys, or 0 for the kernels of 32 rows to a wavefront.
+// On 32 rows a workgroup has read its keys soonest, as long as one round holds the launch; behind that 64 rows, which read them half as
+// often.  D = 128 leaves room for one workgroup on a compute unit, D = 64 for two.  us on the kernels of 128 and 256 rows, on 64 and on 32:
+//   D = 128, causal: 4 heads of 2048 42, 30 and 26; 8 of 2048 (256 workgroups of 64 rows) 43, 31 and 34; 32 of 1024 (512) 26.2, 26.8 and 44
+//   D = 64: 8 heads of 1024 (256 workgroups of 32 rows) 21, 13 and 10.5; 16 of 1024 21, 13 and 15; 32 of 1024 (512 of 64 rows) 22, 18.5 and 27;
+//     512 of short keys lose: 128 heads of 256 8.9, 10 and 19; 1024 of 64 rows pay where causal tiles even out: 32 heads of 2048 causal 52, 41
+//     and 73, not causal 55, 60 and 110
+// Up to 128 keys there is nothing to share (one head of 64: 6.5, 8.0 and 8.3; of 129: 9.4, 8.2 and 8.3).
+int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, bool causal, int cus) {
+  if ((d != 64 && d != 128) || keys <= 128) return 0;
+  const int64_t of32 = heads * ((rows + 31) / 32), of64 = heads * ((rows + 63) / 64);
+  if (of32 <= cus) return 32;
+  if (of64 <= cus) return 64;
+  if (d == 64 && ((of64 <= 2 * cus && keys >= 512) || (of64 <= 4 * cus && causal && keys >= 1024))) return 64;
+  return 0;
+}
+std::string keys_member(const std::string& dtype, int rows, int d) {
+  return dtype + "_" + std::to_string(rows) + (rows == 32 ? "x256x" : "x128x") + std::to_string(d) + "+keys";
+}
+}  // namespace
+
 cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partition_arg_t* out, const cutile_tensor_arg_t* q,
                                    const cutile_tensor_arg_t* k, const cutile_tensor_arg_t* v, float qk_scale,
                                    int32_t input_pos, int32_t query_group_size, int32_t causal,
@@ -2737,7 +2760,7 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   const std::string dt = cutile_dtype_name(q->dtype);
   std::vector<std::string> acceptable, same_bn;
   for (const KernelEntry* entry : kernels_of("fmha"))
-    if (const KernelEntry& e = *entry; dt == e.dtype && e.tile[0] == bm && e.tile[2] == d) {
+    if (const KernelEntry& e = *entry; dt == e.dtype && e.tile[0] == bm && e.tile[2] == d && strchr(e.variant, '+') == nullptr) {
       acceptable.push_back(e.variant);
       if (e.tile[1] == bn_user) same_bn.push_back(e.variant);
     }
@@ -2746,7 +2769,18 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
                  list_variants("fmha").c_str());
   Resolved res;
   BucketScope bucket(dt + "_bm" + std::to_string(bm) + "_d" + std::to_string(d) + (causal ? "|causal" : "|full"));
-  if (cutile_status_t s = resolve_entry("fmha", opts, same_bn.empty() ? acceptable[0] : same_bn[0], acceptable, &res)) return s;
+  const std::string fallback = same_bn.empty() ? acceptable[0] : same_bn[0];
+  int key_rows = 0;   // (a caller that names the key tile means the kernel of that tile)
+  if (bm >= 128 && bn_user == 0 && (int64_t)tg[1] * bm >= ot.shape[1]) {
+    int cus = 256;
+    if (cutile_status_t s = current_device_units(&cus)) return s;
+    key_rows = key_sharing_rows(d, tg[0], ot.shape[1], causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2], causal, cus);
+  }
+  if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, key_rows ? fallback : std::string())) return s;
+  if (key_rows && g_last_source == "size") {
+    if (cutile_status_t s = use_member(&res, "fmha", keys_member(dt, key_rows, d))) return s;
+    tg[1] = div_up(ot.shape[1], key_rows);
+  }
   ArgPacker args;
   args.push_partition(*out);
   args.push_tensor(*q);
@@ -2836,7 +2870,7 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   const char* function = position_start ? "fmha_seq" : "fmha";
   std::vector<const KernelEntry*> fit;
   for (const KernelEntry* entry : kernels_of(function))
-    if (const KernelEntry& e = *entry; strcmp(e.dtype, "f16") == 0 && e.tile[2] == d) fit.push_back(&e);
+    if (const KernelEntry& e = *entry; strcmp(e.dtype, "f16") == 0 && e.tile[2] == d && strchr(e.variant, '+') == nullptr) fit.push_back(&e);
   CUTILE_REQUIRE(!fit.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "no precompiled sequence attention for f16, D = %d; available: %s", d,
                  list_variants(function).c_str());
   const bool long_prefill = rows_cov >= 256 && kv_len > 0;
@@ -2853,7 +2887,16 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   o.generics = nullptr;
   o.n_generics = 0;
   Resolved res;
-  if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res)) return s;
+  int key_rows = 0;   // (a caller that names the key tile, or packs the heads of a group into its tiles, means the kernels of that form)
+  if (pack == 1 && generic_int(opts, 1, 0) == 0 && (!position_start || rows_cov > 128)) {   // (with the position on the device, rows are all that is known of the length: 128 of them see more keys than that)
+    const int64_t seen = position_start ? max_seq : kv_len;
+    int cus = 256;
+    if (cutile_status_t s = current_device_units(&cus)) return s;
+    key_rows = key_sharing_rows(d, heads_cov, rows_cov, causal && !position_start ? std::min<int64_t>((int64_t)query_start + rows_cov, seen) : seen, causal, cus);
+  }
+  if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, key_rows ? acceptable[0] : std::string())) return s;
+  if (key_rows && g_last_source == "size")
+    if (cutile_status_t s = use_member(&res, function, keys_member("f16", key_rows, d))) return s;
   const int32_t kbm = res.entry->tile[0];
   ov.partition_shape[0] = 1; ov.partition_shape[1] = kbm; ov.partition_shape[2] = d;
   for (int i = 0; i < 3; ++i) ov.partition_strides[i] = ov.tensor.strides[i];
