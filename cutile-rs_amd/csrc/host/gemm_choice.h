@@ -145,7 +145,16 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
   // From 96 strips of 128 columns on where y is streamed past the caches (4096 x 14336, 112 strips and two workgroups to each: 22.1 us, 64-column strips 23.0).
   const bool many = s.n >= 192 * 128 || (s.m <= 16 && s.n >= 96 * 128 && streamed_past_caches(s.n, s.k));
   const int64_t strips = (s.n + 63) / 64;
-  if (s.y_cols >= 64 && (s.m <= 32 || (s.m <= 64 && strips <= cus) || (s.m <= 128 && 2 * strips <= cus))) {
+  // 128 x 128 tiles whose K is shared read y once for all the rows, in as many workgroups: from 49 rows on they are the better ones where K is
+  // long enough to be shared (f16, us on strips and on tiles: 112 x 3584 x 10496 43.6, 30; 64 x 2240 x 7680 28.7, 19; 97 x 576 x 3968 18.6, 13.6;
+  // below that line 53 x 3648 x 1984 13.0, 12.9; 120 x 4032 x 1280 10.7, 11.3), and where there is room for more than two workgroups to a
+  // tile or K is very long (58 x 13376 x 4096 29.7, 30.1; 56 x 14784 x 16256 104, 88).  Of up to 48 rows a strip multiplies three
+  // quarters of what it does of 64, and the two are near each other (47 x 3968 x 12096 30.2, 27.9; 39 x 8256 x 2816 18.2, 17.1; 35 x 15936 x
+  // 3328 23.8, 30.4), and one or two tiles of at most 64 rows stay on strips too.  Over 180 products beyond the line 0.70 of the strips' time.
+  const uint64_t wide = tiles_of(s.m, s.n, 128, 128);
+  const bool tiles_share = s.aligned && strcmp(s.dtype, "bf16f32") != 0 && partial_bytes > 0 && s.m > 48 && (s.m > 64 || wide > 2) && s.k >= 28 * 64 &&
+                           (wide * 8 <= (uint64_t)cus * 3 || s.k >= 96 * 64);
+  if (s.y_cols >= 64 && !tiles_share && (s.m <= 32 || (s.m <= 64 && strips <= cus) || (s.m <= 128 && 2 * strips <= cus))) {
     pick(s.m > 32 ? "thin64x64" : s.m > 16 ? "thin32x64" : many && s.y_cols >= 128 ? "thin16x128" : "thin16x64");
     return c;
   }

@@ -126,3 +126,42 @@ def test_weights_that_may_be_cached_keep_plain_loads(fake_hip):
         assert got["symbol"] == "gemm_entry__f16_" + want and got["variant"] == "f16_" + want.replace("_nt", ""), (m, n, k, got)
     ct.gemm(ct.partition(view(20, 8192), [128, 128]), view(20, 6144), view(6144, 8192), 6144, variant="f16_thin16x64")
     assert ct.last_resolved()["symbol"] == "gemm_entry__f16_thin16x64"
+
+
+def test_more_than_48_rows_of_a_long_k_share_it_on_tiles(fake_hip):
+    """128 x 128 tiles with K shared instead of 64-row strips: from the K on that is worth sharing, and only where there is room for partial sums"""
+    ct = fake_hip
+    from test_gemm_tiles import _new_stream
+    buf = torch.empty(40 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+
+    def takes(m, n, k, stream=None, dtype=torch.half):
+        ct.gemm(ct.partition(view(m, n).view(dtype), [128, 128]), view(m, k).view(dtype), view(k, n).view(dtype), k, stream=stream)
+        return ct.last_resolved()["variant"].split("_", 1)[1]
+
+    for m, n, k, strips in ((112, 3584, 10496, False), (49, 1408, 1792, False), (49, 1408, 1728, True), (128, 4096, 1728, True), (58, 12288, 2048, False),
+                            (58, 12416, 2048, True), (32, 512, 8192, True), (33, 1792, 2816, True), (48, 1920, 8192, True), (64, 256, 8192, True), (64, 257, 8192, True), (64, 264, 8192, False),
+                            (100, 1001, 8192, True)):
+        assert takes(m, n, k).startswith("thin") == strips, (m, n, k)
+    assert takes(112, 3584, 10496) == takes(112, 3584, 8192, dtype=torch.bfloat16) == "128x128x64_q2x2"
+    dev, stream = _new_stream(ct)
+    ct.check(ct.lib().cutile_testing_inject_failure(b"hipMallocAsync", 2, 1))
+    assert takes(112, 3584, 10496, stream.value) == "thin64x64"
+    ct.check(ct.lib().cutile_stream_release(dev, stream))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(49, 272, 1800), (64, 2248, 7680), (65, 576, 3976), (128, 3584, 4096), (100, 64, 6408)])
+def test_gpu_long_k_shared_on_tiles_of_few_rows(ct, dev, m, n, k, dtype):
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    x = torch.randn(m, k, device=dev, generator=g).to(dtype)
+    y = (torch.randn(k, n, device=dev, generator=g) / k ** 0.5).to(dtype)
+    z = torch.full((m + 1, n), 7.0, dtype=dtype, device=dev)             # a row behind z that nothing may touch
+    want = (x.double() @ y.double()).cpu().numpy()
+    for _ in range(2):
+        ct.gemm(ct.partition(z[:m], [128, 128]), x, y, k, accumulate=False, generics=["f16" if dtype == torch.float16 else "bf16", 128, 128, 1])
+        torch.cuda.synchronize()
+        assert "thin" not in ct.last_resolved()["variant"]
+        assert rel_l2(z[:m].double().cpu().numpy(), want) <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)   # one rounding over f32 sums
+        assert torch.all(z[m] == 7.0)
