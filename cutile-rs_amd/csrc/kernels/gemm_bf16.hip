@@ -1346,6 +1346,7 @@ extern "C" __global__ void __launch_bounds__(512)
 // Groups of few rows read their B once: what counts is how much of it is on its way.  A workgroup a compute unit with two
 // stages waits for one K tile after another (32 groups of 32 x 4096 x 4096: 263 us, 4.1 TB/s); the ring, with its fetches issued
 // between the products, takes 194 us (5.6 TB/s); 16 groups of 9 x 1024 x 4608 69 -> 48 us, 8 of 47 x 3328 x 512 22 -> 12 us.
+// (For launches of no more than half of the compute units, of more workgroups than those, or of more than 256 groups: gemm_group.hip otherwise.)
 extern "C" __global__ void __launch_bounds__(256)
     group_gemm_nt_desc_entry__f16_128x128x64_d2x2(TensorArg<1> a_ptrs, TensorArg<1> b_ptrs, TensorArg<1> c_ptrs, TensorArg<2> a_metas,
                                                   TensorArg<2> b_metas, TensorArg<2> c_metas, int32_t num_groups) {
