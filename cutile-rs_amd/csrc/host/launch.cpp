@@ -2237,14 +2237,18 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     }
     args.push_val<void*>(ws.partials);
     args.push_val<void*>(ws.counters);
-    if (is_thin(res.entry)) {
+    if (is_thin(res.entry) && !strip) {
       grid[2] = splits;
-    } else {
+    } else {   // tiles on the x axis alone, which holds more than 65535 of them
       args.push_val<uint32_t>(grid[1]);
       args.push_val<uint32_t>(grid[0]);
-      args.push_val<uint32_t>(splits);
-      CUTILE_REQUIRE(blocks * splits <= 0x7fffffffull, CUTILE_ERR_KERNEL_LAUNCH, "gemm: %llu output tiles do not fit a launch grid axis", (unsigned long long)blocks);
-      grid[0] = (uint32_t)(blocks * splits);
+      if (strip)
+        grid[2] = splits;
+      else
+        args.push_val<uint32_t>(splits);
+      const uint64_t along_x = strip ? blocks : blocks * splits;
+      CUTILE_REQUIRE(along_x <= 0x7fffffffull, CUTILE_ERR_KERNEL_LAUNCH, "gemm: %llu output tiles do not fit a launch grid axis", (unsigned long long)blocks);
+      grid[0] = (uint32_t)along_x;
       grid[1] = 1;
     }
     return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);

@@ -39,7 +39,7 @@ struct GemmF32 {
   }
 
   __device__ static void run(const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y, int32_t k_total, int32_t cover_m,
-                             int32_t cover_n, int32_t accumulate, float* partials, uint32_t* counters) {
+                             int32_t cover_n, int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n) {
     __shared__ __attribute__((aligned(16))) float red[WAVES][ROWS][PITCH];
     __shared__ uint32_t last;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -47,8 +47,7 @@ struct GemmF32 {
     const int32_t M = x.shape[0], N = y.shape[1];
     const int64_t lda = x.strides[0], ldb = y.strides[0];
     const int32_t k_valid = min(min(x.shape[1], y.shape[0]), k_total);
-    const uint32_t tiles_n = gridDim.x, tiles_m = gridDim.y;
-    const uint32_t tile = xcd_contiguous(blockIdx.y * tiles_n + blockIdx.x, tiles_m * tiles_n);
+    const uint32_t tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);   // (strips on the x axis alone: y holds 65535 of them)
     const uint32_t per_group = kGroupM * tiles_n, first_m = tile / per_group * kGroupM, group_rows = min(tiles_m - first_m, (uint32_t)kGroupM);
     const int32_t row0 = (int32_t)(first_m + tile % per_group % group_rows) * ROWS;
     const int32_t col_first = (int32_t)(tile % per_group / group_rows) * COLS;   // first column this workgroup stores
@@ -180,8 +179,8 @@ struct GemmF32 {
 #define GEMM_F32_KERNEL(NAME, MB)                                                                                                   \
   extern "C" __global__ void __launch_bounds__(512)                                                                                 \
       gemm_entry__f32_##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k_total, int32_t cover_m, int32_t cover_n,   \
-                             int32_t accumulate, float* partials, uint32_t* counters) {                                             \
-    GemmF32<MB>::run(z, x, y, k_total, cover_m, cover_n, accumulate, partials, counters);                                            \
+                             int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n) {         \
+    GemmF32<MB>::run(z, x, y, k_total, cover_m, cover_n, accumulate, partials, counters, tiles_m, tiles_n);                          \
   }
 GEMM_F32_KERNEL(strip16x64, 1)
 GEMM_F32_KERNEL(strip32x64, 2)

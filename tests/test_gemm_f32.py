@@ -48,3 +48,27 @@ def test_f32_calls_that_the_strips_do_not_take(fake_hip):
         assert ct.last_resolved()["variant"] == "f32_generic"
     ct.gemm(ct.partition(e(64, 128), [16, 16]), e(64, 64), e(64, 128), 64, generics=["f32", 16, 16, 8])
     assert ct.last_resolved()["variant"].startswith("f32_strip") and ct.last_resolved()["source"] == "size"
+
+
+def test_f32_products_of_many_rows_launch(fake_hip):
+    """more strips of rows than a grid's y axis counts (65535), by the rule and by name, on both sides of that line"""
+    ct = fake_hip
+    from test_host_abi import _last
+    x, y, z = torch.empty(4194241, 64), torch.empty(64, 64), torch.empty(4194241, 64)
+    for rows, variant, strips in ((4194240, None, 65535), (4194241, None, 65536), (1048560, "f32_strip16x64", 65535), (1048561, "f32_strip16x64", 65536)):
+        ct.gemm(ct.partition(z[:rows], [64, 64]), x[:rows], y, 64, generics=["f32", 64, 64, 64], variant=variant)
+        grid = _last(ct)[0].grid
+        assert ct.last_resolved()["variant"] == (variant or "f32_strip64x64") and grid[0] * grid[1] * grid[2] == strips
+
+
+@pytest.mark.gpu
+def test_gpu_f32_product_of_many_rows(ct, dev):
+    m = 4194305                                                         # 65537 strips of 64 rows
+    x = torch.arange(m, device=dev, dtype=torch.float32)[:, None] % 4093 + torch.arange(4, device=dev)
+    y, z = torch.ones(4, 64, device=dev), torch.zeros(m, 64, device=dev)
+    y[:, 1::2] = 2
+    ct.gemm(ct.partition(z, [64, 64]), x, y, 4, accumulate=False, generics=["f32", 64, 64, 4])
+    torch.cuda.synchronize()
+    assert ct.last_resolved()["variant"].startswith("f32_strip")
+    want = 4 * x[:, 0] + 6                                              # whole numbers below 2^24: exact
+    assert torch.equal(z[:, 0], want) and torch.equal(z[:, ::2], want[:, None].expand(-1, 32)) and torch.equal(z[:, 1::2], 2 * want[:, None].expand(-1, 32))
