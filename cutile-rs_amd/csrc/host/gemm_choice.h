@@ -19,7 +19,7 @@ struct GemmShape {
 
 struct GemmChoice {
   char variant[48] = "";   // "": the partition's own tile (tuning record, then the table's order)
-  bool shares_k = false;   // one of kRingTiles, with its K tiles shared
+  bool needs_room = false; // the choice counts on room for partial sums: without it the kernel is to be chosen again
 };
 
 // Output tiles of bm x bn of a launch.
@@ -127,7 +127,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
     double us = 1e30;
     for (const F32Strip& r : kF32Strips) {
       const F32Plan p = f32_plan(r, s.m, s.n, s.k, cus, partial_bytes);
-      if (s.y_cols >= 64 && p.us < us * 0.98) us = p.us, best = &r;
+      if (s.y_cols >= 64 && p.us < us * 0.98) us = p.us, best = &r, c.needs_room = p.splits > 1;
     }
     if (best) snprintf(c.variant, sizeof(c.variant), "f32_%s", best->kernel);
     return c;
@@ -171,7 +171,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       const RingPlan p = ring_plan(r, s.m, s.n, s.k, cus, partial_bytes);
       // (128 x 256 against 256 x 128, f16: 619 x 8832 x 4096 56.7 us, 59.0; 620 x 5000 x 4096 40.8, 39.6; 600 x 8192 x 4096 54.1, 55.8; equal for
       // bf16: the prices are good to 5 %, so only where it is the cheaper one by more)
-      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, pick(r.kernel), c.shares_k = p.splits > 1;
+      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, pick(r.kernel), c.needs_room = p.splits > 1;
     }
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
@@ -199,7 +199,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       const Cost& c1 = ring ? r.aligned : r.any;
       const double us = kt / (double)sk * std::max(c1.one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
                         (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      if (us < best * 0.98) best = us, pick(r.kernel), c.shares_k = false;
+      if (us < best * 0.98) best = us, pick(r.kernel), c.needs_room = false;
     }
   }
   return c;

@@ -2147,11 +2147,13 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     if (cutile_status_t s = current_device_units(&cus)) return s;
     const GemmShape shape{dt.c_str(), cover_m, cover_n, y->shape[1], k_valid, fast_layout && full_cover, own_tile != nullptr};
     sized = choose_gemm(shape, cus, partial_bytes);
-    if (sized.shares_k && g_launch_mode != 2) {
+    if (sized.needs_room && g_launch_mode != 2) {
       cutile_device_t device = nullptr;
       if (cutile_status_t s = current_device(&device)) return s;
       // a captured launch has no workspace and takes the best kernel of those that need none: their code objects are loaded here
-      if (cutile_status_t s = load_gemm_images(device)) return s;
+      // (f32: one code object holds them all)
+      if (!in_f32)
+        if (cutile_status_t s = load_gemm_images(device)) return s;
       if (g_launch_mode == 0) ws = split_workspace(device, (hipStream_t)stream);
       if (g_launch_mode == 0 && !ws.partials) sized = choose_gemm(shape, cus, partial_bytes = 0);
     }
@@ -2229,9 +2231,10 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
     const F32Strip* strip = in_f32 ? f32_strip(res.entry->tile[3]) : nullptr;
-    splits = strip ? f32_plan(*strip, cover_m, cover_n, k_valid, cus, kSplitPartialBytes).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
+    splits = strip ? f32_plan(*strip, cover_m, cover_n, k_valid, cus, partial_bytes).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
-    if (splits > 1 && g_launch_mode == 0) {
+    if (partial_bytes == 0) splits = 1;
+    if (splits > 1 && g_launch_mode == 0 && !ws.partials) {
       ws = split_workspace(res.device, (hipStream_t)stream);
       if (!ws.partials) splits = 1;
     }

@@ -50,6 +50,55 @@ def test_f32_calls_that_the_strips_do_not_take(fake_hip):
     assert ct.last_resolved()["variant"].startswith("f32_strip") and ct.last_resolved()["source"] == "size"
 
 
+def _products_that_share_k(ct):
+    f = lambda m, n, k, s=None, v=None: ct.gemm(ct.partition(torch.empty(m, n), [64, 64]), torch.empty(m, k), torch.empty(k, n), k, stream=s, variant=v,
+                                                generics=["f32", 64, 64, 64])
+    # (m, n, k): strip and workgroups with room for partial sums, and without
+    return f, [((64, 4096, 4096), "64x64", "16x64", 256), ((64, 2048, 8192), "32x64", "16x64", 128), ((128, 1024, 8192), "32x64", "16x64", 128),
+               ((200, 512, 8192), "32x64", "16x64", 104)]
+
+
+def test_f32_strips_without_a_workspace_are_chosen_again(fake_hip):
+    """a strip that is the best one only with its K shared gives way to the best of those that share nothing"""
+    ct = fake_hip
+    from test_host_abi import _new_stream, _workgroups
+    launch, cases = _products_that_share_k(ct)
+    for shape, shared, alone, blocks in cases:
+        launch(*shape)
+        assert ct.last_resolved()["variant"] == "f32_strip" + shared and _workgroups(ct) > -(-shape[0] // int(shared[:2])) * shape[1] // 64
+        dev, stream = _new_stream(ct)
+        ct.check(ct.lib().cutile_testing_inject_failure(b"hipMallocAsync", 2, 1))
+        for _ in range(257):                                            # refused, and not asked for again in the next 256 launches
+            launch(*shape, stream.value)
+            assert ct.last_resolved()["variant"] == "f32_strip" + alone and _workgroups(ct) == blocks
+        launch(*shape, stream.value)
+        assert ct.last_resolved()["variant"] == "f32_strip" + shared
+        ct.check(ct.lib().cutile_stream_release(dev, stream))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(64, 1024, 4096), (130, 520, 4099)])
+def test_gpu_captured_f32_product_that_would_share_k(ct, dev, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, y, z = torch.randn(m, k, device=dev, generator=g), torch.randn(k, n, device=dev, generator=g), torch.zeros(m, n, device=dev)
+    launch = lambda stream=None: ct.gemm(ct.partition(z, [64, 64]), x, y, k, accumulate=False, stream=stream, generics=["f32", 64, 64, 1])
+    launch()
+    torch.cuda.synchronize()
+    want = (x.double() @ y.double()).cpu().numpy()
+    graph = ct.CapturedGraph().capture(launch)
+    assert ct.last_resolved()["variant"] == "f32_strip16x64"
+    try:
+        for _ in range(3):
+            for run in (lambda: (graph.launch(), graph.synchronize()), launch):
+                z.zero_()
+                torch.cuda.synchronize()
+                run()
+                torch.cuda.synchronize()
+                assert rel_l2(z.double().cpu().numpy(), want) <= 2.0 ** -24 * (2 + np.sqrt(k))      # (as above)
+    finally:
+        graph.close()
+
+
 def test_f32_products_of_many_rows_launch(fake_hip):
     """more strips of rows than a grid's y axis counts (65535), by the rule and by name, on both sides of that line"""
     ct = fake_hip
