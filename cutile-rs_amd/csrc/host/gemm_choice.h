@@ -161,6 +161,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
   auto tiles = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   const double kt = s.k / 64.0;
   double best = 1e30;
+  bool shares_k = false;   // the kernel picked
   // (up to K = 512 the start and the output of a tile are most of a launch: the partition's own tile, if it has kernels)
   const bool ring = s.aligned && (s.k > 512 || !s.own_tile) && strcmp(s.dtype, "bf16f32") != 0;
   if (ring)
@@ -171,7 +172,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       const RingPlan p = ring_plan(r, s.m, s.n, s.k, cus, partial_bytes);
       // (128 x 256 against 256 x 128, f16: 619 x 8832 x 4096 56.7 us, 59.0; 620 x 5000 x 4096 40.8, 39.6; 600 x 8192 x 4096 54.1, 55.8; equal for
       // bf16: the prices are good to 5 %, so only where it is the cheaper one by more)
-      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, pick(r.kernel), c.needs_room = p.splits > 1;
+      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, pick(r.kernel), shares_k = p.splits > 1;
     }
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
@@ -193,15 +194,16 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
                                          {"staged64x64", 64, 64, 4, {0.52, 0.235, 5.0, 6.0, 1.6e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
     for (const StagedTile& r : kStaged) {
       if (s.y_cols < r.bn) continue;
-      const uint64_t t = tiles(r.bm, r.bn), sk = staged_splits(r.bm, r.bn, t, s.k, cus);
+      const uint64_t t = tiles(r.bm, r.bn), sk = partial_bytes ? staged_splits(r.bm, r.bn, t, s.k, cus) : 1;
       const double w = (double)((t * sk + cus - 1) / cus);
       if (r.per_cu == 1 && w > 2) continue;
       const Cost& c1 = ring ? r.aligned : r.any;
       const double us = kt / (double)sk * std::max(c1.one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
                         (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      if (us < best * 0.98) best = us, pick(r.kernel), c.needs_room = false;
+      if (us < best * 0.98) best = us, pick(r.kernel), shares_k = sk > 1;
     }
   }
+  c.needs_room = shares_k || tiles_share;   // (strips that were passed over share K inside a workgroup, and need none)
   return c;
 }
 

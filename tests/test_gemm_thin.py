@@ -165,3 +165,52 @@ def test_gpu_long_k_shared_on_tiles_of_few_rows(ct, dev, m, n, k, dtype):
         assert "thin" not in ct.last_resolved()["variant"]
         assert rel_l2(z[:m].double().cpu().numpy(), want) <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)   # one rounding over f32 sums
         assert torch.all(z[m] == 7.0)
+
+
+def test_products_without_a_workspace_are_chosen_again(fake_hip):
+    """49 to 128 rows whose best kernel shares K, be it tiles or the 64 x 64 staged ones: strips, whose wavefronts share K by themselves, where there is no
+    room for partial sums, and the best unshared staged tile beyond 128 rows and for unaligned rows"""
+    ct = fake_hip
+    from test_gemm_tiles import _new_stream, _workgroups
+    buf = torch.empty(40 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+
+    def launch(m, n, k, stream=None):
+        ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k, stream=stream)
+        return ct.last_resolved()["variant"].split("_", 1)[1], _workgroups(ct)
+
+    for shape, shared, alone in (((65, 576, 3976), ("staged64x64", 126), ("thin64x64", 18)), ((100, 64, 6408), ("staged64x64", 16), ("thin64x64", 2)),
+                                 ((128, 1920, 2560), ("staged64x64", 300), ("thin64x64", 60)), ((49, 1408, 1792), ("staged64x64", 66), ("thin64x64", 22)),
+                                 ((112, 3584, 10496), ("128x128x64_q2x2", 168), ("thin64x64", 112)), ((200, 515, 4099), ("staged64x64", 288), ("staged64x64", 36))):
+        assert launch(*shape) == shared, (shape, launch(*shape))
+        dev, stream = _new_stream(ct)
+        ct.check(ct.lib().cutile_testing_inject_failure(b"hipMallocAsync", 2, 1))
+        for _ in range(257):                                             # refused, and not asked for again in the next 256 launches
+            assert launch(*shape, stream.value) == alone, shape
+        assert launch(*shape, stream.value) == shared
+        ct.check(ct.lib().cutile_stream_release(dev, stream))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(65, 576, 3976), (128, 1920, 2560), (200, 515, 4099)])
+def test_gpu_captured_product_of_staged_tiles_that_would_share_k(ct, dev, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, y = torch.randn(m, k, device=dev, generator=g).half(), (torch.randn(k, n, device=dev, generator=g) / k ** 0.5).half()
+    z = torch.zeros(m, n, dtype=torch.half, device=dev)
+    launch = lambda stream=None: ct.gemm(ct.partition(z, [128, 128]), x, y, k, accumulate=False, stream=stream, generics=["f16", 128, 128, 1])
+    launch()
+    torch.cuda.synchronize()
+    assert ct.last_resolved()["variant"] == "f16_staged64x64"
+    want = (x.double() @ y.double()).cpu().numpy()
+    graph = ct.CapturedGraph().capture(launch)
+    assert ct.last_resolved()["variant"] == ("f16_thin64x64" if m <= 128 else "f16_staged64x64")
+    try:
+        for _ in range(3):
+            for run in (lambda: (graph.launch(), graph.synchronize()), launch):
+                z.zero_()
+                torch.cuda.synchronize()
+                run()
+                torch.cuda.synchronize()
+                assert rel_l2(z.double().cpu().numpy(), want) <= 2.0 ** -11        # one rounding over f32 sums
+    finally:
+        graph.close()
