@@ -1520,14 +1520,21 @@ cutile_status_t cutile_launch_lm_head_argmax_blocks_f16(cutile_stream_t stream, 
   args.push_tile_grid(tg);
   // Two workgroups per compute unit, each walking a contiguous run of blocks, read fastest (2004 blocks of K = 4096: 156.8 us, one workgroup to
   // a block 164.0; 1448 of 2048: 59.8, 63.1), unless the longest run is more than a fifth above the mean one (1320 of 4096, a sixth
-  // above: 115.2, 122.6; 1692 of 2048, more: 82.9, 77.8): then a workgroup to a block, which the dispatcher evens out (602 blocks of 4096: 67.6 us on 512 runs, 57.3; 1155 of 2560: 75.4, 63.2; 1169 of 1024: 37.5, 27.8).
+  // above: 109.8, 115.3): then a workgroup to a block, which the dispatcher evens out (602 blocks of 4096: 68.0 us on 512 runs, 57.9; 1155 of
+  // 2560: 76.3, 63.4; 1169 of 1024: 37.5, 27.8; 1692 of 4096: 146.7, 137.7), where that leaves the busiest compute unit fewer blocks.  Between three and
+  // three and a third blocks to a compute unit it has four either way, and single ones lose (820 blocks of 4096: 70.9, 78.1; of 2048: 38.5, 42.0; of
+  // 8192: 136.9, 153.4; of 5120: 90.3, 92.5), but for short rows whose last step of 1024 columns is at most three quarters full, or the
+  // only one: runs pay for whole steps (820 of 512: 22.4, 15.6; of 1024: 27.0, 21.6; 1792: 36.8, 36.2; 2304: 52.1, 45.1; 2816: 56.9, 53.7; 3328:
+  // 62.1, 62.6).  Nothing to even out where a compute unit holds no third workgroup (the hidden vector in LDS; 700 of 30720: 475, 481).
   cutile_device_t device = nullptr;
   if (cutile_status_t s = current_device(&device)) return s;
   int cus = 0;
   if (cutile_status_t s = compute_units(device, &cus)) return s;
   const uint32_t runs = (uint32_t)std::max(cus, 1) * 2u;
-  const bool even = tg[0] <= runs || (uint64_t)div_up(tg[0], runs) * runs * 5 <= (uint64_t)tg[0] * 6;
-  uint32_t grid[3] = {even ? std::min(tg[0], runs) : tg[0], 1, 1};
+  const uint32_t longest = div_up(tg[0], runs);
+  const bool uneven = tg[0] > runs && (uint64_t)longest * runs * 5 > (uint64_t)tg[0] * 6 && 3 * (2 * k + 512) <= 160 * 1024;
+  const bool fewer = div_up(tg[0], runs / 2) < 2 * longest, short_rows = k <= 1024 || (k < 3072 && k % 1024 != 0 && k % 1024 <= 768);
+  uint32_t grid[3] = {uneven && (fewer || short_rows) ? tg[0] : std::min(tg[0], runs), 1, 1};
   return launch_packed(res.fn, grid, res.entry->block, (uint32_t)k * 2, stream, args);
 }
 

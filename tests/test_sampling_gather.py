@@ -209,3 +209,14 @@ def test_gpu_lm_head_runs_and_single_blocks(ct, dev, vocab, k):
     # k products in f32 sums: sqrt(k) roundings of 2^-24 of sums of about sqrt(k)
     assert torch.all((top.double() - want).abs() <= 2.0 ** -22 * k + 1e-6)
     assert torch.all((logits[idx.long()] - want).abs() <= 2.0 ** -22 * k + 1e-6)
+
+
+@pytest.mark.parametrize("blocks,k,runs", [(768, 4096, False), (769, 4096, True), (853, 4096, True), (853, 8192, True), (820, 2048, True), (820, 3072, True), (820, 5120, True), (820, 1024, False),
+                                           (820, 1792, False), (820, 1824, True), (820, 2560, False), (820, 2848, True), (1025, 8192, False), (1279, 4096, False), (1692, 2048, False), (854, 1024, True)])
+def test_lm_head_runs_of_two_blocks_where_single_ones_fill_no_better(fake_hip, blocks, k, runs):
+    """between 769 and 853 blocks the busiest of 256 compute units has four blocks in runs and as single ones: single ones for short rows alone"""
+    ct = fake_hip
+    from test_host_abi import _workgroups
+    ct.lm_head_argmax_blocks_f16(torch.empty(1, 1, dtype=torch.half).expand(blocks * 64, k), torch.empty(1, k, dtype=torch.half),
+                                 ct.partition(torch.empty(blocks), [1]), ct.partition(torch.empty(blocks, dtype=torch.int32), [1]), blocks * 64)
+    assert _workgroups(ct) == (512 if runs else blocks)
