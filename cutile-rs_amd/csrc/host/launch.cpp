@@ -3194,7 +3194,7 @@ cutile_status_t cutile_last_resolved_kernel(const char** function, cutile_kernel
   info->variant = g_last_entry->variant;
   memcpy(info->block, g_last_member->block, sizeof(info->block));
   info->lds_bytes = g_last_member->lds_bytes;
-  memcpy(info->tile, g_last_entry->tile, sizeof(info->tile));
+  memcpy(info->tile, g_last_member->tile, sizeof(info->tile));
   return CUTILE_SUCCESS;
 }
 }  // extern "C"

@@ -232,7 +232,7 @@ cutile_status_t cutile_kernel_set_preferred_variant(const char* function, const 
  * cutile_last_resolved_bucket reports after a launch, e.g. "bf16_256x256|tiles>256" for gemm).  This is how the winners of
  * verified tuning records reach the launchers; order of precedence at a launch: the caller's variant, the function-wide
  * pin, the bucket's winner set by this call (explicit run-time choices beat rules and files), the launcher's own rule on
- * extents (gemm and linear_tile*: finer than their buckets), the bucket's winner in a tuning record, the table's order. */
+ * extents (gemm, linear_tile*, fmha and fmha_seq: finer than their buckets), the bucket's winner in a tuning record, the table's order. */
 cutile_status_t cutile_kernel_set_preferred_variant_for(const char* function, const char* bucket, const char* variant);
 /* Tuning records (cutile/src/tune.rs:762-1016): JSON records of autotuner winners, one file per kernel, in the directory
  * `tuned` beside the library (or $CUTILE_TUNING_RECORDS; empty = none), loaded on the first launcher call.  A record is
@@ -331,7 +331,8 @@ typedef struct {
 cutile_status_t cutile_set_launch_mode(int32_t mode);
 cutile_status_t cutile_get_launch_mode(int32_t* mode);
 /* The kernel the calling thread's last launcher call resolved: its table name and the same record cutile_kernel_lookup
- * fills (`function` is NULL after a specialize-only call: nothing was loaded). */
+ * fills (`function` is NULL after a specialize-only call: nothing was loaded).  `variant` is the name that a caller, a pin or a
+ * record can give; where the launcher took a member of that family, the rest of the record describes the member. */
 cutile_status_t cutile_last_resolved_kernel(const char** function, cutile_kernel_info_t* info);
 
 /* Partition::grid — cutile/src/tensor.rs:447-468 */

@@ -40,6 +40,19 @@ def test_short_attention_shares_keys(fake_hip, heads, rows, d, causal, takes):
             ct.set_preferred_variant("fmha", None)
 
 
+def test_a_member_is_described_as_the_kernel_that_it_is(fake_hip):
+    """cutile_last_resolved_kernel: symbol, block, LDS and tile of the kernel that was launched, the variant's name that of its family"""
+    import ctypes as C
+    ct = fake_hip
+    from test_host_abi import _last
+    for rows, d, tile, lds in ((300, 128, (32, 256, 128, 0), 512 * 128 * 2 + 2048), (1500, 64, (64, 128, 64, 0), 512 * 64 * 2 + 2048)):
+        _call(ct, torch.half, 1, 4 if d == 128 else 16, 1, rows, rows, d, True)
+        function, info = C.c_char_p(), ct.KernelInfo()
+        ct.check(ct.lib().cutile_last_resolved_kernel(C.byref(function), C.byref(info)))
+        assert info.variant == f"f16_128x64x{d}".encode() and info.symbol == _last(ct)[0].symbol and tuple(info.block) == (512, 1, 1)
+        assert tuple(info.tile) == tile and info.lds_bytes == lds
+
+
 # ---- HIP kernels (GPU) --------------------------------------------------------------------------
 def _reference(q, k, v, scale, pos, group, causal):
     q, k, v = (t.double().cpu() for t in (q, k, v))
