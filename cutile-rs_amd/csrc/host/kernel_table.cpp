@@ -639,7 +639,7 @@ cutile_status_t cutile_kernel_fingerprint(const char* function, const char* vari
   CUTILE_REQUIRE(function && out, CUTILE_ERR_INVALID_ARGUMENT, "null argument");
   const KernelEntry* entry = nullptr;
   for (const auto& e : kernel_table())
-    if (strcmp(e.function, function) == 0 && (!variant || strcmp(e.variant, variant) == 0)) { entry = &e; break; }
+    if (strcmp(e.function, function) == 0 && (!variant || strcmp(e.variant, variant) == 0 || strcmp(e.symbol, variant) == 0)) { entry = &e; break; }
   CUTILE_REQUIRE(entry, CUTILE_ERR_KERNEL_NOT_FOUND, "no kernel '%s'%s%s; available: %s", function, variant ? " variant " : "",
                  variant ? variant : "", list_variants(function).c_str());
   uint64_t h = 0xcbf29ce484222325ull;   // FNV-1a

@@ -477,7 +477,7 @@ class KernelLauncher : public DeviceOp<KernelLauncher<Fn, ArgOps...>, std::tuple
       size_t index = 0;
       std::apply([&](auto&... a) { (detail::describe_arg(a, index++, max_div, &strides, &specs, &scalars), ...); }, vals);
       char fp[17] = {0};
-      CUTILE_TRY_STATUS(cutile_kernel_fingerprint(fn_name, info.variant, fp));
+      CUTILE_TRY_STATUS(cutile_kernel_fingerprint(fn_name, info.symbol, fp));   // (of a family's member: the code object that it lies in)
       char arch[256] = {0};
       cutile_device_t dev = nullptr;
       CUTILE_TRY_STATUS(cutile_device_get(ctx.device_id(), &dev));

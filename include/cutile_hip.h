@@ -251,7 +251,7 @@ const char* cutile_last_resolved_bucket(void);
  * source_hash, toolchain fingerprint, arch and crate version; here they come from the kernel table):
  * the library version, the device compiler's version text captured at build time, the one target
  * architecture, and a 16-hex-digit fingerprint of the code object that holds `function` (variant == NULL)
- * or of that code object plus one variant's symbol. */
+ * or of that code object plus one variant's symbol (`variant` = its name, or that symbol itself). */
 const char* cutile_library_version(void);
 const char* cutile_toolchain_fingerprint(void);
 const char* cutile_target_arch(void);

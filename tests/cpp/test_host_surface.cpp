@@ -308,6 +308,19 @@ TEST(tile_function_key_distinguishes_everything_that_selects_a_kernel) {
   CHECK(default_key().grid(4, 1, 1).build() != default_key().build() && default_key().grid(4, 1, 1).build() != default_key().grid(8, 1, 1).build());
 }
 
+TEST(cache_keys_name_the_code_object_that_runs) {
+  // a short attention runs on a member of its family that lies in a code object of its own: its fingerprint, not the family's
+  auto s = fresh_stream();
+  auto in = [] { return api::zeros<bf16>({1, 4, 300, 128}); };
+  auto spec = fmha(partition_op(api::zeros<bf16>({4, 300, 128}), {1, 128, 128}), in(), in(), in(), 0.1f, 0, 1).specialize_on(s).unwrap();
+  CHECK(spec.variant() == "bf16_128x64x128" && spec.symbol() == "fmha_entry__bf16_32x256x128_keys");
+  char family[17], member[17], by_symbol[17];
+  CHECK(cutile_kernel_fingerprint("fmha", "bf16_128x64x128", family) == CUTILE_SUCCESS && cutile_kernel_fingerprint("fmha", "bf16_32x256x128+keys", member) == CUTILE_SUCCESS);
+  CHECK(spec.l1_cache_key().source_hash() == member && strcmp(family, member) != 0);
+  CHECK(cutile_kernel_fingerprint("fmha", "fmha_entry__bf16_128x64x128", by_symbol) == CUTILE_SUCCESS && strcmp(family, by_symbol) == 0);
+  CHECK(cutile_kernel_fingerprint("gemm", "fmha_entry__bf16_128x64x128", by_symbol) == CUTILE_ERR_KERNEL_NOT_FOUND);
+}
+
 TEST(launcher_compile_specialize_and_cache_keys) {
   // .compile() / .compile_on() / .specialize() / .l1_cache_key() / .l2_cache_key() / .const_grid() / .compile_options() / _apply
   // (cutile-macro/src/_module.rs:852-923, kernel_launcher_generator.rs:1036-1044)
