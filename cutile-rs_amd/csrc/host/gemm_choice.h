@@ -17,11 +17,6 @@ struct GemmShape {
   bool own_tile;           // the partition's tile has kernels of its own
 };
 
-struct GemmChoice {
-  char variant[48] = "";   // "": the partition's own tile (tuning record, then the table's order)
-  bool needs_room = false; // the choice counts on room for partial sums: without it the kernel is to be chosen again
-};
-
 // Output tiles of bm x bn of a launch.
 inline uint64_t tiles_of(int64_t m, int64_t n, int bm, int bn) { return (uint64_t)((m + bm - 1) / bm) * (uint64_t)((n + bn - 1) / bn); }
 
@@ -120,16 +115,25 @@ inline F32Plan f32_plan(const F32Strip& r, int64_t m, int64_t n, int32_t k, int 
   return best;
 }
 
+struct GemmChoice {
+  char variant[48] = "";   // "": the partition's own tile (tuning record, then the table's order)
+  bool needs_room = false; // the choice counts on room for partial sums: without it the kernel is to be chosen again
+  const RingTile* ring = nullptr;    // the kernel chosen, if it is one of these, and its plan
+  RingPlan ring_plan{};
+  const F32Strip* strip = nullptr;
+  F32Plan strip_plan{};
+};
+
 inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_bytes) {
   GemmChoice c;
   if (strcmp(s.dtype, "f32") == 0) {
-    const F32Strip* best = nullptr;
     double us = 1e30;
     for (const F32Strip& r : kF32Strips) {
       const F32Plan p = f32_plan(r, s.m, s.n, s.k, cus, partial_bytes);
-      if (s.y_cols >= 64 && p.us < us * 0.98) us = p.us, best = &r, c.needs_room = p.splits > 1;
+      if (s.y_cols >= 64 && p.us < us * 0.98) us = p.us, c.strip = &r, c.strip_plan = p;
     }
-    if (best) snprintf(c.variant, sizeof(c.variant), "f32_%s", best->kernel);
+    if (c.strip) snprintf(c.variant, sizeof(c.variant), "f32_%s", c.strip->kernel);
+    c.needs_room = c.strip && c.strip_plan.splits > 1;
     return c;
   }
   if (s.k <= 64) return c;   // one K tile: nothing to stage, split or overlap
@@ -161,6 +165,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
   auto tiles = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   const double kt = s.k / 64.0;
   double best = 1e30;
+  const char* picked = nullptr;
   bool shares_k = false;   // the kernel picked
   // (up to K = 512 the start and the output of a tile are most of a launch: the partition's own tile, if it has kernels)
   const bool ring = s.aligned && (s.k > 512 || !s.own_tile) && strcmp(s.dtype, "bf16f32") != 0;
@@ -169,10 +174,10 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       // a handful of tiles of a short K: 64 x 64 staged ones, priced below (us there and on 128 x 128: 263 x 64 x 1728 9.4, 10.8; 141 x
       // 320 x 2496 11.3, 12.3; beyond, 250 x 384 x 4352 16.3, 14.4)
       if (s.k <= 2560 && tiles_of(s.m, s.n, 128, 128) < 16) break;
-      const RingPlan p = ring_plan(r, s.m, s.n, s.k, cus, partial_bytes);
+      const RingPlan p = cutile::ring_plan(r, s.m, s.n, s.k, cus, partial_bytes);
       // (128 x 256 against 256 x 128, f16: 619 x 8832 x 4096 56.7 us, 59.0; 620 x 5000 x 4096 40.8, 39.6; 600 x 8192 x 4096 54.1, 55.8; equal for
       // bf16: the prices are good to 5 %, so only where it is the cheaper one by more)
-      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, pick(r.kernel), shares_k = p.splits > 1;
+      if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, picked = r.kernel, shares_k = p.splits > 1, c.ring = &r, c.ring_plan = p;
     }
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
@@ -200,9 +205,10 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       const Cost& c1 = ring ? r.aligned : r.any;
       const double us = kt / (double)sk * std::max(c1.one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
                         (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      if (us < best * 0.98) best = us, pick(r.kernel), shares_k = sk > 1;
+      if (us < best * 0.98) best = us, picked = r.kernel, shares_k = sk > 1, c.ring = nullptr;
     }
   }
+  if (picked) pick(picked);
   c.needs_room = shares_k || tiles_share;   // (strips that were passed over share K inside a workgroup, and need none)
   return c;
 }
@@ -243,7 +249,8 @@ inline MxPlan mx_plan(int64_t m, int64_t n, int32_t pieces, int cus, uint64_t pa
 // The kernel by name, or nullptr: the partition's own (tuning record, then the table's order).  us per 64-byte piece of K for
 // one block on each compute unit, measured at K = 4096 (mxfp8: 16 x 4096 9.4 us, 64 x 4096 13.4, 512 x 4096 21 on 64 x 128 blocks, 24 with
 // 128 x 128 tiles; nvfp4: 9.9, 14.7, 24).  The 256 x 256 kernels are the better ones where their tiles come near to filling the chip.
-inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus, uint64_t partial_bytes) {
+// `lone`: what mx_plan says for fp8, where it was asked.
+inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus, uint64_t partial_bytes, MxPlan* lone) {
   if (s.pieces <= 4) return nullptr;   // two steps: nothing to share out
   auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   if (s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
@@ -259,8 +266,8 @@ inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int
     if (us < best) best = us, name = k.name;
   }
   if (!s.fp4) {
-    const MxPlan lone = mx_plan(s.m, s.n, s.pieces, cus, partial_bytes);
-    if (lone.splits && lone.us < best) best = lone.us, name = "128x128x128_e2x2";
+    *lone = mx_plan(s.m, s.n, s.pieces, cus, partial_bytes);
+    if (lone->splits && lone->us < best) best = lone->us, name = "128x128x128_e2x2";
   }
   if (!s.fp4 && blocks(128, 128) > (uint64_t)cus) {   // two workgroups to a compute unit
     const uint64_t b = blocks(128, 128), rest = b % (2 * (uint64_t)cus);

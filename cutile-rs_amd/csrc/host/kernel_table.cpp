@@ -486,6 +486,21 @@ const KernelEntry* find_entry(const char* function, const std::string& variant) 
   return it == index.end() ? nullptr : it->second;
 }
 
+const KernelEntry* member_of(const KernelEntry* family, const char* suffix) {
+  static const auto& index = *[] {   // (every launch that takes a member asks: no name is put together for it)
+    auto* m = new std::unordered_map<const KernelEntry*, std::vector<std::pair<const char*, const KernelEntry*>>>();
+    for (const auto& e : kernel_table())
+      if (const char* plus = strchr(e.variant, '+'))
+        if (const KernelEntry* f = find_entry(e.function, std::string(e.variant, plus))) (*m)[f].emplace_back(plus, &e);
+    return m;
+  }();
+  auto it = index.find(family);
+  if (it != index.end())
+    for (const auto& [name, e] : it->second)
+      if (strcmp(name, suffix) == 0) return e;
+  return nullptr;
+}
+
 std::string list_variants(const char* function) {
   std::string s;
   for (const auto& e : kernel_table())

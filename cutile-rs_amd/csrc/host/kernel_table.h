@@ -32,6 +32,8 @@ const std::vector<KernelEntry>& kernel_table();
 const std::vector<const KernelEntry*>& kernels_of(const char* function);
 // Finds the entry (function, variant); nullptr if absent.
 const KernelEntry* find_entry(const char* function, const std::string& variant);
+// The member of `family` with that suffix ("+..."), nullptr if it has none: variants that only a launcher names.
+const KernelEntry* member_of(const KernelEntry* family, const char* suffix);
 // Resolves the entry's hipFunction_t on `device`, loading its code object on
 // first use (single flight per device).
 cutile_status_t load_entry(cutile_device_t device, const KernelEntry* entry, hipFunction_t* fn);

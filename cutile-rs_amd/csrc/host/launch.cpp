@@ -11,6 +11,7 @@
 #include <dlfcn.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -371,6 +372,7 @@ bool is_scaled_flat(const KernelEntry* e) { return e->image == IMG_SCALED_FLAT; 
 struct ScaledRoom {
   uint64_t bytes = kSplitPartialBytes;
   SplitWorkspace ws;
+  MxPlan lone{0, 0.0};   // what the rule on extents found for this room; splits = 0: nobody has asked, or more tiles than compute units
 };
 
 // Picks the kernel of a block-scaled product.  A kernel tile that is a whole multiple of the partition tile computes the
@@ -398,8 +400,8 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
   std::string sized;
   if (flat) {
     if (cutile_status_t s = current_device_units(cus)) return s;
-    const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes);
-    if (kernel && strcmp(kernel, "128x128x128_e2x2") == 0 && mx_plan(shape.m, shape.n, shape.pieces, *cus, room->bytes).splits > 1 && g_launch_mode != 2) {
+    const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes, &room->lone);
+    if (kernel && strcmp(kernel, "128x128x128_e2x2") == 0 && room->lone.splits > 1 && g_launch_mode != 2) {
       // a captured launch has no workspace and takes the best kernel of those that need none: their code object is loaded here
       cutile_device_t device = nullptr;
       hipFunction_t fn;
@@ -407,7 +409,7 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
       if (cutile_status_t s = load_entry(device, find_entry(function, "mxfp8_bf16_flat64x64"), &fn)) return s;
       if (g_launch_mode == 0) {
         room->ws = split_workspace(device, (hipStream_t)stream);
-        if (!room->ws.partials) kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes = 0);
+        if (!room->ws.partials) kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes = 0, &room->lone);
       }
     }
     if (kernel) sized = prefix + dt + "_" + kernel;
@@ -421,9 +423,8 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
 }
 
 // Replaces the resolved entry by a member of its family ("+" behind the variant's name), which only the launcher names.
-cutile_status_t use_member(Resolved* r, const char* function, const std::string& member) {
-  const KernelEntry* e = find_entry(function, member);
-  CUTILE_REQUIRE(e, CUTILE_ERR_KERNEL_NOT_FOUND, "kernel '%s' has no member '%s'", function, member.c_str());
+cutile_status_t use_member(Resolved* r, const KernelEntry* e) {
+  CUTILE_REQUIRE(e, CUTILE_ERR_KERNEL_NOT_FOUND, "variant '%s' of kernel '%s' lacks a member that this launch needs", r->entry->variant, r->entry->function);
   if (g_launch_mode != 2) {
     if (e != r->entry)
       if (cutile_status_t s = load_entry(r->device, e, &r->fn)) return s;
@@ -473,13 +474,14 @@ cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutil
   args.push_tile_grid(kg);
   uint32_t grid[3] = {kg[0] * kg[1], 1, 1};
   if (strstr(res.entry->variant, "_128x128x128_e2x2") != nullptr && grid[0] <= (uint32_t)cus && pieces >= 4) {   // a compute unit to each tile
-    uint32_t splits = mx_plan(zt.shape[0], zt.shape[1], pieces, cus, kg[0] == div_up(zt.shape[0], 128) && kg[1] == div_up(zt.shape[1], 128) ? room.bytes : 0).splits;
+    uint32_t splits = room.lone.splits ? room.lone.splits
+                                       : mx_plan(zt.shape[0], zt.shape[1], pieces, cus, kg[0] == div_up(zt.shape[0], 128) && kg[1] == div_up(zt.shape[1], 128) ? room.bytes : 0).splits;
     if (splits > 1 && g_launch_mode == 0 && !room.ws.partials) {   // a kernel that the caller or a record names
       room.ws = split_workspace(res.device, (hipStream_t)stream);
       if (!room.ws.partials) splits = 1;
     }
     splits = std::max(splits, 1u);   // (a partial launch may cover fewer tiles than z has)
-    if (cutile_status_t s = use_member(&res, res.entry->function, std::string(res.entry->variant) + "+lone")) return s;
+    if (cutile_status_t s = use_member(&res, member_of(res.entry, "+lone"))) return s;
     args.push_val<void*>(room.ws.partials);
     args.push_val<void*>(room.ws.counters);
     args.push_val<uint32_t>(splits);
@@ -492,24 +494,23 @@ cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutil
 constexpr int64_t kStreamedOutputBytes = 64ll << 20;
 // The code objects of every kernel that the size rule of the GEMM picks from.
 cutile_status_t load_gemm_images(cutile_device_t device) {
-  for (const char* v : {"f16_128x128x64_q2x2", "f16_192x256x64_q2x4", "f16_128x128x64_q2x2+lone"}) {
+  static const KernelEntry* const of_each[] = {find_entry("gemm", "f16_128x128x64_q2x2"), find_entry("gemm", "f16_192x256x64_q2x4"), find_entry("gemm", "f16_128x128x64_q2x2+lone")};
+  for (const KernelEntry* e : of_each) {
     hipFunction_t fn;
-    if (cutile_status_t s = load_entry(device, find_entry("gemm", v), &fn)) return s;
+    if (cutile_status_t s = load_entry(device, e, &fn)) return s;
   }
   return CUTILE_SUCCESS;
 }
 
 // Replaces the resolved family entry by the member for (z read as the initial accumulator?, z past the caches?) and
 // gives the launch grid: one workgroup per compute unit, or per tile if there are fewer tiles.
-cutile_status_t stream_member(Resolved* r, const char* function, bool accumulate, const cutile_tensor_arg_t& zt, uint64_t tiles,
+cutile_status_t stream_member(Resolved* r, bool accumulate, const cutile_tensor_arg_t& zt, uint64_t tiles,
                               uint32_t* grid) {
   const bool past_caches = (int64_t)zt.shape[0] * zt.shape[1] * (int64_t)cutile_dtype_size(zt.dtype) >= kStreamedOutputBytes;
-  std::string member = r->entry->variant;
-  if (!accumulate) member += "+new";
-  if (!past_caches) member += "+cached";
-  const char* family = r->entry->variant;
-  if (cutile_status_t s = use_member(r, function, member)) return s;
-  r->entry = find_entry(function, family);   // the launcher goes on by the family's name
+  const KernelEntry* const family = r->entry;
+  const char* member = accumulate ? past_caches ? "" : "+cached" : past_caches ? "+new" : "+new+cached";
+  if (cutile_status_t s = use_member(r, *member ? member_of(family, member) : family)) return s;
+  r->entry = family;   // the launcher goes on by the family's name
   int cus = 256;
   if (g_launch_mode != 2)
     if (cutile_status_t s = compute_units(r->device, &cus)) return s;
@@ -2205,7 +2206,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   }
   uint32_t stream_grid = 0;
   if (is_stream_variant(res.entry->variant)) {
-    if (cutile_status_t s = stream_member(&res, "gemm", accumulate != 0, zt, (uint64_t)tg[0] * tg[1], &stream_grid)) return s;
+    if (cutile_status_t s = stream_member(&res, accumulate != 0, zt, (uint64_t)tg[0] * tg[1], &stream_grid)) return s;
   } else if (strstr(res.entry->variant, "_p2x4") != nullptr) {   // the walking form: one workgroup per compute unit
     int cus = 256;
     if (g_launch_mode != 2)
@@ -2214,7 +2215,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   }
   uint32_t splits = 1;
   if (const RingTile* ring = row_layout && fast_layout && full_cover ? ring_tile(res.entry->variant, res.entry->tile[0], res.entry->tile[1]) : nullptr) {
-    RingPlan plan = ring_plan(*ring, cover_m, cover_n, k_valid, cus, partial_bytes);
+    RingPlan plan = ring == sized.ring ? sized.ring_plan : ring_plan(*ring, cover_m, cover_n, k_valid, cus, partial_bytes);
     if (plan.splits > 1 && !ws.partials && g_launch_mode == 0) {   // a kernel that the caller or a record names
       ws = split_workspace(res.device, (hipStream_t)stream);
       if (!ws.partials) plan = ring_plan(*ring, cover_m, cover_n, k_valid, cus, 0);
@@ -2222,10 +2223,10 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     splits = plan.splits;
     const char* member = ring->bm == 256 && ring->bn == 256 && splits > 1 ? "+split" : ring->bm == 128 && ring->bn == 128 && !plan.two ? "+lone" : nullptr;
     if (member)
-      if (cutile_status_t s = use_member(&res, "gemm", std::string(res.entry->variant) + member)) return s;
+      if (cutile_status_t s = use_member(&res, member_of(res.entry, member))) return s;
   }
   if (is_thin(res.entry) && !in_f32 && cover_m <= 16 && res.entry->tile[3] == 16 && streamed_past_caches(cover_n, k_valid))   // y is read once
-    if (cutile_status_t s = use_member(&res, "gemm", std::string(res.entry->variant) + "+nt")) return s;
+    if (cutile_status_t s = use_member(&res, member_of(res.entry, "+nt"))) return s;
   ArgPacker args;
   args.push_partition(*z);
   args.push_tensor(*x);
@@ -2238,7 +2239,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
     const F32Strip* strip = in_f32 ? f32_strip(res.entry->tile[3]) : nullptr;
-    splits = strip ? f32_plan(*strip, cover_m, cover_n, k_valid, cus, partial_bytes).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
+    splits = strip ? (strip == sized.strip ? sized.strip_plan : f32_plan(*strip, cover_m, cover_n, k_valid, cus, partial_bytes)).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (partial_bytes == 0) splits = 1;
     if (splits > 1 && g_launch_mode == 0 && !ws.partials) {
@@ -2525,7 +2526,7 @@ cutile_status_t cutile_launch_gemm_persistent(cutile_stream_t stream, const cuti
   if (is_stream_variant(res.entry->variant)) {
     uint32_t unused = 0;
     // (the member only; the launch grid stays the caller's num_tile_blocks, and the accumulators start from zero)
-    if (cutile_status_t s = stream_member(&res, "gemm_persistent", true, zt, m.total, &unused)) return s;
+    if (cutile_status_t s = stream_member(&res, true, zt, m.total, &unused)) return s;
   }
   ArgPacker args;
   args.push_partition(*z);
@@ -2594,7 +2595,7 @@ cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, con
     ahead = (int)grid[0] <= cus && 2 * (int)grid[0] > cus;
   }
   if (ahead)
-    if (cutile_status_t s = use_member(&res, "group_gemm_nt_desc", "f16_128x128x64_d2x2+ahead")) return s;
+    if (cutile_status_t s = use_member(&res, member_of(res.entry, "+ahead"))) return s;
   ArgPacker args;
   for (int i = 0; i < 3; ++i) args.push_tensor(*ptrs[i]);
   for (int i = 0; i < 3; ++i) args.push_tensor(*metas[i]);
@@ -2724,8 +2725,15 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, bool caus
   if (d == 64 && ((of64 <= 2 * cus && keys >= 512) || (of64 <= 4 * cus && causal && keys >= 1024))) return 64;
   return 0;
 }
-std::string keys_member(const std::string& dtype, int rows, int d) {
-  return dtype + "_" + std::to_string(rows) + (rows == 32 ? "x256x" : "x128x") + std::to_string(d) + "+keys";
+// (by their own rows, not by the family whose place they take)
+const KernelEntry* keys_member(const char* function, bool bf16, int rows, int d) {
+  static const auto& members = *[] {
+    auto* m = new std::array<const KernelEntry*, 16>();
+    for (size_t i = 0; i < m->size(); ++i)
+      (*m)[i] = find_entry(i & 8 ? "fmha_seq" : "fmha", std::string(i & 4 ? "bf16_" : "f16_") + (i & 2 ? "64x128x" : "32x256x") + (i & 1 ? "128+keys" : "64+keys"));
+    return m;
+  }();
+  return members[(strcmp(function, "fmha_seq") == 0) * 8 + bf16 * 4 + (rows == 64) * 2 + (d == 128)];
 }
 }  // namespace
 
@@ -2792,7 +2800,7 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   }
   if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, key_rows ? fallback : std::string())) return s;
   if (key_rows && g_last_source == "size") {
-    if (cutile_status_t s = use_member(&res, "fmha", keys_member(dt, key_rows, d))) return s;
+    if (cutile_status_t s = use_member(&res, keys_member("fmha", q->dtype == CUTILE_DTYPE_BF16, key_rows, d))) return s;
     tg[1] = div_up(ot.shape[1], key_rows);
   }
   ArgPacker args;
@@ -2910,7 +2918,7 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   }
   if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, key_rows ? acceptable[0] : std::string())) return s;
   if (key_rows && g_last_source == "size")
-    if (cutile_status_t s = use_member(&res, function, keys_member("f16", key_rows, d))) return s;
+    if (cutile_status_t s = use_member(&res, keys_member(function, false, key_rows, d))) return s;
   const int32_t kbm = res.entry->tile[0];
   ov.partition_shape[0] = 1; ov.partition_shape[1] = kbm; ov.partition_shape[2] = d;
   for (int i = 0; i < 3; ++i) ov.partition_strides[i] = ov.tensor.strides[i];
