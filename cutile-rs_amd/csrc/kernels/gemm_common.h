@@ -89,12 +89,8 @@ __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t total) 
   return xcd * q + min(xcd, r) + id / kNumXcd;
 }
 
-// Tile index for this workgroup: XCD-contiguous, then grouped along M.  Any number of tiles: with the plain order where it is no
-// multiple of 8, each XCD fetched every panel of both operands (f16, us before and after: 1844 x 11264 x 3584 on 128 x 256 tiles, 660 of them,
-// 193 and 154; 902 x 9472 x 3584 on 192 x 256 tiles, 185, 72 and 65).
-__device__ __forceinline__ void tile_coords(uint32_t tiles_m, uint32_t tiles_n, uint32_t* pm,
-                                            uint32_t* pn) {
-  const uint32_t id = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);
+// Tile `id` of an order grouped along M: kGroupM rows of tiles at a time, column by column.
+__device__ __forceinline__ void grouped_tile(uint32_t id, uint32_t tiles_m, uint32_t tiles_n, uint32_t* pm, uint32_t* pn) {
   const uint32_t per_group = kGroupM * tiles_n;
   const uint32_t group = id / per_group;
   const uint32_t first_m = group * kGroupM;
@@ -104,6 +100,14 @@ __device__ __forceinline__ void tile_coords(uint32_t tiles_m, uint32_t tiles_n, 
   *pn = in_group / rows;
 }
 
+// Tile index for this workgroup: XCD-contiguous, then grouped along M.  Any number of tiles: with the plain order where it is no
+// multiple of 8, each XCD fetched every panel of both operands (f16, us before and after: 1844 x 11264 x 3584 on 128 x 256 tiles, 660 of them,
+// 193 and 154; 902 x 9472 x 3584 on 192 x 256 tiles, 185, 72 and 65).
+__device__ __forceinline__ void tile_coords(uint32_t tiles_m, uint32_t tiles_n, uint32_t* pm,
+                                            uint32_t* pn) {
+  grouped_tile(xcd_contiguous(blockIdx.x, tiles_m * tiles_n), tiles_m, tiles_n, pm, pn);
+}
+
 // The same order for a workgroup that walks several tiles: item `id` of a launch of `stride` workgroups (workgroup b
 // takes b, b + stride, ...).  Workgroups are dealt round-robin to the XCDs, so with stride a multiple of 8 all items of
 // a workgroup lie on its XCD, which covers one contiguous eighth of the M-grouped order round by round.
@@ -111,13 +115,7 @@ __device__ __forceinline__ void tile_of_id(uint32_t id, uint32_t tiles_m, uint32
                                            uint32_t* pn) {
   const uint32_t total = tiles_m * tiles_n;
   if (total % kNumXcd == 0 && stride % kNumXcd == 0) id = (id % kNumXcd) * (total / kNumXcd) + id / kNumXcd;
-  const uint32_t per_group = kGroupM * tiles_n;
-  const uint32_t group = id / per_group;
-  const uint32_t first_m = group * kGroupM;
-  const uint32_t rows = min(tiles_m - first_m, (uint32_t)kGroupM);
-  const uint32_t in_group = id % per_group;
-  *pm = first_m + in_group % rows;
-  *pn = in_group / rows;
+  grouped_tile(id, tiles_m, tiles_n, pm, pn);
 }
 
 // Epilogue shared by the pipelined variants: accumulators -> z through LDS.

@@ -48,9 +48,10 @@ struct GemmF32 {
     const int64_t lda = x.strides[0], ldb = y.strides[0];
     const int32_t k_valid = min(min(x.shape[1], y.shape[0]), k_total);
     const uint32_t tile = xcd_contiguous(blockIdx.x, tiles_m * tiles_n);   // (strips on the x axis alone: y holds 65535 of them)
-    const uint32_t per_group = kGroupM * tiles_n, first_m = tile / per_group * kGroupM, group_rows = min(tiles_m - first_m, (uint32_t)kGroupM);
-    const int32_t row0 = (int32_t)(first_m + tile % per_group % group_rows) * ROWS;
-    const int32_t col_first = (int32_t)(tile % per_group / group_rows) * COLS;   // first column this workgroup stores
+    uint32_t pm, pn;
+    grouped_tile(tile, tiles_m, tiles_n, &pm, &pn);
+    const int32_t row0 = (int32_t)pm * ROWS;
+    const int32_t col_first = (int32_t)pn * COLS;                                // first column this workgroup stores
     const int32_t col0 = min(col_first, N - COLS);                               // the last strip is moved back to lie inside y (N >= 64)
 
     const float* yp = (const float*)y.ptr + col0 + l16 * 4 + (int64_t)(grp * 4) * ldb;

@@ -63,7 +63,6 @@ struct GroupAhead {
     __shared__ __attribute__((aligned(16))) Group groups[kMostGroups];
     __shared__ uint32_t wave_tiles[4], wave_k[4], wave_m[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
     // a thread to a group: its descriptors, and the running sum of tiles over the first four wavefronts
     uint32_t mine = 0;

@@ -280,10 +280,9 @@ struct GemmRing16 {
     // stages are free to carry the output (two wavefronts share an x stage, the
     // last two take the y stages).
     __syncthreads();
-    static_assert(kWaves <= 8, "no output band lies in the last y half");
     if (!combine(acc, reinterpret_cast<uint32_t*>(ys1b))) return;
-    static_assert(2 * kEpilogueBytesPerWave<WN> <= kABytes && kEpilogueBytesPerWave<WN> <= kBBytes / 2 && kWaves <= 10,
-                  "the output bands must fit the stages");
+    static_assert(2 * kEpilogueBytesPerWave<WN> <= kABytes && kEpilogueBytesPerWave<WN> <= kBBytes / 2 && kWaves <= 8,
+                  "the output bands must fit the stages, and none lie in the last y half");
     unsigned char* band = wave < 2 ? xs0 : wave < 4 ? xs1 : wave < 6 ? xs2 : wave == 6 ? ys0a : wave == 7 ? ys0b : wave == 8 ? ys1a : ys1b;
     if (wave < 6) band += (wave & 1) * kEpilogueBytesPerWave<WN>;
     store_tile_staged16<TM, TN, OutT>(acc, band, (OutT*)z.ptr, z.strides[0], z.shape[0], z.shape[1], row0 + wm * WM,

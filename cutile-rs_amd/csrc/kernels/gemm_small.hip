@@ -266,9 +266,9 @@ GEMM_STAGED_FAMILY(bf16f32, __bf16, float)
 
 // ---- tiles between 128 x 128 and 256 x 256 (gemm_tiles.h) ----------------------------------------------------------------------
 #define GEMM_TILES_FAMILY(N, T)                                  \
-  GEMM_RING_KERNEL(N##_192x256x64_q2x4, 192, 256, 2, 4, T)       \
-  GEMM_RING_KERNEL(N##_128x256x64_q2x4, 128, 256, 2, 4, T)       \
-  GEMM_RING_KERNEL(N##_256x128x64_q4x2, 256, 128, 4, 2, T)       \
+  GEMM_RING_TILE_KERNEL(N##_192x256x64_q2x4, 192, 256, 2, 4, T)       \
+  GEMM_RING_TILE_KERNEL(N##_128x256x64_q2x4, 128, 256, 2, 4, T)       \
+  GEMM_RING_TILE_KERNEL(N##_256x128x64_q4x2, 256, 128, 4, 2, T)       \
   GEMM_STAGES_KERNEL(N##_192x128x64_q2x2, 192, 128, 2, 4, 4, T)
 GEMM_TILES_FAMILY(bf16, __bf16)
 GEMM_TILES_FAMILY(f16, _Float16)

@@ -188,7 +188,7 @@ struct GemmStages {
                          float* partials, uint32_t* counters, uint32_t splits) {                                                    \
     GemmStages<BM, BN, WVM, WVN, STAGES, T>::run(z, x, y, k, g, accumulate, partials, counters, splits);                            \
   }
-#define GEMM_RING_KERNEL(NAME, BM, BN, WVM, WVN, T)                                                                                  \
+#define GEMM_RING_TILE_KERNEL(NAME, BM, BN, WVM, WVN, T)                                                                                  \
   extern "C" __global__ void __launch_bounds__(WVM * WVN * 64)                                                                      \
       gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k, TileGrid g, int32_t accumulate,               \
                          float* partials, uint32_t* counters, uint32_t splits) {                                                    \

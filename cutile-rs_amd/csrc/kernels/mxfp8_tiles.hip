@@ -47,8 +47,9 @@ struct MxStages {
     const int wm = wave / WAVES_N, wn = wave % WAVES_N, l16 = lane & 15, grp = lane >> 4;
     // split-major order: an XCD's contiguous share is neighbouring tiles on one range of K
     const uint32_t tiles_m = g.x, tiles_n = g.y, tiles = tiles_m * tiles_n, pos = xcd_contiguous(blockIdx.x, tiles * splits), split = pos / tiles, tile = pos % tiles;
-    const uint32_t per_group = kGroupM * tiles_n, first_m = tile / per_group * kGroupM, group_rows = min(tiles_m - first_m, (uint32_t)kGroupM);
-    const int32_t row0 = (int32_t)(first_m + tile % per_group % group_rows) * BM, col0 = (int32_t)(tile % per_group / group_rows) * BN;
+    uint32_t pm, pn;
+    grouped_tile(tile, tiles_m, tiles_n, &pm, &pn);
+    const int32_t row0 = (int32_t)pm * BM, col0 = (int32_t)pn * BN;
     const int32_t M = x.shape[0], N = y.shape[0], K = min(x.shape[1], y.shape[1]);
     const int32_t all_tiles = K / BK, blocks = (all_tiles + 3) / 4;
     const int32_t first = (int32_t)((int64_t)blocks * split / splits) * 4, k_tiles = min((int32_t)((int64_t)blocks * (split + 1) / splits) * 4, all_tiles) - first;
@@ -110,8 +111,8 @@ struct MxStages {
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // Tile kt (phase = kt % 4 = its stage) from fragments `f`; reads tile kt + 1 from `next`, fetches tile kt + 3 into `prev`.  `own` / `other`: the
-    // buffers of this tile's scale block and of the one after it.
+    // Tile kt (phase = kt % 4 = its stage) from fragments `f`; reads tile kt + 1 from `next`, fetches tile kt + 3 into `prev`.  `other`: the
+    // buffer of the scale block after this tile's.
     auto k_tile = [&](const Frags& f, Frags& into, const unsigned char* next, unsigned char* prev, unsigned char* other, int32_t kt, auto phase) {
       constexpr int PH = decltype(phase)::value;
       // tile kt + 1 has landed: tile kt + 2 (with a scale block if it opens one) may be outstanding

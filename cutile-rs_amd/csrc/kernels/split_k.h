@@ -80,8 +80,7 @@ __device__ __forceinline__ SplitTile split_tile(uint32_t tiles_m, uint32_t tiles
   const uint32_t tiles = tiles_m * tiles_n, pos = xcd_contiguous(blockIdx.x, tiles * splits);
   SplitTile t;
   t.split = pos / tiles, t.tile = pos % tiles;
-  const uint32_t per_group = kGroupM * tiles_n, first_m = t.tile / per_group * kGroupM, rows = min(tiles_m - first_m, (uint32_t)kGroupM);
-  t.pm = first_m + t.tile % per_group % rows, t.pn = t.tile % per_group / rows;
+  grouped_tile(t.tile, tiles_m, tiles_n, &t.pm, &t.pn);
   const int32_t k_tiles = (min(min(x.shape[1], y.shape[0]), k) + BK - 1) / BK;
   const int32_t k0 = (int32_t)((int64_t)k_tiles * t.split / splits) * BK, k1 = (int32_t)((int64_t)k_tiles * (t.split + 1) / splits) * BK;
   x.ptr = (unsigned char*)x.ptr + (int64_t)k0 * BYTES;
