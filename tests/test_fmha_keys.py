@@ -79,6 +79,7 @@ def _close(got, ref, dtype):
 def test_gpu_attention_sharing_keys(ct, dev, dtype, d, batch, heads, group, rows, keys, causal, pos):
     q, k, v, out = _call(ct, dtype, batch, heads, group, rows, keys, d, causal, pos=pos, dev=dev)
     torch.cuda.synchronize()
+    assert ct.last_resolved()["symbol"].endswith(f"_64x128x{d}_keys" if heads >= 16 else f"_32x256x{d}_keys")
     assert _close(out, _reference(q, k, v, d ** -0.5, pos, group, causal), dtype)
 
 
@@ -93,6 +94,27 @@ def test_gpu_sequence_attention_sharing_keys(ct, dev, d, rows, start, on_device)
     where = dict(position_start=torch.tensor([start], dtype=torch.int32, device=dev)) if on_device else dict(kv_len=start + rows, query_start=start)
     ct.fmha_seq_f16(q, k, v, ct.partition(out, [64, 1, d]), d ** -0.5, 4, **where)
     torch.cuda.synchronize()
+    assert ct.last_resolved()["symbol"] == f"{'fmha_seq' if on_device else 'fmha'}_entry__f16_32x256x{d}_keys"
     seen = 600 if on_device else start + rows
     ref = _reference(q.permute(1, 0, 2)[None], k[None, :, :seen], v[None, :, :seen], d ** -0.5, start, 4, True)
+    assert _close(out.permute(1, 0, 2), ref, torch.half)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rows,heads,position,causal,member", [(129, 8, 0, True, 32), (200, 8, 255, True, 32), (200, 8, 256, False, 32), (400, 8, 131, False, 32), (300, 32, 599, True, 64),
+                                                               (300, 32, 700, False, 64)])
+def test_gpu_sequence_attention_sharing_keys_up_to_the_position(ct, dev, d, rows, heads, position, causal, member):
+    """keys 0 .. position, which only the device knows: the kernel cuts them off itself; what lies behind them must not be seen"""
+    g = torch.Generator().manual_seed(rows + position)
+    normal = lambda *s: torch.randn(*s, generator=g).half().to(dev)
+    q, k, v = normal(rows, heads, d), normal(2, 640, d), normal(2, 640, d)
+    seen = min(position + 1, 640)
+    k[:, seen:], v[:, seen:] = 100.0, 1000.0
+    out = torch.full((rows, heads, d), 7.0, dtype=torch.half, device=dev)
+    where = torch.tensor([position], dtype=torch.int32, device=dev)
+    ct.fmha_seq_f16(q, k, v, ct.partition(out, [64, 1, d]), d ** -0.5, heads // 2, position_start=where, kv_len_from_position=True, causal=causal)
+    torch.cuda.synchronize()
+    assert ct.last_resolved()["symbol"] == f"fmha_seq_entry__f16_{'32x256' if member == 32 else '64x128'}x{d}_keys"
+    ref = _reference(q.permute(1, 0, 2)[None], k[None, :, :seen], v[None, :, :seen], d ** -0.5, position, heads // 2, causal)
     assert _close(out.permute(1, 0, 2), ref, torch.half)

@@ -152,8 +152,10 @@ def test_more_than_48_rows_of_a_long_k_share_it_on_tiles(fake_hip):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("m,n,k", [(49, 272, 1800), (64, 2248, 7680), (65, 576, 3976), (128, 3584, 4096), (100, 64, 6408)])
-def test_gpu_long_k_shared_on_tiles_of_few_rows(ct, dev, m, n, k, dtype):
+@pytest.mark.parametrize("m,n,k,kernel", [(49, 272, 1800, "staged64x64"), (64, 2248, 7680, "128x128x64_q2x2_lone"), (65, 576, 3976, "staged64x64"),
+                                          (128, 3584, 4096, "128x128x64_q2x2_lone"), (100, 64, 6408, "staged64x64"), (50, 3592, 4104, "128x128x64_q2x2_lone"),
+                                          (127, 1416, 5128, "128x128x64_q2x2_lone")])
+def test_gpu_long_k_shared_on_tiles_of_few_rows(ct, dev, m, n, k, kernel, dtype):
     g = torch.Generator(device="cuda").manual_seed(m + n)
     x = torch.randn(m, k, device=dev, generator=g).to(dtype)
     y = (torch.randn(k, n, device=dev, generator=g) / k ** 0.5).to(dtype)
@@ -162,7 +164,7 @@ def test_gpu_long_k_shared_on_tiles_of_few_rows(ct, dev, m, n, k, dtype):
     for _ in range(2):
         ct.gemm(ct.partition(z[:m], [128, 128]), x, y, k, accumulate=False, generics=["f16" if dtype == torch.float16 else "bf16", 128, 128, 1])
         torch.cuda.synchronize()
-        assert "thin" not in ct.last_resolved()["variant"]
+        assert ct.last_resolved()["symbol"].endswith("_" + kernel)
         assert rel_l2(z[:m].double().cpu().numpy(), want) <= (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8)   # one rounding over f32 sums
         assert torch.all(z[m] == 7.0)
 

@@ -215,9 +215,11 @@ def test_gpu_group_gemm_ahead(ct, dev, shapes, num_sm):
         refs.append(f16v(ab)[:m, :k].astype(np.float64) @ f16v(bb)[:k].astype(np.float64))
     (ap, am), (bp, bm), (cp, cm), (rp, rm), (gp, gm) = [_tables(t, dev) for t in (a_t, b_t, *[[c[:-1] for c in t] for t in (c_t, r_t, g_t)])]
     ct.group_gemm_f16_nt_desc(ap, bp, rp, am, bm, rm, len(shapes), generics=[128, 128, 64, num_sm], variant="f16_128x128x64_d2x2")
+    assert ct.last_resolved()["symbol"].endswith("_d2x2")
     for _ in range(3):
         ct.group_gemm_f16_nt_desc(ap, bp, cp, am, bm, cm, len(shapes), generics=[128, 128, 64, num_sm])
     torch.cuda.synchronize()
+    assert ct.last_resolved()["symbol"].endswith("_d2x2_ahead")
     launch = lambda stream: ct.group_gemm_f16_nt_desc(ap, bp, gp, am, bm, gm, len(shapes), generics=[128, 128, 64, num_sm], stream=stream)
     graph = ct.CapturedGraph().capture(launch)
     try:

@@ -39,6 +39,21 @@ def test_gpu_mxfp8_tiles(ct, dev, m, n, k, out):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(2050, 2180, 640), (130, 33028, 256)])
+def test_gpu_mxfp8_two_stages_beyond_a_tile_to_each_compute_unit(ct, dev, m, n, k):
+    """more tiles than compute units: the two-stage kernel of that name, edges in both directions and a last scale block of one K tile"""
+    xq, xs, x, sx = _operands(m, k, 13, dev)
+    yq, ys, y, sy = _operands(n, k, 14, dev)
+    xw, yw = (torch.from_numpy(oracle.mx_dequantize_e4m3(q, s).astype(np.float64)).to(dev) for q, s in ((xq, xs), (yq, ys)))
+    want = xw @ yw.T.contiguous()
+    z = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=dev)
+    ct.linear_tile_mxfp8(ct.partition(z[:m], [128, 128]), x, y, sx, sy, 1.0, variant="mxfp8_bf16_128x128x128_e2x2")
+    torch.cuda.synchronize()
+    assert ct.last_resolved()["symbol"].endswith("_e2x2")
+    assert float((z[:m].double() - want).norm()) <= 2.0 ** -8 * float(want.norm()) and torch.all(z[m] == 7.0)
+
+
+@pytest.mark.gpu
 def test_gpu_mxfp8_scales_behind_a_row(ct, dev):
     """K = 640: the tile's last scale block reads on into the next row's scales, which are NaN here"""
     k = 640
