@@ -8,12 +8,15 @@
 //  * the operand stages run through from tile to tile: an iterator of its own walks the K tiles three ahead of the ones being
 //    multiplied, across the ends of output tiles, and the output leaves from the accumulators, without LDS;
 //  * B is read past the caches where no group has more than one row of tiles: then it is read once (16 groups of 96 x 6400 x 4608 on
-//    average, some of two rows of tiles: 225 us through the caches, 241 past them);
+//    average, some of two rows of tiles: 225 us through the caches, 241 past them).  us on the ring, here through the caches and here past them,
+//    the same B again at once: 8 groups of 4096 x 2048 24.3, 24.2, 23.9; 32 of 1024 x 1024 24.2, 18.1, 17.2; 8 of 4096 x 4096, 268 MB, 45.4,
+//    45.4, 45.3; sets of B in turn, so that it comes from memory: 27.8, 28.8, 25.8; 26.8, 18.7, 18.1; 49.1, 50.7, 46.4.  (B of 200 to 270 MB
+//    that is just one tile to a compute unit is the one loss with B in the memory-side cache: 8 of 60 x 4096 x 3072 36.9, 37.2, 38.6);
 //  * where there are fewer tiles than half of the workgroups, several share the K tiles of one (split_k.h).
 // Stages, barriers and fragments as in GemmStages (gemm_tiles.h) with four stages.
 // f16, us on the ring and here: 32 groups of 32 x 4096 x 4096 on average 200 and 183 (1.07 GB of B, 5.9 TB/s); 64 of 3.3 x 4608 x 7936
-// 803 and 739; 64 of 2.4 x 768 x 512 36.8 and 19.2; sharing K: 16 of 1 x 6912 x 1024 65.6 and 28.9 (52 unshared), 8 of 8 x 6144 x 1792
-// 60.7 and 35.5 (53).
+// 803 and 739; 64 of 2.4 x 768 x 512 36.8 and 19.2; sharing K, uneven groups, some without a row: 16 of 1 x 6912 x 1024 65.6 and 28.9 (52
+// unshared), 8 of 8 x 6144 x 1792 60.7 and 35.5 (53).
 #include <hip/hip_runtime.h>
 
 #include "gemm_common.h"

@@ -22,9 +22,11 @@ namespace gemm {
 // unit, 64-column ones 26-38, 128-column ones up to 53; and x is read two 32-wide steps at a time for the same reason.
 // NT: y past the caches, for a y that is read once and too large to be found there again (96 MiB and more, 16 rows at most): a streaming
 // read of plain loads fills them first.  f16, one row, weights from memory, us: 4096 x 14336 24.3 -> 22.0 on 128-column strips (64-column ones
-// 23.0), 14336 x 4096 24.7 -> 23.4, 8192 x 28672 83.0 -> 75.0; a block of one new token over these weights 131 -> 120.  A product that runs again
-// at once on the same weights of up to about 200 MB would find them in the memory-side cache (4096 x 14336 19.1 us, with NT 20.1).  Not for
-// 17 to 32 rows, where it gains 2 to 3 % and loses 16 to 32 % in that case, nor for smaller weights, several of which fit that cache.
+// 23.0), 14336 x 4096 24.7 -> 23.4, 8192 x 28672 83.0 -> 75.0; a block of one new token over these weights 131 -> 120.  The price: weights that
+// the memory-side cache (256 MB) still holds when they are read again are read slower (one row, plain and NT: 14336 x 4096 again at once 20.4, 22.0,
+// two of them in turn 20.5, 22.7, four 24.9, 23.2; 8192 x 12288, 201 MB, 31.5, 34.3, two 38.9, 35.6; 8192 x 16384, 268 MB, 41.8, 45.9, two 50.4,
+// 47.1; 8192 x 20480, 336 MB, 63.1, 58.9).  A program that steps through layers of such weights has read more than that cache holds
+// before it comes back to one.  Not for 17 to 32 rows, where it gains 2 to 3 % and costs 16 to 32 %, nor for smaller weights, several of which fit.
 template <typename InT, typename OutT, int MB, int CPL, int WAVES, bool NT>
 struct GemmThin {
   static constexpr int CW = 16 * CPL, ROWS = 16 * MB, kThreads = WAVES * 64;

@@ -20,8 +20,9 @@ namespace gemm {
 // kt + 1, requested STAGES - 2 K tiles ago.  Fragments are double-buffered (a K step of 32 is read while the one before it is
 // multiplied), and eight wavefronts, two to a SIMD, keep the matrix pipe fed across each other's waits (four of them: 178 us where eight
 // take 164 at 1500 x 4096 x 14336).
-// f16, operands from memory, us on the ring and here: 1500 x 4096 x 14336, 256 tiles of 192 x 128, 183 and 164; 1500 x 4096 x 4096
-// 57.5 and 50.7; on 128 x 128 tiles 1500 x 1024 x 4096, 96 of them, 35 and 26, 2048 x 2048 x 2048, 256 of them, 24 and 20.
+// f16, us on the ring and here, operands from memory (and from the caches): 1500 x 4096 x 14336, 256 tiles of 192 x 128, 189 and 169 (181, 157);
+// 1500 x 4096 x 4096 57.7 and 52.1 (54.7, 48.8); on 128 x 128 tiles 1500 x 1024 x 4096, 96 of them, here with K shared by two, 38.6 and 25.5 (35.3,
+// 23.8), 2048 x 2048 x 2048, 256 of them, 24.1 and 22.9.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, typename InT>
 struct GemmStages {
   static constexpr int BK = 64, kWaves = WAVES_M * WAVES_N, kThreads = kWaves * 64;
