@@ -199,11 +199,14 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
                                          {"staged64x64", 64, 64, 4, {0.52, 0.235, 5.0, 6.0, 1.6e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
     for (const StagedTile& r : kStaged) {
       if (s.y_cols < r.bn) continue;
-      const uint64_t t = tiles(r.bm, r.bn), sk = partial_bytes ? staged_splits(r.bm, r.bn, t, s.k, cus) : 1;
+      const uint64_t t = tiles(r.bm, r.bn), would_share = staged_splits(r.bm, r.bn, t, s.k, cus), sk = partial_bytes ? would_share : 1;
       const double w = (double)((t * sk + cus - 1) / cus);
       if (r.per_cu == 1 && w > 2) continue;
       const Cost& c1 = ring ? r.aligned : r.any;
-      const double us = kt / (double)sk * std::max(c1.one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
+      // (a long K that there is no room to share: 0.385 to 0.395 us a K tile, the fit knows short ones alone; captured, us on these and on 128 x 128
+      // tiles: 309 x 2240 x 5184 34.4, 31.2; 184 x 4928 x 4736 32.0, 29.1; 460 x 1792 x 2304 17.8, 17.0)
+      const double one = ring && sk < would_share ? 0.40 : c1.one;
+      const double us = kt / (double)sk * std::max(one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
                         (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
       if (us < best * 0.98) best = us, picked = r.kernel, shares_k = sk > 1, c.ring = nullptr;
     }

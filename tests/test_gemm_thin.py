@@ -216,3 +216,18 @@ def test_gpu_captured_product_of_staged_tiles_that_would_share_k(ct, dev, m, n, 
                 assert rel_l2(z.double().cpu().numpy(), want) <= 2.0 ** -11        # one rounding over f32 sums
     finally:
         graph.close()
+
+
+def test_products_of_a_long_k_without_a_workspace_take_larger_tiles(fake_hip):
+    """beyond 128 rows: 64 x 64 staged tiles pay by their split; where there is none, 128 x 128 tiles are the faster ones"""
+    ct = fake_hip
+    from test_gemm_tiles import _new_stream, _workgroups
+    buf = torch.empty(30 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+    for m, n, k in ((309, 2240, 5184), (332, 2048, 1920), (460, 1792, 2304), (1008, 768, 3968), (156, 3392, 2048), (748, 320, 1728), (184, 4928, 4736), (300, 640, 4096)):
+        dev, stream = _new_stream(ct)
+        ct.check(ct.lib().cutile_testing_inject_failure(b"hipMallocAsync", 2, 1))
+        for _ in range(257):
+            ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k, stream=stream.value)
+        assert ct.last_resolved()["symbol"] == "gemm_entry__f16_128x128x64_q2x2_lone" and _workgroups(ct) == -(-m // 128) * -(-n // 128), (m, n, k)
+        ct.check(ct.lib().cutile_stream_release(dev, stream))
