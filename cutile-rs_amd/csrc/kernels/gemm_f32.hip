@@ -155,23 +155,10 @@ struct GemmF32 {
       for (int o = tid; o < quads; o += WAVES * 64) store(o, wave_sum(o));
       return;
     }
-    float* mine = partials + (int64_t)tile * splits * (ROWS * COLS);
-    for (int o = tid; o < quads; o += WAVES * 64) {
-      const f32x4 v = wave_sum(o);
-      float* p = mine + (int64_t)blockIdx.z * (ROWS * COLS) + o * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) store_partial(p + e, v[e]);
-    }
+    const BlockPartials part(partials + (int64_t)tile * splits * (ROWS * COLS), ROWS * COLS * 4, splits);
+    for (int o = tid; o < quads; o += WAVES * 64) part.store(blockIdx.z, o, wave_sum(o));
     if (!last_to_arrive(counters + tile, splits, &last)) return;
-    for (int o = tid; o < quads; o += WAVES * 64) {
-      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-      for (uint32_t k = 0; k < splits; ++k) {
-        const float* p = mine + (int64_t)k * (ROWS * COLS) + o * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += load_partial(p + e);
-      }
-      store(o, v);
-    }
+    part.add_up<WAVES * 64, (ROWS * COLS / 4 > WAVES * 64 ? 2 : 1)>(quads, store);
   }
 };
 

@@ -3,6 +3,8 @@
 // read 0, stores outside z are dropped.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gemm_common.h"
 #include "gemm_thin.h"
 #include "gemm_tiles.h"
@@ -178,23 +180,24 @@ struct GemmStaged {
     // then a thread takes 8 neighbouring columns of a row at a time: 16-byte accesses of z and of the partial sums.
     OutT* zp = (OutT*)z.ptr;
     const int32_t ldz = z.strides[0];
-    auto store = [&](int r, int u, const float* v) {
-      const int32_t gr = row0 + r, gc = col0 + u * 8;
+    auto store = [&](int r, int c, const float* v, auto width) {   // `width` values from column c of the tile's row r
+      constexpr int W = decltype(width)::value;
+      const int32_t gr = row0 + r, gc = col0 + c;
       if (gr >= cover_m || gc >= cover_n) return;
       OutT* dst = zp + (int64_t)gr * ldz + gc;
-      if (gc >= col_first && gc + 8 <= cover_n) {
-        OutT o[8];
+      if (gc >= col_first && gc + W <= cover_n) {
+        OutT o[W];
         if (accumulate) __builtin_memcpy(o, __builtin_assume_aligned(dst, sizeof(OutT)), sizeof(o));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (OutT)(accumulate ? v[e] + (float)o[e] : v[e]);
+        for (int e = 0; e < W; ++e) o[e] = (OutT)(accumulate ? v[e] + (float)o[e] : v[e]);
         __builtin_memcpy(__builtin_assume_aligned(dst, sizeof(OutT)), o, sizeof(o));
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < W; ++e)
           if (gc + e >= col_first && gc + e < cover_n) dst[e] = (OutT)(accumulate ? v[e] + (float)dst[e] : v[e]);
       }
     };
-    float* mine = partials + (int64_t)tile * splits * (BM * BN);
+    const BlockPartials part(partials + (int64_t)tile * splits * (BM * BN), BM * BN * 4, splits);
     for (int pass = 0; pass < kOutPasses; ++pass) {
       __syncthreads();   // the stages (or the previous pass) have been read
       const int first = pass * kOutRows;
@@ -215,25 +218,19 @@ struct GemmStaged {
         f32x4 v[2] = {*reinterpret_cast<const f32x4*>(lds + r * (BN * 4) + (((2 * u) ^ (r & 15)) << 4)),
                       *reinterpret_cast<const f32x4*>(lds + r * (BN * 4) + (((2 * u + 1) ^ (r & 15)) << 4))};
         const float f[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
-        if (splits == 1)
-          store(first + r, u, f);
-        else
-          store_partials(mine + (int64_t)split * (BM * BN) + (first + r) * BN + u * 8, f);
+        if (splits == 1) {
+          store(first + r, u * 8, f, std::integral_constant<int, 8>{});
+        } else {
+          part.store(split, ((first + r) * UB + u) * 2, v[0]);
+          part.store(split, ((first + r) * UB + u) * 2 + 1, v[1]);
+        }
       }
     }
     if (splits == 1 || !last_to_arrive(counters + tile, splits, &last)) return;
-    for (int o = tid; o < BM * UB; o += kThreads) {
-      const int r = o / UB, u = o % UB;
-      if (row0 + r >= cover_m) break;
-      float sum[8] = {};
-      for (uint32_t k = 0; k < splits; ++k) {
-        float f[8];
-        load_partials(mine + (int64_t)k * (BM * BN) + r * BN + u * 8, f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sum[e] += f[e];
-      }
-      store(r, u, sum);
-    }
+    part.add_up<kThreads, 2>(min(BM, cover_m - row0) * (BN / 4), [&](int o, f32x4 v) {
+      const float f[4] = {v[0], v[1], v[2], v[3]};
+      store(o / (BN / 4), o % (BN / 4) * 4, f, std::integral_constant<int, 4>{});
+    });
   }
 };
 

@@ -166,36 +166,40 @@ struct GemmThin {
         }
       }
     __syncthreads();
-    const int32_t outputs = min(ROWS, cover_m - row0) * CW;
+    const int32_t quads = min(ROWS, cover_m - row0) * (CW / 4);   // four consecutive columns of a row to a thread
     auto wave_sum = [&](int o) {
-      const int r = o / CW, c = o % CW;
-      float v = 0.0f;
+      const int r = o / (CW / 4), c = o % (CW / 4) * 4;
+      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w) v += red[w][r][c];
+      for (int w = 0; w < WAVES; ++w) v += *reinterpret_cast<const f32x4*>(&red[w][r][c]);
       return v;
     };
     OutT* zp = (OutT*)z.ptr;
-    auto store = [&](int o, float v) {
-      const int32_t gc = col0 + o % CW;
-      if (gc < col_first || gc >= cover_n) return;
-      OutT* dst = zp + (int64_t)(row0 + o / CW) * z.strides[0] + gc;
-      if (accumulate) v += (float)*dst;
-      *dst = (OutT)v;
+    auto store = [&](int o, f32x4 v) {
+      const int32_t gc = col0 + o % (CW / 4) * 4;
+      OutT* dst = zp + (int64_t)(row0 + o / (CW / 4)) * z.strides[0] + gc;
+      if (gc >= col_first && gc + 4 <= cover_n) {
+        OutT e[4];
+        if (accumulate) __builtin_memcpy(e, __builtin_assume_aligned(dst, sizeof(OutT)), sizeof(e));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = (OutT)(accumulate ? v[i] + (float)e[i] : v[i]);
+        __builtin_memcpy(__builtin_assume_aligned(dst, sizeof(OutT)), e, sizeof(e));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (gc + i >= col_first && gc + i < cover_n) dst[i] = (OutT)(accumulate ? v[i] + (float)dst[i] : v[i]);
+      }
     };
     const uint32_t splits = gridDim.z;
     if (splits == 1) {
-      for (int o = tid; o < outputs; o += kThreads) store(o, wave_sum(o));
+      for (int o = tid; o < quads; o += kThreads) store(o, wave_sum(o));
       return;
     }
     const uint32_t block = blockIdx.y * gridDim.x + strip;
-    float* mine = partials + (int64_t)block * splits * (ROWS * CW);
-    for (int o = tid; o < outputs; o += kThreads) store_partial(mine + blockIdx.z * (ROWS * CW) + o, wave_sum(o));
+    const BlockPartials part(partials + (int64_t)block * splits * (ROWS * CW), ROWS * CW * 4, splits);
+    for (int o = tid; o < quads; o += kThreads) part.store(blockIdx.z, o, wave_sum(o));
     if (!last_to_arrive(counters + block, splits, &last)) return;
-    for (int o = tid; o < outputs; o += kThreads) {
-      float v = 0.0f;
-      for (uint32_t k = 0; k < splits; ++k) v += load_partial(mine + k * (ROWS * CW) + o);
-      store(o, v);
-    }
+    part.add_up<kThreads, (ROWS * CW / 4 > kThreads ? 2 : 1)>(quads, store);
   }
 };
 

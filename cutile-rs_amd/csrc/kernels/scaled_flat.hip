@@ -239,20 +239,10 @@ struct ScaledFlat {
       for (int o4 = tid; o4 < rows * kQuads; o4 += kThreads) store(o4, sum(o4));
       return;
     }
-    float* const mine = partials + (int64_t)tile * splits * (BM * BN);
-    for (int o4 = tid; o4 < rows * kQuads; o4 += kThreads) {
-      const f32x4 v = sum(o4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) store_partial(mine + (int64_t)split * (BM * BN) + o4 * 4 + e, v[e]);
-    }
+    const BlockPartials part(partials + (int64_t)tile * splits * (BM * BN), BM * BN * 4, splits);
+    for (int o4 = tid; o4 < rows * kQuads; o4 += kThreads) part.store(split, o4, sum(o4));
     if (!last_to_arrive(counters + tile, splits, &last)) return;
-    for (int o4 = tid; o4 < rows * kQuads; o4 += kThreads) {
-      f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-      for (uint32_t k = 0; k < splits; ++k)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += load_partial(mine + (int64_t)k * (BM * BN) + o4 * 4 + e);
-      store(o4, v);
-    }
+    part.add_up<kThreads, (BM * kQuads > kThreads ? 2 : 1)>(rows * kQuads, store);
   }
 };
 

@@ -12,24 +12,47 @@ namespace gemm {
 // launches.  The splits of a block run on different XCDs, whose L2 caches are not coherent with each other, so partials
 // and counter move with agent-scope accesses (past the L2); the workgroup that counts last adds the partials in split
 // order, whatever order they arrived in, so the sum does not depend on timing.
-__device__ __forceinline__ void store_partial(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ float load_partial(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// eight neighbours at once (8-byte aligned)
-__device__ __forceinline__ void store_partials(float* p, const float* f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(p) + i,
-                       (uint64_t)__builtin_bit_cast(uint32_t, f[2 * i]) | (uint64_t)__builtin_bit_cast(uint32_t, f[2 * i + 1]) << 32, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void load_partials(const float* p, float* f) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p) + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    f[2 * i] = __builtin_bit_cast(float, (uint32_t)v);
-    f[2 * i + 1] = __builtin_bit_cast(float, (uint32_t)(v >> 32));
+constexpr int kAgentScope = 16;   // buffer accesses with sc1: past the L2, which the XCDs do not share
+// The partial sums of one block: quads of four neighbouring outputs, numbered as the kernel likes, one copy of `bytes` per split.
+struct BlockPartials {
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t bytes, splits;
+
+  __device__ __forceinline__ BlockPartials(float* mine, uint32_t block_bytes, uint32_t n) : rsrc(make_rsrc(mine, block_bytes * n)), bytes(block_bytes), splits(n) {}
+  __device__ __forceinline__ void store(uint32_t split, int quad, f32x4 v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, quad * 16, split * bytes, kAgentScope);
   }
-}
+  // take(quad, sum in split order) for every quad, dealt to THREADS threads, Q quads of eight splits at a time: a read past the L2 takes about a
+  // microsecond, and one after another (a value, a split) they were much of a launch of few rows (f16, kernel time in us with such reads and
+  // here, K shared by 6 or 7: 17 x 1088 x 7168 13.5, 8.9; 37 x 2048 x 6656 21.5, 15.0; 64 x 2048 x 6656 on 64 x 64 tiles, by 8, 20.5, 16.4).
+  template <int THREADS, int Q, typename F>
+  __device__ __forceinline__ void add_up(int quads, F&& take) const {
+    constexpr uint32_t kOob = 0x80000000u, kAtOnce = 8;
+    for (int o = threadIdx.x; o < quads; o += THREADS * Q) {
+      f32x4 sum[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+      for (uint32_t k = 0; k < splits; k += kAtOnce) {
+        u32x4 v[kAtOnce][Q];
+#pragma unroll
+        for (uint32_t i = 0; i < kAtOnce; ++i)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            const bool wanted = k + i < splits && o + q * THREADS < quads;   // others read 0 and never leave the compute unit
+            v[i][q] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, wanted ? (uint32_t)(o + q * THREADS) * 16 : kOob, k + i < splits ? (k + i) * bytes : 0, kAgentScope);
+          }
+#pragma unroll
+        for (uint32_t i = 0; i < kAtOnce; ++i)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) sum[q] += __builtin_bit_cast(f32x4, v[i][q]);
+      }
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (o + q * THREADS < quads) take(o + q * THREADS, sum[q]);
+    }
+  }
+};
 // Called by the whole workgroup after its partials are stored: true in the workgroup that arrives last of `splits`.
 __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t splits, uint32_t* shared_flag) {
   __builtin_amdgcn_s_waitcnt(0);   // this wavefront's partials have reached memory
@@ -46,7 +69,6 @@ __device__ __forceinline__ bool last_to_arrive(uint32_t* counter, uint32_t split
 // A tile held in a workgroup's accumulators, computed by `splits` workgroups: false in all but the one that arrives last, whose
 // accumulators then hold the sum (in split order).  `mine` = the tile's share of the workspace; a partial tile lies there register
 // by register, thread by thread: 16 bytes a lane, whole lines, and a thread reads only what its namesakes wrote.
-constexpr int kAgentScope = 16;   // buffer accesses with sc1: past the L2, which the XCDs do not share
 template <int TM, int TN, int THREADS>
 __device__ __forceinline__ bool combine_tile(f32x4 (&acc)[TN][TM], float* mine, uint32_t* counter, uint32_t split, uint32_t splits, uint32_t* shared_flag) {
   constexpr uint32_t kTile = TM * TN * THREADS * 16;   // bytes
@@ -55,6 +77,7 @@ __device__ __forceinline__ bool combine_tile(f32x4 (&acc)[TN][TM], float* mine, 
   for (int r = 0; r < TM * TN; ++r)
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[r % TN][r / TN]), part, threadIdx.x * 16, split * kTile + r * (THREADS * 16), kAgentScope);
   if (!last_to_arrive(counter, splits, shared_flag)) return false;
+  // (one partial tile at a time: with the next one's loads in flight beside it 48 and 54 tiles of 128 x 128 took 14.5 us where they take 13.7)
   auto add = [&](uint32_t k) {
 #pragma unroll
     for (int r = 0; r < TM * TN; ++r)
