@@ -392,6 +392,9 @@ std::vector<KernelEntry> build_table() {
       std::string v = "f16_g" + std::to_string(grp) + "_d" + std::to_string(d);
       add("fmha_decode_gqa_split", keep(v), keep("fmha_decode_gqa_split_entry__" + v), IMG_FMHA, 256,
           (uint32_t)(4 * grp * (d + 2) * 4), grp, 0, d, 0, "f16", 0, 3);
+      if (d == 128 && grp <= 2)   // with the merge of the splits behind it (the launcher names it)
+        add("fmha_decode_gqa_split", keep(v + "+merge"), keep("fmha_decode_gqa_split_entry__" + v + "_merge"), IMG_FMHA, 256,
+            (uint32_t)(4 * grp * (d + 2) * 4 + grp * (64 * 4 + 256 * 32)), grp, 0, d, 0, "f16", 0, 3);
     }
   // the same on the matrix cores (heads are the N dimension of a 16x16x32 MFMA, columns beyond GROUP are zero); LDS = 4 wavefronts x 2 stages x 32 V rows
   for (int d : {64, 128, 256})
@@ -399,6 +402,9 @@ std::vector<KernelEntry> build_table() {
       std::string v = "f16_g" + std::to_string(grp) + "_d" + std::to_string(d) + "_mfma";
       add("fmha_decode_gqa_split", keep(v), keep("fmha_decode_gqa_split_entry__" + v), IMG_FMHA, 256, (uint32_t)(4 * 2 * 32 * d * 2), grp,
           0, d, 0, "f16", 0, 3);
+      if (grp <= 4 && (d != 128 || grp > 2))
+        add("fmha_decode_gqa_split", keep(v + "+merge"), keep("fmha_decode_gqa_split_entry__" + v + "_merge"), IMG_FMHA, 256,
+            (uint32_t)(4 * 2 * 32 * d * 2), grp, 0, d, 0, "f16", 0, 3);
     }
   // the batched-layout form of the matrix-core kernel: one workgroup per (batch, KV head, split)
   for (int d : {64, 128, 256})

@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -1765,12 +1766,16 @@ static bool decode_vec_layout(const cutile_tensor_arg_t& t) {
   return t.strides[2] == 1 && t.strides[1] % 8 == 0 && t.strides[0] % 8 == 0 && aligned16(t.ptr);
 }
 
-cutile_status_t cutile_launch_fmha_decode_gqa_split(cutile_stream_t stream, const cutile_tensor_arg_t* q,
-                                                    const cutile_tensor_arg_t* k, const cutile_tensor_arg_t* v,
-                                                    const cutile_partition_arg_t* att_out,
-                                                    const cutile_partition_arg_t* lse_out, float qk_scale,
-                                                    const cutile_tensor_arg_t* position_start,
-                                                    const cutile_launch_opts_t* opts) {
+// The merge that a split launch may do itself: where to, and its counters (fmha.hip, merge_if_last).
+struct MergeInto {
+  const cutile_partition_arg_t* out;
+  uint32_t* arrivals;
+  uint32_t* ahead;
+  bool merged;   // set by the launch: the kernel that it took has the merge
+};
+static cutile_status_t launch_decode_split(cutile_stream_t stream, const cutile_tensor_arg_t* q, const cutile_tensor_arg_t* k, const cutile_tensor_arg_t* v,
+                                           const cutile_partition_arg_t* att_out, const cutile_partition_arg_t* lse_out, float qk_scale,
+                                           const cutile_tensor_arg_t* position_start, const cutile_launch_opts_t* opts, MergeInto* merge) {
   if (cutile_status_t s = check_tensor(q, "q", 3, 3)) return s;
   if (cutile_status_t s = check_tensor(k, "k", 3, 3)) return s;
   if (cutile_status_t s = check_tensor(v, "v", 3, 3)) return s;
@@ -1816,6 +1821,10 @@ cutile_status_t cutile_launch_fmha_decode_gqa_split(cutile_stream_t stream, cons
                  list_variants("fmha_decode_gqa_split").c_str());
   Resolved res;
   if (cutile_status_t s = resolve_entry("fmha_decode_gqa_split", opts, acceptable[0], acceptable, &res)) return s;
+  if (const KernelEntry* e = merge ? member_of(res.entry, "+merge") : nullptr) {
+    if (cutile_status_t s = use_member(&res, e)) return s;
+    merge->merged = true;
+  }
   ArgPacker args;
   args.push_tensor(*q);
   args.push_tensor(*k);
@@ -1826,8 +1835,22 @@ cutile_status_t cutile_launch_fmha_decode_gqa_split(cutile_stream_t stream, cons
   args.push_val<const void*>(position_start->ptr);
   args.push_val<int32_t>(bn);
   args.push_tile_grid(tg);
+  if (merge && merge->merged) {
+    args.push_partition(*merge->out);
+    args.push_val<void*>(merge->arrivals);
+    args.push_val<void*>(merge->ahead);
+  }
   uint32_t grid[3] = {std::min<uint32_t>(tg[0], (uint32_t)kv_heads), tg[1], 1};
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
+}
+
+cutile_status_t cutile_launch_fmha_decode_gqa_split(cutile_stream_t stream, const cutile_tensor_arg_t* q,
+                                                    const cutile_tensor_arg_t* k, const cutile_tensor_arg_t* v,
+                                                    const cutile_partition_arg_t* att_out,
+                                                    const cutile_partition_arg_t* lse_out, float qk_scale,
+                                                    const cutile_tensor_arg_t* position_start,
+                                                    const cutile_launch_opts_t* opts) {
+  return launch_decode_split(stream, q, k, v, att_out, lse_out, qk_scale, position_start, opts, nullptr);
 }
 
 cutile_status_t cutile_launch_attention_decode_kernel_grouped_f16(
@@ -1906,9 +1929,8 @@ cutile_status_t cutile_launch_attention_decode_kernel_grouped_f16(
   return launch_packed(res.fn, tg, res.entry->block, 0, stream, args);
 }
 
-cutile_status_t cutile_launch_splitk_reduce_merge(cutile_stream_t stream, const cutile_tensor_arg_t* att_partial,
-                                                  const cutile_tensor_arg_t* lse_partial, const cutile_partition_arg_t* out,
-                                                  const cutile_launch_opts_t* opts) {
+static cutile_status_t check_merge(const cutile_tensor_arg_t* att_partial, const cutile_tensor_arg_t* lse_partial, const cutile_partition_arg_t* out,
+                                   const cutile_launch_opts_t* opts, uint32_t tg[3]) {
   if (cutile_status_t s = check_tensor(att_partial, "att_partial", 3, 3)) return s;
   if (cutile_status_t s = check_tensor(lse_partial, "lse_partial", 2, 2)) return s;
   if (cutile_status_t s = check_partition(out, "out", 3, 3)) return s;
@@ -1928,9 +1950,18 @@ cutile_status_t cutile_launch_splitk_reduce_merge(cutile_stream_t stream, const 
   if (cutile_status_t s = check_generic(opts, 1, std::to_string(d), "D")) return s;
   if (cutile_status_t s = check_generic(opts, 2, std::to_string(chunk), "CHUNK_D")) return s;
   if (cutile_status_t s = check_generic(opts, 3, std::to_string(att_partial->shape[1] / group), "NUM_KV_SPLITS")) return s;
-  uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   CUTILE_REQUIRE((int64_t)tg[2] * chunk >= d, CUTILE_ERR_KERNEL_LAUNCH, "splitk_reduce_merge: the launch grid must cover all of D");
+  return CUTILE_SUCCESS;
+}
+
+cutile_status_t cutile_launch_splitk_reduce_merge(cutile_stream_t stream, const cutile_tensor_arg_t* att_partial,
+                                                  const cutile_tensor_arg_t* lse_partial, const cutile_partition_arg_t* out,
+                                                  const cutile_launch_opts_t* opts) {
+  uint32_t tg[3];
+  if (cutile_status_t s = check_merge(att_partial, lse_partial, out, opts, tg)) return s;
+  const cutile_tensor_arg_t& ot = out->tensor;
+  const int32_t group = ot.shape[1];
   Resolved res;
   if (cutile_status_t s = resolve_entry("splitk_reduce_merge", opts, "f16", {"f16"}, &res)) return s;
   ArgPacker args;
@@ -1953,7 +1984,7 @@ static std::mutex g_scratch_mutex;
 static scratch_lookup_fn g_scratch_lookup = nullptr;
 static std::string g_scratch_error;
 
-static cutile_status_t scratch_memory(void** ptr, size_t* bytes) {
+static cutile_status_t scratch_memory(void** ptr, size_t* bytes, int* ordinal) {
   if (cutile_status_t s = ensure_init()) return s;
   CUTILE_API_OR_RETURN(api);
   (void)api;
@@ -1980,8 +2011,7 @@ static cutile_status_t scratch_memory(void** ptr, size_t* bytes) {
     fn = g_scratch_lookup;
     if (!fn) return fail(CUTILE_ERR_LIBRARY_INIT, "shared object init failed: %s", g_scratch_error.c_str());
   }
-  int ordinal = -1;
-  const int err = fn(ptr, bytes, &ordinal);
+  const int err = fn(ptr, bytes, ordinal);
   if (err != 0) return from_hip((hipError_t)err, "hipGetSymbolAddress(scratch)");
   return CUTILE_SUCCESS;
 }
@@ -1990,6 +2020,12 @@ cutile_status_t cutile_scratch_capacity(size_t* bytes) {
   CUTILE_REQUIRE(bytes, CUTILE_ERR_INVALID_ARGUMENT, "null argument");
   *bytes = CUTILE_SCRATCH_BYTES;
   return CUTILE_SUCCESS;
+}
+
+// The splits of a launch that its own workgroups merge (fmha.hip, merge_if_last): a lane to a split, a counter to a head, 16-byte stores of out.
+static bool merges_in_split(const cutile_partition_arg_t& out, int32_t kv_heads, int32_t splits) {
+  const cutile_tensor_arg_t& t = out.tensor;
+  return splits <= 64 && kv_heads <= (int32_t)CUTILE_SCRATCH_HEADS && decode_vec_layout(t);
 }
 
 cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, const cutile_tensor_arg_t* q,
@@ -2015,7 +2051,8 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
                  kv_heads, num_kv_splits, group, d, (unsigned long long)need, (unsigned)CUTILE_SCRATCH_BYTES);
   void* base = nullptr;
   size_t capacity = 0;
-  if (cutile_status_t s = scratch_memory(&base, &capacity)) return s;
+  int ordinal = 0;
+  if (cutile_status_t s = scratch_memory(&base, &capacity, &ordinal)) return s;
   CUTILE_REQUIRE(base && need <= capacity, CUTILE_ERR_STATE, "fmha_decode_gqa_noalloc: scratch lookup returned %zu bytes", capacity);
   const int32_t sg = num_kv_splits * group;
   cutile_partition_arg_t att;
@@ -2044,8 +2081,28 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
   split_opts.n_generics = 4;
   // Every (head, split) workgroup of the split kernel writes its GROUP rows and log-sum-exp values, an empty split
   // included, so nothing in the scratch has to start at zero and what an earlier call left there is never read.
-  if (cutile_status_t s = cutile_launch_fmha_decode_gqa_split(stream, q, k, v, &att, &lse, qk_scale, position_start, &split_opts)) return s;
-  return cutile_launch_splitk_reduce_merge(stream, &att.tensor, &lse.tensor, out, nullptr);
+  uint32_t merge_grid[3];
+  if (cutile_status_t s = check_merge(&att.tensor, &lse.tensor, out, nullptr, merge_grid)) return s;
+  MergeInto merge{out, nullptr, nullptr, false};
+  bool together = merges_in_split(*out, kv_heads, num_kv_splits);
+  if (together && g_launch_mode == 0) {
+    // A captured launch takes the two kernels, which leave nothing behind: a graph may be replayed beside other work.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    CUTILE_API_OR_RETURN(api);
+    if (api->hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess) {
+      api->hipGetLastError();   // the launch itself will say why
+      together = false;
+    }
+    together = together && capture == hipStreamCaptureStatusNone;
+    static std::atomic<uint32_t> turn[64];   // per device; half of the sets lie between a launch's own and the one that it clears
+    const uint32_t n = turn[ordinal & 63].fetch_add(1, std::memory_order_relaxed);
+    uint32_t* const counters = (uint32_t*)((char*)base + CUTILE_SCRATCH_BYTES);
+    merge.arrivals = counters + n % CUTILE_SCRATCH_REGIONS * CUTILE_SCRATCH_HEADS;
+    merge.ahead = counters + (n + CUTILE_SCRATCH_REGIONS / 2) % CUTILE_SCRATCH_REGIONS * CUTILE_SCRATCH_HEADS;
+  }
+  if (cutile_status_t s = launch_decode_split(stream, q, k, v, &att, &lse, qk_scale, position_start, &split_opts, together ? &merge : nullptr)) return s;
+  if (merge.merged && g_launch_mode == 0) return CUTILE_SUCCESS;
+  return cutile_launch_splitk_reduce_merge(stream, &att.tensor, &lse.tensor, out, nullptr);   // (without a launch: the code object of a captured call)
 }
 
 // Everything the entry point above does once per device and shape — opening the side library, the symbol lookup

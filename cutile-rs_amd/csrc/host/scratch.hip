@@ -18,7 +18,7 @@
 
 #include "scratch.h"
 
-static __device__ __align__(256) unsigned char scratch[CUTILE_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[CUTILE_SCRATCH_BYTES + CUTILE_SCRATCH_COUNTER_BYTES];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -44,7 +44,7 @@ extern "C" int cutile_scratch_lookup(void** device_ptr, size_t* bytes, int* devi
     size_t n = 0;
     err = hipGetSymbolSize(&n, HIP_SYMBOL(scratch));
     if (err != hipSuccess) return (int)err;
-    if (n != (size_t)CUTILE_SCRATCH_BYTES) return (int)hipErrorInvalidSymbol;
+    if (n != (size_t)CUTILE_SCRATCH_BYTES + CUTILE_SCRATCH_COUNTER_BYTES) return (int)hipErrorInvalidSymbol;
     g_ptr[dev] = p;
   }
   *device_ptr = g_ptr[dev];

@@ -32,6 +32,7 @@
 #include "fmha_common.h"
 #include "kernel_args.h"
 #include "lane_exchange.h"
+#include "split_k.h"
 
 namespace {
 
@@ -749,9 +750,24 @@ __device__ __forceinline__ void load_row(const _Float16* p, uint32_t (&dst)[W]) 
 }
 constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
 constexpr int kNontemporal = 2;     // cache-policy operand of buffer loads: the nt bit
+// partial results: for a later launch, or (MERGED) for a workgroup of this one on any XCD
+template <bool MERGED>
+__device__ __forceinline__ void store_part(_Float16* p, f16x4 v) {
+  if constexpr (MERGED)
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    *reinterpret_cast<f16x4*>(p) = v;
+}
+template <bool MERGED>
+__device__ __forceinline__ void store_lse(float* p, float v) {
+  if constexpr (MERGED)
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    *p = v;
+}
 }  // namespace decode
 
-template <int G, int D>
+template <int G, int D, bool MERGED = false>
 __device__ __forceinline__ void decode_split(const TensorArg<3>& q, const TensorArg<3>& k, const TensorArg<3>& v,
                                              const PartitionArg<3>& att_out, const PartitionArg<2>& lse_out,
                                              float qk_scale, const uint32_t* pos_dev, int32_t bn, const TileGrid& g) {
@@ -921,9 +937,9 @@ __device__ __forceinline__ void decode_split(const TensorArg<3>& q, const Tensor
         f16x4 o;
 #pragma unroll
         for (int j = 0; j < 4; ++j) o[j] = (_Float16)(at[e + j] / safe);
-        *reinterpret_cast<f16x4*>(dst + e) = o;
+        store_part<MERGED>(dst + e, o);
       }
-      if (dl == 0) lb[orow * lse_out.strides[1]] = mt + __builtin_log2f(safe);
+      if (dl == 0) store_lse<MERGED>(lb + orow * lse_out.strides[1], mt + __builtin_log2f(safe));
     }
   }
 }
@@ -959,8 +975,9 @@ struct DecodeSplitView {
   float empty_lse;
 };
 
-template <int G, int D>
-__device__ __forceinline__ void decode_split_mfma_view(const DecodeSplitView& w, float qk_scale) {
+// MERGED: the partial result goes past the L2 for the workgroup that merges the splits of the head; returns the LDS that is free by then.
+template <int G, int D, bool MERGED>
+__device__ __forceinline__ unsigned char* decode_split_mfma_view(const DecodeSplitView& w, float qk_scale) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   constexpr int kWaves = 4, kSlab = 32;
   constexpr int QS = D / 32;                 // K slices of the first product
@@ -1024,7 +1041,7 @@ __device__ __forceinline__ void decode_split_mfma_view(const DecodeSplitView& w,
 #pragma unroll
   for (int i = 0; i < OS; ++i) oacc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  auto slab = [&](int32_t base, const f16x8 (&kreg)[2][QS], const unsigned char* stage) {
+  auto slab = [&](int32_t base, const f16x8 (&kreg)[2][QS], const unsigned char* stage, auto in_flight) {
     f32x4 sc[2];
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
@@ -1060,9 +1077,9 @@ __device__ __forceinline__ void decode_split_mfma_view(const DecodeSplitView& w,
       for (int i = 0; i < OS; ++i) oacc[i] *= alpha;
     }
     m = m_new;
-    // this slab's V rows (requested one slab ago) have landed once at most the 2 QS + kVInstr loads
-    // of the slab requested after them are outstanding
-    __builtin_amdgcn_s_waitcnt(0x0f70 | ((2 * QS + kVInstr) & 15) | ((((2 * QS + kVInstr) >> 4) & 3) << 14));
+    // this slab's V rows (requested one slab ago) have landed once at most the loads of the slab requested after them are outstanding
+    constexpr int kLater = decltype(in_flight)::value;
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (kLater & 15) | (((kLater >> 4) & 3) << 14));
 #pragma unroll
     for (int i = 0; i < OS; ++i) {
       // slice i lies 2 i chunks further; chunk numbers are XOR-swizzled, so the offset is an XOR too
@@ -1076,12 +1093,19 @@ __device__ __forceinline__ void decode_split_mfma_view(const DecodeSplitView& w,
   f16x8 ka[2][QS], kbuf[2][QS];
   const int32_t first = r0 + wave * kSlab, stride = kWaves * kSlab;
   if (first < r1) {
+    // A single slab is followed by no request where splits are short by design (4096 keys in 32 splits are a slab to a wavefront).  The batched kernel and large groups have long ones, whose loop pays for such a branch: 79.4 us became 80.2 at 64 heads of
+    // 16384 keys, and 84 with branches in the loop.
+    const std::integral_constant<int, 2 * QS + kVInstr> one_more;
     request_slab(first, ka, my_stage[0]);
-    for (int32_t base = first; base < r1; base += 2 * stride) {      // wavefront-uniform; slabs past r1 are masked
-      request_slab(base + stride, kbuf, my_stage[1]);
-      slab(base, ka, my_stage[0]);
-      request_slab(base + 2 * stride, ka, my_stage[0]);
-      slab(base + stride, kbuf, my_stage[1]);
+    if (MERGED && first + stride >= r1) {
+      slab(first, ka, my_stage[0], std::integral_constant<int, 0>{});
+    } else {
+      for (int32_t base = first; base < r1; base += 2 * stride) {      // wavefront-uniform; slabs past r1 are masked
+        request_slab(base + stride, kbuf, my_stage[1]);
+        slab(base, ka, my_stage[0], one_more);
+        request_slab(base + 2 * stride, ka, my_stage[0]);
+        slab(base + stride, kbuf, my_stage[1], one_more);
+      }
     }
   }
   __builtin_amdgcn_s_waitcnt(0);
@@ -1122,17 +1146,18 @@ __device__ __forceinline__ void decode_split_mfma_view(const DecodeSplitView& w,
       f16x4 o;
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = (_Float16)(a[j] / safe);
-      *reinterpret_cast<f16x4*>(dst + i * 16 + quad * 4) = o;
+      decode::store_part<MERGED>(dst + i * 16 + quad * 4, o);
     }
-    if (quad == 0) w.lse[(int64_t)col * w.lse_row_stride] = r0 >= r1 ? w.empty_lse : mt + __builtin_log2f(safe);
+    if (quad == 0) decode::store_lse<MERGED>(w.lse + (int64_t)col * w.lse_row_stride, r0 >= r1 ? w.empty_lse : mt + __builtin_log2f(safe));
   }
+  return &vst[0][0][0];
 }
 
 // fmha_decode_gqa_split: q [kv_heads, GROUP, D], k and v [kv_heads, max_seq, D], partial results at row
 // split * GROUP + c of att_out [kv_heads, splits * GROUP, D] and lse_out [kv_heads, splits * GROUP]; the tiles of
 // `bn` keys are dealt to the splits in equal runs.
-template <int G, int D>
-__device__ __forceinline__ void decode_split_mfma(const TensorArg<3>& q, const TensorArg<3>& k, const TensorArg<3>& v,
+template <int G, int D, bool MERGED = false>
+__device__ __forceinline__ unsigned char* decode_split_mfma(const TensorArg<3>& q, const TensorArg<3>& k, const TensorArg<3>& v,
                                                   const PartitionArg<3>& att_out, const PartitionArg<2>& lse_out,
                                                   float qk_scale, const uint32_t* pos_dev, int32_t bn, const TileGrid& g) {
   const int32_t head = blockIdx.x, split = blockIdx.y, splits = (int32_t)g.y;
@@ -1153,7 +1178,7 @@ __device__ __forceinline__ void decode_split_mfma(const TensorArg<3>& q, const T
   w.att_row_stride = att_out.strides[1], w.lse_row_stride = lse_out.strides[1];
   w.empty_sum = (float)bn;
   w.empty_lse = -1.0e30f + __builtin_log2f((float)bn);
-  decode_split_mfma_view<G, D>(w, qk_scale);
+  return decode_split_mfma_view<G, D, MERGED>(w, qk_scale);
 }
 
 // attention_decode_kernel_grouped (cutile-kernels/src/experimental/attention.rs:385-846): the same partial attention in
@@ -1192,7 +1217,7 @@ __device__ __forceinline__ void decode_grouped(const GroupedDecodeArgs& a, const
   w.att_row_stride = a.att_strides[2], w.lse_row_stride = a.lse_strides[2];
   w.empty_sum = 1.0f;
   w.empty_lse = -INFINITY;
-  decode_split_mfma_view<G, D>(w, a.softmax_scale);
+  decode_split_mfma_view<G, D, false>(w, a.softmax_scale);
 }
 
 // out[h, g, :] = sum_s w[g, s] att[h, s*GROUP + g, :], w = exp2(lse - max_s lse) / max(sum, 1e-8).
@@ -1273,6 +1298,106 @@ __device__ __forceinline__ void splitk_merge(const TensorArg<3>& att, const Tens
         *reinterpret_cast<f16x8*>(ob + cidx * 8) = o;
       } else {
         ob[(int64_t)cidx * out.strides[2]] = (_Float16)a[0];
+      }
+    }
+  }
+}
+
+// Split and merge in one launch, up to GROUP 4: the workgroup that stores the last partial result of a KV head merges all of them.  A merge
+// of its own is a launch behind a launch.  Us a pass, two launches and one, keys dealt to 256 workgroups: 8 heads of GROUP 4, D = 128, 300 keys
+// 10.5 and 7.9, 4096 13.2 and 11.6, 131072 85.0 and 83.0; 4 heads of GROUP 2, D = 64, 300 keys 9.9 and 6.0, 16384 12.1 and 10.3.  Larger groups
+// keep the two, where every query head has a workgroup to merge it (GROUP 8, 8 heads, D = 128: 16384 keys 20.3 and 21.4).
+// `arrivals` counts the workgroups of a head, one counter each, and is 0 before and after; the counters of `ahead`, which another launch will
+// use, are cleared, so that what launches that overlapped (two streams: not allowed) may have left in them does not last.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+constexpr int kMostMerged = 64;   // splits (a lane each) and heads (counters)
+struct MergeArgs {
+  PartitionArg<3> out;
+  uint32_t* arrivals;
+  uint32_t* ahead;
+};
+
+// The sums of splitk_merge, value by value and in the same order: row r of 256 / (D / 8) takes the splits r, r + rows, ..., and the rows are added up.
+template <int G, int D>
+__device__ __forceinline__ void merge_if_last(const PartitionArg<3>& att, const PartitionArg<2>& lse, const MergeArgs& a, unsigned char* lds, int32_t splits) {
+  constexpr int kChunks = D / 8, kRows = 256 / kChunks, kMine = kMostMerged / kRows;    // 16-byte chunks of a row; rows; splits of a thread
+  constexpr int kAtOnce = G < 16 / kMine ? G : 16 / kMine;                              // query heads whose partials are read together
+  constexpr int kSums = kAtOnce < D / 32 ? kAtOnce : D / 32;                            // ... and whose sums lie in LDS together
+  static_assert(G % kAtOnce == 0 && kAtOnce % kSums == 0, "query heads in equal shares");
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, head = blockIdx.x;
+  if (head == 0 && blockIdx.y == 0 && tid < kMostMerged) __hip_atomic_store(a.ahead + tid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!gemm::last_to_arrive(a.arrivals + head, (uint32_t)splits, reinterpret_cast<uint32_t*>(lds))) return;
+  __syncthreads();
+  float* const weight = reinterpret_cast<float*>(lds);                                  // [G][kMostMerged]
+  float* const part = weight + G * kMostMerged;                                         // [kSums][256][8]
+  const float* const lb = (const float*)lse.ptr + (int64_t)head * lse.strides[0];
+  const int row = tid / kChunks, chunk = tid % kChunks;
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc((const _Float16*)att.ptr + (int64_t)head * att.strides[0], (uint32_t)(splits * G * att.strides[1] * 2));
+  u32x4 p[kAtOnce][kMine];
+  auto fetch = [&](int g0) {
+#pragma unroll
+    for (int b = 0; b < kAtOnce; ++b)
+#pragma unroll
+      for (int i = 0; i < kMine; ++i) {
+        const int s = row + i * kRows;
+        p[b][i] = __builtin_amdgcn_raw_buffer_load_b128(ra, s < splits ? (uint32_t)((s * G + g0 + b) * att.strides[1] + chunk * 8) * 2 : 0x80000000u, 0, gemm::kAgentScope);
+      }
+  };
+  constexpr int kHeads = (G + 3) / 4;   // query heads whose weights a wavefront computes
+  float e[kHeads];
+#pragma unroll
+  for (int i = 0; i < kHeads; ++i)
+    e[i] = lane < splits && wave + 4 * i < G ? __hip_atomic_load(lb + (int64_t)(lane * G + wave + 4 * i) * lse.strides[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
+  fetch(0);
+#pragma unroll
+  for (int i = 0; i < kHeads; ++i) {
+    if (wave + 4 * i >= G) break;
+    float mx = e[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    const float t = lane < splits ? __builtin_amdgcn_exp2f(e[i] - mx) : 0.0f;
+    float sum = t;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    weight[(wave + 4 * i) * kMostMerged + lane] = t * (1.0f / fmaxf(sum, 1.0e-8f));
+  }
+  __syncthreads();
+  for (int g0 = 0; g0 < G; g0 += kAtOnce) {
+    if (g0 > 0) fetch(g0);
+    float v[kAtOnce][8];
+#pragma unroll
+    for (int b = 0; b < kAtOnce; ++b) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[b][e] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kMine; ++i) {
+        const int s = row + i * kRows;
+        const float w = weight[(g0 + b) * kMostMerged + s];
+        const f16x8 t = __builtin_bit_cast(f16x8, p[b][i]);
+        if (s < splits) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[b][e] = __builtin_fmaf((float)t[e], w, v[b][e]);
+        }
+      }
+    }
+#pragma unroll
+    for (int b0 = 0; b0 < kAtOnce; b0 += kSums) {
+      if (g0 + b0 > 0) __syncthreads();   // the sums before these have been read
+#pragma unroll
+      for (int b = 0; b < kSums; ++b) {
+        *reinterpret_cast<gemm::f32x4*>(part + (b * 256 + tid) * 8) = gemm::f32x4{v[b0 + b][0], v[b0 + b][1], v[b0 + b][2], v[b0 + b][3]};
+        *reinterpret_cast<gemm::f32x4*>(part + (b * 256 + tid) * 8 + 4) = gemm::f32x4{v[b0 + b][4], v[b0 + b][5], v[b0 + b][6], v[b0 + b][7]};
+      }
+      __syncthreads();
+      for (int o = tid; o < kSums * D / 2; o += 256) {   // two neighbouring outputs a thread
+        const int b = o / (D / 2), c = o % (D / 2) * 2;
+        f32x2 r[kRows];
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) r[k] = *reinterpret_cast<const f32x2*>(part + b * 2048 + k * D + c);
+        float lo = r[0][0], hi = r[0][1];
+#pragma unroll
+        for (int k = 1; k < kRows; ++k) lo += r[k][0], hi += r[k][1];
+        *reinterpret_cast<decode::h2*>((_Float16*)a.out.ptr + (int64_t)head * a.out.strides[0] + (int64_t)(g0 + b0 + b) * a.out.strides[1] + c) = decode::h2{(_Float16)lo, (_Float16)hi};
       }
     }
   }
@@ -1372,6 +1497,34 @@ DECODE_SPLIT_MFMA_KERNEL(8, 256)
 DECODE_SPLIT_MFMA_KERNEL(16, 64)
 DECODE_SPLIT_MFMA_KERNEL(16, 128)
 DECODE_SPLIT_MFMA_KERNEL(16, 256)
+
+// The same with the merge behind it, for the kernel that the launcher takes for (GROUP, D) when nobody names one.
+#define DECODE_MERGED_KERNEL(G, D)                                                                 \
+  extern "C" __global__ void __launch_bounds__(256)                                               \
+      fmha_decode_gqa_split_entry__f16_g##G##_d##D##_merge(TensorArg<3> q, TensorArg<3> k, TensorArg<3> v, \
+                                                           PartitionArg<3> att_out, PartitionArg<2> lse_out, \
+                                                           float qk_scale, const uint32_t* position_start, \
+                                                           int32_t bn, TileGrid g, MergeArgs m) {  \
+    __shared__ __attribute__((aligned(16))) unsigned char lds[G * kMostMerged * 4 + G * 256 * 32]; \
+    decode_split<G, D, true>(q, k, v, att_out, lse_out, qk_scale, position_start, bn, g);         \
+    merge_if_last<G, D>(att_out, lse_out, m, lds, (int32_t)g.y);                                   \
+  }
+#define DECODE_MERGED_MFMA_KERNEL(G, D)                                                            \
+  extern "C" __global__ void __launch_bounds__(256)                                               \
+      fmha_decode_gqa_split_entry__f16_g##G##_d##D##_mfma_merge(TensorArg<3> q, TensorArg<3> k, TensorArg<3> v, \
+                                                                PartitionArg<3> att_out, PartitionArg<2> lse_out, \
+                                                                float qk_scale, const uint32_t* position_start, \
+                                                                int32_t bn, TileGrid g, MergeArgs m) { \
+    unsigned char* lds = decode_split_mfma<G, D, true>(q, k, v, att_out, lse_out, qk_scale, position_start, bn, g); \
+    merge_if_last<G, D>(att_out, lse_out, m, lds, (int32_t)g.y);                                   \
+  }
+DECODE_MERGED_KERNEL(1, 128)
+DECODE_MERGED_KERNEL(2, 128)
+DECODE_MERGED_MFMA_KERNEL(4, 128)
+#define DECODE_MERGED_MFMA_GROUPS(D) \
+  DECODE_MERGED_MFMA_KERNEL(1, D) DECODE_MERGED_MFMA_KERNEL(2, D) DECODE_MERGED_MFMA_KERNEL(4, D)
+DECODE_MERGED_MFMA_GROUPS(64)
+DECODE_MERGED_MFMA_GROUPS(256)
 
 #define DECODE_GROUPED_KERNEL(G, D)                                                                \
   extern "C" __global__ void __launch_bounds__(256)                                               \

@@ -571,7 +571,9 @@ cutile_status_t cutile_launch_splitk_reduce_merge(cutile_stream_t stream, const 
  * the process ends.  A call that needs more fails with CUTILE_ERR_KERNEL_LAUNCH before any GPU work.  No device memory
  * is allocated or freed, here or in the kernels.  Every call on one GPU uses that GPU's one array: calls that overlap
  * on one GPU (two streams, two threads) race; calls on one stream are ordered.  Nothing in the array has to start
- * at zero — the split kernel writes every row a merge reads — so nothing is cleared between calls. */
+ * at zero — the split kernel writes every row a merge reads — so nothing is cleared between calls.  Up to GROUP 4, 64
+ * heads and 64 splits the call is one launch, whose workgroups count in 16 KiB behind the array (zeros between
+ * launches); while the stream is being captured, and beyond, it is two. */
 cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, const cutile_tensor_arg_t* q,
                                                       const cutile_tensor_arg_t* k, const cutile_tensor_arg_t* v,
                                                       const cutile_partition_arg_t* out, float qk_scale,
@@ -582,7 +584,7 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
  * 8 MiB then) and loads two code objects: work that is neither allocation-free nor legal while a stream is being
  * captured.  This call does all of it and enqueues nothing (the entry point in compile-only mode: the arguments are
  * checked exactly as a launch checks them, no pointer is dereferenced).  Call it once per device and shape outside any
- * capture; after it, cutile_launch_fmha_decode_gqa_noalloc with the same shapes only enqueues two kernels. */
+ * capture; after it, cutile_launch_fmha_decode_gqa_noalloc with the same shapes only enqueues one kernel or two. */
 cutile_status_t cutile_fmha_decode_gqa_noalloc_prepare(const cutile_tensor_arg_t* q, const cutile_tensor_arg_t* k,
                                                        const cutile_tensor_arg_t* v, const cutile_partition_arg_t* out,
                                                        const cutile_tensor_arg_t* position_start, int32_t num_kv_splits,
