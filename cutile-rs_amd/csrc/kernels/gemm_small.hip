@@ -19,8 +19,12 @@ namespace {
 // ---- medium sizes: register-staged tiles, K split over workgroups -------------------------------------------------------
 // For the outputs that are too few 256 x 256 tiles to fill the chip, and for rows that do not start on 16-byte boundaries
 // (the direct global -> LDS fetches of gemm_bf16.hip cannot take those).  K tiles of 64 go global -> registers -> LDS: two
-// tiles are in flight in registers while a third is multiplied out of one of two LDS stages, so a load has two K tiles to
-// land and one barrier per K tile is enough.  Several workgroups may share the K tiles of a 64 x 64 output tile (SPLIT).
+// tiles are in flight in registers while a third is multiplied out of one of two LDS stages.  The next tile is written to the other stage
+// between the MFMAs of the first K step of 32, the one barrier lies between the two steps, and behind it the registers are loaded again: no
+// phase of a K tile is without MFMAs, and the fragments of a step are read during the one before it.  Against phases of their own (multiply,
+// write, load, barrier), us: f16 336 x 2575 x 1350 17.2 -> 14.6, 215 x 256 x 14720 21.8 -> 15.0, 1846 x 12923 x 374 50.9 -> 42.5; bf16 961 x 7277 x
+// 2155 54.1 -> 44.0, 3136 x 1941 x 5340 99.6 -> 85.6.  With both operands unaligned a 128-byte piece of a row of x lies in two cache lines, which
+// the vector cache does not hold until the next K tile: 2749 x 2583 x 8862 stays at 184.  Several workgroups may share the K tiles of a 64 x 64 output tile (SPLIT).
 template <int BM, int BN, int WAVES_M, int WAVES_N, typename OutT, typename InT>
 struct GemmStaged {
   static constexpr bool SPLIT = BM == 64 && BN == 64;   // the tile that the launcher splits (staged_splits)
@@ -60,7 +64,7 @@ struct GemmStaged {
     const int64_t lda = (int64_t)x.strides[0] * 2, ldb = (int64_t)y.strides[0] * 2;   // bytes
     const int32_t k_valid = min(min(x.shape[1], y.shape[0]), k_total);
     const int32_t row0 = pm * BM, col_first = pn * BN, col0 = max(0, min(col_first, N - BN));   // the last column of tiles is moved back into y
-    const int32_t full = k_valid / BK, kt0 = (int32_t)((int64_t)full * split / splits), kt1 = (int32_t)((int64_t)full * (split + 1) / splits);
+    const int32_t k_tiles = (k_valid + BK - 1) / BK, kt0 = (int32_t)((int64_t)k_tiles * split / splits), kt1 = (int32_t)((int64_t)k_tiles * (split + 1) / splits);
 
     // per-lane byte offsets of the loads (operands end below 2 GiB; the K advance is scalar) and of the LDS writes
     static_assert(kThreads % 16 == 0 && kThreads / 8 % 16 == 0 && kThreads / UB % 16 == 0, "the swizzle terms repeat from load to load");
@@ -77,20 +81,64 @@ struct GemmStaged {
     struct Tile {
       u32x4 a[kALoads], b[kBLoads];
     };
-    auto fetch = [&](Tile& t, int32_t kt) {
+    auto fetch_one = [&](Tile& t, int32_t kt, int i) {
       const int32_t k0 = kt * BK;
-#pragma unroll
-      for (int i = 0; i < kALoads; ++i) t.a[i] = load16(xp + (int64_t)k0 * 2 + a_off[i]);
-#pragma unroll
-      for (int i = 0; i < kBLoads; ++i) t.b[i] = load16(yp + k0 * ldb + i * b_next + b_off);
+      if (i < kALoads)
+        t.a[i] = load16(xp + (int64_t)k0 * 2 + a_off[i]);
+      else
+        t.b[i - kALoads] = load16(yp + k0 * ldb + (i - kALoads) * b_next + b_off);
     };
-    auto stage = [&](const Tile& t, unsigned char* s) {
+    // The last K tile: K positions past the end are 0 on both sides.  Every unit of x is read where it lies inside K: one that the end cuts is read
+    // so that it ends there, and shifted; y rows past the end repeat the last one, and give way to zeros.
+    auto fetch_last = [&](Tile& t, int32_t kt) {
+      const int32_t k0 = kt * BK, rest = k_valid - k0, cut = rest % 8;
+      const bool whole = a_k + 8 <= rest, part = !whole && a_k < rest;
+      const int32_t at = whole ? k0 : k_valid - 8 - a_k;
 #pragma unroll
-      for (int i = 0; i < kALoads; ++i) *reinterpret_cast<u32x4*>(s + a_st + i * (kThreads * 16)) = t.a[i];
+      for (int i = 0; i < kALoads; ++i) {
+        if (k_valid >= 8) {
+          t.a[i] = load16(xp + a_off[i] + at * 2);
+        } else {
+          uint32_t o[4] = {0, 0, 0, 0};
+          for (int e = 0; e < k_valid; ++e) {
+            const uint32_t v = reinterpret_cast<const uint16_t*>(xp + a_off[i] - a_k * 2)[e];
 #pragma unroll
-      for (int i = 0; i < kBLoads; ++i) *reinterpret_cast<u32x4*>(s + b_st + i * (kThreads * 16)) = t.b[i];
+            for (int d = 0; d < 4; ++d)
+              if (e / 2 == d) o[d] |= v << (e % 2 * 16);
+          }
+          t.a[i] = u32x4{o[0], o[1], o[2], o[3]};
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < kBLoads; ++i)
+        t.b[i] = load16(yp + (int64_t)(k0 + min(b_r + i * (kThreads / UB), rest - 1)) * ldb + (b_off - (uint32_t)(b_r * ldb)));
+      const int by = k_valid >= 8 ? (8 - cut) * 16 : 0;   // bits that a cut unit was read too early, 16 to 112
+#pragma unroll
+      for (int i = 0; i < kALoads; ++i) {
+        const uint64_t lo = t.a[i].x | (uint64_t)t.a[i].y << 32, hi = t.a[i].z | (uint64_t)t.a[i].w << 32;
+        const uint64_t down = by == 0 ? lo : by < 64 ? lo >> by | hi << (64 - by) : hi >> (by - 64), up = by < 64 ? hi >> by : 0;
+        const uint64_t nlo = whole ? lo : part ? down : 0, nhi = whole ? hi : part ? up : 0;
+        t.a[i] = u32x4{(uint32_t)nlo, (uint32_t)(nlo >> 32), (uint32_t)nhi, (uint32_t)(nhi >> 32)};
+      }
+#pragma unroll
+      for (int i = 0; i < kBLoads; ++i)
+        if (b_r + i * (kThreads / UB) >= rest) t.b[i] = u32x4{0, 0, 0, 0};
     };
-
+    auto fetch = [&](Tile& t, int32_t kt) {
+      if (kt >= kt1) return;
+      if (kt == k_tiles - 1) {
+        fetch_last(t, kt);
+      } else {
+#pragma unroll
+        for (int i = 0; i < kALoads + kBLoads; ++i) fetch_one(t, kt, i);
+      }
+    };
+    auto stage_one = [&](const Tile& t, unsigned char* s, int i) {
+      if (i < kALoads)
+        *reinterpret_cast<u32x4*>(s + a_st + i * (kThreads * 16)) = t.a[i];
+      else
+        *reinterpret_cast<u32x4*>(s + b_st + (i - kALoads) * (kThreads * 16)) = t.b[i - kALoads];
+    };
     const int tr_row = l16 >> 2, tr_col = (l16 & 3) * 4;
     int a_addr[2], b_addr[TN];
 #pragma unroll
@@ -105,75 +153,77 @@ struct GemmStaged {
     for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto multiply = [&](const unsigned char* s) {
+    struct Frags {
+      bf16x8 a[TM], b[TN];
+    };
+    auto read = [&](const unsigned char* s, int ks, Frags& f, int i) {   // the y fragments and the first x fragment are needed first
+      if (i < TN) {
+        const unsigned char* p = s + b_addr[i] + ks * 32 * (BN * 2);
+        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))p);
+        s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(p + 4 * (BN * 2)));
+        f.b[i] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      } else {
+        f.a[i - TN] = *reinterpret_cast<const bf16x8*>(s + a_addr[ks] + (i - TN) * (16 * BK * 2));
+      }
+    };
+    // The MFMAs of a K step, and between them (sched_barrier keeps the order written) the reads of the next step's fragments, then what
+    // moves the tiles along: writes of `t` to the stage `to`, or loads of K tile `load` into it.
+    constexpr int NB = TM * TN, kUnits = TM + TN, kMoves = kALoads + kBLoads;
+    constexpr std::integral_constant<int, 0> kNothing{};
+    constexpr std::integral_constant<int, 1> kWrite{};
+    constexpr std::integral_constant<int, 2> kLoad{};
+    auto step = [&](const Frags& f, Frags& next, const unsigned char* rd, int rd_ks, bool reads, Tile& t, auto moves, unsigned char* to, int32_t load) {
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 a[TM], b[TN];
+      for (int j = 0; j < NB; ++j) {
+        if (reads) {
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) a[tm] = *reinterpret_cast<const bf16x8*>(s + a_addr[ks] + tm * (16 * BK * 2));
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-          const unsigned char* p = s + b_addr[tn] + ks * 32 * (BN * 2);
-          s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))p);
-          s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(p + 4 * (BN * 2)));
-          b[tn] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          for (int i = 0; i < kUnits; ++i)
+            if (i * NB / kUnits == j) read(rd, rd_ks, next, i);
         }
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-          for (int tm = 0; tm < TM; ++tm) acc[tn][tm] = mfma_16x16x32<InT>(b[tn], a[tm], acc[tn][tm]);
-        __builtin_amdgcn_sched_barrier(0);   // one K step's fragments at a time
+        for (int i = 0; i < kMoves; ++i)
+          if (i * NB / kMoves == j) {
+            if constexpr (decltype(moves)::value == 1) stage_one(t, to, i);
+            if constexpr (decltype(moves)::value == 2) fetch_one(t, load, i);
+          }
+        acc[j % TN][j / TN] = mfma_16x16x32<InT>(f.b[j % TN], f.a[j / TN], acc[j % TN][j / TN]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     };
 
     unsigned char* const s0 = lds;
     unsigned char* const s1 = lds + kStageBytes;
     Tile t0, t1;
+    Frags f0, f1;
     if (kt0 < kt1) {
       fetch(t0, kt0);
-      if (kt0 + 1 < kt1) fetch(t1, kt0 + 1);
-      stage(t0, s0);
-      if (kt0 + 2 < kt1) fetch(t0, kt0 + 2);
-      __syncthreads();
-    }
-    for (int32_t kt = kt0; kt < kt1; kt += 2) {
-      multiply(s0);
-      if (kt + 1 >= kt1) break;
-      stage(t1, s1);
-      if (kt + 3 < kt1) fetch(t1, kt + 3);
-      __syncthreads();
-      multiply(s1);
-      if (kt + 2 >= kt1) break;
-      stage(t0, s0);
-      if (kt + 4 < kt1) fetch(t0, kt + 4);
-      __syncthreads();
-    }
-
-    // The ragged last K tile, straight into a stage: K positions past the end are 0 on both sides.
-    if (k_valid % BK != 0 && split == splits - 1) {
-      const int32_t k0 = full * BK;
-      __syncthreads();
-#pragma unroll 1
-      for (int c = tid; c < BM * 8; c += kThreads) {
-        const uint16_t* row = reinterpret_cast<const uint16_t*>(xp + (int64_t)min(row0 + c / 8, M - 1) * lda);
-        uint32_t h[4];
+      fetch(t1, kt0 + 1);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int32_t k = k0 + c % 8 * 8 + e;
-          const uint32_t v = k < k_valid ? row[k] : 0u;
-          h[e / 2] = e % 2 ? h[e / 2] | v << 16 : v;
-        }
-        *reinterpret_cast<u32x4*>(s0 + a_lds_off(c / 8, c % 8)) = u32x4{h[0], h[1], h[2], h[3]};
-      }
-#pragma unroll 1
-      for (int c = tid; c < BK * UB; c += kThreads) {
-        const int32_t k = k0 + c / UB;
-        u32x4 v = {0, 0, 0, 0};
-        if (k < k_valid) v = load16(yp + k * ldb + (int64_t)(col0 + c % UB * 8) * 2);
-        *reinterpret_cast<u32x4*>(s0 + kABytes + b_lds_off(c / UB, c % UB)) = v;
-      }
+      for (int i = 0; i < kMoves; ++i) stage_one(t0, s0, i);
+      fetch(t0, kt0 + 2);
       __syncthreads();
-      multiply(s0);
+#pragma unroll
+      for (int i = 0; i < kUnits; ++i) read(s0, 0, f0, i);
+    }
+    // Tile kt lies in `cur`, tile kt + 1 in the registers `t` and, behind the barrier, in `next`: every wavefront has read its last fragment of
+    // tile kt - 1 from there in front of the barrier of that tile.
+    auto k_tile = [&](unsigned char* cur, unsigned char* next, Tile& t, int32_t kt, auto loads) {
+      step(f0, f1, cur, 1, true, t, kWrite, next, 0);
+      __syncthreads();
+      step(f1, f0, next, 0, true, t, loads, next, kt + 3);
+    };
+    int32_t kt = kt0;
+    for (; kt + 5 < kt1; kt += 2) {   // (the last K tile is not loaded in here)
+      k_tile(s0, s1, t1, kt, kLoad);
+      k_tile(s1, s0, t0, kt + 1, kLoad);
+    }
+#pragma unroll 1
+    for (; kt < kt1; kt += 2) {       // (behind the last tile nothing is read that was written)
+      k_tile(s0, s1, t1, kt, kNothing);
+      if (kt + 1 >= kt1) break;
+      fetch(t1, kt + 3);
+      k_tile(s1, s0, t0, kt + 1, kNothing);
+      fetch(t0, kt + 4);
     }
 
     // Output: a pass puts kOutRows rows of the tile into the stages as f32 (16-byte chunk c of row r at chunk c ^ (r & 15)),
