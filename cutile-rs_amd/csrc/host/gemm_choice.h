@@ -14,6 +14,7 @@ struct GemmShape {
   int64_t y_cols;          // columns of y (a strip or a tile of the gemm_small.hip kernels must lie inside them)
   int32_t k;
   bool aligned;            // rows on 16-byte boundaries, whole output covered: the ring kernels can take it
+  bool x_aligned;          // the rows of x are
   bool own_tile;           // the partition's tile has kernels of its own
 };
 
@@ -179,36 +180,50 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       // bf16: the prices are good to 5 %, so only where it is the cheaper one by more)
       if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, picked = r.kernel, shares_k = p.splits > 1, c.ring = &r, c.ring_plan = p;
     }
-  // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 94 us, 200 x 50021 x 1024 bf16 587 -> 50 us), and,
+  // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 86 us, 200 x 50021 x 1024 bf16 587 -> 37 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
   if (!s.own_tile || (ring && tiles(128, 128) < (uint64_t)cus / 2)) {
-    // us per K tile: alone on a compute unit, and each of several; us of start and output.  256 x 128 fills a compute unit by itself:
-    // the fewest bytes per product, but nothing runs beside its start and its output, so it is the better one where K is long
-    // against them, and up to two rounds of workgroups (bf16, us with it, and with the best other tile: 2749 x 2583 x 8862 154, 182;
-    // 256 x 32003 x 4096 79, 91; 200 x 50021 x 1024, two rounds, 45, 47; 1000 x 20001 x 1024, three, 68, 59; 2746 x 2163 x 338 15.3, 13.6).
-    // Rows on 16-byte boundaries cost less (the second set, fitted like the ring's; the splits' share too): with the first set, ring tiles
-    // were taken for small outputs of middling K (us with ring, 64 x 64 and two-stage tiles: 220 x 64 x 1408 14.4, 9.3, 11.5; 665 x 320 x 704 9.5,
-    // 6.7, 8.2; from memory 14.6, 10.1, 14.9 and 10.2, 7.7, 10.5).  The two-stage tiles are the better ones where operands are in the
-    // caches and K is about 1500 (936 x 640 x 1536 12.7 us, ring 16.0), and the worse ones where they are not (21.6, 17.5).
+    // us per K tile: alone on a compute unit, and each of several; us of start and output, paid by every round of workgroups; the share by which x
+    // rows off 16-byte boundaries lengthen it all; us of shared K, and for each value of the partial sums.  Least squares over 140 products whose rows
+    // lie off 16-byte boundaries, operands from memory, every tile timed (10 to 13 % rms): over them the tile priced lowest takes 1.005 times the
+    // best one's time.  256 x 256 has the fewest bytes per product and pays most for start and output (bf16, us on it and on the best
+    // other: 200 x 50021 x 1024 37.3, 46.3; 1000 x 20001 x 1024 67, 62; 961 x 7277 x 2155 57, 44), with a short K in many rounds most of all (5587
+    // x 30444 x 164 240, 181 on 64 x 128: nothing runs beside a start or an output on the tiles that fill a compute unit by themselves).
+    // Rows on 16-byte boundaries cost less (the second set: a K tile alone and each of several, start and output, the splits' share).  They compete
+    // with the ring's prices, and were fitted with them, before a K tile's writes and loads lay between its MFMAs; of staged tiles that takes 10 to 30 % off, so
+    // what is chosen by them is right, and some ring tiles of few outputs would be slower by less than that than the staged ones passed over (100 x 1024
+    // x 4096 14.3 us on the ring, 11.8; 665 x 320 x 704 on these 6.8, on the ring 8.0).  With the first set for them, ring tiles were taken for small
+    // outputs of middling K (us with ring, 64 x 64 and two-stage tiles: 220 x 64 x 1408 14.4, 9.3, 11.5).
     // (0.265: with the fitted 0.257 the two K / V projections of 1500 x 1024 x 4096, 384 tiles of 64 x 64, took 42 us each, on the ring 40)
-    struct Cost { double one, more, ends, split, sum; };
-    struct StagedTile { const char* kernel; int bm, bn, per_cu; Cost any, aligned; };
-    static const StagedTile kStaged[] = {{"staged256x128", 256, 128, 1, {1.13, 1.13, 6.5, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
-                                         {"staged128x128", 128, 128, 2, {0.75, 0.62, 5.0, 0, 0}, {0.715, 0.625, 5.05, 0, 0}},
-                                         {"staged64x128", 64, 128, 3, {0.63, 0.38, 5.0, 0, 0}, {0.55, 0.43, 3.9, 0, 0}},
-                                         {"staged64x64", 64, 64, 4, {0.52, 0.235, 5.0, 6.0, 1.6e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
+    struct Any { double one, more, ends, x, split, sum; };
+    struct Aligned { double one, more, ends, split, sum; };
+    struct StagedTile { const char* kernel; int bm, bn, per_cu; Any any; Aligned aligned; };
+    static const StagedTile kStaged[] = {{"staged256x256", 256, 256, 1, {1.14, 0, 12.7, 0.126, 0, 0}, {}},
+                                         {"staged256x128", 256, 128, 1, {0.77, 0, 8.2, 0.142, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
+                                         {"staged128x128", 128, 128, 2, {0.50, 0.52, 6.7, 0.139, 0, 0}, {0.715, 0.625, 5.05, 0, 0}},
+                                         {"staged64x128", 64, 128, 3, {0.32, 0.39, 6.0, 0.074, 0, 0}, {0.55, 0.43, 3.9, 0, 0}},
+                                         {"staged64x64", 64, 64, 4, {0.228, 0.2725, 4.5, 0.046, 2.4, 2.1e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
     for (const StagedTile& r : kStaged) {
-      if (s.y_cols < r.bn) continue;
+      if (s.y_cols < r.bn || (ring && r.bn == 256)) continue;
       const uint64_t t = tiles(r.bm, r.bn), would_share = staged_splits(r.bm, r.bn, t, s.k, cus), sk = partial_bytes ? would_share : 1;
-      const double w = (double)((t * sk + cus - 1) / cus);
-      if (r.per_cu == 1 && w > 2) continue;
-      const Cost& c1 = ring ? r.aligned : r.any;
-      // (a long K that there is no room to share: 0.385 to 0.395 us a K tile, the fit knows short ones alone; captured, us on these and on 128 x 128
-      // tiles: 309 x 2240 x 5184 34.4, 31.2; 184 x 4928 x 4736 32.0, 29.1; 460 x 1792 x 2304 17.8, 17.0)
-      const double one = ring && sk < would_share ? 0.40 : c1.one;
-      const double us = kt / (double)sk * std::max(one * std::max(1.0, w / r.per_cu), c1.more * w) + c1.ends +
-                        (sk > 1 ? c1.split + c1.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      if (us < best * 0.98) best = us, picked = r.kernel, shares_k = sk > 1, c.ring = nullptr;
+      double us;
+      if (ring) {
+        const double w = (double)((t * sk + cus - 1) / cus);
+        if (r.per_cu == 1 && w > 2) continue;
+        const Aligned& a = r.aligned;
+        // (a long K that there is no room to share: priced so that 128 x 128 tiles take it)
+        const double one = sk < would_share ? 0.40 : a.one;
+        us = kt / (double)sk * std::max(one * std::max(1.0, w / r.per_cu), a.more * w) + a.ends + (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
+      } else {
+        const uint64_t slots = (uint64_t)cus * r.per_cu, rounds = t * sk / slots, rest = t * sk % slots;
+        if (r.per_cu == 1 && rounds >= 2 && kt < 8) continue;
+        const Any& a = r.any;
+        const double ends = a.ends + (r.bn == 256 && s.k % 64 != 0 ? 1.8 : 0.0);   // (there a ragged K tile stands behind the sequence)
+        auto round = [&](uint64_t each) { return kt / (double)sk * std::max(a.one, a.more * (double)each) + ends; };
+        us = ((double)rounds * round(r.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0)) * (s.x_aligned ? 1.0 : 1.0 + a.x) +
+             (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
+      }
+      if (us < best * (ring ? 0.98 : 1.0)) best = us, picked = r.kernel, shares_k = sk > 1, c.ring = nullptr;
     }
   }
   if (picked) pick(picked);

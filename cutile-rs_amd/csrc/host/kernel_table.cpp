@@ -260,9 +260,9 @@ std::vector<KernelEntry> build_table() {
     }
   // medium sizes: register-staged tiles, K split over workgroups (any alignment, any partition shape); two LDS stages
   for (const char* dt : {"bf16", "f16", "bf16f32"})
-    for (auto t : {std::array<int, 3>{64, 64, 4}, std::array<int, 3>{64, 128, 4}, std::array<int, 3>{128, 128, 4}, std::array<int, 3>{256, 128, 8}}) {
+    for (auto t : {std::array<int, 3>{64, 64, 4}, std::array<int, 3>{64, 128, 4}, std::array<int, 3>{128, 128, 4}, std::array<int, 3>{256, 128, 8}, std::array<int, 3>{256, 256, 8}}) {
       std::string v = std::string(dt) + "_staged" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
-      add("gemm", keep(v), keep("gemm_entry__" + v), IMG_GEMM_SMALL, (uint32_t)(t[2] * 64), (uint32_t)(2 * 64 * 2 * (t[0] + t[1]) + (t[0] * t[1] == 64 * 64 ? 4 : 0)), 0, t[1],
+      add("gemm", keep(v), keep("gemm_entry__" + v), t[1] == 256 ? IMG_GEMM_TILES : IMG_GEMM_SMALL, (uint32_t)(t[2] * 64), (uint32_t)(2 * 64 * 2 * (t[0] + t[1]) + (t[0] * t[1] == 64 * 64 ? 4 : 0)), 0, t[1],
           64, t[0], dt, 0, 2);
     }
 

@@ -2210,7 +2210,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   uint64_t partial_bytes = kSplitPartialBytes;
   if (row_layout) {
     if (cutile_status_t s = current_device_units(&cus)) return s;
-    const GemmShape shape{dt.c_str(), cover_m, cover_n, y->shape[1], k_valid, fast_layout && full_cover, own_tile != nullptr};
+    const bool x_aligned = aligned16(x->ptr) && x->strides[0] * (int64_t)cutile_dtype_size(x->dtype) % 16 == 0;
+    const GemmShape shape{dt.c_str(), cover_m, cover_n, y->shape[1], k_valid, fast_layout && full_cover, x_aligned, own_tile != nullptr};
     sized = choose_gemm(shape, cus, partial_bytes);
     if (sized.needs_room && g_launch_mode != 2) {
       cutile_device_t device = nullptr;

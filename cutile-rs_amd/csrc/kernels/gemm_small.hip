@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "gemm_common.h"
+#include "gemm_loose.h"
 #include "gemm_thin.h"
 #include "gemm_tiles.h"
 #include "kernel_args.h"
@@ -33,11 +34,7 @@ struct GemmStaged {
   static constexpr int UB = BN / 8;                                    // 16-byte units of a y-tile row
   static constexpr int kALoads = BM * 8 / kThreads, kBLoads = BK * UB / kThreads;
   static constexpr int kABytes = BM * BK * 2, kBBytes = BK * BN * 2, kStageBytes = kABytes + kBBytes;
-  static constexpr int kOutRows = 2 * kStageBytes / (BN * 4) < BM ? 2 * kStageBytes / (BN * 4) : BM;   // output rows the stages hold in f32
-  static constexpr int kOutPasses = (BM + kOutRows - 1) / kOutRows;
-  static constexpr int RPW = kOutRows < WM ? kOutRows : WM;
   static_assert(kALoads * kThreads == BM * 8 && kBLoads * kThreads == BK * UB && UB >= 8, "tile must split evenly");
-  static_assert(kOutRows % WM == 0 || WM % kOutRows == 0, "an output pass takes whole wavefront sub-tiles");
 
   __device__ static __forceinline__ int a_lds_off(int r, int u) { return r * (BK * 2) + ((u ^ ((r >> 1) & 7)) << 4); }
   __device__ static __forceinline__ int b_swizzle(int r) { return (((r & 3) << 2) | (((r >> 3) & 1) << 1)) & (UB - 1); }
@@ -88,15 +85,16 @@ struct GemmStaged {
       else
         t.b[i - kALoads] = load16(yp + k0 * ldb + (i - kALoads) * b_next + b_off);
     };
-    // The last K tile: K positions past the end are 0 on both sides.  Every unit of x is read where it lies inside K: one that the end cuts is read
-    // so that it ends there, and shifted; y rows past the end repeat the last one, and give way to zeros.
-    auto fetch_last = [&](Tile& t, int32_t kt) {
-      const int32_t k0 = kt * BK, rest = k_valid - k0, cut = rest % 8;
-      const bool whole = a_k + 8 <= rest, part = !whole && a_k < rest;
-      const int32_t at = whole ? k0 : k_valid - 8 - a_k;
+    // A ragged last K tile: K positions past the end are 0 on both sides.  Every unit of x is read where it lies inside K: one that the end cuts is
+    // read so that it ends there, and shifted; y rows past the end repeat the last one, and give way to zeros (trim, when the tile is written).
+    const int32_t rest = k_valid - (k_tiles - 1) * BK;
+    const bool whole = a_k + 8 <= rest, partly = !whole && a_k < rest;
+    auto ragged = [&](int32_t kt) { return __builtin_expect(kt == k_tiles - 1 && rest < BK, 0); };   // (out of the way of a short K)
+    auto fetch_ragged = [&](Tile& t) {
+      const int32_t k0 = (k_tiles - 1) * BK, at = whole ? k0 : k_valid - 8 - a_k;
 #pragma unroll
       for (int i = 0; i < kALoads; ++i) {
-        if (k_valid >= 8) {
+        if (__builtin_expect(k_valid >= 8, 1)) {
           t.a[i] = load16(xp + a_off[i] + at * 2);
         } else {
           uint32_t o[4] = {0, 0, 0, 0};
@@ -112,12 +110,14 @@ struct GemmStaged {
 #pragma unroll
       for (int i = 0; i < kBLoads; ++i)
         t.b[i] = load16(yp + (int64_t)(k0 + min(b_r + i * (kThreads / UB), rest - 1)) * ldb + (b_off - (uint32_t)(b_r * ldb)));
-      const int by = k_valid >= 8 ? (8 - cut) * 16 : 0;   // bits that a cut unit was read too early, 16 to 112
+    };
+    auto trim = [&](Tile& t) {
+      const int by = k_valid >= 8 ? (8 - rest % 8) % 8 * 16 : 0;   // bits that a cut unit was read too early, 16 to 112
 #pragma unroll
       for (int i = 0; i < kALoads; ++i) {
         const uint64_t lo = t.a[i].x | (uint64_t)t.a[i].y << 32, hi = t.a[i].z | (uint64_t)t.a[i].w << 32;
         const uint64_t down = by == 0 ? lo : by < 64 ? lo >> by | hi << (64 - by) : hi >> (by - 64), up = by < 64 ? hi >> by : 0;
-        const uint64_t nlo = whole ? lo : part ? down : 0, nhi = whole ? hi : part ? up : 0;
+        const uint64_t nlo = whole ? lo : partly ? down : 0, nhi = whole ? hi : partly ? up : 0;
         t.a[i] = u32x4{(uint32_t)nlo, (uint32_t)(nlo >> 32), (uint32_t)nhi, (uint32_t)(nhi >> 32)};
       }
 #pragma unroll
@@ -126,8 +126,8 @@ struct GemmStaged {
     };
     auto fetch = [&](Tile& t, int32_t kt) {
       if (kt >= kt1) return;
-      if (kt == k_tiles - 1) {
-        fetch_last(t, kt);
+      if (ragged(kt)) {
+        fetch_ragged(t);
       } else {
 #pragma unroll
         for (int i = 0; i < kALoads + kBLoads; ++i) fetch_one(t, kt, i);
@@ -198,6 +198,7 @@ struct GemmStaged {
     if (kt0 < kt1) {
       fetch(t0, kt0);
       fetch(t1, kt0 + 1);
+      if (ragged(kt0)) trim(t0);
 #pragma unroll
       for (int i = 0; i < kMoves; ++i) stage_one(t0, s0, i);
       fetch(t0, kt0 + 2);
@@ -219,67 +220,30 @@ struct GemmStaged {
     }
 #pragma unroll 1
     for (; kt < kt1; kt += 2) {       // (behind the last tile nothing is read that was written)
+      if (ragged(kt + 1)) trim(t1);
       k_tile(s0, s1, t1, kt, kNothing);
       if (kt + 1 >= kt1) break;
       fetch(t1, kt + 3);
+      if (ragged(kt + 2)) trim(t0);
       k_tile(s1, s0, t0, kt + 1, kNothing);
       fetch(t0, kt + 4);
     }
 
-    // Output: a pass puts kOutRows rows of the tile into the stages as f32 (16-byte chunk c of row r at chunk c ^ (r & 15)),
-    // then a thread takes 8 neighbouring columns of a row at a time: 16-byte accesses of z and of the partial sums.
-    OutT* zp = (OutT*)z.ptr;
-    const int32_t ldz = z.strides[0];
-    auto store = [&](int r, int c, const float* v, auto width) {   // `width` values from column c of the tile's row r
-      constexpr int W = decltype(width)::value;
-      const int32_t gr = row0 + r, gc = col0 + c;
-      if (gr >= cover_m || gc >= cover_n) return;
-      OutT* dst = zp + (int64_t)gr * ldz + gc;
-      if (gc >= col_first && gc + W <= cover_n) {
-        OutT o[W];
-        if (accumulate) __builtin_memcpy(o, __builtin_assume_aligned(dst, sizeof(OutT)), sizeof(o));
-#pragma unroll
-        for (int e = 0; e < W; ++e) o[e] = (OutT)(accumulate ? v[e] + (float)o[e] : v[e]);
-        __builtin_memcpy(__builtin_assume_aligned(dst, sizeof(OutT)), o, sizeof(o));
-      } else {
-#pragma unroll
-        for (int e = 0; e < W; ++e)
-          if (gc + e >= col_first && gc + e < cover_n) dst[e] = (OutT)(accumulate ? v[e] + (float)dst[e] : v[e]);
-      }
-    };
+    const LooseOutput<OutT> out{(OutT*)z.ptr, z.strides[0], row0, col0, col_first, cover_m, cover_n, accumulate};
     const BlockPartials part(partials + (int64_t)tile * splits * (BM * BN), BM * BN * 4, splits);
-    for (int pass = 0; pass < kOutPasses; ++pass) {
-      __syncthreads();   // the stages (or the previous pass) have been read
-      const int first = pass * kOutRows;
-      if (wm * WM < first + kOutRows && first < wm * WM + WM) {
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          const int r = wm * WM + tm * 16 + l16 - first;
-          if (kOutPasses > 1 && (wm * WM + tm * 16 < first || wm * WM + tm * 16 >= first + kOutRows)) continue;
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            *reinterpret_cast<f32x4*>(lds + r * (BN * 4) + (((wn * (WN / 4) + tn * 4 + grp) ^ (r & 15)) << 4)) = acc[tn][tm];
-        }
+    output_passes<BM, BN, WM, WN, kThreads, 2 * kStageBytes>(acc, lds, wm, wn, cover_m - row0, [&](int r, int u, f32x4 lo, f32x4 hi) {
+      if (splits == 1) {
+        const float f[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        out.template store<8>(r, u * 8, f);
+      } else {
+        part.store(split, (r * UB + u) * 2, lo);
+        part.store(split, (r * UB + u) * 2 + 1, hi);
       }
-      __syncthreads();
-      for (int o = tid; o < kOutRows * UB; o += kThreads) {
-        const int r = o / UB, u = o % UB;
-        if (first + r >= BM || row0 + first + r >= cover_m) break;   // rows only grow with o
-        f32x4 v[2] = {*reinterpret_cast<const f32x4*>(lds + r * (BN * 4) + (((2 * u) ^ (r & 15)) << 4)),
-                      *reinterpret_cast<const f32x4*>(lds + r * (BN * 4) + (((2 * u + 1) ^ (r & 15)) << 4))};
-        const float f[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
-        if (splits == 1) {
-          store(first + r, u * 8, f, std::integral_constant<int, 8>{});
-        } else {
-          part.store(split, ((first + r) * UB + u) * 2, v[0]);
-          part.store(split, ((first + r) * UB + u) * 2 + 1, v[1]);
-        }
-      }
-    }
+    });
     if (splits == 1 || !last_to_arrive(counters + tile, splits, &last)) return;
     part.add_up<kThreads, 2>(min(BM, cover_m - row0) * (BN / 4), [&](int o, f32x4 v) {
       const float f[4] = {v[0], v[1], v[2], v[3]};
-      store(o / (BN / 4), o % (BN / 4) * 4, f, std::integral_constant<int, 4>{});
+      out.template store<4>(o / (BN / 4), o % (BN / 4) * 4, f);
     });
   }
 };
@@ -295,18 +259,19 @@ GEMM_THIN_FAMILY(bf16, __bf16, __bf16)
 GEMM_THIN_FAMILY(f16, _Float16, _Float16)
 GEMM_THIN_FAMILY(bf16f32, __bf16, float)
 
-#define GEMM_STAGED_KERNEL(NAME, IN_T, OUT_T, BM, BN, WVM, WVN)                                                                     \
-  extern "C" __global__ void __launch_bounds__(WVM * WVN * 64, 2)                                                                   \
+// (PER_SIMD wavefronts to a SIMD: as many workgroups on a compute unit as the launcher's prices say, host/gemm_choice.h)
+#define GEMM_STAGED_KERNEL(NAME, IN_T, OUT_T, BM, BN, WVM, WVN, PER_SIMD)                                                           \
+  extern "C" __global__ void __launch_bounds__(WVM * WVN * 64, PER_SIMD)                                                                   \
       gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k_total, int32_t cover_m, int32_t cover_n,       \
                          int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits) { \
     GemmStaged<BM, BN, WVM, WVN, OUT_T, IN_T>::run(z, x, y, k_total, cover_m, cover_n, accumulate, partials, counters, tiles_m,       \
                                                    tiles_n, splits);                                                                \
   }
 #define GEMM_STAGED_FAMILY(T, IN_T, OUT_T)                     \
-  GEMM_STAGED_KERNEL(T##_staged64x64, IN_T, OUT_T, 64, 64, 2, 2)    \
-  GEMM_STAGED_KERNEL(T##_staged64x128, IN_T, OUT_T, 64, 128, 2, 2)  \
-  GEMM_STAGED_KERNEL(T##_staged128x128, IN_T, OUT_T, 128, 128, 2, 2) \
-  GEMM_STAGED_KERNEL(T##_staged256x128, IN_T, OUT_T, 256, 128, 4, 2)
+  GEMM_STAGED_KERNEL(T##_staged64x64, IN_T, OUT_T, 64, 64, 2, 2, 4)    \
+  GEMM_STAGED_KERNEL(T##_staged64x128, IN_T, OUT_T, 64, 128, 2, 2, 3)  \
+  GEMM_STAGED_KERNEL(T##_staged128x128, IN_T, OUT_T, 128, 128, 2, 2, 2) \
+  GEMM_STAGED_KERNEL(T##_staged256x128, IN_T, OUT_T, 256, 128, 4, 2, 2)
 GEMM_STAGED_FAMILY(bf16, __bf16, __bf16)
 GEMM_STAGED_FAMILY(f16, _Float16, _Float16)
 GEMM_STAGED_FAMILY(bf16f32, __bf16, float)

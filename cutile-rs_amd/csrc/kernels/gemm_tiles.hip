@@ -1,5 +1,6 @@
 // Members of GEMM families that only the launcher names: the 256 x 256 ring with its K shared, the 128 x 128 tile that has a compute unit
-// to itself (gemm_tiles.h), and strips that read y past the caches (gemm_thin.h).
+// to itself (gemm_tiles.h), and strips that read y past the caches (gemm_thin.h); and the register-staged 256 x 256 tiles (gemm_loose.h).
+#include "gemm_loose.h"
 #include "gemm_thin.h"
 #include "gemm_tiles.h"
 
@@ -18,3 +19,7 @@ GEMM_TILES_FAMILY(f16, _Float16)
 GEMM_THIN_NT_FAMILY(bf16, __bf16, __bf16)
 GEMM_THIN_NT_FAMILY(f16, _Float16, _Float16)
 GEMM_THIN_NT_FAMILY(bf16f32, __bf16, float)
+
+GEMM_STAGED_WIDE_KERNEL(bf16_staged256x256, __bf16, __bf16)
+GEMM_STAGED_WIDE_KERNEL(f16_staged256x256, _Float16, _Float16)
+GEMM_STAGED_WIDE_KERNEL(bf16f32_staged256x256, __bf16, float)
