@@ -269,9 +269,11 @@ inline MxPlan mx_plan(int64_t m, int64_t n, int32_t pieces, int cus, uint64_t pa
 // 128 x 128 tiles; nvfp4: 9.9, 14.7, 24).  The 256 x 256 kernels are the better ones where their tiles come near to filling the chip.
 // `lone`: what mx_plan says for fp8, where it was asked.
 inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus, uint64_t partial_bytes, MxPlan* lone) {
-  if (s.pieces <= 4) return nullptr;   // two steps: nothing to share out
+  // a partition whose output other tiles of nvfp4_gemm.hip may compute too
+  const bool tiled = s.fp4 && own_m == own_n && (own_m == 128 || (own_m == 256 && s.pieces > 4));
+  if (s.pieces <= 4 && !tiled) return nullptr;   // two steps: nothing to share out
   auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
-  if (s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
+  if (!tiled && s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
   // (fp8 on 128 x 128: the direct pipeline below is always the cheaper one; only a name reaches flat128x128 there)
   struct Kernel { const char* name; int bm, bn; double fp8, fp4; };
   static const Kernel kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20}, {"flat32x64", 32, 64, 0.12, 0.28}, {"flat64x64", 64, 64, 0.155, 0.36},
@@ -280,8 +282,23 @@ inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int
   double best = 1e30;
   for (const Kernel& k : kFlat) {
     const uint64_t b = blocks(k.bm, k.bn), waves = (b + cus - 1) / cus;
-    const double us = (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + 3.5);
+    if (s.pieces <= 4) break;
+    const double us = (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + (s.fp4 && waves > 1 ? 5.5 : 3.5));
     if (us < best) best = us, name = k.name;
+  }
+  if (tiled) {
+    // Whole tiles, expanded to f16 once for the workgroup: 256 x 256 to a compute unit, or two of 128 x 128.  us per piece of K and round, and of
+    // start and output (bf16 out, us on 256 x 256, 128 x 128 and the best strips: 2476 x 6080 x 896 34.7, 44.7, 54.7; 2940 x 5568 x 1152, 264 of
+    // the large tiles, 75, 54, 60; 2859 x 10368 x 512 47, 57, 67; 4096 x 4096 x 4096 117, 162, 153; 1024 x 4096 x 4096 101, 53, 44; a partition of 128
+    // x 128 had strips or the small tiles whatever the size: 58, 60, 61, 163, 46).
+    const uint64_t large = blocks(256, 256), small = blocks(128, 128), slots = 2 * (uint64_t)cus;
+    auto part = [&](uint64_t rest, double few, double all, double ends) { return rest ? (few + (all - few) * (double)rest / cus) * s.pieces + ends : 0.0; };
+    const double us256 = (double)(large / cus) * (3.5 * s.pieces + 9.5) + part(large % cus, 3.0, 3.5, 9.5);
+    const uint64_t rest = small % slots;
+    const double us128 = (double)(small / slots) * (2.4 * s.pieces + 5.0) + (rest <= (uint64_t)cus ? part(rest, 1.37, 1.52, 5.0) : part(rest - cus, 1.52, 2.4, 5.0));
+    if (us128 < best * 0.98) best = us128, name = "128x128x64_w2x2";
+    if (us256 < best * 0.98) best = us256, name = "256x256x64_q2x4";
+    return name;
   }
   if (!s.fp4) {
     *lone = mx_plan(s.m, s.n, s.pieces, cus, partial_bytes);

@@ -16,9 +16,11 @@
 // bf16 GEMM's bytes); the matrix pipe runs at its 16-bit rate.  The variants of record ("_q") use
 // v_mfma_f32_16x16x32_f16: 1241 against 1141 TFLOP/s at 8192^3 on random operands (see Nvfp4Gemm).
 //
-// Pipeline: register-staged.  For K tile kt+1 every lane fetches 16 bytes (32 values of
-// one row) of x and of y plus the two scale bytes that belong to them; while the MFMAs of
-// tile kt run from the current LDS stage, the fetched values are expanded
+// Pipeline: register-staged.  For a K tile every lane fetches 16 bytes (32 values of
+// one row) of x and of y plus the two scale bytes that belong to them, two tiles ahead of
+// the one that is multiplied (one ahead, 128 x 128 tiles waited for them: 512 x 4096 x 4096
+// 62.9 us, now 47.9; 256 x 256 have the work to cover either: 117 at 4096 x 4096 x 4096);
+// while the MFMAs of tile kt run from the current LDS stage, those of tile kt + 1 are expanded
 // (v_cvt_scalef32_pk_f16_fp4: two values per instruction; v_pk_mul_f16 by the block's
 // scale) and written to the other stage as four 16-byte units.  Rows are 128 bytes of f16
 // with 16-byte unit u stored at unit u ^ ((row >> 1) & 7), so the operand reads of 32 rows
@@ -117,42 +119,48 @@ struct Nvfp4Gemm {
       b_goff[i] = r < N ? (uint32_t)((int64_t)r * ldb + b_half[i] * 16) : kOob;
       b_soff[i] = r < N ? (uint32_t)((int64_t)r * ldsb + b_half[i] * 2) : kOob;
     }
-    u32x4 a_reg[kAPieces], b_reg[kBPieces];
-    uint32_t a_sc[kAPieces], b_sc[kBPieces];      // two e4m3 scale bytes in the low half
-    auto load_global = [&](int32_t kt) {          // K tile kt: packed bytes 32 kt .., scale bytes 4 kt ..
+    struct Packed {
+      u32x4 a[kAPieces], b[kBPieces];
+      uint32_t a_sc[kAPieces], b_sc[kBPieces];    // two e4m3 scale bytes in the low half
+    };
+    const int k_tiles = k_bytes / 32;
+    auto load_global = [&](Packed& p, int32_t kt) {   // K tile kt: packed bytes 32 kt .., scale bytes 4 kt ..; nothing from behind the last one
+      const uint32_t dead = kt < k_tiles ? 0u : kOob;
 #pragma unroll
       for (int i = 0; i < kAPieces; ++i) {
-        a_reg[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, a_goff[i], kt * 32, 0);
-        a_sc[i] = __builtin_amdgcn_raw_buffer_load_b16(rsa, a_soff[i], kt * 4, 0);
+        p.a[i] = __builtin_amdgcn_raw_buffer_load_b128(ra, a_goff[i] | dead, kt * 32, 0);
+        p.a_sc[i] = __builtin_amdgcn_raw_buffer_load_b16(rsa, a_soff[i] | dead, kt * 4, 0);
       }
 #pragma unroll
       for (int i = 0; i < kBPieces; ++i) {
-        b_reg[i] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_goff[i], kt * 32, 0);
-        b_sc[i] = __builtin_amdgcn_raw_buffer_load_b16(rsb, b_soff[i], kt * 4, 0);
+        p.b[i] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_goff[i] | dead, kt * 32, 0);
+        p.b_sc[i] = __builtin_amdgcn_raw_buffer_load_b16(rsb, b_soff[i] | dead, kt * 4, 0);
       }
     };
     // LDS takes a 16-byte write from 8 lanes per cycle (128 bytes): lanes 0-7 are 4 rows x 2 halves, and rows
     // 2j, 2j+1 share their swizzle term, so writing unit d of every row in step d would put both on the same
     // banks.  Odd rows therefore walk their four units in the order 2, 3, 0, 1.
-    auto expand_piece = [&](unsigned char* tile, int row, int half, const u32x4& q, uint32_t sc) {
-      const bool odd = row & 1;
+    // Both stages of x lie in front of both of y, and rows 16 apart share their swizzle term: an address and a 16-bit immediate reach every piece.
+    static_assert(kThreads / 2 % 16 == 0 && BLK % 16 == 0, "the swizzle term repeats from piece to piece");
+    const bool odd = a_row[0] & 1;
+    int w_addr[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) w_addr[d] = lds_off(tid >> 1, (tid & 1) * 4 + (d ^ (odd ? 2 : 0)));
+    auto expand_piece = [&](unsigned char* tile, const u32x4& q, uint32_t sc) {
       const _Float16 s0 = (_Float16)__builtin_amdgcn_cvt_f32_fp8((int)sc, 0);   // e4m3fn -> f32 -> f16: exact
       const _Float16 s1 = (_Float16)__builtin_amdgcn_cvt_f32_fp8((int)sc, 1);
       const _Float16 sa = odd ? s1 : s0, sb = odd ? s0 : s1;
       const uint32_t q0 = odd ? q.z : q.x, q1 = odd ? q.w : q.y, q2 = odd ? q.x : q.z, q3 = odd ? q.y : q.w;
-      const int flip = odd ? 2 : 0;
-      *reinterpret_cast<u32x4*>(tile + lds_off(row, half * 4 + (0 ^ flip))) = expand_fp4x8(q0, sa);
-      *reinterpret_cast<u32x4*>(tile + lds_off(row, half * 4 + (1 ^ flip))) = expand_fp4x8(q1, sa);
-      *reinterpret_cast<u32x4*>(tile + lds_off(row, half * 4 + (2 ^ flip))) = expand_fp4x8(q2, sb);
-      *reinterpret_cast<u32x4*>(tile + lds_off(row, half * 4 + (3 ^ flip))) = expand_fp4x8(q3, sb);
+      *reinterpret_cast<u32x4*>(tile + w_addr[0]) = expand_fp4x8(q0, sa);
+      *reinterpret_cast<u32x4*>(tile + w_addr[1]) = expand_fp4x8(q1, sa);
+      *reinterpret_cast<u32x4*>(tile + w_addr[2]) = expand_fp4x8(q2, sb);
+      *reinterpret_cast<u32x4*>(tile + w_addr[3]) = expand_fp4x8(q3, sb);
     };
-    auto store_lds = [&](int stage) {
-      unsigned char* sa = lds + stage * kStageBytes;
-      unsigned char* sb = sa + kABytes;
+    auto store_lds = [&](const Packed& p, int stage) {
 #pragma unroll
-      for (int i = 0; i < kAPieces; ++i) expand_piece(sa, a_row[i], a_half[i], a_reg[i], a_sc[i]);
+      for (int i = 0; i < kAPieces; ++i) expand_piece(lds + stage * kABytes + i * (kThreads / 2 * kRowBytes), p.a[i], p.a_sc[i]);
 #pragma unroll
-      for (int i = 0; i < kBPieces; ++i) expand_piece(sb, b_row[i], b_half[i], b_reg[i], b_sc[i]);
+      for (int i = 0; i < kBPieces; ++i) expand_piece(lds + 2 * kABytes + stage * kBBytes + i * (kThreads / 2 * kRowBytes), p.b[i], p.b_sc[i]);
     };
 
     typedef float f32x4v __attribute__((ext_vector_type(4)));
@@ -166,27 +174,30 @@ struct Nvfp4Gemm {
 #pragma unroll
         for (int v = 0; v < kAccRegs; ++v) acc[tn][tm][v] = 0.0f;
 
-    const int k_tiles = k_bytes / 32;
-    if (k_tiles > 0) {
-      load_global(0);
-      store_lds(0);
-    }
+    Packed p0, p1;                              // K tile kt + 1 in one, kt + 2 on its way into the other
+    load_global(p0, 0);
+    load_global(p1, 1);
+    store_lds(p0, 0);
+    load_global(p0, 2);
     __syncthreads();
 
     constexpr int kSteps = SHAPE16 ? 2 : 4;     // K steps of 32 or 16 values per tile
-    for (int kt = 0; kt < k_tiles; ++kt) {
-      const int cur = kt & 1;
-      if (kt + 1 < k_tiles) load_global(kt + 1);
-      const unsigned char* sa = lds + cur * kStageBytes;
-      const unsigned char* sb = sa + kABytes;
+    const int frow = SHAPE16 ? l16 : l32;
+    int a_addr[kSteps], b_addr[kSteps];
+#pragma unroll
+    for (int ks = 0; ks < kSteps; ++ks) {
+      const int funit = SHAPE16 ? ks * 4 + grp : ks * 2 + khalf;
+      a_addr[ks] = lds_off(wm * WM + frow, funit);
+      b_addr[ks] = 2 * kABytes + lds_off(wn * WN + frow, funit);
+    }
+    auto k_tile = [&](int cur, Packed& next, int32_t kt) {
 #pragma unroll
       for (int ks = 0; ks < kSteps; ++ks) {
         f16x8 af[TM], bfr[TN];
-        const int frow = SHAPE16 ? l16 : l32, funit = SHAPE16 ? ks * 4 + grp : ks * 2 + khalf;
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) af[tm] = *reinterpret_cast<const f16x8*>(sa + lds_off(wm * WM + tm * BLK + frow, funit));
+        for (int tm = 0; tm < TM; ++tm) af[tm] = *reinterpret_cast<const f16x8*>(lds + a_addr[ks] + cur * kABytes + tm * (BLK * kRowBytes));
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn) bfr[tn] = *reinterpret_cast<const f16x8*>(sb + lds_off(wn * WN + tn * BLK + frow, funit));
+        for (int tn = 0; tn < TN; ++tn) bfr[tn] = *reinterpret_cast<const f16x8*>(lds + b_addr[ks] + cur * kBBytes + tn * (BLK * kRowBytes));
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
@@ -197,9 +208,18 @@ struct Nvfp4Gemm {
               acc[tn][tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
           }
         // the expansion of the next tile rides between the matrix instructions of the later K steps
-        if (ks == (SHAPE16 ? 0 : 1) && kt + 1 < k_tiles) store_lds(cur ^ 1);
+        if (ks == (SHAPE16 ? 0 : 1)) {
+          store_lds(next, cur ^ 1);
+          load_global(next, kt + 3);
+        }
       }
       __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll 1
+    for (int kt = 0; kt < k_tiles; kt += 2) {   // (an odd number of K tiles is followed by one of zeros)
+      k_tile(0, p1, kt);
+      k_tile(1, p0, kt + 1);
     }
 
     OutT* zp = (OutT*)z.ptr;

@@ -1,0 +1,34 @@
+"""NVFP4 products on whole tiles (nvfp4_gemm.hip): one to seven K tiles of 64 (an odd number is followed by one of zeros), edges of the tiles in both
+directions, and outputs of a 128 x 128 partition that 256 x 256 tiles compute."""
+import pytest
+import torch
+
+import oracle
+from util import rel_l2
+
+
+def _dev(a, dev):
+    return torch.from_numpy(a).to(dev)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", ["128x128x64_w2x2", "256x256x64_q2x4", "256x256x64_q4x2", "256x256x64_w4x2"])
+@pytest.mark.parametrize("m,n,tiles", [(1, 4, 1), (130, 132, 2), (257, 260, 3), (128, 256, 6), (300, 516, 7)])
+def test_gpu_tiles_of_k(ct, dev, variant, m, n, tiles):
+    k = 64 * tiles
+    xq, xs = oracle.nvfp4_quantize(oracle.normal_f32((m, k), 971))
+    yq, ys = oracle.nvfp4_quantize(oracle.normal_f32((n, k), 972))
+    ref = oracle.nvfp4_gemm_f32(xq, yq, xs, ys, 0.5)
+    z = torch.full((m + 1, n), 7.0, dtype=torch.float32, device=dev)
+    ct.linear_tile_nvfp4(ct.partition(z[:m], [128, 128] if variant[0] == "1" else [256, 256]), *[_dev(v, dev) for v in (xq, yq, xs, ys)], 0.5, variant="f32_" + variant)
+    assert rel_l2(z[:m].cpu().numpy(), ref) <= 2e-6          # exact products, f32 sums of at most 448 of them in another order
+    assert torch.all(z[m] == 7.0)
+
+
+def test_size_rule_of_a_128_partition(fake_hip):
+    """whole outputs of 240 tiles of 256 x 256 run on those, of a few more than 256 on 128 x 128, of few rows on strips"""
+    ct = fake_hip
+    for m, n, k, want in ((2476, 6080, 896, "256x256x64_q2x4"), (2940, 5568, 1152, "128x128x64_w2x2"), (200, 14336, 4096, "flat128x128"), (8, 4096, 4096, "flat16x64")):
+        u8 = lambda rows, cols: torch.empty(rows, cols, dtype=torch.uint8)
+        ct.linear_tile_nvfp4(ct.partition(torch.empty(m, n, dtype=torch.bfloat16), [128, 128]), u8(m, k // 2), u8(n, k // 2), u8(m, k // 16), u8(n, k // 16), 1.0)
+        assert ct.last_resolved()["variant"] == "bf16_" + want
