@@ -379,11 +379,12 @@ std::vector<KernelEntry> build_table() {
   for (const char* function : {"fmha", "fmha_seq"})
     for (const char* dt : {"bf16", "f16"})
       for (int d : {64, 128})
-        for (int rows : {32, 64}) {
-          if (function[4] == '_' && dt[0] == 'b') continue;
-          std::string v = std::string(dt) + "_" + std::to_string(rows) + "x" + (rows == 32 ? "256x" : "128x") + std::to_string(d);
-          add(function, keep(v + "+keys"), keep(std::string(function) + "_entry__" + v + "_keys"), IMG_FMHA_KEYS, 512,
-              (uint32_t)(512 * d * 2 + 2 * 8 * 32 * 4), rows, rows == 32 ? 256 : 128, d, 0, dt, 0, 3);
+        for (int rows : {32, 64, 128}) {
+          if ((function[4] == '_' && dt[0] == 'b') || (rows == 128 && d == 128)) continue;
+          const std::string v = std::string(dt) + "_" + std::to_string(rows) + "x" + std::to_string(8192 / rows) + "x" + std::to_string(d);
+          const char* const member = rows == 128 ? "halves" : "keys";
+          add(function, keep(v + "+" + member), keep(std::string(function) + "_entry__" + v + "_" + member), IMG_FMHA_KEYS, 512,
+              (uint32_t)(512 * d * 2 + 2 * 8 * 32 * 4), rows, 8192 / rows, d, 0, dt, 0, 3);
         }
 
   // ---- decode attention: one workgroup per (KV head, split); tile = (GROUP, 0, D) ----

@@ -2766,14 +2766,17 @@ cutile_status_t cutile_launch_mapped_shared_cache_update_f32(cutile_stream_t str
 }
 
 namespace {
-// Attention whose longest chain of keys decides its time, not its work (fmha_keys.hip): the query rows of a workgroup whose wavefronts share
-// the keys, or 0 for the kernels of 32 rows to a wavefront.
+// Attention whose longest chain of keys decides its time, not its work (fmha_keys.hip), and of D = 64: the query rows of a workgroup whose
+// wavefronts share the keys, or 0 for the kernels of 32 rows to a wavefront.
 // On 32 rows a workgroup has read its keys soonest, as long as one round holds the launch; behind that 64 rows, which read them half as
 // often.  D = 128 leaves room for one workgroup on a compute unit, D = 64 for two.  us on the kernels of 128 and 256 rows, on 64 and on 32:
 //   D = 128, causal: 4 heads of 2048 42, 30 and 26; 8 of 2048 (256 workgroups of 64 rows) 43, 31 and 34; 32 of 1024 (512) 26.2, 26.8 and 44
 //   D = 64: 8 heads of 1024 (256 workgroups of 32 rows) 21, 13 and 10.5; 16 of 1024 21, 13 and 15; 32 of 1024 (512 of 64 rows) 22, 18.5 and 27;
 //     512 of short keys lose: 128 heads of 256 8.9, 10 and 19; 1024 of 64 rows pay where causal tiles even out: 32 heads of 2048 causal 52, 41
 //     and 73, not causal 55, 60 and 110
+//   Two rounds of 64 rows at D = 128 pay where causal tiles are long (8 heads of 4096 80.8 and 66.5; 32 of 1024 25.6 and 27.0).
+// Every other launch of D = 64 has two wavefronts to 32 rows of the 128-row workgroup (us on one wavefront and on two: 32 heads of 4096 196 and 180, causal 109
+// and 102; 128 of 1024 57 and 54, 43 and 38; 256 of 256 12.1 and 13.1, causal 13.0 and 12.8).
 // Up to 128 keys there is nothing to share (one head of 64: 6.5, 8.0 and 8.3; of 129: 9.4, 8.2 and 8.3).
 int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, bool causal, int cus) {
   if ((d != 64 && d != 128) || keys <= 128) return 0;
@@ -2781,17 +2784,20 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, bool caus
   if (of32 <= cus) return 32;
   if (of64 <= cus) return 64;
   if (d == 64 && ((of64 <= 2 * cus && keys >= 512) || (of64 <= 4 * cus && causal && keys >= 1024))) return 64;
-  return 0;
+  if (d == 128 && causal && of64 <= 2 * cus && keys >= 3072) return 64;
+  return d == 64 && keys >= (causal ? 200 : 300) ? 128 : 0;
 }
 // (by their own rows, not by the family whose place they take)
 const KernelEntry* keys_member(const char* function, bool bf16, int rows, int d) {
   static const auto& members = *[] {
-    auto* m = new std::array<const KernelEntry*, 16>();
-    for (size_t i = 0; i < m->size(); ++i)
-      (*m)[i] = find_entry(i & 8 ? "fmha_seq" : "fmha", std::string(i & 4 ? "bf16_" : "f16_") + (i & 2 ? "64x128x" : "32x256x") + (i & 1 ? "128+keys" : "64+keys"));
+    auto* m = new std::array<const KernelEntry*, 24>();
+    for (size_t i = 0; i < m->size(); ++i) {
+      const char* const rows[] = {"32x256x", "64x128x", "128x64x"};
+      (*m)[i] = find_entry(i / 12 ? "fmha_seq" : "fmha", std::string(i / 6 % 2 ? "bf16_" : "f16_") + rows[i / 2 % 3] + (i & 1 ? "128" : "64") + (i / 2 % 3 == 2 ? "+halves" : "+keys"));
+    }
     return m;
   }();
-  return members[(strcmp(function, "fmha_seq") == 0) * 8 + bf16 * 4 + (rows == 64) * 2 + (d == 128)];
+  return members[(strcmp(function, "fmha_seq") == 0) * 12 + bf16 * 6 + (rows / 64) * 2 + (d == 128)];
 }
 }  // namespace
 

@@ -9,6 +9,12 @@
 // Now a step is bound by the reads of K and V, which every 32 (64) rows repeat: 128 KiB through a compute unit's vector cache at 64 bytes a
 // clock are 0.9 of the 2.4 us that 256 keys take at D = 128, the rest their latency and the barriers.  us before and here: 4 heads of 1700
 // rows, causal, D = 128 36.5 and 23.4; 16 of 1024, D = 64 21 and 13; 16 of 505 12.8 and 7.4; 32 of 296, not causal, D = 128 15.5 and 11.4.
+//
+// "halves": two wavefronts to 32 rows on the 128 rows of Fmha's workgroup, for launches of many tiles too.  At D = 64 a 64-key step of Fmha is one
+// chain of products, exponentials and products on one wavefront of a SIMD; here two wavefronts (four, with two workgroups to a compute unit)
+// have 32 keys each and run across each other's waits: 32 heads of 4096 196 -> 180 us, causal 109 -> 102; 192 of 653 51 -> 47, causal 36 -> 32; 64
+// of 430, causal 11.7 -> 10.4.  (At D = 128 the registers leave one workgroup to a compute unit: 32 heads of 2048 92 us where the
+// ping-pong kernel takes 61.)
 #include <hip/hip_runtime.h>
 
 #include "fmha_common.h"
@@ -27,8 +33,8 @@ struct FmhaKeys {
   static constexpr int DB = D / 32;
   static constexpr int kOutUnits = D / 4;             // 16-byte units of a partial output row
   static constexpr int kOutBytes = 32 * D * 4;        // of a wavefront's partial output
-  static constexpr int kLdsBytes = STAGES * kStageBytes;
-  static_assert(kTileUnits % kThreads == 0 && kWaves * kOutBytes <= kLdsBytes && kOutUnits % S == 0, "the partial outputs lie in the stages");
+  static constexpr int kLdsBytes = STAGES * kStageBytes > kWaves * kOutBytes ? STAGES * kStageBytes : kWaves * kOutBytes;   // (the partial outputs lie in the stages)
+  static_assert(kTileUnits % kThreads == 0 && kOutUnits % S == 0, "equal shares");
   static_assert(D == 64 || D == 128, "swizzles below");
 
   __device__ static __forceinline__ int k_off(int r, int u) { return r * (D * 2) + ((u ^ (r & (kUnitsPerRow - 1))) << 4); }
@@ -244,8 +250,11 @@ FMHA_KEYS_KERNEL(f16_32x256x64_keys, _Float16, 1, 8, 1, 64)
 FMHA_KEYS_KERNEL(bf16_64x128x128_keys, __bf16, 2, 4, 2, 128)
 FMHA_KEYS_KERNEL(f16_64x128x128_keys, _Float16, 2, 4, 2, 128)
 FMHA_KEYS_KERNEL(bf16_64x128x64_keys, __bf16, 2, 4, 2, 64)
+FMHA_KEYS_KERNEL(bf16_128x64x64_halves, __bf16, 4, 2, 2, 64)
 FMHA_KEYS_KERNEL(f16_64x128x64_keys, _Float16, 2, 4, 2, 64)
+FMHA_KEYS_KERNEL(f16_128x64x64_halves, _Float16, 4, 2, 2, 64)
 FMHA_KEYS_SEQ_KERNEL(f16_32x256x128_keys, _Float16, 1, 8, 1, 128)
 FMHA_KEYS_SEQ_KERNEL(f16_32x256x64_keys, _Float16, 1, 8, 1, 64)
 FMHA_KEYS_SEQ_KERNEL(f16_64x128x128_keys, _Float16, 2, 4, 2, 128)
 FMHA_KEYS_SEQ_KERNEL(f16_64x128x64_keys, _Float16, 2, 4, 2, 64)
+FMHA_KEYS_SEQ_KERNEL(f16_128x64x64_halves, _Float16, 4, 2, 2, 64)
