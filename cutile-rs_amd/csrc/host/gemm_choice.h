@@ -32,6 +32,9 @@ struct RingTile {
 // 2 to 8 workgroups (3800 times; 5 to 8 % rms).  Over those sizes the kernel that this prices lowest takes 1.02 times the best one's time.
 constexpr RingTile kRingTiles[] = {{"256x256x64_q2x4", 256, 256, 1.03, 1.36, 8.05}, {"192x256x64_q2x4", 192, 256, 0.82, 1.08, 7.2}, {"256x128x64_q4x2", 256, 128, 0.62, 0.865, 5.95},
                                    {"128x256x64_q2x4", 128, 256, 0.62, 0.845, 5.7}, {"192x128x64_q2x2", 192, 128, 0.44, 0.72, 4.5}, {"128x128x64_q2x2", 128, 128, 0.325, 0.55, 4.2}};
+// A K tile on 192 x 192 (the stages of 192 x 256), by its share of a wide tile's products: 7 x 36 wide and 7 x 15 narrow tiles of K = 4608 144 us
+// priced, 152 measured; 5 x 51 and 5 x 27 of 5120 161, 172; one width 156 and 172 priced, 161 and 179 measured.
+constexpr double kNarrowFew = 0.66, kNarrowAll = 0.86, kNarrowEnds = 6.2;
 // Workgroups that share a tile: each stores its partial tile, and the last one reads them all.  us a value of one output tile, and of all of them.
 constexpr double kShareEach = 4.2e-5, kShareAll = 1.0e-6, kShareOnce = 0.7;
 // The one that a kernel of that tile is, by the tile shape and by the marker of these kernels in its name.
@@ -45,6 +48,7 @@ struct RingPlan {
   uint32_t splits;   // workgroups that share the K tiles of an output tile
   bool two;          // 128 x 128: two workgroups to a compute unit, on the ring (K unshared)
   double us;
+  uint32_t wide = 0, narrow = 0;   // columns of tiles, where those of 192 columns stand beside the ones of 256
 };
 // What the launch costs with the best number of workgroups to an output tile; as priced and as launched.  `partial_bytes` = room for partial tiles, 0: K is not shared.
 inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, int cus, uint64_t partial_bytes) {
@@ -57,6 +61,15 @@ inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, in
     const double us = (double)((kt + s - 1) / s) * ((double)(g / cus) * r.all + (rest ? r.few + (r.all - r.few) * (double)rest / cus : 0.0)) +
                       r.ends * (double)((g + cus - 1) / cus) + (s > 1 ? kShareOnce + (kShareEach * s + kShareAll * (double)g) * (r.bm * r.bn) : 0.0);
     if (us < best.us * 0.98) best = {s, false, us};
+  }
+  if (r.bm == 192 && r.bn == 256 && t > (uint64_t)cus && t < 2 * (uint64_t)cus) {
+    // A second round that is not full: a wide tile to each compute unit first, then narrow ones.
+    const int64_t rows = (m + r.bm - 1) / r.bm, wide = cus / rows, narrow = (n - wide * 256 + 191) / 192;
+    if (wide > 0 && narrow > 0 && rows * (wide + narrow) <= 2 * cus) {
+      const double rest = (double)(rows * (wide + narrow) - cus) / cus;
+      const double us = (double)kt * (r.all + kNarrowFew + (kNarrowAll - kNarrowFew) * rest) + r.ends + kNarrowEnds;
+      if (us < best.us * 0.98) best = {1, false, us, (uint32_t)wide, (uint32_t)narrow};
+    }
   }
   if (r.bm == 128 && r.bn == 128) {
     // two workgroups to a compute unit, each at half its pace as soon as there are more than compute units (1623 x 2944 x

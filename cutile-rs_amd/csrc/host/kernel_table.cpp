@@ -252,7 +252,7 @@ std::vector<KernelEntry> build_table() {
   struct Tile { const char* name; int bm, bn, stages_m, stages_n; };
   for (const char* dt : {"bf16", "f16"})
     for (const Tile& t : {Tile{"192x256x64_q2x4", 192, 256, 3, 2}, Tile{"128x256x64_q2x4", 128, 256, 3, 2}, Tile{"256x128x64_q4x2", 256, 128, 3, 2},
-                          Tile{"192x128x64_q2x2", 192, 128, 4, 4}, Tile{"256x256x64_q2x4+split", 256, 256, 3, 2}, Tile{"128x128x64_q2x2+lone", 128, 128, 5, 5}}) {
+                          Tile{"192x128x64_q2x2", 192, 128, 4, 4}, Tile{"256x256x64_q2x4+split", 256, 256, 3, 2}, Tile{"192x256x64_q2x4+mix", 192, 256, 3, 2}, Tile{"128x128x64_q2x2+lone", 128, 128, 5, 5}}) {
       const std::string v = std::string(dt) + "_" + t.name;
       std::string sym = "gemm_entry__" + v;
       std::replace(sym.begin(), sym.end(), '+', '_');

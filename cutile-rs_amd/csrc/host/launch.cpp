@@ -2271,7 +2271,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
       if (cutile_status_t s = compute_units(res.device, &cus)) return s;
     stream_grid = (uint32_t)std::min<uint64_t>((uint64_t)tg[0] * tg[1], (uint64_t)std::max(cus, 1));
   }
-  uint32_t splits = 1;
+  uint32_t splits = 1, narrow = 0;
   if (const RingTile* ring = row_layout && fast_layout && full_cover ? ring_tile(res.entry->variant, res.entry->tile[0], res.entry->tile[1]) : nullptr) {
     RingPlan plan = ring == sized.ring ? sized.ring_plan : ring_plan(*ring, cover_m, cover_n, k_valid, cus, partial_bytes);
     if (plan.splits > 1 && !ws.partials && g_launch_mode == 0) {   // a kernel that the caller or a record names
@@ -2279,7 +2279,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
       if (!ws.partials) plan = ring_plan(*ring, cover_m, cover_n, k_valid, cus, 0);
     }
     splits = plan.splits;
-    const char* member = ring->bm == 256 && ring->bn == 256 && splits > 1 ? "+split" : ring->bm == 128 && ring->bn == 128 && !plan.two ? "+lone" : nullptr;
+    if (plan.narrow) tg[1] = plan.wide, narrow = plan.narrow;
+    const char* member = plan.narrow ? "+mix" : ring->bm == 256 && ring->bn == 256 && splits > 1 ? "+split" : ring->bm == 128 && ring->bn == 128 && !plan.two ? "+lone" : nullptr;
     if (member)
       if (cutile_status_t s = use_member(&res, member_of(res.entry, member))) return s;
   }
@@ -2328,8 +2329,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   if (is_gemm_tile(res.entry)) {
     args.push_val<void*>(ws.partials);
     args.push_val<void*>(ws.counters);
-    args.push_val<uint32_t>(splits);
-    grid[0] *= splits;
+    args.push_val<uint32_t>(narrow ? narrow : splits);
+    grid[0] = narrow ? tg[0] * (tg[1] + narrow) : grid[0] * splits;
   }
   if (res.entry->tile[0] == 0) {   // any-layout kernel: 64x64 outputs per workgroup over the covered region
     grid[0] = std::max<uint32_t>(1, div_up(cover_m, 64));

@@ -165,7 +165,7 @@ __device__ __forceinline__ void store_z(V v, V* p, bool stream) {
 
 // `write_band(tm)` puts rows [32 tm, 32 tm + 32) of the wavefront's sub-tile into `stage` (f32, row r at r * WN * 4,
 // 16-byte chunk c of row r at chunk c ^ (r & 15)); TM = 32-row bands, WN = columns of the sub-tile.
-template <int TM, int WN, typename OutT, typename BandWriter>
+template <int TM, int WN, typename OutT, int COLS = WN, typename BandWriter>
 __device__ __forceinline__ void store_bands_staged(BandWriter write_band, unsigned char* stage, OutT* zp, int32_t ldz,
                                                    int32_t zM, int32_t zN, int32_t wave_row0, int32_t wave_col0,
                                                    int lane, int32_t accumulate) {
@@ -176,7 +176,7 @@ __device__ __forceinline__ void store_bands_staged(BandWriter write_band, unsign
   constexpr int PASSES = 32 / ROWS_PER_PASS;
   const int rd_row = lane / LANES_PER_ROW, rd_col = (lane % LANES_PER_ROW) * COLS_PER_LANE;
   const int32_t gc = wave_col0 + rd_col;
-  const bool col_ok = gc < zN;
+  const bool col_ok = gc < zN && (COLS == WN || rd_col < COLS);
   const bool stream = (int64_t)zM * zN * (int64_t)sizeof(OutT) >= kStreamedOutputBytes;
   const bool full = gc + COLS_PER_LANE <= zN;  // zN is a multiple of 4: otherwise exactly the first 4 columns are inside
   // Old z, all of it requested before anything is waited for.
@@ -265,14 +265,15 @@ __device__ __forceinline__ void store_tile_staged(f32x16 (&acc)[TN][TM], unsigne
 }
 // accumulators of v_mfma_f32_16x16x32 (TM, TN count 16 x 16 blocks): a lane holds row lane % 16 and the column
 // quadruple lane / 16 of each block; two row blocks make one 32-row band
-template <int TM, int TN, typename OutT>
+// BAND >= 16 TN: columns that a row of the band has room for; the lanes of those beyond 16 TN store nothing.
+template <int TM, int TN, typename OutT, int BAND = TN * 16>
 __device__ __forceinline__ void store_tile_staged16(f32x4_acc (&acc)[TN][TM], unsigned char* stage, OutT* zp, int32_t ldz,
                                                     int32_t zM, int32_t zN, int32_t wave_row0, int32_t wave_col0,
                                                     int lane, int32_t accumulate) {
   static_assert(TM % 2 == 0, "two 16-row blocks per band");
-  constexpr int PITCH = TN * 16 * 4;
+  constexpr int PITCH = BAND * 4;
   const int l16 = lane & 15, grp = lane >> 4;
-  store_bands_staged<TM / 2, TN * 16, OutT>(
+  store_bands_staged<TM / 2, BAND, OutT, TN * 16>(
       [&](int band) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -280,7 +281,7 @@ __device__ __forceinline__ void store_tile_staged16(f32x4_acc (&acc)[TN][TM], un
           for (int tn = 0; tn < TN; ++tn) {
             const int r = h * 16 + l16;
             const f32x4 v = {acc[tn][band * 2 + h][0], acc[tn][band * 2 + h][1], acc[tn][band * 2 + h][2], acc[tn][band * 2 + h][3]};
-            *reinterpret_cast<f32x4*>(stage + r * PITCH + (((tn * 4 + grp) ^ (r & kBandSwizzle<TN * 16>)) << 4)) = v;
+            *reinterpret_cast<f32x4*>(stage + r * PITCH + (((tn * 4 + grp) ^ (r & kBandSwizzle<BAND>)) << 4)) = v;
           }
       },
       stage, zp, ldz, zM, zN, wave_row0, wave_col0, lane, accumulate);

@@ -16,12 +16,13 @@ namespace gemm {
 // 2093 TFLOP/s with it against 1854 (equal, 2463 - 2481, on constant operands).  A block is 16 MFMAs (half of the
 // sub-tile's rows by all of its columns, one 32-wide K step) and lasts as long as a block of GemmRing; the y
 // fragments of a K step serve two blocks, so LDS traffic is unchanged.
-template <int BM, int BN, int WAVES_M, int WAVES_N, typename OutT, typename InT = __bf16>
+// CN < BN: the stages of a BN-column tile hold CN columns (of a tile beside wider ones, gemm_tiles.h); fetches of the others bring nothing.
+template <int BM, int BN, int WAVES_M, int WAVES_N, typename OutT, typename InT = __bf16, int CN = BN>
 struct GemmRing16 {
   static constexpr int BK = 64;
   static constexpr int kWaves = WAVES_M * WAVES_N;
   static constexpr int kThreads = kWaves * 64;
-  static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
+  static constexpr int WM = BM / WAVES_M, WN = CN / WAVES_N, BAND = BN / WAVES_N;   // BAND: columns that a row of an output band has room for
   static constexpr int TM = WM / 16, TN = WN / 16;   // 16 x 16 accumulator blocks of the wavefront's sub-tile
   static constexpr int TMH = TM / 2;                   // x fragments of one MFMA block (half the sub-tile's rows)
   static_assert(TM % 2 == 0, "a block takes half of the sub-tile's rows");
@@ -84,6 +85,9 @@ struct GemmRing16 {
     }
   }
 
+  struct Stages {
+    unsigned char *xs0, *xs1, *xs2, *ys0a, *ys0b, *ys1a, *ys1b;
+  };
   struct AllOfK {
     template <typename Acc>
     __device__ __forceinline__ bool operator()(Acc&, uint32_t*) const { return true; }
@@ -101,12 +105,19 @@ struct GemmRing16 {
     __shared__ __attribute__((aligned(1024))) unsigned char ys0b[kBBytes / 2];  //            K rows 32..63
     __shared__ __attribute__((aligned(1024))) unsigned char ys1a[kBBytes / 2];
     __shared__ __attribute__((aligned(1024))) unsigned char ys1b[kBBytes / 2];
+    run_tile_in(Stages{xs0, xs1, xs2, ys0a, ys0b, ys1a, ys1b}, z, x, y, k_total, pm, pn, accumulate, combine);
+  }
+  template <typename Combine = AllOfK>
+  __device__ static __forceinline__ void run_tile_in(const Stages& stages, const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y,
+                                                     int32_t k_total, uint32_t pm, uint32_t pn, int32_t accumulate, Combine combine = Combine{}) {
+    unsigned char *const xs0 = stages.xs0, *const xs1 = stages.xs1, *const xs2 = stages.xs2;
+    unsigned char *const ys0a = stages.ys0a, *const ys0b = stages.ys0b, *const ys1a = stages.ys1a, *const ys1b = stages.ys1b;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
     const int32_t M = x.shape[0], N = y.shape[1];
     const int32_t lda = x.strides[0], ldb = y.strides[0];
-    const int32_t row0 = pm * BM, col0 = pn * BN;
+    const int32_t row0 = pm * BM, col0 = pn * CN;
     const int32_t k_valid = min(min(x.shape[1], y.shape[0]), k_total);
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(x.ptr, (uint32_t)(((int64_t)(M - 1) * lda + x.shape[1]) * 2));
     // (a group of inner size 0 has no row of y: the prologue's masked fetches must still find themselves out of range)
@@ -132,7 +143,7 @@ struct GemmRing16 {
     for (int i = 0; i < kBInstr; ++i) {
       const int r = (i * kWaves + wave) * kBRowsPerInstr + lane / UB;
       const int u = (lane % UB) ^ b_swizzle(r);
-      b_goff[i] = (col0 + u * 8 < N) ? (uint32_t)(((int64_t)r * ldb + col0 + u * 8) * 2) : kOob;
+      b_goff[i] = (u * 8 < CN && col0 + u * 8 < N) ? (uint32_t)(((int64_t)r * ldb + col0 + u * 8) * 2) : kOob;
     }
     auto fetch_a = [&](unsigned char* stage, int32_t k0, int i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (LDS_PTR(void))(stage + (wave * kAInstr + i) * 1024), 16,
@@ -288,11 +299,11 @@ struct GemmRing16 {
     // last two take the y stages).
     __syncthreads();
     if (!combine(acc, reinterpret_cast<uint32_t*>(ys1b))) return;
-    static_assert(2 * kEpilogueBytesPerWave<WN> <= kABytes && kEpilogueBytesPerWave<WN> <= kBBytes / 2 && kWaves <= 8,
+    static_assert(2 * kEpilogueBytesPerWave<BAND> <= kABytes && kEpilogueBytesPerWave<BAND> <= kBBytes / 2 && kWaves <= 8,
                   "the output bands must fit the stages, and none lie in the last y half");
     unsigned char* band = wave < 2 ? xs0 : wave < 4 ? xs1 : wave < 6 ? xs2 : wave == 6 ? ys0a : ys0b;
-    if (wave < 6) band += (wave & 1) * kEpilogueBytesPerWave<WN>;
-    store_tile_staged16<TM, TN, OutT>(acc, band, (OutT*)z.ptr, z.strides[0], z.shape[0], z.shape[1], row0 + wm * WM,
+    if (wave < 6) band += (wave & 1) * kEpilogueBytesPerWave<BAND>;
+    store_tile_staged16<TM, TN, OutT, BAND>(acc, band, (OutT*)z.ptr, z.strides[0], z.shape[0], z.shape[1], row0 + wm * WM,
                                     col0 + wn * WN, lane, accumulate);
   }
 };

@@ -200,3 +200,35 @@ struct GemmStages {
                                                                              counters + t.tile, t.split, splits, flag);             \
     });                                                                                                                             \
   }
+
+// Tiles of two widths in one launch: `wide` columns of BM x 256 tiles, then columns of BM x 192, in the stages of the former.  Outputs of one and a half to two
+// rounds of workgroups leave compute units idle in the second; with the widths mixed every compute unit has about as much to do.  f16, us on
+// one width and on two: 1344 x 12032 x 4608 161, 152; 900 x 18432 x 5120 179, 172; 560 x 28672 x 4096 148, 141; 1700 x 11000 x 2048 79.6, 76.8.  Where the
+// chip is at its power limit in the first round already, idle units had given it clock: 1500 x 14336 x 4096 161.7, 160.9, and in a block over a prompt of 1500
+// nothing.
+#define GEMM_RING_MIX_KERNEL(NAME, BM, T)                                                                                           \
+  extern "C" __global__ void __launch_bounds__(512)                                                                                 \
+      gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k, TileGrid g, int32_t accumulate,               \
+                         float*, uint32_t*, uint32_t narrow) {                                                                      \
+    using Wide = GemmRing16<BM, 256, 2, 4, T, T>;                                                                                   \
+    using Narrow = GemmRing16<BM, 256, 2, 4, T, T, 192>;                                                                            \
+    __shared__ __attribute__((aligned(1024))) unsigned char xs0[Wide::kABytes];                                                     \
+    __shared__ __attribute__((aligned(1024))) unsigned char xs1[Wide::kABytes];                                                     \
+    __shared__ __attribute__((aligned(1024))) unsigned char xs2[Wide::kABytes];                                                     \
+    __shared__ __attribute__((aligned(1024))) unsigned char ys0a[Wide::kBBytes / 2];                                                \
+    __shared__ __attribute__((aligned(1024))) unsigned char ys0b[Wide::kBBytes / 2];                                                \
+    __shared__ __attribute__((aligned(1024))) unsigned char ys1a[Wide::kBBytes / 2];                                                \
+    __shared__ __attribute__((aligned(1024))) unsigned char ys1b[Wide::kBBytes / 2];                                                \
+    const uint32_t first = g.x * g.y;                                                                                               \
+    uint32_t pm, pn;                                                                                                                \
+    if (blockIdx.x < first) {                                                                                                       \
+      grouped_tile(xcd_contiguous(blockIdx.x, first), g.x, g.y, &pm, &pn);                                                          \
+      Wide::run_tile_in({xs0, xs1, xs2, ys0a, ys0b, ys1a, ys1b}, z, x, y, k, pm, pn, accumulate);                                   \
+    } else {                                                                                                                        \
+      grouped_tile(xcd_contiguous(blockIdx.x - first, g.x * narrow), g.x, narrow, &pm, &pn);                                        \
+      const int32_t at = (int32_t)g.y * 256;                                                                                        \
+      y.ptr = (T*)y.ptr + at, y.shape[1] -= at;                                                                                     \
+      z.ptr = (T*)z.ptr + at, z.shape[1] -= at;                                                                                     \
+      Narrow::run_tile_in({xs0, xs1, xs2, ys0a, ys0b, ys1a, ys1b}, z, x, y, k, pm, pn, accumulate);                                 \
+    }                                                                                                                               \
+  }

@@ -9,7 +9,8 @@ using namespace cutile::gemm;
 
 #define GEMM_TILES_FAMILY(N, T)                                       \
   GEMM_STAGES_KERNEL(N##_128x128x64_q2x2_lone, 128, 128, 2, 4, 5, T)  \
-  GEMM_RING_TILE_KERNEL(N##_256x256x64_q2x4_split, 256, 256, 2, 4, T)
+  GEMM_RING_TILE_KERNEL(N##_256x256x64_q2x4_split, 256, 256, 2, 4, T) \
+  GEMM_RING_MIX_KERNEL(N##_192x256x64_q2x4_mix, 192, T)
 GEMM_TILES_FAMILY(bf16, __bf16)
 GEMM_TILES_FAMILY(f16, _Float16)
 
