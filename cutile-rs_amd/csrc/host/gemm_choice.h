@@ -84,10 +84,25 @@ inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, in
 
 // 16-bit weights of this size are not found in the caches by the launch that reads them next (gemm_thin.h).
 inline bool streamed_past_caches(int64_t n, int32_t k) { return n * k * 2 >= (96ll << 20); }
-// K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8
-// wavefronts (N = K = 4096, one row: 19.1, 12.6, 10.4, 11.3, 15.4 us with 1, 2, 4, 8, 16 splits; K = 1024: 5.0, 5.3, 5.8, 7.2).
-inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus) {
-  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), k / (64 * 8 * 2)));
+// K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8 wavefronts; strips of 16 rows and 64 columns,
+// where a split costs least, one step, as far as 8 splits (operands from memory, one row, us with K / 1024 and K / 512 of them: 64 x 4096 6.6, 5.2; 1024 x 2048 7.5, 5.8;
+// 3072 x 2048 8.0, 6.4; 2560 x 2560 10.5, 6.7; 30 rows of 4096 x 4096, in 4 and 8, 11.6, 13.9).
+inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus, bool narrow) {
+  blocks = std::max<uint64_t>(blocks, 1);
+  if (!narrow) return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / blocks), k / (64 * 8 * 2)));
+  // Where one workgroup to a compute unit leaves some of them idle, two or three (at most 8 to a strip), if the longest share of K, in whole
+  // steps of its wavefronts, is no longer for it - and shorter where K would not be shared at all (4096 x 6144, 96 strips, in 2, 5 and 8: 13.9, 14.3, 13.0 us;
+  // 4096 x 11008, 172, in 1 and 4: 19.7, 18.2; 5120 x 5120, 80, in 3 and 6: 15.4, 13.9; 1024 x 14000, 219, in 1 and 2: 7.5, 9.0).
+  const int64_t halves = k / (64 * 8 * 2), most = k < 1536 ? halves : std::min<int64_t>(k / (64 * 8), std::max<int64_t>(8, halves));   // (1305 x 808 5.6, 5.9)
+  int64_t best = std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / blocks), most));
+  auto share = [&](int64_t s, int64_t deep) { return (double)(deep * ((k + s * 512 - 1) / (s * 512))); };   // steps of a wavefront, workgroup after workgroup
+  if (best * (int64_t)blocks <= cus && best < most)
+    for (int64_t deep = 2; deep <= 3; ++deep) {
+      const int64_t s = std::min<int64_t>({(int64_t)((uint64_t)(deep * cus) / blocks), most, 8});
+      const double was = share(best, (best * (int64_t)blocks + cus - 1) / cus), is = share(s, (s * (int64_t)blocks + cus - 1) / cus);
+      if (s > best && is <= was * (best == 1 ? 0.9 : 1.0)) best = s;
+    }
+  return (uint32_t)best;
 }
 // K splits of a staged launch, as priced below and as launched: 64 x 64 tiles only (64 x 128 with two splits and with none: 336 x
 // 2575 x 1350 21.9, 17.8 us; 586 x 1537 x 1527 25.8, 20.4; 193 x 867 x 1070 17.0, 15.5; 130 x 1001 x 1030 15.8, 14.4), up to two workgroups per compute unit, at least 8 K tiles each (1262 x 128 x 16128, 40 tiles: 99, 54, 40, 32,
