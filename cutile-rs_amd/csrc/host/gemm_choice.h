@@ -271,6 +271,16 @@ struct ScaledShape {
 inline uint32_t scaled_splits(uint64_t blocks, int32_t pieces, int cus) {
   return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / 2 / std::max<uint64_t>(blocks, 1)), pieces / (2 * 8 * 2)));
 }
+// As launched, which the prices below do not know: strips of up to 64 x 64 outputs, whose partial sums are few, in one round of a workgroup to each compute unit, and
+// finer where K is long (partial sums are read eight at a time, split_k.h).  Operands from memory, us as above and so: mxfp8 8 x 4096 x 4096 10.0, 9.3; 1 x 5120 x
+// 5120 15.5, 11.1; 60 x 4096 x 4096 14.2, 12.5; 8 x 896 x 5248 9.3, 7.4; nvfp4 1 x 1088 x 6656 13.2, 10.4; 8 x 896 x 5248 13.4, 10.6.  (Shorter ones in
+// two instead of one: mxfp8 16 x 2048 x 2048 6.5, 7.7; nvfp4 8 x 4096 x 4096 9.4, 10.8.)
+inline uint32_t scaled_launch_splits(uint64_t blocks, int32_t pieces, int cus, bool fp4, int bm, int bn) {
+  const uint32_t priced = scaled_splits(blocks, pieces, cus);
+  if (bm * bn > 64 * 64) return priced;
+  const int64_t most = fp4 ? pieces / 20 : pieces < 64 ? pieces / 32 : pieces / 16;
+  return std::max(priced, (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), most, 8})));
+}
 // fp8 on 128 x 128 tiles that have a compute unit each (mxfp8_tiles.hip), K shared by up to 8 workgroups in whole blocks of 512 positions: us a K tile
 // of 128 where few compute units are busy and where all are, us of start and output, and of partial tiles (113 times of 54 products, 9.5 % rms).
 // Against the two-stage kernel: 1000 x 4096 x 4096 26.5 -> 22.3 us, 1943 x 1472 x 7296 50 -> 37, 459 x 4416 x 512 7.6 -> 6.6; against strips, with K

@@ -451,7 +451,7 @@ cutile_status_t launch_scaled(Resolved& res, cutile_stream_t stream, const cutil
     const uint32_t tiles_m = div_up(zt.shape[0], res.entry->tile[3]), tiles_n = div_up(zt.shape[1], res.entry->tile[1]);
     const uint64_t blocks = (uint64_t)tiles_m * tiles_n;
     SplitWorkspace ws;
-    uint32_t splits = std::min(scaled_splits(blocks, pieces, cus),
+    uint32_t splits = std::min(scaled_launch_splits(blocks, pieces, cus, x->dtype == CUTILE_DTYPE_F4E2M1FNX2, res.entry->tile[3], res.entry->tile[1]),
                                split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (splits > 1 && g_launch_mode == 0) {
       ws = split_workspace(res.device, (hipStream_t)stream);
