@@ -84,17 +84,17 @@ inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, in
 
 // 16-bit weights of this size are not found in the caches by the launch that reads them next (gemm_thin.h).
 inline bool streamed_past_caches(int64_t n, int32_t k) { return n * k * 2 >= (96ll << 20); }
-// K splits of a thin launch: about one workgroup per compute unit, and at least two 64-row steps for each of its 8 wavefronts; strips of 16 rows and 64 columns,
-// where a split costs least, one step, as far as 8 splits (operands from memory, one row, us with K / 1024 and K / 512 of them: 64 x 4096 6.6, 5.2; 1024 x 2048 7.5, 5.8;
-// 3072 x 2048 8.0, 6.4; 2560 x 2560 10.5, 6.7; 30 rows of 4096 x 4096, in 4 and 8, 11.6, 13.9).
-inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus, bool narrow) {
+// K splits of a thin launch: about one workgroup per compute unit, and at least one 64-row step for each of its 8 wavefronts as far as 8 splits, two beyond
+// (operands from memory, us with two steps and with one: 1 x 64 x 4096 6.6, 5.2; 1 x 1024 x 2048 7.5, 5.8; 1 x 2560 x 2560 10.5, 6.7; 20 x 512 x 4096
+// 8.6, 6.6; 30 x 2560 x 2560 13.5, 8.0; 40 x 3000 x 3001 22.2, 16.7; 48 x 2048 x 4096 12.0, 10.2).  Strips of 128 columns, which are many: two steps.
+inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus, int rows, int cols) {
   blocks = std::max<uint64_t>(blocks, 1);
-  if (!narrow) return (uint32_t)std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / blocks), k / (64 * 8 * 2)));
+  const int64_t halves = k / (64 * 8 * 2), most = cols == 128 || (rows == 16 && k < 1536) ? halves : std::min<int64_t>(k / (64 * 8), std::max<int64_t>(8, halves));   // (1 x 808 x 1305 5.6, 5.9)
+  int64_t best = std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / blocks), most));
+  if (rows > 16 || cols == 128) return (uint32_t)best;   // (a second workgroup to a compute unit: 30 x 6144 x 4096 17.1, 19.1; 30 x 3072 x 2048 7.8, 8.5)
   // Where one workgroup to a compute unit leaves some of them idle, two or three (at most 8 to a strip), if the longest share of K, in whole
   // steps of its wavefronts, is no longer for it - and shorter where K would not be shared at all (4096 x 6144, 96 strips, in 2, 5 and 8: 13.9, 14.3, 13.0 us;
   // 4096 x 11008, 172, in 1 and 4: 19.7, 18.2; 5120 x 5120, 80, in 3 and 6: 15.4, 13.9; 1024 x 14000, 219, in 1 and 2: 7.5, 9.0).
-  const int64_t halves = k / (64 * 8 * 2), most = k < 1536 ? halves : std::min<int64_t>(k / (64 * 8), std::max<int64_t>(8, halves));   // (1305 x 808 5.6, 5.9)
-  int64_t best = std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / blocks), most));
   auto share = [&](int64_t s, int64_t deep) { return (double)(deep * ((k + s * 512 - 1) / (s * 512))); };   // steps of a wavefront, workgroup after workgroup
   if (best * (int64_t)blocks <= cus && best < most)
     for (int64_t deep = 2; deep <= 3; ++deep) {
