@@ -2022,10 +2022,11 @@ cutile_status_t cutile_scratch_capacity(size_t* bytes) {
   return CUTILE_SUCCESS;
 }
 
-// The splits of a launch that its own workgroups merge (fmha.hip, merge_if_last): a lane to a split, a counter to a head, 16-byte stores of out.
-static bool merges_in_split(const cutile_partition_arg_t& out, int32_t kv_heads, int32_t splits) {
+// The splits of a launch that its own workgroups merge (fmha.hip, merge_if_last): a lane to a split, a counter to a head, 16-byte stores of out;
+// and counters behind the partial results, which a scratch library built before there were any does not have.
+static bool merges_in_split(const cutile_partition_arg_t& out, int32_t kv_heads, int32_t splits, size_t capacity) {
   const cutile_tensor_arg_t& t = out.tensor;
-  return splits <= 64 && kv_heads <= (int32_t)CUTILE_SCRATCH_HEADS && decode_vec_layout(t);
+  return splits <= 64 && kv_heads <= (int32_t)CUTILE_SCRATCH_HEADS && capacity >= (size_t)CUTILE_SCRATCH_BYTES + CUTILE_SCRATCH_COUNTER_BYTES && decode_vec_layout(t);
 }
 
 cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, const cutile_tensor_arg_t* q,
@@ -2084,7 +2085,7 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
   uint32_t merge_grid[3];
   if (cutile_status_t s = check_merge(&att.tensor, &lse.tensor, out, nullptr, merge_grid)) return s;
   MergeInto merge{out, nullptr, nullptr, false};
-  bool together = merges_in_split(*out, kv_heads, num_kv_splits);
+  bool together = merges_in_split(*out, kv_heads, num_kv_splits, capacity);
   if (together && g_launch_mode == 0) {
     // A captured launch takes the two kernels, which leave nothing behind: a graph may be replayed beside other work.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;

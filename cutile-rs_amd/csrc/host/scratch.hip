@@ -26,7 +26,7 @@ std::mutex g_mutex;
 void* g_ptr[kMaxDevices] = {};
 }  // namespace
 
-// The device address of the calling thread's current GPU's copy of the array.
+// The device address of the calling thread's current GPU's copy of the array, and its size with the counters.
 // Looked up once per device, with that device current (it is: the lookup asks the
 // runtime for the current device and resolves the symbol there).  Returns the
 // hipError_t of the failing runtime call, 0 on success.
@@ -48,7 +48,7 @@ extern "C" int cutile_scratch_lookup(void** device_ptr, size_t* bytes, int* devi
     g_ptr[dev] = p;
   }
   *device_ptr = g_ptr[dev];
-  *bytes = (size_t)CUTILE_SCRATCH_BYTES;
+  *bytes = (size_t)CUTILE_SCRATCH_BYTES + CUTILE_SCRATCH_COUNTER_BYTES;
   if (device_ordinal) *device_ordinal = dev;
   return 0;
 }
