@@ -2024,9 +2024,14 @@ cutile_status_t cutile_scratch_capacity(size_t* bytes) {
 
 // The splits of a launch that its own workgroups merge (fmha.hip, merge_if_last): a lane to a split, a counter to a head, 16-byte stores of out;
 // and counters behind the partial results, which a scratch library built before there were any does not have.
-static bool merges_in_split(const cutile_partition_arg_t& out, int32_t kv_heads, int32_t splits, size_t capacity) {
+// In launches that the compute units hold at once: one and a half workgroups to each, or one where LDS has no room for two.  Beyond, what a merge
+// saves is lost to workgroups that wait for their partial results to pass the L2 and count (two launches and one, us: GROUP 1, D = 64, 64 heads
+// of 100 keys in 64 splits 15.3, 25.0; GROUP 4, D = 256, 12 heads in 32 1.10 times).  1872 sizes up to that line take 0.78 times the time of two
+// launches and none of them more than 1.00; beyond, of 512 to 4096 workgroups, 0.73 to 1.78 times.
+static bool merges_in_split(const cutile_partition_arg_t& out, int32_t kv_heads, int32_t splits, size_t capacity, int cus) {
   const cutile_tensor_arg_t& t = out.tensor;
-  return splits <= 64 && kv_heads <= (int32_t)CUTILE_SCRATCH_HEADS && capacity >= (size_t)CUTILE_SCRATCH_BYTES + CUTILE_SCRATCH_COUNTER_BYTES && decode_vec_layout(t);
+  const int64_t room = t.shape[2] == 256 ? cus : cus * 3 / 2;
+  return splits <= 64 && (int64_t)kv_heads * splits <= room && kv_heads <= (int32_t)CUTILE_SCRATCH_HEADS && capacity >= (size_t)CUTILE_SCRATCH_BYTES + CUTILE_SCRATCH_COUNTER_BYTES && decode_vec_layout(t);
 }
 
 cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, const cutile_tensor_arg_t* q,
@@ -2085,7 +2090,9 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
   uint32_t merge_grid[3];
   if (cutile_status_t s = check_merge(&att.tensor, &lse.tensor, out, nullptr, merge_grid)) return s;
   MergeInto merge{out, nullptr, nullptr, false};
-  bool together = merges_in_split(*out, kv_heads, num_kv_splits, capacity);
+  int cus = 256;
+  if (cutile_status_t s = current_device_units(&cus)) return s;
+  bool together = merges_in_split(*out, kv_heads, num_kv_splits, capacity, cus);
   if (together && g_launch_mode == 0) {
     // A captured launch takes the two kernels, which leave nothing behind: a graph may be replayed beside other work.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;

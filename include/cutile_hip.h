@@ -572,8 +572,9 @@ cutile_status_t cutile_launch_splitk_reduce_merge(cutile_stream_t stream, const 
  * is allocated or freed, here or in the kernels.  Every call on one GPU uses that GPU's one array: calls that overlap
  * on one GPU (two streams, two threads) race; calls on one stream are ordered.  Nothing in the array has to start
  * at zero — the split kernel writes every row a merge reads — so nothing is cleared between calls.  Up to GROUP 4, 64
- * heads and 64 splits the call is one launch, whose workgroups count in 16 KiB behind the array (zeros between
- * launches); while the stream is being captured, and beyond, it is two. */
+ * heads and 64 splits, and one and a half workgroups (a head and a split each) to a compute unit (D = 256: one), the
+ * call is one launch, whose workgroups count in 16 KiB behind the array (zeros between launches); while the stream is
+ * being captured, and beyond, it is two. */
 cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, const cutile_tensor_arg_t* q,
                                                       const cutile_tensor_arg_t* k, const cutile_tensor_arg_t* v,
                                                       const cutile_partition_arg_t* out, float qk_scale,
