@@ -2783,17 +2783,22 @@ namespace {
 //   D = 64: 8 heads of 1024 (256 workgroups of 32 rows) 21, 13 and 10.5; 16 of 1024 21, 13 and 15; 32 of 1024 (512 of 64 rows) 22, 18.5 and 27;
 //     512 of short keys lose: 128 heads of 256 8.9, 10 and 19; 1024 of 64 rows pay where causal tiles even out: 32 heads of 2048 causal 52, 41
 //     and 73, not causal 55, 60 and 110
-//   Two rounds of 64 rows at D = 128 pay where causal tiles are long (8 heads of 4096 80.8 and 66.5; 32 of 1024 25.6 and 27.0).
+//   Two rounds of 64 rows at D = 128 pay where causal tiles are long (8 heads of 4096 80.8 and 66.5; 32 of 1024 25.6 and 27.0) and of
+//     different lengths: keys in front of the rows (`start`) make them alike, and then the 256-row kernel, which reads K and V a quarter as often, is
+//     the better one, the sooner the more workgroups there are (f16; 8 heads of 2408 behind 664 63 and 51, behind 2408 93 and 90, behind 4816 141 and 153; 4
+//     of 8192 behind 1024 170 and 160, behind 4096 225 and 235; 32 of 1024 behind 3000 84 and 111, 40 of 512 behind 7000 143 and 215).  Over 130
+//     launches on this side of the line 0.68 to 1.00 of its time.  (With the position on the device the other kernel is the one of 128 rows: 0.68 to 0.95 of its
+//     time wherever the rows begin, 32 heads of 1024 at 0 33 and 28, behind 3000 113 and 101.)
 // Every other launch of D = 64 has two wavefronts to 32 rows of the 128-row workgroup (us on one wavefront and on two: 32 heads of 4096 196 and 180, causal 109
 // and 102; 128 of 1024 57 and 54, 43 and 38; 256 of 256 12.1 and 13.1, causal 13.0 and 12.8).
 // Up to 128 keys there is nothing to share (one head of 64: 6.5, 8.0 and 8.3; of 129: 9.4, 8.2 and 8.3).
-int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, bool causal, int cus) {
+int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t start, bool causal, int cus) {
   if ((d != 64 && d != 128) || keys <= 128) return 0;
   const int64_t of32 = heads * ((rows + 31) / 32), of64 = heads * ((rows + 63) / 64);
   if (of32 <= cus) return 32;
   if (of64 <= cus) return 64;
   if (d == 64 && ((of64 <= 2 * cus && keys >= 512) || (of64 <= 4 * cus && causal && keys >= 1024))) return 64;
-  if (d == 128 && causal && of64 <= 2 * cus && keys >= 3072) return 64;
+  if (d == 128 && causal && of64 <= 2 * cus && keys >= 3072 && (double)start <= (double)rows * (1.1 - 0.45 * (double)of64 / cus)) return 64;
   return d == 64 && keys >= (causal ? 200 : 300) ? 128 : 0;
 }
 // (by their own rows, not by the family whose place they take)
@@ -2869,7 +2874,7 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   if (bm >= 128 && bn_user == 0 && (int64_t)tg[1] * bm >= ot.shape[1]) {
     int cus = 256;
     if (cutile_status_t s = current_device_units(&cus)) return s;
-    key_rows = key_sharing_rows(d, tg[0], ot.shape[1], causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2], causal, cus);
+    key_rows = key_sharing_rows(d, tg[0], ot.shape[1], causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2], input_pos, causal, cus);
   }
   if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, key_rows ? fallback : std::string())) return s;
   if (key_rows && g_last_source == "size") {
@@ -2987,7 +2992,7 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
     const int64_t seen = position_start ? max_seq : kv_len;
     int cus = 256;
     if (cutile_status_t s = current_device_units(&cus)) return s;
-    key_rows = key_sharing_rows(d, heads_cov, rows_cov, causal && !position_start ? std::min<int64_t>((int64_t)query_start + rows_cov, seen) : seen, causal, cus);
+    key_rows = key_sharing_rows(d, heads_cov, rows_cov, causal && !position_start ? std::min<int64_t>((int64_t)query_start + rows_cov, seen) : seen, position_start ? 0 : query_start, causal, cus);
   }
   if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, key_rows ? acceptable[0] : std::string())) return s;
   if (key_rows && g_last_source == "size")
