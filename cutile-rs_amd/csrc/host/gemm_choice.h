@@ -153,6 +153,20 @@ struct GemmChoice {
   F32Plan strip_plan{};
 };
 
+// Register-staged tiles and their prices (choose_gemm), for rows off 16-byte boundaries and on them.  (Tables are constants of this file: a
+// static of an inline function is one object for all builds of the library in a process, whichever is loaded first.)
+struct StagedTile {
+  const char* kernel;
+  int bm, bn, per_cu;
+  struct Any { double one, more, ends, x, split, sum; } any;
+  struct Aligned { double one, more, ends, split, sum; } aligned;
+};
+constexpr StagedTile kStaged[] = {{"staged256x256", 256, 256, 1, {1.14, 0, 12.7, 0.126, 0, 0}, {}},
+                                  {"staged256x128", 256, 128, 1, {0.77, 0, 8.2, 0.142, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
+                                  {"staged128x128", 128, 128, 2, {0.50, 0.52, 6.7, 0.139, 0, 0}, {0.715, 0.625, 5.05, 0, 0}},
+                                  {"staged64x128", 64, 128, 3, {0.32, 0.39, 6.0, 0.074, 0, 0}, {0.55, 0.43, 3.9, 0, 0}},
+                                  {"staged64x64", 64, 64, 4, {0.228, 0.2725, 4.5, 0.046, 2.4, 2.1e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
+
 inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_bytes) {
   GemmChoice c;
   if (strcmp(s.dtype, "f32") == 0) {
@@ -223,14 +237,6 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
     // x 4096 14.3 us on the ring, 11.8; 665 x 320 x 704 on these 6.8, on the ring 8.0).  With the first set for them, ring tiles were taken for small
     // outputs of middling K (us with ring, 64 x 64 and two-stage tiles: 220 x 64 x 1408 14.4, 9.3, 11.5).
     // (0.265: with the fitted 0.257 the two K / V projections of 1500 x 1024 x 4096, 384 tiles of 64 x 64, took 42 us each, on the ring 40)
-    struct Any { double one, more, ends, x, split, sum; };
-    struct Aligned { double one, more, ends, split, sum; };
-    struct StagedTile { const char* kernel; int bm, bn, per_cu; Any any; Aligned aligned; };
-    static const StagedTile kStaged[] = {{"staged256x256", 256, 256, 1, {1.14, 0, 12.7, 0.126, 0, 0}, {}},
-                                         {"staged256x128", 256, 128, 1, {0.77, 0, 8.2, 0.142, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
-                                         {"staged128x128", 128, 128, 2, {0.50, 0.52, 6.7, 0.139, 0, 0}, {0.715, 0.625, 5.05, 0, 0}},
-                                         {"staged64x128", 64, 128, 3, {0.32, 0.39, 6.0, 0.074, 0, 0}, {0.55, 0.43, 3.9, 0, 0}},
-                                         {"staged64x64", 64, 64, 4, {0.228, 0.2725, 4.5, 0.046, 2.4, 2.1e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
     for (const StagedTile& r : kStaged) {
       if (s.y_cols < r.bn || (ring && r.bn == 256)) continue;
       const uint64_t t = tiles(r.bm, r.bn), would_share = staged_splits(r.bm, r.bn, t, s.k, cus), sk = partial_bytes ? would_share : 1;
@@ -238,14 +244,14 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       if (ring) {
         const double w = (double)((t * sk + cus - 1) / cus);
         if (r.per_cu == 1 && w > 2) continue;
-        const Aligned& a = r.aligned;
+        const StagedTile::Aligned& a = r.aligned;
         // (a long K that there is no room to share: priced so that 128 x 128 tiles take it)
         const double one = sk < would_share ? 0.40 : a.one;
         us = kt / (double)sk * std::max(one * std::max(1.0, w / r.per_cu), a.more * w) + a.ends + (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
       } else {
         const uint64_t slots = (uint64_t)cus * r.per_cu, rounds = t * sk / slots, rest = t * sk % slots;
         if (r.per_cu == 1 && rounds >= 2 && kt < 8) continue;
-        const Any& a = r.any;
+        const StagedTile::Any& a = r.any;
         const double ends = a.ends + (r.bn == 256 && s.k % 64 != 0 ? 1.8 : 0.0);   // (there a ragged K tile stands behind the sequence)
         auto round = [&](uint64_t each) { return kt / (double)sk * std::max(a.one, a.more * (double)each) + ends; };
         us = ((double)rounds * round(r.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0)) * (s.x_aligned ? 1.0 : 1.0 + a.x) +
@@ -302,6 +308,14 @@ inline MxPlan mx_plan(int64_t m, int64_t n, int32_t pieces, int cus, uint64_t pa
   }
   return best;
 }
+// Strips of scaled_flat.hip, us a piece of K of each format.
+struct FlatStrip {
+  const char* name;
+  int bm, bn;
+  double fp8, fp4;
+};
+constexpr FlatStrip kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20}, {"flat32x64", 32, 64, 0.12, 0.28}, {"flat64x64", 64, 64, 0.155, 0.36},
+                               {"flat64x128", 64, 128, 0.27, 0.62}, {"flat128x128", 128, 128, 0.52, 1.12}};
 // The kernel by name, or nullptr: the partition's own (tuning record, then the table's order).  us per 64-byte piece of K for
 // one block on each compute unit, measured at K = 4096 (mxfp8: 16 x 4096 9.4 us, 64 x 4096 13.4, 512 x 4096 21 on 64 x 128 blocks, 24 with
 // 128 x 128 tiles; nvfp4: 9.9, 14.7, 24).  The 256 x 256 kernels are the better ones where their tiles come near to filling the chip.
@@ -313,12 +327,9 @@ inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int
   auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
   if (!tiled && s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
   // (fp8 on 128 x 128: the direct pipeline below is always the cheaper one; only a name reaches flat128x128 there)
-  struct Kernel { const char* name; int bm, bn; double fp8, fp4; };
-  static const Kernel kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20}, {"flat32x64", 32, 64, 0.12, 0.28}, {"flat64x64", 64, 64, 0.155, 0.36},
-                                 {"flat64x128", 64, 128, 0.27, 0.62}, {"flat128x128", 128, 128, 0.52, 1.12}};
   const char* name = nullptr;
   double best = 1e30;
-  for (const Kernel& k : kFlat) {
+  for (const FlatStrip& k : kFlat) {
     const uint64_t b = blocks(k.bm, k.bn), waves = (b + cus - 1) / cus;
     if (s.pieces <= 4) break;
     const double us = (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + (s.fp4 && waves > 1 ? 5.5 : 3.5));

@@ -784,6 +784,16 @@ def test_lds_bytes_of_the_table_are_those_of_the_code_objects(fake_hip, image, e
         assert ct.kernel_lookup(function, variant=variant).lds_bytes == int(re.search(r"\.group_segment_fixed_size: (\d+)", kernel)[1]), symbol
 
 
+def test_two_builds_in_one_process_share_no_tables(fake_hip):
+    """A static of an inline function is a symbol that the loader makes one of in a process: a second build of the library then priced its
+    kernels by the first one's table, and where the layout had changed divided by zero."""
+    import subprocess
+
+    symbols = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--dyn-syms", "-W", fake_hip.TESTING_LIB_PATH], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert "cutile_launch_gemm" in symbols
+    assert [s for s in symbols.splitlines() if "UNIQUE" in s and ("_ZZN6cutile" in s or "_ZN6cutile" in s)] == []
+
+
 def test_shipped_tuning_records_are_those_of_this_build():
     """a change to a kernel's code object makes the library refuse its record, and with it the measured winners: re-tune
     (cutile-rs_amd/bin/tune_baseline) or delete it"""
