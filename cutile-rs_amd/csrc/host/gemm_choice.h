@@ -87,20 +87,36 @@ inline bool streamed_past_caches(int64_t n, int32_t k) { return n * k * 2 >= (96
 // K splits of a thin launch: about one workgroup per compute unit, and at least one 64-row step for each of its 8 wavefronts as far as 8 splits, two beyond
 // (operands from memory, us with two steps and with one: 1 x 64 x 4096 6.6, 5.2; 1 x 1024 x 2048 7.5, 5.8; 1 x 2560 x 2560 10.5, 6.7; 20 x 512 x 4096
 // 8.6, 6.6; 30 x 2560 x 2560 13.5, 8.0; 40 x 3000 x 3001 22.2, 16.7; 48 x 2048 x 4096 12.0, 10.2).  Strips of 128 columns, which are many: two steps.
-inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus, int rows, int cols) {
+// `aligned`: rows on 16-byte boundaries.  Off them a step takes longer and sharing pays sooner (K in 1 and in 2: 16 x 7552 x 1856 7.7,
+// 8.4; 8 x 5730 x 1852 8.4, 7.6).  Over 917 products of 1 to 128 rows (K 1024 to 16384) the split chosen here takes 1.015 of the best one's time in the mean, and
+// at most 1.08 of what two steps to a wavefront take; the three rules that `aligned` selects take their part of them from as much as 1.21 to 1.04.
+inline uint32_t thin_splits(uint64_t blocks, int32_t k, int cus, int rows, int cols, bool aligned) {
   blocks = std::max<uint64_t>(blocks, 1);
-  const int64_t halves = k / (64 * 8 * 2), most = cols == 128 || (rows == 16 && k < 1536) ? halves : std::min<int64_t>(k / (64 * 8), std::max<int64_t>(8, halves));   // (1 x 808 x 1305 5.6, 5.9)
-  int64_t best = std::max<int64_t>(1, std::min<int64_t>((int64_t)((uint64_t)cus / blocks), most));
+  const int64_t halves = k / (64 * 8 * 2), n = (int64_t)blocks;
+  // Beyond a quarter of the compute units a short K gains nothing from one step to a wavefront (us in 1 and more: 8 x 5632 x 1536 6.5, 7.2; 7 x 4288 x 2048
+  // in 2 and 4 6.7, 7.4; 22 x 7616 x 1600 7.7, 8.6; 120 x 3648 x 1088 9.0, 9.6) but where three shares of the strips lie evenly over the XCDs (24 x 5120 x 1536 8.3, 7.2).
+  const bool short_k = aligned && n * 9 > 2 * cus && (rows == 64 ? k < 1152 : k < 2240 && !(n % 8 == 0 && n * 3 <= cus && k >= 1536));
+  const int64_t most = cols == 128 || (rows == 16 && k < 1536) || short_k ? halves : std::min<int64_t>(k / (64 * 8), std::max<int64_t>(8, halves));   // (1 x 808 x 1305 5.6, 5.9)
+  int64_t best = std::max<int64_t>(1, std::min<int64_t>(cus / n, most));
+  if (aligned && best * n * 2 > cus) {   // no more of them than the longest share asks for, if they come out even (12 x 3072 x 3072 in 3, 5 and 6: 7.2, 7.9, 7.9 us)
+    const int64_t steps = k / 64, longest = (steps + 8 * best - 1) / (8 * best), even = steps / std::max<int64_t>(8 * longest, 1);
+    if (even > 0 && even * 8 * longest == steps) best = even;
+  }
   if (rows > 16 || cols == 128) return (uint32_t)best;   // (a second workgroup to a compute unit: 30 x 6144 x 4096 17.1, 19.1; 30 x 3072 x 2048 7.8, 8.5)
   // Where one workgroup to a compute unit leaves some of them idle, two or three (at most 8 to a strip), if the longest share of K, in whole
-  // steps of its wavefronts, is no longer for it - and shorter where K would not be shared at all (4096 x 6144, 96 strips, in 2, 5 and 8: 13.9, 14.3, 13.0 us;
-  // 4096 x 11008, 172, in 1 and 4: 19.7, 18.2; 5120 x 5120, 80, in 3 and 6: 15.4, 13.9; 1024 x 14000, 219, in 1 and 2: 7.5, 9.0).
+  // steps of its wavefronts, is shorter for it, or no longer where the last round is nearly full (1 x 4480 x 4096 in 3 and 8, 560 workgroups: 8.9, 10.1; 3 x 6080 x 3072
+  // in 2 and 6, 570: 9.1, 10.0) - and shorter by a tenth where K would not be shared at all, of 2560 and more (3 x 10304 x 2496 in 1 and 3: 11.5, 11.9).
+  // (4096 x 6144, 96 strips, in 2, 5 and 8: 13.9, 14.3, 13.0 us; 4096 x 11008, 172, in 1 and 4: 19.7, 18.2; 5120 x 5120, 80, in 3 and 6: 15.4, 13.9;
+  // 1024 x 14000, 219, in 1 and 2: 7.5, 9.0).
+  if (aligned && best == 1 && k < 2560) return 1;
   auto share = [&](int64_t s, int64_t deep) { return (double)(deep * ((k + s * 512 - 1) / (s * 512))); };   // steps of a wavefront, workgroup after workgroup
-  if (best * (int64_t)blocks <= cus && best < most)
+  const bool alone = best == 1;
+  if (best * n <= cus && best < most)
     for (int64_t deep = 2; deep <= 3; ++deep) {
-      const int64_t s = std::min<int64_t>({(int64_t)((uint64_t)(deep * cus) / blocks), most, 8});
-      const double was = share(best, (best * (int64_t)blocks + cus - 1) / cus), is = share(s, (s * (int64_t)blocks + cus - 1) / cus);
-      if (s > best && is <= was * (best == 1 ? 0.9 : 1.0)) best = s;
+      const int64_t s = std::min<int64_t>({deep * cus / n, most, 8});
+      if (s <= best || s * n <= (deep - 1) * cus) continue;
+      const double was = share(best, (best * n + cus - 1) / cus) * (best == 1 ? 0.9 : 1.0), is = share(s, deep);
+      if (is < was || (is == was && (!aligned || alone || s * n * 10 >= 9 * deep * cus))) best = s;
     }
   return (uint32_t)best;
 }

@@ -18,6 +18,19 @@ def test_k_goes_to_a_workgroup_for_each_eight_steps(fake_hip, m, strip):
         assert _workgroups(ct) == 3 * shares, k
 
 
+def test_shares_where_strips_fill_a_quarter_of_the_compute_units_and_more(fake_hip):
+    """a short K of aligned rows in fewer shares than there are steps, even shares as they are, a second workgroup to a compute unit only for a
+    shorter or a nearly full round; rows off 16-byte boundaries are shared as far as steps go"""
+    ct = fake_hip
+    from test_host_abi import _workgroups
+    for m, n, k, shares in [(8, 5632, 1536, 1), (7, 4288, 2048, 2), (22, 7616, 1600, 1), (56, 7808, 1088, 1), (24, 5120, 1536, 3), (24, 3520, 1536, 3), (10, 4224, 2240, 3),
+                            (12, 3072, 3072, 3), (1, 2048, 5120, 5), (1, 4480, 4096, 3), (3, 6080, 3072, 2), (1, 4096, 4096, 8), (1, 6144, 4096, 8), (1, 10304, 2496, 1),
+                            (1, 9984, 2688, 3), (8, 5633, 1536, 3), (7, 4283, 2048, 4), (22, 7610, 1600, 2)]:
+        x, y, z = torch.empty(m, k, dtype=torch.half), torch.empty(k, n, dtype=torch.half), torch.empty(m, n, dtype=torch.half)
+        ct.gemm(ct.partition(z, [128, 128]), x, y, k, accumulate=False, generics=["f16", 128, 128, 1])
+        assert "thin" in ct.last_resolved()["variant"] and _workgroups(ct) == -(-n // 64) * shares, (m, n, k, _workgroups(ct) / -(-n // 64))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,strip", [(1, 16), (16, 16), (17, 32), (31, 32), (33, 64), (70, 64)])
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
