@@ -190,7 +190,7 @@ struct Nvfp4Gemm {
       a_addr[ks] = lds_off(wm * WM + frow, funit);
       b_addr[ks] = 2 * kABytes + lds_off(wn * WN + frow, funit);
     }
-    auto k_tile = [&](int cur, Packed& next, int32_t kt) {
+    auto k_tile = [&](int cur, Packed& next, int32_t kt, auto more) {   // more: a K tile comes behind this one
 #pragma unroll
       for (int ks = 0; ks < kSteps; ++ks) {
         f16x8 af[TM], bfr[TN];
@@ -208,18 +208,34 @@ struct Nvfp4Gemm {
               acc[tn][tm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bfr[tn], af[tm], acc[tn][tm], 0, 0, 0);
           }
         // the expansion of the next tile rides between the matrix instructions of the later K steps
-        if (ks == (SHAPE16 ? 0 : 1)) {
+        if (decltype(more)::value && ks == (SHAPE16 ? 0 : 1)) {
           store_lds(next, cur ^ 1);
           load_global(next, kt + 3);
         }
       }
-      __syncthreads();
+      if (decltype(more)::value) __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
     };
+    constexpr std::true_type kMore{};
+    constexpr std::false_type kLast{};
+    if constexpr (BM == 128 && BN == 128) {
+      // Of an even number the last tile expands nothing behind itself, and an odd one has no partner of zeros: at K = 128, two tiles, that was half
+      // of the expansions.  us: 988 x 5056 x 128 10.3 -> 9.7, 495 x 11392 x 256 12.7 -> 11.7, 988 x 5056 x 512 16.6 -> 15.3, x 4096 73 -> 69.  (The 256 x
+      // 256 kernels have no registers for another copy of the tile's code.)
+      int32_t kt = 0;
 #pragma unroll 1
-    for (int kt = 0; kt < k_tiles; kt += 2) {   // (an odd number of K tiles is followed by one of zeros)
-      k_tile(0, p1, kt);
-      k_tile(1, p0, kt + 1);
+      for (;; kt += 2) {
+        k_tile(0, p1, kt, kMore);
+        if (kt + 2 >= k_tiles) break;
+        k_tile(1, p0, kt + 1, kMore);
+      }
+      if (kt + 2 == k_tiles) k_tile(1, p0, kt + 1, kLast);
+    } else {
+#pragma unroll 1
+      for (int32_t kt = 0; kt < k_tiles; kt += 2) {   // (an odd number of K tiles is followed by one of zeros)
+        k_tile(0, p1, kt, kMore);
+        k_tile(1, p0, kt + 1, kMore);
+      }
     }
 
     OutT* zp = (OutT*)z.ptr;
