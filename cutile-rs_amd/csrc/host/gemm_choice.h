@@ -324,14 +324,15 @@ inline MxPlan mx_plan(int64_t m, int64_t n, int32_t pieces, int cus, uint64_t pa
   }
   return best;
 }
-// Strips of scaled_flat.hip, us a piece of K of each format.
+// Strips of scaled_flat.hip, us a piece of K of each format while they fit the chip once; and of fp4 strips in more rounds than one, a piece in a round that
+// few and that all compute units have, and start and output of a round.
 struct FlatStrip {
   const char* name;
   int bm, bn;
-  double fp8, fp4;
+  double fp8, fp4, few, all, ends;
 };
-constexpr FlatStrip kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20}, {"flat32x64", 32, 64, 0.12, 0.28}, {"flat64x64", 64, 64, 0.155, 0.36},
-                               {"flat64x128", 64, 128, 0.27, 0.62}, {"flat128x128", 128, 128, 0.52, 1.12}};
+constexpr FlatStrip kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20, 0.20, 0.20, 5.5}, {"flat32x64", 32, 64, 0.12, 0.28, 0.28, 0.28, 5.5}, {"flat64x64", 64, 64, 0.155, 0.36, 0.294, 0.297, 4.5},
+                               {"flat64x128", 64, 128, 0.27, 0.62, 0.534, 0.561, 4.8}, {"flat128x128", 128, 128, 0.52, 1.12, 1.053, 1.08, 5.4}};
 // The kernel by name, or nullptr: the partition's own (tuning record, then the table's order).  us per 64-byte piece of K for
 // one block on each compute unit, measured at K = 4096 (mxfp8: 16 x 4096 9.4 us, 64 x 4096 13.4, 512 x 4096 21 on 64 x 128 blocks, 24 with
 // 128 x 128 tiles; nvfp4: 9.9, 14.7, 24).  The 256 x 256 kernels are the better ones where their tiles come near to filling the chip.
@@ -345,24 +346,28 @@ inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int
   // (fp8 on 128 x 128: the direct pipeline below is always the cheaper one; only a name reaches flat128x128 there)
   const char* name = nullptr;
   double best = 1e30;
+  auto rounds = [&](uint64_t g, uint64_t at_once, double few, double all, double ends) {
+    const uint64_t rest = g % at_once;
+    return (double)(g / at_once) * (all * s.pieces + ends) + (rest ? (few + (all - few) * (double)rest / (double)at_once) * s.pieces + ends : 0.0);
+  };
   for (const FlatStrip& k : kFlat) {
     const uint64_t b = blocks(k.bm, k.bn), waves = (b + cus - 1) / cus;
     if (s.pieces <= 4) break;
-    const double us = (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + (s.fp4 && waves > 1 ? 5.5 : 3.5));
+    const double us = s.fp4 && waves > 1 ? rounds(b, cus, k.few, k.all, k.ends) : (double)waves * ((s.fp4 ? k.fp4 : k.fp8) * s.pieces / scaled_splits(b, s.pieces, cus) + 3.5);
     if (us < best) best = us, name = k.name;
   }
   if (tiled) {
-    // Whole tiles, expanded to f16 once for the workgroup: 256 x 256 to a compute unit, or two of 128 x 128.  us per piece of K and round, and of
-    // start and output (bf16 out, us on 256 x 256, 128 x 128 and the best strips: 2476 x 6080 x 896 34.7, 44.7, 54.7; 2940 x 5568 x 1152, 264 of
-    // the large tiles, 75, 54, 60; 2859 x 10368 x 512 47, 57, 67; 4096 x 4096 x 4096 117, 162, 153; 1024 x 4096 x 4096 101, 53, 44; a partition of 128
-    // x 128 had strips or the small tiles whatever the size: 58, 60, 61, 163, 46).
-    const uint64_t large = blocks(256, 256), small = blocks(128, 128), slots = 2 * (uint64_t)cus;
-    auto part = [&](uint64_t rest, double few, double all, double ends) { return rest ? (few + (all - few) * (double)rest / cus) * s.pieces + ends : 0.0; };
-    const double us256 = (double)(large / cus) * (3.5 * s.pieces + 9.5) + part(large % cus, 3.0, 3.5, 9.5);
-    const uint64_t rest = small % slots;
-    const double us128 = (double)(small / slots) * (2.4 * s.pieces + 5.0) + (rest <= (uint64_t)cus ? part(rest, 1.37, 1.52, 5.0) : part(rest - cus, 1.52, 2.4, 5.0));
-    if (us128 < best * 0.98) best = us128, name = "128x128x64_w2x2";
-    if (us256 < best * 0.98) best = us256, name = "256x256x64_q2x4";
+    // Whole tiles, expanded to f16 once for the workgroup: 256 x 256 to a compute unit, or two of 128 x 128 (2.37 a piece as soon as any has two).  Least
+    // squares, as for strips in several rounds, over 400 products of 17 to 4096 rows, operands from memory, every kernel timed (256 x 256 2.6 % rms, 128 x 128 7.8, strips 5):
+    // the kernel priced lowest takes 1.035 of the best one's time, and nowhere more than 1.04 of what strips and two-stage tiles alone took, where prices
+    // by rounds of strips and a tile's own had taken up to 1.24 (bf16 out, us on 256 x 256, 128 x 128 and the best strips: 2476 x 6080 x 896 34.7, 44.7, 54.7;
+    // 2940 x 5568 x 1152, 264 of the large tiles, 75, 54, 60; 4096 x 4096 x 4096 117, 162, 153; 1024 x 4096 x 4096 101, 53, 44; 1587 x 3328 x 7040 176, 124, 107).
+    const uint64_t small = blocks(128, 128), rest = small % (2 * (uint64_t)cus);
+    const double us256 = rounds(blocks(256, 256), cus, 2.48, 3.42, 12.1);
+    const double us128 = (double)(small / (2 * (uint64_t)cus)) * (2.48 * s.pieces + 4.5) +
+                         (rest <= (uint64_t)cus ? rounds(rest, cus, 0.87, 1.62, 4.5) : (2.37 + 0.11 * (double)(rest - cus) / cus) * s.pieces + 4.5);
+    if (us128 < best) best = us128, name = "128x128x64_w2x2";
+    if (us256 < best) best = us256, name = "256x256x64_q2x4";
     return name;
   }
   if (!s.fp4) {

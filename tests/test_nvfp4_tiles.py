@@ -26,9 +26,10 @@ def test_gpu_tiles_of_k(ct, dev, variant, m, n, tiles):
 
 
 def test_size_rule_of_a_128_partition(fake_hip):
-    """whole outputs of 240 tiles of 256 x 256 run on those, of a few more than 256 on 128 x 128, of few rows on strips"""
+    """whole outputs of 240 tiles of 256 x 256 run on those, of a few more than 256 on 128 x 128, of few rows on strips, and of a long K in some rounds too"""
     ct = fake_hip
-    for m, n, k, want in ((2476, 6080, 896, "256x256x64_q2x4"), (2940, 5568, 1152, "128x128x64_w2x2"), (200, 14336, 4096, "flat128x128"), (8, 4096, 4096, "flat16x64")):
+    for m, n, k, want in ((2476, 6080, 896, "256x256x64_q2x4"), (2940, 5568, 1152, "128x128x64_w2x2"), (200, 14336, 4096, "flat128x128"), (8, 4096, 4096, "flat16x64"),
+                          (1587, 3328, 7040, "flat64x128"), (3174, 1472, 7168, "flat64x64"), (305, 11456, 1664, "flat64x128")):
         u8 = lambda rows, cols: torch.empty(rows, cols, dtype=torch.uint8)
         ct.linear_tile_nvfp4(ct.partition(torch.empty(m, n, dtype=torch.bfloat16), [128, 128]), u8(m, k // 2), u8(n, k // 2), u8(m, k // 16), u8(n, k // 16), 1.0)
         assert ct.last_resolved()["variant"] == "bf16_" + want
