@@ -296,12 +296,15 @@ inline uint32_t scaled_splits(uint64_t blocks, int32_t pieces, int cus) {
 // As launched, which the prices below do not know: strips of up to 64 x 64 outputs, whose partial sums are few, in one round of a workgroup to each compute unit, and
 // finer where K is long (partial sums are read eight at a time, split_k.h).  Operands from memory, us as above and so: mxfp8 8 x 4096 x 4096 10.0, 9.3; 1 x 5120 x
 // 5120 15.5, 11.1; 60 x 4096 x 4096 14.2, 12.5; 8 x 896 x 5248 9.3, 7.4; nvfp4 1 x 1088 x 6656 13.2, 10.4; 8 x 896 x 5248 13.4, 10.6.  (Shorter ones in
-// two instead of one: mxfp8 16 x 2048 x 2048 6.5, 7.7; nvfp4 8 x 4096 x 4096 9.4, 10.8.)
+// two instead of one: mxfp8 16 x 2048 x 2048 6.5, 7.7; nvfp4 8 x 4096 x 4096 9.4, 10.8; and mxfp8 of less than 90 pieces and up to 32 rows where strips leave room for two only:
+// 15 x 8128 x 4736 11.1, 12.4; 1 x 8000 x 4096 9.1, 9.9; 12 x 7424 x 5632 12.2, 13.0; beyond, 2 x 8192 x 7552 20.2, 16.1.)  Over 110 products that are
+// shared finer than priced, of 1 to 100 rows, 0.85 of the time as priced, the slowest 1.02.
 inline uint32_t scaled_launch_splits(uint64_t blocks, int32_t pieces, int cus, bool fp4, int bm, int bn) {
   const uint32_t priced = scaled_splits(blocks, pieces, cus);
   if (bm * bn > 64 * 64) return priced;
-  const int64_t most = fp4 ? pieces / 20 : pieces < 64 ? pieces / 32 : pieces / 16;
-  return std::max(priced, (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1)), most, 8})));
+  const int64_t fit = (int64_t)((uint64_t)cus / std::max<uint64_t>(blocks, 1));
+  const int64_t most = fp4 ? pieces / 20 : pieces < 64 ? pieces / 32 : fit == 2 && bm < 64 && pieces < 90 ? 1 : pieces / 16;
+  return std::max(priced, (uint32_t)std::max<int64_t>(1, std::min<int64_t>({fit, most, 8})));
 }
 // fp8 on 128 x 128 tiles that have a compute unit each (mxfp8_tiles.hip), K shared by up to 8 workgroups in whole blocks of 512 positions: us a K tile
 // of 128 where few compute units are busy and where all are, us of start and output, and of partial tiles (113 times of 54 products, 9.5 % rms).

@@ -103,3 +103,16 @@ def test_gpu_register_staged_mxfp8_tiles_of_128(ct, dev, out):
     ct.linear_tile_mxfp8(ct.partition(z[:m], [128, 128]), *[_dev(v, dev) for v in (xq, yq, xs, ys)], 1.0, variant=f"mxfp8_{out}_128x128x128_w2x2")
     torch.cuda.synchronize()
     assert rel_l2(z[:m].float().cpu().numpy(), ref) <= (1e-4 if out == "f32" else 4e-3) and torch.all(z[m] == 7.0)
+
+
+def test_strips_are_shared_by_as_many_workgroups_as_there_are_compute_units(fake_hip):
+    """K of strips of up to 64 x 64 outputs, by the extents, on 256 compute units; short ones, and mxfp8 of less than 90 pieces in pairs, by their prices alone"""
+    ct = fake_hip
+    from test_host_abi import _workgroups
+    u8 = lambda rows, cols: torch.empty(rows, cols, dtype=torch.uint8)
+    for fp4, m, n, k, shares in [(0, 16, 2048, 2048, 1), (0, 8, 896, 5248, 5), (0, 1, 5120, 5120, 3), (0, 8, 4096, 4096, 4), (0, 60, 4096, 4096, 4), (0, 15, 8128, 4736, 1),
+                                 (0, 12, 7424, 5632, 1), (0, 2, 8192, 7552, 2), (0, 16, 512, 8192, 8), (1, 8, 4096, 4096, 1), (1, 1, 1088, 6656, 2), (1, 8, 896, 5248, 2)]:
+        args = (u8(m, k // 2), u8(n, k // 2), u8(m, k // 16), u8(n, k // 16)) if fp4 else (u8(m, k), u8(n, k), u8(m, k // 32), u8(n, k // 32))
+        (ct.linear_tile_nvfp4 if fp4 else ct.linear_tile_mxfp8)(ct.partition(torch.empty(m, n, dtype=torch.bfloat16), [128, 128]), *args, 1.0)
+        rows, cols = map(int, ct.last_resolved()["variant"].split("flat")[1].split("x"))
+        assert _workgroups(ct) == -(-m // rows) * -(-n // cols) * shares, (fp4, m, n, k, ct.last_resolved()["variant"], _workgroups(ct))
