@@ -2790,7 +2790,9 @@ namespace {
 //     launches on this side of the line 0.68 to 1.00 of its time.  (With the position on the device the other kernel is the one of 128 rows: 0.68 to 0.95 of its
 //     time wherever the rows begin, 32 heads of 1024 at 0 33 and 28, behind 3000 113 and 101.)
 // Every other launch of D = 64 has two wavefronts to 32 rows of the 128-row workgroup (us on one wavefront and on two: 32 heads of 4096 196 and 180, causal 109
-// and 102; 128 of 1024 57 and 54, 43 and 38; 256 of 256 12.1 and 13.1, causal 13.0 and 12.8).
+// and 102; 128 of 1024 57 and 54, 43 and 38), but where one wavefront has its keys as soon: while two workgroups to a compute unit are one round up to 448
+// keys without a mask (160 of 221 11.6 and 12.7, 128 of 354 14.6 and 15.4) and 256 under it (144 of 246 10.8 and 10.9), and under the mask up to 1000 with a
+// quarter of a round or less behind it (128 of 578 19.9 and 21.1, 192 of 294 14.3 and 14.8).  Over 500 launches of 100 to 6000 keys 0.94 of the time that all launches on one wavefront took, at most 1.02.
 // Up to 128 keys there is nothing to share (one head of 64: 6.5, 8.0 and 8.3; of 129: 9.4, 8.2 and 8.3).
 int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t start, bool causal, int cus) {
   if ((d != 64 && d != 128) || keys <= 128) return 0;
@@ -2799,7 +2801,10 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t s
   if (of64 <= cus) return 64;
   if (d == 64 && ((of64 <= 2 * cus && keys >= 512) || (of64 <= 4 * cus && causal && keys >= 1024))) return 64;
   if (d == 128 && causal && of64 <= 2 * cus && keys >= 3072 && (double)start <= (double)rows * (1.1 - 0.45 * (double)of64 / cus)) return 64;
-  return d == 64 && keys >= (causal ? 200 : 300) ? 128 : 0;
+  const int64_t of128 = heads * ((rows + 127) / 128);
+  const bool once = of128 <= 2 * cus;
+  if (d != 64 || keys < (causal ? (once ? 257 : 200) : once ? 448 : 300)) return 0;
+  return causal && rows > 256 && keys < 1000 && !once && 2 * of128 <= 5 * cus ? 0 : 128;
 }
 // (by their own rows, not by the family whose place they take)
 const KernelEntry* keys_member(const char* function, bool bf16, int rows, int d) {

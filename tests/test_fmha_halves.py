@@ -6,6 +6,19 @@ import torch
 from test_fmha_keys import _call, _close, _reference
 
 
+@pytest.mark.parametrize("heads,rows,causal,takes", [
+    (32, 2048, False, True), (32, 2049, True, True), (160, 221, False, False), (112, 447, False, False), (96, 448, False, True), (260, 300, False, True), (260, 299, False, False),
+    (160, 256, True, False), (160, 257, True, True), (300, 199, True, False), (300, 200, True, True), (128, 578, True, False), (132, 600, True, True), (192, 294, True, False), (80, 931, True, False), (64, 1100, True, True), (512, 150, True, False),
+    (240, 380, True, True),
+])
+def test_which_launches_have_two_wavefronts_to_a_row_block(fake_hip, heads, rows, causal, takes):
+    """D = 64, of 256 compute units: a round is 512 workgroups"""
+    ct = fake_hip
+    from test_host_abi import _last
+    _call(ct, torch.half, 1, heads, 1, rows, rows, 64, causal)
+    assert _last(ct)[0].symbol.decode() == "fmha_entry__f16_128x64x64" + ("_halves" if takes else "")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.half, torch.bfloat16])
 @pytest.mark.parametrize("batch,heads,group,rows,keys,causal,pos", [

@@ -1,4 +1,4 @@
-"""Attention whose workgroups share the keys of 32 or 64 query rows (short launches): which calls take it, and its results"""
+"""Attention whose workgroups share the keys of 32 or 64 query rows (short launches), or of 128 (D = 64): which calls take it, and its results"""
 import numpy as np
 import pytest
 import torch
@@ -16,8 +16,8 @@ def _call(ct, dtype, batch, heads, group, rows, keys, d, causal, pos=0, bm=128, 
 # ---- launcher on the recording runtime (CPU) ----------------------------------------------------
 @pytest.mark.parametrize("heads,rows,d,causal,takes", [
     (4, 2048, 128, True, 32), (4, 2049, 128, True, 64), (8, 2048, 128, False, 64), (8, 2049, 128, True, 0), (1, 128, 128, True, 0), (1, 129, 128, False, 32),
-    (8, 1024, 64, True, 32), (8, 1025, 64, True, 64), (32, 1024, 64, False, 64), (128, 256, 64, True, 0), (32, 2048, 64, True, 64), (32, 2048, 64, False, 0),
-    (32, 2049, 64, True, 0), (4, 512, 256, True, 0),
+    (8, 1024, 64, True, 32), (8, 1025, 64, True, 64), (32, 1024, 64, False, 64), (128, 256, 64, True, 0), (32, 2048, 64, True, 64), (32, 2048, 64, False, 128),
+    (32, 2049, 64, True, 128), (4, 512, 256, True, 0),
 ])
 def test_short_attention_shares_keys(fake_hip, heads, rows, d, causal, takes):
     ct = fake_hip
@@ -25,10 +25,10 @@ def test_short_attention_shares_keys(fake_hip, heads, rows, d, causal, takes):
     bm = 256 if d == 128 and rows > 128 else 128
     _call(ct, torch.bfloat16, 1, heads, 1, rows, rows, d, causal, bm=bm)
     rec = _last(ct)[0]
-    assert rec.symbol.endswith(b"_keys") == (takes > 0)
+    assert rec.symbol.endswith((b"_keys", b"_halves")) == (takes > 0)
     assert tuple(rec.grid) == (heads, -(-rows // (takes or bm)), 1)
     if takes:
-        assert rec.symbol.decode() == f"fmha_entry__bf16_{takes}x{256 if takes == 32 else 128}x{d}_keys" and tuple(rec.block) == (512, 1, 1)
+        assert rec.symbol.decode() == f"fmha_entry__bf16_{takes}x{8192 // takes}x{d}_{'halves' if takes == 128 else 'keys'}" and tuple(rec.block) == (512, 1, 1)
         for kw in ({"variant": f"bf16_128x64x{d}"}, {"generics": [128, 64, d]}):      # a kernel or a key tile that the caller names
             _call(ct, torch.bfloat16, 1, heads, 1, rows, rows, d, causal, **kw)
             assert _last(ct)[0].symbol.decode() == f"fmha_entry__bf16_128x64x{d}"
