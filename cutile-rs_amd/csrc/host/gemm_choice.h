@@ -169,19 +169,22 @@ struct GemmChoice {
   F32Plan strip_plan{};
 };
 
-// Register-staged tiles and their prices (choose_gemm), for rows off 16-byte boundaries and on them.  (Tables are constants of this file: a
-// static of an inline function is one object for all builds of the library in a process, whichever is loaded first.)
+// Register-staged tiles and their prices (choose_gemm): us per K tile, alone on a compute unit and for each of several; us of start and output, paid by every round
+// of workgroups; the share by which x rows off 16-byte boundaries lengthen it all; us of shared K, and for each value of the partial sums.  (Tables are
+// constants of this file: a static of an inline function is one object for all builds of the library in a process, whichever is loaded first.)
 struct StagedTile {
   const char* kernel;
   int bm, bn, per_cu;
-  struct Any { double one, more, ends, x, split, sum; } any;
-  struct Aligned { double one, more, ends, split, sum; } aligned;
+  struct Prices { double one, more, ends, x, split, sum; } any, aligned;
 };
+// Rows off 16-byte boundaries, least squares over 140 products, operands from memory, every tile timed (10 to 13 % rms): over them the tile priced lowest takes
+// 1.005 times the best one's time, over 400 more with K up to 700 1.004.  Rows on them, 520 products of 65 to 2500 rows and up to 128 tiles of 128 x 128, with and without a workspace (4 to 6 %
+// rms), 64 x 64 tiles 2 % dearer than fitted, as ring tiles of that price are the better ones, and the larger ones 20 % (805 x 1792 x 3264 22.2 us, ring 18.5).
 constexpr StagedTile kStaged[] = {{"staged256x256", 256, 256, 1, {1.14, 0, 12.7, 0.126, 0, 0}, {}},
-                                  {"staged256x128", 256, 128, 1, {0.77, 0, 8.2, 0.142, 0, 0}, {0.98, 0.98, 6.2, 0, 0}},
-                                  {"staged128x128", 128, 128, 2, {0.50, 0.52, 6.7, 0.139, 0, 0}, {0.715, 0.625, 5.05, 0, 0}},
-                                  {"staged64x128", 64, 128, 3, {0.32, 0.39, 6.0, 0.074, 0, 0}, {0.55, 0.43, 3.9, 0, 0}},
-                                  {"staged64x64", 64, 64, 4, {0.228, 0.2725, 4.5, 0.046, 2.4, 2.1e-6}, {0.32, 0.265, 3.6, 4.1, 4.4e-6}}};
+                                  {"staged256x128", 256, 128, 1, {0.77, 0, 8.2, 0.142, 0, 0}, {}},
+                                  {"staged128x128", 128, 128, 2, {0.50, 0.52, 6.7, 0.139, 0, 0}, {0.56, 0.28, 7.2, 0, 0, 0}},
+                                  {"staged64x128", 64, 128, 3, {0.32, 0.39, 6.0, 0.074, 0, 0}, {0.40, 0.30, 5.9, 0, 0, 0}},
+                                  {"staged64x64", 64, 64, 4, {0.228, 0.2725, 4.5, 0.046, 2.4, 2.1e-6}, {0.165, 0.238, 4.3, 0, 2.7, 1.9e-6}}};
 
 inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_bytes) {
   GemmChoice c;
@@ -241,38 +244,24 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 86 us, 200 x 50021 x 1024 bf16 587 -> 37 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
   if (!s.own_tile || (ring && tiles(128, 128) < (uint64_t)cus / 2)) {
-    // us per K tile: alone on a compute unit, and each of several; us of start and output, paid by every round of workgroups; the share by which x
-    // rows off 16-byte boundaries lengthen it all; us of shared K, and for each value of the partial sums.  Least squares over 140 products whose rows
-    // lie off 16-byte boundaries, operands from memory, every tile timed (10 to 13 % rms): over them the tile priced lowest takes 1.005 times the
-    // best one's time.  256 x 256 has the fewest bytes per product and pays most for start and output (bf16, us on it and on the best
-    // other: 200 x 50021 x 1024 37.3, 46.3; 1000 x 20001 x 1024 67, 62; 961 x 7277 x 2155 57, 44), with a short K in many rounds most of all (5587
-    // x 30444 x 164 240, 181 on 64 x 128: nothing runs beside a start or an output on the tiles that fill a compute unit by themselves).
-    // Rows on 16-byte boundaries cost less (the second set: a K tile alone and each of several, start and output, the splits' share).  They compete
-    // with the ring's prices, and were fitted with them, before a K tile's writes and loads lay between its MFMAs; of staged tiles that takes 10 to 30 % off, so
-    // what is chosen by them is right, and some ring tiles of few outputs would be slower by less than that than the staged ones passed over (100 x 1024
-    // x 4096 14.3 us on the ring, 11.8; 665 x 320 x 704 on these 6.8, on the ring 8.0).  With the first set for them, ring tiles were taken for small
-    // outputs of middling K (us with ring, 64 x 64 and two-stage tiles: 220 x 64 x 1408 14.4, 9.3, 11.5).
-    // (0.265: with the fitted 0.257 the two K / V projections of 1500 x 1024 x 4096, 384 tiles of 64 x 64, took 42 us each, on the ring 40)
+    // 256 x 256 has the fewest bytes per product and pays most for start and output (bf16, us on it and on the best other: 200 x 50021 x 1024 37.3, 46.3;
+    // 1000 x 20001 x 1024 67, 62; 961 x 7277 x 2155 57, 44), with a short K in many rounds most of all (5587 x 30444 x 164 240, 181 on 64 x 128: nothing
+    // runs beside a start or an output on the tiles that fill a compute unit by themselves).  Of aligned rows 64 x 64 tiles that share K are the better ones of few outputs (us there and on the
+    // ring: 1919 x 64 x 3264 10.9, 13.9; 173 x 832 x 3328 11.5, 14.2; 100 x 1024 x 4096 11.8, 14.3), and without a workspace of more (309 x 2240 x 5184 25, 31; 150 x
+    // 3456 x 9536 57, 81): over those 520 products, and over 680 more of sizes that models have, the kernel priced
+    // lowest takes 1.004 of the best one's time (1.02 before, 1.16 without a workspace).
     for (const StagedTile& r : kStaged) {
-      if (s.y_cols < r.bn || (ring && r.bn == 256)) continue;
-      const uint64_t t = tiles(r.bm, r.bn), would_share = staged_splits(r.bm, r.bn, t, s.k, cus), sk = partial_bytes ? would_share : 1;
-      double us;
-      if (ring) {
-        const double w = (double)((t * sk + cus - 1) / cus);
-        if (r.per_cu == 1 && w > 2) continue;
-        const StagedTile::Aligned& a = r.aligned;
-        // (a long K that there is no room to share: priced so that 128 x 128 tiles take it)
-        const double one = sk < would_share ? 0.40 : a.one;
-        us = kt / (double)sk * std::max(one * std::max(1.0, w / r.per_cu), a.more * w) + a.ends + (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      } else {
-        const uint64_t slots = (uint64_t)cus * r.per_cu, rounds = t * sk / slots, rest = t * sk % slots;
-        if (r.per_cu == 1 && rounds >= 2 && kt < 8) continue;
-        const StagedTile::Any& a = r.any;
-        const double ends = a.ends + (r.bn == 256 && s.k % 64 != 0 ? 1.8 : 0.0);   // (there a ragged K tile stands behind the sequence)
-        auto round = [&](uint64_t each) { return kt / (double)sk * std::max(a.one, a.more * (double)each) + ends; };
-        us = ((double)rounds * round(r.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0)) * (s.x_aligned ? 1.0 : 1.0 + a.x) +
-             (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
-      }
+      if (s.y_cols < r.bn || (ring && r.bm == 256)) continue;
+      const uint64_t t = tiles(r.bm, r.bn), sk = partial_bytes ? staged_splits(r.bm, r.bn, t, s.k, cus) : 1;
+      const uint64_t slots = (uint64_t)cus * r.per_cu, rounds = t * sk / slots, rest = t * sk % slots;
+      if (r.per_cu == 1 && rounds >= 2 && kt < 8) continue;
+      const StagedTile::Prices& a = ring ? r.aligned : r.any;
+      const double ends = a.ends + (r.bn == 256 && s.k % 64 != 0 ? 1.8 : 0.0);   // (there a ragged K tile stands behind the sequence)
+      auto round = [&](uint64_t each) { return kt / (double)sk * std::max(a.one, a.more * (double)each) + ends; };
+      double us = ((double)rounds * round(r.per_cu) + (rest ? round((rest + cus - 1) / cus) : 0.0)) * (s.x_aligned ? 1.0 : 1.0 + a.x) +
+                  (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
+      // (a row of tiles of a large y: at 3.5 TB/s, ring tiles have more of it in flight; us here and there 54 x 7680 x 6272 34.3, 29.2; 64 x 4096 x 4096 18.0, 14.8)
+      if (ring && s.m <= 64) us = std::max(us, a.ends + a.split + (double)(s.n * s.k) * 2 / 3.5e6);
       if (us < best * (ring ? 0.98 : 1.0)) best = us, picked = r.kernel, shares_k = sk > 1, c.ring = nullptr;
     }
   }

@@ -152,9 +152,9 @@ def test_more_than_48_rows_of_a_long_k_share_it_on_tiles(fake_hip):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("m,n,k,kernel", [(49, 272, 1800, "staged64x64"), (64, 2248, 7680, "128x128x64_q2x2_lone"), (65, 576, 3976, "staged64x64"),
-                                          (128, 3584, 4096, "128x128x64_q2x2_lone"), (100, 64, 6408, "staged64x64"), (50, 3592, 4104, "128x128x64_q2x2_lone"),
-                                          (127, 1416, 5128, "128x128x64_q2x2_lone")])
+@pytest.mark.parametrize("m,n,k,kernel", [(49, 272, 1800, "staged64x64"), (64, 2248, 7680, "staged64x64"), (65, 576, 3976, "staged64x64"), (100, 64, 6408, "staged64x64"),
+                                          (50, 3592, 4104, "staged64x64"), (127, 1416, 5128, "staged64x64"), (64, 7688, 6280, "128x128x64_q2x2_lone"),
+                                          (50, 7048, 4168, "128x128x64_q2x2_lone"), (128, 3584, 4096, "128x128x64_q2x2_lone"), (127, 2952, 5128, "128x128x64_q2x2_lone")])
 def test_gpu_long_k_shared_on_tiles_of_few_rows(ct, dev, m, n, k, kernel, dtype):
     g = torch.Generator(device="cuda").manual_seed(m + n)
     x = torch.randn(m, k, device=dev, generator=g).to(dtype)
@@ -218,16 +218,29 @@ def test_gpu_captured_product_of_staged_tiles_that_would_share_k(ct, dev, m, n, 
         graph.close()
 
 
-def test_products_of_a_long_k_without_a_workspace_take_larger_tiles(fake_hip):
-    """beyond 128 rows: 64 x 64 staged tiles pay by their split; where there is none, 128 x 128 tiles are the faster ones"""
+def test_products_of_a_long_k_without_a_workspace(fake_hip):
+    """beyond 128 rows, K not shared: 64 x 64 staged tiles while a compute unit has one or two of them (us there and on 128 x 128 ring tiles: 309 x 2240 x 5184
+    24.4, 30.9; 332 x 2048 x 1920 11.8, 14.3; 1008 x 768 x 3968 19.8, 25.7; 184 x 4928 x 4736 29.6, 35.1; 300 x 640 x 4096 19.5, 25.5), ring tiles of more outputs (1500 x
+    1024 x 4096 30.3, 26.2; 1119 x 1792 x 5056 37.3, 32.2)"""
     ct = fake_hip
     from test_gemm_tiles import _new_stream, _workgroups
     buf = torch.empty(30 << 20, dtype=torch.half)
     view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
-    for m, n, k in ((309, 2240, 5184), (332, 2048, 1920), (460, 1792, 2304), (1008, 768, 3968), (156, 3392, 2048), (748, 320, 1728), (184, 4928, 4736), (300, 640, 4096)):
+    for m, n, k, staged in ((309, 2240, 5184, 1), (332, 2048, 1920, 1), (460, 1792, 2304, 1), (1008, 768, 3968, 1), (156, 3392, 2048, 1), (748, 320, 1728, 1), (184, 4928, 4736, 1),
+                            (300, 640, 4096, 1), (1500, 1024, 4096, 0), (1800, 1024, 2048, 0)):
         dev, stream = _new_stream(ct)
         ct.check(ct.lib().cutile_testing_inject_failure(b"hipMallocAsync", 2, 1))
         for _ in range(257):
             ct.gemm(ct.partition(view(m, n), [128, 128]), view(m, k), view(k, n), k, stream=stream.value)
-        assert ct.last_resolved()["symbol"] == "gemm_entry__f16_128x128x64_q2x2_lone" and _workgroups(ct) == -(-m // 128) * -(-n // 128), (m, n, k)
+        tile = 64 if staged else 128
+        assert ct.last_resolved()["symbol"] == "gemm_entry__f16_" + ("staged64x64" if staged else "128x128x64_q2x2_lone"), (m, n, k)
+        assert _workgroups(ct) == -(-m // tile) * -(-n // tile), (m, n, k)
         ct.check(ct.lib().cutile_stream_release(dev, stream))
+
+
+def test_few_outputs_of_aligned_rows_share_k_on_staged_tiles(fake_hip):
+    ct = fake_hip
+    for m, n, k, want in [(1919, 64, 3264, "staged64x64"), (173, 832, 3328, "staged64x64"), (100, 1024, 4096, "staged64x64"), (335, 832, 1920, "staged64x64"),
+                          (54, 7680, 6272, "128x128x64_q2x2"), (64, 4096, 4096, "128x128x64_q2x2"), (64, 2240, 7680, "staged64x64"), (805, 1792, 3264, "128x128x64_q2x2"), (1500, 1024, 4096, "128x128x64_q2x2")]:
+        ct.gemm(ct.partition(torch.empty(m, n, dtype=torch.half), [128, 128]), torch.empty(m, k, dtype=torch.half), torch.empty(k, n, dtype=torch.half), k, accumulate=False)
+        assert ct.last_resolved()["variant"] == "f16_" + want, (m, n, k)
