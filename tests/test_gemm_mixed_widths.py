@@ -37,3 +37,15 @@ def test_launch_of_two_widths(fake_hip):
     for m, n, k, mix, groups in ((1500, 14336, 4096, True, 8 * (32 + 32)), (1344, 12032, 4608, True, 7 * (36 + 15)), (1536, 16384, 3072, False, 512), (1536, 8192, 4096, False, 256)):
         ct.gemm(ct.partition(view(m, n), [256, 256]), view(m, k), view(k, n), k, variant="f16_192x256x64_q2x4")
         assert ct.last_resolved()["symbol"].endswith("_mix") == mix and _workgroups(ct) == groups, (m, n, k)
+
+
+def test_which_sizes_take_two_widths(fake_hip):
+    """nobody names a kernel: f16 and bf16, partitions of 256 x 256 and of 128 x 128; two rounds of one width and outputs of one round keep that"""
+    ct = fake_hip
+    bufs = {dt: torch.empty(118 << 20, dtype=dt) for dt in (torch.half, torch.bfloat16)}
+    for m, n, k, mix in ((1344, 12032, 4608, True), (900, 18432, 5120, True), (560, 28672, 4096, True), (2048, 8960, 3584, True), (1536, 16384, 3072, False), (1536, 8192, 4096, False)):
+        for dt, buf in bufs.items():
+            view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+            for tile in (256, 128):
+                ct.gemm(ct.partition(view(m, n), [tile, tile]), view(m, k), view(k, n), k, accumulate=False)
+                assert ct.last_resolved()["symbol"].endswith("_192x256x64_q2x4" + ("_mix" if mix else "")), (m, n, k, dt, tile, ct.last_resolved()["symbol"])

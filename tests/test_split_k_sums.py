@@ -5,10 +5,13 @@ import torch
 from util import rel_l2
 
 
+SHAPES = [(1, 64, 9216, 9), (15, 67, 9300, 9), (16, 64, 16384, 16), (17, 130, 10240, 10), (33, 64, 16389, 16), (48, 65, 9216, 9)]   # workgroups to a strip, f16 and bf16
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("m,n,k,splits", [(1, 64, 9216, 9), (15, 67, 9300, 9), (16, 64, 16384, 16), (17, 130, 10240, 10), (33, 64, 16389, 16), (48, 65, 9216, 9)])
-def test_gpu_sums_of_more_than_eight_splits(ct, dev, m, n, k, splits, dtype):
+@pytest.mark.parametrize("m,n,k", [s[:3] for s in SHAPES])
+def test_gpu_sums_of_more_than_eight_splits(ct, dev, m, n, k, dtype):
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     x = torch.randn(m, k, device=dev, generator=g).to(dtype)
     y = (torch.randn(k, n, device=dev, generator=g) / k ** 0.5).to(dtype)
@@ -28,11 +31,14 @@ def test_gpu_sums_of_more_than_eight_splits(ct, dev, m, n, k, splits, dtype):
         first = z
 
 
-def test_as_many_splits_as_the_test_above_means(fake_hip):
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_as_many_splits_as_the_test_above_means(fake_hip, dtype):
+    """f32 strips share K by powers of two: sixteen of them in each of the six"""
     ct = fake_hip
     from test_gemm_tiles import _workgroups
-    buf = torch.empty(1 << 21, dtype=torch.half)
-    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
-    for m, n, k, splits in ((1, 64, 9216, 9), (16, 64, 16384, 16), (33, 64, 16389, 16)):
-        ct.gemm(ct.partition(view(m, n), [64, 64]), view(m, k), view(k, n), k, generics=["f16", 64, 64, 1])
-        assert "thin" in ct.last_resolved()["variant"] and _workgroups(ct) == splits, (m, n, k, _workgroups(ct))
+    for m, n, k, splits in SHAPES:
+        ct.gemm(ct.partition(torch.empty(m, n, dtype=dtype), [64, 64]), torch.empty(m, k, dtype=dtype), torch.empty(k, n, dtype=dtype), k)
+        variant = ct.last_resolved()["variant"]
+        rows, cols = map(int, variant.split("strip" if dtype == torch.float32 else "thin")[1].split("x"))
+        strips = -(-m // rows) * -(-n // cols)
+        assert _workgroups(ct) == strips * (16 if dtype == torch.float32 else splits), (m, n, k, variant, _workgroups(ct))
