@@ -375,7 +375,7 @@ std::vector<KernelEntry> build_table() {
     add("fmha_seq", keep(v), keep("fmha_seq_entry__" + v), IMG_FMHA, (uint32_t)(t[0] / 32 * 64),
         (uint32_t)(2 * 2 * t[1] * t[2] * 2), t[0], t[1], t[2], 0, "f16", 0, 3);
   }
-  // wavefronts that share the keys of 32 or 64 query rows: for the launcher's own rule alone, whatever rows the caller's partition has
+  // wavefronts that share the keys of 32 or 64 query rows, or (D = 64) of 128, two to each 32 of them: for the launcher's own rule alone, whatever rows the caller's partition has
   for (const char* function : {"fmha", "fmha_seq"})
     for (const char* dt : {"bf16", "f16"})
       for (int d : {64, 128})

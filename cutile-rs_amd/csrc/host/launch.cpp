@@ -2022,7 +2022,8 @@ cutile_status_t cutile_scratch_capacity(size_t* bytes) {
   return CUTILE_SUCCESS;
 }
 
-// The splits of a launch that its own workgroups merge (fmha.hip, merge_if_last): a lane to a split, a counter to a head, 16-byte stores of out;
+// The splits of a launch that its own workgroups merge (fmha.hip, merge_if_last): a lane to a split, a counter to a head, rows of out on 16-byte
+// boundaries as the other kernels of this path have them (the stores, two values each, would do with 4);
 // and counters behind the partial results, which a scratch library built before there were any does not have.
 // In launches that the compute units hold at once: one and a half workgroups to each, or one where LDS has no room for two.  Beyond, what a merge
 // saves is lost to workgroups that wait for their partial results to pass the L2 and count (two launches and one, us: GROUP 1, D = 64, 64 heads

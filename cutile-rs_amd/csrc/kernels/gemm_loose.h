@@ -10,6 +10,20 @@
 namespace cutile {
 namespace gemm {
 
+// ---- a K tile of 64 of register-staged tiles in LDS ------------------------------------------------------------------------------
+// Byte offsets of 16-byte unit u of row r of the x tile (eight units a row) and of the y tile (UB), and a load from any 2-byte boundary.
+template <int BN>
+struct StagedLayout {
+  static constexpr int BK = 64, UB = BN / 8;
+  __device__ static __forceinline__ int a_lds_off(int r, int u) { return r * (BK * 2) + ((u ^ ((r >> 1) & 7)) << 4); }
+  __device__ static __forceinline__ int b_lds_off(int r, int u) { return r * (BN * 2) + ((u ^ ((((r & 3) << 2) | (((r >> 3) & 1) << 1)) & (UB - 1))) << 4); }
+  __device__ static __forceinline__ u32x4 load16(const unsigned char* p) {
+    u32x4 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
+    return v;
+  }
+};
+
 // ---- an output tile on any 2-byte boundaries -----------------------------------------------------------------------------
 // `width` values from column c of the tile's row r; the columns before col_first are another tile's (the last tile of a row is moved back into z).
 template <typename OutT>
@@ -72,18 +86,9 @@ __device__ __forceinline__ void output_passes(const f32x4 (&acc)[TN][TM], unsign
 // asks for another in its place.  One barrier per K tile, behind three of its four blocks of 16 MFMAs.  For
 // outputs of 129 to 256 such tiles, two rounds of 256 x 128, and for a long K in many rounds: bf16 200 x 50021 x 1024 46.3 -> 37.3 us.
 template <typename OutT, typename InT>
-struct GemmStagedWide {
-  static constexpr int BM = 256, BN = 256, BK = 64, kThreads = 512, WM = 128, WN = 64, TM = 8, TN = 4, TMH = 4, UB = BN / 8;
+struct GemmStagedWide : StagedLayout<256> {
+  static constexpr int BM = 256, BN = 256, kThreads = 512, WM = 128, WN = 64, TM = 8, TN = 4, TMH = 4;
   static constexpr int kABytes = BM * BK * 2, kStageBytes = kABytes + BK * BN * 2, kPieces = 8, kQueue = 12;
-
-  __device__ static __forceinline__ int a_lds_off(int r, int u) { return r * (BK * 2) + ((u ^ ((r >> 1) & 7)) << 4); }
-  __device__ static __forceinline__ int b_swizzle(int r) { return ((r & 3) << 2) | (((r >> 3) & 1) << 1); }
-  __device__ static __forceinline__ int b_lds_off(int r, int u) { return r * (BN * 2) + ((u ^ b_swizzle(r)) << 4); }
-  __device__ static __forceinline__ u32x4 load16(const unsigned char* p) {   // any 2-byte boundary
-    u32x4 v;
-    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
-    return v;
-  }
 
   __device__ static void run(const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y, int32_t k_total, int32_t cover_m, int32_t cover_n,
                              int32_t accumulate, uint32_t tiles_m, uint32_t tiles_n) {

@@ -27,23 +27,15 @@ namespace {
 // 2155 54.1 -> 44.0, 3136 x 1941 x 5340 99.6 -> 85.6.  With both operands unaligned a 128-byte piece of a row of x lies in two cache lines, which
 // the vector cache does not hold until the next K tile: 2749 x 2583 x 8862 stays at 184.  Several workgroups may share the K tiles of a 64 x 64 output tile (SPLIT).
 template <int BM, int BN, int WAVES_M, int WAVES_N, typename OutT, typename InT>
-struct GemmStaged {
+struct GemmStaged : StagedLayout<BN> {
+  using Layout = StagedLayout<BN>;
+  using Layout::a_lds_off, Layout::b_lds_off, Layout::load16;
   static constexpr bool SPLIT = BM == 64 && BN == 64;   // the tile that the launcher splits (staged_splits)
-  static constexpr int BK = 64, kWaves = WAVES_M * WAVES_N, kThreads = kWaves * 64;
+  static constexpr int BK = Layout::BK, UB = Layout::UB, kWaves = WAVES_M * WAVES_N, kThreads = kWaves * 64;
   static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 16, TN = WN / 16;
-  static constexpr int UB = BN / 8;                                    // 16-byte units of a y-tile row
   static constexpr int kALoads = BM * 8 / kThreads, kBLoads = BK * UB / kThreads;
   static constexpr int kABytes = BM * BK * 2, kBBytes = BK * BN * 2, kStageBytes = kABytes + kBBytes;
   static_assert(kALoads * kThreads == BM * 8 && kBLoads * kThreads == BK * UB && UB >= 8, "tile must split evenly");
-
-  __device__ static __forceinline__ int a_lds_off(int r, int u) { return r * (BK * 2) + ((u ^ ((r >> 1) & 7)) << 4); }
-  __device__ static __forceinline__ int b_swizzle(int r) { return (((r & 3) << 2) | (((r >> 3) & 1) << 1)) & (UB - 1); }
-  __device__ static __forceinline__ int b_lds_off(int r, int u) { return r * (BN * 2) + ((u ^ b_swizzle(r)) << 4); }
-  __device__ static __forceinline__ u32x4 load16(const unsigned char* p) {   // any 2-byte boundary
-    u32x4 v;
-    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
-    return v;
-  }
 
   __device__ static void run(const PartitionArg<2>& z, const TensorArg<2>& x, const TensorArg<2>& y, int32_t k_total, int32_t cover_m,
                              int32_t cover_n, int32_t accumulate, float* partials, uint32_t* counters, uint32_t tiles_m, uint32_t tiles_n,

@@ -582,7 +582,7 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
                                                       int32_t bn);
 /* Warm-up for the entry point above; like it, without a counterpart in the reference.  The first call of the entry
  * point on a device opens the side library that holds the array, looks the array's address up (the runtime places the
- * 8 MiB then) and loads two code objects: work that is neither allocation-free nor legal while a stream is being
+ * 8 MiB then) and loads the code object of the kernels: work that is neither allocation-free nor legal while a stream is being
  * captured.  This call does all of it and enqueues nothing (the entry point in compile-only mode: the arguments are
  * checked exactly as a launch checks them, no pointer is dereferenced).  Call it once per device and shape outside any
  * capture; after it, cutile_launch_fmha_decode_gqa_noalloc with the same shapes only enqueues one kernel or two. */
