@@ -203,9 +203,9 @@ struct GemmStages {
 
 // Tiles of two widths in one launch: `wide` columns of BM x 256 tiles, then columns of BM x 192, in the stages of the former.  Outputs of one and a half to two
 // rounds of workgroups leave compute units idle in the second; with the widths mixed every compute unit has about as much to do.  f16, us on
-// one width and on two: 1344 x 12032 x 4608 161, 152; 900 x 18432 x 5120 179, 172; 560 x 28672 x 4096 148, 141; 1700 x 11000 x 2048 79.6, 76.8.  Where the
-// chip is at its power limit in the first round already, idle units had given it clock: 1500 x 14336 x 4096 161.7, 160.9, and in a block over a prompt of 1500
-// nothing.
+// one width and on two: 1344 x 12032 x 4608 161, 152; 900 x 18432 x 5120 179, 172; 560 x 28672 x 4096 148, 141; 1700 x 11000 x 2048 79.6, 76.8.  Least
+// where idle units had given the others clock (1.93 GHz with two widths, below the chip's 2.4): 1500 x 14336 x 4096 161.7, 160.9, in a block over a prompt of
+// 1500 167.3, 163.7.  400 drawn products of one to two rounds take 0.995 of the time before, at most 1.035 (within what the card varies).
 #define GEMM_RING_MIX_KERNEL(NAME, BM, T)                                                                                           \
   extern "C" __global__ void __launch_bounds__(512)                                                                                 \
       gemm_entry__##NAME(PartitionArg<2> z, TensorArg<2> x, TensorArg<2> y, int32_t k, TileGrid g, int32_t accumulate,               \
