@@ -243,7 +243,9 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
     }
   // Staged tiles: the only ones for unaligned rows (6198 x 3583 x 1194 f16 1150 -> 86 us, 200 x 50021 x 1024 bf16 587 -> 37 us), and,
   // split along K, the better ones for outputs of less than about 64 tiles of 128 x 128.
-  if (!s.own_tile || (ring && tiles(128, 128) < (uint64_t)cus / 2)) {
+  // (of more tiles, aligned and of a partition without kernels of its own, ring tiles are the better ones for any K: 105 products of 128 tiles and more, with staged
+  // ones 1.01 to 1.17 times the best one's time by their K, 2966 x 9808 x 2832 224 us, ring 154)
+  if (ring ? tiles(128, 128) < (uint64_t)cus / 2 : !s.own_tile) {
     // 256 x 256 has the fewest bytes per product and pays most for start and output (bf16, us on it and on the best other: 200 x 50021 x 1024 37.3, 46.3;
     // 1000 x 20001 x 1024 67, 62; 961 x 7277 x 2155 57, 44), with a short K in many rounds most of all (5587 x 30444 x 164 240, 181 on 64 x 128: nothing
     // runs beside a start or an output on the tiles that fill a compute unit by themselves).  Of aligned rows 64 x 64 tiles that share K are the better ones of few outputs (us there and on the

@@ -244,3 +244,14 @@ def test_few_outputs_of_aligned_rows_share_k_on_staged_tiles(fake_hip):
                           (54, 7680, 6272, "128x128x64_q2x2"), (64, 4096, 4096, "128x128x64_q2x2"), (64, 2240, 7680, "staged64x64"), (805, 1792, 3264, "128x128x64_q2x2"), (1500, 1024, 4096, "128x128x64_q2x2")]:
         ct.gemm(ct.partition(torch.empty(m, n, dtype=torch.half), [128, 128]), torch.empty(m, k, dtype=torch.half), torch.empty(k, n, dtype=torch.half), k, accumulate=False)
         assert ct.last_resolved()["variant"] == "f16_" + want, (m, n, k)
+
+
+def test_aligned_partitions_without_kernels_of_their_own(fake_hip):
+    """96 x 96: staged tiles while there are less than 128 tiles of 128 x 128, ring tiles beyond, whatever K"""
+    ct = fake_hip
+    buf = torch.empty(30 << 20, dtype=torch.half)
+    view = lambda rows, cols: buf[:rows * cols].view(rows, cols)
+    for m, n, k, staged in [(335, 832, 1920, True), (700, 640, 136, True), (2966, 9808, 2832, False), (1773, 4064, 608, False), (5390, 1072, 1296, False), (681, 10696, 2368, False),
+                            (1556, 9448, 640, False), (1556, 9448, 136, False)]:
+        ct.gemm(ct.partition(view(m, n), [96, 96]), view(m, k), view(k, n), k, accumulate=False, generics=["f16", 96, 96, 1])
+        assert ("staged" in ct.last_resolved()["variant"]) == staged, (m, n, k, ct.last_resolved()["variant"])
