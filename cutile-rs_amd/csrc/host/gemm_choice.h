@@ -334,8 +334,11 @@ constexpr FlatStrip kFlat[] = {{"flat16x64", 16, 64, 0.09, 0.20, 0.20, 0.20, 5.5
 inline const char* choose_scaled(const ScaledShape& s, int own_m, int own_n, int cus, uint64_t partial_bytes, MxPlan* lone) {
   // a partition whose output other tiles of nvfp4_gemm.hip may compute too
   const bool tiled = s.fp4 && own_m == own_n && (own_m == 128 || (own_m == 256 && s.pieces > 4));
-  if (s.pieces <= 4 && !tiled) return nullptr;   // two steps: nothing to share out
   auto blocks = [&](int bm, int bn) { return (uint64_t)((s.m + bm - 1) / bm) * (uint64_t)((s.n + bn - 1) / bn); };
+  // fp4 of up to 128 values: too short for strips; start and output of a 256 x 256 tile are most of it (us there and on 128 x 128: 256 x 128
+  // 9.2, 5.5; 988 x 5056 14.8, 9.7; 381 x 15296 15.0, 10.4; of more than a round of the small ones 1504 x 10432 16.3, 18.4)
+  if (s.fp4 && s.pieces <= 1) return own_m == 256 && own_n == 256 && blocks(128, 128) <= 2 * (uint64_t)cus ? "128x128x64_w2x2" : nullptr;
+  if (s.pieces <= 4 && !tiled) return nullptr;   // two steps: nothing to share out
   if (!tiled && s.m > 64 && own_m == 256 && own_n == 256 && blocks(256, 256) * 4 >= (uint64_t)cus * 3) return nullptr;
   // (fp8 on 128 x 128: the direct pipeline below is always the cheaper one; only a name reaches flat128x128 there)
   const char* name = nullptr;

@@ -399,7 +399,7 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
   });
   *cus = 256;
   std::string sized;
-  if (flat) {
+  if (flat || (shape.fp4 && full_cover && shape.pieces <= 1)) {
     if (cutile_status_t s = current_device_units(cus)) return s;
     const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes, &room->lone);
     if (kernel && strcmp(kernel, "128x128x128_e2x2") == 0 && room->lone.splits > 1 && g_launch_mode != 2) {

@@ -218,10 +218,11 @@ struct Nvfp4Gemm {
     };
     constexpr std::true_type kMore{};
     constexpr std::false_type kLast{};
-    if constexpr (BM == 128 && BN == 128) {
+    if constexpr (BM * BN < 256 * 256) {
       // Of an even number the last tile expands nothing behind itself, and an odd one has no partner of zeros: at K = 128, two tiles, that was half
       // of the expansions.  us: 988 x 5056 x 128 10.3 -> 9.7, 495 x 11392 x 256 12.7 -> 11.7, 988 x 5056 x 512 16.6 -> 15.3, x 4096 73 -> 69.  (The 256 x
-      // 256 kernels have no registers for another copy of the tile's code.)
+      // 256 kernels have no registers for another copy of the tile's code, nor for a branch around the expansion, 115 -> 168 us at 4096 x 4096 x 4096; they
+      // lose 0.3 us by it, 9 x 3840 x 256 8.4 -> 8.7; up to K = 128 the launcher gives theirs to these while one round has them.)
       int32_t kt = 0;
 #pragma unroll 1
       for (;; kt += 2) {
