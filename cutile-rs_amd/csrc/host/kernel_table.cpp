@@ -384,7 +384,10 @@ std::vector<KernelEntry> build_table() {
           const std::string v = std::string(dt) + "_" + std::to_string(rows) + "x" + std::to_string(8192 / rows) + "x" + std::to_string(d);
           const char* const member = rows == 128 ? "halves" : "keys";
           add(function, keep(v + "+" + member), keep(std::string(function) + "_entry__" + v + "_" + member), IMG_FMHA_KEYS, 512,
-              (uint32_t)(512 * d * 2 + 2 * 8 * 32 * 4), rows, 8192 / rows, d, 0, dt, 0, 3);
+              (uint32_t)(512 * d * 2 + 2 * 8 * 32 * 4 + (rows == 64 && d == 128 ? 64 * 128 * 2 : 0)), rows, 8192 / rows, d, 0, dt, 0, 3);
+          if (rows == 64 && d == 128)   // up to 256 keys
+            add(function, keep(v + "+few"), keep(std::string(function) + "_entry__" + dt + "_few_64x128x128_keys"), IMG_FMHA_KEYS, 512, (uint32_t)(512 * d * 2 + 2 * 8 * 32 * 4), 64, 128, d,
+                0, dt, 0, 3);
         }
 
   // ---- decode attention: one workgroup per (KV head, split); tile = (GROUP, 0, D) ----

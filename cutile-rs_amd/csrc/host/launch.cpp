@@ -2780,16 +2780,14 @@ namespace {
 // wavefronts share the keys, or 0 for the kernels of 32 rows to a wavefront.
 // On 32 rows a workgroup has read its keys soonest, as long as one round holds the launch; behind that 64 rows, which read them half as
 // often.  D = 128 leaves room for one workgroup on a compute unit, D = 64 for two.  us on the kernels of 128 and 256 rows, on 64 and on 32:
-//   D = 128, causal: 4 heads of 2048 42, 30 and 26; 8 of 2048 (256 workgroups of 64 rows) 43, 31 and 34; 32 of 1024 (512) 26.2, 26.8 and 44
+//   D = 128, causal: 4 heads of 2048 42, 23 and 21; 8 of 2048 (256 workgroups of 64 rows) 43, 25 and 27; 32 of 1024 (512) 26, 27 and 38
 //   D = 64: 8 heads of 1024 (256 workgroups of 32 rows) 21, 13 and 10.5; 16 of 1024 21, 13 and 15; 32 of 1024 (512 of 64 rows) 22, 18.5 and 27;
 //     512 of short keys lose: 128 heads of 256 8.9, 10 and 19; 1024 of 64 rows pay where causal tiles even out: 32 heads of 2048 causal 52, 41
 //     and 73, not causal 55, 60 and 110
-//   Two rounds of 64 rows at D = 128 pay where causal tiles are long (8 heads of 4096 80.8 and 66.5; 32 of 1024 25.6 and 27.0) and of
-//     different lengths: keys in front of the rows (`start`) make them alike, and then the 256-row kernel, which reads K and V a quarter as often, is
-//     the better one, the sooner the more workgroups there are (f16; 8 heads of 2408 behind 664 63 and 51, behind 2408 93 and 90, behind 4816 141 and 153; 4
-//     of 8192 behind 1024 170 and 160, behind 4096 225 and 235; 32 of 1024 behind 3000 84 and 111, 40 of 512 behind 7000 143 and 215).  Over 130
-//     launches on this side of the line 0.68 to 1.00 of its time.  (With the position on the device the other kernel is the one of 128 rows: 0.68 to 0.95 of its
-//     time wherever the rows begin, 32 heads of 1024 at 0 33 and 28, behind 3000 113 and 101.)
+//   Two rounds of 64 rows at D = 128 pay where causal tiles are long and of different lengths: keys in front of the rows (`start`) make them alike, and then the
+//     256-row kernel, which reads K and V a quarter as often, is the better one, the sooner the more workgroups there are (f16; 4 heads of 4320 82 and 41, 8 of 3811 74
+//     and 50, 6 of 5408 106 and 68; 16 of 2855 behind 6467 205 and 238).  Shorter ones, which also gain (8 heads of 2066 45 and 26, 16 of 1839 44 and 33; not 64 of 427, 16 and
+//     22), are left where they are.  (With the position on the device the other kernel is the one of 128 rows.)
 // Every other launch of D = 64 has two wavefronts to 32 rows of the 128-row workgroup (us on one wavefront and on two: 32 heads of 4096 196 and 180, causal 109
 // and 102; 128 of 1024 57 and 54, 43 and 38), but where one wavefront has its keys as soon: while two workgroups to a compute unit are one round up to 448
 // keys without a mask (160 of 221 11.6 and 12.7, 128 of 354 14.6 and 15.4) and 256 under it (144 of 246 10.8 and 10.9), and under the mask up to 1000 with a
@@ -2807,17 +2805,71 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t s
   if (d != 64 || keys < (causal ? (once ? 257 : 200) : once ? 448 : 300)) return 0;
   return causal && rows > 256 && keys < 1000 && !once && 2 * of128 <= 5 * cus ? 0 : 128;
 }
+// The kernel of those rows, and the keys of its query tiles dealt to several workgroups where a round of them leaves compute units idle: `steps` key steps
+// to each.  What a step costs grows with the share of the compute units at work; bringing the results together costs a part for each and one for
+// all (fitted to 204, 271, 298 and 36 launches of one round: the pick takes 1.01 of the best one's time).  One round only: behind it nothing was left to gain.
+// us, keys not dealt out and dealt: D = 128, 32 rows: 8 heads of 17 rows behind 3905 keys 27 and 12.9, 12 of 28 behind 5078 33 and 15.2, 16 of 200 behind 4000
+// 28.7 and 22.3; D = 64, 4 heads of 40 behind 4000 14.5 and 9.4.
+struct KeyPlan {
+  int rows = 0;
+  int32_t steps = 1 << 28;   // more than there can be
+  uint32_t shares = 1;
+};
+KeyPlan key_plan(int d, int64_t heads, int64_t rows, int64_t keys, int64_t start, bool causal, int cus, bool may_share) {
+  KeyPlan plan;
+  plan.rows = key_sharing_rows(d, heads, rows, keys, start, causal, cus);
+  if ((plan.rows != 32 && plan.rows != 64) || keys <= 256) return plan;
+  struct Costs {
+    int step;
+    double begin, each, load, share, all;
+  };
+  auto best = [&](int of, double* price) {
+    static constexpr Costs kCosts[2][2] = {{{256, 5.3, 0.64, 0.54, 0.15, 1.1}, {128, 5.3, 0.98, 0.04, 0.12, 2.2}},       // D = 64: 32 rows, 64
+                                           {{256, 7.6, 1.18, 0.43, 0.27, 1.7}, {256, 8.7, 1.62, 0.37, 0.67, 2.0}}};      // D = 128
+    const Costs& c = kCosts[d == 128][of == 64];
+    const int64_t tiles = heads * ((rows + of - 1) / of), steps = (keys + c.step - 1) / c.step;
+    const int64_t room = std::min<int64_t>(cus / tiles, (int64_t)(kSplitPartialBytes / (size_t)(of * (d + 2) * 4)) / tiles);
+    KeyPlan r;
+    r.rows = of;
+    *price = c.begin + c.each * (double)steps * (1 + c.load * (double)tiles / cus);
+    if (may_share && tiles <= (int64_t)kSplitCounters)
+      for (int64_t want = 2; want <= std::min<int64_t>({room, steps, 32}); ++want) {
+        const int64_t each = (steps + want - 1) / want, shares = (steps + each - 1) / each;
+        const double p = c.begin + c.each * (double)each * (1 + c.load * (double)(tiles * shares) / cus) + c.all + c.share * (double)shares;
+        if (p < *price) *price = p, r.steps = (int32_t)each, r.shares = (uint32_t)shares;
+      }
+    return r;
+  };
+  double price, other;
+  KeyPlan mine = best(plan.rows, &price);
+  if (plan.rows == 32 && d == 128) {   // (64 rows read K and V half as often; the prices are good to some per cent)
+    const KeyPlan wider = best(64, &other);
+    if (other < 0.92 * price) mine = wider;
+  }
+  return mine;
+}
+void push_key_shares(ArgPacker& args, const KeyPlan& k, const SplitWorkspace& ws) {
+  args.push_val<void*>(ws.partials);
+  args.push_val<void*>(ws.counters);
+  args.push_val<int32_t>(k.steps);
+  args.push_val<int32_t>(0);
+}
 // (by their own rows, not by the family whose place they take)
-const KernelEntry* keys_member(const char* function, bool bf16, int rows, int d) {
+const KernelEntry* keys_member(const char* function, bool bf16, int rows, int d, int64_t keys) {
   static const auto& members = *[] {
-    auto* m = new std::array<const KernelEntry*, 24>();
-    for (size_t i = 0; i < m->size(); ++i) {
+    auto* m = new std::array<const KernelEntry*, 28>();
+    for (size_t i = 0; i < 24; ++i) {
       const char* const rows[] = {"32x256x", "64x128x", "128x64x"};
       (*m)[i] = find_entry(i / 12 ? "fmha_seq" : "fmha", std::string(i / 6 % 2 ? "bf16_" : "f16_") + rows[i / 2 % 3] + (i & 1 ? "128" : "64") + (i / 2 % 3 == 2 ? "+halves" : "+keys"));
     }
+    for (size_t i = 0; i < 4; ++i) (*m)[24 + i] = find_entry(i / 2 ? "fmha_seq" : "fmha", i & 1 ? "bf16_64x128x128+few" : "f16_64x128x128+few");
     return m;
   }();
-  return members[(strcmp(function, "fmha_seq") == 0) * 12 + bf16 * 6 + (rows / 64) * 2 + (d == 128)];
+  const bool seq = strcmp(function, "fmha_seq") == 0;
+  // Up to 256 keys, one step of wavefronts with keys of their own, the end of it counts: eight partial outputs to add up, where two wavefronts to each 32 keys leave four
+  // (D = 128, 80 heads of 132 8.9 and 10.0 us, 64 of 171 9.6 and 10.2, 48 of 249 10.3 and 10.7; of 294 11.0 and 9.1)
+  if (rows == 64 && d == 128 && keys <= 256) return members[24 + seq * 2 + bf16];
+  return members[seq * 12 + bf16 * 6 + (rows / 64) * 2 + (d == 128)];
 }
 }  // namespace
 
@@ -2876,16 +2928,22 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   Resolved res;
   BucketScope bucket(dt + "_bm" + std::to_string(bm) + "_d" + std::to_string(d) + (causal ? "|causal" : "|full"));
   const std::string fallback = same_bn.empty() ? acceptable[0] : same_bn[0];
-  int key_rows = 0;   // (a caller that names the key tile means the kernel of that tile)
+  KeyPlan plan;   // (a caller that names the key tile means the kernel of that tile)
+  int cus = 256;
+  const int64_t seen = causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2];
+  auto plan_keys = [&](bool may_share) { plan = key_plan(d, tg[0], ot.shape[1], seen, input_pos, causal, cus, may_share); };
   if (bm >= 128 && bn_user == 0 && (int64_t)tg[1] * bm >= ot.shape[1]) {
-    int cus = 256;
     if (cutile_status_t s = current_device_units(&cus)) return s;
-    key_rows = key_sharing_rows(d, tg[0], ot.shape[1], causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2], input_pos, causal, cus);
+    plan_keys(true);
   }
-  if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, key_rows ? fallback : std::string())) return s;
-  if (key_rows && g_last_source == "size") {
-    if (cutile_status_t s = use_member(&res, keys_member("fmha", q->dtype == CUTILE_DTYPE_BF16, key_rows, d))) return s;
-    tg[1] = div_up(ot.shape[1], key_rows);
+  if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, plan.rows ? fallback : std::string())) return s;
+  const bool by_keys = plan.rows && g_last_source == "size";
+  SplitWorkspace ws;
+  if (by_keys) {
+    if (plan.shares > 1 && g_launch_mode == 0) ws = split_workspace(res.device, (hipStream_t)stream);
+    if (!ws.partials) plan_keys(false);
+    if (cutile_status_t s = use_member(&res, keys_member("fmha", q->dtype == CUTILE_DTYPE_BF16, plan.rows, d, seen))) return s;
+    tg[1] = div_up(ot.shape[1], plan.rows);
   }
   ArgPacker args;
   args.push_partition(*out);
@@ -2897,7 +2955,8 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   args.push_val<int32_t>(query_group_size);
   args.push_val<int32_t>(causal ? 1 : 0);
   args.push_tile_grid(tg);
-  uint32_t grid[3] = {tg[0], tg[1], 1};
+  if (by_keys) push_key_shares(args, plan, ws);
+  uint32_t grid[3] = {tg[0], tg[1], by_keys ? plan.shares : 1};
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 
@@ -2993,16 +3052,22 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   o.generics = nullptr;
   o.n_generics = 0;
   Resolved res;
-  int key_rows = 0;   // (a caller that names the key tile, or packs the heads of a group into its tiles, means the kernels of that form)
+  KeyPlan plan;   // (a caller that names the key tile, or packs the heads of a group into its tiles, means the kernels of that form)
+  int cus = 256;
+  const int64_t there = position_start ? max_seq : kv_len, seen = causal && !position_start ? std::min<int64_t>((int64_t)query_start + rows_cov, there) : there;
+  auto plan_keys = [&](bool may_share) { plan = key_plan(d, heads_cov, rows_cov, seen, position_start ? 0 : query_start, causal, cus, may_share); };
   if (pack == 1 && generic_int(opts, 1, 0) == 0 && (!position_start || rows_cov > 128)) {   // (with the position on the device, rows are all that is known of the length: 128 of them see more keys than that)
-    const int64_t seen = position_start ? max_seq : kv_len;
-    int cus = 256;
     if (cutile_status_t s = current_device_units(&cus)) return s;
-    key_rows = key_sharing_rows(d, heads_cov, rows_cov, causal && !position_start ? std::min<int64_t>((int64_t)query_start + rows_cov, seen) : seen, position_start ? 0 : query_start, causal, cus);
+    plan_keys(true);
   }
-  if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, key_rows ? acceptable[0] : std::string())) return s;
-  if (key_rows && g_last_source == "size")
-    if (cutile_status_t s = use_member(&res, keys_member(function, false, key_rows, d))) return s;
+  if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, plan.rows ? acceptable[0] : std::string())) return s;
+  const bool by_keys = plan.rows && g_last_source == "size";
+  SplitWorkspace ws;
+  if (by_keys) {
+    if (plan.shares > 1 && g_launch_mode == 0) ws = split_workspace(res.device, (hipStream_t)stream);
+    if (!ws.partials) plan_keys(false);
+    if (cutile_status_t s = use_member(&res, keys_member(function, false, plan.rows, d, seen))) return s;
+  }
   const int32_t kbm = res.entry->tile[0];
   ov.partition_shape[0] = 1; ov.partition_shape[1] = kbm; ov.partition_shape[2] = d;
   for (int i = 0; i < 3; ++i) ov.partition_strides[i] = ov.tensor.strides[i];
@@ -3022,7 +3087,8 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   args.push_val<int32_t>(query_group_size);
   args.push_val<int32_t>(causal ? 1 : 0);
   args.push_tile_grid(kg);
-  uint32_t grid[3] = {kg[0], kg[1], 1};
+  if (by_keys) push_key_shares(args, plan, ws);
+  uint32_t grid[3] = {kg[0], kg[1], by_keys ? plan.shares : 1};
   return launch_packed(res.fn, grid, res.entry->block, 0, stream, args);
 }
 
