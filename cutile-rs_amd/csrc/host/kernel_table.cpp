@@ -335,7 +335,9 @@ std::vector<KernelEntry> build_table() {
         (uint32_t)(((t[0] == 256 ? 2 : 3) * t[0] * 64 + 2 * 64 * t[1]) * 2), t[0], t[1], 64, 0, "f16", 0, 2);
   }
   add("group_gemm_nt_desc", "f16_128x128x64_d2x2+ahead", "group_gemm_nt_desc_entry__f16_128x128x64_d2x2_ahead", IMG_GEMM_GROUP, 512,
-      4 * (128 * 64 + 64 * 128) * 2 + 256 * 64 + 48, 128, 128, 64, 0, "f16", 0, 2);
+      4 * (128 * 64 + 64 * 128) * 2 + 256 * 64 + 64, 128, 128, 64, 0, "f16", 0, 2);
+  add("group_gemm_nt_desc", "f16_256x256x64_q2x4+ahead", "group_gemm_nt_desc_entry__f16_256x256x64_q2x4_ahead", IMG_GEMM_GROUP, 512, (3 * 256 * 64 + 2 * 64 * 256) * 2, 256,
+      256, 64, 0, "f16", 0, 2);
   for (const char* dt : {"bf16", "f16", "f32"})
     add("gemm_persistent", keep(std::string(dt) + "_generic"), keep(std::string("gemm_persistent_entry__") + dt + "_generic"),
         IMG_GEMM, 256, (uint32_t)((64 * 17 + 16 * 65) * 4), 0, 0, 0, 0, dt, 0, 2);

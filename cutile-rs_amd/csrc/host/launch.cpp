@@ -2653,7 +2653,7 @@ cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, con
   Resolved res;
   if (cutile_status_t s = resolve_entry("group_gemm_nt_desc", &o, acceptable[0], acceptable, &res)) return s;
   bool ahead = false;
-  if (bm == 128 && bn == 128 && num_groups <= kMostGroupsAhead && g_last_source == "table") {   // (no caller or pin names the ring)
+  if (bm == bn && (bm == 128 || bm == 256) && num_groups <= kMostGroupsAhead && g_last_source == "table") {   // (no caller or pin names the ring)
     int cus = 256;
     if (g_launch_mode != 2)
       if (cutile_status_t s = compute_units(res.device, &cus)) return s;
