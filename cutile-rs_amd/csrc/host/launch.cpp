@@ -1665,14 +1665,16 @@ static cutile_status_t launch_qk_norm_rope_kv(const char* name, cutile_stream_t 
   args.push_val<int32_t>(max_seq);
   args.push_val<int64_t>(q_row_stride);
   args.push_val<int64_t>(kv_row_stride);
-  uint32_t grid[3] = {std::min<uint32_t>((uint32_t)seq_len, 1u << 20), 1, 1};   // one workgroup per position
-  // lanes per workgroup: rows * D/16 lane slots per position; the size that idles the fewest lanes in the last pass
-  const uint32_t lane_slots = (uint32_t)(num_q_heads + 2 * num_kv_heads) * (uint32_t)(d / 16);
-  uint32_t block[3] = {256, 1, 1}, best_idle = UINT32_MAX;
-  for (uint32_t b : {256u, 192u, 128u, 64u}) {
-    const uint32_t idle = (lane_slots + b - 1) / b * b - lane_slots;
-    if (idle < best_idle) best_idle = idle, block[0] = b;
-  }
+  uint32_t grid[3] = {std::min<uint32_t>((uint32_t)seq_len, 1u << 20), 1, 1};
+  // Lanes per workgroup: as few passes over the rows * D/16 lane slots of a position as 256 lanes take, on the smallest workgroup that takes no more.  A pass is a
+  // trip to memory, 0.4 to 0.6 us one after another: below 1024 positions each has a workgroup of its own (a position's table is then computed more than
+  // once).  D = 128, us with the size that idles the fewest lanes, before, and here: one position of 28 + 28 heads (64 lanes, 11 passes) 9.2 and 3.0, of 32 + 8 3.6 and 2.9;
+  // 222 of 36 + 9 8.7 and 4.2, 1500 of 24 + 6 11.0 and 8.4 (one workgroup each; two 8.4 as well, 2048 of 32 + 8 11.6 and 12.1).
+  const uint32_t lane_slots = (uint32_t)(num_q_heads + 2 * num_kv_heads) * (uint32_t)(d / 16), passes = div_up(lane_slots, 256);
+  uint32_t block[3] = {256, 1, 1};
+  for (uint32_t b : {192u, 128u, 64u})
+    if (div_up(lane_slots, b) == passes) block[0] = b;
+  if (seq_len < 1024) grid[1] = std::min(passes, 65535u);
   return launch_packed(res.fn, grid, block, 0, stream, args);
 }
 

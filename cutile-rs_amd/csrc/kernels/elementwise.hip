@@ -1017,9 +1017,9 @@ extern "C" __global__ void __launch_bounds__(kThreads)
 // q, q_out: rows of num_q_heads * D every q_row_stride elements; k, v: num_kv_heads * D every kv_row_stride;
 // the caches are [num_kv_heads, max_seq, D].  The decode form is the same work for one position whose q, k
 // and v rows sit back to back and whose position is read from device memory.
-// One workgroup per position: the D/2 (cos, sin) pairs are computed once into LDS; a lane holds 8 rotation
+// One workgroup per position, or one to each pass over its rows (blockIdx.y): the D/2 (cos, sin) pairs are computed once into LDS; a lane holds 8 rotation
 // pairs of one row (two 16-byte accesses), D/16 neighbouring lanes hold a row and sum its squares.  The workgroup
-// size (64 .. 256 lanes) is the launcher's: the one that leaves the fewest lanes idle in the last pass over the rows.
+// size (64 .. 256 lanes) and the number of workgroups to a position are the launcher's.
 namespace {
 struct FusedRowsArgs {
   const _Float16 *q, *k, *v, *q_weight, *k_weight;
@@ -1121,7 +1121,7 @@ extern "C" __global__ void __launch_bounds__(kThreads)
     for (int32_t i = threadIdx.x; i < a.half; i += threads) sincosf((float)pos_i * inv_freq[i], &sn_tab[i], &cs_tab[i]);
     __syncthreads();
     // (requesting rows before the table is computed costs registers, hence residency: measured 4.9 - 5.3 against 5.4 TB/s)
-    for (int32_t t = (int32_t)threadIdx.x; t < slots; t += threads) {
+    for (int32_t t = (int32_t)(blockIdx.y * threads + threadIdx.x); t < slots; t += threads * (int32_t)gridDim.y) {
       const int32_t r = t >> a.chunk_shift, c = t & (a.chunks - 1);
       u32x4 lo = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
       if (r < a.rows) {
