@@ -16,6 +16,7 @@ struct GemmShape {
   bool aligned;            // rows on 16-byte boundaries, whole output covered: the ring kernels can take it
   bool x_aligned;          // the rows of x are
   bool own_tile;           // the partition's tile has kernels of its own
+  bool whole_k;            // K in whole tiles of 64 that both operands have, columns of z in units of 8: 192 x 384 tiles can take it
 };
 
 // Output tiles of bm x bn of a launch.
@@ -35,6 +36,9 @@ constexpr RingTile kRingTiles[] = {{"256x256x64_q2x4", 256, 256, 1.03, 1.36, 8.0
 // A K tile on 192 x 192 (the stages of 192 x 256), by its share of a wide tile's products: 7 x 36 wide and 7 x 15 narrow tiles of K = 4608 144 us
 // priced, 152 measured; 5 x 51 and 5 x 27 of 5120 161, 172; one width 156 and 172 priced, 161 and 179 measured.
 constexpr double kNarrowFew = 0.66, kNarrowAll = 0.86, kNarrowEnds = 6.2;
+// A K tile on 192 x 384 (gemm_wide.h): least squares over 150 products of 100 to 880 such tiles, K 576 to 14336 (4.3 % rms).  Of the 150 it is picked in 12, 0.78 to
+// 0.89 of the other kernels' time; in none where it is slower, and three that it would do in 0.95 to 0.96 stay with the others.
+constexpr double kWideFew = 1.13, kWideAll = 1.69, kWideEnds = 8.6;
 // Workgroups that share a tile: each stores its partial tile, and the last one reads them all.  us a value of one output tile, and of all of them.
 constexpr double kShareEach = 4.2e-5, kShareAll = 1.0e-6, kShareOnce = 0.7;
 // The one that a kernel of that tile is, by the tile shape and by the marker of these kernels in its name.
@@ -49,9 +53,11 @@ struct RingPlan {
   bool two;          // 128 x 128: two workgroups to a compute unit, on the ring (K unshared)
   double us;
   uint32_t wide = 0, narrow = 0;   // columns of tiles, where those of 192 columns stand beside the ones of 256
+  bool by_384 = false;             // 192 x 384 tiles
 };
 // What the launch costs with the best number of workgroups to an output tile; as priced and as launched.  `partial_bytes` = room for partial tiles, 0: K is not shared.
-inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, int cus, uint64_t partial_bytes) {
+// `wide_tiles`: 192 x 256 may be 192 x 384.
+inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, int cus, uint64_t partial_bytes, bool wide_tiles = false) {
   const uint64_t t = tiles_of(m, n, r.bm, r.bn);
   const int64_t kt = (k + 63) / 64;
   RingPlan best{1, false, 1e30};
@@ -70,6 +76,12 @@ inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, in
       const double us = (double)kt * (r.all + kNarrowFew + (kNarrowAll - kNarrowFew) * rest) + r.ends + kNarrowEnds;
       if (us < best.us * 0.98) best = {1, false, us, (uint32_t)wide, (uint32_t)narrow};
     }
+  }
+  if (wide_tiles && r.bm == 192 && r.bn == 256) {
+    const uint64_t g = tiles_of(m, n, 192, 384), rest = g % cus;
+    const double us = (double)kt * ((double)(g / cus) * kWideAll + (rest ? kWideFew + (kWideAll - kWideFew) * (double)rest / cus : 0.0)) +
+                      kWideEnds * (double)((g + cus - 1) / cus);
+    if (us < best.us * 0.98) best = {1, false, us, 0, 0, true};
   }
   if (r.bm == 128 && r.bn == 128) {
     // two workgroups to a compute unit, each at half its pace as soon as there are more than compute units (1623 x 2944 x
@@ -236,7 +248,7 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
       // a handful of tiles of a short K: 64 x 64 staged ones, priced below (us there and on 128 x 128: 263 x 64 x 1728 9.4, 10.8; 141 x
       // 320 x 2496 11.3, 12.3; beyond, 250 x 384 x 4352 16.3, 14.4)
       if (s.k <= 2560 && tiles_of(s.m, s.n, 128, 128) < 16) break;
-      const RingPlan p = cutile::ring_plan(r, s.m, s.n, s.k, cus, partial_bytes);
+      const RingPlan p = cutile::ring_plan(r, s.m, s.n, s.k, cus, partial_bytes, s.whole_k);
       // (128 x 256 against 256 x 128, f16: 619 x 8832 x 4096 56.7 us, 59.0; 620 x 5000 x 4096 40.8, 39.6; 600 x 8192 x 4096 54.1, 55.8; equal for
       // bf16: the prices are good to 5 %, so only where it is the cheaper one by more)
       if (p.us < best * (r.bm < r.bn && r.bm == 128 ? 0.94 : 0.98)) best = p.us, picked = r.kernel, shares_k = p.splits > 1, c.ring = &r, c.ring_plan = p;

@@ -258,6 +258,10 @@ std::vector<KernelEntry> build_table() {
       std::replace(sym.begin(), sym.end(), '+', '_');
       add("gemm", keep(v), keep(sym), strchr(t.name, '+') ? IMG_GEMM_TILES : IMG_GEMM_SMALL, 512, (uint32_t)((t.stages_m * t.bm + t.stages_n * t.bn) * 64 * 2), t.bm, t.bn, 64, 0, dt, 0, 2);
     }
+  // 192 x 384 (gemm_wide.h), which launches of mixed widths take where it is one round: two stages, the x ones as large as 256 rows
+  for (const char* dt : {"bf16", "f16"})
+    add("gemm", keep(std::string(dt) + "_192x256x64_q2x4+wide"), keep(std::string("gemm_entry__") + dt + "_wide_192x256x64_q2x4_mix"), IMG_GEMM_TILES, 512,
+        (uint32_t)(2 * (256 + 384) * 64 * 2), 192, 256, 64, 0, dt, 0, 2);
   // medium sizes: register-staged tiles, K split over workgroups (any alignment, any partition shape); two LDS stages
   for (const char* dt : {"bf16", "f16", "bf16f32"})
     for (auto t : {std::array<int, 3>{64, 64, 4}, std::array<int, 3>{64, 128, 4}, std::array<int, 3>{128, 128, 4}, std::array<int, 3>{256, 128, 8}, std::array<int, 3>{256, 256, 8}}) {
