@@ -16,7 +16,7 @@ struct GemmShape {
   bool aligned;            // rows on 16-byte boundaries, whole output covered: the ring kernels can take it
   bool x_aligned;          // the rows of x are
   bool own_tile;           // the partition's tile has kernels of its own
-  bool whole_k;            // K in whole tiles of 64 that both operands have, columns of z in units of 8: 192 x 384 tiles can take it
+  bool whole_k;            // K in whole tiles of 64 that both operands have, columns of z in units of 8: the wider tiles can take it
 };
 
 // Output tiles of bm x bn of a launch.
@@ -36,9 +36,14 @@ constexpr RingTile kRingTiles[] = {{"256x256x64_q2x4", 256, 256, 1.03, 1.36, 8.0
 // A K tile on 192 x 192 (the stages of 192 x 256), by its share of a wide tile's products: 7 x 36 wide and 7 x 15 narrow tiles of K = 4608 144 us
 // priced, 152 measured; 5 x 51 and 5 x 27 of 5120 161, 172; one width 156 and 172 priced, 161 and 179 measured.
 constexpr double kNarrowFew = 0.66, kNarrowAll = 0.86, kNarrowEnds = 6.2;
-// A K tile on 192 x 384 (gemm_wide.h): least squares over 150 products of 100 to 880 such tiles, K 576 to 14336 (4.3 % rms).  Of the 150 it is picked in 12, 0.78 to
-// 0.89 of the other kernels' time; in none where it is slower, and three that it would do in 0.95 to 0.96 stay with the others.
-constexpr double kWideFew = 1.13, kWideAll = 1.69, kWideEnds = 8.6;
+// Wider tiles (gemm_wide.h), priced as above: least squares over 420 products of 200 to 1100 tiles of 192 x 256, K 576 to 14336 (3 to 4 % rms), by 1.08, which is what the
+// times of the tiles above were over their prices in those products (median).  Of the 420 they are picked in 138, 0.80 to 1.02 of the other tiles' time, 0.91 in the mean.
+struct WideTile {
+  const char* member;
+  int bm, bn;
+  double few, all, ends;
+};
+constexpr WideTile kWideTiles[] = {{"+w192x320", 192, 320, 0.94, 1.51, 7.1}, {"+w192x384", 192, 384, 1.02, 1.65, 8.5}, {"+w192x448", 192, 448, 1.14, 1.90, 9.3}, {"+w256x320", 256, 320, 1.09, 1.84, 9.4}};
 // Workgroups that share a tile: each stores its partial tile, and the last one reads them all.  us a value of one output tile, and of all of them.
 constexpr double kShareEach = 4.2e-5, kShareAll = 1.0e-6, kShareOnce = 0.7;
 // The one that a kernel of that tile is, by the tile shape and by the marker of these kernels in its name.
@@ -53,10 +58,10 @@ struct RingPlan {
   bool two;          // 128 x 128: two workgroups to a compute unit, on the ring (K unshared)
   double us;
   uint32_t wide = 0, narrow = 0;   // columns of tiles, where those of 192 columns stand beside the ones of 256
-  bool by_384 = false;             // 192 x 384 tiles
+  const WideTile* by = nullptr;    // these tiles instead
 };
 // What the launch costs with the best number of workgroups to an output tile; as priced and as launched.  `partial_bytes` = room for partial tiles, 0: K is not shared.
-// `wide_tiles`: 192 x 256 may be 192 x 384.
+// `wide_tiles`: a launch by the name of 192 x 256 may be on wider ones.
 inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, int cus, uint64_t partial_bytes, bool wide_tiles = false) {
   const uint64_t t = tiles_of(m, n, r.bm, r.bn);
   const int64_t kt = (k + 63) / 64;
@@ -77,12 +82,12 @@ inline RingPlan ring_plan(const RingTile& r, int64_t m, int64_t n, int32_t k, in
       if (us < best.us * 0.98) best = {1, false, us, (uint32_t)wide, (uint32_t)narrow};
     }
   }
-  if (wide_tiles && r.bm == 192 && r.bn == 256) {
-    const uint64_t g = tiles_of(m, n, 192, 384), rest = g % cus;
-    const double us = (double)kt * ((double)(g / cus) * kWideAll + (rest ? kWideFew + (kWideAll - kWideFew) * (double)rest / cus : 0.0)) +
-                      kWideEnds * (double)((g + cus - 1) / cus);
-    if (us < best.us * 0.98) best = {1, false, us, 0, 0, true};
-  }
+  if (wide_tiles && r.bm == 192 && r.bn == 256)
+    for (const WideTile& w : kWideTiles) {
+      const uint64_t g = tiles_of(m, n, w.bm, w.bn), rest = g % cus;
+      const double us = (double)kt * ((double)(g / cus) * w.all + (rest ? w.few + (w.all - w.few) * (double)rest / cus : 0.0)) + w.ends * (double)((g + cus - 1) / cus);
+      if (us < best.us * 0.98) best = {1, false, us, 0, 0, &w};
+    }
   if (r.bm == 128 && r.bn == 128) {
     // two workgroups to a compute unit, each at half its pace as soon as there are more than compute units (1623 x 2944 x
     // 14016 f16, 299 tiles: 214 us, 192 x 128 tiles 151; 619 x 8832 x 7552 bf16, 345 tiles: 137, 256 x 128 tiles 90)

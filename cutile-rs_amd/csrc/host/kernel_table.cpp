@@ -258,10 +258,13 @@ std::vector<KernelEntry> build_table() {
       std::replace(sym.begin(), sym.end(), '+', '_');
       add("gemm", keep(v), keep(sym), strchr(t.name, '+') ? IMG_GEMM_TILES : IMG_GEMM_SMALL, 512, (uint32_t)((t.stages_m * t.bm + t.stages_n * t.bn) * 64 * 2), t.bm, t.bn, 64, 0, dt, 0, 2);
     }
-  // 192 x 384 (gemm_wide.h), which launches of mixed widths take where it is one round: two stages, the x ones as large as 256 rows
+  // wider tiles (gemm_wide.h), members of the family whose launches may be of mixed widths: two stages
   for (const char* dt : {"bf16", "f16"})
-    add("gemm", keep(std::string(dt) + "_192x256x64_q2x4+wide"), keep(std::string("gemm_entry__") + dt + "_wide_192x256x64_q2x4_mix"), IMG_GEMM_TILES, 512,
-        (uint32_t)(2 * (256 + 384) * 64 * 2), 192, 256, 64, 0, dt, 0, 2);
+    for (auto t : {std::array<int, 2>{192, 320}, std::array<int, 2>{192, 384}, std::array<int, 2>{192, 448}, std::array<int, 2>{256, 320}}) {
+      const std::string tile = "w" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
+      add("gemm", keep(std::string(dt) + "_192x256x64_q2x4+" + tile), keep(std::string("gemm_entry__") + dt + "_" + tile + "_192x256x64_q2x4_mix"), IMG_GEMM_TILES, 512,
+          (uint32_t)(2 * (t[0] + t[1]) * 64 * 2), 192, 256, 64, 0, dt, 0, 2);
+    }
   // medium sizes: register-staged tiles, K split over workgroups (any alignment, any partition shape); two LDS stages
   for (const char* dt : {"bf16", "f16", "bf16f32"})
     for (auto t : {std::array<int, 3>{64, 64, 4}, std::array<int, 3>{64, 128, 4}, std::array<int, 3>{128, 128, 4}, std::array<int, 3>{256, 128, 8}, std::array<int, 3>{256, 256, 8}}) {

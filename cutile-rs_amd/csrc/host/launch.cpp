@@ -2286,15 +2286,15 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   uint32_t splits = 1, narrow = 0;
   if (const RingTile* ring = row_layout && fast_layout && full_cover ? ring_tile(res.entry->variant, res.entry->tile[0], res.entry->tile[1]) : nullptr) {
     // (a kernel that the caller or a record names has that kernel's tiles)
-    RingPlan plan = ring == sized.ring && !(sized.ring_plan.by_384 && g_last_source != "size") ? sized.ring_plan : ring_plan(*ring, cover_m, cover_n, k_valid, cus, partial_bytes);
+    RingPlan plan = ring == sized.ring && !(sized.ring_plan.by && g_last_source != "size") ? sized.ring_plan : ring_plan(*ring, cover_m, cover_n, k_valid, cus, partial_bytes);
     if (plan.splits > 1 && !ws.partials && g_launch_mode == 0) {   // a kernel that the caller or a record names
       ws = split_workspace(res.device, (hipStream_t)stream);
       if (!ws.partials) plan = ring_plan(*ring, cover_m, cover_n, k_valid, cus, 0);
     }
     splits = plan.splits;
     if (plan.narrow) tg[1] = plan.wide, narrow = plan.narrow;
-    if (plan.by_384) tg[1] = div_up(cover_n, 384);
-    const char* member = plan.by_384 ? "+wide" : plan.narrow ? "+mix" : ring->bm == 256 && ring->bn == 256 && splits > 1 ? "+split" : ring->bm == 128 && ring->bn == 128 && !plan.two ? "+lone" : nullptr;
+    if (plan.by) tg[0] = div_up(cover_m, plan.by->bm), tg[1] = div_up(cover_n, plan.by->bn);
+    const char* member = plan.by ? plan.by->member : plan.narrow ? "+mix" : ring->bm == 256 && ring->bn == 256 && splits > 1 ? "+split" : ring->bm == 128 && ring->bn == 128 && !plan.two ? "+lone" : nullptr;
     if (member)
       if (cutile_status_t s = use_member(&res, member_of(res.entry, member))) return s;
   }
