@@ -255,7 +255,7 @@ def tensor_arg(t, dtype: Optional[int] = None) -> TensorArg:
     return a
 
 
-@dataclass
+@dataclass(slots=True)
 class Partition:
     """``tensor.partition(shape)`` of the reference (cutile/src/tensor.rs:1417-1429): a
     mutable tensor divided into disjoint tiles; its grid defines the launch grid."""
@@ -284,7 +284,12 @@ class Partition:
 
 
 def partition(tensor, shape: Sequence[int], prefix: bool = False, dtype: Optional[int] = None) -> Partition:
-    return Partition(tensor, list(shape), prefix, dtype)
+    p = _new_partition(Partition)
+    p.tensor, p.shape, p.prefix, p.dtype = tensor, list(shape), prefix, dtype
+    return p
+
+
+_new_partition = Partition.__new__       # (a launch makes one or more; the class's own call takes 0.1 us longer)
 
 
 OWNED = 0     # map-shape sentinel of an owned (not streamed) axis, cutile/src/tensor.rs:331-337
@@ -362,48 +367,58 @@ def _stream(stream) -> int:
     return _raw_stream(torch._C._cuda_getDevice())
 
 
-_launchers: dict = {}    # entry launchers of the loaded library behind the marshalling extension
+def _stream_source():
+    """what a launch without a stream asks each time: (ordinal of torch's device, handle of its current stream there), or None without a GPU"""
+    import torch
+
+    _stream(None)
+    return None if _raw_stream is None else (torch._C._cuda_getDevice, _raw_stream)
 
 
-def _launcher(name: str):
-    if not _launchers:
-        import importlib.util
-
-        path = os.path.join(_HERE, "lib", "cutile_marshal.so")
-        if not os.path.exists(path):
-            raise ImportError(f"{path} is missing: run `python cutile-rs_amd/build.py` (or __graft_entry__.build()) first")
-        import torch  # noqa: F401  (the extension reads its tensors)
-
-        spec = importlib.util.spec_from_file_location("cutile_marshal", path)
-        marshal = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(marshal)
-        _launchers.update({n: marshal.launcher(n, C.cast(getattr(lib(), "cutile_launch_" + n), C.c_void_p).value, tensor_arg, Partition)
-                           for n in marshal.names()})
-    return _launchers[name]
+_marshal = None          # the marshalling extension, once something was launched
 
 
-def _launch(name: str, *args) -> None:
-    """cutile_launch_<name>: tensors, (tensor, element type), partitions, numbers and (grid, generics, variant) in the order of
-    the C signature"""
-    status = (_launchers.get(name) or _launcher(name))(*args)
-    if status:
-        check(status)
+class _Launchers:
+    """Attribute ``name`` calls ``cutile_launch_<name>``: the stream or None for torch's current one, then tensors, (tensor, element type), partitions,
+    numbers and (grid, generics, variant) in the order of the C signature.  Raises what ``check`` raises."""
+
+    def __getattr__(self, name: str):
+        global _marshal
+        if _marshal is None:
+            import importlib.util
+
+            path = os.path.join(_HERE, "lib", "cutile_marshal.so")
+            if not os.path.exists(path):
+                raise ImportError(f"{path} is missing: run `python cutile-rs_amd/build.py` (or __graft_entry__.build()) first")
+            import torch  # noqa: F401  (the extension reads its tensors)
+
+            spec = importlib.util.spec_from_file_location("cutile_marshal", path)
+            _marshal = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(_marshal)
+        if name not in _marshal.names():
+            raise AttributeError(name)
+        launcher = _marshal.launcher(name, C.cast(getattr(lib(), "cutile_launch_" + name), C.c_void_p).value, tensor_arg, Partition, _stream_source, check)
+        setattr(self, name, launcher)
+        return launcher
+
+
+_c = _Launchers()
 
 
 # ---- entry launchers (reference argument order) ---------------------------------------------
 def saxpy(y: Partition, a: float, x, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """y <- a*x + y.  cutile-examples/examples/saxpy.rs:12-17."""
-    _launch("saxpy", _stream(stream), y, float(a), x, (grid, generics, variant))
+    _c.saxpy(stream, y, float(a), x, (grid, generics, variant))
 
 
 def axpy(z: Partition, a: float, x, y, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """z <- a*x + y (rank 1)."""
-    _launch("axpy", _stream(stream), z, float(a), x, y, (grid, generics, variant))
+    _c.axpy(stream, z, float(a), x, y, (grid, generics, variant))
 
 
 def add(z: Partition, x, y, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """z <- x + y.  README.md:29-38 of the reference."""
-    _launch("add", _stream(stream), z, x, y, (grid, generics, variant))
+    _c.add(stream, z, x, y, (grid, generics, variant))
 
 
 def full(value, t: Partition, *, stream=None, grid=None, variant=None) -> None:
@@ -424,28 +439,28 @@ def eye(t: Partition, *, stream=None, grid=None, generics=None) -> None:
 
 def relu(input_output: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-examples/examples/async_mlp.rs:56-61: max(0, x) in place over [D] tiles of an f32 vector"""
-    _launch("relu", _stream(stream), input_output, (grid, generics, None))
+    _c.relu(stream, input_output, (grid, generics, None))
 
 
 def dropout(p: float, x, x_keep, out: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-examples/examples/dropout.rs:17-32: out = select(x_keep > p, x_keep, 0) / (1 - p); x is never read"""
-    _launch("dropout", _stream(stream), float(p), x, x_keep, out, (grid, generics, None))
+    _c.dropout(stream, float(p), x, x_keep, out, (grid, generics, None))
 
 
 def scale_ptr(out_ptr: int, in_ptr: int, scale: float, length: int, *, stream=None, grid=None) -> None:
     """cutile-examples/examples/scale_ptr.rs:26-80: out[i] = in[i] * scale for i < length on raw device pointers (f32);
     the launch grid is required, as for every launcher without a partition argument"""
-    _launch("scale_ptr", _stream(stream), int(out_ptr), int(in_ptr), float(scale), int(length), (grid, None, None))
+    _c.scale_ptr(stream, int(out_ptr), int(in_ptr), float(scale), int(length), (grid, None, None))
 
 
 def matvec(z: Partition, x, y, k: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-examples/examples/async_mlp.rs:38-54: z[r] += sum_k x[r, k] * y[k] over [BM] tiles of z (f32)"""
-    _launch("matvec", _stream(stream), z, x, y, int(k), (grid, generics, None))
+    _c.matvec(stream, z, x, y, int(k), (grid, generics, None))
 
 
 def batch_matmul(c: Partition, a, b, k: int, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-examples/examples/batch_matmul.rs:16-44: c[p] = a[p] . b[p] over [1, BM, BN] tiles of c"""
-    _launch("batch_matmul", _stream(stream), c, a, b, int(k), (grid, generics, variant))
+    _c.batch_matmul(stream, c, a, b, int(k), (grid, generics, variant))
 
 
 def linspace(t: Partition, start: float, step: float, *, stream=None, grid=None) -> None:
@@ -454,53 +469,53 @@ def linspace(t: Partition, start: float, step: float, *, stream=None, grid=None)
 
 
 def convert(src, dst: Partition, *, stream=None, grid=None) -> None:
-    _launch("convert", _stream(stream), src, dst, (grid, None, None))
+    _c.convert(stream, src, dst, (grid, None, None))
 
 
 def rms_norm_f16(x, w, out: Partition, eps: float, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-kernels/src/norms.rs:16-60."""
-    _launch("rms_norm_f16", _stream(stream), x, w, out, float(eps), (grid, generics, variant))
+    _c.rms_norm_f16(stream, x, w, out, float(eps), (grid, generics, variant))
 
 
 def rms_norm_f32(x, w, out: Partition, eps: float, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """the f32 example form, cutile-examples/examples/rms_norm.rs:17-61 (square root rounded toward minus infinity)"""
-    _launch("rms_norm_f32", _stream(stream), x, w, out, float(eps), (grid, generics, variant))
+    _c.rms_norm_f32(stream, x, w, out, float(eps), (grid, generics, variant))
 
 
 def rms_norm_all_f16(x, w, out: Partition, eps: float, *, generics, stream=None, grid=None) -> None:
     """cutile-benchmarks/benches/rmsnorm.rs:20-66: every operation in f16; generics = [N, BLOCK_SIZE]."""
-    _launch("rms_norm_all_f16", _stream(stream), x, w, out, float(eps), (grid, generics, None))
+    _c.rms_norm_all_f16(stream, x, w, out, float(eps), (grid, generics, None))
 
 
 def softmax_all_f16(x, y: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-benchmarks/benches/softmax.rs:19-35 with its own arithmetic: every operation in f16."""
-    _launch("softmax_all_f16", _stream(stream), x, y, (grid, generics, None))
+    _c.softmax_all_f16(stream, x, y, (grid, generics, None))
 
 
 def softmax(x, y: Partition, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-benchmarks/benches/softmax.rs:19-35."""
-    _launch("softmax", _stream(stream), x, y, (grid, generics, variant))
+    _c.softmax(stream, x, y, (grid, generics, variant))
 
 
 def add_rms_norm_f16(residual, x, w, out: Partition, residual_out: Partition, eps: float, *, stream=None, grid=None,
                      generics=None, variant=None) -> None:
     """combined = residual + x; out = RMSNorm(combined) * w; residual_out = combined (cutile-kernels norms.rs:68-136)"""
-    _launch("add_rms_norm_f16", _stream(stream), residual, x, w, out, residual_out, float(eps), (grid, generics, variant))
+    _c.add_rms_norm_f16(stream, residual, x, w, out, residual_out, float(eps), (grid, generics, variant))
 
 
 def qk_norm_f16(q, k, q_weight, k_weight, out: Partition, eps: float, num_q_rows: int, *, stream=None, grid=None,
                 generics=None, variant=None) -> None:
     """rows < num_q_rows of out: RMSNorm(q) * q_weight; the rest: RMSNorm(k) * k_weight (norms.rs:143-216)"""
-    _launch("qk_norm_f16", _stream(stream), q, k, q_weight, k_weight, out, float(eps), int(num_q_rows), (grid, generics, variant))
+    _c.qk_norm_f16(stream, q, k, q_weight, k_weight, out, float(eps), int(num_q_rows), (grid, generics, variant))
 
 
 def add_2d_f16(out: Partition, lhs, rhs, *, stream=None, grid=None, generics=None, variant=None) -> None:
-    _launch("add_2d_f16", _stream(stream), out, lhs, rhs, (grid, generics, variant))
+    _c.add_2d_f16(stream, out, lhs, rhs, (grid, generics, variant))
 
 
 def silu_mul_2d_f16(out: Partition, gate, up, *, stream=None, grid=None, generics=None, variant=None) -> None:
     """out = sigmoid(gate) * gate * up (pointwise.rs:46-78)"""
-    _launch("silu_mul_2d_f16", _stream(stream), out, gate, up, (grid, generics, variant))
+    _c.silu_mul_2d_f16(stream, out, gate, up, (grid, generics, variant))
 
 
 def rope_f16(out: Partition, x, inv_freq, position_start=0, *, k=None, num_q_heads: int = 0, stream=None, grid=None,
@@ -508,7 +523,7 @@ def rope_f16(out: Partition, x, inv_freq, position_start=0, *, k=None, num_q_hea
     """Rotary embedding (positional.rs).  `position_start` is an int (rope_seq_f16) or a one-element
     uint32/int32 device tensor (the dynpos forms); with `k`, heads >= num_q_heads of out come from k."""
     by_value = isinstance(position_start, int)
-    _launch("rope_f16", _stream(stream), x, k, inv_freq, None if by_value else (position_start, U32), position_start if by_value else 0, out,
+    _c.rope_f16(stream, x, k, inv_freq, None if by_value else (position_start, U32), position_start if by_value else 0, out,
             int(num_q_heads), (grid, generics, None))
 
 
@@ -516,14 +531,14 @@ def kv_cache_update_f16(new_k, new_v, k_cache: Partition, v_cache: Partition, po
                         grid=None, generics=None) -> None:
     """cache[h, position_start + s] = new[s, h] (kv_cache.rs); position_start: int or one-element device tensor"""
     by_value = isinstance(position_start, int)
-    _launch("kv_cache_update_f16", _stream(stream), new_k, new_v, k_cache, v_cache, None if by_value else (position_start, U32),
+    _c.kv_cache_update_f16(stream, new_k, new_v, k_cache, v_cache, None if by_value else (position_start, U32),
             position_start if by_value else 0, int(seq_len), (grid, generics, None))
 
 
 def fmha_decode_gqa_split(q, k, v, att_out: Partition, lse_out: Partition, qk_scale: float, position_start, *, stream=None,
                           grid=None, generics=None, variant=None) -> None:
     """split-KV decode attention (attention.rs:737-902); position_start: one-element device tensor"""
-    _launch("fmha_decode_gqa_split", _stream(stream), q, k, v, att_out, lse_out, float(qk_scale), (position_start, U32), (grid, generics, variant))
+    _c.fmha_decode_gqa_split(stream, q, k, v, att_out, lse_out, float(qk_scale), (position_start, U32), (grid, generics, variant))
 
 
 def attention_decode_kernel_grouped_f16(q, k, v, att, lse, softmax_scale: float, s_kv, *, tile_n: int = 64,
@@ -536,19 +551,19 @@ def attention_decode_kernel_grouped_f16(q, k, v, att, lse, softmax_scale: float,
             raise ValueError(f"attention_decode_kernel_grouped: expected rank {rank} with unit innermost stride")
         return t.data_ptr(), tuple(t.shape), t.stride()[:-1]
     qgts = int(query_group_tile_size) if query_group_tile_size is not None else max(int(q.shape[2]), 1)
-    _launch("attention_decode_kernel_grouped_f16", _stream(stream), *group(q, 4), *group(k, 4), *group(v, 4), *group(att, 5), *group(lse, 4),
+    _c.attention_decode_kernel_grouped_f16(stream, *group(q, 4), *group(k, 4), *group(v, 4), *group(att, 5), *group(lse, 4),
             float(softmax_scale), s_kv.data_ptr(), int(tile_n), int(kv_len_per_split), qgts, (grid, generics, None))
 
 
 def splitk_reduce_merge(att_partial, lse_partial, out: Partition, *, stream=None, grid=None, generics=None) -> None:
-    _launch("splitk_reduce_merge", _stream(stream), att_partial, lse_partial, out, (grid, generics, None))
+    _c.splitk_reduce_merge(stream, att_partial, lse_partial, out, (grid, generics, None))
 
 
 def fmha_decode_gqa_noalloc(q, k, v, out: Partition, qk_scale: float, position_start, num_kv_splits: int, bn: int = 64, *,
                             stream=None) -> None:
     """split-KV decode attention and merge in one call that allocates nothing: the partial results live in the
     library's device-resident scratch array (8 MiB per GPU); position_start: one-element device tensor"""
-    _launch("fmha_decode_gqa_noalloc", _stream(stream), q, k, v, out, float(qk_scale), (position_start, U32), int(num_kv_splits), int(bn))
+    _c.fmha_decode_gqa_noalloc(stream, q, k, v, out, float(qk_scale), (position_start, U32), int(num_kv_splits), int(bn))
 
 
 def fmha_decode_gqa_noalloc_prepare(q, k, v, out: Partition, position_start, num_kv_splits: int, bn: int = 64) -> None:
@@ -568,7 +583,7 @@ def scratch_capacity() -> int:
 def gemm(z: Partition, x, y, k: int, *, accumulate: bool = True, stream=None, grid=None, generics=None,
          variant=None) -> None:
     """cutile-benchmarks/benches/gemm.rs:20-41 (z is read as the initial accumulator)."""
-    _launch("gemm", _stream(stream), z, x, y, int(k), int(accumulate), (grid, generics, variant))
+    _c.gemm(stream, z, x, y, int(k), int(accumulate), (grid, generics, variant))
 
 
 def gemm_persistent(z: MappedPartition, x, y, *, stream=None, grid=None, generics=None, variant=None) -> None:
@@ -629,7 +644,7 @@ def mapped_tile_index(z: MappedPartition, *, stream=None, grid=None) -> None:
 def fmha(out: Partition, q, k, v, qk_scale: float, input_pos: int = 0, query_group_size: int = 1, *,
          causal: bool = False, stream=None, grid=None, generics=None, variant=None) -> None:
     """cutile-examples/examples/flash_attention_causal.rs:19-134."""
-    _launch("fmha", _stream(stream), out, q, k, v, float(qk_scale), int(input_pos), int(query_group_size), int(causal), (grid, generics, variant))
+    _c.fmha(stream, out, q, k, v, float(qk_scale), int(input_pos), int(query_group_size), int(causal), (grid, generics, variant))
 
 
 KVBM_STACKED_NHD, KVBM_STACKED_HND = 0, 1
@@ -649,7 +664,7 @@ def kvbm_copy_f16(to_stacked: bool, stacked_layout: int, contiguous_layout: int,
 
 def add_rms_norm_decode_raw_f16(residual, x, w, out, residual_out, eps: float, *, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/norms.rs:22-153: one row of N halves, the tensors' addresses passed as raw pointers"""
-    _launch("add_rms_norm_decode_raw_f16", _stream(stream), *[t.data_ptr() for t in (residual, x, w, out, residual_out)], float(eps), int(w.numel()),
+    _c.add_rms_norm_decode_raw_f16(stream, *[t.data_ptr() for t in (residual, x, w, out, residual_out)], float(eps), int(w.numel()),
             (None, generics, None))
 
 
@@ -661,14 +676,14 @@ def qk_norm_rope_kv_prefill_raw_f16(q, k, v, q_weight, k_weight, inv_freq, q_out
     for t in tensors:
         if not t.is_contiguous():
             raise CutileError(-5, "qk_norm_rope_kv_prefill_raw_f16: raw-pointer kernel, every tensor must be contiguous")
-    _launch("qk_norm_rope_kv_prefill_raw_f16", _stream(stream), *[t.data_ptr() for t in tensors], float(eps), int(position_start), int(seq_len),
+    _c.qk_norm_rope_kv_prefill_raw_f16(stream, *[t.data_ptr() for t in tensors], float(eps), int(position_start), int(seq_len),
             int(q.shape[1]), int(k.shape[1]), int(q.shape[2]), int(k_cache.shape[1]), (None, generics, None))
 
 
 def qk_norm_rope_kv_decode_raw_f16(qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache, position_start, eps: float,
                                    num_q_heads: int, num_kv_heads: int, *, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/fused_transformer.rs:356-625; qkv: one token's q, k and v heads back to back"""
-    _launch("qk_norm_rope_kv_decode_raw_f16", _stream(stream), *[t.data_ptr() for t in (qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache)],
+    _c.qk_norm_rope_kv_decode_raw_f16(stream, *[t.data_ptr() for t in (qkv, q_weight, k_weight, inv_freq, q_out, k_cache, v_cache)],
             (position_start, U32), float(eps), int(num_q_heads), int(num_kv_heads), int(k_cache.shape[2]), int(k_cache.shape[1]), (None, generics, None))
 
 
@@ -676,7 +691,7 @@ def group_gemm_f16_nt_desc(a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, nu
                            generics=None, variant=None) -> None:
     """cutile-kernels/src/experimental/moe.rs:67-128: pointer tables (int64) and descriptor tables (int32 [groups, 8]:
     rows, cols, row stride) in device memory; generics [BM, BN, BK, NUM_SM]"""
-    _launch("group_gemm_f16_nt_desc", _stream(stream), a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, int(num_groups), (grid, generics, variant))
+    _c.group_gemm_f16_nt_desc(stream, a_ptrs, b_ptrs, c_ptrs, a_metas, b_metas, c_metas, int(num_groups), (grid, generics, variant))
 
 
 def _u32_partition(p: Partition) -> Partition:
@@ -686,28 +701,28 @@ def _u32_partition(p: Partition) -> Partition:
 
 def argmax_blocks_f16(logits, block_max: Partition, block_idx: Partition, length: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/argmax.rs:21-71; block_idx: an int32 / uint32 tensor of u32 indices"""
-    _launch("argmax_blocks_f16", _stream(stream), logits, block_max, _u32_partition(block_idx), int(length), (grid, generics, None))
+    _c.argmax_blocks_f16(stream, logits, block_max, _u32_partition(block_idx), int(length), (grid, generics, None))
 
 
 def lm_head_argmax_blocks_f16(weights, hidden, block_max: Partition, block_idx: Partition, vocab_size: int, *, stream=None,
                               grid=None, generics=None) -> None:
     """cutile-kernels/src/argmax.rs:88-158"""
-    _launch("lm_head_argmax_blocks_f16", _stream(stream), weights, hidden, block_max, _u32_partition(block_idx), int(vocab_size), (grid, generics, None))
+    _c.lm_head_argmax_blocks_f16(stream, weights, hidden, block_max, _u32_partition(block_idx), int(vocab_size), (grid, generics, None))
 
 
 def argmax_reduce_blocks_to_u32(block_max, block_idx, out: Partition, num_blocks: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/argmax.rs:173-213"""
-    _launch("argmax_reduce_blocks_to_u32", _stream(stream), block_max, (block_idx, U32), _u32_partition(out), int(num_blocks), (grid, generics, None))
+    _c.argmax_reduce_blocks_to_u32(stream, block_max, (block_idx, U32), _u32_partition(out), int(num_blocks), (grid, generics, None))
 
 
 def embedding_batch_f16(token_ids, table, out: Partition, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/embeddings.rs:21-41; token_ids: an int32 / uint32 tensor of u32 ids"""
-    _launch("embedding_batch_f16", _stream(stream), (token_ids, U32), table, out, (grid, generics, None))
+    _c.embedding_batch_f16(stream, (token_ids, U32), table, out, (grid, generics, None))
 
 
 def gather_row_f16(src, out: Partition, row_idx: int, *, stream=None, grid=None, generics=None) -> None:
     """cutile-kernels/src/pointwise.rs:86-99"""
-    _launch("gather_row_f16", _stream(stream), src, out, int(row_idx), (grid, generics, None))
+    _c.gather_row_f16(stream, src, out, int(row_idx), (grid, generics, None))
 
 
 def fmha_seq_f16(q, k, v, out: Partition, qk_scale: float, query_group_size: int, *, kv_len: int = 0, query_start: int = 0,
@@ -719,7 +734,7 @@ def fmha_seq_f16(q, k, v, out: Partition, qk_scale: float, query_group_size: int
       flash_attn_causal_seq_dynpos_f16 (:128-231) position_start (one u32 on the device), kv_len_from_position
       fmha_prefill_causal (:242-391), fmha_prefill_gqa (:408-587)   kv_len, query_start by value, causal or not
       fmha_causal (:598-726)                      position_start, every key of k"""
-    _launch("fmha_seq_f16", _stream(stream), q, k, v, out, float(qk_scale), int(query_group_size), int(kv_len), int(query_start),
+    _c.fmha_seq_f16(stream, q, k, v, out, float(qk_scale), int(query_group_size), int(kv_len), int(query_start),
             (position_start, U32) if position_start is not None else None, int(kv_len_from_position), int(causal), (grid, generics, variant))
 
 
@@ -727,7 +742,7 @@ def fmha_prefill_gqa_lpt_raw_f16(q, k, v, out, qk_scale: float, query_group_size
                                  causal: bool = True, stream=None, generics=None) -> None:
     """cutile-kernels/src/experimental/attention.rs:22-377; contiguous q / out [q_len, q_heads, D] and k / v [kv_heads, kv_len, D]
     passed as raw addresses"""
-    _launch("fmha_prefill_gqa_lpt_raw_f16", _stream(stream), *[t.data_ptr() for t in (q, k, v, out)], float(qk_scale), int(query_group_size),
+    _c.fmha_prefill_gqa_lpt_raw_f16(stream, *[t.data_ptr() for t in (q, k, v, out)], float(qk_scale), int(query_group_size),
             int(q.shape[0]), int(kv_len), int(query_start), int(q.shape[1]) // int(group), int(group), int(q.shape[2]), int(causal), (None, generics, None))
 
 
@@ -735,7 +750,7 @@ def linear_tile_mxfp8(z: Partition, x, y, x_scales, y_scales, alpha: float = 1.0
                       generics=None, variant=None) -> None:
     """cutile-examples/examples/mxfp8.rs:34-64.  x, y: uint8 (or float8_e4m3fn) tensors of
     e4m3fn bytes; scales: uint8 (or float8_e8m0fnu) tensors of e8m0 bytes."""
-    _launch("linear_tile_mxfp8", _stream(stream), z, (x, F8E4M3FN), (y, F8E4M3FN), (x_scales, F8E8M0FNU), (y_scales, F8E8M0FNU), float(alpha),
+    _c.linear_tile_mxfp8(stream, z, (x, F8E4M3FN), (y, F8E4M3FN), (x_scales, F8E8M0FNU), (y_scales, F8E8M0FNU), float(alpha),
             (grid, generics, variant))
 
 
@@ -743,7 +758,7 @@ def linear_tile_nvfp4(z: Partition, x, y, x_scales, y_scales, alpha: float = 1.0
                       generics=None, variant=None) -> None:
     """cutile-examples/examples/nvfp4.rs:24-78.  x [M, K/2], y [N, K/2]: uint8 tensors of packed e2m1 pairs (low
     nibble first); scales [M, K/16], [N, K/16]: uint8 (or float8_e4m3fn) tensors of e4m3fn bytes; z f32 or bf16."""
-    _launch("linear_tile_nvfp4", _stream(stream), z, (x, F4E2M1FNX2), (y, F4E2M1FNX2), (x_scales, F8E4M3FN), (y_scales, F8E4M3FN), float(alpha),
+    _c.linear_tile_nvfp4(stream, z, (x, F4E2M1FNX2), (y, F4E2M1FNX2), (x_scales, F8E4M3FN), (y_scales, F8E4M3FN), float(alpha),
             (grid, generics, variant))
 
 

@@ -25,7 +25,11 @@ PyObject *s_tensor, *s_shape, *s_prefix, *s_dtype, *s_arg;   // attribute names 
 struct Binding {
   PyObject* tensor_arg;        // tensor_arg(object, element type or None) -> the ABI's record as a ctypes structure
   PyObject* partition_type;    // the class Partition; objects of any other class are asked for their record: o.arg()
+  PyObject* stream_source;     // () -> (ordinal of the current device, (ordinal) -> handle of its current stream), or None without a GPU
+  PyObject* check;             // check(status) raises
 };
+// That pair, once it is known: a GPU that torch has found stays.
+PyObject *s_device_of = nullptr, *s_stream_of = nullptr;
 
 // Copies a ctypes structure; takes the reference.
 template <typename T>
@@ -131,6 +135,35 @@ bool fill_partition(PyObject* o, const Binding& b, cutile_partition_arg_t* p) {
   Py_XDECREF(prefix);
   Py_XDECREF(dtype);
   return ok;
+}
+
+// The stream of a launch: the caller's, or the current one of torch.
+bool read_stream(PyObject* o, const Binding& b, void** stream) {
+  PyObject* handle;
+  if (o != Py_None) {
+    handle = PyNumber_Long(o);
+  } else {
+    if (!s_stream_of) {
+      PyObject* pair = PyObject_CallNoArgs(b.stream_source);
+      if (!pair) return false;
+      if (pair == Py_None || !PyArg_ParseTuple(pair, "OO", &s_device_of, &s_stream_of)) {
+        const bool none = pair == Py_None;
+        Py_DECREF(pair);
+        *stream = nullptr;
+        return none;
+      }
+      Py_INCREF(s_device_of);
+      Py_INCREF(s_stream_of);
+      Py_DECREF(pair);
+    }
+    PyObject* device = PyObject_CallNoArgs(s_device_of);
+    handle = device ? PyObject_CallOneArg(s_stream_of, device) : nullptr;
+    Py_XDECREF(device);
+  }
+  if (!handle) return false;
+  *stream = PyLong_AsVoidPtr(handle);
+  Py_DECREF(handle);
+  return !PyErr_Occurred();
 }
 
 // ---- one Python argument -> one argument of the launcher ----
@@ -260,18 +293,20 @@ struct From<const cutile_launch_opts_t*> {   // (grid or None, generics or None,
 };
 
 template <typename... A, size_t... I>
-PyObject* call_with(cutile_status_t (*fn)(A...), const Binding& b, PyObject* const* args, std::index_sequence<I...>) {
+PyObject* call_with(cutile_status_t (*fn)(cutile_stream_t, A...), const Binding& b, PyObject* const* args, std::index_sequence<I...>) {
+  void* stream;
   std::tuple<From<A>...> from;
-  if (!(std::get<I>(from).read(args[I], b) && ...)) return nullptr;
+  if (!read_stream(args[0], b, &stream) || !(std::get<I>(from).read(args[1 + I], b) && ...)) return nullptr;
   cutile_status_t status;
   Py_BEGIN_ALLOW_THREADS   // a launch may wait for room in a full queue
-  status = fn(std::get<I>(from).get()...);
+  status = fn((cutile_stream_t)stream, std::get<I>(from).get()...);
   Py_END_ALLOW_THREADS
-  return PyLong_FromLong(status);
+  if (status == CUTILE_SUCCESS) Py_RETURN_NONE;
+  return PyObject_CallFunction(b.check, "i", (int)status);
 }
 template <typename... A>
-PyObject* call(cutile_status_t (*fn)(A...), const Binding& b, PyObject* const* args, Py_ssize_t n) {
-  if (n != (Py_ssize_t)sizeof...(A)) return PyErr_Format(PyExc_TypeError, "the launcher takes %zd arguments, got %zd", (Py_ssize_t)sizeof...(A), n);
+PyObject* call(cutile_status_t (*fn)(cutile_stream_t, A...), const Binding& b, PyObject* const* args, Py_ssize_t n) {
+  if (n != 1 + (Py_ssize_t)sizeof...(A)) return PyErr_Format(PyExc_TypeError, "the launcher takes %zd arguments, got %zd", 1 + (Py_ssize_t)sizeof...(A), n);
   return call_with(fn, b, args, std::make_index_sequence<sizeof...(A)>());
 }
 
@@ -301,6 +336,8 @@ void launcher_dealloc(PyObject* self) {
   Binding& b = ((Launcher*)self)->binding;
   Py_XDECREF(b.tensor_arg);
   Py_XDECREF(b.partition_type);
+  Py_XDECREF(b.stream_source);
+  Py_XDECREF(b.check);
   PyObject_Free(self);
 }
 PyTypeObject launcher_type = {PyVarObject_HEAD_INIT(nullptr, 0) "cutile_marshal.Launcher", sizeof(Launcher)};
@@ -332,8 +369,8 @@ PyObject* names(PyObject*, PyObject*) {
 PyObject* launcher(PyObject*, PyObject* args) {
   const char* name;
   unsigned long long address;
-  PyObject *tensor_arg, *partition_type;
-  if (!PyArg_ParseTuple(args, "sKOO", &name, &address, &tensor_arg, &partition_type)) return nullptr;
+  PyObject *tensor_arg, *partition_type, *stream_source, *check;
+  if (!PyArg_ParseTuple(args, "sKOOOO", &name, &address, &tensor_arg, &partition_type, &stream_source, &check)) return nullptr;
   for (auto& k : kLaunchers)
     if (strcmp(k.name, name) == 0) {
       Launcher* l = PyObject_New(Launcher, &launcher_type);
@@ -342,7 +379,9 @@ PyObject* launcher(PyObject*, PyObject* args) {
       l->address = (void*)(uintptr_t)address;
       Py_INCREF(tensor_arg);
       Py_INCREF(partition_type);
-      l->binding = {tensor_arg, partition_type};
+      Py_INCREF(stream_source);
+      Py_INCREF(check);
+      l->binding = {tensor_arg, partition_type, stream_source, check};
       l->invoke = k.invoke;
       return (PyObject*)l;
     }
@@ -350,7 +389,7 @@ PyObject* launcher(PyObject*, PyObject* args) {
 }
 
 PyMethodDef methods[] = {{"names", names, METH_NOARGS, "names of the launchers this module can call"},
-                         {"launcher", launcher, METH_VARARGS, "launcher(name, address, tensor_arg, Partition): the callable for cutile_launch_<name> at that address"},
+                         {"launcher", launcher, METH_VARARGS, "launcher(name, address, tensor_arg, Partition, stream_source, check): the callable for cutile_launch_<name> at that address"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "cutile_marshal", nullptr, -1, methods};
 

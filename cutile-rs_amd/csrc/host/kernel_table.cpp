@@ -43,7 +43,7 @@ struct ClassWinner {
   std::string variant;
   bool from_record;
 };
-std::unordered_map<std::string, ClassWinner> g_bucket_preferred;   // every launch of a function with shape classes looks here
+std::map<std::string, ClassWinner, std::less<>> g_bucket_preferred;   // every launch of a function with shape classes looks here
 std::atomic<size_t> g_run_time_winners{0};   // how many of them the program named
 void count_run_time_winners() {   // under g_pref_mutex
   size_t n = 0;
@@ -491,17 +491,17 @@ const std::vector<const KernelEntry*>& kernels_of(const char* function) {
 
 // (function, variant) -> entry.  Every launch looks its kernel up at least once, so the table is indexed once
 // (the first entry of a key wins, as a scan in table order would find it).
-const KernelEntry* find_entry(const char* function, const std::string& variant) {
-  static const std::unordered_map<std::string, const KernelEntry*> index = [] {
-    std::unordered_map<std::string, const KernelEntry*> m;
-    for (const auto& e : kernel_table()) m.emplace(std::string(e.function) + '|' + e.variant, &e);
+const KernelEntry* find_entry(std::string_view function, std::string_view variant) {
+  using Key = std::pair<std::string_view, std::string_view>;   // (into the table, which stays)
+  struct Hash {
+    size_t operator()(const Key& k) const { return std::hash<std::string_view>()(k.first) * 31 + std::hash<std::string_view>()(k.second); }
+  };
+  static const auto& index = *[] {
+    auto* m = new std::unordered_map<Key, const KernelEntry*, Hash>();
+    for (const auto& e : kernel_table()) m->emplace(Key(e.function, e.variant), &e);
     return m;
   }();
-  std::string key;
-  key.reserve(strlen(function) + 1 + variant.size());
-  key.append(function).push_back('|');
-  key.append(variant);
-  auto it = index.find(key);
+  auto it = index.find(Key(function, variant));
   return it == index.end() ? nullptr : it->second;
 }
 
@@ -537,24 +537,23 @@ std::string preferred_variant(const char* function) {
   return it == g_preferred.end() ? std::string() : it->second;
 }
 
-std::string class_winner(const char* function, const std::string& bucket, bool* from_record) {
+Name class_winner(std::string_view function, std::string_view bucket, bool* from_record) {
   *from_record = false;
-  if (bucket.empty()) return std::string();
-  std::string key;
-  key.reserve(96);
-  key.append(function).append("|").append(bucket);
+  if (bucket.empty()) return Name();
+  Name key(function);
+  (key += "|") += bucket;
   std::lock_guard<std::mutex> lock(g_pref_mutex);
-  auto it = g_bucket_preferred.find(key);
-  if (it == g_bucket_preferred.end()) return std::string();
+  auto it = g_bucket_preferred.find(std::string_view(key));
+  if (it == g_bucket_preferred.end()) return Name();
   *from_record = it->second.from_record;
   return it->second.variant;
 }
 
-std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time) {
-  if (at_run_time && g_run_time_winners.load(std::memory_order_acquire) == 0) return std::string();
+Name preferred_variant_for(std::string_view function, std::string_view bucket, bool at_run_time) {
+  if (at_run_time && g_run_time_winners.load(std::memory_order_acquire) == 0) return Name();
   bool from_record = false;
-  std::string variant = class_winner(function, bucket, &from_record);
-  return from_record == at_run_time ? std::string() : variant;
+  const Name variant = class_winner(function, bucket, &from_record);
+  return from_record == at_run_time ? Name() : variant;
 }
 
 cutile_status_t set_class_winner(const char* function, const char* bucket, const char* variant, bool from_record) {

@@ -5,8 +5,10 @@
 // (workgroup shape, LDS bytes, the tile shape it implements).
 #pragma once
 #include <string>
+#include <string_view>
 #include <vector>
 
+#include "names.h"
 #include "runtime_state.h"
 
 namespace cutile {
@@ -31,7 +33,7 @@ const std::vector<KernelEntry>& kernel_table();
 // The entries of one function, in table order; empty if there are none.
 const std::vector<const KernelEntry*>& kernels_of(const char* function);
 // Finds the entry (function, variant); nullptr if absent.
-const KernelEntry* find_entry(const char* function, const std::string& variant);
+const KernelEntry* find_entry(std::string_view function, std::string_view variant);
 // The member of `family` with that suffix ("+..."), nullptr if it has none: variants that only a launcher names.
 const KernelEntry* member_of(const KernelEntry* family, const char* suffix);
 // Resolves the entry's hipFunction_t on `device`, loading its code object on
@@ -40,9 +42,9 @@ cutile_status_t load_entry(cutile_device_t device, const KernelEntry* entry, hip
 // Preferred variant set through cutile_kernel_set_preferred_variant, or "".
 std::string preferred_variant(const char* function);
 // Winner of (function, shape-class bucket), or "", and whether a tuning record names it (otherwise the program did, at run time).
-std::string class_winner(const char* function, const std::string& bucket, bool* from_record);
+Name class_winner(std::string_view function, std::string_view bucket, bool* from_record);
 // The winner of (function, shape-class bucket) that the program set at run time, or (at_run_time false) that a tuning record names; or "".
-std::string preferred_variant_for(const char* function, const std::string& bucket, bool at_run_time);
+Name preferred_variant_for(std::string_view function, std::string_view bucket, bool at_run_time);
 cutile_status_t set_class_winner(const char* function, const char* bucket, const char* variant, bool from_record);
 void clear_bucket_preferences();
 // Loads the tuning records once per process (tuning.cpp); cheap afterwards.

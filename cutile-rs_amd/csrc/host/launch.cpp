@@ -23,6 +23,7 @@
 #include "common.h"
 #include "gemm_choice.h"
 #include "kernel_table.h"
+#include "names.h"
 #include "runtime_state.h"
 #include "scratch.h"
 #include "../kernels/mapped_partition.h"
@@ -156,7 +157,7 @@ thread_local std::string g_bucket;
 thread_local std::string g_last_source;
 thread_local std::string g_last_bucket;
 struct BucketScope {
-  explicit BucketScope(std::string b) { g_bucket = std::move(b); }
+  explicit BucketScope(const Name& b) { g_bucket.assign(b.c_str(), b.size()); }
   ~BucketScope() { g_bucket.clear(); }
 };
 thread_local const KernelEntry* g_last_entry = nullptr;
@@ -238,7 +239,7 @@ int64_t numel(const cutile_tensor_arg_t& t) {
 }
 
 // Optional .generics() check: entry i of the caller's list must equal `expect`.
-cutile_status_t check_generic(const cutile_launch_opts_t* o, int i, const std::string& expect, const char* what) {
+cutile_status_t check_generic(const cutile_launch_opts_t* o, int i, const Name& expect, const char* what) {
   if (!o || !o->generics || i >= o->n_generics) return CUTILE_SUCCESS;
   CUTILE_REQUIRE(o->generics[i] && expect == o->generics[i], CUTILE_ERR_KERNEL_LAUNCH,
                  "generic %s: launcher was given '%s' but the arguments imply '%s'", what,
@@ -266,7 +267,7 @@ cutile_status_t resolve_grid(const cutile_partition_arg_t* out, const cutile_lau
   return cutile_infer_launch_grid(explicit_grid, parts, 1, grid);
 }
 
-cutile_status_t load_resolved(const char* function, const std::string& variant, Resolved* r) {
+cutile_status_t load_resolved(const char* function, const Name& variant, Resolved* r) {
   r->entry = find_entry(function, variant);
   CUTILE_REQUIRE(r->entry, CUTILE_ERR_KERNEL_NOT_FOUND, "no variant '%s' of kernel '%s'; available: %s",
                  variant.c_str(), function, list_variants(function).c_str());
@@ -284,12 +285,12 @@ cutile_status_t load_resolved(const char* function, const std::string& variant, 
 // `sized` (the launcher's own rule for extents that the shape classes of the tuning records do not tell apart), the shape
 // class's winner of a verified tuning record, then `fallback` (the table's order).  A pin or a winner that does not fit
 // these arguments is passed over, not an error.
-cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* opts, const std::string& fallback,
-                              const std::vector<std::string>& acceptable, Resolved* r, const std::string& sized = std::string()) {
-  std::string want;
+cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* opts, const Name& fallback,
+                              const Names& acceptable, Resolved* r, const Name& sized = Name()) {
+  Name want;
   g_last_source = "caller";
   g_last_bucket = g_bucket;
-  auto fits = [&](const std::string& v) { return !v.empty() && std::find(acceptable.begin(), acceptable.end(), v) != acceptable.end(); };
+  auto fits = [&](const Name& v) { return !v.empty() && std::find(acceptable.begin(), acceptable.end(), v) != acceptable.end(); };
   if (opts && opts->variant) want = opts->variant;
   if (want.empty()) {
     std::string pref = preferred_variant(function);
@@ -298,7 +299,7 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
       g_last_source = "pinned";
     }
   }
-  std::string winner;
+  Name winner;
   bool from_record = false;
   if (want.empty() && !g_bucket.empty()) {
     ensure_tuning_records_loaded();
@@ -310,7 +311,7 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
     g_last_source = "size";
   } else if (!winner.empty()) {
     want = winner;
-    g_last_source = "record:" + g_bucket;
+    g_last_source.assign("record:").append(g_bucket);
   } else if (want.empty() && fits(sized)) {
     want = sized;
     g_last_source = "size";
@@ -321,7 +322,7 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
   }
   if (!acceptable.empty() && std::find(acceptable.begin(), acceptable.end(), want) == acceptable.end()) {
     std::string list;
-    for (auto& a : acceptable) list += (list.empty() ? "" : ", ") + a;
+    for (auto& a : acceptable) list.append(list.empty() ? "" : ", ").append(a.c_str());
     return fail(CUTILE_ERR_KERNEL_NOT_FOUND, "variant '%s' of kernel '%s' does not fit these arguments; fitting: %s",
                 want.c_str(), function, list.c_str());
   }
@@ -336,7 +337,7 @@ cutile_status_t resolve_own(const char* function, const char* variant, const cha
 }
 
 // The table's first kernel for a partition's tile shape, or nullptr.
-const KernelEntry* first_of_tile(const char* function, const std::string& dtype, int bm, int bn) {
+const KernelEntry* first_of_tile(const char* function, const Name& dtype, int bm, int bn) {
   for (const KernelEntry* e : kernels_of(function))
     if (e->tile[0] == bm && e->tile[1] == bn && dtype == e->dtype) return e;
   return nullptr;
@@ -379,10 +380,11 @@ struct ScaledRoom {
 // Picks the kernel of a block-scaled product.  A kernel tile that is a whole multiple of the partition tile computes the
 // same output when the launch covers the whole tensor (a 16 x 16 example partition runs on the 32 x 32 kernel), and so do
 // the kernels on wave-private stages, which take `flat` launches: whole outputs, scale rows on 4-byte boundaries.
-cutile_status_t resolve_scaled(const char* function, const char* prefix, const std::string& dt, int bm, int bn, bool full_cover, bool flat,
-                               const ScaledShape& shape, const cutile_launch_opts_t* opts, const std::string& missing, cutile_stream_t stream, int* cus,
+template <typename Missing>
+cutile_status_t resolve_scaled(const char* function, const char* prefix, const Name& dt, int bm, int bn, bool full_cover, bool flat,
+                               const ScaledShape& shape, const cutile_launch_opts_t* opts, Missing missing, cutile_stream_t stream, int* cus,
                                ScaledRoom* room, Resolved* res) {
-  std::vector<const KernelEntry*> fit, others;
+  Few<const KernelEntry*, 12> fit, others;
   for (const KernelEntry* e : kernels_of(function)) {
     if (e->image == IMG_MX_TILES || dt != e->dtype) continue;   // (members, which only launch_scaled names)
     if (is_scaled_flat(e)) {
@@ -391,14 +393,14 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
       fit.push_back(e);
     }
   }
-  CUTILE_REQUIRE(!fit.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "%s; available: %s", missing.c_str(), list_variants(function).c_str());
-  std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
+  CUTILE_REQUIRE(!fit.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "%s; available: %s", missing().c_str(), list_variants(function).c_str());
+  sort_few(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
     bool ea = a->tile[0] == bm && a->tile[1] == bn, eb = b->tile[0] == bm && b->tile[1] == bn;
     if (ea != eb) return ea;
     return a->tile[0] * a->tile[1] < b->tile[0] * b->tile[1];
   });
   *cus = 256;
-  std::string sized;
+  Name sized;
   if (flat || (shape.fp4 && full_cover && shape.pieces <= 1)) {
     if (cutile_status_t s = current_device_units(cus)) return s;
     const char* kernel = choose_scaled(shape, fit[0]->tile[0], fit[0]->tile[1], *cus, room->bytes, &room->lone);
@@ -417,7 +419,7 @@ cutile_status_t resolve_scaled(const char* function, const char* prefix, const s
   }
   if (!sized.empty() && !(opts && opts->variant) && preferred_variant(function).empty() && preferred_variant_for(function, g_bucket, true).empty())
     return resolve_own(function, sized.c_str(), "size", res);
-  std::vector<std::string> acceptable;
+  Names acceptable;
   for (const KernelEntry* e : fit) acceptable.push_back(e->variant);
   for (const KernelEntry* e : others) acceptable.push_back(e->variant);
   return resolve_entry(function, opts, acceptable[0], acceptable, res, sized);
@@ -520,10 +522,10 @@ cutile_status_t stream_member(Resolved* r, bool accumulate, const cutile_tensor_
 }
 
 // Shape classes of tuning records: row lengths by the next power of two (at least 256).
-std::string pow2_class(int64_t n) {
+Name pow2_class(int64_t n) {
   int64_t p = 256;
   while (p < n) p *= 2;
-  return "<=" + std::to_string(p);
+  return "<=" + num(p);
 }
 
 const char* float_dtype_name(cutile_dtype_t dt) { return kDTypes[dt].name; }
@@ -564,7 +566,7 @@ cutile_status_t cutile_infer_launch_grid(const uint32_t explicit_grid[3], const 
                                          int32_t n_partitions, uint32_t grid[3]) {
   CUTILE_REQUIRE(grid && (partitions || n_partitions <= 0), CUTILE_ERR_INVALID_ARGUMENT, "null argument");
   struct Bound { uint32_t g[3]; bool exact; };
-  std::vector<Bound> bounds;
+  Few<Bound, 4> bounds;
   for (int i = 0; i < n_partitions; ++i) {
     Bound b;
     if (cutile_status_t s = cutile_partition_grid(partitions[i], b.g)) return s;
@@ -744,7 +746,7 @@ static cutile_status_t launch_elementwise3(const char* fn_name, cutile_stream_t 
     if (cutile_status_t s = check_tensor(in1, "y", rank, rank)) return s;
   CUTILE_REQUIRE(in0->dtype == ot.dtype && (!in1 || in1->dtype == ot.dtype), CUTILE_ERR_KERNEL_LAUNCH,
                  "%s: all operands must have element type %s", fn_name, cutile_dtype_name(ot.dtype));
-  const std::string dt = cutile_dtype_name(ot.dtype);
+  const Name dt = cutile_dtype_name(ot.dtype);
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   uint32_t full[3];
@@ -754,8 +756,8 @@ static cutile_status_t launch_elementwise3(const char* fn_name, cutile_stream_t 
   bool flat_ok = is_contiguous(ot) && is_contiguous(*in0) && same_shape(ot, *in0) && aligned16(ot.ptr) &&
                  aligned16(in0->ptr) && (rank == 1 || full_cover);
   if (in1) flat_ok = flat_ok && is_contiguous(*in1) && same_shape(ot, *in1) && aligned16(in1->ptr);
-  const std::string r = "_r" + std::to_string(rank);
-  std::vector<std::string> acceptable;
+  const Name r = "_r" + num(rank);
+  Names acceptable;
   if (flat_ok && find_entry(fn_name, dt + r + "_flat")) acceptable.push_back(dt + r + "_flat");
   if (find_entry(fn_name, dt + r + "_tiled")) acceptable.push_back(dt + r + "_tiled");
   CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "no precompiled variant of %s<%s> for rank %d; available: %s",
@@ -802,7 +804,7 @@ static cutile_status_t launch_pointwise_2d_f16(const char* name, const char* ker
                                                const cutile_tensor_arg_t* b, const cutile_launch_opts_t* opts) {
   CUTILE_REQUIRE(out && out->tensor.rank == 2 && out->tensor.dtype == CUTILE_DTYPE_F16 && out->partition_shape[0] == 1,
                  CUTILE_ERR_KERNEL_LAUNCH, "%s: out must be a rank-2 f16 tensor partitioned [1, BLOCK_SIZE]", name);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(out->partition_shape[1]), "BLOCK_SIZE")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(out->partition_shape[1]), "BLOCK_SIZE")) return s;
   cutile_launch_opts_t o = opts ? *opts : cutile_launch_opts_t{};
   o.generics = nullptr;   // validated above; the kernels themselves are keyed by the element type
   o.n_generics = 0;
@@ -830,7 +832,7 @@ static cutile_status_t launch_creation(const char* fn_name, cutile_stream_t stre
   if (cutile_status_t s = check_partition(t, "tensor", 1, 1)) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(t, opts, tg)) return s;
-  const std::string dt = cutile_dtype_name(t->tensor.dtype);
+  const Name dt = cutile_dtype_name(t->tensor.dtype);
   Resolved res;
   if (cutile_status_t s = resolve_entry(fn_name, opts, dt, {dt}, &res)) return s;
   ArgPacker args;
@@ -858,8 +860,8 @@ cutile_status_t cutile_launch_arange(cutile_stream_t stream, const cutile_partit
 cutile_status_t cutile_launch_eye(cutile_stream_t stream, const cutile_partition_arg_t* t, const cutile_launch_opts_t* opts) {
   if (cutile_status_t s = check_partition(t, "tensor", 2, 2)) return s;
   CUTILE_REQUIRE(t->tensor.dtype == CUTILE_DTYPE_F32, CUTILE_ERR_KERNEL_LAUNCH, "eye: tensor must be f32");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(t->partition_shape[0]), "BR")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(t->partition_shape[1]), "BC")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(t->partition_shape[0]), "BR")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(t->partition_shape[1]), "BC")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(t, opts, tg)) return s;
   Resolved res;
@@ -882,7 +884,7 @@ cutile_status_t cutile_launch_relu(cutile_stream_t stream, const cutile_partitio
                                    const cutile_launch_opts_t* opts) {
   if (cutile_status_t s = check_partition(input_output, "input_output", 1, 1)) return s;
   CUTILE_REQUIRE(input_output->tensor.dtype == CUTILE_DTYPE_F32, CUTILE_ERR_KERNEL_LAUNCH, "relu: tensor must be f32");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(input_output->partition_shape[0]), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(input_output->partition_shape[0]), "D")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(input_output, opts, tg)) return s;
   Resolved res;
@@ -902,7 +904,7 @@ cutile_status_t cutile_launch_dropout(cutile_stream_t stream, float p, const cut
   if (cutile_status_t s = check_partition(out, "out", 1, 1)) return s;
   CUTILE_REQUIRE(x->dtype == CUTILE_DTYPE_F32 && x_keep->dtype == CUTILE_DTYPE_F32 && out->tensor.dtype == CUTILE_DTYPE_F32,
                  CUTILE_ERR_KERNEL_LAUNCH, "dropout: x, x_keep and out must be f32");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(out->partition_shape[0]), "S")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(out->partition_shape[0]), "S")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   Resolved res;
@@ -941,11 +943,11 @@ cutile_status_t cutile_launch_matvec(cutile_stream_t stream, const cutile_partit
   if (cutile_status_t s = check_tensor(y, "y", 1, 1)) return s;
   CUTILE_REQUIRE(z->tensor.dtype == CUTILE_DTYPE_F32 && x->dtype == CUTILE_DTYPE_F32 && y->dtype == CUTILE_DTYPE_F32,
                  CUTILE_ERR_KERNEL_LAUNCH, "matvec: z, x and y must be f32");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(z->partition_shape[0]), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(z->partition_shape[0]), "BM")) return s;
   const int bk = generic_int(opts, 1, 1);
   CUTILE_REQUIRE(bk > 0, CUTILE_ERR_KERNEL_LAUNCH, "matvec: BK must be positive");
   CUTILE_REQUIRE(k >= 0, CUTILE_ERR_KERNEL_LAUNCH, "matvec: k must be non-negative");
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(k), "K")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(k), "K")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(z, opts, tg)) return s;
   Resolved res;
@@ -973,7 +975,7 @@ cutile_status_t cutile_launch_convert(cutile_stream_t stream, const cutile_tenso
   if (cutile_status_t s = check_partition(dst, "dst", 1, 1)) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(dst, opts, tg)) return s;
-  const std::string v = std::string(cutile_dtype_name(src->dtype)) + "_" + cutile_dtype_name(dst->tensor.dtype);
+  const Name v = Name(cutile_dtype_name(src->dtype)) + "_" + cutile_dtype_name(dst->tensor.dtype);
   Resolved res;
   if (cutile_status_t s = resolve_entry("convert", opts, v, {v}, &res)) return s;
   ArgPacker args;
@@ -989,19 +991,19 @@ cutile_status_t cutile_launch_convert(cutile_stream_t stream, const cutile_tenso
 // Measured on MI355X: up to 4 vectors (64 bytes) per lane stream at full rate, so
 // among those the smallest capacity wins and wider segments are split over more
 // wavefronts; only segments too long for that take more vectors per lane.
-static std::vector<std::string> fitting_row_variants(const char* fn_name, const std::string& prefix, int64_t seg_len) {
-  std::vector<const KernelEntry*> fit;
+static Names fitting_row_variants(const char* fn_name, const Name& prefix, int64_t seg_len) {
+  Few<const KernelEntry*, 12> fit;
   for (const KernelEntry* entry : kernels_of(fn_name))
     if (const KernelEntry& e = *entry; e.capacity >= seg_len &&
         strncmp(e.variant, prefix.c_str(), prefix.size()) == 0)
       fit.push_back(&e);
-  std::stable_sort(fit.begin(), fit.end(), [](const KernelEntry* a, const KernelEntry* b) {
+  sort_few(fit.begin(), fit.end(), [](const KernelEntry* a, const KernelEntry* b) {
     const int va = std::max(a->tile[2], 4), vb = std::max(b->tile[2], 4);
     if (va != vb) return va < vb;
     if (a->capacity != b->capacity) return a->capacity < b->capacity;
     return a->tile[3] < b->tile[3];  // fewer wavefronts per segment first
   });
-  std::vector<std::string> names;
+  Names names;
   for (auto* e : fit) names.push_back(e->variant);
   return names;
 }
@@ -1009,7 +1011,7 @@ static std::vector<std::string> fitting_row_variants(const char* fn_name, const 
 // The any-layout kernels of a row-wise function, behind the ones that fit: `held` rows of `bytes` (adjacent elements) are at most what
 // the "generic" kernels hold in registers (kAnyRowMost, rowwise.hip), everything else is walked.  Both take every call.
 static bool row_held(bool adjacent, int64_t bytes) { return adjacent && bytes <= 32768; }
-static void add_any_layout(bool held, const std::string& prefix, std::vector<std::string>* acceptable) {
+static void add_any_layout(bool held, const Name& prefix, Names* acceptable) {
   acceptable->push_back(prefix + (held ? "generic" : "walk"));
   acceptable->push_back(prefix + (held ? "walk" : "generic"));
 }
@@ -1058,7 +1060,7 @@ cutile_status_t cutile_launch_rms_norm_f16(cutile_stream_t stream, const cutile_
                  out->partition_shape[1]);
   CUTILE_REQUIRE(ot.shape[1] == n && ot.shape[0] <= x->shape[0], CUTILE_ERR_KERNEL_LAUNCH,
                  "rms_norm_f16: out is [%d, %d] but x is [%d, %d]", ot.shape[0], ot.shape[1], x->shape[0], n);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(n), "N")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(n), "N")) return s;
   const int block = generic_int(opts, 1, 0);
   CUTILE_REQUIRE(block >= 0 && (block == 0 || n % block == 0), CUTILE_ERR_KERNEL_LAUNCH,
                  "rms_norm_f16: N = %d is not a multiple of BLOCK_SIZE = %d", n, block);
@@ -1068,7 +1070,7 @@ cutile_status_t cutile_launch_rms_norm_f16(cutile_stream_t stream, const cutile_
   const bool vec_ok = n % 8 == 0 && x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1 &&
                       x->strides[0] % 8 == 0 && ot.strides[0] % 8 == 0 && aligned16(x->ptr) && aligned16(ot.ptr) &&
                       aligned16(w->ptr);
-  std::vector<std::string> acceptable;
+  Names acceptable;
   if (vec_ok) acceptable = fitting_row_variants("rms_norm_f16", "", n);
   const bool held = row_held(x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1, 2 * (int64_t)n);
   add_any_layout(held, "", &acceptable);
@@ -1103,7 +1105,7 @@ cutile_status_t cutile_launch_rms_norm_f32(cutile_stream_t stream, const cutile_
                  "rms_norm: out must be partitioned [1, %d], got [%d, %d]", n, out->partition_shape[0], out->partition_shape[1]);
   CUTILE_REQUIRE(ot.shape[1] == n && ot.shape[0] <= x->shape[0], CUTILE_ERR_KERNEL_LAUNCH,
                  "rms_norm: out is [%d, %d] but x is [%d, %d]", ot.shape[0], ot.shape[1], x->shape[0], n);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(n), "N")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(n), "N")) return s;
   const int block = generic_int(opts, 1, 0);
   CUTILE_REQUIRE(block >= 0 && (block == 0 || n % block == 0), CUTILE_ERR_KERNEL_LAUNCH,
                  "rms_norm: N = %d is not a multiple of BLOCK_SIZE = %d", n, block);
@@ -1143,7 +1145,7 @@ cutile_status_t cutile_launch_rms_norm_all_f16(cutile_stream_t stream, const cut
                  out->partition_shape[1]);
   CUTILE_REQUIRE(ot.shape[1] == n && ot.shape[0] <= x->shape[0], CUTILE_ERR_KERNEL_LAUNCH,
                  "rms_norm_all_f16: out is [%d, %d] but x is [%d, %d]", ot.shape[0], ot.shape[1], x->shape[0], n);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(n), "N")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(n), "N")) return s;
   const int block = generic_int(opts, 1, 0);
   CUTILE_REQUIRE(block > 0, CUTILE_ERR_KERNEL_LAUNCH,
                  "rms_norm_all_f16: the generics [N, BLOCK_SIZE] are required (BLOCK_SIZE is the width of the f16 accumulator tile)");
@@ -1158,7 +1160,7 @@ cutile_status_t cutile_launch_rms_norm_all_f16(cutile_stream_t stream, const cut
   cutile_launch_opts_t o = opts ? *opts : cutile_launch_opts_t{};
   o.generics = nullptr;
   o.n_generics = 0;
-  const std::string variant = "v" + std::to_string(v);
+  const Name variant = "v" + num(v);
   Resolved res;
   if (cutile_status_t s = resolve_entry("rms_norm_all_f16", &o, variant, {variant}, &res)) return s;
   ArgPacker args;
@@ -1182,8 +1184,8 @@ cutile_status_t cutile_launch_softmax_all_f16(cutile_stream_t stream, const cuti
   CUTILE_REQUIRE(x->dtype == CUTILE_DTYPE_F16 && yt.dtype == CUTILE_DTYPE_F16, CUTILE_ERR_KERNEL_LAUNCH,
                  "softmax_all_f16: x and y must be f16");
   const int32_t bm = y->partition_shape[0], bn = y->partition_shape[1];
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bn), "BN")) return s;
   CUTILE_REQUIRE(is_pow2(bn) && bn <= 16384, CUTILE_ERR_KERNEL_NOT_FOUND,
                  "softmax_all_f16: BN = %d must be a power of two, at most 16384 (the row is held in one wavefront's registers)", bn);
   uint32_t tg[3];
@@ -1198,7 +1200,7 @@ cutile_status_t cutile_launch_softmax_all_f16(cutile_stream_t stream, const cuti
   cutile_launch_opts_t o = opts ? *opts : cutile_launch_opts_t{};
   o.generics = nullptr;
   o.n_generics = 0;
-  const std::string variant = "c" + std::to_string(ch) + "v" + std::to_string(v);
+  const Name variant = "c" + num(ch) + "v" + num(v);
   Resolved res;
   if (cutile_status_t s = resolve_entry("softmax_all_f16", &o, variant, {variant}, &res)) return s;
   ArgPacker args;
@@ -1246,7 +1248,7 @@ static cutile_status_t launch_fused_norm(const char* fn, cutile_stream_t stream,
                    CUTILE_ERR_KERNEL_LAUNCH, "%s: out is [%d, %d] but residual is [%d, %d] and x [%d, %d]", fn, ot.shape[0],
                    ot.shape[1], a->shape[0], n, b->shape[0], n);
   }
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(n), "N")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(n), "N")) return s;
   uint32_t tg[3];
   if (out2) {
     uint32_t explicit_grid[3] = {0, 0, 0};
@@ -1259,7 +1261,7 @@ static cutile_status_t launch_fused_norm(const char* fn, cutile_stream_t stream,
   auto row_ok = [&](const cutile_tensor_arg_t& t) { return t.strides[1] == 1 && t.strides[0] % 8 == 0 && aligned16(t.ptr); };
   const bool vec_ok = n % 8 == 0 && row_ok(*a) && row_ok(*b) && row_ok(ot) && (!out2 || row_ok(out2->tensor)) &&
                       w->strides[0] == 1 && aligned16(w->ptr) && (!w2 || (w2->strides[0] == 1 && aligned16(w2->ptr)));
-  std::vector<std::string> acceptable;
+  Names acceptable;
   if (vec_ok) acceptable = fitting_row_variants(fn, "", n);
   auto unit = [](const cutile_tensor_arg_t& t) { return t.strides[t.rank - 1] == 1; };
   const bool held = row_held(unit(*a) && unit(*b) && unit(*w) && (!w2 || unit(*w2)) && unit(ot) && (!out2 || unit(out2->tensor)), 2 * (int64_t)n);
@@ -1321,7 +1323,7 @@ cutile_status_t cutile_launch_add_rms_norm_decode_raw_f16(cutile_stream_t stream
     return pa;
   };
   cutile_partition_arg_t op = part(out), rp = part(residual_out);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(n), "N")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(n), "N")) return s;
   cutile_launch_opts_t o = opts ? *opts : cutile_launch_opts_t{};
   o.generics = nullptr;
   o.n_generics = 0;
@@ -1368,8 +1370,8 @@ cutile_status_t cutile_launch_rope_f16(cutile_stream_t stream, const cutile_tens
                        ((uintptr_t)position_start_dev->ptr & 3) == 0,
                    CUTILE_ERR_KERNEL_LAUNCH, "rope: position_start must be one aligned u32");
   }
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(d), "D")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(half), "HALF_D")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(half), "HALF_D")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   CUTILE_REQUIRE(tg[2] == 2, CUTILE_ERR_KERNEL_LAUNCH, "rope: the launch grid must cover both halves of D (grid.z = 2, got %u)", tg[2]);
@@ -1414,8 +1416,8 @@ cutile_status_t cutile_launch_kv_cache_update_f16(cutile_stream_t stream, const 
   CUTILE_REQUIRE(k_cache->partition_shape[0] == 1 && v_cache->partition_shape[0] == 1 && block > 0 && d % block == 0 &&
                      v_cache->partition_shape[1] == k_cache->partition_shape[1] && v_cache->partition_shape[2] == block,
                  CUTILE_ERR_KERNEL_LAUNCH, "kv_cache_update: caches must be partitioned [1, rows, BLOCK_SIZE] with BLOCK_SIZE dividing D = %d", d);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(d), "D")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(block), "BLOCK_SIZE")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(block), "BLOCK_SIZE")) return s;
   uint32_t explicit_grid[3] = {0, 0, 0};
   if (opts) memcpy(explicit_grid, opts->grid, sizeof(explicit_grid));
   const cutile_partition_arg_t* parts[2] = {k_cache, v_cache};
@@ -1508,7 +1510,7 @@ cutile_status_t cutile_launch_lm_head_argmax_blocks_f16(cutile_stream_t stream, 
   CUTILE_REQUIRE(k % 32 == 0, CUTILE_ERR_KERNEL_LAUNCH, "lm_head_argmax_blocks_f16: K = %d must be a multiple of 32", k);
   CUTILE_REQUIRE(k <= 30720, CUTILE_ERR_KERNEL_NOT_FOUND, "lm_head_argmax_blocks_f16: K = %d exceeds the 30720 the precompiled kernel keeps in LDS", k);
   CUTILE_REQUIRE(vocab_size >= 0, CUTILE_ERR_KERNEL_LAUNCH, "lm_head_argmax_blocks_f16: vocab_size must be non-negative");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(k), "K")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(k), "K")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = argmax_outputs_grid("lm_head_argmax_blocks_f16", block_max, block_idx, opts, tg)) return s;
   Resolved res;
@@ -1583,8 +1585,8 @@ cutile_status_t cutile_launch_embedding_batch_f16(cutile_stream_t stream, const 
   CUTILE_REQUIRE(out->partition_shape[0] == 1 && ot.shape[1] == d && ot.shape[0] <= token_ids->shape[0], CUTILE_ERR_KERNEL_LAUNCH,
                  "embedding_batch_f16: out [%d, %d] tiles [%d, %d] must be [tokens <= %d, D = %d] partitioned [1, BLOCK_SIZE]",
                  ot.shape[0], ot.shape[1], out->partition_shape[0], block, token_ids->shape[0], d);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(d), "D")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(block), "BLOCK_SIZE")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(block), "BLOCK_SIZE")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   Resolved res;
@@ -1606,7 +1608,7 @@ cutile_status_t cutile_launch_gather_row_f16(cutile_stream_t stream, const cutil
   CUTILE_REQUIRE(src->dtype == CUTILE_DTYPE_F16 && out->tensor.dtype == CUTILE_DTYPE_F16, CUTILE_ERR_KERNEL_LAUNCH,
                  "gather_row_f16: src and out must be f16");
   CUTILE_REQUIRE(row_idx >= 0, CUTILE_ERR_KERNEL_LAUNCH, "gather_row_f16: row_idx must be non-negative");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(out->partition_shape[0]), "BLOCK_SIZE")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(out->partition_shape[0]), "BLOCK_SIZE")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   Resolved res;
@@ -1644,9 +1646,9 @@ static cutile_status_t launch_qk_norm_rope_kv(const char* name, cutile_stream_t 
     CUTILE_REQUIRE(position_start >= 0 && (int64_t)position_start + seq_len <= max_seq, CUTILE_ERR_KERNEL_LAUNCH,
                    "%s: positions %d .. %lld do not fit the %d rows of the caches", name, position_start,
                    (long long)position_start + seq_len, max_seq);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(d), "D")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(d / 2), "HALF_D")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(max_seq), "MAX_SEQ")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(d / 2), "HALF_D")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(max_seq), "MAX_SEQ")) return s;
   if (seq_len == 0 || num_q_heads + num_kv_heads == 0) return CUTILE_SUCCESS;
   cutile_launch_opts_t o = opts ? *opts : cutile_launch_opts_t{};
   o.generics = nullptr;
@@ -1798,8 +1800,8 @@ static cutile_status_t launch_decode_split(cutile_stream_t stream, const cutile_
   CUTILE_REQUIRE(att_out->partition_shape[0] == 1 && att_out->partition_shape[1] == group && att_out->partition_shape[2] == d &&
                      lse_out->partition_shape[0] == 1 && lse_out->partition_shape[1] == group,
                  CUTILE_ERR_KERNEL_LAUNCH, "fmha_decode_gqa_split: att_out must be partitioned [1, %d, %d] and lse_out [1, %d]", group, d, group);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(group), "GROUP")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(group), "GROUP")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(d), "D")) return s;
   const int bn = generic_int(opts, 1, 64);
   CUTILE_REQUIRE(bn > 0, CUTILE_ERR_KERNEL_LAUNCH, "fmha_decode_gqa_split: BN must be positive");
   uint32_t explicit_grid[3] = {0, 0, 0};
@@ -1807,16 +1809,16 @@ static cutile_status_t launch_decode_split(cutile_stream_t stream, const cutile_
   const cutile_partition_arg_t* parts[2] = {att_out, lse_out};
   uint32_t tg[3];
   if (cutile_status_t s = cutile_infer_launch_grid(explicit_grid, parts, 2, tg)) return s;
-  if (cutile_status_t s = check_generic(opts, 3, std::to_string(tg[1]), "NUM_KV_SPLITS")) return s;
+  if (cutile_status_t s = check_generic(opts, 3, num(tg[1]), "NUM_KV_SPLITS")) return s;
   CUTILE_REQUIRE(decode_vec_layout(*q) && decode_vec_layout(*k) && decode_vec_layout(*v) && decode_vec_layout(at) &&
                      ((uintptr_t)position_start->ptr & 3) == 0 && ((uintptr_t)lt.ptr & 3) == 0,
                  CUTILE_ERR_KERNEL_NOT_FOUND, "fmha_decode_gqa_split: precompiled variants need unit head-dim stride and 16-byte aligned rows");
   // The matrix-core variant first: from GROUP 4 on the vector-ALU one no longer keeps up with HBM, and at D = 64 and
   // 256 it is the slower one for every group; only GROUP 1 and 2 at D = 128 measured (3 %) faster on the vector ALUs.
-  const std::string plain = "f16_g" + std::to_string(group) + "_d" + std::to_string(d);
-  std::vector<std::string> acceptable;
+  const Name plain = "f16_g" + num(group) + "_d" + num(d);
+  Names acceptable;
   const bool vector_first = group <= 2 && d == 128;
-  for (const std::string& name : {vector_first ? plain : plain + "_mfma", vector_first ? plain + "_mfma" : plain})
+  for (const Name& name : {vector_first ? plain : plain + "_mfma", vector_first ? plain + "_mfma" : plain})
     if (find_entry("fmha_decode_gqa_split", name)) acceptable.push_back(name);
   CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND,
                  "no precompiled variant of fmha_decode_gqa_split<GROUP=%d, D=%d>; available: %s", group, d,
@@ -1882,12 +1884,12 @@ cutile_status_t cutile_launch_attention_decode_kernel_grouped_f16(
   // with a remainder the tile program's splits overlap (its first tile is start / TILE_N rounded down, attention.rs:640-641)
   CUTILE_REQUIRE(kv_len_per_split % tile_n == 0, CUTILE_ERR_KERNEL_NOT_FOUND,
                  "%s: the precompiled kernels need KV_LEN_PER_SPLIT (%d) to be a multiple of TILE_N (%d)", fn, kv_len_per_split, tile_n);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(d), "HEAD_DIM")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(tile_n), "TILE_N")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(kv_len_per_split), "KV_LEN_PER_SPLIT")) return s;
-  if (cutile_status_t s = check_generic(opts, 3, std::to_string(group), "NUM_Q_HEAD_PER_KV")) return s;
-  if (cutile_status_t s = check_generic(opts, 4, std::to_string(query_group_tile_size), "QUERY_GROUP_TILE_SIZE")) return s;
-  if (cutile_status_t s = check_generic(opts, 5, std::to_string(splits), "NUM_KV_SPLITS")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(d), "HEAD_DIM")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(tile_n), "TILE_N")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(kv_len_per_split), "KV_LEN_PER_SPLIT")) return s;
+  if (cutile_status_t s = check_generic(opts, 3, num(group), "NUM_Q_HEAD_PER_KV")) return s;
+  if (cutile_status_t s = check_generic(opts, 4, num(query_group_tile_size), "QUERY_GROUP_TILE_SIZE")) return s;
+  if (cutile_status_t s = check_generic(opts, 5, num(splits), "NUM_KV_SPLITS")) return s;
   auto rows_ok = [&](const int32_t* strides, int n) {
     for (int i = 0; i < n; ++i)
       if (strides[i] < 0 || strides[i] % 8 != 0) return false;
@@ -1906,7 +1908,7 @@ cutile_status_t cutile_launch_attention_decode_kernel_grouped_f16(
                    "%s: launch grid (%u, %u, %u) is not (batch, kv heads, NUM_KV_SPLITS) = (%u, %u, %u)", fn, opts->grid[0],
                    opts->grid[1], opts->grid[2], tg[0], tg[1], tg[2]);
   }
-  const std::string name = "f16_g" + std::to_string(group) + "_d" + std::to_string(d);
+  const Name name = "f16_g" + num(group) + "_d" + num(d);
   CUTILE_REQUIRE(find_entry(fn, name), CUTILE_ERR_KERNEL_NOT_FOUND,
                  "no precompiled variant of %s<NUM_Q_HEAD_PER_KV=%d, HEAD_DIM=%d>; available: %s", fn, group, d, list_variants(fn).c_str());
   Resolved res;
@@ -1948,10 +1950,10 @@ static cutile_status_t check_merge(const cutile_tensor_arg_t* att_partial, const
   const int32_t chunk = out->partition_shape[2];
   CUTILE_REQUIRE(out->partition_shape[0] == 1 && out->partition_shape[1] == group && chunk > 0 && d % chunk == 0,
                  CUTILE_ERR_KERNEL_LAUNCH, "splitk_reduce_merge: out must be partitioned [1, %d, CHUNK_D] with CHUNK_D dividing D = %d", group, d);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(group), "GROUP")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(d), "D")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(chunk), "CHUNK_D")) return s;
-  if (cutile_status_t s = check_generic(opts, 3, std::to_string(att_partial->shape[1] / group), "NUM_KV_SPLITS")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(group), "GROUP")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(chunk), "CHUNK_D")) return s;
+  if (cutile_status_t s = check_generic(opts, 3, num(att_partial->shape[1] / group), "NUM_KV_SPLITS")) return s;
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
   CUTILE_REQUIRE((int64_t)tg[2] * chunk >= d, CUTILE_ERR_KERNEL_LAUNCH, "splitk_reduce_merge: the launch grid must cover all of D");
   return CUTILE_SUCCESS;
@@ -2082,7 +2084,7 @@ cutile_status_t cutile_launch_fmha_decode_gqa_noalloc(cutile_stream_t stream, co
   lse.tensor.strides[0] = sg; lse.tensor.strides[1] = 1;
   lse.partition_shape[0] = 1; lse.partition_shape[1] = group;
   lse.partition_strides[0] = lse.partition_strides[1] = 1;
-  const std::string g_s = std::to_string(group), bn_s = std::to_string(bn), d_s = std::to_string(d), n_s = std::to_string(num_kv_splits);
+  const Name g_s = num(group), bn_s = num(bn), d_s = num(d), n_s = num(num_kv_splits);
   const char* generics[4] = {g_s.c_str(), bn_s.c_str(), d_s.c_str(), n_s.c_str()};
   cutile_launch_opts_t split_opts;
   memset(&split_opts, 0, sizeof(split_opts));
@@ -2138,17 +2140,17 @@ cutile_status_t cutile_launch_softmax(cutile_stream_t stream, const cutile_tenso
   CUTILE_REQUIRE(x->dtype == yt.dtype && (x->dtype == CUTILE_DTYPE_F16 || x->dtype == CUTILE_DTYPE_F32),
                  CUTILE_ERR_KERNEL_LAUNCH, "softmax: x and y must both be f16 or both f32");
   const int32_t bm = y->partition_shape[0], bn = y->partition_shape[1];
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bn), "BN")) return s;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(y, opts, tg)) return s;
-  const std::string dt = cutile_dtype_name(x->dtype);
+  const Name dt = cutile_dtype_name(x->dtype);
   const int e = 16 / (int)cutile_dtype_size(x->dtype);
   const uint64_t rows = std::min<uint64_t>((uint64_t)tg[0] * bm, yt.shape[0]);
   const bool vec_ok = bn % e == 0 && x->shape[1] % e == 0 && yt.shape[1] % e == 0 && x->strides[1] == 1 &&
                       yt.strides[1] == 1 && x->strides[0] % e == 0 && yt.strides[0] % e == 0 && aligned16(x->ptr) &&
                       aligned16(yt.ptr) && (uint64_t)x->shape[0] >= rows;
-  std::vector<std::string> acceptable;
+  Names acceptable;
   if (vec_ok) acceptable = fitting_row_variants("softmax", dt + "_w", bn);
   const int64_t row_bytes = (int64_t)bn * (int64_t)cutile_dtype_size(x->dtype);
   const bool held = row_held(x->strides[1] == 1 && yt.strides[1] == 1, row_bytes);
@@ -2183,8 +2185,8 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
                  cutile_dtype_name(x->dtype), cutile_dtype_name(zt.dtype));
   const int32_t bm = z->partition_shape[0], bn = z->partition_shape[1];
   const int bk_user = generic_int(opts, 3, 64);
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(bn), "BN")) return s;
   CUTILE_REQUIRE(bk_user > 0, CUTILE_ERR_KERNEL_LAUNCH, "gemm: BK must be positive");
   CUTILE_REQUIRE(k >= 0, CUTILE_ERR_KERNEL_LAUNCH, "gemm: k must be non-negative");
   // The tile program runs k / BK whole K tiles (integer division).
@@ -2198,7 +2200,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
                            aligned16(zt.ptr) && x->shape[1] % 8 == 0 && y->shape[1] % 8 == 0 && zt.shape[1] % 4 == 0 &&
                            k_total % 8 == 0 && extent_bytes_2d(*x) < kDescriptorLimit && extent_bytes_2d(*y) < kDescriptorLimit &&
                            extent_bytes_2d(zt) < kDescriptorLimit;   // larger operands: the any-layout kernel (64-bit addresses)
-  const std::string dt = in_f32 ? "f32" : in_f16 ? "f16" : zt.dtype == CUTILE_DTYPE_BF16 ? "bf16" : "bf16f32";
+  const Name dt = in_f32 ? "f32" : in_f16 ? "f16" : zt.dtype == CUTILE_DTYPE_BF16 ? "bf16" : "bf16f32";
   // The ring-pipelined variants on 32 x 32 x 16 ("_r") fetch whole K tiles only ("_q" masks a ragged last tile).
   const int32_t k_valid = std::min(std::min(x->shape[1], y->shape[0]), k_total);
   // The streaming variants ("_s": one workgroup per compute unit walks its share of the tiles, the operand ring
@@ -2241,7 +2243,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
   // every kernel that fits these arguments: those of the partition's tile first, then those of other tiles, which compute the
   // same output when the launch covers all of z
   auto fitting = [&] {
-    std::vector<std::string> acceptable, others;
+    Names acceptable, others;
     for (const KernelEntry* entry : kernels_of("gemm")) {
       const KernelEntry& e = *entry;
       if (dt != e.dtype || strchr(e.variant, '+') != nullptr) continue;
@@ -2254,14 +2256,14 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
           others.push_back(e.variant);
       }
     }
-    acceptable.insert(acceptable.end(), others.begin(), others.end());
+    for (const Name& o : others) acceptable.push_back(o);
     acceptable.push_back(dt + "_generic");
     return acceptable;
   };
   Resolved res;
   // shape class for tuning records: the tile, and whether the tiles fit one wave of workgroups over the 256 CUs
-  BucketScope bucket(dt + "_" + std::to_string(bm) + "x" + std::to_string(bn) + ((uint64_t)tg[0] * tg[1] <= 256 ? "|tiles<=256" : "|tiles>256"));
-  const std::string fallback = record_first ? sized.variant : own_tile ? own_tile->variant : dt + "_generic";
+  BucketScope bucket(dt + "_" + num(bm) + "x" + num(bn) + ((uint64_t)tg[0] * tg[1] <= 256 ? "|tiles<=256" : "|tiles>256"));
+  const Name fallback = record_first ? sized.variant : own_tile ? own_tile->variant : dt + "_generic";
   if (record_first) sized.variant[0] = 0;
   ensure_tuning_records_loaded();
   if ((opts && opts->variant) || !preferred_variant("gemm").empty() || !preferred_variant_for("gemm", g_bucket, true).empty() ||
@@ -2366,14 +2368,14 @@ cutile_status_t cutile_launch_batch_matmul(cutile_stream_t stream, const cutile_
                  cutile_dtype_name(ct.dtype), cutile_dtype_name(a->dtype), cutile_dtype_name(b->dtype));
   CUTILE_REQUIRE(c->partition_shape[0] == 1, CUTILE_ERR_KERNEL_LAUNCH, "batch_matmul: c must be partitioned [1, BM, BN]");
   const int32_t bm = c->partition_shape[1], bn = c->partition_shape[2];
-  const std::string dt = cutile_dtype_name(ct.dtype);
+  const Name dt = cutile_dtype_name(ct.dtype);
   if (cutile_status_t s = check_generic(opts, 0, dt, "E")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(bn), "BN")) return s;
   const int bk_user = generic_int(opts, 3, 64);
   CUTILE_REQUIRE(bk_user > 0, CUTILE_ERR_KERNEL_LAUNCH, "batch_matmul: BK must be positive");
   CUTILE_REQUIRE(k >= 0, CUTILE_ERR_KERNEL_LAUNCH, "batch_matmul: k must be non-negative");
-  if (cutile_status_t s = check_generic(opts, 4, std::to_string(k), "K")) return s;
+  if (cutile_status_t s = check_generic(opts, 4, num(k), "K")) return s;
   const int32_t k_total = (k / bk_user) * bk_user;
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(c, opts, tg)) return s;
@@ -2388,7 +2390,7 @@ cutile_status_t cutile_launch_batch_matmul(cutile_stream_t stream, const cutile_
   const bool fast_layout = ct.dtype != CUTILE_DTYPE_F32 && slice_ok(*a) && slice_ok(*b) && slice_ok(ct) && k_total % 8 == 0 &&
                            (uint32_t)a->shape[0] >= batches && (uint32_t)b->shape[0] >= batches;
   const int32_t k_valid = std::min(std::min(a->shape[2], b->shape[1]), k_total);
-  std::vector<std::string> acceptable;
+  Names acceptable;
   if (fast_layout)
     for (const KernelEntry* entry : kernels_of("batch_matmul"))
       if (const KernelEntry& e = *entry; dt == e.dtype && e.tile[0] == bm && e.tile[1] == bn &&
@@ -2565,10 +2567,10 @@ cutile_status_t cutile_launch_gemm_persistent(cutile_stream_t stream, const cuti
   const int32_t bm = z->partition_shape[0], bn = z->partition_shape[1];
   const char* dt = in_f32 ? "f32" : in_f16 ? "f16" : "bf16";
   if (cutile_status_t s = check_generic(opts, 0, dt, "T")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(bn), "BN")) return s;
-  if (cutile_status_t s = check_generic(opts, 4, std::to_string(zm->map_shape[0]), "MAP_SHAPE[0]")) return s;
-  if (cutile_status_t s = check_generic(opts, 5, std::to_string(zm->map_shape[1]), "MAP_SHAPE[1]")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 4, num(zm->map_shape[0]), "MAP_SHAPE[0]")) return s;
+  if (cutile_status_t s = check_generic(opts, 5, num(zm->map_shape[1]), "MAP_SHAPE[1]")) return s;
   const int bk_user = generic_int(opts, 3, 64);
   CUTILE_REQUIRE(bk_user > 0, CUTILE_ERR_KERNEL_LAUNCH, "gemm_persistent: BK must be positive");
   // launch checks the reference derives from the kernel body (persistent_gemm.rs:20-26): the K tiles of x must exist in y
@@ -2587,13 +2589,13 @@ cutile_status_t cutile_launch_gemm_persistent(cutile_stream_t stream, const cuti
   const int32_t kx = x->shape[1];
   const bool whole_tiles = zt.shape[0] % bm == 0 && zt.shape[1] % bn == 0 && x->shape[0] >= zt.shape[0] && y->shape[1] >= zt.shape[1] &&
                            y->shape[0] >= kx && kx % 64 == 0 && kx >= 192 && m.rank == 2;
-  std::vector<std::string> acceptable;
+  Names acceptable;
   if (fast_layout)
     for (const KernelEntry* entry : kernels_of("gemm_persistent"))
       if (const KernelEntry& e = *entry; strcmp(e.dtype, dt) == 0 && e.tile[0] == bm && e.tile[1] == bn &&
           strchr(e.variant, '+') == nullptr && (whole_tiles || !is_stream_variant(e.variant)))
         acceptable.push_back(e.variant);
-  acceptable.push_back(std::string(dt) + "_generic");
+  acceptable.push_back(Name(dt) + "_generic");
   Resolved res;
   if (cutile_status_t s = resolve_entry("gemm_persistent", opts, acceptable[0], acceptable, &res)) return s;
   if (is_stream_variant(res.entry->variant)) {
@@ -2646,7 +2648,7 @@ cutile_status_t cutile_launch_group_gemm_f16_nt_desc(cutile_stream_t stream, con
   CUTILE_REQUIRE(!grid[0] || num_sm_generic <= 0 || (uint32_t)num_sm_generic == grid[0], CUTILE_ERR_KERNEL_LAUNCH,
                  "group_gemm_f16_nt_desc: the launch grid (%u) must equal NUM_SM = %d", grid[0], num_sm_generic);
   if (!grid[0]) grid[0] = (uint32_t)num_sm_generic;
-  std::vector<std::string> acceptable;
+  Names acceptable;
   for (const KernelEntry* entry : kernels_of("group_gemm_nt_desc"))
     if (const KernelEntry& e = *entry; e.tile[0] == bm && e.tile[1] == bn && strchr(e.variant, '+') == nullptr) acceptable.push_back(e.variant);
   CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND,
@@ -2690,7 +2692,7 @@ cutile_status_t cutile_launch_mapped_tile_index(cutile_stream_t stream, const cu
   MappedArg m;
   uint32_t grid[3];
   if (cutile_status_t s = mapped_launch_grid(zm, opts, &m, grid)) return s;
-  const std::string want = "i32_r" + std::to_string(z->tensor.rank);
+  const Name want = "i32_r" + num(z->tensor.rank);
   Resolved res;
   if (cutile_status_t s = resolve_entry("mapped_tile_index", opts, want, {want}, &res)) return s;
   ArgPacker args;
@@ -2710,7 +2712,7 @@ cutile_status_t cutile_launch_mapped_tile_index_within(cutile_stream_t stream, c
   uint32_t grid[3];
   if (cutile_status_t s = mapped_launch_grid(zm, opts, &full, grid)) return s;
   if (cutile_status_t s = mapped_subrange(zm, ranges, &m, &range, grid)) return s;
-  const std::string want = "i32_r" + std::to_string(z->tensor.rank);
+  const Name want = "i32_r" + num(z->tensor.rank);
   Resolved res;
   if (cutile_status_t s = resolve_entry("mapped_tile_index_within", opts, want, {want}, &res)) return s;
   ArgPacker args;
@@ -2905,8 +2907,8 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
                      k->shape[2] == v->shape[2],
                  CUTILE_ERR_KERNEL_LAUNCH, "fmha: k / v shapes do not match q");
   CUTILE_REQUIRE(input_pos >= 0, CUTILE_ERR_KERNEL_LAUNCH, "fmha: input_pos must be non-negative");
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(d), "D")) return s;
   const int bn_user = generic_int(opts, 1, 0);
   uint32_t tg[3];
   if (cutile_status_t s = resolve_grid(out, opts, tg)) return s;
@@ -2920,8 +2922,8 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   CUTILE_REQUIRE(extent_bytes_2d(m, d, q->strides[2], 2) < kDescriptorLimit && extent_bytes_2d(k->shape[2], d, k->strides[2], 2) < kDescriptorLimit &&
                      extent_bytes_2d(v->shape[2], d, v->strides[2], 2) < kDescriptorLimit && extent_bytes_2d(m, d, ot.strides[1], 2) < kDescriptorLimit,
                  CUTILE_ERR_KERNEL_NOT_FOUND, "fmha: the rows of one (batch, head) of q, k, v and out must each end below 2 GiB from the first");
-  const std::string dt = cutile_dtype_name(q->dtype);
-  std::vector<std::string> acceptable, same_bn;
+  const Name dt = cutile_dtype_name(q->dtype);
+  Names acceptable, same_bn;
   for (const KernelEntry* entry : kernels_of("fmha"))
     if (const KernelEntry& e = *entry; dt == e.dtype && e.tile[0] == bm && e.tile[2] == d && strchr(e.variant, '+') == nullptr) {
       acceptable.push_back(e.variant);
@@ -2931,8 +2933,8 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
                  "no precompiled variant of fmha<%s, BM=%d, D=%d>; available: %s", dt.c_str(), bm, d,
                  list_variants("fmha").c_str());
   Resolved res;
-  BucketScope bucket(dt + "_bm" + std::to_string(bm) + "_d" + std::to_string(d) + (causal ? "|causal" : "|full"));
-  const std::string fallback = same_bn.empty() ? acceptable[0] : same_bn[0];
+  BucketScope bucket(dt + "_bm" + num(bm) + "_d" + num(d) + (causal ? "|causal" : "|full"));
+  const Name fallback = same_bn.empty() ? acceptable[0] : same_bn[0];
   KeyPlan plan;   // (a caller that names the key tile means the kernel of that tile)
   int cus = 256;
   const int64_t seen = causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2];
@@ -2941,7 +2943,7 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
     if (cutile_status_t s = current_device_units(&cus)) return s;
     plan_keys(true);
   }
-  if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, plan.rows ? fallback : std::string())) return s;
+  if (cutile_status_t s = resolve_entry("fmha", opts, fallback, acceptable, &res, plan.rows ? fallback : Name())) return s;
   const bool by_keys = plan.rows && g_last_source == "size";
   SplitWorkspace ws;
   if (by_keys) {
@@ -2994,8 +2996,8 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   CUTILE_REQUIRE(out->partition_shape[2] == d && pack > 0 && query_group_size % pack == 0, CUTILE_ERR_KERNEL_LAUNCH,
                  "sequence attention: out must be partitioned [BM, G, %d] with G dividing query_group_size = %d, got [%d, %d, %d]",
                  d, query_group_size, bm, pack, out->partition_shape[2]);
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(d), "D")) return s;
   if (position_start) {
     if (cutile_status_t s = check_tensor(position_start, "position_start", 1, 1)) return s;
     CUTILE_REQUIRE(position_start->dtype == CUTILE_DTYPE_U32 && position_start->shape[0] == 1 &&
@@ -3038,18 +3040,18 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   ov.tensor.strides[0] = ot.strides[1]; ov.tensor.strides[1] = ot.strides[0]; ov.tensor.strides[2] = 1;
   // kernel tile: the ping-pong kernel for long D = 128 prefills, else the largest tile of that D
   const char* function = position_start ? "fmha_seq" : "fmha";
-  std::vector<const KernelEntry*> fit;
+  Few<const KernelEntry*, 12> fit;
   for (const KernelEntry* entry : kernels_of(function))
     if (const KernelEntry& e = *entry; strcmp(e.dtype, "f16") == 0 && e.tile[2] == d && strchr(e.variant, '+') == nullptr) fit.push_back(&e);
   CUTILE_REQUIRE(!fit.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "no precompiled sequence attention for f16, D = %d; available: %s", d,
                  list_variants(function).c_str());
   const bool long_prefill = rows_cov >= 256 && kv_len > 0;
-  std::stable_sort(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
+  sort_few(fit.begin(), fit.end(), [&](const KernelEntry* a, const KernelEntry* b) {
     const bool pa = strstr(a->variant, "_pp") != nullptr, pb = strstr(b->variant, "_pp") != nullptr;
     if (pa != pb) return long_prefill ? pa : pb;
     return a->tile[0] > b->tile[0];
   });
-  std::vector<std::string> acceptable;
+  Names acceptable;
   for (auto* e : fit)
     if (kv_len > 0 || strstr(e->variant, "_pp") == nullptr) acceptable.push_back(e->variant);   // an empty key range: the plain kernels only
   CUTILE_REQUIRE(!acceptable.empty(), CUTILE_ERR_KERNEL_NOT_FOUND, "no precompiled sequence attention for f16, D = %d and an empty key range", d);
@@ -3065,7 +3067,7 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
     if (cutile_status_t s = current_device_units(&cus)) return s;
     plan_keys(true);
   }
-  if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, plan.rows ? acceptable[0] : std::string())) return s;
+  if (cutile_status_t s = resolve_entry(function, &o, acceptable[0], acceptable, &res, plan.rows ? acceptable[0] : Name())) return s;
   const bool by_keys = plan.rows && g_last_source == "size";
   SplitWorkspace ws;
   if (by_keys) {
@@ -3127,8 +3129,8 @@ cutile_status_t cutile_launch_fmha_prefill_gqa_lpt_raw_f16(cutile_stream_t strea
   const int32_t bm = std::max(1, generic_int(opts, 0, 64));
   op.partition_shape[0] = bm, op.partition_shape[1] = group, op.partition_shape[2] = d;
   for (int i = 0; i < 3; ++i) op.partition_strides[i] = op.tensor.strides[i];
-  if (cutile_status_t s = check_generic(opts, 2, std::to_string(d), "D")) return s;
-  if (cutile_status_t s = check_generic(opts, 3, std::to_string(group), "GROUP")) return s;
+  if (cutile_status_t s = check_generic(opts, 2, num(d), "D")) return s;
+  if (cutile_status_t s = check_generic(opts, 3, num(group), "GROUP")) return s;
   cutile_launch_opts_t o = opts ? *opts : cutile_launch_opts_t{};
   o.generics = nullptr;
   o.n_generics = 0;
@@ -3157,8 +3159,8 @@ cutile_status_t cutile_launch_linear_tile_mxfp8(cutile_stream_t stream, const cu
   CUTILE_REQUIRE(zt.shape[0] == M && zt.shape[1] == N, CUTILE_ERR_KERNEL_LAUNCH, "linear_tile: z is [%d, %d], expected [%d, %d]",
                  zt.shape[0], zt.shape[1], M, N);
   const int32_t bm = z->partition_shape[0], bn = z->partition_shape[1];
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bn), "BN")) return s;
   const int bk_user = generic_int(opts, 2, 128);
   CUTILE_REQUIRE(bk_user > 0 && bk_user % 32 == 0 && generic_int(opts, 3, bk_user / 32) == bk_user / 32,
                  CUTILE_ERR_KERNEL_LAUNCH, "linear_tile: BK must be a multiple of 32 and BK_SCALES = BK/32");
@@ -3180,10 +3182,10 @@ cutile_status_t cutile_launch_linear_tile_mxfp8(cutile_stream_t stream, const cu
                  "linear_tile: precompiled variants address an operand with 32-bit byte offsets: x, y, the scales and z must each end "
                  "below 2 GiB from their first element (x spans %lld bytes, y %lld, z %lld)",
                  (long long)extent_bytes_2d(*x), (long long)extent_bytes_2d(*y), (long long)extent_bytes_2d(zt));
-  const std::string dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
-  const std::string missing = "no precompiled variant of linear_tile<" + std::to_string(bm) + ", " + std::to_string(bn) + ", " + std::to_string(bk_user) +
-                              ", " + std::to_string(bk_user / 32) + "> -> " + dt;
-  BucketScope bucket("mxfp8_" + dt + "_" + std::to_string(bm) + "x" + std::to_string(bn));
+  const Name dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
+  auto missing = [&] { return "no precompiled variant of linear_tile<" + num(bm) + ", " + num(bn) + ", " + num(bk_user) +
+                              ", " + num(bk_user / 32) + "> -> " + dt; };
+  BucketScope bucket("mxfp8_" + dt + "_" + num(bm) + "x" + num(bn));
   Resolved res;
   int cus = 256;
   ScaledRoom room;
@@ -3216,8 +3218,8 @@ cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cu
   CUTILE_REQUIRE(zt.shape[0] == M && zt.shape[1] == N, CUTILE_ERR_KERNEL_LAUNCH,
                  "linear_tile (nvfp4): z is [%d, %d], expected [%d, %d]", zt.shape[0], zt.shape[1], M, N);
   const int32_t bm = z->partition_shape[0], bn = z->partition_shape[1];
-  if (cutile_status_t s = check_generic(opts, 0, std::to_string(bm), "BM")) return s;
-  if (cutile_status_t s = check_generic(opts, 1, std::to_string(bn), "BN")) return s;
+  if (cutile_status_t s = check_generic(opts, 0, num(bm), "BM")) return s;
+  if (cutile_status_t s = check_generic(opts, 1, num(bn), "BN")) return s;
   const int bk_user = generic_int(opts, 2, 64);
   CUTILE_REQUIRE(bk_user > 0 && bk_user % 16 == 0 && generic_int(opts, 3, bk_user / 2) == bk_user / 2 &&
                      generic_int(opts, 4, bk_user / 16) == bk_user / 16,
@@ -3242,9 +3244,9 @@ cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cu
                  "linear_tile (nvfp4): precompiled variants address an operand with 32-bit byte offsets: x, y, the scales and z must each "
                  "end below 2 GiB from their first element (x spans %lld bytes, y %lld, z %lld)",
                  (long long)extent_bytes_2d(*x), (long long)extent_bytes_2d(*y), (long long)extent_bytes_2d(zt));
-  const std::string dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
-  const std::string missing = "no precompiled variant of nvfp4 linear_tile<" + std::to_string(bm) + ", " + std::to_string(bn) + ", " + std::to_string(bk_user) +
-                              ", " + std::to_string(bk_user / 2) + ", " + std::to_string(bk_user / 16) + "> -> " + dt;
+  const Name dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
+  auto missing = [&] { return "no precompiled variant of nvfp4 linear_tile<" + num(bm) + ", " + num(bn) + ", " + num(bk_user) +
+                              ", " + num(bk_user / 2) + ", " + num(bk_user / 16) + "> -> " + dt; };
   const bool flat = full_cover && KP >= 128 && xs->strides[0] % 4 == 0 && ys->strides[0] % 4 == 0 && ((uintptr_t)xs->ptr & 3) == 0 && ((uintptr_t)ys->ptr & 3) == 0;
   Resolved res;
   int cus = 256;
