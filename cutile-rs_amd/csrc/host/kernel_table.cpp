@@ -540,10 +540,14 @@ std::string preferred_variant(const char* function) {
 Name class_winner(std::string_view function, std::string_view bucket, bool* from_record) {
   *from_record = false;
   if (bucket.empty()) return Name();
-  Name key(function);
-  (key += "|") += bucket;
+  char key[128];
+  const size_t n = function.size() + 1 + bucket.size();
+  if (n > sizeof(key)) return Name();   // longer than any that has a winner
+  memcpy(key, function.data(), function.size());
+  key[function.size()] = '|';
+  memcpy(key + function.size() + 1, bucket.data(), bucket.size());
   std::lock_guard<std::mutex> lock(g_pref_mutex);
-  auto it = g_bucket_preferred.find(std::string_view(key));
+  auto it = g_bucket_preferred.find(std::string_view(key, n));
   if (it == g_bucket_preferred.end()) return Name();
   *from_record = it->second.from_record;
   return it->second.variant;

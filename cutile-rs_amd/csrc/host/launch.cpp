@@ -18,6 +18,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "common.h"
@@ -285,12 +286,13 @@ cutile_status_t load_resolved(const char* function, const Name& variant, Resolve
 // `sized` (the launcher's own rule for extents that the shape classes of the tuning records do not tell apart), the shape
 // class's winner of a verified tuning record, then `fallback` (the table's order).  A pin or a winner that does not fit
 // these arguments is passed over, not an error.
-cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* opts, const Name& fallback,
-                              const Names& acceptable, Resolved* r, const Name& sized = Name()) {
+// `each(f)`: f(name) for every kernel that fits, until it returns true; whether it did.
+template <typename Each>
+cutile_status_t resolve_among(const char* function, const cutile_launch_opts_t* opts, const Name& fallback, Each each, Resolved* r, const Name& sized = Name()) {
   Name want;
   g_last_source = "caller";
   g_last_bucket = g_bucket;
-  auto fits = [&](const Name& v) { return !v.empty() && std::find(acceptable.begin(), acceptable.end(), v) != acceptable.end(); };
+  auto fits = [&](const Name& v) { return !v.empty() && each([&](const char* name) { return v == name; }); };
   if (opts && opts->variant) want = opts->variant;
   if (want.empty()) {
     std::string pref = preferred_variant(function);
@@ -320,13 +322,26 @@ cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* 
     want = fallback;
     g_last_source = "table";
   }
-  if (!acceptable.empty() && std::find(acceptable.begin(), acceptable.end(), want) == acceptable.end()) {
+  if (!fits(want)) {
     std::string list;
-    for (auto& a : acceptable) list.append(list.empty() ? "" : ", ").append(a.c_str());
+    each([&](const char* name) {
+      list.append(list.empty() ? "" : ", ").append(name);
+      return false;
+    });
     return fail(CUTILE_ERR_KERNEL_NOT_FOUND, "variant '%s' of kernel '%s' does not fit these arguments; fitting: %s",
                 want.c_str(), function, list.c_str());
   }
   return load_resolved(function, want, r);
+}
+
+cutile_status_t resolve_entry(const char* function, const cutile_launch_opts_t* opts, const Name& fallback,
+                              const Names& acceptable, Resolved* r, const Name& sized = Name()) {
+  auto each = [&](auto f) {
+    for (const Name& n : acceptable)
+      if (f(n.c_str())) return true;
+    return false;
+  };
+  return resolve_among(function, opts, fallback, each, r, sized);
 }
 
 // Nobody but the launcher has a say (no caller's variant, pin or record) and its choice is known to fit.
@@ -991,29 +1006,44 @@ cutile_status_t cutile_launch_convert(cutile_stream_t stream, const cutile_tenso
 // Measured on MI355X: up to 4 vectors (64 bytes) per lane stream at full rate, so
 // among those the smallest capacity wins and wider segments are split over more
 // wavefronts; only segments too long for that take more vectors per lane.
-static Names fitting_row_variants(const char* fn_name, const Name& prefix, int64_t seg_len) {
-  Few<const KernelEntry*, 12> fit;
-  for (const KernelEntry* entry : kernels_of(fn_name))
-    if (const KernelEntry& e = *entry; e.capacity >= seg_len &&
-        strncmp(e.variant, prefix.c_str(), prefix.size()) == 0)
-      fit.push_back(&e);
-  sort_few(fit.begin(), fit.end(), [](const KernelEntry* a, const KernelEntry* b) {
-    const int va = std::max(a->tile[2], 4), vb = std::max(b->tile[2], 4);
-    if (va != vb) return va < vb;
-    if (a->capacity != b->capacity) return a->capacity < b->capacity;
-    return a->tile[3] < b->tile[3];  // fewer wavefronts per segment first
-  });
-  Names names;
-  for (auto* e : fit) names.push_back(e->variant);
-  return names;
+// (The order does not depend on the launch: a function's kernels are sorted once.)
+static const std::vector<const KernelEntry*>& row_kernels(const char* fn_name) {
+  static const auto& index = *[] {
+    auto* m = new std::unordered_map<std::string_view, std::vector<const KernelEntry*>>();
+    for (const KernelEntry& e : kernel_table())
+      if (e.capacity > 0) (*m)[e.function].push_back(&e);
+    for (auto& kernels : *m)
+      std::stable_sort(kernels.second.begin(), kernels.second.end(), [](const KernelEntry* a, const KernelEntry* b) {
+        const int va = std::max(a->tile[2], 4), vb = std::max(b->tile[2], 4);
+        if (va != vb) return va < vb;
+        if (a->capacity != b->capacity) return a->capacity < b->capacity;
+        return a->tile[3] < b->tile[3];  // fewer wavefronts per segment first
+      });
+    return m;
+  }();
+  static const std::vector<const KernelEntry*> none;
+  auto it = index.find(fn_name);
+  return it == index.end() ? none : it->second;
 }
 
 // The any-layout kernels of a row-wise function, behind the ones that fit: `held` rows of `bytes` (adjacent elements) are at most what
 // the "generic" kernels hold in registers (kAnyRowMost, rowwise.hip), everything else is walked.  Both take every call.
 static bool row_held(bool adjacent, int64_t bytes) { return adjacent && bytes <= 32768; }
-static void add_any_layout(bool held, const Name& prefix, Names* acceptable) {
-  acceptable->push_back(prefix + (held ? "generic" : "walk"));
-  acceptable->push_back(prefix + (held ? "walk" : "generic"));
+// Picks the kernel: of those whose names begin with `prefix` the ones that hold `seg_len` values (`in_registers` launches), then the any-layout ones.
+static cutile_status_t resolve_rows(const char* fn_name, const cutile_launch_opts_t* opts, const Name& prefix, int64_t seg_len, bool in_registers, bool held, Resolved* r) {
+  const Name any[2] = {prefix + (held ? "generic" : "walk"), prefix + (held ? "walk" : "generic")};
+  auto each = [&](auto f) {
+    if (in_registers)
+      for (const KernelEntry* e : row_kernels(fn_name))
+        if (e->capacity >= seg_len && strncmp(e->variant, prefix.c_str(), prefix.size()) == 0 && f(e->variant)) return true;
+    return f(any[0].c_str()) || f(any[1].c_str());
+  };
+  Name first;
+  each([&](const char* name) {
+    first = name;
+    return true;
+  });
+  return resolve_among(fn_name, opts, first, each, r);
 }
 
 // Launch grid of a row-wise kernel over `segments` tile rows: register-resident
@@ -1070,13 +1100,10 @@ cutile_status_t cutile_launch_rms_norm_f16(cutile_stream_t stream, const cutile_
   const bool vec_ok = n % 8 == 0 && x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1 &&
                       x->strides[0] % 8 == 0 && ot.strides[0] % 8 == 0 && aligned16(x->ptr) && aligned16(ot.ptr) &&
                       aligned16(w->ptr);
-  Names acceptable;
-  if (vec_ok) acceptable = fitting_row_variants("rms_norm_f16", "", n);
   const bool held = row_held(x->strides[1] == 1 && ot.strides[1] == 1 && w->strides[0] == 1, 2 * (int64_t)n);
-  add_any_layout(held, "", &acceptable);
   Resolved res;
   BucketScope bucket("n" + pow2_class(n));
-  if (cutile_status_t s = resolve_entry("rms_norm_f16", opts, acceptable[0], acceptable, &res)) return s;
+  if (cutile_status_t s = resolve_rows("rms_norm_f16", opts, "", n, vec_ok, held, &res)) return s;
 
   ArgPacker args;
   args.push_tensor(*x);
@@ -1261,13 +1288,10 @@ static cutile_status_t launch_fused_norm(const char* fn, cutile_stream_t stream,
   auto row_ok = [&](const cutile_tensor_arg_t& t) { return t.strides[1] == 1 && t.strides[0] % 8 == 0 && aligned16(t.ptr); };
   const bool vec_ok = n % 8 == 0 && row_ok(*a) && row_ok(*b) && row_ok(ot) && (!out2 || row_ok(out2->tensor)) &&
                       w->strides[0] == 1 && aligned16(w->ptr) && (!w2 || (w2->strides[0] == 1 && aligned16(w2->ptr)));
-  Names acceptable;
-  if (vec_ok) acceptable = fitting_row_variants(fn, "", n);
   auto unit = [](const cutile_tensor_arg_t& t) { return t.strides[t.rank - 1] == 1; };
   const bool held = row_held(unit(*a) && unit(*b) && unit(*w) && (!w2 || unit(*w2)) && unit(ot) && (!out2 || unit(out2->tensor)), 2 * (int64_t)n);
-  add_any_layout(held, "", &acceptable);
   Resolved res;
-  if (cutile_status_t s = resolve_entry(fn, opts, acceptable[0], acceptable, &res)) return s;
+  if (cutile_status_t s = resolve_rows(fn, opts, "", n, vec_ok, held, &res)) return s;
   ArgPacker args;
   args.push_tensor(*a);
   args.push_tensor(*b);
@@ -2150,14 +2174,11 @@ cutile_status_t cutile_launch_softmax(cutile_stream_t stream, const cutile_tenso
   const bool vec_ok = bn % e == 0 && x->shape[1] % e == 0 && yt.shape[1] % e == 0 && x->strides[1] == 1 &&
                       yt.strides[1] == 1 && x->strides[0] % e == 0 && yt.strides[0] % e == 0 && aligned16(x->ptr) &&
                       aligned16(yt.ptr) && (uint64_t)x->shape[0] >= rows;
-  Names acceptable;
-  if (vec_ok) acceptable = fitting_row_variants("softmax", dt + "_w", bn);
   const int64_t row_bytes = (int64_t)bn * (int64_t)cutile_dtype_size(x->dtype);
   const bool held = row_held(x->strides[1] == 1 && yt.strides[1] == 1, row_bytes);
-  add_any_layout(held, dt + "_", &acceptable);
   Resolved res;
   BucketScope bucket(dt + "|bn" + pow2_class(bn));
-  if (cutile_status_t s = resolve_entry("softmax", opts, acceptable[0], acceptable, &res)) return s;
+  if (cutile_status_t s = resolve_rows("softmax", opts, dt + "_", bn, vec_ok, held, &res)) return s;
   ArgPacker args;
   args.push_tensor(*x);
   args.push_partition(*y);
@@ -3183,8 +3204,8 @@ cutile_status_t cutile_launch_linear_tile_mxfp8(cutile_stream_t stream, const cu
                  "below 2 GiB from their first element (x spans %lld bytes, y %lld, z %lld)",
                  (long long)extent_bytes_2d(*x), (long long)extent_bytes_2d(*y), (long long)extent_bytes_2d(zt));
   const Name dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
-  auto missing = [&] { return "no precompiled variant of linear_tile<" + num(bm) + ", " + num(bn) + ", " + num(bk_user) +
-                              ", " + num(bk_user / 32) + "> -> " + dt; };
+  auto missing = [&] { return std::string("no precompiled variant of linear_tile<") + num(bm).c_str() + ", " + num(bn).c_str() + ", " + num(bk_user).c_str() +
+                              ", " + num(bk_user / 32).c_str() + "> -> " + dt.c_str(); };
   BucketScope bucket("mxfp8_" + dt + "_" + num(bm) + "x" + num(bn));
   Resolved res;
   int cus = 256;
@@ -3245,8 +3266,8 @@ cutile_status_t cutile_launch_linear_tile_nvfp4(cutile_stream_t stream, const cu
                  "end below 2 GiB from their first element (x spans %lld bytes, y %lld, z %lld)",
                  (long long)extent_bytes_2d(*x), (long long)extent_bytes_2d(*y), (long long)extent_bytes_2d(zt));
   const Name dt = zt.dtype == CUTILE_DTYPE_F32 ? "f32" : "bf16";
-  auto missing = [&] { return "no precompiled variant of nvfp4 linear_tile<" + num(bm) + ", " + num(bn) + ", " + num(bk_user) +
-                              ", " + num(bk_user / 2) + ", " + num(bk_user / 16) + "> -> " + dt; };
+  auto missing = [&] { return std::string("no precompiled variant of nvfp4 linear_tile<") + num(bm).c_str() + ", " + num(bn).c_str() + ", " + num(bk_user).c_str() +
+                              ", " + num(bk_user / 2).c_str() + ", " + num(bk_user / 16).c_str() + "> -> " + dt.c_str(); };
   const bool flat = full_cover && KP >= 128 && xs->strides[0] % 4 == 0 && ys->strides[0] % 4 == 0 && ((uintptr_t)xs->ptr & 3) == 0 && ((uintptr_t)ys->ptr & 3) == 0;
   Resolved res;
   int cus = 256;

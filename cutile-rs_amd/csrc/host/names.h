@@ -13,7 +13,7 @@ namespace cutile {
 // A kernel's or a shape class's name.  Longer text than its room is cut off, and is then the name of nothing.
 class Name {
   uint8_t n_ = 0;
-  char s_[79];
+  char s_[47];   // (the longest name of a kernel has 34)
 
  public:
   Name() { s_[0] = 0; }

@@ -10,7 +10,7 @@ def test_names_beyond_their_room_are_refused(fake_hip):
     launch = lambda **kw: ct.rms_norm_f16(x, w, ct.partition(out, [1, 64]), 1e-6, **kw)
     launch()
     taken = ct.last_resolved()["symbol"].split("__")[1]
-    for name in (taken + "x", taken + "x" * 200, "x" * 77, "x" * 78, "x" * 79):
+    for name in (taken + "x", taken + "x" * 200, "x" * 45, "x" * 46, "x" * 47):
         with pytest.raises(ct.CutileError):
             launch(variant=name)
     launch(variant=taken)
