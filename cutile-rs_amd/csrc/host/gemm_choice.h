@@ -177,6 +177,29 @@ inline F32Plan f32_plan(const F32Strip& r, int64_t m, int64_t n, int32_t k, int 
   return best;
 }
 
+// The same for 64 x 64 tiles of aligned rows with a workspace, priced by the number of workgroups: up to one to a compute unit, which shares no K where
+// that many tiles are there already (us, K shared by as many as staged_splits says, and here: 262 x 2240 x 2304 on 128 x 128 tiles shared by two 15.4, unshared 12.4; 557 x 1408 x
+// 1728 13.2, 10.8; 374 x 1344 x 1024 9.7, 8.1; 403 x 960 x 1344 by two and none 10.9, 9.3).  Least squares over 1133
+// times of 260 products of 66 to 1800 rows, K shared by 1 to 8 (6.5 % rms); over the 231 of them that are not strips the kernel and split chosen take 0.98 of the time
+// before, 41 are chosen otherwise, 0.88 in the mean, one of them slower (706 x 448 x 8512 18.8, 19.5; with a rule that follows the prices alone 80, of which 5 by 2 to 12 %).
+struct StagedPlan {
+  uint32_t splits;
+  double us;
+};
+inline StagedPlan staged_plan(int64_t m, int64_t n, int32_t k, int cus) {
+  const int64_t t = (int64_t)tiles_of(m, n, 64, 64), kt = (k + 63) / 64;
+  const uint32_t even = staged_splits(64, 64, (uint64_t)t, k, cus);
+  StagedPlan best{1, 0.0};
+  double least = 1e30;
+  for (uint32_t s = 1; s <= 8; ++s) {
+    if (s > 1 && s != even && (kt < 4 * s || t * s > 2 * cus)) continue;
+    const double x = (double)(t * s) / cus, rate = x <= 1.0 ? 0.214 + 0.046 * x : 0.368 + 0.163 * (x - 1.0);
+    const double us = 4.47 + (double)((kt + s - 1) / s) * rate + (s > 1 ? 2.04 + 0.11 * s + 1.88e-6 * (double)(m * n * (int64_t)s) : 0.0);
+    if (us * (s == even ? 0.9 : 1.0) < least) least = us * (s == even ? 0.9 : 1.0), best = {s, us};
+  }
+  return best;
+}
+
 struct GemmChoice {
   char variant[48] = "";   // "": the partition's own tile (tuning record, then the table's order)
   bool needs_room = false; // the choice counts on room for partial sums: without it the kernel is to be chosen again
@@ -184,6 +207,7 @@ struct GemmChoice {
   RingPlan ring_plan{};
   const F32Strip* strip = nullptr;
   F32Plan strip_plan{};
+  uint32_t staged = 0;               // K splits of a staged kernel, where they are not staged_splits'
 };
 
 // Register-staged tiles and their prices (choose_gemm): us per K tile, alone on a compute unit and for each of several; us of start and output, paid by every round
@@ -281,6 +305,11 @@ inline GemmChoice choose_gemm(const GemmShape& s, int cus, uint64_t partial_byte
                   (sk > 1 ? a.split + a.sum * (double)(s.m * s.n * (int64_t)sk) : 0.0);
       // (a row of tiles of a large y: at 3.5 TB/s, ring tiles have more of it in flight; us here and there 54 x 7680 x 6272 34.3, 29.2; 64 x 4096 x 4096 18.0, 14.8)
       if (ring && s.m <= 64) us = std::max(us, a.ends + a.split + (double)(s.n * s.k) * 2 / 3.5e6);
+      if (ring && r.bm == 64 && r.bn == 64 && partial_bytes && t <= 2 * (uint64_t)cus && s.m > 64) {
+        const StagedPlan p = staged_plan(s.m, s.n, s.k, cus);
+        if (us < best * 0.98 || p.us < best * 0.96) picked = r.kernel, shares_k = p.splits > 1, c.ring = nullptr, c.staged = p.splits;
+        continue;
+      }
       if (us < best * (ring ? 0.98 : 1.0)) best = us, picked = r.kernel, shares_k = sk > 1, c.ring = nullptr;
     }
   }

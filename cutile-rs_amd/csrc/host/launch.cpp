@@ -2335,7 +2335,7 @@ cutile_status_t cutile_launch_gemm(cutile_stream_t stream, const cutile_partitio
     uint32_t grid[3] = {div_up(cover_n, res.entry->tile[1]), div_up(cover_m, res.entry->tile[3]), 1};
     const uint64_t blocks = (uint64_t)grid[0] * grid[1];
     const F32Strip* strip = in_f32 ? f32_strip(res.entry->tile[3]) : nullptr;
-    splits = strip ? (strip == sized.strip ? sized.strip_plan : f32_plan(*strip, cover_m, cover_n, k_valid, cus, partial_bytes)).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus, res.entry->tile[3], res.entry->tile[1], fast_layout) : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
+    splits = strip ? (strip == sized.strip ? sized.strip_plan : f32_plan(*strip, cover_m, cover_n, k_valid, cus, partial_bytes)).splits : is_thin(res.entry) ? thin_splits(blocks, k_valid, cus, res.entry->tile[3], res.entry->tile[1], fast_layout) : sized.staged && g_last_source == "size" ? sized.staged : staged_splits(res.entry->tile[3], res.entry->tile[1], blocks, k_valid, cus);
     splits = std::min(splits, split_limit(blocks, (uint64_t)res.entry->tile[1] * res.entry->tile[3]));
     if (partial_bytes == 0) splits = 1;
     if (splits > 1 && g_launch_mode == 0 && !ws.partials) {
