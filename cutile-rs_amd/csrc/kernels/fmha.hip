@@ -593,10 +593,14 @@ struct FmhaPingPong {
       }
       if (mine - j == 2) {
         tile(j, kb0, kb1, vb0, vb1, std::false_type{});
-        tile(j + 1, kb1, kb0, vb1, vb0, std::true_type{});
-      } else {
-        tile(j, kb0, kb1, vb0, vb1, std::true_type{});
+        ++j;
       }
+      // The last tile is one copy of its code for either parity, its buffers chosen at run time (it refills none that it reads).  With a copy to each
+      // the odd one spilled (180 bytes a lane), and every launch with an odd number of tiles in some workgroup paid 5 to 8 us for it.  us before and now: 128
+      // heads of 300 rows 22.2, 14.3, causal 21.2, 13.5; of 170 17.2, 10.2; 256 of 787 144, 111, causal 95, 89; even numbers 0.98 to 1.00 (4 x 32 x
+      // 4096 889, 862, causal 494, 485).  (One loop that is left between its two tiles, without the copy above: even numbers 1.02 to 1.05.)
+      const bool odd = j & 1;
+      tile(j, odd ? kb1 : kb0, odd ? kb0 : kb1, odd ? vb1 : vb0, odd ? vb0 : vb1, std::true_type{});
       if (LATE) {
         for (j = mine; j < tc; ++j) {
           if (j & 1) idle_tile(j, kb1, vb0); else idle_tile(j, kb0, vb1);
