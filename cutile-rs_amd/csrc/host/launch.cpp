@@ -2814,8 +2814,10 @@ namespace {
 //     and 73, not causal 55, 60 and 110
 //   Two rounds of 64 rows at D = 128 pay where causal tiles are long and of different lengths: keys in front of the rows (`start`) make them alike, and then the
 //     256-row kernel, which reads K and V a quarter as often, is the better one, the sooner the more workgroups there are (f16; 4 heads of 4320 82 and 41, 8 of 3811 74
-//     and 50, 6 of 5408 106 and 68; 16 of 2855 behind 6467 205 and 238).  Shorter ones, which also gain (8 heads of 2066 45 and 26, 16 of 1839 44 and 33; not 64 of 427, 16 and
-//     22), are left where they are.  (With the position on the device the other kernel is the one of 128 rows.)
+//     and 50, 6 of 5408 106 and 68; 16 of 2855 behind 6467 205 and 238).  So do shorter ones without keys in front of them, from about 1100 keys on, and from 830
+//     where the second round is half empty (8 heads of 2312 47 and 27, 16 of 1355 31 and 23.5, 12 of 2401 50 and 36, 20 of 868 22 and 19; not 24 of 788 behind that line,
+//     20.4 and 19.7, 28 of 938 23.3 and 23.7 or 64 of 440 14.4 and 19.8; over 50 launches beyond it 0.55 to 1.03, 0.76 in the mean).  3001 to 3071 keys, and a
+//     second round of up to 12 workgroups, are left where they were.  (With the position on the device the other kernel is the one of 128 rows.)
 // Every other launch of D = 64 has two wavefronts to 32 rows of the 128-row workgroup (us on one wavefront and on two: 32 heads of 4096 196 and 180, causal 109
 // and 102; 128 of 1024 57 and 54, 43 and 38), but where one wavefront has its keys as soon: while two workgroups to a compute unit are one round up to 448
 // keys without a mask (160 of 221 11.6 and 12.7, 128 of 354 14.6 and 15.4) and 256 under it (144 of 246 10.8 and 10.9), and under the mask up to 1000 with a
@@ -2827,6 +2829,7 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t s
   if (of32 <= cus) return 32;
   if (of64 <= cus) return 64;
   if (d == 64 && ((of64 <= 2 * cus && keys >= 512) || (of64 <= 4 * cus && causal && keys >= 1024))) return 64;
+  if (d == 128 && causal && start == 0 && of64 <= 2 * cus && 20 * of64 > 21 * cus && keys >= (20 * of64 <= 29 * cus ? 830 : 1100) && keys <= 3000) return 64;
   if (d == 128 && causal && of64 <= 2 * cus && keys >= 3072 && (double)start <= (double)rows * (1.1 - 0.45 * (double)of64 / cus)) return 64;
   const int64_t of128 = heads * ((rows + 127) / 128);
   const bool once = of128 <= 2 * cus;
