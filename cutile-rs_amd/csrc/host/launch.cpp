@@ -1546,23 +1546,23 @@ cutile_status_t cutile_launch_lm_head_argmax_blocks_f16(cutile_stream_t stream, 
   args.push_partition(*block_idx);
   args.push_val<int32_t>(vocab_size);
   args.push_tile_grid(tg);
-  // Two workgroups per compute unit, each walking a contiguous run of blocks, read fastest (2004 blocks of K = 4096: 156.8 us, one workgroup to
-  // a block 164.0; 1448 of 2048: 59.8, 63.1), unless the longest run is more than a fifth above the mean one (1320 of 4096, a sixth
-  // above: 109.8, 115.3): then a workgroup to a block, which the dispatcher evens out (602 blocks of 4096: 68.0 us on 512 runs, 57.9; 1155 of
-  // 2560: 76.3, 63.4; 1169 of 1024: 37.5, 27.8; 1692 of 4096: 146.7, 137.7), where that leaves the busiest compute unit fewer blocks.  Between three and
-  // three and a third blocks to a compute unit it has four either way, and single ones lose (820 blocks of 4096: 70.9, 78.1; of 2048: 38.5, 42.0; of
-  // 8192: 136.9, 153.4; of 5120: 90.3, 92.5), but for short rows whose last step of 1024 columns is at most three quarters full, or the
-  // only one: runs pay for whole steps (820 of 512: 22.4, 15.6; of 1024: 27.0, 21.6; 1792: 36.8, 36.2; 2304: 52.1, 45.1; 2816: 56.9, 53.7; 3328:
-  // 62.1, 62.6).  Nothing to even out where a compute unit holds no third workgroup (the hidden vector in LDS; 700 of 30720: 475, 481).
+  // Two workgroups per compute unit, each walking a contiguous run of blocks, read fastest (2004 blocks of K = 4096: 158.0 us, one workgroup to
+  // a block 162.6; 1536 of 1024: 33.4, 35.1), unless the longest run is more than a sixth above the mean one and a workgroup to a block, which the
+  // dispatcher evens out, leaves the busiest compute unit fewer blocks (520 blocks of 4096: 66 us on 512 runs, 55; 1155 of 2560: 66.5, 60.7; 2150 of
+  // 1024: 49.9, 46.3; of 4096: 184.7, 177.1).  Between three and three and a third blocks to a compute unit it has four either way, and single
+  // ones lose (820 blocks of 4096: 70.5 us, 78.8; of 2048: 38.0, 42.2), but for short rows whose last step of 1024 columns is at most three quarters
+  // full, or the only one (820 of 512: 14.7, 13.5; of 1024: 22.3, 22.3; of 1536: 30.4, 30.5).  Nothing to even out where a compute unit holds no
+  // third workgroup (the hidden vector in LDS; 700 of 30720: 475, 481).
   cutile_device_t device = nullptr;
   if (cutile_status_t s = current_device(&device)) return s;
   int cus = 0;
   if (cutile_status_t s = compute_units(device, &cus)) return s;
   const uint32_t runs = (uint32_t)std::max(cus, 1) * 2u;
   const uint32_t longest = div_up(tg[0], runs);
-  const bool uneven = tg[0] > runs && (uint64_t)longest * runs * 5 > (uint64_t)tg[0] * 6 && 3 * (2 * k + 512) <= 160 * 1024;
+  const uint64_t in_runs = (uint64_t)longest * runs;
   const bool fewer = div_up(tg[0], runs / 2) < 2 * longest, short_rows = k <= 1024 || (k < 3072 && k % 1024 != 0 && k % 1024 <= 768);
-  uint32_t grid[3] = {uneven && (fewer || short_rows) ? tg[0] : std::min(tg[0], runs), 1, 1};
+  const bool uneven = (fewer && in_runs * 6 > (uint64_t)tg[0] * 7) || (short_rows && in_runs * 5 > (uint64_t)tg[0] * 6);
+  uint32_t grid[3] = {tg[0] > runs && uneven && 3 * (2 * k + 512) <= 160 * 1024 ? tg[0] : std::min(tg[0], runs), 1, 1};
   return launch_packed(res.fn, grid, res.entry->block, (uint32_t)k * 2, stream, args);
 }
 

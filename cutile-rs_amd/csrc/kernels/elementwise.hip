@@ -799,36 +799,44 @@ extern "C" __global__ void __launch_bounds__(kThreads)
 
 // logits[r] = sum_k f32(weights[r, k]) * f32(hidden[0, k]) for the 64 rows of block b, then the block's winner.
 // The weights are read once, 16 bytes per lane and nontemporally (a [vocab, K] matrix streams through once per
-// token); the hidden vector sits in LDS.  A workgroup takes a contiguous run of blocks, as many as the launch gives it (a
-// stream of this kind reads fastest from few resident wavefronts); a wavefront takes
-// 16 of a block's 64 rows, two at a time, 1024 columns per step, and requests the next step's weights before it
-// multiplies the current ones.
+// token); the hidden vector sits in LDS.  Bound by the read rate where the loads in flight suffice.  A workgroup takes a contiguous run of
+// blocks, as many as the launch gives it (a stream of this kind reads fastest from few resident wavefronts); a wavefront takes
+// 16 of a block's 64 rows, eight loads a step, and requests the next step's weights before it multiplies the current ones.
+// A step is 2048 columns of two rows or, where those would be less than three quarters full, 512 columns of eight: loads past a row's end
+// ask for nothing, so half-full steps keep half as many bytes in flight (300 blocks of K = 512 12.0 -> 8.2 us, of 1024 14.0 -> 11.3, 1398 of
+// 512 32.5 -> 18.7, 1536 of 1024 39.5 -> 33.4, 2004 of 2560 106.6 -> 99.0).  Workgroups with a run of blocks take eight rows up to seven eighths (1320
+// of 1536 50.2 -> 48.3, of 5120 142.1 -> 138.2), those of a single block two (592 of 1536 24.7 us, on eight 25.3; of 5120 67.0, 68.0).  Fuller steps
+// stay on two rows: eight streams a wavefront read slower (2004 of 4096: 158.0 us on two rows, 164.1 on four, 169.9 on eight).  A
+// lane's sums run over the same columns in the same order either way.
+// The logits of a block lie in the half of LDS of its parity, so one barrier a block orders both; the wavefronts take the blocks'
+// winners in turn.
 namespace {
 
-constexpr int kLmRows = 64, kLmRowsPerWave = kLmRows / (kThreads / 64), kLmChunksPerStep = 64 * 4;
+constexpr int kLmRows = 64, kLmRowsPerWave = kLmRows / (kThreads / 64), kLmLoads = 8;
 
 struct LmHeadArgs {
   const _Float16* wp;
   const _Float16* hs;      // hidden in LDS
-  float* row_logit;        // kLmRows entries of LDS
-  Best* scratch;
+  float* row_logit;        // two times kLmRows entries of LDS: a block's logits lie in the half of its parity
   float* block_max;
   uint32_t* block_idx;
   int64_t w_stride0, max_stride, idx_stride;
-  int32_t w_rows, chunks, steps_per_pair, steps_per_block, b_begin, vocab_size;
+  int32_t w_rows, chunks, steps_per_group, steps_per_block, b_begin, vocab_size;
   int lane, wave;
 };
 
-typedef Vec16<_Float16> LmTile[2][4];
+template <int R>
+using LmTile = Vec16<_Float16>[R][kLmLoads / R];
 
-__device__ __forceinline__ void lm_head_issue(LmTile& w, const LmHeadArgs& a, int32_t step) {
+template <int R>
+__device__ __forceinline__ void lm_head_issue(LmTile<R>& w, const LmHeadArgs& a, int32_t step) {
   const int32_t b = a.b_begin + step / a.steps_per_block, in_block = step % a.steps_per_block;
-  const int64_t r0 = (int64_t)b * kLmRows + (in_block / a.steps_per_pair * (kThreads / 64) + a.wave) * 2;
-  const int32_t c0 = in_block % a.steps_per_pair * kLmChunksPerStep;
+  const int64_t r0 = (int64_t)b * kLmRows + (in_block / a.steps_per_group * (kThreads / 64) + a.wave) * R;
+  const int32_t c0 = in_block % a.steps_per_group * (64 * kLmLoads / R);
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < R; ++t)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < kLmLoads / R; ++u) {
       const int32_t c = c0 + u * 64 + a.lane;
       w[t][u].raw = u32x4{0, 0, 0, 0};   // a row beyond the matrix reads as zeros, like a padded tile load
       if (r0 + t < a.w_rows && c < a.chunks)
@@ -836,39 +844,56 @@ __device__ __forceinline__ void lm_head_issue(LmTile& w, const LmHeadArgs& a, in
     }
 }
 
-__device__ __forceinline__ void lm_head_consume(const LmTile& w, float (&acc)[2], const LmHeadArgs& a, int32_t step) {
+template <int R>
+__device__ __forceinline__ void lm_head_consume(const LmTile<R>& w, float (&acc)[R], const LmHeadArgs& a, int32_t step) {
   const int32_t b = a.b_begin + step / a.steps_per_block, in_block = step % a.steps_per_block;
-  const int32_t pair = in_block / a.steps_per_pair, part = in_block % a.steps_per_pair;
+  const int32_t group = in_block / a.steps_per_group, part = in_block % a.steps_per_group;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int32_t c = part * kLmChunksPerStep + u * 64 + a.lane;
+  for (int u = 0; u < kLmLoads / R; ++u) {
+    const int32_t c = part * (64 * kLmLoads / R) + u * 64 + a.lane;
     if (c < a.chunks) {
       Vec16<_Float16> h;
       h.raw = *reinterpret_cast<const u32x4*>(a.hs + (int64_t)c * 8);
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < R; ++t)
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[t] = __builtin_fmaf((float)w[t][u].v[e], (float)h.v[e], acc[t]);
     }
   }
-  if (part + 1 < a.steps_per_pair) return;
+  if (part + 1 < a.steps_per_group) return;
+  float* logits = a.row_logit + (b & 1) * kLmRows;
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
+  for (int t = 0; t < R; ++t) {
     acc[t] = lanes::across_wave<lanes::Sum>(acc[t]);
-    if (a.lane == 0) a.row_logit[(pair * (kThreads / 64) + a.wave) * 2 + t] = acc[t];
+    if (a.lane == 0) logits[(group * (kThreads / 64) + a.wave) * R + t] = acc[t];
     acc[t] = 0.0f;
   }
   if (in_block + 1 < a.steps_per_block) return;
   __syncthreads();
-  Best mine = {-INFINITY, INT32_MAX};
-  if (threadIdx.x < kLmRows) {
-    const int64_t idx = (int64_t)b * kLmRows + threadIdx.x;
-    mine = Best{idx < a.vocab_size ? a.row_logit[threadIdx.x] : kMaskedLogit, (int32_t)idx};
-  }
-  const Best r = block_best(mine, a.scratch);   // its barrier also orders these reads before the next block's writes
-  if (threadIdx.x == 0) {
+  if (a.wave != (b & (kThreads / 64 - 1))) return;
+  const int64_t idx = (int64_t)b * kLmRows + a.lane;
+  Best r = {idx < a.vocab_size ? logits[a.lane] : kMaskedLogit, (int32_t)idx};
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) r = better(r, Best{__shfl_xor(r.v, o, 64), __shfl_xor(r.i, o, 64)});
+  if (a.lane == 0) {
     a.block_max[(int64_t)b * a.max_stride] = r.v;
     a.block_idx[(int64_t)b * a.idx_stride] = (uint32_t)r.i;
+  }
+}
+
+template <int R>
+__device__ __forceinline__ void lm_head_run(LmHeadArgs& a, int32_t blocks) {
+  a.steps_per_group = max((a.chunks + 64 * kLmLoads / R - 1) / (64 * kLmLoads / R), 1);
+  a.steps_per_block = a.steps_per_group * (kLmRowsPerWave / R);
+  const int32_t steps = blocks * a.steps_per_block;
+  float acc[R] = {};
+  LmTile<R> even, odd;
+  lm_head_issue<R>(even, a, 0);
+  for (int32_t s = 0; s < steps; s += 2) {
+    if (s + 1 < steps) lm_head_issue<R>(odd, a, s + 1);
+    lm_head_consume<R>(even, acc, a, s);
+    if (s + 2 < steps) lm_head_issue<R>(even, a, s + 2);
+    if (s + 1 < steps) lm_head_consume<R>(odd, acc, a, s + 1);
   }
 }
 
@@ -878,7 +903,7 @@ extern "C" __global__ void __launch_bounds__(kThreads)
     lm_head_argmax_blocks_entry__f16(TensorArg<2> weights, TensorArg<2> hidden, PartitionArg<1> block_max,
                                      PartitionArg<1> block_idx, int32_t vocab_size, TileGrid g) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  __shared__ float row_logit[kLmRows];
+  __shared__ float row_logit[2 * kLmRows];
   __shared__ Best scratch[kThreads / 64];
   const int32_t n_blocks = min((int32_t)g.x, min(block_max.shape[0], block_idx.shape[0]));
   const int32_t b_begin = (int32_t)((int64_t)blockIdx.x * n_blocks / gridDim.x);
@@ -895,23 +920,16 @@ extern "C" __global__ void __launch_bounds__(kThreads)
   __syncthreads();
   if (vec) {
     LmHeadArgs a;
-    a.wp = wp, a.hs = hs, a.row_logit = row_logit, a.scratch = scratch;
+    a.wp = wp, a.hs = hs, a.row_logit = row_logit;
     a.block_max = (float*)block_max.ptr, a.block_idx = (uint32_t*)block_idx.ptr;
     a.w_stride0 = weights.strides[0], a.max_stride = block_max.strides[0], a.idx_stride = block_idx.strides[0];
     a.w_rows = weights.shape[0], a.chunks = k_len / 8;
-    a.steps_per_pair = max((a.chunks + kLmChunksPerStep - 1) / kLmChunksPerStep, 1);
-    a.steps_per_block = a.steps_per_pair * (kLmRowsPerWave / 2);
     a.b_begin = b_begin, a.vocab_size = vocab_size, a.lane = lane, a.wave = wave;
-    const int32_t steps = (b_end - b_begin) * a.steps_per_block;
-    float acc[2] = {0.0f, 0.0f};
-    LmTile even, odd;
-    lm_head_issue(even, a, 0);
-    for (int32_t s = 0; s < steps; s += 2) {
-      if (s + 1 < steps) lm_head_issue(odd, a, s + 1);
-      lm_head_consume(even, acc, a, s);
-      if (s + 2 < steps) lm_head_issue(even, a, s + 2);
-      if (s + 1 < steps) lm_head_consume(odd, acc, a, s + 1);
-    }
+    const int32_t spans = (a.chunks + 63) / 64, full = (spans + 3) / 4 * 4;   // of 512 columns
+    if (spans * 4 < full * 3 || (spans * 8 < full * 7 && (int32_t)gridDim.x < n_blocks))
+      lm_head_run<8>(a, b_end - b_begin);
+    else
+      lm_head_run<2>(a, b_end - b_begin);
     return;
   }
   for (int32_t b = b_begin; b < b_end; ++b) {
