@@ -178,9 +178,8 @@ inline F32Plan f32_plan(const F32Strip& r, int64_t m, int64_t n, int32_t k, int 
 }
 
 // The same for 64 x 64 tiles of aligned rows with a workspace, priced by the number of workgroups: up to one to a compute unit, which shares no K where
-// that many tiles are there already (us, K shared by as many as staged_splits says, and here: 262 x 2240 x 2304 on 128 x 128 tiles shared by two 15.4, unshared 12.4; 557 x 1408 x
-// 1728 13.2, 10.8; 374 x 1344 x 1024 9.7, 8.1; 403 x 960 x 1344 by two and none 10.9, 9.3).  Least squares over 1133
-// times of 260 products of 66 to 1800 rows, K shared by 1 to 8 (6.5 % rms); over the 231 of them that are not strips the kernel and split chosen take 0.98 of the time
+// that many tiles are there already (us, K shared by as many as staged_splits says or on 128 x 128 tiles, and here: 272 x 2176 x 1536 17.3, 13.0, both from memory; 374 x 1344 x 1024 9.7, 8.1 from the caches).  Least squares over 1133
+// times of 260 products of 66 to 1800 rows, K shared by 1 to 8 (6.5 % rms); without the floor below, over the 231 of them that are not strips, the kernel and split chosen take 0.98 of the time
 // before, 41 are chosen otherwise, 0.88 in the mean, one of them slower (706 x 448 x 8512 18.8, 19.5; with a rule that follows the prices alone 80, of which 5 by 2 to 12 %).
 struct StagedPlan {
   uint32_t splits;
@@ -193,7 +192,11 @@ inline StagedPlan staged_plan(int64_t m, int64_t n, int32_t k, int cus) {
   double least = 1e30;
   for (uint32_t s = 1; s <= 8; ++s) {
     if (s > 1 && s != even && (kt < 4 * s || t * s > 2 * cus)) continue;
-    const double x = (double)(t * s) / cus, rate = x <= 1.0 ? 0.214 + 0.046 * x : 0.368 + 0.163 * (x - 1.0);
+    const double x = (double)(t * s) / cus, fitted = x <= 1.0 ? 0.214 + 0.046 * x : 0.368 + 0.163 * (x - 1.0);
+    // (fitted with operands that the caches still hold; from memory a K tile of an unshared tile is 0.36 us however few there are, and the kernels it is
+    // compared with are 8 % slower.  At 0.30 no one of 56 products from memory loses by more than 1.3 %; unpriced 174 x 2048 x 2048 14.7 -> 16.1 us, 230 x 2560 x 2560 17.6 ->
+    // 19.6, while 272 x 2176 x 1536 17.3 -> 13.0, 230 x 3072 x 1024 12.9 -> 10.3 stay)
+    const double rate = s == 1 ? std::max(fitted, 0.30) : fitted;
     const double us = 4.47 + (double)((kt + s - 1) / s) * rate + (s > 1 ? 2.04 + 0.11 * s + 1.88e-6 * (double)(m * n * (int64_t)s) : 0.0);
     if (us * (s == even ? 0.9 : 1.0) < least) least = us * (s == even ? 0.9 : 1.0), best = {s, us};
   }

@@ -5,7 +5,7 @@ import torch
 from util import rel_l2
 
 # m, n, k, workgroups to a tile
-SIZES = [(262, 2240, 2304, 1), (557, 1408, 1728, 1), (374, 1344, 1024, 1), (403, 960, 1344, 1), (222, 1152, 3520, 3), (587, 256, 9024, 6), (1050, 256, 1088, 1)]
+SIZES = [(272, 2176, 1536, 1), (230, 3072, 1024, 1), (557, 1408, 1728, 1), (374, 1344, 1024, 1), (403, 960, 1344, 2), (222, 1152, 3520, 3), (587, 256, 9024, 6)]
 
 
 def test_how_many_share_a_tile(fake_hip):
@@ -22,6 +22,8 @@ def test_how_many_share_a_tile(fake_hip):
         assert launch(m, n, k) == ("f16_staged64x64", shares), (m, n, k, launch(m, n, k))
     # more tiles than two to a compute unit, and strips: as before
     assert launch(1500, 4096, 4096)[0] != "f16_staged64x64" and launch(40, 2240, 2304)[0] == "f16_thin64x64"
+    # a long K unshared is dearer from memory than from the caches
+    assert launch(262, 2240, 2304)[0] == launch(174, 2048, 2048)[0] == "f16_128x128x64_q2x2"
     # a kernel that the caller names shares K as it always did
     assert launch(262, 2240, 2304, variant="f16_staged64x64") == ("f16_staged64x64", 2)
 
