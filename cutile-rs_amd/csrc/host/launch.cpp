@@ -27,6 +27,7 @@
 #include "names.h"
 #include "runtime_state.h"
 #include "scratch.h"
+#include "../kernels/key_steps.h"
 #include "../kernels/mapped_partition.h"
 
 using cutile::MappedArg;
@@ -2843,7 +2844,7 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t s
 // 28.7 and 22.3; D = 64, 4 heads of 40 behind 4000 14.5 and 9.4.
 struct KeyPlan {
   int rows = 0;
-  int32_t steps = 1 << 28;   // more than there can be
+  int32_t steps = 1 << 25;   // more than there can be
   uint32_t shares = 1;
 };
 KeyPlan key_plan(int d, int64_t heads, int64_t rows, int64_t keys, int64_t start, bool causal, int cus, bool may_share) {
@@ -2961,7 +2962,7 @@ cutile_status_t cutile_launch_fmha(cutile_stream_t stream, const cutile_partitio
   const Name fallback = same_bn.empty() ? acceptable[0] : same_bn[0];
   KeyPlan plan;   // (a caller that names the key tile means the kernel of that tile)
   int cus = 256;
-  const int64_t seen = causal ? std::min<int64_t>((int64_t)input_pos + ot.shape[1], k->shape[2]) : k->shape[2];
+  const int32_t seen = keys_seen(ot.shape[1], ot.shape[1], input_pos, k->shape[2], causal);
   auto plan_keys = [&](bool may_share) { plan = key_plan(d, tg[0], ot.shape[1], seen, input_pos, causal, cus, may_share); };
   if (bm >= 128 && bn_user == 0 && (int64_t)tg[1] * bm >= ot.shape[1]) {
     if (cutile_status_t s = current_device_units(&cus)) return s;
@@ -3085,7 +3086,7 @@ cutile_status_t cutile_launch_fmha_seq_f16(cutile_stream_t stream, const cutile_
   Resolved res;
   KeyPlan plan;   // (a caller that names the key tile, or packs the heads of a group into its tiles, means the kernels of that form)
   int cus = 256;
-  const int64_t there = position_start ? max_seq : kv_len, seen = causal && !position_start ? std::min<int64_t>((int64_t)query_start + rows_cov, there) : there;
+  const int32_t seen = position_start ? max_seq : keys_seen(rows_cov, rows_cov, query_start, kv_len, causal);   // (at most, with the position on the device)
   auto plan_keys = [&](bool may_share) { plan = key_plan(d, heads_cov, rows_cov, seen, position_start ? 0 : query_start, causal, cus, may_share); };
   if (pack == 1 && generic_int(opts, 1, 0) == 0 && (!position_start || rows_cov > 128)) {   // (with the position on the device, rows are all that is known of the length: 128 of them see more keys than that)
     if (cutile_status_t s = current_device_units(&cus)) return s;

@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fmha_common.h"
+#include "key_steps.h"
 #include "split_k.h"
 
 namespace {
@@ -211,10 +212,10 @@ struct FmhaKeys {
       const uint32_t off = q0 + l32 < q_len ? (uint32_t)(((int64_t)(q0 + l32) * q_ld + ks * 16 + half * 8) * 2) : kOob;
       qf[ks] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(rq, off, 0, 0));
     }
-    const int32_t keys = causal ? min(input_pos + (q_tile + 1) * BM, k_len) : k_len;   // that any row of the workgroup sees
-    const int32_t all_steps = (keys + BN - 1) / BN, steps = shares_of.steps;
-    const uint32_t shares = (uint32_t)((all_steps + steps - 1) / steps), tile = (uint32_t)bh * g.y + (uint32_t)q_tile;
-    const int32_t j0 = (int32_t)blockIdx.z * steps, tc = min(all_steps, j0 + steps);   // key steps of this workgroup
+    const int32_t keys = keys_seen((q_tile + 1) * BM, q_len, input_pos, k_len, causal);   // that any row of the workgroup sees
+    const KeySteps mine = key_steps(keys, BN, shares_of.steps, blockIdx.z, gridDim.z);
+    const uint32_t shares = mine.shares, tile = (uint32_t)bh * g.y + (uint32_t)q_tile;
+    const int32_t j0 = mine.first, tc = mine.end;   // key steps of this workgroup
     if (blockIdx.z > 0 && j0 >= tc) return;
 
     int ld_row[kLoads], ld_unit[kLoads];
@@ -375,10 +376,10 @@ struct FmhaOwnKeys {
     head_and_tile(g.x, g.y, causal, (uint32_t)group_size, &bh, &q_tile);
     const int32_t batch = bh / H, head = bh % H, kv_head = head / group_size;
     const int32_t q_len = q.shape[2], k_len = k.shape[2], q0 = q_tile * BM;
-    const int32_t keys = causal ? min(input_pos + q0 + BM, k_len) : k_len;   // that any row sees
-    const int32_t all_steps = (keys + BN - 1) / BN, steps = shares_of.steps;
-    const uint32_t shares = (uint32_t)((all_steps + steps - 1) / steps), tile = (uint32_t)bh * g.y + (uint32_t)q_tile;
-    const int32_t j0 = (int32_t)blockIdx.z * steps, tc = min(all_steps, j0 + steps);   // key steps of this workgroup
+    const int32_t keys = keys_seen(q0 + BM, q_len, input_pos, k_len, causal);   // that any row sees
+    const KeySteps mine = key_steps(keys, BN, shares_of.steps, blockIdx.z, gridDim.z);
+    const uint32_t shares = mine.shares, tile = (uint32_t)bh * g.y + (uint32_t)q_tile;
+    const int32_t j0 = mine.first, tc = mine.end;   // key steps of this workgroup
     if (blockIdx.z > 0 && j0 >= tc) return;
     const int32_t my_end = min(tc, (keys - wave * 32 + BN - 1) / BN);   // behind this wavefront's last step with a key that any row sees
 
