@@ -2849,6 +2849,7 @@ struct KeyPlan {
 };
 KeyPlan key_plan(int d, int64_t heads, int64_t rows, int64_t keys, int64_t start, bool causal, int cus, bool may_share) {
   KeyPlan plan;
+  if (heads <= 0 || rows <= 0) return plan;   // the grid of a launch that covers nothing is refused
   plan.rows = key_sharing_rows(d, heads, rows, keys, start, causal, cus);
   if ((plan.rows != 32 && plan.rows != 64) || keys <= 256) return plan;
   struct Costs {

@@ -79,6 +79,21 @@ def test_a_launch_has_the_workgroups_that_its_kernel_counts(fake_hip, kernel_ste
     assert shared > 100
 
 
+@pytest.mark.parametrize("start", [0, 300])
+def test_a_launch_that_covers_nothing_is_refused(fake_hip, start):
+    ct = fake_hip
+    q, kv, out = torch.empty(1, 4, 300, 128).half(), torch.empty(1, 4, 300 + start, 128).half(), torch.empty(4, 300, 128).half()
+    seq, position = torch.empty(300, 4, 128).half(), torch.tensor([start], dtype=torch.int32)
+    for causal in (True, False):
+        for grid in ((0, 2, 1), (4, 0, 1), (0, 0, 1)):
+            with pytest.raises(ct.CutileError, match="zero axis"):
+                ct.fmha(ct.partition(out, [1, 256, 128], prefix=True), q, kv, kv, 0.1, start, 1, causal=causal, grid=grid)
+        for grid in ((3, 0, 1), (0, 4, 1)):
+            for where in (dict(kv_len=300 + start, query_start=start), dict(position_start=position)):
+                with pytest.raises(ct.CutileError, match="zero axis"):
+                    ct.fmha_seq_f16(seq, kv[0], kv[0], ct.partition(torch.empty_like(seq), [128, 1, 128], prefix=True), 0.1, 1, causal=causal, grid=grid, **where)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("heads,group,rows,start,there", [(8, 4, 17, 4079, 4200), (4, 1, 33, 2015, 2100), (2, 1, 129, 895, 1100), (8, 4, 17, 4079, 4096)])
