@@ -347,8 +347,7 @@ struct GroupAhead {
       const __amdgpu_buffer_rsrc_t part = make_rsrc(partials + (size_t)(cw.tile - whole) * splits * (BM * BN), kTile * splits);
       if (active) {
 #pragma unroll
-        for (int r = 0; r < NB; ++r)
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[r % TN][r / TN]), part, threadIdx.x * 16, split * kTile + r * (kThreads * 16), kAgentScope);
+        for (int r = 0; r < NB; ++r) store_partial(acc[r % TN][r / TN], part, split * kTile + r * (kThreads * 16) + threadIdx.x * 16);
       }
       if (!last_to_arrive(counters + (cw.tile - whole), splits, flag) || !active) return;
       clear();

@@ -13,6 +13,11 @@ namespace gemm {
 // and counter move with agent-scope accesses (past the L2); the workgroup that counts last adds the partials in split
 // order, whatever order they arrived in, so the sum does not depend on timing.
 constexpr int kAgentScope = 16;   // buffer accesses with sc1: past the L2, which the XCDs do not share
+// 16 bytes of a partial sum.  No scalar offset: a 16-byte store that has one reads its data registers for some cycles after it issues, and the
+// compiler, which guards only the other form, may reuse them in the next instruction.
+__device__ __forceinline__ void store_partial(f32x4 v, __amdgpu_buffer_rsrc_t to, uint32_t at) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), to, at, 0, kAgentScope);
+}
 // The partial sums of one block: quads of four neighbouring outputs, numbered as the kernel likes, one copy of `bytes` per split.
 struct BlockPartials {
   __amdgpu_buffer_rsrc_t rsrc;
@@ -20,7 +25,7 @@ struct BlockPartials {
 
   __device__ __forceinline__ BlockPartials(float* mine, uint32_t block_bytes, uint32_t n) : rsrc(make_rsrc(mine, block_bytes * n)), bytes(block_bytes), splits(n) {}
   __device__ __forceinline__ void store(uint32_t split, int quad, f32x4 v) const {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, quad * 16, split * bytes, kAgentScope);
+    store_partial(v, rsrc, split * bytes + quad * 16);
   }
   // take(quad, sum in split order) for every quad, dealt to THREADS threads, Q quads of eight splits at a time: a read past the L2 takes about a
   // microsecond, and one after another (a value, a split) they were much of a launch of few rows (f16, kernel time in us with such reads and
@@ -75,7 +80,7 @@ __device__ __forceinline__ bool combine_tile(f32x4 (&acc)[TN][TM], float* mine, 
   const __amdgpu_buffer_rsrc_t part = make_rsrc(mine, kTile * splits);
 #pragma unroll
   for (int r = 0; r < TM * TN; ++r)
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[r % TN][r / TN]), part, threadIdx.x * 16, split * kTile + r * (THREADS * 16), kAgentScope);
+    store_partial(acc[r % TN][r / TN], part, split * kTile + r * (THREADS * 16) + threadIdx.x * 16);
   if (!last_to_arrive(counter, splits, shared_flag)) return false;
   // (one partial tile at a time: with the next one's loads in flight beside it 48 and 54 tiles of 128 x 128 took 14.5 us where they take 13.7)
   auto add = [&](uint32_t k) {

@@ -1,4 +1,8 @@
 """Partial sums of outputs whose K is shared by more workgroups than are read at once (split_k.h): nine and sixteen of them, one row to a full strip."""
+import os
+import re
+import subprocess
+
 import pytest
 import torch
 
@@ -42,3 +46,20 @@ def test_as_many_splits_as_the_test_above_means(fake_hip, dtype):
         rows, cols = map(int, variant.split("strip" if dtype == torch.float32 else "thin")[1].split("x"))
         strips = -(-m // rows) * -(-n // cols)
         assert _workgroups(ct) == strips * (16 if dtype == torch.float32 else splits), (m, n, k, variant, _workgroups(ct))
+
+
+def test_no_wide_store_leaves_its_data_unguarded():
+    """A 16-byte buffer store with its offset in a scalar register reads its data registers for some cycles after it issues; the compiler guards their next write only
+    where there is no such offset.  In every code object each store of that form has two idle cycles behind it."""
+    lib = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cutile-rs_amd", "lib")
+    objects = sorted(f for f in os.listdir(lib) if f.endswith(".hsaco"))
+    assert "gemmsmall.hsaco" in objects
+    guarded = 0
+    for name in objects:
+        text = subprocess.run(["/opt/rocm/llvm/bin/llvm-objdump", "-d", "--no-show-raw-insn", os.path.join(lib, name)], stdout=subprocess.PIPE, text=True, check=True).stdout
+        lines = text.splitlines()
+        for store, behind in zip(lines, lines[1:]):
+            if re.match(r"\s*buffer_store_dwordx[34] v\[\d+:\d+\], (v\d+|off), s\[\d+:\d+\], (s\d+|m0|vcc|exec|ttmp)", store):
+                assert re.match(r"\s*s_nop [1-9]", behind), (name, store, behind)
+                guarded += 1
+    assert guarded > 0      # those of the streaming kernels, which wait by themselves
