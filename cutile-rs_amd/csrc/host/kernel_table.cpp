@@ -263,7 +263,7 @@ std::vector<KernelEntry> build_table() {
     for (auto t : {std::array<int, 2>{192, 320}, std::array<int, 2>{192, 384}, std::array<int, 2>{192, 448}, std::array<int, 2>{256, 320}}) {
       const std::string tile = "w" + std::to_string(t[0]) + "x" + std::to_string(t[1]);
       add("gemm", keep(std::string(dt) + "_192x256x64_q2x4+" + tile), keep(std::string("gemm_entry__") + dt + "_" + tile + "_192x256x64_q2x4_mix"), IMG_GEMM_TILES, 512,
-          (uint32_t)(2 * (t[0] + t[1]) * 64 * 2), 192, 256, 64, 0, dt, 0, 2);
+          (uint32_t)(2 * (t[0] + t[1]) * 64 * 2), t[0], t[1], 64, 0, dt, 0, 2);
     }
   // medium sizes: register-staged tiles, K split over workgroups (any alignment, any partition shape); two LDS stages
   for (const char* dt : {"bf16", "f16", "bf16f32"})

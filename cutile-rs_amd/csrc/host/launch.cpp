@@ -352,10 +352,10 @@ cutile_status_t resolve_own(const char* function, const char* variant, const cha
   return load_resolved(function, variant, r);
 }
 
-// The table's first kernel for a partition's tile shape, or nullptr.
+// The table's first kernel for a partition's tile shape, or nullptr (a member of a family is no partition's kernel).
 const KernelEntry* first_of_tile(const char* function, const Name& dtype, int bm, int bn) {
   for (const KernelEntry* e : kernels_of(function))
-    if (e->tile[0] == bm && e->tile[1] == bn && dtype == e->dtype) return e;
+    if (e->tile[0] == bm && e->tile[1] == bn && dtype == e->dtype && strchr(e->variant, '+') == nullptr) return e;
   return nullptr;
 }
 
