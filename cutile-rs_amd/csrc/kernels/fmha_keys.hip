@@ -380,6 +380,8 @@ struct FmhaOwnKeys {
     const int32_t j0 = mine.first, tc = mine.end;   // key steps of this workgroup
     if (blockIdx.z > 0 && j0 >= tc) return;
     const int32_t my_end = min(tc, (keys - wave * 32 + BN - 1) / BN);   // behind this wavefront's last step with a key that any row sees
+    static_assert(R <= 2, "a last step has all row blocks, or the second alone");
+    const int32_t low_end = min(tc, (keys_seen(q0 + 32, q_len, input_pos, k_len, causal) - wave * 32 + BN - 1) / BN);   // the last one with a key that the first 32 rows see
 
     const T* qb = (const T*)q.ptr + (int64_t)batch * q.strides[0] + (int64_t)head * q.strides[1];
     const T* kb = (const T*)k.ptr + (int64_t)batch * k.strides[0] + (int64_t)kv_head * k.strides[1];
@@ -455,7 +457,9 @@ struct FmhaOwnKeys {
     constexpr int kWaitOlder = (kInstr & 15) | (7 << 4) | (15 << 8);               // all but the newest kInstr requests have landed
     constexpr int kReadsHome = 15 | (3 << 14) | (7 << 4);                          // LDS reads only
 
-    for (int32_t j = j0; j < my_end; ++j) {
+    // a key step of row blocks B0 ..
+    auto step = [&](int32_t j, auto from) {
+      constexpr int B0 = decltype(from)::value;
       const int32_t first = j * BN + wave * 32;   // of the wavefront's keys
       __builtin_amdgcn_s_waitcnt(kWaitOlder);     // K (V behind it may be on its way)
       __builtin_amdgcn_sched_barrier(0);
@@ -471,7 +475,7 @@ struct FmhaOwnKeys {
       __builtin_amdgcn_sched_barrier(0);
       f32x16 s[R];
 #pragma unroll
-      for (int b = 0; b < R; ++b)
+      for (int b = B0; b < R; ++b)
 #pragma unroll
         for (int e = 0; e < 16; ++e) s[b][e] = 0.0f;
       if constexpr (kQInLds) {
@@ -479,7 +483,7 @@ struct FmhaOwnKeys {
         vec8 ring[kRing][R];
         auto read_q = [&](int ks, vec8 (&into)[R]) {
 #pragma unroll
-          for (int b = 0; b < R; ++b) into[b] = *reinterpret_cast<const vec8*>(q_lds + (q_at ^ (ks << 5)) + b * 32 * (D * 2));
+          for (int b = B0; b < R; ++b) into[b] = *reinterpret_cast<const vec8*>(q_lds + (q_at ^ (ks << 5)) + b * 32 * (D * 2));
         };
 #pragma unroll
         for (int ks = 0; ks < kAhead; ++ks) read_q(ks, ring[ks]);
@@ -487,19 +491,19 @@ struct FmhaOwnKeys {
         for (int ks = 0; ks < KS; ++ks) {
           if (ks + kAhead < KS) read_q(ks + kAhead, ring[(ks + kAhead) % kRing]);
 #pragma unroll
-          for (int b = 0; b < R; ++b) s[b] = E::mfma(kf[ks], ring[ks % kRing][b], s[b]);
+          for (int b = B0; b < R; ++b) s[b] = E::mfma(kf[ks], ring[ks % kRing][b], s[b]);
           __builtin_amdgcn_sched_barrier(0);
         }
       } else {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-          for (int b = 0; b < R; ++b) s[b] = E::mfma(kf[ks], qf[b * KS + ks], s[b]);
+          for (int b = B0; b < R; ++b) s[b] = E::mfma(kf[ks], qf[b * KS + ks], s[b]);
       }
       // s[b][e] belongs to key first + (e/4)*8 + half*4 + e%4 and to this lane's query row of block b
       vec8 pf[R][2];
 #pragma unroll
-      for (int b = 0; b < R; ++b) {
+      for (int b = B0; b < R; ++b) {
         if (first + 31 > all_see) {
           const int32_t lim = (causal ? min(q0 + b * 32 + l32 + input_pos, k_len - 1) : k_len - 1) - half * 4 - first;   // last key the lane may see
 #pragma unroll
@@ -556,8 +560,13 @@ struct FmhaOwnKeys {
 #pragma unroll
       for (int n = 0; n < NO; ++n)
 #pragma unroll
-        for (int b = 0; b < R; ++b) o_acc[b][n % DB] = E::mfma(vf[n], pf[b][n / DB], o_acc[b][n % DB]);
-    }
+        for (int b = B0; b < R; ++b) o_acc[b][n % DB] = E::mfma(vf[n], pf[b][n / DB], o_acc[b][n % DB]);
+    };
+    int32_t j = j0;
+    for (; j < low_end; ++j) step(j, std::integral_constant<int, 0>{});
+    // (keys that only the other block's rows see: zero times a value that is not finite would not be zero in the first one.  A branch around the products instead spills 316 bytes a lane)
+    if constexpr (R > 1)
+      if (j < my_end) step(j, std::integral_constant<int, 1>{});
     __builtin_amdgcn_s_waitcnt(0);   // trailing (zero-filling) fetches must not land in what follows
 
     // The partial outputs, row block by row block: row l32, 16-byte unit u of it at u ^ (row & 15), in LDS that other wavefronts have done with, too.
