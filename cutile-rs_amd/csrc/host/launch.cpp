@@ -2851,16 +2851,14 @@ KeyPlan key_plan(int d, int64_t heads, int64_t rows, int64_t keys, int64_t start
   KeyPlan plan;
   if (heads <= 0 || rows <= 0) return plan;   // the grid of a launch that covers nothing is refused
   plan.rows = key_sharing_rows(d, heads, rows, keys, start, causal, cus);
-  if ((plan.rows != 32 && plan.rows != 64) || keys <= 256) return plan;
+  if ((plan.rows != 32 && (plan.rows != 64 || d == 64)) || keys <= 256) return plan;   // (64 rows at D = 64, or 128: more tiles than half of the compute units)
   struct Costs {
-    int step;
     double begin, each, load, share, all;
   };
   auto best = [&](int of, double* price) {
-    static constexpr Costs kCosts[2][2] = {{{256, 5.3, 0.64, 0.54, 0.15, 1.1}, {128, 5.3, 0.98, 0.04, 0.12, 2.2}},       // D = 64: 32 rows, 64
-                                           {{256, 7.6, 1.18, 0.43, 0.27, 1.7}, {256, 8.7, 1.62, 0.37, 0.67, 2.0}}};      // D = 128
-    const Costs& c = kCosts[d == 128][of == 64];
-    const int64_t tiles = heads * ((rows + of - 1) / of), steps = (keys + c.step - 1) / c.step;
+    static constexpr Costs kCosts[3] = {{5.3, 0.64, 0.54, 0.15, 1.1}, {7.6, 1.18, 0.43, 0.27, 1.7}, {8.7, 1.62, 0.37, 0.67, 2.0}};   // D = 64; D = 128: 32 rows, 64
+    const Costs& c = kCosts[d == 64 ? 0 : of == 32 ? 1 : 2];
+    const int64_t tiles = heads * ((rows + of - 1) / of), steps = (keys + 255) / 256;
     const int64_t room = std::min<int64_t>(cus / tiles, (int64_t)(kSplitPartialBytes / (size_t)(of * (d + 2) * 4)) / tiles);
     KeyPlan r;
     r.rows = of;

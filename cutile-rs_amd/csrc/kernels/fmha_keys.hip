@@ -103,6 +103,11 @@ struct Bands {
   int in_first;
   __device__ __forceinline__ unsigned char* operator[](int w) const { return (w < in_first ? first + w * (32 * D * 4) : second + (w - in_first) * (32 * D * 4)); }
 };
+template <int D>
+struct OneBand {
+  unsigned char* first;
+  __device__ __forceinline__ unsigned char* operator[](int w) const { return first + w * (32 * D * 4); }
+};
 
 // What a lane has of the results of a row block (32 query rows) whose keys S wavefronts share: four columns of PASSES rows.
 template <int S, int D>
@@ -110,30 +115,37 @@ struct RowShare {
   static constexpr int UNITS = D / 4 / S, ROWS = 64 / UNITS, PASSES = 32 / ROWS;   // 16-byte units of a row to a wavefront, rows at a time
 };
 
-// The partial outputs and statistics that those wavefronts left in LDS (from wavefront `first` on), added up in the order of a step's keys: wavefront wk its share of the columns.
-template <int S, int D, int N>
-__device__ __forceinline__ void merge_block(const Bands<D>& bands, const float (*row_max)[32], const float (*row_sum)[32], int first, int wk, int at, f32x4 (&o)[N],
-                                            float (&m)[N], float (&l)[N]) {
+// Pass p over the partial outputs and statistics that those wavefronts left in LDS (from wavefront `first` on), added up in the order of a step's keys: wavefront wk its share of the columns.
+template <int S, int D, typename BANDS>
+__device__ __forceinline__ void merge_pass(const BANDS& bands, const float (*row_max)[32], const float (*row_sum)[32], int first, int wk, int p, f32x4& o, float& m, float& l) {
   using H = RowShare<S, D>;
   const int lane = threadIdx.x & 63, unit = wk * H::UNITS + lane % H::UNITS;
+  const int r = p * H::ROWS + lane / H::UNITS;
+  float top = -INFINITY;
 #pragma unroll
-  for (int p = 0; p < H::PASSES; ++p) {
-    const int r = p * H::ROWS + lane / H::UNITS;
-    float top = -INFINITY;
+  for (int s = 0; s < S; ++s) top = fmaxf(top, row_max[first + s][r]);
+  const float use = top == -INFINITY ? 0.0f : top;
+  float sum = 0.0f;
+  f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int s = 0; s < S; ++s) top = fmaxf(top, row_max[first + s][r]);
-    const float use = top == -INFINITY ? 0.0f : top;
-    float sum = 0.0f;
-    f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < S; ++s) {
+    const float w = __builtin_amdgcn_exp2f(row_max[first + s][r] - use);
+    sum = __builtin_fmaf(row_sum[first + s][r], w, sum);
+    const f32x4 part = *reinterpret_cast<const f32x4*>(bands[first + s] + r * (D * 4) + ((unit ^ (r & 15)) << 4));
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const float w = __builtin_amdgcn_exp2f(row_max[first + s][r] - use);
-      sum = __builtin_fmaf(row_sum[first + s][r], w, sum);
-      const f32x4 part = *reinterpret_cast<const f32x4*>(bands[first + s] + r * (D * 4) + ((unit ^ (r & 15)) << 4));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(part[e], w, t[e]);
-    }
-    o[at + p] = t, m[at + p] = top, l[at + p] = sum;
+    for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(part[e], w, t[e]);
+  }
+  o = t, m = top, l = sum;
+}
+
+// Four columns of row `qr`, from `unit` on.
+template <typename T>
+__device__ __forceinline__ void store_row(const PartitionArg<3>& out, int32_t bh, int32_t q_len, int32_t qr, int unit, const f32x4& o, float l) {
+  using E = Elem<T>;
+  const float sum = fmaxf(l, 1.0e-8f);   // a row that saw no key: 0 (as in Fmha)
+  if (qr < out.shape[1] && qr < q_len) {
+    const u32x2 w = {E::pack2(o[0] / sum, o[1] / sum), E::pack2(o[2] / sum, o[3] / sum)};
+    *reinterpret_cast<u32x2*>((T*)out.ptr + (int64_t)bh * out.strides[0] + (int64_t)qr * out.strides[1] + unit * 4) = w;
   }
 }
 
@@ -142,7 +154,6 @@ template <typename T, int B, int S, int D, int TILE_ROWS>
 __device__ __forceinline__ void store_rows(const PartitionArg<3>& out, int32_t bh, int32_t q_len, int32_t tile_row0, int block0, int wk, f32x4 (&o)[B * RowShare<S, D>::PASSES],
                                            float (&m)[B * RowShare<S, D>::PASSES], float (&l)[B * RowShare<S, D>::PASSES], const KeyShares& ks, uint32_t tile, uint32_t shares,
                                            uint32_t* flag) {
-  using E = Elem<T>;
   using H = RowShare<S, D>;
   constexpr int N = B * H::PASSES;
   const int lane = threadIdx.x & 63, unit = wk * H::UNITS + lane % H::UNITS;
@@ -151,16 +162,10 @@ __device__ __forceinline__ void store_rows(const PartitionArg<3>& out, int32_t b
   for (int p = 0; p < N; ++p) row[p] = (block0 + p / H::PASSES) * 32 + p % H::PASSES * H::ROWS + lane / H::UNITS;
   if (shares > 1 && !add_key_shares<N, TILE_ROWS, 512>(ks, tile, blockIdx.z, shares, o, m, l, row, wk == 0 && lane % H::UNITS == 0, flag)) return;
 #pragma unroll
-  for (int p = 0; p < N; ++p) {
-    const float sum = fmaxf(l[p], 1.0e-8f);   // a row that saw no key: 0 (as in Fmha)
-    const int32_t qr = tile_row0 + row[p];
-    if (qr < out.shape[1] && qr < q_len) {
-      const u32x2 w = {E::pack2(o[p][0] / sum, o[p][1] / sum), E::pack2(o[p][2] / sum, o[p][3] / sum)};
-      *reinterpret_cast<u32x2*>((T*)out.ptr + (int64_t)bh * out.strides[0] + (int64_t)qr * out.strides[1] + unit * 4) = w;
-    }
-  }
+  for (int p = 0; p < N; ++p) store_row<T>(out, bh, q_len, tile_row0 + row[p], unit, o[p], l[p]);
 }
 
+// One workgroup to all keys of a query tile: its launches are those whose tiles are more than half of the compute units.
 template <typename T, int R, int S, int STAGES, int D>
 struct FmhaKeys {
   using E = Elem<T>;
@@ -181,7 +186,7 @@ struct FmhaKeys {
   }
 
   __device__ static __forceinline__ void run(const PartitionArg<3>& out, const TensorArg<4>& q, const TensorArg<4>& k, const TensorArg<4>& v,
-                                             float qk_scale, int32_t input_pos, int32_t group_size, int32_t causal, const TileGrid& g, const KeyShares& shares_of) {
+                                             float qk_scale, int32_t input_pos, int32_t group_size, int32_t causal, const TileGrid& g, const KeyShares&) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[kLdsBytes];
     __shared__ float row_max[kWaves][32], row_sum[kWaves][32];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -211,10 +216,7 @@ struct FmhaKeys {
       qf[ks] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(rq, off, 0, 0));
     }
     const int32_t keys = keys_seen((q_tile + 1) * BM, q_len, input_pos, k_len, causal);   // that any row of the workgroup sees
-    const KeySteps mine = key_steps(keys, BN, shares_of.steps, blockIdx.z, gridDim.z);
-    const uint32_t shares = mine.shares, tile = (uint32_t)bh * g.y + (uint32_t)q_tile;
-    const int32_t j0 = mine.first, tc = mine.end;   // key steps of this workgroup
-    if (blockIdx.z > 0 && j0 >= tc) return;
+    const int32_t tc = (keys + BN - 1) / BN;
 
     int ld_row[kLoads], ld_unit[kLoads];
 #pragma unroll
@@ -251,13 +253,13 @@ struct FmhaKeys {
     const int32_t all_see = causal ? min(q0 + input_pos, k_len - 1) : k_len - 1;             // last key that every row of the wavefront sees
     const int32_t any_sees = causal ? min(q0 + 31 + input_pos, k_len - 1) : k_len - 1;       // last key that one of them sees
 
-    if (tc > j0) {
-      load_global(j0);
+    if (tc > 0) {
+      load_global(0);
       store_lds(0);
     }
     __syncthreads();
-    for (int32_t j = j0; j < tc; ++j) {
-      const int cur = STAGES == 2 ? (j - j0) & 1 : 0;
+    for (int32_t j = 0; j < tc; ++j) {
+      const int cur = STAGES == 2 ? j & 1 : 0;
       if (j + 1 < tc) load_global(j + 1);
       const unsigned char* sk = lds + cur * kStageBytes;
       const unsigned char* sv = sk + kTileBytes;
@@ -334,10 +336,15 @@ struct FmhaKeys {
         *reinterpret_cast<f32x4*>(lds + wave * kOutBytes + l32 * (D * 4) + (((db * 8 + qd * 2 + half) ^ (l32 & 15)) << 4)) = w;
       }
     __syncthreads();
-    f32x4 o[RowShare<S, D>::PASSES];
-    float m[RowShare<S, D>::PASSES], l[RowShare<S, D>::PASSES];
-    merge_block<S, D>(Bands<D>{lds, lds, kWaves}, row_max, row_sum, wr * S, wk, 0, o, m, l);
-    store_rows<T, 1, S, D, BM>(out, bh, q_len, q_tile * BM, wr, wk, o, m, l, shares_of, tile, shares, reinterpret_cast<uint32_t*>(lds));
+    using Share = RowShare<S, D>;
+    const OneBand<D> bands{lds};
+#pragma unroll
+    for (int p = 0; p < Share::PASSES; ++p) {   // (a row's sums leave as soon as they are there: held back for the rows behind them they cost 1 to 2 % of a short launch)
+      f32x4 o;
+      float m, l;
+      merge_pass<S, D>(bands, row_max, row_sum, wr * S, wk, p, o, m, l);
+      store_row<T>(out, bh, q_len, q0 + p * Share::ROWS + lane / Share::UNITS, wk * Share::UNITS + lane % Share::UNITS, o, l);
+    }
   }
 };
 
@@ -587,7 +594,8 @@ struct FmhaOwnKeys {
           *reinterpret_cast<f32x4*>(bands[wave] + l32 * (D * 4) + (((db * 8 + qd * 2 + half) ^ (l32 & 15)) << 4)) = w;
         }
       __syncthreads();
-      merge_block<kWaves, D>(bands, row_max, row_sum, 0, wave, b * Share::PASSES, o, m, l);
+#pragma unroll
+      for (int p = 0; p < Share::PASSES; ++p) merge_pass<kWaves, D>(bands, row_max, row_sum, 0, wave, p, o[b * Share::PASSES + p], m[b * Share::PASSES + p], l[b * Share::PASSES + p]);
     }
     store_rows<T, R, kWaves, D, BM>(out, bh, q_len, q0, 0, wave, o, m, l, shares_of, tile, shares, reinterpret_cast<uint32_t*>(ks_lds));
   }
