@@ -805,7 +805,9 @@ extern "C" __global__ void __launch_bounds__(kThreads)
 // A step is 2048 columns of two rows or, where those would be less than three quarters full, 512 columns of eight: loads past a row's end
 // ask for nothing, so half-full steps keep half as many bytes in flight (300 blocks of K = 512 12.0 -> 8.2 us, of 1024 14.0 -> 11.3, 1398 of
 // 512 32.5 -> 18.7, 1536 of 1024 39.5 -> 33.4, 2004 of 2560 106.6 -> 99.0).  Workgroups with a run of blocks take eight rows up to seven eighths (1320
-// of 1536 50.2 -> 48.3, of 5120 142.1 -> 138.2), those of a single block two (592 of 1536 24.7 us, on eight 25.3; of 5120 67.0, 68.0).  Fuller steps
+// of 1536 50.2 -> 48.3, of 5120 142.1 -> 138.2), those of a single block two (592 of 1536 24.7 us, on eight 25.3; of 5120 67.0, 68.0), also for
+// more than 768 columns where the busiest of 256 compute units has four of them (us on two rows and on eight: 790 blocks of 960 20.0, 21.0, of 896 19.2, 19.9, 820 of
+// 1024 21.7, 22.1; of 768 18.0, 18.0; 600 blocks of 960 16.7, 15.9, 1155 of 960 26.2, 25.8).  Fuller steps
 // stay on two rows: eight streams a wavefront read slower (2004 of 4096: 158.0 us on two rows, 164.1 on four, 169.9 on eight).  A
 // lane's sums run over the same columns in the same order either way.
 // The logits of a block lie in the half of LDS of its parity, so one barrier a block orders both; the wavefronts take the blocks'
@@ -926,7 +928,8 @@ extern "C" __global__ void __launch_bounds__(kThreads)
     a.w_rows = weights.shape[0], a.chunks = k_len / 8;
     a.b_begin = b_begin, a.vocab_size = vocab_size, a.lane = lane, a.wave = wave;
     const int32_t spans = (a.chunks + 63) / 64, full = (spans + 3) / 4 * 4;   // of 512 columns
-    if (spans * 4 < full * 3 || (spans * 8 < full * 7 && (int32_t)gridDim.x < n_blocks))
+    const bool runs = (int32_t)gridDim.x < n_blocks, four = !runs && n_blocks > 768 && n_blocks <= 1024 && spans == 2 && k_len > 768;
+    if (!four && spans * (runs ? 8 : 4) < full * (runs ? 7 : 3))
       lm_head_run<8>(a, b_end - b_begin);
     else
       lm_head_run<2>(a, b_end - b_begin);
