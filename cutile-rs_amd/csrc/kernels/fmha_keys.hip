@@ -160,7 +160,7 @@ __device__ __forceinline__ void store_rows(const PartitionArg<3>& out, int32_t b
   int row[N];
 #pragma unroll
   for (int p = 0; p < N; ++p) row[p] = (block0 + p / H::PASSES) * 32 + p % H::PASSES * H::ROWS + lane / H::UNITS;
-  if (shares > 1 && !add_key_shares<N, TILE_ROWS, 512>(ks, tile, blockIdx.z, shares, o, m, l, row, wk == 0 && lane % H::UNITS == 0, flag)) return;
+  if (!add_key_shares<N, TILE_ROWS, 512>(ks, tile, blockIdx.z, shares, o, m, l, row, wk == 0 && lane % H::UNITS == 0, flag)) return;
 #pragma unroll
   for (int p = 0; p < N; ++p) store_row<T>(out, bh, q_len, tile_row0 + row[p], unit, o[p], l[p]);
 }
@@ -388,7 +388,7 @@ struct FmhaOwnKeys {
     if (blockIdx.z > 0 && j0 >= tc) return;
     const int32_t my_end = min(tc, (keys - wave * 32 + BN - 1) / BN);   // behind this wavefront's last step with a key that any row sees
     static_assert(R <= 2, "a last step has all row blocks, or the second alone");
-    const int32_t low_end = min(tc, (keys_seen(q0 + 32, q_len, input_pos, k_len, causal) - wave * 32 + BN - 1) / BN);   // the last one with a key that the first 32 rows see
+    const int32_t low_end = R == 1 ? my_end : min(tc, (keys_seen(q0 + 32, q_len, input_pos, k_len, causal) - wave * 32 + BN - 1) / BN);   // the last one with a key that the first 32 rows see
 
     const T* qb = (const T*)q.ptr + (int64_t)batch * q.strides[0] + (int64_t)head * q.strides[1];
     const T* kb = (const T*)k.ptr + (int64_t)batch * k.strides[0] + (int64_t)kv_head * k.strides[1];
@@ -595,9 +595,13 @@ struct FmhaOwnKeys {
         }
       __syncthreads();
 #pragma unroll
-      for (int p = 0; p < Share::PASSES; ++p) merge_pass<kWaves, D>(bands, row_max, row_sum, 0, wave, p, o[b * Share::PASSES + p], m[b * Share::PASSES + p], l[b * Share::PASSES + p]);
+      for (int p = 0; p < Share::PASSES; ++p) {
+        const int at = b * Share::PASSES + p;
+        merge_pass<kWaves, D>(bands, row_max, row_sum, 0, wave, p, o[at], m[at], l[at]);
+        if (shares == 1) store_row<T>(out, bh, q_len, q0 + b * 32 + p * Share::ROWS + lane / Share::UNITS, wave * Share::UNITS + lane % Share::UNITS, o[at], l[at]);
+      }
     }
-    store_rows<T, R, kWaves, D, BM>(out, bh, q_len, q0, 0, wave, o, m, l, shares_of, tile, shares, reinterpret_cast<uint32_t*>(ks_lds));
+    if (shares > 1) store_rows<T, R, kWaves, D, BM>(out, bh, q_len, q0, 0, wave, o, m, l, shares_of, tile, shares, reinterpret_cast<uint32_t*>(ks_lds));
   }
 };
 
