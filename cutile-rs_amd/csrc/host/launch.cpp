@@ -2839,7 +2839,7 @@ int key_sharing_rows(int d, int64_t heads, int64_t rows, int64_t keys, int64_t s
 }
 // The kernel of those rows, and the keys of its query tiles dealt to several workgroups where a round of them leaves compute units idle: `steps` key steps
 // to each.  What a step costs grows with the share of the compute units at work; bringing the results together costs a part for each and one for
-// all (fitted to 204, 271, 298 and 36 launches of one round: the pick takes 1.01 of the best one's time).  One round only: behind it nothing was left to gain.
+// all (fitted to 204, 298 and 36 launches of one round: the pick takes 1.01 of the best one's time).  One round only: behind it nothing was left to gain.
 // us, keys not dealt out and dealt: D = 128, 32 rows: 8 heads of 17 rows behind 3905 keys 27 and 12.9, 12 of 28 behind 5078 33 and 15.2, 16 of 200 behind 4000
 // 28.7 and 22.3; D = 64, 4 heads of 40 behind 4000 14.5 and 9.4.
 struct KeyPlan {
